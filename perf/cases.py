@@ -51,14 +51,14 @@ def listed():
         # Attention of one layer over a long prompt.
         dict(name="prompt attention", kind="prompt_attention", heads=32, kv_heads=8, dim=128, tokens=4096),
         # The quantised transformer as served: a prompt, the next token of one sequence, of a batch of sequences.
-        dict(name="transformer, prompt", kind="w4_prompt", tokens=700, **SMALL),
-        dict(name="transformer, token", kind="w4_token", context=2048, **SMALL),
-        dict(name="transformer, batch", kind="w4_batch", batch=32, shortest=1024, longest=2048, **SMALL),
+        dict(name="transformer prompt", kind="w4_prompt", tokens=700, **SMALL),
+        dict(name="transformer token", kind="w4_token", context=2048, **SMALL),
+        dict(name="transformer batch", kind="w4_batch", batch=32, shortest=1024, longest=2048, **SMALL),
         # Layered decoders: a long prompt, and a short prompt with the tokens of a reply behind it.
-        dict(name="recurrent and routed, prompt", kind="layered_prompt", tokens=2048, **BAROVIK),
-        dict(name="recurrent and routed, reply", kind="layered_reply", tokens=64, reply=24, **BAROVIK_SMALL),
-        dict(name="side by side, prompt", kind="layered_prompt", tokens=3001, **KOKETAR),
-        dict(name="side by side, reply", kind="layered_reply", tokens=64, reply=24, **KOKETAR_SMALL),
+        dict(name="recurrent and routed prompt", kind="layered_prompt", tokens=2048, **BAROVIK),
+        dict(name="recurrent and routed reply", kind="layered_reply", tokens=64, reply=24, **BAROVIK_SMALL),
+        dict(name="side by side prompt", kind="layered_prompt", tokens=3001, **KOKETAR),
+        dict(name="side by side reply", kind="layered_reply", tokens=64, reply=24, **KOKETAR_SMALL),
     ]
 
 
