@@ -43,6 +43,8 @@ size_t w4a16_gemv_workspace_bytes(uint32_t m, uint32_t n, uint32_t k);
 // The same for the prefill GEMM (m > kGemvMaxRows), which splits K over workgroups when its
 // tiles would leave half the CUs idle; without the workspace and the counters it does not split.
 size_t w4a16_gemm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k);
+// True when the linear takes the small tiles of w4a16_rows.hip, which need no workspace.
+bool w4a16_rows_ok(const W4LinearArgs &args);
 
 // Optional RMS normalisation of the activation rows on their way into a decode kernel
 // (weight == nullptr: none): the kernel multiplies by half(x * gain * r) (weight_first) or

@@ -51,6 +51,13 @@ hipError_t launch_w4a16_gemv_mfma_dual_swiglu(const W4DualSwigluArgs &args, hipS
 bool w4a16_gemv_quad_ok(const W4LinearArgs &args);
 hipError_t launch_w4a16_gemv_quad_linear(const W4LinearArgs &args, hipStream_t stream);
 
+// More rows than the GEMVs take, fewer tiles than the large ones need (w4a16_rows.hip).
+bool w4a16_rows_ok(const W4QkvArgs &args);
+bool w4a16_rows_ok(const W4DualSwigluArgs &args);
+hipError_t launch_w4a16_rows_linear(const W4LinearArgs &args, hipStream_t stream);
+hipError_t launch_w4a16_rows_qkv(const W4QkvArgs &args, hipStream_t stream);
+hipError_t launch_w4a16_rows_dual_swiglu(const W4DualSwigluArgs &args, hipStream_t stream);
+
 hipError_t launch_w4a16_gemm_linear(const W4LinearArgs &args, hipStream_t stream);
 hipError_t launch_w4a16_gemm_dual_swiglu(const W4DualSwigluArgs &args, hipStream_t stream);
 

@@ -1,0 +1,404 @@
+// W4A16 products of a batch's rows (more than the streaming GEMVs take, fewer than a prompt's) and of prompts over small
+// matrices: tiles of 16, 32 or 64 activation rows by 32 or 64 weight columns, so that the launch has about a workgroup
+// per CU where 128 x 128 tiles leave most of them empty or pad most of their rows.
+//
+// What bounds it at many rows of K: the weights from HBM (31 MB at 4096 x 14336: 6.5 us at a copy's rate) and the
+// activation rows, which every workgroup reads again, from L2; at a CU's rate of filling LDS (about 80 bytes a
+// nanosecond) 32 rows take 3 us and 64 rows 6 us of their own.  With a short K, the start of a launch and two or three
+// trips to memory.
+//
+//  * A workgroup is CT x P waves.  A step covers P scale groups (64 K values each) of the tile's rows and columns; wave
+//    (ct, p) multiplies group p of the step into the 32 columns ct.  The waves that share columns split K this way at the
+//    finest grain, so a step's requests are whole lines of every row, and their sums meet once, at the end, in LDS.
+//  * Both operands go global -> LDS as direct copies, a ring of STAGES steps, waited for by count, one barrier a step.
+//    16-byte pieces are XOR-ed by the row, so that the rows an operand read touches lie in different banks.
+//  * A lane of the 32 x 32 x 16 product holds 32 K values (16 bytes) of one weight row and its partner lane the other
+//    half of the same scale group: four products a group, on exact integers, and the group's fp16 scale is one float32
+//    multiply-add per sum, as in the GEMVs (the 128 x 128 tiles round q * s to half).
+//  * The scales of the tile are copied to LDS ahead of everything else (a dword each).
+//
+// Measured at 24 x 4096 x 14336 (us): 13.3 (128 x 128 tiles 27 to 31), of which 4.9 the launch's start, first trip to memory and
+// epilogue; the copies alone take 9.3 and the products alone 10.6 of the same launch: 85 vector instructions a wave and
+// step (52 of them the decode) beside 24 KB of copies.  Tried without gain: operands read a step ahead of their use,
+// two column blocks a wave, a start of the walk over K that differs by workgroup, deeper rings.
+#include <algorithm>
+
+#include "kernels.h"
+#include "kernels_internal.h"
+#include "w4_common.h"
+
+namespace llmopt {
+namespace {
+
+struct RowsParams {
+  const uint16_t *x;
+  uint32_t m, k;
+  // One matrix, the two of a gated pair (tile columns alternate), or several that multiply the same rows: their column
+  // tiles follow each other.
+  const uint8_t *w[3];
+  const uint16_t *s[3];
+  uint16_t *y[3];
+  uint32_t n[3];
+  uint32_t tiles[3];
+  uint32_t segments;
+  const uint16_t *addend;
+  uint32_t addend_stride;
+};
+
+// base + offset (bytes, per lane) to consecutive LDS places: sixteen bytes a lane ...
+__device__ __forceinline__ void copy16_to_lds(const void *base, uint32_t offset, uint32_t lds_address) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(lds_address) : "memory");
+}
+// ... or two, stored as a dword.
+__device__ __forceinline__ void copy2_to_lds(const void *base, uint32_t offset, uint32_t lds_address) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_ushort %0, %1" : : "v"(offset), "s"(base), "s"(lds_address) : "memory");
+}
+
+// Eight weights of a dword as exact halves in K order.
+__device__ __forceinline__ h8_t w4_exact_natural(uint32_t word) {
+  const W4Pairs q = w4_decode_pairs(word);
+  const uint32_t p04 = as_u32(q.p04), p15 = as_u32(q.p15), p26 = as_u32(q.p26), p37 = as_u32(q.p37);
+  uint4 packed;
+  packed.x = __builtin_amdgcn_perm(p15, p04, 0x05040100u);
+  packed.y = __builtin_amdgcn_perm(p37, p26, 0x05040100u);
+  packed.z = __builtin_amdgcn_perm(p15, p04, 0x07060302u);
+  packed.w = __builtin_amdgcn_perm(p37, p26, 0x07060302u);
+  return __builtin_bit_cast(h8_t, packed);
+}
+
+// Scales of a tile in LDS: blocks of eight columns by eight groups, a dword each.
+constexpr uint32_t scale_lds_bytes(uint32_t columns, uint32_t groups) { return columns / 8 * ((groups + 7) / 8) * 256; }
+
+template <int ROWS, int CT, int P, int STAGES, bool DUAL>
+__global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(RowsParams p) {
+  constexpr int WAVES = CT * P, COLUMNS = CT * 32, STEP = P * 64;
+  constexpr int RT = (ROWS + 31) / 32;                      // 32-row blocks of a wave
+  constexpr int X_PIECES = STEP / 8, W_PIECES = STEP / 32;  // 16-byte pieces of a row and step
+  constexpr int X_BYTES = ROWS * X_PIECES * 16, W_BYTES = COLUMNS * W_PIECES * 16, STAGE_BYTES = X_BYTES + W_BYTES;
+  constexpr int X_COPIES = X_BYTES / 1024 / WAVES, COPIES = X_COPIES + 1;  // of a wave and step
+  static_assert(X_BYTES == X_COPIES * WAVES * 1024 && W_BYTES == WAVES * 1024, "a step divides over the waves");
+  static_assert(!DUAL || CT % 2 == 0, "gate and up columns of an output lie in one tile");
+  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ct = wave / P, part = wave % P;
+  const uint32_t groups = p.k / 64, steps = (groups + P - 1) / P;
+
+  uint32_t segment = 0, tile = blockIdx.x;
+  if (!DUAL)
+    while (segment + 1 < p.segments && tile >= p.tiles[segment]) tile -= p.tiles[segment++];
+  const uint32_t n = p.n[segment], m0 = blockIdx.y * ROWS;
+  const uint32_t n0 = tile * (DUAL ? COLUMNS / 2 : COLUMNS);
+  // Of a tile column: its row in the matrix, from the tile's first one (columns past n are never stored).  The 32-column
+  // blocks of a pair's tile alternate between gate and up.
+  auto weight_row = [&](uint32_t column) __attribute__((always_inline)) {
+    return min(DUAL ? (column >> 6) * 32 + (column & 31) : column, n - 1 - n0);
+  };
+  auto matrix_of = [&](uint32_t column) __attribute__((always_inline)) { return DUAL ? (column >> 5) & 1 : segment; };
+
+  const uint32_t scale_bytes = scale_lds_bytes(COLUMNS, groups);
+  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)rows_lds;
+  const uint32_t ring = lds_base + scale_bytes;
+  const uint32_t group_blocks = (groups + 7) / 8;
+  for (uint32_t block = wave; block < COLUMNS / 8 * group_blocks; block += WAVES) {
+    const uint32_t column = block / group_blocks * 8;
+    const uint16_t *scales = p.s[matrix_of(column)] + (size_t)n0 * groups;
+    const uint32_t row = weight_row(column + (lane & 7)), group = min(block % group_blocks * 8 + (lane >> 3), groups - 1);
+    copy2_to_lds(scales, (row * groups + group) * 2, lds_base + block * 256);
+  }
+
+  // Copies of a step: lane l fills consecutive 16-byte places; the piece it fetches is the one that the swizzle puts there.
+  const uint8_t *x_base = reinterpret_cast<const uint8_t *>(p.x + (size_t)m0 * p.k);
+  uint32_t x_row[X_COPIES], x_at[X_COPIES];  // bytes
+#pragma unroll
+  for (int c = 0; c < X_COPIES; ++c) {
+    const uint32_t place = (wave * X_COPIES + c) * 64 + lane, row = place / X_PIECES;
+    x_row[c] = min(row, p.m - 1 - m0) * p.k * 2;
+    x_at[c] = (place % X_PIECES ^ (row & 15)) * 16;
+  }
+  auto w_twist = [](uint32_t row) __attribute__((always_inline)) {
+    return W_PIECES >= 16 ? row & 15 : W_PIECES == 8 ? (row >> 1) & 7 : (row >> 2) & 3;
+  };
+  const uint32_t w_place = wave * 64 + lane, w_column = w_place / W_PIECES;
+  const uint8_t *w_base = p.w[matrix_of(wave * 64 / W_PIECES)] + (size_t)n0 * (p.k / 2);
+  const uint32_t w_row = weight_row(w_column) * (p.k / 2), w_at = (w_place % W_PIECES ^ w_twist(w_column)) * 16;
+  auto request = [&](uint32_t step) __attribute__((always_inline)) {
+    const uint32_t stage = ring + step % STAGES * STAGE_BYTES, k0 = step * STEP;
+    const uint8_t *x = x_base + (size_t)k0 * 2, *w = w_base + k0 / 2;
+    if (k0 + STEP <= p.k) {
+      copy16_to_lds(w, w_row + w_at, stage + X_BYTES + wave * 1024);
+#pragma unroll
+      for (int c = 0; c < X_COPIES; ++c) copy16_to_lds(x, x_row[c] + x_at[c], stage + (wave * X_COPIES + c) * 1024);
+    } else {  // the end of the rows: their last pieces again, which nothing multiplies
+      copy16_to_lds(w, w_row + min(w_at, (p.k - k0) / 2 - 16), stage + X_BYTES + wave * 1024);
+#pragma unroll
+      for (int c = 0; c < X_COPIES; ++c)
+        copy16_to_lds(x, x_row[c] + min(x_at[c], (p.k - k0) * 2 - 16), stage + (wave * X_COPIES + c) * 1024);
+    }
+  };
+
+  f16x_t acc[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[r][i] = 0.0f;
+
+  const int column = ct * 32 + (lane & 31), half = lane >> 5;
+  const uint32_t x_read_row = ROWS < 32 ? (lane & (ROWS - 1)) : (lane & 31);
+  const uint32_t w_read = X_BYTES + (column * W_PIECES + ((part * 2 + half) ^ w_twist(column))) * 16;
+  uint32_t x_read[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x_read[j] = (x_read_row * X_PIECES + ((part * 8 + half * 4 + j) ^ (x_read_row & 15))) * 16;
+  const uint32_t *scale_read = reinterpret_cast<const uint32_t *>(rows_lds) + (column >> 3) * group_blocks * 64 + (column & 7);
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < (int)steps) request(s);
+  for (uint32_t s = 0; s < steps; ++s) {
+    // this step has landed once only the copies of the STAGES - 2 steps behind it are under way
+    if (s + STAGES - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"((STAGES - 2) * COPIES) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + STAGES - 1 < steps) request(s + STAGES - 1);  // into the place of the step before, which every wave has read
+    const uint32_t group = s * P + part;
+    if (group >= groups) continue;  // (the same for the whole wave, and its last step)
+    const unsigned char *stage = rows_lds + scale_bytes + s % STAGES * STAGE_BYTES;
+    const u32x4_t packed = *reinterpret_cast<const u32x4_t *>(stage + w_read);
+    h8_t x[RT][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+        x[r][j] = *reinterpret_cast<const h8_t *>(stage + x_read[j] + r * 32 * X_PIECES * 16);
+    const float scale = half_bits_to_float((uint16_t)scale_read[(group >> 3) * 64 + (group & 7) * 8]);
+    f16x_t sum[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum[r][i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const h8_t w = w4_exact_natural(packed[j]);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) sum[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[r][j], w, sum[r], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[r][i] = fmaf(scale, sum[r][i], acc[r][i]);
+  }
+
+  // The waves' sums meet in LDS: [part][row][column], added in the order of the parts.
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+  float *sums = reinterpret_cast<float *>(rows_lds + scale_bytes);
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = r * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
+      if (ROWS >= 32 || row < ROWS) sums[(part * ROWS + row) * COLUMNS + column] = acc[r][i];
+    }
+  __syncthreads();
+  constexpr int OUT = DUAL ? COLUMNS / 2 : COLUMNS, QUADS = ROWS * OUT / 4;
+  uint16_t *y = p.y[segment];
+  const bool whole = (n & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0;
+  for (int q = tid; q < QUADS; q += WAVES * 64) {
+    const uint32_t row = q / (OUT / 4), c = q % (OUT / 4) * 4, at = m0 + row;
+    if (at >= p.m || n0 + c >= n) continue;
+    // of a pair: 32 gate columns, then the 32 up columns of the same outputs
+    const uint32_t from = DUAL ? (c >> 5) * 64 + (c & 31) : c;
+    f4_t value = {0.f, 0.f, 0.f, 0.f}, up = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+      value += *reinterpret_cast<const f4_t *>(sums + (k * ROWS + row) * COLUMNS + from);
+      if (DUAL) up += *reinterpret_cast<const f4_t *>(sums + (k * ROWS + row) * COLUMNS + from + 32);
+    }
+    uint16_t out[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = value[e];
+      if (DUAL) v = v / (1.0f + __expf(-v)) * up[e];
+      if (!DUAL && p.addend != nullptr && n0 + c + e < n)
+        v += half_bits_to_float(p.addend[(size_t)at * p.addend_stride + n0 + c + e]);
+      out[e] = float_to_half_bits(v);
+    }
+    uint16_t *to = y + (size_t)at * n + n0 + c;
+    if (whole) {
+      *reinterpret_cast<ushort4 *>(to) = ushort4{out[0], out[1], out[2], out[3]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n0 + c + e < n) to[e] = out[e];
+    }
+  }
+}
+
+constexpr uint32_t kLdsBytes = 160 * 1024;
+
+template <int ROWS, int CT, int P, int STAGES>
+constexpr uint32_t rows_lds_bytes(uint32_t k) {
+  const uint32_t ring = STAGES * (ROWS * P * 128 + CT * 32 * P * 32), sums = P * ROWS * CT * 32 * 4;
+  return scale_lds_bytes(CT * 32, k / 64) + (ring > sums ? ring : sums);
+}
+
+template <int ROWS, int CT, int P, int STAGES, bool DUAL>
+hipError_t run_rows(RowsParams &p, hipStream_t stream) {
+  const auto kernel = w4a16_rows_kernel<ROWS, CT, P, STAGES, DUAL>;
+  const uint32_t bytes = rows_lds_bytes<ROWS, CT, P, STAGES>(p.k);
+  if (bytes > kLdsBytes) return hipErrorInvalidValue;
+  static bool allowed[kMaxDevices] = {};
+  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), kLdsBytes, allowed)) return status;
+  constexpr uint32_t columns = DUAL ? CT * 16 : CT * 32;
+  uint32_t tiles = 0;
+  for (uint32_t i = 0; i < p.segments; ++i) tiles += p.tiles[i] = (p.n[i] + columns - 1) / columns;
+  kernel<<<dim3(tiles, (p.m + ROWS - 1) / ROWS), CT * P * 64, bytes, stream>>>(p);
+  return hipGetLastError();
+}
+
+// The tile of a launch; kNone: the 128 x 128 and larger tiles of w4a16_gemm.hip.
+enum class Tile { kNone, k32x32, k32x64, k32x64Deep, k32x64Long, k64x64, k64x128 };
+
+// A launch takes as long as one workgroup while each CU has at most one of them, and a workgroup the longer the larger
+// its tile and K are (us, K = 576 / 2048 / 4096 / 8192, one round): 32 x 32 4.1 / 6.1 / 8.8 / 13.7, 32 x 64 4.6 / 7.8 /
+// 11.3 / 21, 64 x 64 5.9 / 10.3 / 16.4 / 29, 64 x 128 7.1 / 14.9 / 25.7 / 47.  So: the smallest tile that needs one round,
+// and the large tiles once even 64 x 128 would need a second.  Measured against those, us (m, K, n):
+// 24 x 4096 x 14336 13.3 / 30.8; 24 x 4096 x 4096 8.7 / 16.7; 64 x 14336 x 4096 23.5 / 38.5; 128 x 4096 x 4096 11.8 / 17.4;
+// 200 x 4096 x 4096 16.9 / 21.4; 512 x 4096 x 4096 28 / 33; 1024 x 2048 x 2048 16.5 / 28.3; 700 x 576 x 576 5.3 / 9.5;
+// 700 x 1536 x 576 7.0 / 13.7; 700 x 576 x 1536 7.4 / 9.5; beyond: 200 x 4096 x 14336 53.6 / 43.5, 700 x 8192 x 2048 47 / 42.
+// With few steps (K < 1536) three workgroups of the shallow 32 x 64 ring share a CU: two rounds of it are still fast.
+Tile pick_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint32_t k) {
+  auto rounds = [&](uint32_t rows, uint32_t columns) {
+    uint64_t tiles = 0;
+    for (uint32_t i = 0; i < matrices; ++i) tiles += (n[i] + columns - 1) / columns;
+    return (double)(tiles * ((m + rows - 1) / rows)) / device_compute_units();
+  };
+  if (rounds(32, 32) <= 1 && rows_lds_bytes<32, 1, 8, 3>(k) <= kLdsBytes) return Tile::k32x32;
+  if (k < 1536) {
+    if (rounds(32, 64) <= 2) return Tile::k32x64;
+  } else if (rounds(32, 64) <= 1) {
+    if (rows_lds_bytes<32, 2, 8, 3>(k) <= kLdsBytes) return Tile::k32x64Deep;
+    if (rows_lds_bytes<32, 2, 4, 4>(k) <= kLdsBytes) return Tile::k32x64Long;
+  }
+  if (k >= 1536 && k <= 6144 && rounds(64, 64) <= 1) return Tile::k64x64;
+  if (k <= 6144 && rounds(64, 128) <= 1.125) return Tile::k64x128;
+  return Tile::kNone;
+}
+
+// The same for a gated pair, by output columns (half of a tile's).  The large tiles take two accumulator sets, so the
+// small ones win for longer: us (m, K, n) 24 x 4096 x 14336 20.4 / 61.7, 64 x 4096 x 4096 12.6 / 58, 64 x 8192 x 2048
+// 26 / 108, 128 x 4096 x 14336 55 / 64 (two rounds), 512 x 2048 x 2048 15.9 / 31.8, 1024 x 2048 x 2048 26.3 / 34.4,
+// 700 x 576 x 1536 10.9 / 16.0; beyond: 200 x 4096 x 14336 105 / 78, 2048 x 2048 x 2048 49 / 46.
+Tile pick_pair_tile(uint32_t m, uint32_t n, uint32_t k) {
+  auto rounds = [&](uint32_t rows, uint32_t columns) {
+    return (double)((uint64_t)((n + columns - 1) / columns) * ((m + rows - 1) / rows)) / device_compute_units();
+  };
+  if (rounds(32, 32) <= 1) {
+    if (k < 1536) return Tile::k32x64;
+    if (rows_lds_bytes<32, 2, 8, 3>(k) <= kLdsBytes) return Tile::k32x64Deep;
+    if (rows_lds_bytes<32, 2, 4, 4>(k) <= kLdsBytes) return Tile::k32x64Long;
+  }
+  if (rounds(64, 32) <= 1 && rows_lds_bytes<64, 2, 4, 3>(k) <= kLdsBytes) return Tile::k64x64;
+  if (rounds(32, 32) <= 2 && k <= 8192) return Tile::k32x64;
+  if (rounds(64, 64) <= 2 && rows_lds_bytes<64, 4, 2, 2>(k) <= kLdsBytes) return Tile::k64x128;
+  return Tile::kNone;
+}
+
+template <bool DUAL>
+hipError_t launch_tile(Tile tile, RowsParams &p, hipStream_t stream) {
+  switch (tile) {
+    case Tile::k32x32:
+      if constexpr (!DUAL) return run_rows<32, 1, 8, 3, false>(p, stream);
+      return hipErrorInvalidValue;
+    case Tile::k32x64: return run_rows<32, 2, 4, 2, DUAL>(p, stream);
+    case Tile::k32x64Deep: return run_rows<32, 2, 8, 3, DUAL>(p, stream);
+    case Tile::k32x64Long: return run_rows<32, 2, 4, 4, DUAL>(p, stream);
+    case Tile::k64x64: return run_rows<64, 2, 4, 3, DUAL>(p, stream);
+    case Tile::k64x128: return run_rows<64, 4, 2, 2, DUAL>(p, stream);
+    case Tile::kNone: break;
+  }
+  return hipErrorInvalidValue;
+}
+
+bool pieces_aligned(const void *x, const void *w) {
+  return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+}
+
+// The copies name a tile's bytes by 32-bit offsets from its first row.
+bool offsets_fit(uint32_t k) { return k <= (1u << 24); }
+
+// Up to about 48k outputs of small matrices the matrix-core GEMV's row groups are as fast or faster (us, m x K x n:
+// 24 x 2048 x 2048 5.4 / 6.1, 40 x 576 x 576 3.8 / 4.1; 100 x 576 x 960 6.1 / 4.2, 40 x 2048 x 2048 6.4 / 6.1).
+constexpr uint64_t kRowGroupOutputs = 49152;
+
+bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k) {
+  if (m <= kGemvMaxRows || !offsets_fit(k)) return false;
+  return !(w4a16_gemv_mfma_row_groups_ok(m, columns, k) && m * columns <= kRowGroupOutputs);
+}
+
+}  // namespace
+
+bool w4a16_rows_ok(const W4LinearArgs &a) {
+  return a.y_f32 == nullptr && rows_wanted(a.m, a.n, a.k) && pieces_aligned(a.x, a.w.weight) &&
+         pick_tile(a.m, &a.n, 1, a.k) != Tile::kNone;
+}
+
+hipError_t launch_w4a16_rows_linear(const W4LinearArgs &a, hipStream_t stream) {
+  RowsParams p = {};
+  p.x = a.x;
+  p.m = a.m;
+  p.k = a.k;
+  p.w[0] = a.w.weight;
+  p.s[0] = a.w.scale;
+  p.y[0] = a.y;
+  p.n[0] = a.n;
+  p.segments = 1;
+  p.addend = a.has_addend ? a.addend : nullptr;
+  p.addend_stride = a.addend_row_stride;
+  return launch_tile<false>(pick_tile(a.m, &a.n, 1, a.k), p, stream);
+}
+
+bool w4a16_rows_ok(const W4QkvArgs &a) {
+  for (int i = 0; i < 3; ++i)
+    if (a.n[i] == 0 || !pieces_aligned(a.x, a.w[i].weight)) return false;
+  return a.norm.weight == nullptr && rows_wanted(a.m, (uint64_t)a.n[0] + a.n[1] + a.n[2], a.k) &&
+         pick_tile(a.m, a.n, 3, a.k) != Tile::kNone;
+}
+
+hipError_t launch_w4a16_rows_qkv(const W4QkvArgs &a, hipStream_t stream) {
+  RowsParams p = {};
+  p.x = a.x;
+  p.m = a.m;
+  p.k = a.k;
+  for (int i = 0; i < 3; ++i) {
+    p.w[i] = a.w[i].weight;
+    p.s[i] = a.w[i].scale;
+    p.y[i] = a.y[i];
+    p.n[i] = a.n[i];
+  }
+  p.segments = 3;
+  return launch_tile<false>(pick_tile(a.m, a.n, 3, a.k), p, stream);
+}
+
+bool w4a16_rows_ok(const W4DualSwigluArgs &a) {
+  return a.norm.weight == nullptr && rows_wanted(a.m, 2ull * a.n, a.k) && pieces_aligned(a.x, a.gate.weight) &&
+         pieces_aligned(a.x, a.up.weight) && pick_pair_tile(a.m, a.n, a.k) != Tile::kNone;
+}
+
+hipError_t launch_w4a16_rows_dual_swiglu(const W4DualSwigluArgs &a, hipStream_t stream) {
+  RowsParams p = {};
+  p.x = a.x;
+  p.m = a.m;
+  p.k = a.k;
+  p.w[0] = a.gate.weight;
+  p.s[0] = a.gate.scale;
+  p.w[1] = a.up.weight;
+  p.s[1] = a.up.scale;
+  p.y[0] = a.product;
+  p.n[0] = a.n;
+  p.segments = 1;
+  return launch_tile<true>(pick_pair_tile(a.m, a.n, a.k), p, stream);
+}
+
+}  // namespace llmopt

@@ -1,0 +1,95 @@
+"""The small tiles of w4a16_rows.hip against float64 products of the oracle's dequantised weights: every tile its rule can
+choose, at sizes that leave remainders of rows, columns and K steps.  The kernel keeps the nibbles exact and sums in
+float32, so its error is the output's rounding: half a unit in the last place, 2^-11 relative at most (the tolerance
+of the other linears, 1e-3, is twice that)."""
+import struct
+
+import numpy as np
+import pytest
+
+import oracle
+from tests.gpu_util import assert_close_to_oracle, linear_grid, u32s, w4_case
+from tests.test_gpu_w4a16 import run_linear
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def runtime():
+    from llmopt_amd.native import Runtime
+    rt = Runtime()
+    yield rt
+    rt.close()
+
+
+def product(x, packed, scale):
+    return x.astype(np.float64) @ oracle.w4_dequant(packed, scale).astype(np.float64).T
+
+
+# 32 x 32: one round of workgroups; 32 x 64 with a short K, with a K that fits its deep ring, with a longer one;
+# 64 x 64; 64 x 128 with long and with short K
+@pytest.mark.parametrize("m,n,k", [
+    (129, 33, 64), (9, 5500, 1088), (70, 1000, 1088), (17, 1000, 14400), (24, 4096, 4096),
+    (300, 1001, 832), (600, 700, 64), (700, 576, 576),
+    (33, 4129, 1536), (33, 4100, 4096), (33, 4129, 4160), (130, 3000, 8256),
+    (200, 2601, 1600), (193, 2600, 6144), (520, 2001, 1536), (1100, 1000, 576)])
+@pytest.mark.parametrize("addend", ["none", "bias", "residual"])
+def test_small_tiles(runtime, m, n, k, addend):
+    rng = np.random.default_rng(m * 7919 + n * 31 + k)
+    x, packed, scale, bias = w4_case(rng, m, n, k, bias=True)
+    expected = product(x, packed, scale)
+    if addend == "none":
+        out = run_linear(runtime, x, packed, scale)
+    elif addend == "bias":
+        out, expected = run_linear(runtime, x, packed, scale, bias=bias), expected + bias.astype(np.float64)
+    else:
+        residual = rng.standard_normal((m, n)).astype(np.float16)
+        out, expected = run_linear(runtime, x, packed, scale, residual=residual), expected + residual.astype(np.float64)
+    assert_close_to_oracle(out, expected, f"linear {m}x{n}x{k} {addend}")
+
+
+def test_exact_integers_and_infinities(runtime):
+    """Whole-number activations and a scale of one give the product itself; an infinity stays in its row."""
+    m, n, k = 129, 257, 320
+    rng = np.random.default_rng(1)
+    x, packed, _, _ = w4_case(rng, m, n, k)
+    x = rng.integers(-4, 5, (m, k)).astype(np.float16)
+    scale = np.ones((n, k // 64), dtype=np.float16)
+    expected = product(x, packed, scale)
+    np.testing.assert_array_equal(run_linear(runtime, x, packed, scale), expected.astype(np.float16))
+    x[5, 319] = np.inf
+    out = run_linear(runtime, x, packed, scale)
+    assert not np.isfinite(out[5]).any()
+    rows = np.arange(m) != 5
+    np.testing.assert_array_equal(out[rows], expected.astype(np.float16)[rows])
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (300, 200, 64), (100, 1537, 576), (300, 1536, 576), (600, 1000, 576), (700, 1536, 576),
+    (70, 1601, 1600), (33, 2000, 4096), (65, 1000, 8256), (24, 2000, 14400), (40, 8192, 1536), (24, 14336, 1600),
+    (500, 1999, 1600)])
+def test_small_pair_tiles(runtime, m, n, k):
+    rng = np.random.default_rng(m * 104729 + n * 13 + k)
+    x, gate, gate_scale, _ = w4_case(rng, m, n, k)
+    _, up, up_scale, _ = w4_case(rng, 1, n, k)
+    out = runtime.buffer_of_bytes(np.full((m, n), np.nan, dtype=np.float16))
+    runtime.dispatch("llmopt_w4a16_dual_swiglu_f16_g64_m4",
+                     [runtime.buffer_of_bytes(a) for a in (x, gate, gate_scale, up, up_scale)] + [out],
+                     u32s(m, n, k) + struct.pack("<f", 1e-5), grid=(linear_grid(((m + 3) // 4) * n), 1, 1), group=(256, 1, 1))
+    g = product(x, gate, gate_scale)
+    assert_close_to_oracle(out.numpy(np.float16, (m, n)), g / (1.0 + np.exp(-g)) * product(x, up, up_scale), f"pair {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("m,k,sizes", [(129, 64, (64, 33, 1)), (700, 576, (576, 192, 192)), (300, 832, (577, 191, 193)),
+                                       (200, 1600, (1024, 256, 257)), (40, 2048, (2048, 512, 512)), (520, 2048, (1024, 512, 500)),
+                                       (1100, 576, (600, 200, 201))])
+def test_small_tiles_over_three_matrices(runtime, m, k, sizes):
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    mats = [w4_case(rng, 1, n, k)[1:3] for n in sizes]
+    outs = [runtime.buffer_of_bytes(np.full((m, n), np.nan, dtype=np.float16)) for n in sizes]
+    runtime.dispatch("llmopt_w4a16_qkv_linear_f16_g64_m4",
+                     [runtime.buffer_of_bytes(x)] + [runtime.buffer_of_bytes(a) for pair in mats for a in pair] + outs,
+                     u32s(m, k, *sizes), grid=(linear_grid(m * sum(sizes)), 1, 1), group=(256, 1, 1))
+    for (packed, scale), out, n in zip(mats, outs, sizes):
+        assert_close_to_oracle(out.numpy(np.float16, (m, n)), product(x, packed, scale), f"three matrices {m}x{n}x{k}")
