@@ -191,6 +191,11 @@ int llmopt_hip_batch_barrier(llmopt_hip_batch *batch);
 int llmopt_hip_commit_batch(llmopt_hip_batch *batch);
 /* caml_llmopt_metal_commit_batch_async (:1359-1370): launches without waiting. */
 int llmopt_hip_commit_batch_async(llmopt_hip_batch *batch);
+/* No reference counterpart: one kernel on device memory that the caller owns, launched on `hip_stream` (which becomes the
+ * context's stream; another one is drained first) and not waited for.  The memory has to stay valid until the work
+ * queued on that stream so far is done.  Several threads may call it for one context. */
+int llmopt_hip_launch(llmopt_hip_library *library, const char *name, void *const *pointers, const size_t *lengths,
+                      uint32_t count, const void *parameters, uint32_t parameter_bytes, void *hip_stream);
 /* Commit for measurement: the counterpart of committing under
  * LLMOPT_PROFILE_BATCH, where the reference reports the command buffer's GPU
  * time (native/ocaml_metal_stubs.m:1337-1347).  Runs the recorded work once

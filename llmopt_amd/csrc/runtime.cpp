@@ -15,6 +15,8 @@
 
 #include <algorithm>
 #include <memory>
+#include <string_view>
+#include <unordered_map>
 
 namespace llmopt {
 
@@ -69,10 +71,14 @@ const std::vector<KernelEntryPoint> &kernel_table() {
 }
 
 const KernelEntryPoint *find_kernel(const char *name) {
+  static const std::unordered_map<std::string_view, const KernelEntryPoint *> by_name = [] {
+    std::unordered_map<std::string_view, const KernelEntryPoint *> found;
+    for (const KernelEntryPoint &entry : kernel_table()) found.emplace(entry.name, &entry);  // the first of a name
+    return found;
+  }();
   if (name == nullptr) return nullptr;
-  for (const KernelEntryPoint &entry : kernel_table())
-    if (strcmp(entry.name, name) == 0) return &entry;
-  return nullptr;
+  const auto entry = by_name.find(name);
+  return entry == by_name.end() ? nullptr : entry->second;
 }
 
 // ---- handler helpers --------------------------------------------------------
@@ -306,6 +312,14 @@ int llmopt_hip_device_name(llmopt_hip_context *context, char *out, size_t capaci
 int llmopt_hip_context_set_stream(llmopt_hip_context *context, void *hip_stream) {
   if (context == nullptr) return fail(LLMOPT_ERR_FAILURE, "HIP context has been finalized");
   if (int status = use_device(context)) return status;
+  if (!context->owns_stream && context->stream == static_cast<hipStream_t>(hip_stream)) {
+    // Nothing changes, and launches stay ordered on the one stream: no reason to wait for it.  (A stream that is being
+    // captured is still turned down below: a recorded launch would keep the address of scratch memory that may move.)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(context->stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone)
+      return LLMOPT_OK;
+    (void)hipGetLastError();
+  }
   LLMOPT_HIP_TRY(hipStreamSynchronize(context->stream), "HIP stream synchronize failed");
   if (context->owns_stream && context->stream) (void)hipStreamDestroy(context->stream);
   context->stream = static_cast<hipStream_t>(hip_stream);
@@ -602,6 +616,32 @@ int llmopt_hip_dispatch(llmopt_hip_library *library, const llmopt_hip_dispatch_i
     status = fail(LLMOPT_ERR_FAILURE, "HIP dispatch failed");
   drop_record(&record);
   return status;
+}
+
+int llmopt_hip_launch(llmopt_hip_library *library, const char *name, void *const *pointers, const size_t *lengths,
+                      uint32_t count, const void *parameters, uint32_t parameter_bytes, void *hip_stream) {
+  if (library == nullptr) return fail(LLMOPT_ERR_FAILURE, "HIP library has been finalized");
+  const KernelEntryPoint *entry = find_kernel(name);
+  if (entry == nullptr) return fail(LLMOPT_ERR_FAILURE, "HIP library does not contain the selected kernel");
+  if ((count > 0 && (pointers == nullptr || lengths == nullptr)) || (parameter_bytes > 0 && parameters == nullptr))
+    return fail(LLMOPT_ERR_INVALID, "HIP launch arguments are missing");
+  try {
+    DispatchRecord record;
+    record.name = entry->name;
+    record.buffers.reserve(count);
+    for (uint32_t i = 0; i < count; ++i) {
+      if (pointers[i] == nullptr || lengths[i] == 0) return fail(LLMOPT_ERR_INVALID, "HIP buffer cannot be empty");
+      record.buffers.push_back({static_cast<uint8_t *>(pointers[i]), lengths[i]});
+    }
+    const uint8_t *bytes = static_cast<const uint8_t *>(parameters);
+    record.parameters.assign(bytes, bytes + parameter_bytes);
+    for (int i = 0; i < 3; ++i) record.grid[i] = record.group[i] = 1;
+    std::lock_guard<std::mutex> lock(library->context->launch_mutex);
+    if (int status = llmopt_hip_context_set_stream(library->context, hip_stream)) return status;
+    return entry->handler(library->context, record);
+  } catch (const std::exception &error) {
+    return fail(LLMOPT_ERR_FAILURE, "HIP launch failed: %s", error.what());
+  }
 }
 
 static int require_active_batch(llmopt_hip_batch *batch) {

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -38,6 +39,7 @@ struct llmopt_hip_context : llmopt::RefCounted {
   int device = 0;
   hipStream_t stream = nullptr;
   bool owns_stream = false;
+  std::mutex launch_mutex;  // llmopt_hip_launch: the stream and the launch on it are one step
   std::string name;
   int compute_units = 256;
   // Scratch for kernels that need device memory beyond inputs and outputs

@@ -96,6 +96,8 @@ def lib() -> ctypes.CDLL:
         "llmopt_hip_sample_f32": (ctypes.c_int, [vp, i64, ctypes.c_double, i64, ctypes.c_double, ctypes.c_double,
                                                  i64, ctypes.POINTER(i64)]),
         "llmopt_hip_dispatch": (ctypes.c_int, [vp, item_p]),
+        "llmopt_hip_launch": (ctypes.c_int, [vp, ctypes.c_char_p, vp, vp, ctypes.c_uint32, ctypes.c_char_p, ctypes.c_uint32,
+                                             vp]),
         "llmopt_hip_begin_batch": (ctypes.c_int, [vp, pp]),
         "llmopt_hip_release_batch": (None, [vp]),
         "llmopt_hip_batch_dispatch": (ctypes.c_int, [vp, vp, item_p]),
@@ -144,7 +146,7 @@ EXPORTED_SYMBOLS = (
     "llmopt_hip_buffer_contents", "llmopt_hip_buffer_length", "llmopt_hip_buffer_device_pointer",
     "llmopt_hip_buffer_copy", "llmopt_hip_buffer_write", "llmopt_hip_buffer_set_int64",
     "llmopt_hip_buffer_set_u32_array", "llmopt_hip_buffer_argmax_f16", "llmopt_hip_f16_argmax",
-    "llmopt_hip_sample_f16", "llmopt_hip_f32_argmax", "llmopt_hip_sample_f32", "llmopt_hip_dispatch",
+    "llmopt_hip_sample_f16", "llmopt_hip_f32_argmax", "llmopt_hip_sample_f32", "llmopt_hip_dispatch", "llmopt_hip_launch",
     "llmopt_hip_begin_batch", "llmopt_hip_release_batch", "llmopt_hip_batch_dispatch",
     "llmopt_hip_batch_dispatch_all", "llmopt_hip_batch_copy", "llmopt_hip_batch_barrier",
     "llmopt_hip_commit_batch", "llmopt_hip_commit_batch_async",
@@ -267,6 +269,11 @@ def attention_q8_paged_no_alloc(parameters: bytes, query: Buffer, current_key: B
         slots.byte_length // 4, output.device_pointer))
 
 
+# ctypes array types of 0 to 16 addresses and sizes (making a type costs more than filling one)
+_POINTERS = [ctypes.c_void_p * n for n in range(17)]
+_LENGTHS = [ctypes.c_size_t * n for n in range(17)]
+
+
 class Runtime:
     """Context + library (the `t` of lib/metal_native.ml:130-135, minus the package)."""
 
@@ -354,6 +361,15 @@ class Runtime:
         _check(lib().llmopt_hip_dispatch(self._library, ctypes.byref(item)))
         del keep
         return name
+
+    def launch(self, name: bytes, pointers: Sequence[int], lengths: Sequence[int], parameters: bytes, stream: int) -> None:
+        """One kernel on device memory of the caller's, queued on `stream` and not waited for: what dispatching it
+        through wrapped buffers and a batch does, as one call."""
+        count = len(pointers)
+        status = lib().llmopt_hip_launch(self._library, name, _POINTERS[count](*pointers), _LENGTHS[count](*lengths), count,
+                                         parameters, len(parameters), stream)
+        if status < 0:
+            _check(status)
 
     def begin_batch(self) -> "Batch":
         return Batch(self)

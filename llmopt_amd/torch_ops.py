@@ -4,9 +4,9 @@ The reference registers
 `w4a16_linear(Tensor input, Tensor packed_weight, Tensor scale, Tensor? bias) -> Tensor`
 in the `llmopt` namespace (python/llmopt_backend/quantization.py:174-185) and
 backs it with its native runtime (native/metal_runtime.cpp:139-147).  This
-module registers the same schema for ROCm tensors: the tensors' device memory
-is wrapped as buffers of the HIP backend (no copies), the kernel is recorded
-on torch's current stream and nothing waits for it.
+module registers the same schema for ROCm tensors: the kernel runs on the
+tensors' own device memory (no copies), is queued on torch's current stream
+and nothing waits for it.
 
     import llmopt_amd.torch_ops            # registers the operator
     y = torch.ops.llmopt.w4a16_linear(x, packed, scale, bias)
@@ -25,12 +25,17 @@ import torch
 from .native import Runtime
 
 GROUP_SIZE = 64
+_ONE_ROW, _ROWS = b"llmopt_w4a16_linear_f16_g64", b"llmopt_w4a16_linear_f16_g64_m4"
+_PARAMETERS = struct.Struct("<5I").pack  # m, n, k, has_bias, bias_row_stride
 _library: Optional[torch.library.Library] = None
 _runtimes: dict[int, Runtime] = {}
 _lock = threading.Lock()
 
 
 def _runtime(device_index: int) -> Runtime:
+    runtime = _runtimes.get(device_index)
+    if runtime is not None:
+        return runtime
     with _lock:
         runtime = _runtimes.get(device_index)
         if runtime is None:
@@ -66,25 +71,19 @@ def _check_arguments(input, packed_weight, scale, bias):
 
 def _w4a16_linear_hip(input, packed_weight, scale, bias=None):
     n, k = _check_arguments(input, packed_weight, scale, bias)
-    x = input.contiguous().view(-1, k)
-    m = x.shape[0]
-    output = torch.empty((m, n), dtype=torch.float16, device=input.device)
+    x, packed_weight, scale = input.contiguous(), packed_weight.contiguous(), scale.contiguous()
+    m = x.numel() // k if k else x.view(-1, k).shape[0]
+    output = torch.empty((*input.shape[:-1], n), dtype=torch.float16, device=input.device)
     if m == 0:
-        return output.view(*input.shape[:-1], n)
-    packed_weight, scale = packed_weight.contiguous(), scale.contiguous()
-    bias = bias.contiguous() if bias is not None else None
+        return output
+    addend = bias.contiguous() if bias is not None else scale
     runtime = _runtime(input.device.index if input.device.index is not None else torch.cuda.current_device())
-    runtime.set_stream(torch.cuda.current_stream(input.device).cuda_stream)
-    wrap = lambda t: runtime.wrap(t.data_ptr(), t.numel() * t.element_size())
-    b_scale = wrap(scale)
-    buffers = [wrap(x), wrap(packed_weight), b_scale, wrap(bias) if bias is not None else b_scale, wrap(output)]
-    name = "llmopt_w4a16_linear_f16_g64" if m == 1 else "llmopt_w4a16_linear_f16_g64_m4"
-    columns = m * n if m == 1 else ((m + 3) // 4) * n
-    batch = runtime.begin_batch()
-    batch.dispatch(name, buffers, struct.pack("<5I", m, n, k, 1 if bias is not None else 0, 0),
-                   grid=(((columns + 7) // 8) * 256, 1, 1), group=(256, 1, 1))
-    batch.commit_async()  # ordered on torch's stream; the tensors above outlive the launch call
-    return output.view(*input.shape[:-1], n)
+    # queued on torch's stream; the tensors above outlive the launch call
+    runtime.launch(_ONE_ROW if m == 1 else _ROWS,
+                   (x.data_ptr(), packed_weight.data_ptr(), scale.data_ptr(), addend.data_ptr(), output.data_ptr()),
+                   (m * k * 2, n * k // 2, scale.numel() * 2, addend.numel() * 2, m * n * 2),
+                   _PARAMETERS(m, n, k, 1 if bias is not None else 0, 0), torch.cuda.current_stream(input.device).cuda_stream)
+    return output
 
 
 def _w4a16_linear_meta(input, packed_weight, scale, bias=None):

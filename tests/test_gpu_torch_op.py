@@ -60,3 +60,37 @@ def test_meta_kernel(op):
              torch.empty((8, 32), dtype=torch.uint8, device="meta"),
              torch.empty((8, 1), dtype=torch.float16, device="meta"), None)
     assert out.shape == (5, 8) and out.dtype == torch.float16
+
+
+def test_calls_in_a_row_on_one_and_on_alternating_streams(op):
+    """Nothing waits between calls on one stream, not even where they share the context's scratch memory (8 rows of K =
+    14336 and 130 of K = 16384 over few columns: K split over workgroups); a stream's calls come after those before."""
+    rng = np.random.default_rng(3)
+    device = torch.device("cuda:0")
+    cases = [w4_case(rng, m, n, k, bias=True) for m, n, k in ((1, 576, 576), (8, 256, 14336), (130, 128, 16384), (24, 1000, 4096))]
+    tensors = [[torch.from_numpy(a).to(device) for a in case] for case in cases]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = []
+    for turn in range(24):
+        with torch.cuda.stream(streams[turn // 8]):
+            outs.append(op(*tensors[turn % 4]))
+        if turn % 8 == 7 and turn // 8 + 1 < len(streams):
+            streams[turn // 8 + 1].wait_stream(streams[turn // 8])
+    for turn in range(6):
+        with torch.cuda.stream(streams[turn % 3]):
+            outs.append(op(*tensors[turn % 4]))
+    torch.cuda.synchronize()
+    for turn, out in enumerate(outs):
+        case = (turn if turn < 24 else turn - 24) % 4
+        assert_close_to_oracle(out.cpu().numpy(), oracle.w4a16_linear(*cases[case]), f"call {turn}")
+
+
+def test_refused_shapes(op):
+    device = torch.device("cuda:0")
+    half = lambda *shape: torch.zeros(shape, dtype=torch.float16, device=device)
+    with pytest.raises(RuntimeError):
+        op(half(3, 0), torch.zeros((8, 0), dtype=torch.uint8, device=device), half(8, 0), None)
+    with pytest.raises(RuntimeError):
+        op(half(3, 64), torch.zeros((0, 32), dtype=torch.uint8, device=device), half(0, 1), None)
+    assert op(half(0, 64), torch.zeros((8, 32), dtype=torch.uint8, device=device), half(8, 1), None).shape == (0, 8)
