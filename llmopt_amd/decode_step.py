@@ -96,12 +96,16 @@ class DecodeConfig:
         return self.kv_layout.bytes_per_token
 
 
+@functools.lru_cache(maxsize=64)
+def _inverse_frequencies(d: int, theta: float) -> np.ndarray:
+    return (theta ** (-np.arange(0, d, 2, dtype=np.float64) / d)).astype(np.float32)
+
+
 def rope_rows(config: DecodeConfig, positions) -> tuple[np.ndarray, np.ndarray]:
     """cos / sin rows for the given positions, duplicated into both halves
     (Serving_rope_table.create, lib/serving_rope_table.ml:156-172): the angle is
     f32(inv_freq * f32(position)), cos/sin in f64 -> f32 -> f16."""
-    d = config.head_dim
-    inv_freq = (config.rope_theta ** (-np.arange(0, d, 2, dtype=np.float64) / d)).astype(np.float32)
+    inv_freq = _inverse_frequencies(config.head_dim, config.rope_theta)
     angle = (inv_freq[None, :] * np.asarray(positions, dtype=np.float32)[:, None]).astype(np.float32)
     cos = np.cos(angle.astype(np.float64)).astype(np.float32).astype(np.float16)
     sin = np.sin(angle.astype(np.float64)).astype(np.float32).astype(np.float16)
@@ -194,14 +198,16 @@ class DecodeStep:
         self.pool, self.slots = pool, slots
         self.tokens = b(np.zeros(batch, dtype=np.int64))
         self.token_ids = b(np.zeros(batch, dtype=np.uint32))
-        self.past_lengths = b(np.asarray(past_lengths, dtype=np.uint32))
         self.slot_offsets = b(np.asarray(slot_offsets, dtype=np.uint32))
-        self.new_slots = b(np.asarray(new_slots, dtype=np.uint32))
-        cos, sin = rope_rows(c, positions)
-        # cosine rows, then sine rows, in one buffer (the fused launch takes them as one)
-        self.trig = b(np.concatenate([cos, sin]))
-        self.cos = self.trig.view(0, cos.nbytes)
-        self.sin = self.trig.view(cos.nbytes, sin.nbytes)
+        # What changes from step to step lies in one buffer, so that `seek` writes it at once: context lengths, slots of the
+        # new tokens, and cosine rows, then sine rows (the fused launch takes those as one buffer).
+        words, trig_bytes = (4 * batch + 255) // 256 * 256, 2 * batch * c.head_dim * 2
+        self.state = runtime.create_buffer(2 * words + trig_bytes)
+        self._state_words = words
+        self.past_lengths, self.new_slots = self.state.view(0, 4 * batch), self.state.view(words, 4 * batch)
+        self.trig = self.state.view(2 * words, trig_bytes)
+        self.cos, self.sin = self.trig.view(0, trig_bytes // 2), self.trig.view(trig_bytes // 2, trig_bytes // 2)
+        self._write_state(np.asarray(past_lengths, dtype=np.uint32), np.asarray(new_slots, dtype=np.uint32), positions)
         self.device = device_weights if device_weights is not None else {
             "embedding": b(weights["embedding"]),
             "final_norm": b(weights["final_norm"]),
@@ -413,13 +419,17 @@ class DecodeStep:
         self.host_positions[:] = positions
         if int(self.host_lengths.max()) > self.max_past:
             raise ValueError("context grew beyond max_context")
-        self.past_lengths.write(self.host_lengths)
-        self.new_slots.write(self.slots_host[self.host_offsets + self.host_lengths])
-        cos, sin = rope_rows(self.config, self.host_positions)
-        self.cos.write(cos)
-        self.sin.write(sin)
+        self._write_state(self.host_lengths, self.slots_host[self.host_offsets + self.host_lengths], self.host_positions)
         if self.reference_entries:
             self.set_reference_past(int(self.host_lengths[0]))
+
+    def _write_state(self, lengths, new_slots, positions) -> None:
+        words, cos_sin = self._state_words, rope_rows(self.config, positions)
+        state = np.zeros(2 * words + cos_sin[0].nbytes * 2, dtype=np.uint8)
+        state[:4 * self.batch] = lengths.view(np.uint8)
+        state[words:words + 4 * self.batch] = np.ascontiguousarray(new_slots).view(np.uint8)
+        state[2 * words:] = np.concatenate(cos_sin).view(np.uint8).reshape(-1)
+        self.state.write(state)
 
     def record(self, batch) -> None:
         for name, buffers, parameters, grid, group in self.dispatches:

@@ -212,12 +212,20 @@ class Buffer:
         return out.raw
 
     def numpy(self, dtype, shape=None) -> np.ndarray:
-        array = np.frombuffer(self.contents(), dtype=dtype).copy()
+        dtype, length = np.dtype(dtype), self.byte_length
+        if length % dtype.itemsize:
+            raise ValueError("buffer size must be a multiple of element size")
+        array = np.empty(length // dtype.itemsize, dtype=dtype)
+        _check(lib().llmopt_hip_buffer_contents(self.handle, array.ctypes.data, length))
         return array if shape is None else array.reshape(shape)
 
     def write(self, data, offset: int = 0) -> None:
-        raw = np.ascontiguousarray(data).tobytes() if not isinstance(data, (bytes, bytearray)) else bytes(data)
-        _check(lib().llmopt_hip_buffer_write(self.handle, offset, raw, len(raw)))
+        if isinstance(data, (bytes, bytearray)):
+            raw = bytes(data)
+            _check(lib().llmopt_hip_buffer_write(self.handle, offset, raw, len(raw)))
+            return
+        array = np.ascontiguousarray(data)
+        _check(lib().llmopt_hip_buffer_write(self.handle, offset, array.ctypes.data, array.nbytes))
 
     def copy_to(self, destination: "Buffer") -> None:
         _check(lib().llmopt_hip_buffer_copy(self.handle, destination.handle))

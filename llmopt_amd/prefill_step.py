@@ -28,12 +28,34 @@ from .decode_step import DecodeConfig, linear_grid, rope_rows, u32s
 from .native import Buffer, Runtime
 
 
+class PrefillWork:
+    """What the steps of prompts of up to `tokens` tokens write and read besides the pool; one step at a time uses it."""
+
+    def __init__(self, runtime: Runtime, config: DecodeConfig, tokens: int):
+        c, create, b = config, runtime.create_buffer, runtime.buffer_of_bytes
+        h, qd, kvd = c.hidden, c.q_heads * c.head_dim, c.kv_heads * c.head_dim
+        self.token_count = tokens
+        self.tokens = b(np.zeros(tokens, dtype=np.int64))
+        self.token_id = b(np.zeros(1, dtype=np.uint32))
+        cos, sin = rope_rows(c, np.arange(tokens))
+        self.cos, self.sin = b(cos), b(sin)
+        self.buffers = {
+            "x": [create(tokens * h * 2), create(tokens * h * 2)],
+            "q": create(tokens * qd * 2), "k": create(tokens * kvd * 2), "v": create(tokens * kvd * 2),
+            "q_rot": create(tokens * qd * 2), "k_rot": create(tokens * kvd * 2),
+            "attention": create(tokens * qd * 2),
+            "product": create(tokens * c.mlp * 2),
+        }
+
+
 class PrefillStep:
     """Device buffers and the dispatch list that prefills `tokens` prompt tokens of one sequence
-    into pool slots `slots[0 .. tokens)` (positions 0 .. tokens - 1)."""
+    into pool slots `slots[0 .. tokens)` (positions 0 .. tokens - 1).  work: buffers to share with other
+    steps (of at least as many tokens), else the step's own."""
 
     def __init__(self, runtime: Runtime, config: DecodeConfig, weights: dict, tokens: int, pool: Buffer,
-                 slots: Buffer, device_weights: dict | None = None, reference_entries: bool = False):
+                 slots: Buffer, device_weights: dict | None = None, reference_entries: bool = False,
+                 work: PrefillWork | None = None):
         if tokens < 2:
             raise ValueError("a prefill has at least two tokens (one token is a decode step)")
         if config.head_dim not in (64, 128, 256, 512):
@@ -43,10 +65,10 @@ class PrefillStep:
         b = runtime.buffer_of_bytes
         c = config
         self.pool, self.slots = pool, slots
-        self.tokens = b(np.zeros(tokens, dtype=np.int64))
-        self.token_id = b(np.zeros(1, dtype=np.uint32))
-        cos, sin = rope_rows(c, np.arange(tokens))
-        self.cos, self.sin = b(cos), b(sin)
+        if work is not None and work.token_count < tokens:
+            raise ValueError(f"shared buffers hold {work.token_count} tokens, the step has {tokens}")
+        work = work or PrefillWork(runtime, config, tokens)
+        self.tokens, self.token_id, self.cos, self.sin = work.tokens, work.token_id, work.cos, work.sin
         self.device = device_weights if device_weights is not None else {
             "embedding": b(weights["embedding"]),
             "final_norm": b(weights["final_norm"]),
@@ -54,15 +76,7 @@ class PrefillStep:
             "layers": [{key: (tuple(b(a) for a in value) if isinstance(value, tuple) else b(value))
                         for key, value in layer.items()} for layer in weights["layers"]],
         }
-        create = runtime.create_buffer
-        h, qd, kvd = c.hidden, c.q_heads * c.head_dim, c.kv_heads * c.head_dim
-        self.work = {
-            "x": [create(tokens * h * 2), create(tokens * h * 2)],
-            "q": create(tokens * qd * 2), "k": create(tokens * kvd * 2), "v": create(tokens * kvd * 2),
-            "q_rot": create(tokens * qd * 2), "k_rot": create(tokens * kvd * 2),
-            "attention": create(tokens * qd * 2),
-            "product": create(tokens * c.mlp * 2),
-        }
+        self.work, h = work.buffers, c.hidden
         # the LM head reads the last token's row of the residual stream
         self.last_row = self.work["x"][0].view((tokens - 1) * h * 2, h * 2)
         self.dispatches = self._build()

@@ -10,13 +10,13 @@ from __future__ import annotations
 
 import dataclasses
 import os
-from typing import Sequence as Tokens
+from typing import Optional, Sequence as Tokens
 
 import numpy as np
 
 from .decode_step import DecodeConfig, DecodeStep, u32s
-from .native import Prebaked, Runtime
-from .prefill_step import PrefillStep
+from .native import DispatchList, Prebaked, Runtime
+from .prefill_step import PrefillStep, PrefillWork
 from .sequence_state import Sequence, StatePool
 from .weight_archive import WeightArchive
 
@@ -46,7 +46,11 @@ class W4a16Model:
         self._slots_host = np.arange(max_context + 1, dtype=np.uint32)
         self._slots = runtime.buffer_of_bytes(self._slots_host)
         self._steps: dict[int, tuple] = {}
-        self._last = runtime.create_buffer(config.vocabulary * 2)
+        self._last = runtime.create_buffer(config.vocabulary * 2)         # of the last decode
+        self._prompt_last = runtime.create_buffer(config.vocabulary * 2)  # of the one place a prompt's step wanted
+        # the buffers of the longest prompt so far, and the lists of prompts over them by slot and token count
+        self._prompt_work: Optional[PrefillWork] = None
+        self._prompts: dict[tuple[int, int], tuple[PrefillStep, DispatchList]] = {}
 
     @staticmethod
     def load(runtime: Runtime, directory: str, config: dict, activations: str = "bfloat16", **options) -> "W4a16Model":
@@ -94,6 +98,20 @@ class W4a16Model:
         sequence.position += 1
         return out
 
+    def _prompt(self, slot: int, tokens: int) -> tuple[PrefillStep, DispatchList]:
+        """The step of a prompt in a slot's pool, and its launches up to the last layer."""
+        if self._prompt_work is None or self._prompt_work.token_count < tokens:
+            self._prompts.clear()
+            self._prompt_work = None  # (given back before the larger buffers are made)
+            self._prompt_work = PrefillWork(self.runtime, self.config, tokens)
+        if (slot, tokens) not in self._prompts:
+            if len(self._prompts) >= 64:
+                self._prompts.clear()
+            step = PrefillStep(self.runtime, self.config, {}, tokens, self._slot_pool(slot), self._slots,
+                               device_weights=self.device, work=self._prompt_work)
+            self._prompts[slot, tokens] = step, DispatchList(step.dispatches[:-1])  # (LM heads go with the wanted places)
+        return self._prompts[slot, tokens]
+
     def logits_row(self) -> np.ndarray:
         return self._last.numpy(np.float16, (self.vocabulary,)).astype(np.float32)
 
@@ -105,12 +123,11 @@ class W4a16Model:
         rows = np.zeros((len(want), self.vocabulary), dtype=np.float32)
         if sequence.position == 0 and len(tokens) > 1:
             c = self.config
-            prefill = PrefillStep(self.runtime, c, {}, len(tokens), self._slot_pool(sequence.slot), self._slots,
-                                  device_weights=self.device)
+            prefill, layers = self._prompt(sequence.slot, len(tokens))
             prefill.tokens.write(np.asarray(tokens, dtype=np.int64))
             batch = self.runtime.begin_batch()
-            prefill.record(batch)
-            logits = [self.runtime.create_buffer(self.vocabulary * 2) for _ in want]
+            batch.dispatch_all(layers)
+            logits = [self._prompt_last if len(want) == 1 else self.runtime.create_buffer(self.vocabulary * 2) for _ in want]
             for place, out in zip(want, logits):
                 batch.dispatch(*self._lm_head(prefill.work["x"][0].view(place * c.hidden * 2, c.hidden * 2), out,
                                               prefill.token_id))

@@ -78,3 +78,28 @@ def test_command_line(folder, capsys):
     assert [int(t) for t in capsys.readouterr().out.split()] == generate_by_steps(runtime, weights, prompt, 4)
     assert cli.main(["models"]) == 0
     assert capsys.readouterr().out.split() == ["Barovik", "Koketar", "W4A16Transformer"]
+
+
+def test_prompts_share_their_buffers(folder):
+    """Prompts of changing lengths in both slots, decoded tokens between them: every prompt's logits and the tokens behind
+    it are, bit for bit, those of a model that has seen nothing else, and a prompt leaves the last decode's logits alone."""
+    path, _ = folder
+    model = model_registry.load_model(str(path), slots=2, max_context=128)
+    rng = np.random.default_rng(6)
+    held = None
+    for n, wants in ((40, 1), (9, 1), (64, 3), (9, 0), (100, 1), (64, 1), (40, 2)):
+        prompt = rng.integers(0, 1000, n).tolist()
+        want = sorted(rng.choice(n, wants, replace=False).tolist())
+        sequence = model.open()
+        before = model.logits_row()
+        logits = model.step(sequence, prompt, want)
+        np.testing.assert_array_equal(model.logits_row(), before)
+        fresh = model_registry.load_model(str(path), slots=1, max_context=128)
+        own = fresh.open()
+        np.testing.assert_array_equal(logits, fresh.step(own, prompt, want))
+        for token in (5, 17):
+            assert model.decode(sequence, token) == fresh.decode(own, token)
+        np.testing.assert_array_equal(model.logits_row(), fresh.logits_row())
+        if held is not None:
+            model.close(held)
+        held = sequence  # the next prompt takes the other slot
