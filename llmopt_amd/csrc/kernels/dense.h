@@ -246,6 +246,11 @@ size_t delta_workspace_bytes(const DeltaArgs &args);
 hipError_t launch_delta_step(const DeltaArgs &args, hipStream_t stream);
 hipError_t launch_delta_prefill(const DeltaArgs &args, hipStream_t stream);
 
+// One token through both mixers side by side (mixer_step.hip); squares: scratch of mixer_step_squares bytes.
+bool mixer_step_ok(const ChunkAttentionArgs &attention, const DeltaArgs &delta);
+size_t mixer_step_squares(const DeltaArgs &delta);
+hipError_t launch_mixer_step(const ChunkAttentionArgs &attention, const DeltaArgs &delta, float *squares, hipStream_t stream);
+
 // ---- routed experts -------------------------------------------------------------------------------------
 
 struct RoutePlan {

@@ -207,11 +207,11 @@ int joint_input(llmopt_hip_context *context, const DispatchRecord &record) {
 // k norm bf16 [dim], frequencies f64 [rotated / 2], step words, key ring, value ring, out (from column 0 on, stride
 // ld_out).  One token: projected and out are float32 rows, q and k stay as they are.
 template <bool F32>
-int rotary_attention(llmopt_hip_context *context, const DispatchRecord &record) {
+int read_rotary_attention(const DispatchRecord &record, ChunkAttentionArgs *out) {
   if (int status = require_buffer_count(record, 8)) return status;
   if (int status = require_parameter_bytes(record, 64)) return status;
   const char *name = record.name.c_str();
-  ChunkAttentionArgs a = {};
+  ChunkAttentionArgs &a = *out = {};
   a.f32 = F32;
   a.m = param_u32(record, 0);
   a.heads = param_u32(record, 4);
@@ -251,14 +251,25 @@ int rotary_attention(llmopt_hip_context *context, const DispatchRecord &record) 
     a.row = as_f32(record.buffers[0]);
     a.out_row = as_f32(record.buffers[7]);
     a.workspace_bytes = chunk_attention_workspace_bytes(a);
+  } else {
+    a.qkv = record.buffers[0].device;
+    a.out = record.buffers[7].device;
+  }
+  return LLMOPT_OK;
+}
+
+template <bool F32>
+int rotary_attention(llmopt_hip_context *context, const DispatchRecord &record) {
+  ChunkAttentionArgs a;
+  if (int status = read_rotary_attention<F32>(record, &a)) return status;
+  const char *name = record.name.c_str();
+  if (a.m == 1) {
     if (a.workspace_bytes) {
       a.workspace = context_workspace(context, a.workspace_bytes);
       if (a.workspace == nullptr) return LLMOPT_ERR_FAILURE;
     }
     return launched(launch_chunk_attention(a, context->stream), name);
   }
-  a.qkv = record.buffers[0].device;
-  a.out = record.buffers[7].device;
   if (int status = launched(launch_rotate_heads(a, context->stream), name)) return status;
   if (int status = launched(launch_chunk_attention(a, context->stream), name)) return status;
   return launched(launch_chunk_cache_write(a, context->stream), name);
@@ -271,11 +282,11 @@ int rotary_attention(llmopt_hip_context *context, const DispatchRecord &record) 
 // [heads * vdim, gate_rank], norm weight [vdim], convolution weights, its ring, state f32 [slots][heads][dim][vdim], step
 // words, out (columns out_first .. of rows of ld_out).  One token: projected and out are float32 rows.
 template <bool F32>
-int gated_delta(llmopt_hip_context *context, const DispatchRecord &record) {
+int read_gated_delta(const DispatchRecord &record, DeltaArgs *out) {
   if (int status = require_buffer_count(record, 12)) return status;
   if (int status = require_parameter_bytes(record, 72)) return status;
   const char *name = record.name.c_str();
-  DeltaArgs a = {};
+  DeltaArgs &a = *out = {};
   a.f32 = F32;
   a.m = param_u32(record, 0);
   a.heads = param_u32(record, 4);
@@ -332,8 +343,19 @@ int gated_delta(llmopt_hip_context *context, const DispatchRecord &record) {
     a.decay_in = row + decay_first;
     a.gate_in = row + gate_first;
     a.out_row = as_f32(record.buffers[11]) + out_first;
-    return launched(launch_delta_step(a, context->stream), name);
   }
+  return LLMOPT_OK;
+}
+
+template <bool F32>
+int gated_delta(llmopt_hip_context *context, const DispatchRecord &record) {
+  DeltaArgs a;
+  if (int status = read_gated_delta<F32>(record, &a)) return status;
+  const char *name = record.name.c_str();
+  if (a.m == 1) return launched(launch_delta_step(a, context->stream), name);
+  const uint32_t first = param_u32(record, 32), decay_first = param_u32(record, 36), gate_first = param_u32(record, 40),
+                 out_first = param_u32(record, 60);
+  const uint64_t element = kElement<F32>, n_decay = (uint64_t)a.heads * a.dim, n_out = (uint64_t)a.heads * a.vdim;
   const uint8_t *projected = reinterpret_cast<const uint8_t *>(record.buffers[0].device);
   Scratch scratch;
   const size_t decay = scratch.want((size_t)a.m * n_decay * 4), gate = scratch.want((size_t)a.m * n_out * element);
@@ -359,6 +381,39 @@ int gated_delta(llmopt_hip_context *context, const DispatchRecord &record) {
   a.out = reinterpret_cast<uint8_t *>(record.buffers[11].device) + out_first * element;
   a.workspace = scratch.at<void>(workspace);
   return launched(launch_delta_prefill(a, context->stream), name);
+}
+
+// One token through llmopt_rotary_attention and llmopt_gated_delta, sharing launches where the sizes allow
+// (mixer_step_ok).  The first's buffers and parameters; then the second's parameters and those of its buffers that are not
+// among the first's (row, step words, out): decay weights, dt bias, log decay rate, gate weights, norm weight, convolution
+// weights, its ring, state.
+template <bool F32>
+int rotary_attention_gated_delta(llmopt_hip_context *context, const DispatchRecord &record) {
+  constexpr size_t kLeftBuffers = 8, kLeftBytes = 64;
+  if (int status = require_buffer_count(record, kLeftBuffers + 8)) return status;
+  if (int status = require_parameter_bytes(record, kLeftBytes + 72)) return status;
+  if (param_u32(record, 0) != 1 || param_u32(record, kLeftBytes) != 1)
+    return fail(LLMOPT_ERR_INVALID, "%s takes one token", record.name.c_str());
+  DispatchRecord left, right;
+  left.name = right.name = record.name;
+  const std::vector<BoundBuffer> &all = record.buffers;
+  left.buffers.assign(all.begin(), all.begin() + kLeftBuffers);
+  right.buffers = {all[0], all[0], all[8], all[9], all[10], all[11], all[12], all[13], all[14], all[15], all[4], all[7]};
+  left.parameters.assign(record.parameters.begin(), record.parameters.begin() + kLeftBytes);
+  right.parameters.assign(record.parameters.begin() + kLeftBytes, record.parameters.end());
+  ChunkAttentionArgs a;
+  DeltaArgs d;
+  if (int status = read_rotary_attention<F32>(left, &a)) return status;
+  if (int status = read_gated_delta<F32>(right, &d)) return status;
+  if (!mixer_step_ok(a, d)) {
+    if (int status = rotary_attention<F32>(context, left)) return status;
+    return gated_delta<F32>(context, right);
+  }
+  Scratch scratch;
+  const size_t partial = scratch.want(a.workspace_bytes), squares = scratch.want(mixer_step_squares(d));
+  if (!scratch.get(context)) return LLMOPT_ERR_FAILURE;
+  a.workspace = scratch.at<void>(partial);
+  return launched(launch_mixer_step(a, d, scratch.at<float>(squares), context->stream), record.name.c_str());
 }
 
 // {u32 m, n, k}; x [m, k] (one token: f32), weight [n, k], out f32 [m, n] = x w^T.
@@ -458,6 +513,8 @@ void register_parallel_kernels(std::vector<KernelEntryPoint> &table) {
   table.push_back({"llmopt_rotary_attention_f32", "attention", rotary_attention<true>});
   table.push_back({"llmopt_gated_delta_bf16", "triangular-recurrence", gated_delta<false>});
   table.push_back({"llmopt_gated_delta_f32", "triangular-recurrence", gated_delta<true>});
+  table.push_back({"llmopt_rotary_attention_gated_delta_bf16", "attention", rotary_attention_gated_delta<false>});
+  table.push_back({"llmopt_rotary_attention_gated_delta_f32", "attention", rotary_attention_gated_delta<true>});
   table.push_back({"llmopt_linear_store_bf16", "linear", linear_store<false>});
   table.push_back({"llmopt_linear_store_f32", "linear", linear_store<true>});
   table.push_back({"llmopt_pending_gated_ffn_bf16", "gated-linear", pending_gated_ffn<false>});

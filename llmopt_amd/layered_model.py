@@ -473,17 +473,21 @@ class LayeredModel:
                 u32s(m, c.width, columns.total, columns.split, columns.conv, right.channels, right.taps, slots) + pending,
                 *grid)]
         stream.joined()
-        out.append(("llmopt_rotary_attention" + s,
-                    [work.projected, d["q_norm"], d["k_norm"], d["frequencies"], work.step, keys, values, work.mixed],
-                    u32s(m, left.heads, left.kv_heads, left.dim, left.vdim, columns.split, mixer.out, ring.capacity,
-                         ring.span, 1, slots, left.rotation.dims) + struct.pack("<ff", left.scale, left.softcap) + eps +
-                    struct.pack("<f", mixer.left_scale), *grid))
-        out.append(("llmopt_gated_delta" + s,
-                    [work.projected, work.extra, d["decay"], d["dt_bias"], d["A_log"], d["gate"], d["norm"], d["conv"],
-                     conv_ring, state, work.step, work.mixed],
-                    u32s(m, right.heads, right.kv_heads, right.dim, right.vdim, right.taps, slots, columns.split, columns.conv,
-                         columns.decay, columns.gate, columns.split, *d["ranks"], mixer.out, left.out) + eps +
-                    struct.pack("<f", mixer.right_scale), *grid))
+        attention = ([work.projected, d["q_norm"], d["k_norm"], d["frequencies"], work.step, keys, values, work.mixed],
+                     u32s(m, left.heads, left.kv_heads, left.dim, left.vdim, columns.split, mixer.out, ring.capacity,
+                          ring.span, 1, slots, left.rotation.dims) + struct.pack("<ff", left.scale, left.softcap) + eps +
+                     struct.pack("<f", mixer.left_scale))
+        delta = ([work.projected, work.extra, d["decay"], d["dt_bias"], d["A_log"], d["gate"], d["norm"], d["conv"],
+                  conv_ring, state, work.step, work.mixed],
+                 u32s(m, right.heads, right.kv_heads, right.dim, right.vdim, right.taps, slots, columns.split, columns.conv,
+                      columns.decay, columns.gate, columns.split, *d["ranks"], mixer.out, left.out) + eps +
+                 struct.pack("<f", mixer.right_scale))
+        if m == 1:  # both mixers of a token share their launches
+            out.append(("llmopt_rotary_attention_gated_delta" + s, attention[0] + delta[0][2:10],
+                        attention[1] + delta[1], *grid))
+        else:
+            out.append(("llmopt_rotary_attention" + s, *attention, *grid))
+            out.append(("llmopt_gated_delta" + s, *delta, *grid))
         out.append(("llmopt_linear_store" + s, [work.mixed, d["o"], work.output], u32s(m, c.width, mixer.out), *grid))
         stream.pending = d["norm1"]
         if layer.ffn is not None:
