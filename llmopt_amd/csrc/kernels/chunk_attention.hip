@@ -8,9 +8,11 @@
 // Keys and values live in a ring per sequence slot and head: position p in row p % capacity, capacity >=
 // chunk or window, so that a ring of one holds everything later tokens can see.
 //
-//  * chunk_prefill_kernel: a portion of a prompt.  Four waves walk the keys of 64 * QT query rows of one
-//    head, 64 keys a stage through LDS; keys before the portion come from the ring, the others from the
-//    portion's own rows.  S^T = K Q^T leaves every lane four consecutive keys of one query row, which is
+//  * chunk_prefill_kernel: a portion of a prompt.  Waves of 16 query rows of one head each walk its keys,
+//    64 keys a stage through LDS; keys before the portion come from the ring, the others from the
+//    portion's own rows.  Bound by the latency of a stage (products, softmax, products in turn): eight waves a
+//    workgroup and four a SIMD, where a wave of twice the rows left two, took 16 heads of 128 over 3001 rows from
+//    138 us to 119; matrix units are then busy for 30% of the time, and a second stage in LDS gives nothing.  S^T = K Q^T leaves every lane four consecutive keys of one query row, which is
 //    the B operand of O^T += V^T P^T up to a permutation of the contraction index that the V^T operand
 //    follows: probabilities never leave their lane (bf16: as a high and a low part, so that the weights keep
 //    float32 accuracy in the product).  Caps of at most kFixedMaxCap bound the exponent, so
@@ -33,30 +35,44 @@ namespace {
 constexpr int kStageKeys = 64;
 constexpr float kFixedMaxCap = 40.0f;
 
-template <typename T, int ND, int NE>
+constexpr int kCompute = 256;  // compute units
+
+// The stage, and where KS == 2 the second half's sums in its place.
+template <typename T, int ND, int NE, int WAVES, int KS>
 constexpr int prefill_lds_bytes() {
-  return kStageKeys * (ND * 32 + 16 / (int)sizeof(T) + value_stride<T, NE>()) * (int)sizeof(T);
+  const int stage = kStageKeys * (ND * 32 + 16 / (int)sizeof(T) + value_stride<T, NE>()) * (int)sizeof(T);
+  const int sums = KS == 2 ? WAVES / 2 * 64 * (NE * 4 + 2) * 4 : 0;
+  return stage > sums ? stage : sums;
 }
 
-template <typename T, int ND, int NE, int QT, bool FIXED>
-__global__ __launch_bounds__(256, ND * 2 + NE <= 16 || sizeof(T) == 2 ? 2 : 1) void chunk_prefill_kernel(ChunkAttentionArgs a) {
+// Eight waves keep to the registers that let a compute unit hold two workgroups.
+template <typename T, int ND, int NE, int WAVES, int KS, bool FIXED>
+__global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : ND * 2 + NE <= 16 || sizeof(T) == 2 ? 2 : 1) void
+chunk_prefill_kernel(ChunkAttentionArgs a) {
   constexpr int DP = ND * 32, EP = NE * 16;
+  constexpr int ROW_WAVES = WAVES / KS, ROWS = ROW_WAVES * 16, KEYS = kStageKeys / KS, KT = KEYS / 16;
   constexpr int SK = DP + 16 / (int)sizeof(T), SV = value_stride<T, NE>();
-  constexpr int K_LOADS = kStageKeys * DP / 8 / 256, V_PIECES = EP / 8;
-  constexpr int V_LOADS = (kStageKeys * V_PIECES + 255) / 256;
+  constexpr int K_LOADS = kStageKeys * DP / 8 / (WAVES * 64), V_PIECES = EP / 8;
+  constexpr int V_LOADS = (kStageKeys * V_PIECES + WAVES * 64 - 1) / (WAVES * 64);
   extern __shared__ __attribute__((aligned(16))) char lds[];
   T *lds_k = reinterpret_cast<T *>(lds);
   T *lds_v = lds_k + kStageKeys * SK;
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, column = lane & 15, quad = lane >> 4;
-  // heads of one key / value head follow each other kv_heads apart, so that they share an XCD's L2 when
-  // kv_heads is a multiple of the eight XCDs; the longest rows of all heads come first
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int column = lane & 15, quad = lane >> 4, row_wave = wave % ROW_WAVES, first_key = wave / ROW_WAVES * KEYS;
+  // Heads of one key / value head follow each other kv_heads apart, so that they share an XCD's L2 when
+  // kv_heads is a multiple of the eight XCDs.  Late rows see more keys: tiles are dealt in rounds of one
+  // workgroup a compute unit, the longest round first, and in turn from short to long and from long to short, so
+  // that the second workgroup of a compute unit is short where its first one is long (16 heads of 3001 rows: 119 us
+  // with the longest first, 112 so).
   const uint32_t per = a.heads / a.kv_heads, group = blockIdx.x % a.kv_heads;
   const uint32_t head = group * per + blockIdx.x / a.kv_heads;
-  const uint32_t tile = gridDim.y - 1 - blockIdx.y;
+  const uint32_t around = max(kCompute / a.heads, 1u), round = blockIdx.y / around, step = blockIdx.y % around;
+  const uint32_t left = gridDim.y - round * around;  // tiles of this round and later ones
+  const uint32_t tile = gridDim.y <= around || (round & 1) ? left - 1 - step : left - min(left, around) + step;
   const uint32_t p0 = a.state[kStatePosition], slot = a.state[kStateSlot];
-  const uint32_t row_first = tile * 64 * QT;
-  const uint32_t row_end = min(row_first + 64 * QT, a.m);
+  const uint32_t row_first = tile * ROWS;
+  const uint32_t row_end = min(row_first + ROWS, a.m);
   const uint32_t ld = a.ld;
   const T *qkv = static_cast<const T *>(a.qkv);
   const T *fresh_k = qkv + a.heads * a.dim + group * a.dim;
@@ -67,21 +83,16 @@ __global__ __launch_bounds__(256, ND * 2 + NE <= 16 || sizeof(T) == 2 ? 2 : 1) v
   const bool vec = a.dim % 8 == 0 && a.vdim % 8 == 0 && ld % 8 == 0;
 
   // queries of this wave: operand columns
-  Frag<T> fq[QT][ND];
-  uint32_t low[QT], query[QT];  // visible positions of the lane's row: low .. query
+  Frag<T> fq[ND];
+  const uint32_t row = row_first + row_wave * 16 + column, own = min(row, a.m - 1);
+  const uint32_t query = p0 + own, low = first_seen(query, a.cache);  // visible positions of the lane's row: low .. query
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    const uint32_t r = min(row_first + (wave * QT + t) * 16 + column, a.m - 1);
-    query[t] = p0 + r;
-    low[t] = first_seen(query[t], a.cache);
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      const int k = d * 32 + quad * 8;
-      fq[t][d] = load_piece(qkv + (size_t)r * ld + head * a.dim + k, (int)a.dim - k, vec);
-    }
+  for (int d = 0; d < ND; ++d) {
+    const int k = d * 32 + quad * 8;
+    fq[d] = load_piece(qkv + (size_t)own * ld + head * a.dim + k, (int)a.dim - k, vec);
   }
-  const uint32_t wave_first = p0 + min(row_first + wave * QT * 16, a.m - 1);
-  const uint32_t wave_last = p0 + min(row_first + (wave + 1) * QT * 16 - 1, a.m - 1);
+  const uint32_t wave_first = p0 + min(row_first + row_wave * 16, a.m - 1);
+  const uint32_t wave_last = p0 + min(row_first + (row_wave + 1) * 16 - 1, a.m - 1);
   const uint32_t wave_low = first_seen(wave_first, a.cache);
   const uint32_t wave_low_last = first_seen(wave_last, a.cache);
 
@@ -91,17 +102,11 @@ __global__ __launch_bounds__(256, ND * 2 + NE <= 16 || sizeof(T) == 2 ? 2 : 1) v
   const float sink = has_sink ? (float)reinterpret_cast<const __bf16 *>(a.sink)[head] * kLog2e : 0.0f;
   const float cap = a.softcap * kLog2e;
   const float inner = capped ? 2.0f * a.scale / a.softcap * kLog2e : a.scale * kLog2e;
-  float top[QT], total[QT];
+  float top = FIXED ? fmaxf(sink, 0.0f) : first_key == 0 && has_sink ? sink : -1e30f;
+  float total = has_sink && first_key == 0 && quad == 0 ? exp2_raw(sink - top) : 0.0f;
+  f32x4 out[NE];
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    top[t] = has_sink ? (FIXED ? fmaxf(sink, 0.0f) : sink) : (FIXED ? 0.0f : -1e30f);
-    total[t] = has_sink && quad == 0 ? exp2_raw(sink - top[t]) : 0.0f;
-  }
-  f32x4 out[NE][QT];
-#pragma unroll
-  for (int e = 0; e < NE; ++e)
-#pragma unroll
-    for (int t = 0; t < QT; ++t) out[e][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int e = 0; e < NE; ++e) out[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   const uint32_t last = p0 + row_end - 1;
   const uint32_t key_begin = first_seen(p0 + row_first, a.cache);
@@ -111,14 +116,14 @@ __global__ __launch_bounds__(256, ND * 2 + NE <= 16 || sizeof(T) == 2 ? 2 : 1) v
   auto fetch = [&](uint32_t base) {
 #pragma unroll
     for (int i = 0; i < K_LOADS; ++i) {
-      const int index = i * 256 + tid, row = index / (DP / 8), piece = (index % (DP / 8)) * 8;
+      const int index = i * WAVES * 64 + tid, row = index / (DP / 8), piece = (index % (DP / 8)) * 8;
       const uint32_t j = min(base + row, last);
       const T *source = j < p0 ? cache_k + (size_t)(j % a.cache.capacity) * a.dim : fresh_k + (size_t)(j - p0) * ld;
       reg_k[i] = load_piece(source + piece, (int)a.dim - piece, vec);
     }
 #pragma unroll
     for (int i = 0; i < V_LOADS; ++i) {
-      const int index = i * 256 + tid, row = min(index / V_PIECES, kStageKeys - 1), piece = (index % V_PIECES) * 8;
+      const int index = i * WAVES * 64 + tid, row = min(index / V_PIECES, kStageKeys - 1), piece = (index % V_PIECES) * 8;
       const uint32_t j = min(base + row, last);
       const T *source = j < p0 ? cache_v + (size_t)(j % a.cache.capacity) * a.vdim : fresh_v + (size_t)(j - p0) * ld;
       reg_v[i] = load_piece(source + piece, (int)a.vdim - piece, vec);
@@ -127,14 +132,102 @@ __global__ __launch_bounds__(256, ND * 2 + NE <= 16 || sizeof(T) == 2 ? 2 : 1) v
   auto stash = [&] {
 #pragma unroll
     for (int i = 0; i < K_LOADS; ++i) {
-      const int index = i * 256 + tid;
+      const int index = i * WAVES * 64 + tid;
       *reinterpret_cast<Frag<T> *>(lds_k + index / (DP / 8) * SK + (index % (DP / 8)) * 8) = reg_k[i];
     }
 #pragma unroll
     for (int i = 0; i < V_LOADS; ++i) {
-      const int index = i * 256 + tid;
+      const int index = i * WAVES * 64 + tid;
       if (index < kStageKeys * V_PIECES)
         *reinterpret_cast<Frag<T> *>(lds_v + index / V_PIECES * SV + (index % V_PIECES) * 8) = reg_v[i];
+    }
+  };
+
+  auto multiply = [&](uint32_t base) {  // base: the first of this wave's keys in the stage
+    f32x4 score[KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) score[kt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+        const Frag<T> fk = *reinterpret_cast<const Frag<T> *>(lds_k + (first_key + kt * 16 + column) * SK + d * 32 + quad * 8);
+        score[kt] = mma(fk, fq[d], score[kt]);
+      }
+      if (KS == 1) __builtin_amdgcn_sched_barrier(0);  // four operands at a time: registers
+    }
+    // Only a stage with a border pays for the mask: behind its own branch, which all of a wave takes alike (with a
+    // test beside each score 16 heads of 3001 rows took 114 us for 96).
+    const bool whole = base >= wave_low_last && base + KEYS - 1 <= wave_first;
+    auto mask = [&](float hidden) {
+      const uint32_t from = low - base - quad * 4, count = query - low;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) score[kt][r] = kt * 16 + r - from <= count ? score[kt][r] : hidden;
+    };
+    if (FIXED) {
+      const float high = cap - top;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float tail = __builtin_amdgcn_rcpf(1.0f + exp2_raw(score[kt][r] * inner));
+          score[kt][r] = exp2_raw(fmaf(-2.0f * cap, tail, high));
+        }
+      if (!whole) mask(0.0f);
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) total += score[kt][r];
+    } else {
+      if (capped) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            score[kt][r] = fmaf(-2.0f * cap, __builtin_amdgcn_rcpf(1.0f + exp2_raw(score[kt][r] * inner)), cap);
+      } else {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) score[kt] *= inner;
+      }
+      if (!whole) mask(-INFINITY);
+      float best = top;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) best = fmaxf(best, score[kt][r]);
+      best = fmaxf(best, __shfl_xor(best, 16, 64));
+      best = fmaxf(best, __shfl_xor(best, 32, 64));
+      const float alpha = exp2_raw(top - best);
+      top = best;
+      total *= alpha;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) out[e] *= alpha;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          score[kt][r] = exp2_raw(score[kt][r] - best);
+          total += score[kt][r];
+        }
+    }
+#pragma unroll
+    for (int ks = 0; ks < KT / 2; ++ks) {
+      WideFrag<T> fp;  // the weights keep float32 accuracy
+#pragma unroll
+      for (int r = 0; r < 4; r += 2) {
+        fp.set_pair(r, score[2 * ks][r], score[2 * ks][r + 1]);
+        fp.set_pair(4 + r, score[2 * ks + 1][r], score[2 * ks + 1][r + 1]);
+      }
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const T *keys = lds_v + (first_key + ks * 32 + quad * 4) * SV + e * 16;
+        const auto first = four_keys(keys, SV, lane), second = four_keys(keys + 16 * SV, SV, lane);
+        const Frag<T> fv = __builtin_shufflevector(first, second, 0, 1, 2, 3, 4, 5, 6, 7);
+        out[e] = mma_wide_b(fv, fp, out[e]);
+        if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
     }
   };
 
@@ -144,126 +237,51 @@ __global__ __launch_bounds__(256, ND * 2 + NE <= 16 || sizeof(T) == 2 ? 2 : 1) v
     stash();
     __syncthreads();
     if (base + kStageKeys <= last) fetch(base + kStageKeys);
-    if (base > wave_last || base + kStageKeys <= wave_low) continue;
-
-    f32x4 score[4][QT];
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-#pragma unroll
-      for (int t = 0; t < QT; ++t) score[kt][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int d = 0; d < ND; ++d) {
-        const Frag<T> fk = *reinterpret_cast<const Frag<T> *>(lds_k + (kt * 16 + column) * SK + d * 32 + quad * 8);
-#pragma unroll
-        for (int t = 0; t < QT; ++t) score[kt][t] = mma(fk, fq[t][d], score[kt][t]);
-      }
-      __builtin_amdgcn_sched_barrier(0);  // operands of one key tile at a time: registers
-    }
-    const bool whole = base >= wave_low_last && base + kStageKeys - 1 <= wave_first;  // no border in this stage
-    auto seen = [&](int t, int kt, int r) {
-      const uint32_t j = base + kt * 16 + quad * 4 + r;
-      return j >= low[t] && j <= query[t];
-    };
-    if (FIXED) {
-#pragma unroll
-      for (int t = 0; t < QT; ++t) {
-        const float high = cap - top[t];
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float tail = __builtin_amdgcn_rcpf(1.0f + exp2_raw(score[kt][t][r] * inner));
-            score[kt][t][r] = exp2_raw(fmaf(-2.0f * cap, tail, high));
-          }
-        if (!whole) {
-#pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (!seen(t, kt, r)) score[kt][t][r] = 0.0f;
-        }
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) total[t] += score[kt][t][r];
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < QT; ++t) {
-        float best = top[t];
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float s = score[kt][t][r] * inner;
-            if (capped) s = fmaf(-2.0f * cap, __builtin_amdgcn_rcpf(1.0f + exp2_raw(s)), cap);
-            if (!whole && !seen(t, kt, r)) s = -INFINITY;
-            score[kt][t][r] = s;
-            best = fmaxf(best, s);
-          }
-        best = fmaxf(best, __shfl_xor(best, 16, 64));
-        best = fmaxf(best, __shfl_xor(best, 32, 64));
-        const float alpha = exp2_raw(top[t] - best);
-        top[t] = best;
-        total[t] *= alpha;
-#pragma unroll
-        for (int e = 0; e < NE; ++e)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) out[e][t][r] *= alpha;
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            score[kt][t][r] = exp2_raw(score[kt][t][r] - best);
-            total[t] += score[kt][t][r];
-          }
-      }
-    }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      WideFrag<T> fp[QT];  // the weights keep float32 accuracy
-#pragma unroll
-      for (int t = 0; t < QT; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          fp[t].set(r, score[2 * ks][t][r]);
-          fp[t].set(4 + r, score[2 * ks + 1][t][r]);
-        }
-#pragma unroll
-      for (int e = 0; e < NE; ++e) {
-        const T *keys = lds_v + (ks * 32 + quad * 4) * SV + e * 16;
-        const auto first = four_keys(keys, SV, lane), second = four_keys(keys + 16 * SV, SV, lane);
-        const Frag<T> fv = __builtin_shufflevector(first, second, 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-        for (int t = 0; t < QT; ++t) out[e][t] = mma_wide_b(fv, fp[t], out[e][t]);
-        if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-      }
-    }
+    const uint32_t begin = base + first_key;
+    if (begin <= wave_last && begin + KEYS > wave_low) multiply(begin);
   }
 
+  if constexpr (KS == 2) {  // the second half's sums join the first's through the stage's LDS
+    constexpr int WORDS = NE * 4 + 2;
+    float *other = reinterpret_cast<float *>(lds) + row_wave * 64 * WORDS + lane;
+    __syncthreads();
+    if (first_key) {
 #pragma unroll
-  for (int t = 0; t < QT; ++t) {
-    float sum = total[t];
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
-    const float inverse = a.out_scale / sum;
-    const uint32_t r = row_first + (wave * QT + t) * 16 + column;
-    if (r >= a.m) continue;
-    T *target = static_cast<T *>(a.out) + (size_t)r * a.ld_out + head * a.vdim;
+      for (int e = 0; e < NE; ++e)
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      const uint32_t c = e * 16 + quad * 4;
-      typedef T x4 __attribute__((ext_vector_type(4)));
-      if (vec && a.ld_out % 4 == 0 && c < a.vdim) {
-        x4 packed;
+        for (int r = 0; r < 4; ++r) other[(e * 4 + r) * 64] = out[e][r];
+      other[NE * 4 * 64] = top;
+      other[(NE * 4 + 1) * 64] = total;
+    }
+    __syncthreads();
+    if (first_key) return;
+    const float its_top = other[NE * 4 * 64], best = fmaxf(top, its_top);
+    const float mine = exp2_raw(top - best), its = exp2_raw(its_top - best);
+    total = total * mine + other[(NE * 4 + 1) * 64] * its;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) packed[i] = (T)(out[e][t][i] * inverse);
-        *reinterpret_cast<x4 *>(target + c) = packed;
-      } else {
+    for (int e = 0; e < NE; ++e)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (c + i < a.vdim) target[c + i] = (T)(out[e][t][i] * inverse);
-      }
+      for (int r = 0; r < 4; ++r) out[e][r] = out[e][r] * mine + other[(e * 4 + r) * 64] * its;
+  }
+  float sum = total;
+  sum += __shfl_xor(sum, 16, 64);
+  sum += __shfl_xor(sum, 32, 64);
+  const float inverse = a.out_scale / sum;
+  if (row >= a.m) return;
+  T *target = static_cast<T *>(a.out) + (size_t)row * a.ld_out + head * a.vdim;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const uint32_t c = e * 16 + quad * 4;
+    typedef T x4 __attribute__((ext_vector_type(4)));
+    if (vec && a.ld_out % 4 == 0 && c < a.vdim) {
+      x4 packed;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) packed[i] = (T)(out[e][i] * inverse);
+      *reinterpret_cast<x4 *>(target + c) = packed;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (c + i < a.vdim) target[c + i] = (T)(out[e][i] * inverse);
     }
   }
 }
@@ -342,24 +360,39 @@ hipError_t run_decode(const ChunkAttentionArgs &a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <typename T, int ND, int NE, bool FIXED>
+template <typename T, int ND, int NE, int WAVES, int KS, bool FIXED>
 hipError_t run_prefill_kernel(const ChunkAttentionArgs &a, hipStream_t stream) {
-  constexpr int QT = sizeof(T) == 2 && ND <= 4 && NE <= 8 ? 2 : 1;
-  constexpr int bytes = prefill_lds_bytes<T, ND, NE>();
+  constexpr int bytes = prefill_lds_bytes<T, ND, NE, WAVES, KS>(), rows = WAVES / KS * 16;
   static bool allowed[kMaxDevices] = {};
+  const auto kernel = chunk_prefill_kernel<T, ND, NE, WAVES, KS, FIXED>;
   if (bytes > 64 * 1024)
-    if (hipError_t status = allow_dynamic_lds(
-            reinterpret_cast<const void *>(chunk_prefill_kernel<T, ND, NE, QT, FIXED>), bytes, allowed))
-      return status;
-  const dim3 grid(a.heads, (a.m + 64 * QT - 1) / (64 * QT));
-  chunk_prefill_kernel<T, ND, NE, QT, FIXED><<<grid, 256, bytes, stream>>>(a);
+    if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
+  kernel<<<dim3(a.heads, (a.m + rows - 1) / rows), WAVES * 64, bytes, stream>>>(a);
   return hipGetLastError();
 }
 
+template <typename T, int ND, int NE, int WAVES, int KS>
+hipError_t run_prefill_tile(const ChunkAttentionArgs &a, hipStream_t stream) {
+  if (a.softcap > 0.0f && a.softcap <= kFixedMaxCap) return run_prefill_kernel<T, ND, NE, WAVES, KS, true>(a, stream);
+  return run_prefill_kernel<T, ND, NE, WAVES, KS, false>(a, stream);
+}
+
+// A wave's registers hold 16 query rows of heads up to 128 twice a SIMD beside a second workgroup (bfloat16); wider
+// heads and float32 leave room for four waves.  Eight waves are 128 rows, or 64 rows of which each half of the waves
+// takes half the keys of a stage: twice the workgroups, half the chain.  That is the better one while 128-row tiles
+// leave compute units with one workgroup or none (700 rows: 16 heads of 128 21.9 us for 28.4, 32 heads 21.9 for
+// 30.0; 2048 rows, 16 heads of 64 38.9 for 56.5) and for heads up to 64 always, whose stages are short and whose
+// keys are cheap to bring in twice (3001 rows, 16 heads of 64: the same 53 us either way).  Beyond that it brings
+// in twice the keys for nothing (3001 rows, 16 heads of 128: 102.7 us for 92.3; 2048 rows, 32 heads: 97.9 for 89.1).
 template <typename T, int ND, int NE>
 hipError_t run_prefill(const ChunkAttentionArgs &a, hipStream_t stream) {
-  if (a.softcap > 0.0f && a.softcap <= kFixedMaxCap) return run_prefill_kernel<T, ND, NE, true>(a, stream);
-  return run_prefill_kernel<T, ND, NE, false>(a, stream);
+  if constexpr (sizeof(T) == 2 && ND <= 4 && NE <= 8) {
+    if constexpr (ND > 2 || NE > 4)
+      if ((uint64_t)a.heads * ((a.m + 127) / 128) > kCompute) return run_prefill_tile<T, ND, NE, 8, 1>(a, stream);
+    return run_prefill_tile<T, ND, NE, 8, 2>(a, stream);
+  } else {
+    return run_prefill_tile<T, ND, NE, 4, 1>(a, stream);
+  }
 }
 
 template <typename T, int ND, int NE>

@@ -60,6 +60,7 @@ template <>
 struct WideFrag<float> {
   f32x8 v;
   __device__ __forceinline__ void set(int i, float x) { v[i] = x; }
+  __device__ __forceinline__ void set_pair(int i, float x, float y) { v[i] = x, v[i + 1] = y; }
 };
 template <>
 struct WideFrag<__bf16> {
@@ -67,6 +68,15 @@ struct WideFrag<__bf16> {
   __device__ __forceinline__ void set(int i, float x) {
     hi[i] = (__bf16)x;
     lo[i] = (__bf16)(x - (float)hi[i]);
+  }
+  // the elements of one register (i even): one conversion for both
+  __device__ __forceinline__ void set_pair(int i, float x, float y) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const bf16x2 high = {(__bf16)x, (__bf16)y};
+    const uint32_t bits = __builtin_bit_cast(uint32_t, high);
+    hi[i] = high[0], hi[i + 1] = high[1];
+    lo[i] = (__bf16)(x - __builtin_bit_cast(float, bits << 16));
+    lo[i + 1] = (__bf16)(y - __builtin_bit_cast(float, bits & 0xffff0000u));
   }
 };
 __device__ __forceinline__ f32x4 mma_wide(const WideFrag<float> &a, f32x8 b, f32x4 c) { return mma(a.v, b, c); }

@@ -1,0 +1,88 @@
+"""Attention of a portion of a prompt over chunks and windows, at the edges of its tiles: 64 rows whose keys the waves
+halve, 128 rows of heads that fill the compute units, four waves for wide heads; against float64 on the same bfloat16
+values.  A weighted mean of values is rounded to bfloat16 (2^-9 of itself); its weights carry 17 bits, and scores of
+order ten summed in float32 move them by less: 2^-13 of the largest value in all."""
+import struct
+
+import numpy as np
+import pytest
+
+from llmopt_amd.safetensors_file import from_bfloat16, to_bfloat16
+from tests.gpu_util import u32s
+
+pytestmark = pytest.mark.gpu
+GRID = ((1, 1, 1), (256, 1, 1))
+
+
+@pytest.fixture(scope="module")
+def runtime():
+    from llmopt_amd.native import Runtime
+    rt = Runtime()
+    yield rt
+    rt.close()
+
+
+# rows, heads, kv_heads, dim, vdim, span, softcap, sink, position of the first row, sliding
+@pytest.mark.parametrize("m,heads,kv,dim,vdim,span,softcap,sink,first,sliding", [
+    (2, 4, 2, 64, 64, 256, 0.0, True, 0, False),
+    (15, 3, 1, 32, 32, 100, 30.0, True, 33, False),
+    (16, 4, 4, 64, 32, 64, 50.0, False, 31, False),
+    (17, 2, 2, 40, 24, 33, 30.0, True, 32, False),
+    (63, 4, 2, 64, 128, 128, 0.0, True, 1, False),
+    (64, 4, 2, 128, 128, 4096, 30.0, False, 64, False),
+    (65, 4, 2, 128, 64, 96, 0.0, True, 95, False),
+    (129, 8, 2, 128, 128, 512, 30.0, True, 127, False),
+    (33, 4, 2, 256, 64, 64, 0.0, True, 40, False),
+    (70, 2, 1, 64, 256, 64, 30.0, False, 0, False),
+    (1025, 32, 8, 128, 128, 700, 30.0, True, 500, False),     # 128-row tiles, bounded scores
+    (1153, 32, 4, 72, 48, 2048, 0.0, False, 3, False),        # 128-row tiles of narrower heads
+    (1100, 32, 8, 128, 128, 300, 0.0, False, 250, True),      # 128-row tiles, a window
+    (300, 6, 2, 64, 64, 97, 0.0, False, 200, True),
+    (31, 6, 3, 128, 40, 1, 0.0, False, 5, True),              # a window of one
+])
+def test_tiles(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sliding):
+    rng = np.random.default_rng(m * 31 + heads)
+    capacity, slots, slot, scale = span, 2, 1, dim ** -0.5
+    n = heads * dim + kv * (dim + vdim)
+    bf16 = lambda *shape: to_bfloat16(rng.standard_normal(shape, dtype=np.float32))
+    rows, sinks = bf16(m, n), bf16(heads)
+    ring_k, ring_v = bf16(slots, kv, capacity, dim), bf16(slots, kv, capacity, vdim)
+    put = runtime.buffer_of_bytes
+    b_rows, b_k, b_v = put(rows), put(ring_k), put(ring_v)
+    step, out = put(np.array([first, slot], dtype=np.uint32)), runtime.create_buffer(m * heads * vdim * 2)
+    if sliding:
+        one = put(to_bfloat16(np.ones(dim, dtype=np.float32)))
+        runtime.dispatch("llmopt_rotary_attention_bf16", [b_rows, one, one, step, step, b_k, b_v, out],
+                         u32s(m, heads, kv, dim, vdim, n, heads * vdim, capacity, span, 1, slots, 0) +
+                         struct.pack("<ffff", scale, softcap, 1e-6, 1.0), *GRID)
+        rows = b_rows.numpy(np.uint16).reshape(m, n)  # normed in place
+    else:
+        runtime.dispatch("llmopt_chunk_attention_bf16", [b_rows, put(sinks), step, b_k, b_v, out],
+                         u32s(m, heads, kv, dim, vdim, capacity, span, slots, int(sink)) + struct.pack("<ff", scale, softcap),
+                         *GRID)
+    got = from_bfloat16(out.numpy(np.uint16)).reshape(m, heads, vdim).astype(np.float64)
+    assert np.isfinite(got).all()
+
+    wide = lambda a: from_bfloat16(a).astype(np.float64)
+    q = wide(rows[:, :heads * dim]).reshape(m, heads, dim)
+    fresh_k = wide(rows[:, heads * dim:heads * dim + kv * dim]).reshape(m, kv, dim)
+    fresh_v = wide(rows[:, heads * dim + kv * dim:]).reshape(m, kv, vdim)
+    begin = max(0, first - span)
+    past = np.arange(begin, first) % capacity
+    positions, seen_by = np.arange(begin, first + m), np.arange(first, first + m)
+    gap = seen_by[:, None] - positions[None, :]
+    visible = (gap >= 0) & ((gap < span) if sliding else (seen_by[:, None] // span == positions[None, :] // span))
+    for head in range(heads):
+        group = head // (heads // kv)
+        keys = np.concatenate([wide(ring_k[slot, group])[past], fresh_k[:, group]])
+        values = np.concatenate([wide(ring_v[slot, group])[past], fresh_v[:, group]])
+        score = q[:, head] @ keys.T * scale
+        if softcap:
+            score = softcap * np.tanh(score / softcap)
+        score = np.where(visible, score, -np.inf)
+        top = np.maximum(score.max(axis=1), wide(sinks)[head] if sink and not sliding else -np.inf)
+        weights = np.exp(score - top[:, None])
+        total = weights.sum(axis=1) + (np.exp(wide(sinks)[head] - top) if sink and not sliding else 0.0)
+        expected = weights @ values / total[:, None]
+        error = np.abs(got[:, head] - expected)
+        assert (error <= 2.0 ** -8 * np.abs(expected) + 2.0 ** -13 * np.abs(values).max()).all(), (head, error.max())
