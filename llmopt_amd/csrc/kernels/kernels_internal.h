@@ -57,6 +57,10 @@ bool w4a16_rows_ok(const W4DualSwigluArgs &args);
 hipError_t launch_w4a16_rows_linear(const W4LinearArgs &args, hipStream_t stream);
 hipError_t launch_w4a16_rows_qkv(const W4QkvArgs &args, hipStream_t stream);
 hipError_t launch_w4a16_rows_dual_swiglu(const W4DualSwigluArgs &args, hipStream_t stream);
+// y [rows / 2, n]: the float32 sums of the products of rows 2r and 2r + 1 (see launch_rms_norm_split).
+bool w4a16_rows_pairs_ok(const uint16_t *x, const W4Matrix &w, uint32_t rows, uint32_t n, uint32_t k);
+hipError_t launch_w4a16_rows_pairs(const uint16_t *x, const W4Matrix &w, float *y, uint32_t rows, uint32_t n, uint32_t k,
+                                   hipStream_t stream);
 
 hipError_t launch_w4a16_gemm_linear(const W4LinearArgs &args, hipStream_t stream);
 hipError_t launch_w4a16_gemm_dual_swiglu(const W4DualSwigluArgs &args, hipStream_t stream);

@@ -43,6 +43,7 @@ struct RowsParams {
   uint32_t segments;
   const uint16_t *addend;
   uint32_t addend_stride;
+  float *pairs;  // [m / 2, n]: in place of y, the float32 sums of rows 2r and 2r + 1
 };
 
 // base + offset (bytes, per lane) to consecutive LDS places: sixteen bytes a lane ...
@@ -202,6 +203,30 @@ __global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(RowsParams p) {
     }
   __syncthreads();
   constexpr int OUT = DUAL ? COLUMNS / 2 : COLUMNS, QUADS = ROWS * OUT / 4;
+  if (!DUAL && p.pairs != nullptr) {
+    const bool whole = (n & 3) == 0 && (reinterpret_cast<uintptr_t>(p.pairs) & 15) == 0;
+    for (int q = tid; q < QUADS / 2; q += WAVES * 64) {
+      const uint32_t row = q / (OUT / 4) * 2, c = q % (OUT / 4) * 4, at = m0 + row;
+      if (at >= p.m || n0 + c >= n) continue;
+      f4_t value[2];
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        value[r] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < P; ++k) value[r] += *reinterpret_cast<const f4_t *>(sums + (k * ROWS + row + r) * COLUMNS + c);
+      }
+      const f4_t sum = value[0] + value[1];
+      float *to = p.pairs + (size_t)(at / 2) * n + n0 + c;
+      if (whole) {
+        *reinterpret_cast<f4_t *>(to) = sum;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n0 + c + e < n) to[e] = sum[e];
+      }
+    }
+    return;
+  }
   uint16_t *y = p.y[segment];
   const bool whole = (n & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0;
   for (int q = tid; q < QUADS; q += WAVES * 64) {
@@ -337,6 +362,21 @@ bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k) {
   return !(w4a16_gemv_mfma_row_groups_ok(m, columns, k) && m * columns <= kRowGroupOutputs);
 }
 
+// Logits: as above while the launch is about one round of small tiles.  Beyond, where the 128 x 128 tiles have no float32
+// results, the tile that decodes the weights least often of those whose scales fit LDS beside the ring; with a long K up
+// to 24 rows stay with the matrix-core GEMV, which streams them better.  Head with its argmax in rows / 2 tokens, us,
+// tiles / GEMV (rows, K, n): 10 x 576 x 49152 22.4 / 30.8, 64 x 576 x 49152 27 / 58, 128 x 576 x 49152 33 / 78,
+// 24 x 2048 x 32000 38.1 / 38.9, 32 x 2048 x 32000 39.1 / 47, 64 x 2048 x 32000 45 / 62, 24 x 4096 x 32000 68.3 / 61.3,
+// 32 x 4096 x 32000 69 / 90, 128 x 4096 x 32000 97 / 193, 64 x 8192 x 16000 122 / 231.
+Tile pick_pairs_tile(uint32_t rows, uint32_t n, uint32_t k) {
+  const Tile small = pick_tile(rows, &n, 1, k);
+  if (small != Tile::kNone) return small;
+  if (k >= 1536 && rows <= 24) return Tile::kNone;
+  if (rows > 32 && rows_lds_bytes<64, 4, 2, 2>(k) <= kLdsBytes) return Tile::k64x128;
+  if (rows_lds_bytes<32, 2, 4, 2>(k) <= kLdsBytes) return Tile::k32x64;
+  return Tile::kNone;
+}
+
 }  // namespace
 
 bool w4a16_rows_ok(const W4LinearArgs &a) {
@@ -357,6 +397,24 @@ hipError_t launch_w4a16_rows_linear(const W4LinearArgs &a, hipStream_t stream) {
   p.addend = a.has_addend ? a.addend : nullptr;
   p.addend_stride = a.addend_row_stride;
   return launch_tile<false>(pick_tile(a.m, &a.n, 1, a.k), p, stream);
+}
+
+bool w4a16_rows_pairs_ok(const uint16_t *x, const W4Matrix &w, uint32_t rows, uint32_t n, uint32_t k) {
+  return rows_wanted(rows, n, k) && pieces_aligned(x, w.weight) && pick_pairs_tile(rows, n, k) != Tile::kNone;
+}
+
+hipError_t launch_w4a16_rows_pairs(const uint16_t *x, const W4Matrix &w, float *y, uint32_t rows, uint32_t n, uint32_t k,
+                                   hipStream_t stream) {
+  RowsParams p = {};
+  p.x = x;
+  p.m = rows;
+  p.k = k;
+  p.w[0] = w.weight;
+  p.s[0] = w.scale;
+  p.n[0] = n;
+  p.segments = 1;
+  p.pairs = y;
+  return launch_tile<false>(pick_pairs_tile(rows, n, k), p, stream);
 }
 
 bool w4a16_rows_ok(const W4QkvArgs &a) {

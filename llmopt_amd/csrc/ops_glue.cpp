@@ -216,13 +216,15 @@ int lm_head(llmopt_hip_context *context, const DispatchRecord &record, LmHeadVar
   if (variant.extra)
     if (int status = require_buffer_size(record.buffers[5], (uint64_t)m * n * 2, "logits")) return status;
 
-  // workspace: normalised activation (hi and lo row per input row) | float32 partial logits
-  // [2m, n] | candidates | GEMV scratch
+  // workspace: normalised activation (hi and lo row per input row) | float32 logits [m, n], or [2m, n] from the
+  // decode GEMV | candidates | GEMV scratch
   const uint32_t gemv_rows = 2 * m;
   const size_t normalized_bytes = round_up_256((size_t)gemv_rows * k * 2);
-  const size_t logits_bytes = round_up_256((size_t)gemv_rows * n * 4);
+  const W4Matrix weights = {record.buffers[2].device, as_f16(record.buffers[3])};
+  const bool tiles = w4a16_rows_pairs_ok(nullptr, weights, gemv_rows, n, k);  // (the workspace is aligned)
+  const size_t logits_bytes = round_up_256((size_t)(tiles ? m : gemv_rows) * n * 4);
   const size_t candidate_bytes = round_up_256((size_t)m * 256 * 8);
-  const size_t gemv_bytes = w4a16_gemv_workspace_bytes(std::min(gemv_rows, kGemvMaxRows), n, k);
+  const size_t gemv_bytes = tiles ? 0 : w4a16_gemv_workspace_bytes(std::min(gemv_rows, kGemvMaxRows), n, k);
   uint8_t *workspace = static_cast<uint8_t *>(
       context_workspace(context, normalized_bytes + logits_bytes + candidate_bytes + gemv_bytes));
   if (workspace == nullptr) return LLMOPT_ERR_FAILURE;
@@ -243,15 +245,21 @@ int lm_head(llmopt_hip_context *context, const DispatchRecord &record, LmHeadVar
   norm.epsilon = epsilon;
   if (int status = launched(launch_rms_norm_split(norm, context->stream), name)) return status;
 
-  // the decode GEMV keeps float32 results; more rows go through it in groups: of eight a launch, or - when one
-  // workgroup covers K, so that nothing is handed over between workgroups - up to 128 rows a launch as row groups
-  // of one grid (the 64 rows of 32 sequences at 49152 x 576: one launch instead of eight)
+  // More than the decode GEMV's eight rows go through small tiles, whose sums of a hi and a lo row are the logits (32
+  // sequences at 49152 x 576: the products 14 us where the GEMV's row groups took 43, and half the logits to read).  Where
+  // the tiles do not take the matrix or are not the faster ones, the decode GEMV, which keeps float32 results, runs in
+  // groups of eight rows: of a launch each, or - when one workgroup covers K, so that nothing is handed over between
+  // workgroups - of one grid.
+  if (tiles) {
+    if (int status = launched(launch_w4a16_rows_pairs(normalized, weights, logits, gemv_rows, n, k, context->stream), name))
+      return status;
+  }
   const uint32_t rows_per_launch = w4a16_gemv_mfma_needs_split(k) ? kGemvMaxRows : 128;
-  for (uint32_t first = 0; first < gemv_rows; first += rows_per_launch) {
+  for (uint32_t first = 0; !tiles && first < gemv_rows; first += rows_per_launch) {
     const uint32_t rows = std::min(rows_per_launch, gemv_rows - first);
     W4LinearArgs linear = {};
     linear.x = normalized + (size_t)first * k;
-    linear.w = {record.buffers[2].device, as_f16(record.buffers[3])};
+    linear.w = weights;
     linear.y = nullptr;
     linear.y_f32 = logits + (size_t)first * n;
     linear.m = rows;
@@ -269,7 +277,7 @@ int lm_head(llmopt_hip_context *context, const DispatchRecord &record, LmHeadVar
       return status;
   }
   uint16_t *half_logits = variant.extra ? as_f16_out(record.buffers[5]) : nullptr;
-  if (int status = launched(launch_argmax_candidates(logits, candidates, m, n, true, half_logits, context->stream),
+  if (int status = launched(launch_argmax_candidates(logits, candidates, m, n, !tiles, half_logits, context->stream),
                             name))
     return status;
   if (variant.stage1) return LLMOPT_OK;

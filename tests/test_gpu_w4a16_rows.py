@@ -9,6 +9,7 @@ import pytest
 
 import oracle
 from tests.gpu_util import assert_close_to_oracle, linear_grid, u32s, w4_case
+from tests.test_gpu_glue import check_tokens, lm_head_oracle, run_lm_head
 from tests.test_gpu_w4a16 import run_linear
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +94,19 @@ def test_small_tiles_over_three_matrices(runtime, m, k, sizes):
                      u32s(m, k, *sizes), grid=(linear_grid(m * sum(sizes)), 1, 1), group=(256, 1, 1))
     for (packed, scale), out, n in zip(mats, outs, sizes):
         assert_close_to_oracle(out.numpy(np.float16, (m, n)), product(x, packed, scale), f"three matrices {m}x{n}x{k}")
+
+
+# float32 logits from pairs of rows: one round of small tiles, 32 x 64 with short and with long K, 64 x 128, and the
+# matrix-core GEMV on the other side of the rule (few rows, long K)
+@pytest.mark.parametrize("m,n,k", [
+    (30, 2047, 64), (5, 33001, 576), (16, 16387, 576), (17, 33003, 320), (130, 10001, 576), (13, 24001, 1600),
+    (40, 20002, 1536), (12, 24001, 1536)])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+def test_logits_of_several_rows(runtime, m, n, k, dtype):
+    rng = np.random.default_rng(m * 31 + n)
+    x, packed, scale, _ = w4_case(rng, m, n, k)
+    x, weight = x.astype(dtype), rng.uniform(0.5, 1.5, k).astype(np.float16)
+    tokens, logits = run_lm_head(runtime, x, weight, packed, scale, 1e-5, extra=True)
+    expected = lm_head_oracle(x, weight, packed, scale, 1e-5)
+    check_tokens(tokens, expected)
+    assert_close_to_oracle(logits, expected, f"logits {m}x{n}x{k}")
