@@ -82,8 +82,8 @@ constexpr int kWavesPerBlock = 4;  // consecutive 32-row slabs of one head
 // MASK: 0 no mask, 1 a mask of bytes, 2 of halves, 3 the mask as one bit per (row, key), which the pass over the
 // mask ahead of this kernel leaves (every score is then tested; without one the instantiation carries
 // nothing of it).
-// KEYSPLIT: the four waves of a workgroup share ONE slab of 32 query rows and take a quarter of every
-// 128-key stage each; their partial results meet in LDS at the end.  For launches with fewer
+// KEYSPLIT: the waves of a workgroup share ONE slab of 32 query rows and take 32 keys of every stage each (a
+// quarter of 128, or an eighth of 256); their partial results meet in LDS at the end.  For launches with fewer
 // workgroups than CUs, which last as long as one wave's walk over all the keys of the last slab: the
 // walk is a quarter as long and there are four times as many workgroups.
 template <int D>
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
   // V rows are swizzled by twice the key within the row's first sixteen pieces at most: reads 8 and 16 keys
   // further down must find the same swizzle
   constexpr int VMASK = (PIECES < 16 ? PIECES : 16) - 1;
-  static_assert((STAGE_KEYS == 128 || STAGE_KEYS == 64 || STAGE_KEYS == 32) && COPIES >= 1 &&
+  static_assert((STAGE_KEYS == 256 || STAGE_KEYS == 128 || STAGE_KEYS == 64 || STAGE_KEYS == 32) && COPIES >= 1 &&
                     COPIES * KEYS_PER_COPY * WAVES == STAGE_KEYS,
                 "stage");
   static_assert(!KEYSPLIT || STAGE_KEYS == 32 * WAVES, "a tile of every stage per wave");
@@ -530,7 +530,7 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
       for (int r = 0; r < 16; ++r)
         share_out[(wave * D + 32 * jj + (r >> 2) * 8 + half * 4 + (r & 3)) * 32 + row_lane] = out_acc[jj][r];
     __syncthreads();
-    constexpr int PER_THREAD = D / 8;  // head_dim values per thread: 32 rows x 8 threads a row
+    constexpr int PER_THREAD = D / 2 / WAVES;  // head_dim values per thread: 32 rows x 2 WAVES threads a row
     const uint32_t out_row_index = q0 + (threadIdx.x & 31);
     const uint32_t d0 = (threadIdx.x >> 5) * PER_THREAD;
     float best = -INFINITY;
@@ -904,6 +904,13 @@ hipError_t launch_dense_attention(const DenseAttentionArgs &a, hipStream_t strea
       }
       if (geometry.key_split) {
         const uint32_t grid = (uint32_t)((a.query_length + 31) / 32) * a.heads * a.batches;
+        // One workgroup per CU that walks several stages: eight waves and 256-key stages (128 KB) halve the walk again
+        // (us, query rows / keys / heads, eight / four waves: 700 / 700 / 9 10.2 / 11.5, 900 / 900 / 9 11.7 / 14.5,
+        // 64 / 2000 / 9 15.1 / 17.3, 400 / 4000 / 9 29.8 / 40.5).  Walks of a few stages are as short either way (512 / 512 /
+        // 9 8.4 / 8.3), and where two workgroups would share a CU that room is worth more (700 / 700 / 32 20.6 / 14.0,
+        // 2048 / 2048 / 9 26.7 / 20.0).  With a mask the map of stages counts in 128 keys.
+        if (a.head_dim == 64 && mask == 0 && a.key_length > 512 && grid <= (uint32_t)device_compute_units() * 9 / 8)
+          return launch_tile32_instance<64, 8, 256, 0, true>(grid, scheduled, stream);
         if (a.head_dim == 64) return launch_tile32<64, 4, 128, true>(mask_kind, grid, scheduled, stream);
         return launch_tile32<128, 4, 128, true>(mask_kind, grid, scheduled, stream);
       }

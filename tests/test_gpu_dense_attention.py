@@ -332,6 +332,16 @@ def test_small_launches_split_the_keys_of_a_slab_over_the_waves(runtime, dim, he
 
 
 @pytest.mark.parametrize("heads,kv_heads,new,past,mode", [
+    (3, 1, 700, 0, "causal"), (2, 2, 33, 480, "causal"), (4, 2, 45, 900, "none"), (2, 1, 257, 256, "causal"),
+    (1, 1, 18, 1030, "none"),
+])
+def test_long_walks_of_few_slabs_take_eight_waves(runtime, heads, kv_heads, new, past, mode):
+    """Heads of 64, more than 512 keys and about a workgroup a CU at most: eight shares of every 256-key stage; waves
+    and whole stages without keys under the causal limit, partial last stages and slabs, both layouts."""
+    check_attention_case(runtime, 64, heads, kv_heads, new, past, mode)
+
+
+@pytest.mark.parametrize("heads,kv_heads,new,past,mode", [
     (4, 2, 300, 0, "causal"), (2, 1, 45, 211, "causal"), (2, 2, 33, 100, "none"), (3, 1, 130, 70, "bool"),
     (2, 2, 64, 191, "f16"), (8, 4, 16, 0, "causal"),
 ])
