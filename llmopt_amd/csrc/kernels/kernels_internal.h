@@ -56,6 +56,9 @@ bool w4a16_rows_ok(const W4QkvArgs &args);
 bool w4a16_rows_ok(const W4DualSwigluArgs &args);
 hipError_t launch_w4a16_rows_linear(const W4LinearArgs &args, hipStream_t stream);
 hipError_t launch_w4a16_rows_qkv(const W4QkvArgs &args, hipStream_t stream);
+// launch_w4a16_rows_qkv and launch_rotary_qk_pack in one launch; the queries and keys before their rotation are not kept.
+bool w4a16_rows_pack_ok(const W4QkvArgs &args, const RotaryPackArgs &rotary);
+hipError_t launch_w4a16_rows_qkv_pack(const W4QkvArgs &args, const RotaryPackArgs &rotary, hipStream_t stream);
 hipError_t launch_w4a16_rows_dual_swiglu(const W4DualSwigluArgs &args, hipStream_t stream);
 // y [rows / 2, n]: the float32 sums of the products of rows 2r and 2r + 1 (see launch_rms_norm_split).
 bool w4a16_rows_pairs_ok(const uint16_t *x, const W4Matrix &w, uint32_t rows, uint32_t n, uint32_t k);

@@ -169,13 +169,15 @@ __device__ __forceinline__ float wave_max(float value) {
 // Q8 cache quantiser of one 64-wide group, one element per lane (lib/metal_cache_source.ml:62-80):
 // the stored scale half(max|x| / 127) (1.0 for an all-zero group) and this lane's int8 value
 // clamp(rint(x / float(scale)), -127, 127).
-__device__ __forceinline__ int8_t q8_quantize(float x, uint16_t *stored_scale) {
-  const float maximum = wave_max(fabsf(x));
+__device__ __forceinline__ int8_t q8_quantize_by(float x, float maximum, uint16_t *stored_scale) {
   const uint16_t stored = float_to_half_bits(maximum == 0.0f ? 1.0f : maximum / 127.0f);
   const float scale = half_bits_to_float(stored);
   const float rounded = rintf(x / scale);
   *stored_scale = stored;
   return (int8_t)(int)fminf(fmaxf(rounded, -127.0f), 127.0f);
+}
+__device__ __forceinline__ int8_t q8_quantize(float x, uint16_t *stored_scale) {
+  return q8_quantize_by(x, wave_max(fabsf(x)), stored_scale);
 }
 
 }  // namespace llmopt

@@ -22,6 +22,7 @@
 // step (52 of them the decode) beside 24 KB of copies.  Tried without gain: operands read a step ahead of their use,
 // two column blocks a wave, a start of the walk over K that differs by workgroup, deeper rings.
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.h"
 #include "kernels_internal.h"
@@ -44,6 +45,17 @@ struct RowsParams {
   const uint16_t *addend;
   uint32_t addend_stride;
   float *pairs;  // [m / 2, n]: in place of y, the float32 sums of rows 2r and 2r + 1
+};
+
+// A QKV launch whose queries and keys are rotated and whose keys and values also go to their tokens' Q8 pool slots, in
+// the arithmetic of launch_rotary_qk_pack: heads of 64 columns, one sequence.  y[0] and y[1] are then the rotated
+// outputs [head, token, 64].  One layer's launch at 700 x 576 x (576, 192, 192): 8.2 us where the projection and the
+// rotation with the pack take 7.0 + 5.5, most of either the start of a launch.
+struct PackParams : RowsParams {
+  const uint16_t *cosine, *sine;  // [token, 64]
+  const uint32_t *slots;
+  uint8_t *pool;
+  uint32_t token_stride, token_elements, segment_offset[2];
 };
 
 // base + offset (bytes, per lane) to consecutive LDS places: sixteen bytes a lane ...
@@ -70,8 +82,10 @@ __device__ __forceinline__ h8_t w4_exact_natural(uint32_t word) {
 // Scales of a tile in LDS: blocks of eight columns by eight groups, a dword each.
 constexpr uint32_t scale_lds_bytes(uint32_t columns, uint32_t groups) { return columns / 8 * ((groups + 7) / 8) * 256; }
 
-template <int ROWS, int CT, int P, int STAGES, bool DUAL>
-__global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(RowsParams p) {
+template <int ROWS, int CT, int P, int STAGES, bool DUAL, class Params>
+__global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
+  constexpr bool PACK = std::is_same_v<Params, PackParams>;
+  static_assert(!PACK || (!DUAL && CT % 2 == 0), "whole heads in a tile");
   constexpr int WAVES = CT * P, COLUMNS = CT * 32, STEP = P * 64;
   constexpr int RT = (ROWS + 31) / 32;                      // 32-row blocks of a wave
   constexpr int X_PIECES = STEP / 8, W_PIECES = STEP / 32;  // 16-byte pieces of a row and step
@@ -203,6 +217,56 @@ __global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(RowsParams p) {
     }
   __syncthreads();
   constexpr int OUT = DUAL ? COLUMNS / 2 : COLUMNS, QUADS = ROWS * OUT / 4;
+  if constexpr (PACK) {
+    typedef uint16_t u16x4_t __attribute__((ext_vector_type(4), aligned(2)));
+    typedef uint32_t any_u32_t __attribute__((aligned(1)));
+    // a head of a row is sixteen neighbouring lanes
+    for (int q = tid; q < QUADS; q += WAVES * 64) {
+      const uint32_t row = q / (OUT / 4), c = q % (OUT / 4) * 4, at = m0 + row;
+      if (at >= p.m || n0 + c >= n) continue;
+      const uint32_t head = (n0 + c) / 64, d = c % 64;
+      f4_t value = {0.f, 0.f, 0.f, 0.f}, other = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < P; ++k) {
+        value += *reinterpret_cast<const f4_t *>(sums + (k * ROWS + row) * COLUMNS + c);
+        other += *reinterpret_cast<const f4_t *>(sums + (k * ROWS + row) * COLUMNS + (c ^ 32));
+      }
+      u16x4_t out;
+      float wide[4];
+      if (segment < 2) {
+        const u16x4_t cosine = *reinterpret_cast<const u16x4_t *>(p.cosine + (size_t)at * 64 + d);
+        const u16x4_t sine = *reinterpret_cast<const u16x4_t *>(p.sine + (size_t)at * 64 + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const _Float16 turned = rotate_half_value((_Float16)value[e], (_Float16)other[e], __builtin_bit_cast(_Float16, (uint16_t)cosine[e]),
+                                                    __builtin_bit_cast(_Float16, (uint16_t)sine[e]), d < 32);
+          out[e] = __builtin_bit_cast(uint16_t, turned);
+          wide[e] = (float)turned;
+        }
+        *reinterpret_cast<u16x4_t *>(p.y[segment] + ((size_t)head * p.m + at) * 64 + d) = out;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          out[e] = float_to_half_bits(value[e]);
+          wide[e] = half_bits_to_float(out[e]);
+        }
+        *reinterpret_cast<u16x4_t *>(p.y[2] + (size_t)at * n + n0 + c) = out;
+      }
+      if (segment == 0) continue;
+      float maximum = fmaxf(fmaxf(fabsf(wide[0]), fabsf(wide[1])), fmaxf(fabsf(wide[2]), fabsf(wide[3])));
+#pragma unroll
+      for (int lanes = 1; lanes < 16; lanes *= 2) maximum = fmaxf(maximum, __shfl_xor(maximum, lanes, 64));
+      uint16_t stored;
+      uint32_t packed = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) packed |= (uint32_t)(uint8_t)q8_quantize_by(wide[e], maximum, &stored) << (8 * e);
+      uint8_t *slot = p.pool + (size_t)p.slots[at] * p.token_stride;
+      const uint32_t offset = p.segment_offset[segment - 1] + head * 64;
+      *reinterpret_cast<any_u32_t *>(slot + offset + d) = packed;
+      if (d == 0) reinterpret_cast<uint16_t *>(slot + p.token_elements)[offset / 64] = stored;
+    }
+    return;
+  }
   if (!DUAL && p.pairs != nullptr) {
     const bool whole = (n & 3) == 0 && (reinterpret_cast<uintptr_t>(p.pairs) & 15) == 0;
     for (int q = tid; q < QUADS / 2; q += WAVES * 64) {
@@ -268,9 +332,9 @@ constexpr uint32_t rows_lds_bytes(uint32_t k) {
   return scale_lds_bytes(CT * 32, k / 64) + (ring > sums ? ring : sums);
 }
 
-template <int ROWS, int CT, int P, int STAGES, bool DUAL>
-hipError_t run_rows(RowsParams &p, hipStream_t stream) {
-  const auto kernel = w4a16_rows_kernel<ROWS, CT, P, STAGES, DUAL>;
+template <int ROWS, int CT, int P, int STAGES, bool DUAL, class Params>
+hipError_t run_rows(Params &p, hipStream_t stream) {
+  const auto kernel = w4a16_rows_kernel<ROWS, CT, P, STAGES, DUAL, Params>;
   const uint32_t bytes = rows_lds_bytes<ROWS, CT, P, STAGES>(p.k);
   if (bytes > kLdsBytes) return hipErrorInvalidValue;
   static bool allowed[kMaxDevices] = {};
@@ -330,11 +394,11 @@ Tile pick_pair_tile(uint32_t m, uint32_t n, uint32_t k) {
   return Tile::kNone;
 }
 
-template <bool DUAL>
-hipError_t launch_tile(Tile tile, RowsParams &p, hipStream_t stream) {
+template <bool DUAL, class Params>
+hipError_t launch_tile(Tile tile, Params &p, hipStream_t stream) {
   switch (tile) {
     case Tile::k32x32:
-      if constexpr (!DUAL) return run_rows<32, 1, 8, 3, false>(p, stream);
+      if constexpr (!DUAL && std::is_same_v<Params, RowsParams>) return run_rows<32, 1, 8, 3, false>(p, stream);
       return hipErrorInvalidValue;
     case Tile::k32x64: return run_rows<32, 2, 4, 2, DUAL>(p, stream);
     case Tile::k32x64Deep: return run_rows<32, 2, 8, 3, DUAL>(p, stream);
@@ -437,6 +501,43 @@ hipError_t launch_w4a16_rows_qkv(const W4QkvArgs &a, hipStream_t stream) {
   }
   p.segments = 3;
   return launch_tile<false>(pick_tile(a.m, a.n, 3, a.k), p, stream);
+}
+
+// A tile of whole heads: where the rule takes half a head's columns, the 64-column one, whose few microseconds more are
+// less than another launch.
+static Tile pick_pack_tile(const W4QkvArgs &a) {
+  const Tile tile = pick_tile(a.m, a.n, 3, a.k);
+  if (tile != Tile::k32x32) return tile;
+  if (a.k < 1536) return Tile::k32x64;
+  if (rows_lds_bytes<32, 2, 8, 3>(a.k) <= kLdsBytes) return Tile::k32x64Deep;
+  return rows_lds_bytes<32, 2, 4, 4>(a.k) <= kLdsBytes ? Tile::k32x64Long : Tile::kNone;
+}
+
+bool w4a16_rows_pack_ok(const W4QkvArgs &a, const RotaryPackArgs &r) {
+  return w4a16_rows_ok(a) && r.rotary.batches == 1 && r.rotary.width == 64 && pick_pack_tile(a) != Tile::kNone;
+}
+
+hipError_t launch_w4a16_rows_qkv_pack(const W4QkvArgs &a, const RotaryPackArgs &r, hipStream_t stream) {
+  PackParams p = {};
+  p.x = a.x;
+  p.m = a.m;
+  p.k = a.k;
+  uint16_t *const out[3] = {r.rotary.q_output, r.rotary.k_output, a.y[2]};
+  for (int i = 0; i < 3; ++i) {
+    p.w[i] = a.w[i].weight;
+    p.s[i] = a.w[i].scale;
+    p.y[i] = out[i];
+    p.n[i] = a.n[i];
+  }
+  p.segments = 3;
+  p.cosine = r.rotary.cosine;
+  p.sine = r.rotary.sine;
+  p.slots = r.pack.slots;
+  p.pool = r.pack.pool;
+  p.token_stride = r.pack.token_stride;
+  p.token_elements = r.pack.token_elements;
+  for (int i = 0; i < 2; ++i) p.segment_offset[i] = r.pack.segment_offset[i];
+  return launch_tile<false>(pick_pack_tile(a), p, stream);
 }
 
 bool w4a16_rows_ok(const W4DualSwigluArgs &a) {

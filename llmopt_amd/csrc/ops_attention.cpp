@@ -129,18 +129,10 @@ int cache_pack_pair_batched(llmopt_hip_context *context, const DispatchRecord &r
 // then AttentionCachePairParams (11 words); buffers: q_input, k_input, cosine, sine, q_output,
 // k_output (also the quantiser's key source), value source, slots, pool.
 int rotary_qk_pack_batched(llmopt_hip_context *context, const DispatchRecord &record) {
-  if (int status = require_buffer_count(record, 9)) return status;
-  if (int status = require_parameter_bytes(record, 28 + 44)) return status;
-  RotaryPackArgs args = {};
-  if (int status = parse_rotary_qk(record, &args.rotary)) return status;
-  if (int status = parse_pack_pair(record, 28, 5, 6, 7, 8, true, &args.pack)) return status;
-  if ((uint64_t)args.pack.items != (uint64_t)args.rotary.batches * args.rotary.tokens ||
-      args.pack.heads != args.rotary.k_heads || args.pack.head_dim != args.rotary.width)
-    return fail(LLMOPT_ERR_INVALID, "%s requires the same tokens (sequences x tokens items), KV heads and width "
-                "in both parameter blocks", record.name.c_str());
+  RotaryPackArgs args;
+  if (int status = parse_rotary_qk_pack(record, &args)) return status;
   return launched(launch_rotary_qk_pack(args, context->stream), record.name.c_str());
 }
-
 // buffers: pool, slots, destination; AttentionCacheParams.
 int cache_unpack(llmopt_hip_context *context, const DispatchRecord &record) {
   if (int status = require_buffer_count(record, 3)) return status;
@@ -471,6 +463,20 @@ int speculative_attention(llmopt_hip_context *context, const DispatchRecord &rec
 }
 
 }  // namespace
+
+int parse_rotary_qk_pack(const DispatchRecord &record, RotaryPackArgs *out) {
+  if (int status = require_buffer_count(record, 9)) return status;
+  if (int status = require_parameter_bytes(record, 28 + 44)) return status;
+  RotaryPackArgs args = {};
+  if (int status = parse_rotary_qk(record, &args.rotary)) return status;
+  if (int status = parse_pack_pair(record, 28, 5, 6, 7, 8, true, &args.pack)) return status;
+  if ((uint64_t)args.pack.items != (uint64_t)args.rotary.batches * args.rotary.tokens ||
+      args.pack.heads != args.rotary.k_heads || args.pack.head_dim != args.rotary.width)
+    return fail(LLMOPT_ERR_INVALID, "%s requires the same tokens (sequences x tokens items), KV heads and width "
+                "in both parameter blocks", record.name.c_str());
+  *out = args;
+  return LLMOPT_OK;
+}
 
 void register_cache_kernels(std::vector<KernelEntryPoint> &table) {
   static const char *const cache = "cache";

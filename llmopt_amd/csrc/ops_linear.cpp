@@ -5,6 +5,7 @@
 #include <cmath>
 
 #include "kernels/kernels.h"
+#include "kernels/kernels_internal.h"
 #include "runtime.h"
 
 namespace llmopt {
@@ -151,6 +152,55 @@ int w4a16_qkv_linear(llmopt_hip_context *context, const DispatchRecord &record) 
 // qOut, kOut, vOut; parameters W4A16QKVParams + f32 epsilon.
 int rms_w4a16_qkv_linear(llmopt_hip_context *context, const DispatchRecord &record) {
   return qkv_linear(context, record, true);
+}
+
+// Extension (no reference kernel): llmopt_rms_w4a16_qkv_linear_f16_g64 followed by llmopt_rotary_qk_pack_q8_batched on
+// its outputs, as one launch of the projection where its tiles hold whole heads and as those launches (the projection's
+// queries and keys in scratch) elsewhere.  buffers: input, norm weight, qW, qS, kW, kS, vW, vS, cosine, sine, q_output,
+// k_output, vOut, slots, pool; parameters: W4A16QKVParams + f32 epsilon (24 bytes), then the rotation's 72.
+int rms_w4a16_qkv_rotary_pack_prompt(llmopt_hip_context *context, const DispatchRecord &record) {
+  if (int status = require_buffer_count(record, 15)) return status;
+  if (int status = require_parameter_bytes(record, 24 + 28 + 44)) return status;
+  const char *name = record.name.c_str();
+  W4QkvArgs args = {};
+  args.m = param_u32(record, 0);
+  args.k = param_u32(record, 4);
+  static const char *const labels[3] = {"query", "key", "value"};
+  for (int i = 0; i < 3; ++i) {
+    args.n[i] = param_u32(record, 8 + 4 * i);
+    if (int status = check_w4_shape(name, args.m, args.n[i], args.k)) return status;
+    if (int status = check_w4_matrix(record.buffers[2 + 2 * i], record.buffers[3 + 2 * i], args.n[i], args.k, labels[i]))
+      return status;
+    args.w[i] = {record.buffers[2 + 2 * i].device, as_f16(record.buffers[3 + 2 * i])};
+  }
+  if (int status = require_buffer_size(record.buffers[0], (uint64_t)args.m * args.k * 2, "input")) return status;
+  const size_t bytes[3] = {(size_t)args.m * args.k * 2, (size_t)args.m * args.n[0] * 2, (size_t)args.m * args.n[1] * 2};
+  // scratch: normalised rows | queries | keys
+  const size_t at[2] = {(bytes[0] + 255) & ~(size_t)255, ((bytes[0] + 255) & ~(size_t)255) + ((bytes[1] + 255) & ~(size_t)255)};
+  uint8_t *scratch = static_cast<uint8_t *>(context_workspace(context, at[1] + bytes[2]));
+  if (scratch == nullptr) return LLMOPT_ERR_FAILURE;
+  DispatchRecord rotation = {};
+  rotation.name = record.name;
+  rotation.buffers = {{scratch + at[0], bytes[1]}, {scratch + at[1], bytes[2]}};
+  rotation.buffers.insert(rotation.buffers.end(), record.buffers.begin() + 8, record.buffers.end());
+  rotation.parameters.assign(record.parameters.begin() + 24, record.parameters.end());
+  RotaryPackArgs pack = {};
+  if (int status = parse_rotary_qk_pack(rotation, &pack)) return status;
+  const RotaryQkArgs &r = pack.rotary;
+  if ((uint64_t)r.batches * r.tokens != args.m || (uint64_t)r.q_heads * r.width != args.n[0] ||
+      (uint64_t)r.k_heads * r.width != args.n[1] || args.n[2] != args.n[1] || r.width % 64 != 0)
+    return fail(LLMOPT_ERR_INVALID, "%s requires the projections of the rotation's tokens and heads", name);
+  args.y[0] = reinterpret_cast<uint16_t *>(scratch + at[0]);
+  args.y[1] = reinterpret_cast<uint16_t *>(scratch + at[1]);
+  args.y[2] = reinterpret_cast<uint16_t *>(record.buffers[12].device);
+  args.x = as_f16(record.buffers[0]);
+  const W4Norm norm = {as_f16(record.buffers[1]), param_f32(record, 20), 0};
+  if (int status = normalise_input(context, record, norm, args.m, args.k, (uint64_t)args.n[0] + 2 * (uint64_t)args.n[1], &args.x,
+                                   &args.norm))
+    return status;
+  if (w4a16_rows_pack_ok(args, pack)) return launched(launch_w4a16_rows_qkv_pack(args, pack, context->stream), name);
+  if (int status = launched(launch_w4a16_qkv(args, context->stream), name)) return status;
+  return launched(launch_rotary_qk_pack(pack, context->stream), name);
 }
 
 // W4A16SwiGLUFFNParams {u32 m, n, k; f32 eps}: n = intermediate width, k = hidden width
@@ -406,6 +456,7 @@ void register_linear_kernels(std::vector<KernelEntryPoint> &table) {
   table.push_back({"llmopt_w4a16_qkv_linear_f16_g64_m4", qkv, w4a16_qkv_linear});
   table.push_back({"llmopt_w4a16_qkv_linear_f16_g64_m8", qkv, w4a16_qkv_linear});
   table.push_back({"llmopt_rms_w4a16_qkv_linear_f16_g64", qkv, rms_w4a16_qkv_linear});
+  table.push_back({"llmopt_rms_w4a16_qkv_rotary_pack_prompt_q8_f16_g64", qkv, rms_w4a16_qkv_rotary_pack_prompt});
   table.push_back({"llmopt_rms_w4a16_dual_swiglu_f16_g64", ffn, rms_w4a16_dual_swiglu});
   table.push_back({"llmopt_w4a16_dual_swiglu_f16_g64", ffn, w4a16_dual_swiglu});
   table.push_back({"llmopt_w4a16_dual_swiglu_f16_g64_m4", ffn, w4a16_dual_swiglu});

@@ -137,6 +137,9 @@ struct RotaryQkArgs;
 // RotaryQKParams (the first 28 parameter bytes) and the six rotary buffers (the first six of
 // the record), checked as llmopt_rotary_qk_f16_simd_h64 checks them.
 int parse_rotary_qk(const DispatchRecord &record, RotaryQkArgs *out);
+struct RotaryPackArgs;
+// The parameters (28 + 44 bytes) and nine buffers of llmopt_rotary_qk_pack_q8_batched, checked as it checks them.
+int parse_rotary_qk_pack(const DispatchRecord &record, RotaryPackArgs *out);
 
 // Resolves, for the current device, the address of the static scratch array behind
 // llmopt_hip_attention_q8_paged_no_alloc (once per device).

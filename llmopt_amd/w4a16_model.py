@@ -108,7 +108,7 @@ class W4a16Model:
             if len(self._prompts) >= 64:
                 self._prompts.clear()
             step = PrefillStep(self.runtime, self.config, {}, tokens, self._slot_pool(slot), self._slots,
-                               device_weights=self.device, work=self._prompt_work)
+                               device_weights=self.device, packed_projection=True, work=self._prompt_work)
             self._prompts[slot, tokens] = step, DispatchList(step.dispatches[:-1])  # (LM heads go with the wanted places)
         return self._prompts[slot, tokens]
 

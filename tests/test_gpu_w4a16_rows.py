@@ -110,3 +110,59 @@ def test_logits_of_several_rows(runtime, m, n, k, dtype):
     expected = lm_head_oracle(x, weight, packed, scale, 1e-5)
     check_tokens(tokens, expected)
     assert_close_to_oracle(logits, expected, f"logits {m}x{n}x{k}")
+
+
+# width, query heads, key / value heads, tokens: two launches (few tokens: the decode projection; heads of 128), 32 x 64
+# where half a head's columns would be the tile, 32 x 64, 64 x 64 and 64 x 128 tiles of whole heads, large tiles
+@pytest.mark.parametrize("k,heads,kv_heads,dim,tokens", [
+    (576, 9, 3, 64, 7), (576, 9, 3, 64, 40), (320, 4, 2, 128, 200), (576, 9, 3, 64, 90), (64, 3, 1, 64, 333), (576, 9, 3, 64, 700),
+    (2048, 8, 2, 64, 70), (4160, 16, 8, 64, 33), (1600, 32, 8, 64, 193), (576, 32, 8, 64, 520), (576, 32, 8, 64, 2048)])
+def test_projection_with_rotation_and_pack(runtime, k, heads, kv_heads, dim, tokens):
+    """The entry against the two that it joins: the rotated queries and keys, the values and the pool bit for bit where
+    both run the same tile, slots in any order, a key / value row of zeros (whose scale is one), bytes of other layers and tokens left alone."""
+    rng = np.random.default_rng(tokens + k)
+    n = (heads * dim, kv_heads * dim, kv_heads * dim)
+    x, norm = rng.standard_normal((tokens, k)).astype(np.float16), rng.uniform(0.5, 1.5, k).astype(np.float16)
+    x[tokens // 2] = 0
+    put = runtime.buffer_of_bytes
+    matrices = [put(a) for rows in n for a in w4_case(rng, 1, rows, k)[1:3]]
+    angle = rng.uniform(0, 6.3, (tokens, dim // 2)).astype(np.float32)
+    cosine, sine = (put(np.concatenate([f(angle)] * 2, axis=1).astype(np.float16)) for f in (np.cos, np.sin))
+    elements, stride = 4 * n[1], 4 * n[1] + 4 * n[1] // 32 + 6
+    slots = put(rng.permutation(tokens + 3)[:tokens].astype(np.uint32))
+    pool = rng.integers(0, 256, (tokens + 3) * stride, dtype=np.uint8)
+    projection = u32s(tokens, k, *n) + struct.pack("<f", 1e-5)
+    pack = u32s(1, tokens, heads, kv_heads, dim, dim // 2, 1) + \
+        u32s(tokens, n[1], 3 * n[1], kv_heads, dim, 64, elements, elements // 64, stride, tokens, 0)
+    results = []
+    for joined in (False, True):
+        create = lambda i: put(np.full(tokens * n[i], np.nan, dtype=np.float16))
+        q_out, k_out, v_out, b_pool = create(0), create(1), create(2), put(pool)
+        if joined:
+            runtime.dispatch("llmopt_rms_w4a16_qkv_rotary_pack_prompt_q8_f16_g64",
+                             [put(x), put(norm), *matrices, cosine, sine, q_out, k_out, v_out, slots, b_pool],
+                             projection + pack, (linear_grid(sum(n)), 1, 1), (256, 1, 1))
+        else:
+            q, k_raw = create(0), create(1)
+            runtime.dispatch("llmopt_rms_w4a16_qkv_linear_f16_g64", [put(x), put(norm), *matrices, q, k_raw, v_out],
+                             projection, (linear_grid(sum(n)), 1, 1), (256, 1, 1))
+            runtime.dispatch("llmopt_rotary_qk_pack_q8_batched",
+                             [q, k_raw, cosine, sine, q_out, k_out, v_out, slots, b_pool], pack, (256, 1, 1), (256, 1, 1))
+        results.append([b.numpy(np.uint8) for b in (q_out, k_out, v_out, b_pool)])
+    if (k, tokens) in ((576, 90), (4160, 33)):
+        # the projection alone takes the tile of half a head's columns, whose sums add in another order: a value moves by
+        # one rounding to half (2^-10 of itself) at most and takes two of them and their products' roundings along, a
+        # scale by as many units in its last place, a quantised value by one step
+        for two, one in zip(*(r[:3] for r in results)):
+            two, one = two.view(np.float16).astype(np.float32), one.view(np.float16).astype(np.float32)
+            assert np.abs(one - two).max() <= 4 * 2.0 ** -10 * np.abs(two).max()
+        two, one = (r[3].reshape(-1, stride) for r in results)
+        scales = slice(elements, elements + elements // 32)
+        for a, b, steps in ((one[:, :elements].view(np.int8), two[:, :elements].view(np.int8), 1),
+                            (np.ascontiguousarray(one[:, scales]).view(np.uint16),
+                             np.ascontiguousarray(two[:, scales]).view(np.uint16), 4)):
+            assert np.abs(a.astype(np.int32) - b.astype(np.int32)).max() <= steps
+        return
+    for name, two, one in zip(("queries", "keys", "values", "pool"), *results):
+        np.testing.assert_array_equal(one, two, err_msg=name)
+    assert np.isfinite(results[1][0].view(np.float16)).all()
