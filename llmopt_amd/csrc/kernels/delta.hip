@@ -58,14 +58,23 @@ __device__ __forceinline__ WideFrag<__bf16> load_wide<__bf16>(const __bf16 *p, s
 template <typename T, int N>
 __device__ __forceinline__ void store_wide(T *p, size_t plane, const float (&v)[N]) {
   typedef T xn __attribute__((ext_vector_type(N)));
-  xn high, low;
+  static_assert(N % 2 == 0 && N <= 8, "pairs of a fragment");
+  xn high;
+  if constexpr (kPlanes<T> == 2) {
+    xn low;
+    WideFrag<T> pairs;
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    high[i] = (T)v[i];
-    low[i] = (T)(v[i] - (float)high[i]);
+    for (int i = 0; i < N; i += 2) {
+      pairs.set_pair(i, v[i], v[i + 1]);
+#pragma unroll
+      for (int e = i; e < i + 2; ++e) high[e] = pairs.hi[e], low[e] = pairs.lo[e];
+    }
+    *reinterpret_cast<xn *>(p + plane) = low;
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) high[i] = v[i];
   }
   *reinterpret_cast<xn *>(p) = high;
-  if (kPlanes<T> == 2) *reinterpret_cast<xn *>(p + plane) = low;
 }
 // Matrices that become matrix-core operands lie in operand order: blocks of 16 rows and 32 contraction indices, lane
 // (index / 8) * 16 + row of a block holding eight of them, so that an operand is one contiguous kilobyte.
@@ -354,8 +363,9 @@ __device__ __forceinline__ f32x4 block_product(f32x4 a, f32x4 b, f32x4 c) {
 }
 
 // SLICES: dim <= 64 SLICES.  Wherever a thread owns a channel or value column it has the sixteen tokens of block `wave`.
-template <typename T, int SLICES, int TAPS>
-__global__ __launch_bounds__(256, SLICES <= 2 ? 2 : 1) void delta_chunk_kernel(DeltaArgs a, DeltaWorkspace w) {
+// WAVES: a SIMD's, as many workgroups a compute unit.
+template <typename T, int SLICES, int TAPS, int WAVES>
+__global__ __launch_bounds__(256, WAVES) void delta_chunk_kernel(DeltaArgs a, DeltaWorkspace w) {
   __shared__ __attribute__((aligned(16))) float lds_k[Q * kSliceStride], lds_q[Q * kSliceStride], lds_l[Q * kSliceStride];
   __shared__ __attribute__((aligned(16))) float lds_total[4][kSlice], lds_beta[Q];
   float *lds_n = lds_q, *lds_t = lds_k;  // N and (I + N)^-1, once the slices are done
@@ -484,24 +494,25 @@ __global__ __launch_bounds__(256, SLICES <= 2 ? 2 : 1) void delta_chunk_kernel(D
       }
       if (safe) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float from_middle = l[e] - 0.5f * lds_total[wave][at + e];
-          const float up = __expf(from_middle);
-          later_k.set(e, kv[e] * up);
-          later_q.set(e, qv[e] * up);
-          earlier.set(e, kv[e] * __expf(-from_middle));
+        for (int e = 0; e < 8; e += 2) {
+          const float middle[2] = {l[e] - 0.5f * lds_total[wave][at + e], l[e + 1] - 0.5f * lds_total[wave][at + e + 1]};
+          const float up[2] = {__expf(middle[0]), __expf(middle[1])};
+          later_k.set_pair(e, kv[e] * up[0], kv[e + 1] * up[1]);
+          later_q.set_pair(e, qv[e] * up[0], qv[e + 1] * up[1]);
+          earlier.set_pair(e, kv[e] * __expf(-middle[0]), kv[e + 1] * __expf(-middle[1]));
         }
         own_k = mma_wide_both(earlier, later_k, own_k);
         own_q = mma_wide_both(earlier, later_q, own_q);
       }
       float between[8];  // the decay of the blocks between
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float factor = __expf(l[e]);
-        qv[e] *= factor;
-        later_k.set(e, kv[e] * factor);
-        later_q.set(e, qv[e]);
-        between[e] = 0.0f;
+      for (int e = 0; e < 8; e += 2) {
+        const float factor[2] = {__expf(l[e]), __expf(l[e + 1])};
+        qv[e] *= factor[0];
+        qv[e + 1] *= factor[1];
+        later_k.set_pair(e, kv[e] * factor[0], kv[e + 1] * factor[1]);
+        later_q.set_pair(e, qv[e], qv[e + 1]);
+        between[e] = between[e + 1] = 0.0f;
       }
 #pragma unroll
       for (int j = 2; j >= 0; --j) {
@@ -513,9 +524,12 @@ __global__ __launch_bounds__(256, SLICES <= 2 ? 2 : 1) void delta_chunk_kernel(D
           const f32x4 k4 = *reinterpret_cast<const f32x4 *>(lds_k + other + half * 4);
           const f32x4 total = *reinterpret_cast<const f32x4 *>(&lds_total[j][at + half * 4]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            earlier.set(half * 4 + e, k4[e] * __expf(total[e] - l4[e] + between[half * 4 + e]));
-            between[half * 4 + e] += total[e];
+          for (int e = 0; e < 4; e += 2) {
+            float *gap = between + half * 4 + e;
+            earlier.set_pair(half * 4 + e, k4[e] * __expf(total[e] - l4[e] + gap[0]),
+                             k4[e + 1] * __expf(total[e + 1] - l4[e + 1] + gap[1]));
+            gap[0] += total[e];
+            gap[1] += total[e + 1];
           }
         }
         acc_k[j] = mma_wide_both(earlier, later_k, acc_k[j]);
@@ -635,9 +649,10 @@ __global__ __launch_bounds__(256, SLICES <= 2 ? 2 : 1) void delta_chunk_kernel(D
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < 8; e += 2) {
       const int j = s * 32 + quad * 8 + e;
-      solve[s].set(e, j <= token ? lds_t[token * kSliceStride + j] * lds_beta[j] : 0.0f);
+      solve[s].set_pair(e, j <= token ? lds_t[token * kSliceStride + j] * lds_beta[j] : 0.0f,
+                        j + 1 <= token ? lds_t[token * kSliceStride + j + 1] * lds_beta[j + 1] : 0.0f);
     }
   const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
   for (uint32_t tile = 0; tile < w.ep; tile += 16) {
@@ -793,8 +808,10 @@ __global__ __launch_bounds__(512) void delta_state_kernel(DeltaArgs a, DeltaWork
 
 // The parallel part: a workgroup per chunk and head, 16 tokens a wave, all value columns, so that a head's norm
 // stays in the wave.  The workgroups behind the chunks' ones: the step's last inputs into the convolution's ring.
+// Bound by the latency of its operands (the chunk's state, U and queries: 130 KB a workgroup): 3001 tokens of 16 heads
+// of 128 x 128 take 32 us with three workgroups a compute unit, 58 with one.
 template <typename T, int STEPS, int NE>
-__global__ __launch_bounds__(256) void delta_output_kernel(DeltaArgs a, DeltaWorkspace w) {
+__global__ __launch_bounds__(256, STEPS <= 4 && NE <= 8 ? 3 : 1) void delta_output_kernel(DeltaArgs a, DeltaWorkspace w) {
   constexpr uint32_t np = STEPS * 32;
   const uint32_t chunk = blockIdx.x, head = blockIdx.y;
   if (chunk >= w.chunks) {
@@ -805,7 +822,7 @@ __global__ __launch_bounds__(256) void delta_output_kernel(DeltaArgs a, DeltaWor
     for (uint32_t c = threadIdx.x; c < w.channels; c += 256) ring[c] = to_f32(input[c]);
     return;
   }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, column = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, column = lane & 15, quad = lane >> 4;
   const size_t each = (size_t)chunk * a.heads + head, plane = (size_t)Q * np, state_plane = (size_t)w.ep * np;
   const int token = wave * 16 + column;
   const uint32_t row = chunk * Q + token;
@@ -818,49 +835,69 @@ __global__ __launch_bounds__(256) void delta_output_kernel(DeltaArgs a, DeltaWor
   for (int s = 0; s < 2; ++s) {
     const f32x8 eight = *reinterpret_cast<const f32x8 *>(scores + s * 32);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) weight[s].set(e, eight[e]);
+    for (int e = 0; e < 8; e += 2) weight[s].set_pair(e, eight[e], eight[e + 1]);
   }
+  // A tile's operands are requested together, at scalar addresses and the lane's offset: a 64-bit address a lane for each
+  // of them, which is what pointers with the lane inside become, filled two hundred registers and left a workgroup a
+  // compute unit with four requests under way.
+  const T *states = static_cast<const T *>(w.states) + each * kPlanes<T> * state_plane;
+  const T *written = static_cast<const T *>(w.u) + each * kPlanes<T> * w.ep * Q;
+  const uint32_t lane_bytes = lane * 8 * sizeof(T);
+  auto at = [&](const T *uniform) { return reinterpret_cast<const T *>(reinterpret_cast<const char *>(uniform) + lane_bytes); };
+  const int tiles = (a.vdim + 15) / 16;
+  struct Operands {
+    WideFrag<T> state[STEPS], u[2];
+  };
+  auto load = [&](Operands &o, int t) {
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) o.state[s] = load_wide<T>(at(states + (size_t)t * 16 * np + s * 512), state_plane);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) o.u[s] = load_wide<T>(at(written + t * 16 * Q + s * 512), (size_t)w.ep * Q);
+  };
   f32x4 out[NE];
   float square = 0.0f;
 #pragma unroll
   for (int t = 0; t < NE; ++t) {
     out[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    if (t * 16 >= (int)a.vdim) continue;
-    const T *states = static_cast<const T *>(w.states) + each * kPlanes<T> * state_plane + (size_t)t * 16 * np + lane * 8;
+    Operands o;
+    load(o, min(t, tiles - 1));  // (a tile that is not there: the last again; a branch would spread the requests)
+    __builtin_amdgcn_sched_barrier(0);  // the requests stay ahead of the arithmetic
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s) out[t] = mma_wide_both(load_wide<T>(states + s * 512, state_plane), fq[s], out[t]);
-    const T *u = static_cast<const T *>(w.u) + each * kPlanes<T> * w.ep * Q + t * 16 * Q + lane * 8;
+    for (int s = 0; s < STEPS; ++s) out[t] = mma_wide_both(o.state[s], fq[s], out[t]);
 #pragma unroll
     for (int s = 0; s < 2; ++s)
       if (s * 32 <= wave * 16 + 15)  // the others come later than all of the wave's tokens
-        out[t] = mma_wide_both(load_wide<T>(u + s * 512, (size_t)w.ep * Q), weight[s], out[t]);
+        out[t] = mma_wide_both(o.u[s], weight[s], out[t]);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       if (t * 16 + quad * 4 + r < (int)a.vdim) square = fmaf(out[t][r], out[t][r], square);
+    __builtin_amdgcn_sched_barrier(0);
   }
   square += __shfl_xor(square, 16, 64);
   square += __shfl_xor(square, 32, 64);
   const float scale = a.out_scale / sqrtf(square / (float)a.vdim + a.epsilon);
   if (row >= a.m) return;
-  const T *gate = static_cast<const T *>(a.gate) + ((size_t)row * a.heads + head) * a.vdim;
-  T *target = static_cast<T *>(a.out) + (size_t)row * a.ld_out + (size_t)head * a.vdim;
+  // (the lane's four columns of a tile at one address and a constant)
+  const T *gate = static_cast<const T *>(a.gate) + ((size_t)row * a.heads + head) * a.vdim + quad * 4;
+  T *target = static_cast<T *>(a.out) + (size_t)row * a.ld_out + (size_t)head * a.vdim + quad * 4;
+  const uint16_t *norm = a.norm + quad * 4;
   typedef T x4 __attribute__((ext_vector_type(4)));
   const bool vec = a.vdim % 4 == 0 && a.ld_out % 4 == 0 && reinterpret_cast<size_t>(a.out) % sizeof(x4) == 0;
 #pragma unroll
   for (int t = 0; t < NE; ++t) {
-    const uint32_t v = t * 16 + quad * 4;
-    if (v >= a.vdim) continue;
+    const int left = (int)a.vdim - t * 16 - quad * 4;
+    if (left <= 0) continue;
     if (vec) {
-      const x4 g = *reinterpret_cast<const x4 *>(gate + v);
+      const x4 g = *reinterpret_cast<const x4 *>(gate + t * 16);
       x4 packed;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) packed[r] = (T)(out[t][r] * scale * bf16_at(a.norm, v + r) * sigmoid_f32(to_f32(g[r])));
-      *reinterpret_cast<x4 *>(target + v) = packed;
+      for (int r = 0; r < 4; ++r) packed[r] = (T)(out[t][r] * scale * bf16_at(norm, t * 16 + r) * sigmoid_f32(to_f32(g[r])));
+      *reinterpret_cast<x4 *>(target + t * 16) = packed;
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (v + r < a.vdim)
-          target[v + r] = (T)(out[t][r] * scale * bf16_at(a.norm, v + r) * sigmoid_f32(to_f32(gate[v + r])));
+        if (r < left)
+          target[t * 16 + r] = (T)(out[t][r] * scale * bf16_at(norm, t * 16 + r) * sigmoid_f32(to_f32(gate[t * 16 + r])));
     }
   }
 }
@@ -884,9 +921,14 @@ hipError_t run_scan(const DeltaArgs &a, const DeltaWorkspace &w, hipStream_t str
 template <typename T, int TAPS>
 hipError_t run_chunks(const DeltaArgs &a, const DeltaWorkspace &w, hipStream_t stream) {
   const dim3 grid(w.chunks, a.heads);
-  if (a.dim <= 64) delta_chunk_kernel<T, 1, TAPS><<<grid, 256, 0, stream>>>(a, w);
-  else if (a.dim <= 128) delta_chunk_kernel<T, 2, TAPS><<<grid, 256, 0, stream>>>(a, w);
-  else delta_chunk_kernel<T, 4, TAPS><<<grid, 256, 0, stream>>>(a, w);
+  // Heads of up to 128: a third workgroup a compute unit costs the registers' last ten a trip to scratch, and is the better
+  // one once two a compute unit do not hold them all (3001 tokens of 16 heads, 752 workgroups, 71 us for 98; of 8 heads,
+  // 376 workgroups, 48 for 45.5).  LDS (53 KB) holds three.  Heads of 64 fit anyway, wider ones take all registers.
+  const bool many = (uint64_t)w.chunks * a.heads > 2 * (uint64_t)device_compute_units();
+  if (a.dim <= 64) delta_chunk_kernel<T, 1, TAPS, 2><<<grid, 256, 0, stream>>>(a, w);
+  else if (a.dim <= 128 && many) delta_chunk_kernel<T, 2, TAPS, 3><<<grid, 256, 0, stream>>>(a, w);
+  else if (a.dim <= 128) delta_chunk_kernel<T, 2, TAPS, 2><<<grid, 256, 0, stream>>>(a, w);
+  else delta_chunk_kernel<T, 4, TAPS, 1><<<grid, 256, 0, stream>>>(a, w);
   return hipGetLastError();
 }
 
