@@ -241,11 +241,10 @@ __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int r = 0; r < 4; r += 2) {
-        const float p[2] = {exp2_raw(score[kt][r] - best), exp2_raw(score[kt][r + 1] - best)};
-        total += p[0];
-        total += p[1];
-        fp.set_pair(kt * 4 + r, p[0], p[1]);
+      for (int r = 0; r < 4; ++r) {
+        const float p = exp2_raw(score[kt][r] - best);
+        total += p;
+        fp.set(kt * 4 + r, p);
       }
     total += __shfl_xor(total, 16, 64);
     total += __shfl_xor(total, 32, 64);

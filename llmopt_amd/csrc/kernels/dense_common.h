@@ -59,11 +59,16 @@ struct WideFrag;
 template <>
 struct WideFrag<float> {
   f32x8 v;
+  __device__ __forceinline__ void set(int i, float x) { v[i] = x; }
   __device__ __forceinline__ void set_pair(int i, float x, float y) { v[i] = x, v[i + 1] = y; }
 };
 template <>
 struct WideFrag<__bf16> {
   bf16x8 hi, lo;
+  __device__ __forceinline__ void set(int i, float x) {
+    hi[i] = (__bf16)x;
+    lo[i] = (__bf16)(x - (float)hi[i]);
+  }
   // the elements of one register (i even), which share their conversions (set one at a time each takes its own)
   __device__ __forceinline__ void set_pair(int i, float x, float y) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));

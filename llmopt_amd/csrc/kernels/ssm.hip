@@ -341,8 +341,7 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
     for (int s = 0; s < 2; ++s) {
       WideFrag<T> fx;
 #pragma unroll
-      for (int e = 0; e < 8; e += 2)
-        fx.set_pair(e, to_f32(o.x[s][e]) * o.tail[s][e], to_f32(o.x[s][e + 1]) * o.tail[s][e + 1]);
+      for (int e = 0; e < 8; ++e) fx.set(e, to_f32(o.x[s][e]) * o.tail[s][e]);
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         if ((wave + 4 * t) * 16 < (int)w.np) state[t] = mma_wide_b(o.b[t][s], fx, state[t]);
@@ -399,15 +398,10 @@ __global__ __launch_bounds__(256) void ssm_output_kernel(SsmArgs a, SsmWorkspace
     const f32x8 sc = *reinterpret_cast<const f32x8 *>(score + j0), d = *reinterpret_cast<const f32x8 *>(dt + j0);
     const f32x8 high = *reinterpret_cast<const f32x8 *>(sum + j0), low = *reinterpret_cast<const f32x8 *>(sum + Q + j0);
 #pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      float two[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const float decayed = __expf((own_high - high[e + h]) + (own_low - low[e + h])) * d[e + h];
-        const int j = j0 + e + h;
-        two[h] = j > token ? 0.0f : fmaf(sc[e + h], decayed, j == token ? skip : 0.0f);
-      }
-      weight[s].set_pair(e, two[0], two[1]);
+    for (int e = 0; e < 8; ++e) {
+      const float decayed = __expf((own_high - high[e]) + (own_low - low[e])) * d[e];
+      const int j = j0 + e;
+      weight[s].set(e, j > token ? 0.0f : fmaf(sc[e], decayed, j == token ? skip : 0.0f));
     }
   }
   const float scale = __expf(own_high);
