@@ -76,8 +76,12 @@ void llmopt_hip_release_context(llmopt_hip_context *context);
 int llmopt_hip_device_name(llmopt_hip_context *context, char *out, size_t capacity);
 
 /* Runs later work of this context on an existing HIP stream (hipStream_t
- * passed as void*), e.g. PyTorch's current stream.  No reference counterpart:
- * Metal command queues are private to the context. */
+ * passed as void*), e.g. PyTorch's current stream; the stream before it is
+ * drained.  A stream that is being captured is refused (LLMOPT_ERR_INVALID)
+ * and its capture left as it is: a recorded launch would keep addresses of
+ * scratch memory that a later launch may move (the retained plans below are
+ * the graphs that follow it).  No reference counterpart: Metal command queues
+ * are private to the context. */
 int llmopt_hip_context_set_stream(llmopt_hip_context *context, void *hip_stream);
 /* Blocks until all work queued on the context's stream has finished. */
 int llmopt_hip_context_synchronize(llmopt_hip_context *context);
@@ -192,7 +196,8 @@ int llmopt_hip_commit_batch(llmopt_hip_batch *batch);
 /* caml_llmopt_metal_commit_batch_async (:1359-1370): launches without waiting. */
 int llmopt_hip_commit_batch_async(llmopt_hip_batch *batch);
 /* No reference counterpart: one kernel on device memory that the caller owns, launched on `hip_stream` (which becomes the
- * context's stream; another one is drained first) and not waited for.  The memory has to stay valid until the work
+ * context's stream; another one is drained first, and one that is being captured is refused, as by
+ * llmopt_hip_context_set_stream) and not waited for.  The memory has to stay valid until the work
  * queued on that stream so far is done.  Several threads may call it for one context. */
 int llmopt_hip_launch(llmopt_hip_library *library, const char *name, void *const *pointers, const size_t *lengths,
                       uint32_t count, const void *parameters, uint32_t parameter_bytes, void *hip_stream);

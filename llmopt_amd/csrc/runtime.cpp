@@ -312,17 +312,20 @@ int llmopt_hip_device_name(llmopt_hip_context *context, char *out, size_t capaci
 int llmopt_hip_context_set_stream(llmopt_hip_context *context, void *hip_stream) {
   if (context == nullptr) return fail(LLMOPT_ERR_FAILURE, "HIP context has been finalized");
   if (int status = use_device(context)) return status;
-  if (!context->owns_stream && context->stream == static_cast<hipStream_t>(hip_stream)) {
-    // Nothing changes, and launches stay ordered on the one stream: no reason to wait for it.  (A stream that is being
-    // captured is still turned down below: a recorded launch would keep the address of scratch memory that may move.)
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(context->stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone)
-      return LLMOPT_OK;
+  const hipStream_t stream = static_cast<hipStream_t>(hip_stream);
+  // Not a stream that is being captured, whether the context is on it already or not: a recorded launch would keep the
+  // addresses of the context's scratch memory, which a later launch may move.  Nothing is waited for on the way to the
+  // error, so that the capture goes on without this call.
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
+    return fail(LLMOPT_ERR_INVALID, "HIP context cannot launch on a stream that is being captured");
   }
+  // Nothing changes, and launches stay ordered on the one stream: no reason to wait for it.
+  if (!context->owns_stream && context->stream == stream) return LLMOPT_OK;
   LLMOPT_HIP_TRY(hipStreamSynchronize(context->stream), "HIP stream synchronize failed");
   if (context->owns_stream && context->stream) (void)hipStreamDestroy(context->stream);
-  context->stream = static_cast<hipStream_t>(hip_stream);
+  context->stream = stream;
   context->owns_stream = false;
   return LLMOPT_OK;
 }

@@ -94,3 +94,30 @@ def test_refused_shapes(op):
     with pytest.raises(RuntimeError):
         op(half(3, 64), torch.zeros((0, 32), dtype=torch.uint8, device=device), half(0, 1), None)
     assert op(half(0, 64), torch.zeros((8, 32), dtype=torch.uint8, device=device), half(8, 1), None).shape == (0, 8)
+
+
+@pytest.mark.parametrize("same", [False, True])
+def test_a_stream_under_capture_is_refused(op, same):
+    """The first call on a stream that is being captured, after calls on it or on another one, is an error that leaves
+    the capture whole: what else is recorded replays, and the operator goes on outside."""
+    rng = np.random.default_rng(4)
+    device = torch.device("cuda:0")
+    case = w4_case(rng, 8, 256, 14336)  # K split over workgroups: the context's scratch memory is in use
+    tensors = [torch.from_numpy(a).to(device) for a in case[:3]] + [None]
+    x = torch.arange(100, dtype=torch.float32, device=device)
+    torch.cuda.synchronize()
+    warm, captured = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(captured if same else warm):
+        op(*tensors)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=captured):
+        with pytest.raises(RuntimeError, match="captured"):
+            op(*tensors)
+        y = x + 1
+    for turn in range(3):
+        x += turn
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, x + 1)
+        assert_close_to_oracle(op(*tensors).cpu().numpy(), oracle.w4a16_linear(*case[:3], None), "after the capture")
