@@ -201,13 +201,17 @@ class DecodeStep:
         self.slot_offsets = b(np.asarray(slot_offsets, dtype=np.uint32))
         # What changes from step to step lies in one buffer, so that `seek` writes it at once: context lengths, slots of the
         # new tokens, and cosine rows, then sine rows (the fused launch takes those as one buffer).
-        words, trig_bytes = (4 * batch + 255) // 256 * 256, 2 * batch * c.head_dim * 2
+        # Arrays may be strided, and longer than the batch.
+        first_slots = np.asarray(new_slots, dtype=np.uint32)
+        words = (max(self.host_lengths.nbytes, first_slots.nbytes) + 255) // 256 * 256
+        trig_bytes = 2 * self.host_positions.size * c.head_dim * 2
         self.state = runtime.create_buffer(2 * words + trig_bytes)
         self._state_words = words
-        self.past_lengths, self.new_slots = self.state.view(0, 4 * batch), self.state.view(words, 4 * batch)
+        self.past_lengths = self.state.view(0, self.host_lengths.nbytes)
+        self.new_slots = self.state.view(words, first_slots.nbytes)
         self.trig = self.state.view(2 * words, trig_bytes)
         self.cos, self.sin = self.trig.view(0, trig_bytes // 2), self.trig.view(trig_bytes // 2, trig_bytes // 2)
-        self._write_state(np.asarray(past_lengths, dtype=np.uint32), np.asarray(new_slots, dtype=np.uint32), positions)
+        self._write_state(self.host_lengths, first_slots, self.host_positions)
         self.device = device_weights if device_weights is not None else {
             "embedding": b(weights["embedding"]),
             "final_norm": b(weights["final_norm"]),
@@ -426,9 +430,9 @@ class DecodeStep:
     def _write_state(self, lengths, new_slots, positions) -> None:
         words, cos_sin = self._state_words, rope_rows(self.config, positions)
         state = np.zeros(2 * words + cos_sin[0].nbytes * 2, dtype=np.uint8)
-        state[:4 * self.batch] = lengths.view(np.uint8)
-        state[words:words + 4 * self.batch] = np.ascontiguousarray(new_slots).view(np.uint8)
-        state[2 * words:] = np.concatenate(cos_sin).view(np.uint8).reshape(-1)
+        for at, part in ((0, lengths), (words, new_slots), (2 * words, np.concatenate(cos_sin))):
+            part = np.ascontiguousarray(part).reshape(-1).view(np.uint8)
+            state[at:at + part.size] = part
         self.state.write(state)
 
     def record(self, batch) -> None:
