@@ -384,11 +384,12 @@ hipError_t run_prefill_tile(const ChunkAttentionArgs &a, hipStream_t stream) {
 // 30.0; 2048 rows, 16 heads of 64 38.9 for 56.5) and for heads up to 64 always, whose stages are short and whose
 // keys are cheap to bring in twice (3001 rows, 16 heads of 64: the same 53 us either way).  Beyond that it brings
 // in twice the keys for nothing (3001 rows, 16 heads of 128: 102.7 us for 92.3; 2048 rows, 32 heads: 97.9 for 89.1).
+// A grid has at most 65536 rows of workgroups: portions of more 64-row tiles than that take the 128-row ones.
 template <typename T, int ND, int NE>
 hipError_t run_prefill(const ChunkAttentionArgs &a, hipStream_t stream) {
   if constexpr (sizeof(T) == 2 && ND <= 4 && NE <= 8) {
-    if constexpr (ND > 2 || NE > 4)
-      if ((uint64_t)a.heads * ((a.m + 127) / 128) > kCompute) return run_prefill_tile<T, ND, NE, 8, 1>(a, stream);
+    const bool many = (uint64_t)a.heads * ((a.m + 127) / 128) > kCompute;
+    if ((many && (ND > 2 || NE > 4)) || (a.m + 63) / 64 > 65536) return run_prefill_tile<T, ND, NE, 8, 1>(a, stream);
     return run_prefill_tile<T, ND, NE, 8, 2>(a, stream);
   } else {
     return run_prefill_tile<T, ND, NE, 4, 1>(a, stream);

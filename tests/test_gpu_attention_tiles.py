@@ -11,6 +11,7 @@ from llmopt_amd.safetensors_file import from_bfloat16, to_bfloat16
 from tests.gpu_util import u32s
 
 pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
 GRID = ((1, 1, 1), (256, 1, 1))
 
 
@@ -86,3 +87,25 @@ def test_tiles(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sli
         expected = weights @ values / total[:, None]
         error = np.abs(got[:, head] - expected)
         assert (error <= 2.0 ** -8 * np.abs(expected) + 2.0 ** -13 * np.abs(values).max()).all(), (head, error.max())
+
+
+def test_portion_of_more_tiles_than_a_grid_has_rows(runtime):
+    """64 * 65536 rows and a few: chunks of 64 stand alone, a thousand of them and the last ones against float64."""
+    m, dim, span = 64 * 65536 + 70, 32, 64
+    generator = torch.Generator(device="cuda").manual_seed(5)
+    rows = torch.randn(m, 3 * dim, generator=generator, device="cuda", dtype=torch.bfloat16)
+    step, sinks = torch.zeros(2, dtype=torch.int32, device="cuda"), torch.zeros(8, dtype=torch.bfloat16, device="cuda")
+    keys, values = (torch.zeros(span, dim, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    out = torch.full((m, dim), float("nan"), dtype=torch.bfloat16, device="cuda")
+    torch.cuda.synchronize()
+    wrap = lambda t: runtime.wrap(t.data_ptr(), t.numel() * t.element_size())
+    runtime.dispatch("llmopt_chunk_attention_bf16", [wrap(t) for t in (rows, sinks, step, keys, values, out)],
+                     u32s(m, 1, 1, dim, dim, span, span, 1, 0) + struct.pack("<ff", dim ** -0.5, 0.0), *GRID)
+    chunks = (m + span - 1) // span
+    for chunk in [0, 1, *torch.linspace(2, chunks - 4, 1000).long().tolist(), chunks - 3, chunks - 2, chunks - 1]:
+        part = rows[chunk * span:(chunk + 1) * span].double()
+        q, k, v = part[:, :dim], part[:, dim:2 * dim], part[:, 2 * dim:]
+        seen = torch.ones(len(part), len(part), dtype=torch.bool, device="cuda").tril()
+        expected = torch.softmax((q @ k.T * dim ** -0.5).masked_fill(~seen, float("-inf")), dim=1) @ v
+        error = (out[chunk * span:(chunk + 1) * span].double() - expected).abs()
+        assert (error <= 2.0 ** -8 * expected.abs() + 2.0 ** -13 * v.abs().max()).all(), (chunk, error.max())
