@@ -431,13 +431,14 @@ bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k) {
 // to 24 rows stay with the matrix-core GEMV, which streams them better.  Head with its argmax in rows / 2 tokens, us,
 // tiles / GEMV (rows, K, n): 10 x 576 x 49152 22.4 / 30.8, 64 x 576 x 49152 27 / 58, 128 x 576 x 49152 33 / 78,
 // 24 x 2048 x 32000 38.1 / 38.9, 32 x 2048 x 32000 39.1 / 47, 64 x 2048 x 32000 45 / 62, 24 x 4096 x 32000 68.3 / 61.3,
-// 32 x 4096 x 32000 69 / 90, 128 x 4096 x 32000 97 / 193, 64 x 8192 x 16000 122 / 231.
+// 32 x 4096 x 32000 69 / 90, 128 x 4096 x 32000 97 / 193, 64 x 8192 x 16000 122 / 231.  A tile's rows are a row of the
+// grid, which has at most 65536.
 Tile pick_pairs_tile(uint32_t rows, uint32_t n, uint32_t k) {
   const Tile small = pick_tile(rows, &n, 1, k);
   if (small != Tile::kNone) return small;
   if (k >= 1536 && rows <= 24) return Tile::kNone;
-  if (rows > 32 && rows_lds_bytes<64, 4, 2, 2>(k) <= kLdsBytes) return Tile::k64x128;
-  if (rows_lds_bytes<32, 2, 4, 2>(k) <= kLdsBytes) return Tile::k32x64;
+  if (rows > 32 && rows <= 65536 * 64 && rows_lds_bytes<64, 4, 2, 2>(k) <= kLdsBytes) return Tile::k64x128;
+  if (rows <= 65536 * 32 && rows_lds_bytes<32, 2, 4, 2>(k) <= kLdsBytes) return Tile::k32x64;
   return Tile::kNone;
 }
 

@@ -13,6 +13,7 @@ from tests.test_gpu_glue import check_tokens, lm_head_oracle, run_lm_head
 from tests.test_gpu_w4a16 import run_linear
 
 pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
 
 
 @pytest.fixture(scope="module")
@@ -166,3 +167,30 @@ def test_projection_with_rotation_and_pack(runtime, k, heads, kv_heads, dim, tok
     for name, two, one in zip(("queries", "keys", "values", "pool"), *results):
         np.testing.assert_array_equal(one, two, err_msg=name)
     assert np.isfinite(results[1][0].view(np.float16)).all()
+
+
+def test_logits_of_more_rows_than_a_grid_of_tiles_has():
+    """A hi and a lo row each of 32 * 65536 tokens and some: every token's logits against float64.  They are rounded to
+    half, 2^-11 of the value; the GEMV's weights are nibbles with a bias of up to 1032, which a second sum takes out
+    again: 64 additions of 2^-24 of sums up to 1040 times those of the activations each."""
+    from llmopt_amd.native import Runtime
+    runtime = Runtime()
+    m, n, k = 32 * 65536 + 40, 5, 64
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x = torch.randn(m, k, generator=g, device="cuda").half()
+    norm, scale = (torch.rand(*shape, generator=g, device="cuda").half() for shape in ((k,), (n, 1)))
+    packed = torch.randint(0, 256, (n, k // 2), generator=g, device="cuda").to(torch.uint8)
+    ids, logits = torch.zeros(m, dtype=torch.int32, device="cuda"), torch.full((m, n), float("nan"), device="cuda").half()
+    torch.cuda.synchronize()
+    wrap = lambda t: runtime.wrap(t.data_ptr(), t.numel() * t.element_size())
+    runtime.dispatch("llmopt_w4a16_lm_head_argmax_extra_f16", [wrap(t) for t in (x, norm, packed, scale, ids, logits)],
+                     u32s(m, n, k) + struct.pack("<f", 1e-5), (256, 1, 1), (256, 1, 1))
+    q = torch.stack([packed & 15, packed >> 4], dim=-1).reshape(n, k).double()
+    weight = torch.where(q >= 8, q - 16, q) * scale.double()
+    rows = x.double() / torch.sqrt(x.double().square().mean(1, keepdim=True) + 1e-5) * norm.double()
+    expected = rows @ weight.T
+    sums = 2 * 64 * 2.0 ** -24 * 1040 * rows.abs().sum(1, keepdim=True) * scale.double().T
+    assert ((logits.double() - expected).abs() <= 2.0 ** -11 * expected.abs() + sums).all()
+    chosen = expected.gather(1, ids.long()[:, None])[:, 0]
+    assert (chosen >= expected.max(1).values - 2 * sums.max(1).values).all()
+    runtime.close()
