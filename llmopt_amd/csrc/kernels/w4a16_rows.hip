@@ -27,6 +27,7 @@
 #include "kernels.h"
 #include "kernels_internal.h"
 #include "w4_common.h"
+#include "w4a16_rows_rule.h"
 
 namespace llmopt {
 namespace {
@@ -78,9 +79,6 @@ __device__ __forceinline__ h8_t w4_exact_natural(uint32_t word) {
   packed.w = __builtin_amdgcn_perm(p37, p26, 0x07060302u);
   return __builtin_bit_cast(h8_t, packed);
 }
-
-// Scales of a tile in LDS: blocks of eight columns by eight groups, a dword each.
-constexpr uint32_t scale_lds_bytes(uint32_t columns, uint32_t groups) { return columns / 8 * ((groups + 7) / 8) * 256; }
 
 template <int ROWS, int CT, int P, int STAGES, bool DUAL, class Params>
 __global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
@@ -324,21 +322,13 @@ __global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
   }
 }
 
-constexpr uint32_t kLdsBytes = 160 * 1024;
-
-template <int ROWS, int CT, int P, int STAGES>
-constexpr uint32_t rows_lds_bytes(uint32_t k) {
-  const uint32_t ring = STAGES * (ROWS * P * 128 + CT * 32 * P * 32), sums = P * ROWS * CT * 32 * 4;
-  return scale_lds_bytes(CT * 32, k / 64) + (ring > sums ? ring : sums);
-}
-
 template <int ROWS, int CT, int P, int STAGES, bool DUAL, class Params>
 hipError_t run_rows(Params &p, hipStream_t stream) {
   const auto kernel = w4a16_rows_kernel<ROWS, CT, P, STAGES, DUAL, Params>;
   const uint32_t bytes = rows_lds_bytes<ROWS, CT, P, STAGES>(p.k);
-  if (bytes > kLdsBytes) return hipErrorInvalidValue;
+  if (bytes > kRowsLdsBytes) return hipErrorInvalidValue;
   static bool allowed[kMaxDevices] = {};
-  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), kLdsBytes, allowed)) return status;
+  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), kRowsLdsBytes, allowed)) return status;
   constexpr uint32_t columns = DUAL ? CT * 16 : CT * 32;
   uint32_t tiles = 0;
   for (uint32_t i = 0; i < p.segments; ++i) tiles += p.tiles[i] = (p.n[i] + columns - 1) / columns;
@@ -346,107 +336,35 @@ hipError_t run_rows(Params &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The tile of a launch; kNone: the 128 x 128 and larger tiles of w4a16_gemm.hip.
-enum class Tile { kNone, k32x32, k32x64, k32x64Deep, k32x64Long, k64x64, k64x128 };
-
-// A launch takes as long as one workgroup while each CU has at most one of them, and a workgroup the longer the larger
-// its tile and K are (us, K = 576 / 2048 / 4096 / 8192, one round): 32 x 32 4.1 / 6.1 / 8.8 / 13.7, 32 x 64 4.6 / 7.8 /
-// 11.3 / 21, 64 x 64 5.9 / 10.3 / 16.4 / 29, 64 x 128 7.1 / 14.9 / 25.7 / 47.  So: the smallest tile that needs one round,
-// and the large tiles once even 64 x 128 would need a second.  Measured against those, us (m, K, n):
-// 24 x 4096 x 14336 13.3 / 30.8; 24 x 4096 x 4096 8.7 / 16.7; 64 x 14336 x 4096 23.5 / 38.5; 128 x 4096 x 4096 11.8 / 17.4;
-// 200 x 4096 x 4096 16.9 / 21.4; 512 x 4096 x 4096 28 / 33; 1024 x 2048 x 2048 16.5 / 28.3; 700 x 576 x 576 5.3 / 9.5;
-// 700 x 1536 x 576 7.0 / 13.7; 700 x 576 x 1536 7.4 / 9.5; beyond: 200 x 4096 x 14336 53.6 / 43.5, 700 x 8192 x 2048 47 / 42.
-// With few steps (K < 1536) three workgroups of the shallow 32 x 64 ring share a CU: two rounds of it are still fast.
-Tile pick_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint32_t k) {
-  auto rounds = [&](uint32_t rows, uint32_t columns) {
-    uint64_t tiles = 0;
-    for (uint32_t i = 0; i < matrices; ++i) tiles += (n[i] + columns - 1) / columns;
-    return (double)(tiles * ((m + rows - 1) / rows)) / device_compute_units();
-  };
-  if (rounds(32, 32) <= 1 && rows_lds_bytes<32, 1, 8, 3>(k) <= kLdsBytes) return Tile::k32x32;
-  if (k < 1536) {
-    if (rounds(32, 64) <= 2) return Tile::k32x64;
-  } else if (rounds(32, 64) <= 1) {
-    if (rows_lds_bytes<32, 2, 8, 3>(k) <= kLdsBytes) return Tile::k32x64Deep;
-    if (rows_lds_bytes<32, 2, 4, 4>(k) <= kLdsBytes) return Tile::k32x64Long;
-  }
-  if (k >= 1536 && k <= 6144 && rounds(64, 64) <= 1) return Tile::k64x64;
-  if (k <= 6144 && rounds(64, 128) <= 1.125) return Tile::k64x128;
-  return Tile::kNone;
-}
-
-// The same for a gated pair, by output columns (half of a tile's).  The large tiles take two accumulator sets, so the
-// small ones win for longer: us (m, K, n) 24 x 4096 x 14336 20.4 / 61.7, 64 x 4096 x 4096 12.6 / 58, 64 x 8192 x 2048
-// 26 / 108, 128 x 4096 x 14336 55 / 64 (two rounds), 512 x 2048 x 2048 15.9 / 31.8, 1024 x 2048 x 2048 26.3 / 34.4,
-// 700 x 576 x 1536 10.9 / 16.0; beyond: 200 x 4096 x 14336 105 / 78, 2048 x 2048 x 2048 49 / 46.
-Tile pick_pair_tile(uint32_t m, uint32_t n, uint32_t k) {
-  auto rounds = [&](uint32_t rows, uint32_t columns) {
-    return (double)((uint64_t)((n + columns - 1) / columns) * ((m + rows - 1) / rows)) / device_compute_units();
-  };
-  if (rounds(32, 32) <= 1) {
-    if (k < 1536) return Tile::k32x64;
-    if (rows_lds_bytes<32, 2, 8, 3>(k) <= kLdsBytes) return Tile::k32x64Deep;
-    if (rows_lds_bytes<32, 2, 4, 4>(k) <= kLdsBytes) return Tile::k32x64Long;
-  }
-  if (rounds(64, 32) <= 1 && rows_lds_bytes<64, 2, 4, 3>(k) <= kLdsBytes) return Tile::k64x64;
-  if (rounds(32, 32) <= 2 && k <= 8192) return Tile::k32x64;
-  if (rounds(64, 64) <= 2 && rows_lds_bytes<64, 4, 2, 2>(k) <= kLdsBytes) return Tile::k64x128;
-  return Tile::kNone;
-}
-
 template <bool DUAL, class Params>
-hipError_t launch_tile(Tile tile, Params &p, hipStream_t stream) {
+hipError_t launch_tile(RowsTile tile, Params &p, hipStream_t stream) {
   switch (tile) {
-    case Tile::k32x32:
+    case RowsTile::k32x32:
       if constexpr (!DUAL && std::is_same_v<Params, RowsParams>) return run_rows<32, 1, 8, 3, false>(p, stream);
       return hipErrorInvalidValue;
-    case Tile::k32x64: return run_rows<32, 2, 4, 2, DUAL>(p, stream);
-    case Tile::k32x64Deep: return run_rows<32, 2, 8, 3, DUAL>(p, stream);
-    case Tile::k32x64Long: return run_rows<32, 2, 4, 4, DUAL>(p, stream);
-    case Tile::k64x64: return run_rows<64, 2, 4, 3, DUAL>(p, stream);
-    case Tile::k64x128: return run_rows<64, 4, 2, 2, DUAL>(p, stream);
-    case Tile::kNone: break;
+    case RowsTile::k32x64: return run_rows<32, 2, 4, 2, DUAL>(p, stream);
+    case RowsTile::k32x64Deep: return run_rows<32, 2, 8, 3, DUAL>(p, stream);
+    case RowsTile::k32x64Long: return run_rows<32, 2, 4, 4, DUAL>(p, stream);
+    case RowsTile::k64x64: return run_rows<64, 2, 4, 3, DUAL>(p, stream);
+    case RowsTile::k64x128: return run_rows<64, 4, 2, 2, DUAL>(p, stream);
+    case RowsTile::kNone: break;
   }
   return hipErrorInvalidValue;
 }
+
+static_assert(kRowGroup == kGemvMaxRows);
+
+uint32_t cus() { return (uint32_t)device_compute_units(); }
 
 bool pieces_aligned(const void *x, const void *w) {
   return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
 }
 
-// The copies name a tile's bytes by 32-bit offsets from its first row.
-bool offsets_fit(uint32_t k) { return k <= (1u << 24); }
-
-// Up to about 48k outputs of small matrices the matrix-core GEMV's row groups are as fast or faster (us, m x K x n:
-// 24 x 2048 x 2048 5.4 / 6.1, 40 x 576 x 576 3.8 / 4.1; 100 x 576 x 960 6.1 / 4.2, 40 x 2048 x 2048 6.4 / 6.1).
-constexpr uint64_t kRowGroupOutputs = 49152;
-
-bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k) {
-  if (m <= kGemvMaxRows || !offsets_fit(k)) return false;
-  return !(w4a16_gemv_mfma_row_groups_ok(m, columns, k) && m * columns <= kRowGroupOutputs);
-}
-
-// Logits: as above while the launch is about one round of small tiles.  Beyond, where the 128 x 128 tiles have no float32
-// results, the tile that decodes the weights least often of those whose scales fit LDS beside the ring; with a long K up
-// to 24 rows stay with the matrix-core GEMV, which streams them better.  Head with its argmax in rows / 2 tokens, us,
-// tiles / GEMV (rows, K, n): 10 x 576 x 49152 22.4 / 30.8, 64 x 576 x 49152 27 / 58, 128 x 576 x 49152 33 / 78,
-// 24 x 2048 x 32000 38.1 / 38.9, 32 x 2048 x 32000 39.1 / 47, 64 x 2048 x 32000 45 / 62, 24 x 4096 x 32000 68.3 / 61.3,
-// 32 x 4096 x 32000 69 / 90, 128 x 4096 x 32000 97 / 193, 64 x 8192 x 16000 122 / 231.  A tile's rows are a row of the
-// grid, which has at most 65536.
-Tile pick_pairs_tile(uint32_t rows, uint32_t n, uint32_t k) {
-  const Tile small = pick_tile(rows, &n, 1, k);
-  if (small != Tile::kNone) return small;
-  if (k >= 1536 && rows <= 24) return Tile::kNone;
-  if (rows > 32 && rows <= 65536 * 64 && rows_lds_bytes<64, 4, 2, 2>(k) <= kLdsBytes) return Tile::k64x128;
-  if (rows <= 65536 * 32 && rows_lds_bytes<32, 2, 4, 2>(k) <= kLdsBytes) return Tile::k32x64;
-  return Tile::kNone;
-}
-
 }  // namespace
 
 bool w4a16_rows_ok(const W4LinearArgs &a) {
-  return a.y_f32 == nullptr && rows_wanted(a.m, a.n, a.k) && pieces_aligned(a.x, a.w.weight) &&
-         pick_tile(a.m, &a.n, 1, a.k) != Tile::kNone;
+  return a.y_f32 == nullptr && pieces_aligned(a.x, a.w.weight) &&
+         linear_rows_tile(a.m, a.n, a.k, cus()) != RowsTile::kNone;
 }
 
 hipError_t launch_w4a16_rows_linear(const W4LinearArgs &a, hipStream_t stream) {
@@ -461,11 +379,11 @@ hipError_t launch_w4a16_rows_linear(const W4LinearArgs &a, hipStream_t stream) {
   p.segments = 1;
   p.addend = a.has_addend ? a.addend : nullptr;
   p.addend_stride = a.addend_row_stride;
-  return launch_tile<false>(pick_tile(a.m, &a.n, 1, a.k), p, stream);
+  return launch_tile<false>(linear_rows_tile(a.m, a.n, a.k, cus()), p, stream);
 }
 
 bool w4a16_rows_pairs_ok(const uint16_t *x, const W4Matrix &w, uint32_t rows, uint32_t n, uint32_t k) {
-  return rows_wanted(rows, n, k) && pieces_aligned(x, w.weight) && pick_pairs_tile(rows, n, k) != Tile::kNone;
+  return pieces_aligned(x, w.weight) && logits_rows_tile(rows, n, k, cus()) != RowsTile::kNone;
 }
 
 hipError_t launch_w4a16_rows_pairs(const uint16_t *x, const W4Matrix &w, float *y, uint32_t rows, uint32_t n, uint32_t k,
@@ -479,14 +397,13 @@ hipError_t launch_w4a16_rows_pairs(const uint16_t *x, const W4Matrix &w, float *
   p.n[0] = n;
   p.segments = 1;
   p.pairs = y;
-  return launch_tile<false>(pick_pairs_tile(rows, n, k), p, stream);
+  return launch_tile<false>(logits_rows_tile(rows, n, k, cus()), p, stream);
 }
 
 bool w4a16_rows_ok(const W4QkvArgs &a) {
   for (int i = 0; i < 3; ++i)
     if (a.n[i] == 0 || !pieces_aligned(a.x, a.w[i].weight)) return false;
-  return a.norm.weight == nullptr && rows_wanted(a.m, (uint64_t)a.n[0] + a.n[1] + a.n[2], a.k) &&
-         pick_tile(a.m, a.n, 3, a.k) != Tile::kNone;
+  return a.norm.weight == nullptr && qkv_rows_tile(a.m, a.n, a.k, cus()) != RowsTile::kNone;
 }
 
 hipError_t launch_w4a16_rows_qkv(const W4QkvArgs &a, hipStream_t stream) {
@@ -501,21 +418,11 @@ hipError_t launch_w4a16_rows_qkv(const W4QkvArgs &a, hipStream_t stream) {
     p.n[i] = a.n[i];
   }
   p.segments = 3;
-  return launch_tile<false>(pick_tile(a.m, a.n, 3, a.k), p, stream);
-}
-
-// A tile of whole heads: where the rule takes half a head's columns, the 64-column one, whose few microseconds more are
-// less than another launch.
-static Tile pick_pack_tile(const W4QkvArgs &a) {
-  const Tile tile = pick_tile(a.m, a.n, 3, a.k);
-  if (tile != Tile::k32x32) return tile;
-  if (a.k < 1536) return Tile::k32x64;
-  if (rows_lds_bytes<32, 2, 8, 3>(a.k) <= kLdsBytes) return Tile::k32x64Deep;
-  return rows_lds_bytes<32, 2, 4, 4>(a.k) <= kLdsBytes ? Tile::k32x64Long : Tile::kNone;
+  return launch_tile<false>(qkv_rows_tile(a.m, a.n, a.k, cus()), p, stream);
 }
 
 bool w4a16_rows_pack_ok(const W4QkvArgs &a, const RotaryPackArgs &r) {
-  return w4a16_rows_ok(a) && r.rotary.batches == 1 && r.rotary.width == 64 && pick_pack_tile(a) != Tile::kNone;
+  return w4a16_rows_ok(a) && r.rotary.batches == 1 && r.rotary.width == 64 && pack_rows_tile(a.m, a.n, a.k, cus()) != RowsTile::kNone;
 }
 
 hipError_t launch_w4a16_rows_qkv_pack(const W4QkvArgs &a, const RotaryPackArgs &r, hipStream_t stream) {
@@ -538,12 +445,12 @@ hipError_t launch_w4a16_rows_qkv_pack(const W4QkvArgs &a, const RotaryPackArgs &
   p.token_stride = r.pack.token_stride;
   p.token_elements = r.pack.token_elements;
   for (int i = 0; i < 2; ++i) p.segment_offset[i] = r.pack.segment_offset[i];
-  return launch_tile<false>(pick_pack_tile(a), p, stream);
+  return launch_tile<false>(pack_rows_tile(a.m, a.n, a.k, cus()), p, stream);
 }
 
 bool w4a16_rows_ok(const W4DualSwigluArgs &a) {
-  return a.norm.weight == nullptr && rows_wanted(a.m, 2ull * a.n, a.k) && pieces_aligned(a.x, a.gate.weight) &&
-         pieces_aligned(a.x, a.up.weight) && pick_pair_tile(a.m, a.n, a.k) != Tile::kNone;
+  return a.norm.weight == nullptr && pieces_aligned(a.x, a.gate.weight) &&
+         pieces_aligned(a.x, a.up.weight) && gated_rows_tile(a.m, a.n, a.k, cus()) != RowsTile::kNone;
 }
 
 hipError_t launch_w4a16_rows_dual_swiglu(const W4DualSwigluArgs &a, hipStream_t stream) {
@@ -558,7 +465,7 @@ hipError_t launch_w4a16_rows_dual_swiglu(const W4DualSwigluArgs &a, hipStream_t 
   p.y[0] = a.product;
   p.n[0] = a.n;
   p.segments = 1;
-  return launch_tile<true>(pick_pair_tile(a.m, a.n, a.k), p, stream);
+  return launch_tile<true>(gated_rows_tile(a.m, a.n, a.k, cus()), p, stream);
 }
 
 }  // namespace llmopt

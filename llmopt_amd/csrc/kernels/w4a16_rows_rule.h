@@ -1,0 +1,123 @@
+// Which W4A16 products take the small tiles of w4a16_rows.hip, and which tile: rules on sizes alone (and the number of
+// compute units), without HIP, so that a host test can ask them.
+#pragma once
+
+#include <stdint.h>
+
+namespace llmopt {
+
+// Rows by columns of a workgroup's tile; kNone: another kernel (the matrix-core GEMV's row groups, or the 128 x 128 and
+// larger tiles of w4a16_gemm.hip).
+enum class RowsTile { kNone, k32x32, k32x64, k32x64Deep, k32x64Long, k64x64, k64x128 };
+
+// The matrix-core GEMV: rows of one group, and the longest K that one workgroup covers.
+constexpr uint32_t kRowGroup = 8, kRowGroupK = 4096;
+// More rows than a group, as groups of one grid: small matrices, whose weights every group decodes again.
+inline bool row_groups_fit(uint32_t m, uint64_t columns, uint32_t k) {
+  return m > kRowGroup && m <= 128 && k <= kRowGroupK && columns * k / 2 <= (4u << 20);
+}
+
+constexpr uint32_t kRowsLdsBytes = 160 * 1024;
+
+// Scales of a tile in LDS: blocks of eight columns by eight groups, a dword each.
+constexpr uint32_t scale_lds_bytes(uint32_t columns, uint32_t groups) { return columns / 8 * ((groups + 7) / 8) * 256; }
+
+template <int ROWS, int CT, int P, int STAGES>
+constexpr uint32_t rows_lds_bytes(uint32_t k) {
+  const uint32_t ring = STAGES * (ROWS * P * 128 + CT * 32 * P * 32), sums = P * ROWS * CT * 32 * 4;
+  return scale_lds_bytes(CT * 32, k / 64) + (ring > sums ? ring : sums);
+}
+
+// Up to about 48k outputs of small matrices the matrix-core GEMV's row groups are as fast or faster (us, m x K x n:
+// 24 x 2048 x 2048 5.4 / 6.1, 40 x 576 x 576 3.8 / 4.1; 100 x 576 x 960 6.1 / 4.2, 40 x 2048 x 2048 6.4 / 6.1).
+constexpr uint64_t kRowGroupOutputs = 49152;
+
+// (The copies name a tile's bytes by 32-bit offsets from its first row.)
+inline bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k) {
+  if (m <= kRowGroup || k > (1u << 24)) return false;
+  return !(row_groups_fit(m, columns, k) && m * columns <= kRowGroupOutputs);
+}
+
+// A launch takes as long as one workgroup while each CU has at most one of them, and a workgroup the longer the larger
+// its tile and K are (us, K = 576 / 2048 / 4096 / 8192, one round): 32 x 32 4.1 / 6.1 / 8.8 / 13.7, 32 x 64 4.6 / 7.8 /
+// 11.3 / 21, 64 x 64 5.9 / 10.3 / 16.4 / 29, 64 x 128 7.1 / 14.9 / 25.7 / 47.  So: the smallest tile that needs one round,
+// and the large tiles once even 64 x 128 would need a second.  Measured against those, us (m, K, n):
+// 24 x 4096 x 14336 13.3 / 30.8; 24 x 4096 x 4096 8.7 / 16.7; 64 x 14336 x 4096 23.5 / 38.5; 128 x 4096 x 4096 11.8 / 17.4;
+// 200 x 4096 x 4096 16.9 / 21.4; 512 x 4096 x 4096 28 / 33; 1024 x 2048 x 2048 16.5 / 28.3; 700 x 576 x 576 5.3 / 9.5;
+// 700 x 1536 x 576 7.0 / 13.7; 700 x 576 x 1536 7.4 / 9.5; beyond: 200 x 4096 x 14336 53.6 / 43.5, 700 x 8192 x 2048 47 / 42.
+// With few steps (K < 1536) three workgroups of the shallow 32 x 64 ring share a CU: two rounds of it are still fast.
+inline RowsTile rows_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint32_t k, uint32_t cus) {
+  auto rounds = [&](uint32_t rows, uint32_t columns) {
+    uint64_t tiles = 0;
+    for (uint32_t i = 0; i < matrices; ++i) tiles += (n[i] + columns - 1) / columns;
+    return (double)(tiles * ((m + rows - 1) / rows)) / cus;
+  };
+  if (rounds(32, 32) <= 1 && rows_lds_bytes<32, 1, 8, 3>(k) <= kRowsLdsBytes) return RowsTile::k32x32;
+  if (k < 1536) {
+    if (rounds(32, 64) <= 2) return RowsTile::k32x64;
+  } else if (rounds(32, 64) <= 1) {
+    if (rows_lds_bytes<32, 2, 8, 3>(k) <= kRowsLdsBytes) return RowsTile::k32x64Deep;
+    if (rows_lds_bytes<32, 2, 4, 4>(k) <= kRowsLdsBytes) return RowsTile::k32x64Long;
+  }
+  if (k >= 1536 && k <= 6144 && rounds(64, 64) <= 1) return RowsTile::k64x64;
+  if (k <= 6144 && rounds(64, 128) <= 1.125) return RowsTile::k64x128;
+  return RowsTile::kNone;
+}
+
+inline RowsTile linear_rows_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
+  return rows_wanted(m, n, k) ? rows_tile(m, &n, 1, k, cus) : RowsTile::kNone;
+}
+
+inline RowsTile qkv_rows_tile(uint32_t m, const uint32_t *n, uint32_t k, uint32_t cus) {
+  return rows_wanted(m, (uint64_t)n[0] + n[1] + n[2], k) ? rows_tile(m, n, 3, k, cus) : RowsTile::kNone;
+}
+
+// QKV with the rotation and the Q8 pack: a tile of whole heads.  Where the rule takes half a head's columns, the 64-column
+// one, whose few microseconds more are less than another launch.
+inline RowsTile pack_rows_tile(uint32_t m, const uint32_t *n, uint32_t k, uint32_t cus) {
+  const RowsTile tile = qkv_rows_tile(m, n, k, cus);
+  if (tile != RowsTile::k32x32) return tile;
+  if (k < 1536) return RowsTile::k32x64;
+  if (rows_lds_bytes<32, 2, 8, 3>(k) <= kRowsLdsBytes) return RowsTile::k32x64Deep;
+  return rows_lds_bytes<32, 2, 4, 4>(k) <= kRowsLdsBytes ? RowsTile::k32x64Long : RowsTile::kNone;
+}
+
+// A gated pair, by output columns (half of a tile's).  The large tiles take two accumulator sets, so the
+// small ones win for longer: us (m, K, n) 24 x 4096 x 14336 20.4 / 61.7, 64 x 4096 x 4096 12.6 / 58, 64 x 8192 x 2048
+// 26 / 108, 128 x 4096 x 14336 55 / 64 (two rounds), 512 x 2048 x 2048 15.9 / 31.8, 1024 x 2048 x 2048 26.3 / 34.4,
+// 700 x 576 x 1536 10.9 / 16.0; beyond: 200 x 4096 x 14336 105 / 78, 2048 x 2048 x 2048 49 / 46.
+inline RowsTile gated_rows_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
+  if (!rows_wanted(m, 2ull * n, k)) return RowsTile::kNone;
+  auto rounds = [&](uint32_t rows, uint32_t columns) {
+    return (double)((uint64_t)((n + columns - 1) / columns) * ((m + rows - 1) / rows)) / cus;
+  };
+  if (rounds(32, 32) <= 1) {
+    if (k < 1536) return RowsTile::k32x64;
+    if (rows_lds_bytes<32, 2, 8, 3>(k) <= kRowsLdsBytes) return RowsTile::k32x64Deep;
+    if (rows_lds_bytes<32, 2, 4, 4>(k) <= kRowsLdsBytes) return RowsTile::k32x64Long;
+  }
+  if (rounds(64, 32) <= 1 && rows_lds_bytes<64, 2, 4, 3>(k) <= kRowsLdsBytes) return RowsTile::k64x64;
+  if (rounds(32, 32) <= 2 && k <= 8192) return RowsTile::k32x64;
+  if (rounds(64, 64) <= 2 && rows_lds_bytes<64, 4, 2, 2>(k) <= kRowsLdsBytes) return RowsTile::k64x128;
+  return RowsTile::kNone;
+}
+
+// Logits of rows / 2 tokens (a hi and a lo row each): as above while the launch is about one round of small tiles.  Beyond,
+// where the 128 x 128 tiles have no float32
+// results, the tile that decodes the weights least often of those whose scales fit LDS beside the ring; with a long K up
+// to 24 rows stay with the matrix-core GEMV, which streams them better.  Head with its argmax in rows / 2 tokens, us,
+// tiles / GEMV (rows, K, n): 10 x 576 x 49152 22.4 / 30.8, 64 x 576 x 49152 27 / 58, 128 x 576 x 49152 33 / 78,
+// 24 x 2048 x 32000 38.1 / 38.9, 32 x 2048 x 32000 39.1 / 47, 64 x 2048 x 32000 45 / 62, 24 x 4096 x 32000 68.3 / 61.3,
+// 32 x 4096 x 32000 69 / 90, 128 x 4096 x 32000 97 / 193, 64 x 8192 x 16000 122 / 231.  A tile's rows are a row of the
+// grid, which has at most 65536.
+inline RowsTile logits_rows_tile(uint32_t rows, uint32_t n, uint32_t k, uint32_t cus) {
+  if (!rows_wanted(rows, n, k)) return RowsTile::kNone;
+  const RowsTile small = rows_tile(rows, &n, 1, k, cus);
+  if (small != RowsTile::kNone) return small;
+  if (k >= 1536 && rows <= 24) return RowsTile::kNone;
+  if (rows > 32 && rows <= 65536 * 64 && rows_lds_bytes<64, 4, 2, 2>(k) <= kRowsLdsBytes) return RowsTile::k64x128;
+  if (rows <= 65536 * 32 && rows_lds_bytes<32, 2, 4, 2>(k) <= kRowsLdsBytes) return RowsTile::k32x64;
+  return RowsTile::kNone;
+}
+
+}  // namespace llmopt

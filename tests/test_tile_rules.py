@@ -1,0 +1,51 @@
+"""Which tile a product takes, asked of the rules that the launches use: every tile is reached by a size that the GPU tests
+run, and sizes that were measured on both sides of a line lie on the faster one (256 compute units)."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from tests import test_gpu_w4a16_rows
+
+CUS = 256
+KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "kernels")
+SOURCE = """
+#include "w4a16_rows_rule.h"
+using namespace llmopt;
+extern "C" {
+int linear_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)linear_rows_tile(m, n, k, cus); }
+int gated_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)gated_rows_tile(m, n, k, cus); }
+int logits_tile(uint32_t tokens, uint32_t n, uint32_t k, uint32_t cus) { return (int)logits_rows_tile(2 * tokens, n, k, cus); }
+int qkv_tile(uint32_t m, uint32_t q, uint32_t kv, uint32_t k, uint32_t cus) {
+  const uint32_t n[3] = {q, kv, kv};
+  return (int)qkv_rows_tile(m, n, k, cus);
+}
+}
+"""
+NONE, K32X32, K32X64, K32X64_DEEP, K32X64_LONG, K64X64, K64X128 = range(7)
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("rules")
+    (folder / "rules.cpp").write_text(SOURCE)
+    library = str(folder / "rules.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", KERNELS, str(folder / "rules.cpp"),
+                    "-o", library], check=True)
+    return ctypes.CDLL(library)
+
+
+def sizes(test, names):
+    """The sizes that a GPU test is run at."""
+    return next(mark.args[1] for mark in test.pytestmark if mark.name == "parametrize" and mark.args[0] == names)
+
+
+def test_gpu_tests_reach_every_tile(rules):
+    tests = test_gpu_w4a16_rows
+    assert {rules.linear_tile(m, n, k, CUS) for m, n, k in sizes(tests.test_small_tiles, "m,n,k")} >= set(range(1, 7))
+    assert {rules.gated_tile(m, n, k, CUS) for m, n, k in sizes(tests.test_small_pair_tiles, "m,n,k")} >= set(range(2, 7))
+    three = sizes(tests.test_small_tiles_over_three_matrices, "m,k,sizes")
+    assert {rules.qkv_tile(m, n[0], n[1], k, CUS) for m, k, n in three} >= {K32X32, K32X64, K32X64_DEEP, K64X128}
+    heads = {rules.logits_tile(m, n, k, CUS) for m, n, k in sizes(tests.test_logits_of_several_rows, "m,n,k")}
+    assert heads >= {K32X32, K32X64, K64X128}
