@@ -28,14 +28,27 @@ constexpr uint32_t rows_lds_bytes(uint32_t k) {
   return scale_lds_bytes(CT * 32, k / 64) + (ring > sums ? ring : sums);
 }
 
-// Up to about 48k outputs of small matrices the matrix-core GEMV's row groups are as fast or faster (us, m x K x n:
-// 24 x 2048 x 2048 5.4 / 6.1, 40 x 576 x 576 3.8 / 4.1; 100 x 576 x 960 6.1 / 4.2, 40 x 2048 x 2048 6.4 / 6.1).
+// The matrix-core GEMV's row groups are the better ones while they are few: up to two workgroups a CU, counted as eight
+// rows by sixteen columns, of which a gated pair has both matrices in one.  The tiles' shortest launch is longer than
+// theirs, more so with a long K; a third workgroup on a CU adds a whole round to them.  Each call behind the launch that
+// writes its activations, us (m x K x n, GEMV / tiles):
+// at 512 workgroups and below: 64 x 1024 x 1024 6.1 / 6.3, 32 x 2048 x 2048 7.2 / 8.1, 64 x 4096 x 1024 9.2 / 10.8,
+// 16 x 2048 x 4096 7.1 / 8.0, 80 x 3072 x 768 8.2 / 9.4; pairs 64 x 1024 x 1024 6.7 / 7.0, 32 x 2048 x 2048 8.3 / 9.4,
+// 56 x 1536 x 576 6.8 / 8.5, 64 x 4096 x 1024 11.9 / 13.4, 128 x 2048 x 512 8.8 / 9.7;
+// above: 72 x 1024 x 1024 7.0 / 6.3, 33 x 2048 x 2048 8.3 / 8.0, 72 x 4096 x 1024 12.3 / 11.0, 96 x 3072 x 768 10.3 / 9.6;
+// pairs 72 x 1024 x 1024 7.9 / 7.1, 40 x 2048 x 2048 10.8 / 9.5, 128 x 1536 x 576 11.2 / 8.8.
+// Up to K = 512 a tile's launch is as short: there, and for the three matrices of QKV, whose groups are three launches'
+// worth, the line is 48k outputs (pairs 64 x 512 x 1024 6.0 / 5.9, 33 x 512 x 2048 6.5 / 5.9).
 constexpr uint64_t kRowGroupOutputs = 49152;
 
+inline bool row_groups_few(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
+  return k > 512 && (uint64_t)((m + kRowGroup - 1) / kRowGroup) * ((n + 15) / 16) <= 2ull * cus;
+}
+
 // (The copies name a tile's bytes by 32-bit offsets from its first row.)
-inline bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k) {
+inline bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k, bool few) {
   if (m <= kRowGroup || k > (1u << 24)) return false;
-  return !(row_groups_fit(m, columns, k) && m * columns <= kRowGroupOutputs);
+  return !(row_groups_fit(m, columns, k) && (few || m * columns <= kRowGroupOutputs));
 }
 
 // A launch takes as long as one workgroup while each CU has at most one of them, and a workgroup the longer the larger
@@ -65,11 +78,11 @@ inline RowsTile rows_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint
 }
 
 inline RowsTile linear_rows_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
-  return rows_wanted(m, n, k) ? rows_tile(m, &n, 1, k, cus) : RowsTile::kNone;
+  return rows_wanted(m, n, k, row_groups_few(m, n, k, cus)) ? rows_tile(m, &n, 1, k, cus) : RowsTile::kNone;
 }
 
 inline RowsTile qkv_rows_tile(uint32_t m, const uint32_t *n, uint32_t k, uint32_t cus) {
-  return rows_wanted(m, (uint64_t)n[0] + n[1] + n[2], k) ? rows_tile(m, n, 3, k, cus) : RowsTile::kNone;
+  return rows_wanted(m, (uint64_t)n[0] + n[1] + n[2], k, false) ? rows_tile(m, n, 3, k, cus) : RowsTile::kNone;
 }
 
 // QKV with the rotation and the Q8 pack: a tile of whole heads.  Where the rule takes half a head's columns, the 64-column
@@ -87,7 +100,7 @@ inline RowsTile pack_rows_tile(uint32_t m, const uint32_t *n, uint32_t k, uint32
 // 26 / 108, 128 x 4096 x 14336 55 / 64 (two rounds), 512 x 2048 x 2048 15.9 / 31.8, 1024 x 2048 x 2048 26.3 / 34.4,
 // 700 x 576 x 1536 10.9 / 16.0; beyond: 200 x 4096 x 14336 105 / 78, 2048 x 2048 x 2048 49 / 46.
 inline RowsTile gated_rows_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
-  if (!rows_wanted(m, 2ull * n, k)) return RowsTile::kNone;
+  if (!rows_wanted(m, 2ull * n, k, row_groups_few(m, n, k, cus))) return RowsTile::kNone;
   auto rounds = [&](uint32_t rows, uint32_t columns) {
     return (double)((uint64_t)((n + columns - 1) / columns) * ((m + rows - 1) / rows)) / cus;
   };
@@ -111,7 +124,7 @@ inline RowsTile gated_rows_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus
 // 32 x 4096 x 32000 69 / 90, 128 x 4096 x 32000 97 / 193, 64 x 8192 x 16000 122 / 231.  A tile's rows are a row of the
 // grid, which has at most 65536.
 inline RowsTile logits_rows_tile(uint32_t rows, uint32_t n, uint32_t k, uint32_t cus) {
-  if (!rows_wanted(rows, n, k)) return RowsTile::kNone;
+  if (!rows_wanted(rows, n, k, false)) return RowsTile::kNone;
   const RowsTile small = rows_tile(rows, &n, 1, k, cus);
   if (small != RowsTile::kNone) return small;
   if (k >= 1536 && rows <= 24) return RowsTile::kNone;

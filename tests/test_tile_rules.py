@@ -49,3 +49,24 @@ def test_gpu_tests_reach_every_tile(rules):
     assert {rules.qkv_tile(m, n[0], n[1], k, CUS) for m, k, n in three} >= {K32X32, K32X64, K32X64_DEEP, K64X128}
     heads = {rules.logits_tile(m, n, k, CUS) for m, n, k in sizes(tests.test_logits_of_several_rows, "m,n,k")}
     assert heads >= {K32X32, K32X64, K64X128}
+
+
+@pytest.mark.parametrize("m,k,n", [(64, 1024, 1024), (32, 2048, 2048), (64, 4096, 1024), (16, 2048, 4096), (80, 3072, 768),
+                                   (40, 1536, 1536), (128, 4096, 512), (40, 1280, 1280)])
+def test_few_row_groups(rules, m, k, n):
+    """Up to two groups a CU the GEMV is the faster one, beyond that a tile is."""
+    assert rules.linear_tile(m, n, k, CUS) == NONE
+    assert rules.linear_tile(m + 24, n, k, CUS) != NONE or m + 24 > 128
+    assert rules.linear_tile(m + 24, n + 512, k, CUS) != NONE
+
+
+@pytest.mark.parametrize("m,k,n", [(64, 1024, 1024), (32, 2048, 2048), (56, 1536, 576), (64, 4096, 1024), (128, 2048, 512),
+                                   (16, 1024, 4096), (40, 768, 768), (128, 1024, 512), (112, 4096, 256)])
+def test_few_row_groups_of_pairs(rules, m, k, n):
+    assert rules.gated_tile(m, n, k, CUS) == NONE
+
+
+@pytest.mark.parametrize("m,k,n", [(72, 1024, 1024), (40, 2048, 2048), (72, 4096, 1024), (128, 1536, 576), (64, 512, 1024),
+                                   (33, 512, 2048), (16, 2048, 4096)])
+def test_pairs_beyond_the_row_groups(rules, m, k, n):
+    assert rules.gated_tile(m, n, k, CUS) != NONE
