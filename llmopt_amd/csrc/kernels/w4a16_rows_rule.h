@@ -57,9 +57,7 @@ inline bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k, bool few) {
 // and the large tiles once even 64 x 128 would need a second.  Measured against those, us (m, K, n):
 // 24 x 4096 x 14336 13.3 / 30.8; 24 x 4096 x 4096 8.7 / 16.7; 64 x 14336 x 4096 23.5 / 38.5; 128 x 4096 x 4096 11.8 / 17.4;
 // 200 x 4096 x 4096 16.9 / 21.4; 512 x 4096 x 4096 28 / 33; 1024 x 2048 x 2048 16.5 / 28.3; 700 x 576 x 576 5.3 / 9.5;
-// 700 x 1536 x 576 7.0 / 13.7; 700 x 576 x 1536 7.4 / 9.5; beyond: 200 x 4096 x 14336 53.6 / 43.5, 700 x 8192 x 2048 47 / 42,
-// and a second round of a few tiles: 700 x 1472 x 3000 (264 tiles of 64 x 128) 19.2 / 17.0, 700 x 4096 x 3072 (264) 53.2 /
-// 45.5, 384 x 4096 x 6144 (288) 53.4 / 45.2.
+// 700 x 1536 x 576 7.0 / 13.7; 700 x 576 x 1536 7.4 / 9.5; beyond: 200 x 4096 x 14336 53.6 / 43.5, 700 x 8192 x 2048 47 / 42.
 // With few steps (K < 1536) three workgroups of the shallow 32 x 64 ring share a CU: two rounds of it are still fast.
 inline RowsTile rows_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint32_t k, uint32_t cus) {
   auto rounds = [&](uint32_t rows, uint32_t columns) {
@@ -75,7 +73,7 @@ inline RowsTile rows_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint
     if (rows_lds_bytes<32, 2, 4, 4>(k) <= kRowsLdsBytes) return RowsTile::k32x64Long;
   }
   if (k >= 1536 && k <= 6144 && rounds(64, 64) <= 1) return RowsTile::k64x64;
-  if (k <= 6144 && rounds(64, 128) <= 1) return RowsTile::k64x128;
+  if (k <= 6144 && rounds(64, 128) <= 1.125) return RowsTile::k64x128;
   return RowsTile::kNone;
 }
 

@@ -70,10 +70,3 @@ def test_few_row_groups_of_pairs(rules, m, k, n):
                                    (33, 512, 2048), (16, 2048, 4096)])
 def test_pairs_beyond_the_row_groups(rules, m, k, n):
     assert rules.gated_tile(m, n, k, CUS) != NONE
-
-
-@pytest.mark.parametrize("m,k,n", [(700, 1472, 3000), (700, 4096, 3072), (384, 4096, 6144), (768, 3072, 3072), (384, 1024, 6144)])
-def test_no_second_round_of_small_tiles(rules, m, k, n):
-    """A few tiles more than compute units take two rounds: the large tiles."""
-    assert rules.linear_tile(m, n, k, CUS) == NONE
-    assert rules.qkv_tile(m, n // 2, n // 4, k, CUS) == NONE
