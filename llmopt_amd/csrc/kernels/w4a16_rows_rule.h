@@ -54,10 +54,16 @@ inline bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k, bool few) {
 // A launch takes as long as one workgroup while each CU has at most one of them, and a workgroup the longer the larger
 // its tile and K are (us, K = 576 / 2048 / 4096 / 8192, one round): 32 x 32 4.1 / 6.1 / 8.8 / 13.7, 32 x 64 4.6 / 7.8 /
 // 11.3 / 21, 64 x 64 5.9 / 10.3 / 16.4 / 29, 64 x 128 7.1 / 14.9 / 25.7 / 47.  So: the smallest tile that needs one round,
-// and the large tiles once even 64 x 128 would need a second.  Measured against those, us (m, K, n):
+// and the large tiles once even 64 x 128 would need more than an eighth of a second one.  Measured against those, us (m, K,
+// n):
 // 24 x 4096 x 14336 13.3 / 30.8; 24 x 4096 x 4096 8.7 / 16.7; 64 x 14336 x 4096 23.5 / 38.5; 128 x 4096 x 4096 11.8 / 17.4;
 // 200 x 4096 x 4096 16.9 / 21.4; 512 x 4096 x 4096 28 / 33; 1024 x 2048 x 2048 16.5 / 28.3; 700 x 576 x 576 5.3 / 9.5;
 // 700 x 1536 x 576 7.0 / 13.7; 700 x 576 x 1536 7.4 / 9.5; beyond: 200 x 4096 x 14336 53.6 / 43.5, 700 x 8192 x 2048 47 / 42.
+// At the line the small tiles are not the faster ones, but the more exact ones: the large tiles round q * s to half, 2.8e-4
+// off float64 for 2.1e-4.  The first tiles of a second round, 700 x 1472 x 3000 (264 of 64 x 128) 19.2 / 17.0, 700 x 4096 x
+// 3072 (264) 53.2 / 45.5, 384 x 4096 x 6144 (288) 53.4 / 45.2; a long K that the large tiles split over workgroups while
+// half the CUs have none of them, 300 x 3072 x 4096 22.3 / 21.4, 300 x 4096 x 4096 28.8 / 28.0, 200 x 6144 x 6144 42.1 /
+// 38.7, 600 x 6144 x 2048 42.5 / 32.6.
 // With few steps (K < 1536) three workgroups of the shallow 32 x 64 ring share a CU: two rounds of it are still fast.
 inline RowsTile rows_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint32_t k, uint32_t cus) {
   auto rounds = [&](uint32_t rows, uint32_t columns) {
