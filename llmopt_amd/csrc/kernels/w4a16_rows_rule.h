@@ -121,17 +121,19 @@ inline RowsTile gated_rows_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus
   return RowsTile::kNone;
 }
 
-// Logits of rows / 2 tokens (a hi and a lo row each): as above while the launch is about one round of small tiles.  Beyond,
-// where the 128 x 128 tiles have no float32
-// results, the tile that decodes the weights least often of those whose scales fit LDS beside the ring; with a long K up
-// to 24 rows stay with the matrix-core GEMV, which streams them better.  Head with its argmax in rows / 2 tokens, us,
-// tiles / GEMV (rows, K, n): 10 x 576 x 49152 22.4 / 30.8, 64 x 576 x 49152 27 / 58, 128 x 576 x 49152 33 / 78,
-// 24 x 2048 x 32000 38.1 / 38.9, 32 x 2048 x 32000 39.1 / 47, 64 x 2048 x 32000 45 / 62, 24 x 4096 x 32000 68.3 / 61.3,
-// 32 x 4096 x 32000 69 / 90, 128 x 4096 x 32000 97 / 193, 64 x 8192 x 16000 122 / 231.  A tile's rows are a row of the
-// grid, which has at most 65536.
+// Logits of rows / 2 tokens (a hi and a lo row each).  The tile is the one above while the launch is about one round, and
+// beyond, where the 128 x 128 tiles have no float32 results, the one that decodes the weights least often of those whose
+// scales fit LDS beside the ring.  With a long K a few rows stay with the matrix-core GEMV, which streams the weights better
+// than a tile that is mostly padding.  Head with its argmax behind the launch that writes its rows, us, GEMV / tiles (tokens,
+// K, n): to the GEMV 8 x 2048 x 32000 44.1 / 48.7, 12 x 2048 x 32000 47.1 / 48.9 (64 x 128 tiles), 8 x 3072 x 32000 56 / 62,
+// 8 x 4096 x 16384 52.6 / 62.6, 12 x 4096 x 32000 77 / 82, 8 x 8192 x 8192 82 / 90, 16 x 2048 x 2048 27.1 / 28.1 (two GEMV
+// workgroups a CU); to the tiles 5 x 576 x 49152 32.9 / 24.6, 32 x 576 x 49152 61 / 31, 12 x 1536 x 32000 42.1 / 38.0,
+// 12 x 2048 x 16384 39.6 / 37.0, 16 x 2048 x 32000 56.7 / 49.0, 12 x 4096 x 16384 64.8 / 62.4, 20 x 4096 x 32000 110 / 83,
+// 64 x 4096 x 32000 197 / 107, 16 x 8192 x 8192 107 / 90.  A tile's rows are a row of the grid, which has at most 65536.
 inline RowsTile logits_rows_tile(uint32_t rows, uint32_t n, uint32_t k, uint32_t cus) {
-  if (!rows_wanted(rows, n, k, false)) return RowsTile::kNone;
+  if (!rows_wanted(rows, n, k, k >= 1280 && rows <= 32 && row_groups_few(rows, n, k, cus))) return RowsTile::kNone;
   const RowsTile small = rows_tile(rows, &n, 1, k, cus);
+  if (k >= 2048 && (rows <= 16 || (rows <= 24 && small == RowsTile::k64x128))) return RowsTile::kNone;
   if (small != RowsTile::kNone) return small;
   if (k >= 1536 && rows <= 24) return RowsTile::kNone;
   if (rows > 32 && rows <= 65536 * 64 && rows_lds_bytes<64, 4, 2, 2>(k) <= kRowsLdsBytes) return RowsTile::k64x128;

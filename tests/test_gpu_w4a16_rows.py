@@ -101,7 +101,7 @@ def test_small_tiles_over_three_matrices(runtime, m, k, sizes):
 # matrix-core GEMV on the other side of the rule (few rows, long K)
 @pytest.mark.parametrize("m,n,k", [
     (30, 2047, 64), (5, 33001, 576), (16, 16387, 576), (17, 33003, 320), (130, 10001, 576), (13, 24001, 1600),
-    (40, 20002, 1536), (12, 24001, 1536)])
+    (40, 20002, 1536), (12, 24001, 1536), (8, 16401, 2048), (12, 33001, 2112)])
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
 def test_logits_of_several_rows(runtime, m, n, k, dtype):
     rng = np.random.default_rng(m * 31 + n)

@@ -48,7 +48,7 @@ def test_gpu_tests_reach_every_tile(rules):
     three = sizes(tests.test_small_tiles_over_three_matrices, "m,k,sizes")
     assert {rules.qkv_tile(m, n[0], n[1], k, CUS) for m, k, n in three} >= {K32X32, K32X64, K32X64_DEEP, K64X128}
     heads = {rules.logits_tile(m, n, k, CUS) for m, n, k in sizes(tests.test_logits_of_several_rows, "m,n,k")}
-    assert heads >= {K32X32, K32X64, K64X128}
+    assert heads >= {NONE, K32X32, K32X64, K64X128}
 
 
 @pytest.mark.parametrize("m,k,n", [(64, 1024, 1024), (32, 2048, 2048), (64, 4096, 1024), (16, 2048, 4096), (80, 3072, 768),
@@ -70,3 +70,13 @@ def test_few_row_groups_of_pairs(rules, m, k, n):
                                    (33, 512, 2048), (16, 2048, 4096)])
 def test_pairs_beyond_the_row_groups(rules, m, k, n):
     assert rules.gated_tile(m, n, k, CUS) != NONE
+
+
+@pytest.mark.parametrize("tokens,k,n,tiles", [
+    (8, 2048, 32000, False), (12, 2048, 32000, False), (8, 3072, 32000, False), (8, 4096, 16384, False), (12, 4096, 32000, False),
+    (8, 8192, 8192, False), (16, 2048, 2048, False), (5, 2048, 16384, False), (4, 2048, 32000, False),
+    (5, 576, 49152, True), (32, 576, 49152, True), (12, 1536, 32000, True), (12, 2048, 16384, True), (16, 2048, 32000, True),
+    (12, 4096, 16384, True), (20, 4096, 32000, True), (64, 4096, 32000, True), (16, 8192, 8192, True), (20, 4096, 8192, True)])
+def test_logits(rules, tokens, k, n, tiles):
+    """Few rows and a long K stay with the GEMV also where 64 x 128 tiles would be one round."""
+    assert (rules.logits_tile(tokens, n, k, CUS) != NONE) == tiles
