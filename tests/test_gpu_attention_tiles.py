@@ -89,6 +89,39 @@ def test_tiles(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sli
         assert (error <= 2.0 ** -8 * np.abs(expected) + 2.0 ** -13 * np.abs(values).max()).all(), (head, error.max())
 
 
+# rows, heads, kv_heads, dim, span, position of the first row: tiles in the order of their keys (several rounds of up to 64
+# tiles, a chunk's end among them: 5, 16 and 64 tiles), more tiles than are ranked, one chunk, one round
+@pytest.mark.parametrize("m,heads,kv,dim,span,first", [
+    (300, 64, 8, 64, 512, 3000), (300, 64, 8, 128, 100, 37), (1024, 32, 8, 64, 700, 650), (4096, 8, 2, 32, 1000, 999),
+    (4090, 16, 2, 32, 63, 5), (4100, 8, 2, 32, 1000, 7), (700, 64, 8, 64, 2048, 100), (200, 4, 2, 64, 64, 10)])
+def test_float32_portions_over_the_ends_of_chunks(runtime, m, heads, kv, dim, span, first):
+    """Against float64: sums of up to 1000 weights and 128 products in float32, and exponentials a few units off, move a
+    weighted mean by less than 2^-15 of the largest value."""
+    g = torch.Generator(device="cuda").manual_seed(m + heads)
+    normal = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    rows, ring_k, ring_v = normal(m, (heads + 2 * kv) * dim), normal(kv, span, dim), normal(kv, span, dim)
+    out, sinks = torch.full((m, heads, dim), float("nan"), device="cuda"), torch.zeros(heads, device="cuda").bfloat16()
+    step = torch.tensor([first, 0], dtype=torch.int32, device="cuda")
+    at = torch.arange(first, first + m, device="cuda")
+    begin = first - first % span
+    past = torch.arange(begin, first, device="cuda")
+    places = torch.cat([past, at])
+    seen = (places[None] <= at[:, None]) & (places[None] // span == at[:, None] // span)
+    split = lambda a, h: a.double().view(m, h, dim)
+    q, k, v = split(rows[:, :heads * dim], heads), split(rows[:, heads * dim:(heads + kv) * dim], kv), split(rows[:, (heads + kv) * dim:], kv)
+    old_k, old_v = ring_k[:, past % span].double(), ring_v[:, past % span].double()
+    torch.cuda.synchronize()
+    wrap = lambda t: runtime.wrap(t.data_ptr(), t.numel() * t.element_size())
+    runtime.dispatch("llmopt_chunk_attention_f32", [wrap(t) for t in (rows, sinks, step, ring_k, ring_v, out)],
+                     u32s(m, heads, kv, dim, dim, span, span, 1, 0) + struct.pack("<ff", dim ** -0.5, 0.0), *GRID)
+    for head in range(heads):
+        group = head // (heads // kv)
+        keys, values = torch.cat([old_k[group], k[:, group]]), torch.cat([old_v[group], v[:, group]])
+        score = (q[:, head] @ keys.T * dim ** -0.5).masked_fill(~seen, float("-inf"))
+        error = (out[:, head].double() - torch.softmax(score, dim=1) @ values).abs().max()
+        assert error <= 2.0 ** -15 * values.abs().max(), (head, error)  # (a row that no tile wrote is NaN)
+
+
 def test_portion_of_more_tiles_than_a_grid_has_rows(runtime):
     """64 * 65536 rows and a few: chunks of 64 stand alone, a thousand of them and the last ones against float64."""
     m, dim, span = 64 * 65536 + 70, 32, 64
