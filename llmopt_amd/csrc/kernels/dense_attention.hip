@@ -14,6 +14,7 @@
 //    (any D up to 512, every option); the direct restatement.
 #include <algorithm>
 
+#include "dense_attention_rule.h"
 #include "kernels.h"
 #include "kernels_internal.h"
 #include "w4_common.h"
@@ -904,12 +905,8 @@ hipError_t launch_dense_attention(const DenseAttentionArgs &a, hipStream_t strea
       }
       if (geometry.key_split) {
         const uint32_t grid = (uint32_t)((a.query_length + 31) / 32) * a.heads * a.batches;
-        // One workgroup per CU that walks several stages: eight waves and 256-key stages (128 KB) halve the walk again
-        // (us, query rows / keys / heads, eight / four waves: 700 / 700 / 9 10.2 / 11.5, 900 / 900 / 9 11.7 / 14.5,
-        // 64 / 2000 / 9 15.1 / 17.3, 400 / 4000 / 9 29.8 / 40.5).  Walks of a few stages are as short either way (512 / 512 /
-        // 9 8.4 / 8.3), and where two workgroups would share a CU that room is worth more (700 / 700 / 32 20.6 / 14.0,
-        // 2048 / 2048 / 9 26.7 / 20.0).  With a mask the map of stages counts in 128 keys.
-        if (a.head_dim == 64 && mask == 0 && a.key_length > 512 && grid <= (uint32_t)device_compute_units() * 9 / 8)
+        if (eight_wave_slabs(a.head_dim, mask != 0, a.causal != 0, a.query_length, a.key_length, a.past_length, grid,
+                             (uint32_t)device_compute_units()))
           return launch_tile32_instance<64, 8, 256, 0, true>(grid, scheduled, stream);
         if (a.head_dim == 64) return launch_tile32<64, 4, 128, true>(mask_kind, grid, scheduled, stream);
         return launch_tile32<128, 4, 128, true>(mask_kind, grid, scheduled, stream);

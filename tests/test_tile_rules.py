@@ -11,12 +11,16 @@ from tests import test_gpu_w4a16_rows
 CUS = 256
 KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "kernels")
 SOURCE = """
+#include "dense_attention_rule.h"
 #include "w4a16_rows_rule.h"
 using namespace llmopt;
 extern "C" {
 int linear_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)linear_rows_tile(m, n, k, cus); }
 int gated_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)gated_rows_tile(m, n, k, cus); }
 int logits_tile(uint32_t tokens, uint32_t n, uint32_t k, uint32_t cus) { return (int)logits_rows_tile(2 * tokens, n, k, cus); }
+int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, uint32_t heads, uint32_t cus) {
+  return eight_wave_slabs(64, false, causal != 0, rows, keys, past, (rows + 31) / 32 * heads, cus);
+}
 int qkv_tile(uint32_t m, uint32_t q, uint32_t kv, uint32_t k, uint32_t cus) {
   const uint32_t n[3] = {q, kv, kv};
   return (int)qkv_rows_tile(m, n, k, cus);
@@ -80,3 +84,15 @@ def test_pairs_beyond_the_row_groups(rules, m, k, n):
 def test_logits(rules, tokens, k, n, tiles):
     """Few rows and a long K stay with the GEMV also where 64 x 128 tiles would be one round."""
     assert (rules.logits_tile(tokens, n, k, CUS) != NONE) == tiles
+
+
+@pytest.mark.parametrize("causal,rows,keys,past,heads,eight", [
+    (1, 700, 700, 0, 9, 1), (1, 900, 900, 0, 9, 1), (1, 64, 2000, 1936, 9, 1), (1, 400, 4000, 3600, 9, 1), (0, 32, 4096, 0, 9, 1),
+    (1, 1000, 1000, 0, 9, 1), (0, 512, 560, 0, 16, 1), (1, 512, 1024, 512, 16, 1),
+    # a second round
+    (0, 560, 560, 0, 16, 0), (1, 560, 560, 0, 16, 0), (0, 1000, 1000, 0, 9, 0), (1, 1025, 1025, 0, 9, 0),
+    (1, 512, 512, 0, 9, 0), (1, 700, 700, 0, 32, 0), (1, 2048, 2048, 0, 9, 0),
+    # keys beyond the causal limit of the last row are not walked
+    (1, 32, 4096, 0, 9, 0), (1, 64, 2000, 0, 16, 0), (1, 100, 520, 0, 3, 0), (1, 32, 4096, 224, 9, 0), (1, 32, 4096, 225, 9, 1), (1, 400, 4000, 0, 9, 1)])
+def test_eight_waves_a_slab(rules, causal, rows, keys, past, heads, eight):
+    assert rules.eight_waves(causal, rows, keys, past, heads, CUS) == eight
