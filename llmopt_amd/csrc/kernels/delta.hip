@@ -25,6 +25,7 @@
 // cores as a high and a low part.  Position 0 starts from a zero state and zero history.
 #include <algorithm>
 
+#include "delta_rule.h"
 #include "dense.h"
 #include "dense_common.h"
 #include "kernels_internal.h"
@@ -921,10 +922,7 @@ hipError_t run_scan(const DeltaArgs &a, const DeltaWorkspace &w, hipStream_t str
 template <typename T, int TAPS>
 hipError_t run_chunks(const DeltaArgs &a, const DeltaWorkspace &w, hipStream_t stream) {
   const dim3 grid(w.chunks, a.heads);
-  // Heads of up to 128: a third workgroup a compute unit costs the registers' last ten a trip to scratch, and is the better
-  // one once two a compute unit do not hold them all (3001 tokens of 16 heads, 752 workgroups, 71 us for 98; of 8 heads,
-  // 376 workgroups, 48 for 45.5).  LDS (53 KB) holds three.  Heads of 64 fit anyway, wider ones take all registers.
-  const bool many = (uint64_t)w.chunks * a.heads > 2 * (uint64_t)device_compute_units();
+  const bool many = three_delta_workgroups((uint64_t)w.chunks * a.heads, (uint32_t)device_compute_units());
   if (a.dim <= 64) delta_chunk_kernel<T, 1, TAPS, 2><<<grid, 256, 0, stream>>>(a, w);
   else if (a.dim <= 128 && many) delta_chunk_kernel<T, 2, TAPS, 3><<<grid, 256, 0, stream>>>(a, w);
   else if (a.dim <= 128) delta_chunk_kernel<T, 2, TAPS, 2><<<grid, 256, 0, stream>>>(a, w);

@@ -11,6 +11,7 @@ from tests import test_gpu_w4a16_rows
 CUS = 256
 KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "kernels")
 SOURCE = """
+#include "delta_rule.h"
 #include "dense_attention_rule.h"
 #include "w4a16_rows_rule.h"
 using namespace llmopt;
@@ -20,6 +21,9 @@ int gated_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)g
 int logits_tile(uint32_t tokens, uint32_t n, uint32_t k, uint32_t cus) { return (int)logits_rows_tile(2 * tokens, n, k, cus); }
 int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, uint32_t heads, uint32_t cus) {
   return eight_wave_slabs(64, false, causal != 0, rows, keys, past, (rows + 31) / 32 * heads, cus);
+}
+int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
+  return three_delta_workgroups((tokens + 63) / 64 * heads, cus);
 }
 int qkv_tile(uint32_t m, uint32_t q, uint32_t kv, uint32_t k, uint32_t cus) {
   const uint32_t n[3] = {q, kv, kv};
@@ -96,3 +100,10 @@ def test_logits(rules, tokens, k, n, tiles):
     (1, 32, 4096, 0, 9, 0), (1, 64, 2000, 0, 16, 0), (1, 100, 520, 0, 3, 0), (1, 32, 4096, 224, 9, 0), (1, 32, 4096, 225, 9, 1), (1, 400, 4000, 0, 9, 1)])
 def test_eight_waves_a_slab(rules, causal, rows, keys, past, heads, eight):
     assert rules.eight_waves(causal, rows, keys, past, heads, CUS) == eight
+
+
+@pytest.mark.parametrize("tokens,heads,three", [(3001, 16, 1), (2115, 16, 1), (4096, 32, 1), (3001, 32, 1), (3001, 8, 0),
+                                                (2048, 16, 0), (4096, 16, 0), (1000, 64, 0), (100, 4, 0)])
+def test_three_workgroups_of_the_delta_rule(rules, tokens, heads, three):
+    """Where they save a round, and only there."""
+    assert rules.three_workgroups(tokens, heads, CUS) == three
