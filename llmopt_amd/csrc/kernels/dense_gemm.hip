@@ -15,10 +15,10 @@
 //  * workgroups are dealt to the XCDs in contiguous runs (blockIdx % 8 is the XCD), and inside a run
 //    eight row tiles share a column of weight tiles: both operands are re-read from that XCD's L2.
 #include <algorithm>
-#include <cmath>
 
 #include "dense.h"
 #include "dense_common.h"
+#include "dense_tile_rule.h"
 #include "kernels_internal.h"
 
 namespace llmopt {
@@ -496,55 +496,23 @@ hipError_t pick_routed(const DenseLinearArgs &a, hipStream_t stream) {
   return a.f32 ? run_registers<float, 64, GATED, true>(a, stream) : run_registers<__bf16, 64, GATED, true>(a, stream);
 }
 
-// Tiles, and what a round of them takes on 256 CUs at K = 2048 (us, weights from HBM; a round's time goes with K): with
-// one workgroup on a CU, and with two where the tile's ring leaves room for them.  The eight-wave tiles keep two stages of
-// copies under way instead of one, which covers the trip to HBM when a CU has no second workgroup to fill the wait.
-struct TileRound {
-  uint32_t rows, columns;
-  float one, two;  // two == 0: the ring takes the CU
-};
-constexpr TileRound kTileRounds[] = {
-    {256, 256, 53.0f, 0.0f},  // 8 waves, 2 stages
-    {128, 128, 31.0f, 38.0f}, // 4 waves, 2 stages
-    {192, 128, 34.0f, 52.0f}, // 4 waves, 2 stages
-    {128, 192, 35.0f, 55.0f}, // 4 waves, 2 stages
-    {192, 128, 29.0f, 0.0f},  // 8 waves, 3 stages
-    {128, 128, 23.0f, 0.0f},  // 8 waves, 3 stages
-    {64, 128, 15.3f, 0.0f},   // 8 waves, 4 stages
-    {64, 64, 11.2f, 17.0f},   // 4 waves, 4 stages
-    {32, 64, 8.5f, 13.7f},    // 4 waves, 6 stages
-};
-
-// The tile with the least time by these.  Measured, us (m x n x k), before (the largest tile that gives every CU work) and
-// now: 2048 x 2048 x 4096 58 / 47, 2048 x 2048 x 8192 97 / 86, 2048 x 8576 x 2048 94 / 80, 2048 x 6144 x 2048 69 / 56,
-// 3001 x 2048 x 4096 67 / 63, 1024 x 2048 x 4096 34 / 31, 512 x 6144 x 2048 28 / 23; 3001 x 9504 x 2048 118, 512 x 2048 x
-// 4096 22, 64 x 4384 x 1024 7.0 as before.
 template <int GATED>
 hipError_t pick_gemm(const DenseLinearArgs &a, hipStream_t stream) {
   if (a.f32) return run_registers<float, 32, GATED, false>(a, stream);
   if (a.k % kStageK != 0 || a.ldx % 8 != 0) return run_registers<__bf16, 32, GATED, false>(a, stream);
-  const uint64_t columns = (uint64_t)a.n * (GATED ? 2 : 1), cus = (uint64_t)device_compute_units();
-  int best = 0;
-  float least = INFINITY;
-  for (int i = 0; i < (int)(sizeof(kTileRounds) / sizeof(kTileRounds[0])); ++i) {
-    const TileRound &t = kTileRounds[i];
-    const uint64_t tiles = ((a.m + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns);
-    const uint64_t slots = t.two > 0.0f ? 2 * cus : cus, rest = tiles % slots;
-    const float full = t.two > 0.0f ? t.two : t.one;
-    const float time = (float)(tiles / slots) * full + (rest == 0 ? 0.0f : rest <= cus ? t.one : t.two);
-    if (time < least) least = time, best = i;
+  switch (dense_tile(a.m, (uint64_t)a.n * (GATED ? 2 : 1), a.k, (uint32_t)device_compute_units())) {
+    case DenseTile::k256x256: return run_direct<256, 256, 2, 8, 2, GATED, false>(a, stream);
+    case DenseTile::k128x128: return run_direct<128, 128, 2, 4, 2, GATED, false>(a, stream);
+    case DenseTile::k192x128: return run_direct<192, 128, 2, 4, 2, GATED, false>(a, stream);
+    case DenseTile::k128x192: return run_direct<128, 192, 2, 4, 2, GATED, false>(a, stream);
+    case DenseTile::k192x128Eight: return run_direct<192, 128, 2, 8, 3, GATED, false>(a, stream);
+    case DenseTile::k128x128Eight: return run_direct<128, 128, 4, 8, 3, GATED, false>(a, stream);
+    case DenseTile::k64x128Eight: return run_direct<64, 128, 2, 8, 4, GATED, false>(a, stream);
+    case DenseTile::k64x64: return run_direct<64, 64, 2, 4, 4, GATED, false>(a, stream);
+    case DenseTile::k32x64: return run_direct<32, 64, 2, 4, 6, GATED, false>(a, stream);
+    case DenseTile::k64x128: return run_direct<64, 128, 2, 4, 3, GATED, false>(a, stream);
   }
-  switch (best) {
-    case 0: return run_direct<256, 256, 2, 8, 2, GATED, false>(a, stream);
-    case 1: return run_direct<128, 128, 2, 4, 2, GATED, false>(a, stream);
-    case 2: return run_direct<192, 128, 2, 4, 2, GATED, false>(a, stream);
-    case 3: return run_direct<128, 192, 2, 4, 2, GATED, false>(a, stream);
-    case 4: return run_direct<192, 128, 2, 8, 3, GATED, false>(a, stream);
-    case 5: return run_direct<128, 128, 4, 8, 3, GATED, false>(a, stream);
-    case 6: return run_direct<64, 128, 2, 8, 4, GATED, false>(a, stream);
-    case 7: return run_direct<64, 64, 2, 4, 4, GATED, false>(a, stream);
-  }
-  return run_direct<32, 64, 2, 4, 6, GATED, false>(a, stream);
+  return hipErrorInvalidValue;
 }
 
 // ---- row-wise kernels ------------------------------------------------------------------------------

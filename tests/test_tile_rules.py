@@ -13,6 +13,7 @@ KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "k
 SOURCE = """
 #include "delta_rule.h"
 #include "dense_attention_rule.h"
+#include "dense_tile_rule.h"
 #include "w4a16_rows_rule.h"
 using namespace llmopt;
 extern "C" {
@@ -25,12 +26,15 @@ int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, ui
 int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
   return three_delta_workgroups((tokens + 63) / 64 * heads, cus);
 }
+int product_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_tile(m, n, k, cus); }
 int qkv_tile(uint32_t m, uint32_t q, uint32_t kv, uint32_t k, uint32_t cus) {
   const uint32_t n[3] = {q, kv, kv};
   return (int)qkv_rows_tile(m, n, k, cus);
 }
 }
 """
+DENSE = ("256x256", "128x128", "192x128", "128x192", "192x128 eight waves", "128x128 eight waves", "64x128 eight waves", "64x64",
+         "32x64", "64x128")
 NONE, K32X32, K32X64, K32X64_DEEP, K32X64_LONG, K64X64, K64X128 = range(7)
 
 
@@ -107,3 +111,11 @@ def test_eight_waves_a_slab(rules, causal, rows, keys, past, heads, eight):
 def test_three_workgroups_of_the_delta_rule(rules, tokens, heads, three):
     """Where they save a round, and only there."""
     assert rules.three_workgroups(tokens, heads, CUS) == three
+
+
+@pytest.mark.parametrize("m,n,k,tile", [
+    (700, 4096, 128, "64x128"), (1500, 2048, 128, "64x128"), (3001, 1024, 256, "64x128"), (700, 4096, 512, "128x128 eight waves"),
+    (1500, 2048, 64, "128x128 eight waves"), (2048, 2048, 4096, "128x128 eight waves"), (64, 4096, 128, "32x64"),
+    (3001, 2048, 128, "192x128 eight waves"), (2048, 6144, 2048, "256x256"), (512, 6144, 2048, "128x128 eight waves")])
+def test_product_tiles(rules, m, n, k, tile):
+    assert DENSE[rules.product_tile(m, n, k, CUS)] == tile
