@@ -25,10 +25,11 @@ def values(rng, *shape, gain=1.0):
 
 
 # 32 x 64, 64 x 64, 64 x 128, 128 x 128 with eight and with four waves, 192 x 128 with eight and with four,
-# 128 x 192, 256 x 256
+# 128 x 192, 256 x 256, 64 x 128 with four waves (test_tile_rules.py checks which sizes take which)
 @pytest.mark.parametrize("m,n,k", [(2, 5, 64), (33, 700, 192), (500, 2000, 64), (700, 1023, 128), (1023, 2047, 64),
                                    (2047, 2045, 192), (1500, 6001, 64), (2999, 2046, 128), (2047, 8570, 64),
-                                   (2046, 6200, 128), (3000, 9503, 64)])
+                                   (2046, 6200, 128), (3000, 9503, 64), (1000, 5551, 64), (1000, 6357, 64), (2047, 2045, 64),
+                                   (1499, 2047, 256)])
 def test_tiles(runtime, m, n, k):
     rng = np.random.default_rng(m + n + k)
     (x, fx), (w, fw) = values(rng, m, k), values(rng, n, k)
@@ -41,7 +42,8 @@ def test_tiles(runtime, m, n, k):
 
 
 @pytest.mark.parametrize("m,width,ff", [(40, 128, 300), (500, 128, 1000), (700, 64, 3000), (1023, 128, 1500),
-                                        (2047, 64, 4285), (3000, 64, 3999)])
+                                        (2047, 64, 4285), (3000, 64, 3999), (500, 64, 1210), (1000, 64, 2827),
+                                        (1000, 64, 3230), (2047, 64, 3129), (1023, 64, 1500)])
 def test_gated_tiles(runtime, m, width, ff):
     """Norm, gated pair and down projection: what is rounded to bfloat16 between them (the normed rows and the products,
     half a unit, 2^-9, each) shows in the output at that size."""
@@ -59,3 +61,63 @@ def test_gated_tiles(runtime, m, width, ff):
     expected = (g / (1.0 + np.exp(-g)) * (h @ fup.T)) @ fdown.T
     error = out.numpy(np.float32, (m, width)) - x - expected
     assert np.sqrt(np.mean(error ** 2)) <= 4 * 2.0 ** -9 * np.sqrt(np.mean(expected ** 2))
+
+
+ROW_SIZES = [(33, 701, 64), (500, 2000, 64), (1023, 2047, 64), (2047, 2045, 64), (1000, 5551, 64), (1000, 6357, 64),
+             (1500, 6001, 64), (2999, 2046, 64), (3000, 9503, 64), (1499, 2047, 256)]
+
+
+def normed(rng, m, k):
+    stream = rng.standard_normal((m, k)).astype(np.float32)
+    norm, fnorm = values(rng, k)
+    x = stream.astype(np.float64)
+    return stream, norm, x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-6) * fnorm
+
+
+def assert_rows(got, h, weight, mixed=None):
+    """A normed value is rounded to bfloat16 before the product and the result after it: seven fraction bits, half a unit is
+    up to 2^-8 of the value; 2^-12 for the norm's and the sums' float32."""
+    expected = h @ weight.T
+    bound = (2.0 ** -8 + 2.0 ** -12) * (np.abs(h) @ np.abs(weight).T)
+    if mixed is not None:
+        expected = (expected + mixed) / 2  # (a half of each)
+    assert got.shape == expected.shape and np.isfinite(got).all()
+    assert np.all(np.abs(got - expected) <= bound + (2.0 ** -8 + 2.0 ** -12) * np.abs(expected))
+
+
+@pytest.mark.parametrize("m,n,k", ROW_SIZES)
+def test_rows_with_mixed_values(runtime, m, n, k):
+    """bfloat16 rows out of every tile: QKV, whose last columns are mixed with another layer's."""
+    rng = np.random.default_rng(m + n)
+    stream, norm, h = normed(rng, m, k)
+    weight, fweight = values(rng, n, k, gain=k ** -0.5)
+    first = rng.standard_normal((m, n - 16)).astype(np.float32)
+    put = runtime.buffer_of_bytes
+    out = put(np.full((m, n), 0x7fc0, dtype=np.uint16))  # NaN
+    rings = [put(np.zeros(size, dtype=np.uint16)) for size in (8, n - 16)]
+    runtime.dispatch("llmopt_rms_qkv_chunk_bf16", [put(stream), put(norm), put(weight), put(np.zeros(2, dtype=np.uint32)), out,
+                                                   put(first), *rings],
+                     u32s(m, k, 1, 1, 8, n - 16) + struct.pack("<fIf", 1e-6, 2, 0.5) + u32s(1, 1, 1), *GRID)
+    got = from_bfloat16(out.numpy(np.uint16)).reshape(m, n).astype(np.float64)
+    assert_rows(got[:, :16], h, fweight[:16])
+    assert_rows(got[:, 16:], h, fweight[16:], first.astype(np.float64))
+
+
+@pytest.mark.parametrize("m,n,k", ROW_SIZES)
+def test_rows_split_in_two(runtime, m, n, k):
+    """The same with the last columns, a time step a head, as float32 in an array of their own."""
+    rng = np.random.default_rng(m * 3 + n)
+    heads, vdim = (5, 3) if n % 2 else (4, 3)
+    states = (n - heads - 2 * heads * vdim) // 2
+    columns, channels = n - heads, heads * vdim + 2 * states
+    stream, norm, h = normed(rng, m, k)
+    weight, fweight = values(rng, n, k, gain=k ** -0.5)
+    put = runtime.buffer_of_bytes
+    zeros = lambda size, dtype: put(np.zeros(size, dtype=dtype))
+    out, steps = put(np.full((m, columns), 0x7fc0, dtype=np.uint16)), put(np.full((m, heads), np.nan, dtype=np.float32))
+    runtime.dispatch("llmopt_rms_ssm_input_bf16",
+                     [put(stream), put(norm), put(weight), zeros(2, np.uint32), zeros(channels * 4, np.uint16),
+                      zeros(channels, np.uint16), zeros(heads, np.uint16), zeros(channels * 4, np.float32), out, steps],
+                     u32s(m, k, heads, vdim, 1, states, 4, 1) + struct.pack("<f", 1e-6), *GRID)
+    assert_rows(from_bfloat16(out.numpy(np.uint16)).reshape(m, columns).astype(np.float64), h, fweight[:columns])
+    assert_rows(steps.numpy(np.float32, (m, heads)).astype(np.float64), h, fweight[columns:])

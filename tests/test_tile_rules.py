@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from tests import test_gpu_w4a16_rows
+from tests import test_gpu_dense_tiles, test_gpu_w4a16_rows
 
 CUS = 256
 KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "kernels")
@@ -111,6 +111,13 @@ def test_eight_waves_a_slab(rules, causal, rows, keys, past, heads, eight):
 def test_three_workgroups_of_the_delta_rule(rules, tokens, heads, three):
     """Where they save a round, and only there."""
     assert rules.three_workgroups(tokens, heads, CUS) == three
+
+
+def test_gpu_tests_reach_every_product_tile(rules):
+    tests, every = test_gpu_dense_tiles, set(range(len(DENSE)))
+    assert {rules.product_tile(*size, CUS) for size in sizes(tests.test_tiles, "m,n,k")} == every
+    assert {rules.product_tile(m, 2 * ff, width, CUS) for m, width, ff in sizes(tests.test_gated_tiles, "m,width,ff")} == every
+    assert {rules.product_tile(*size, CUS) for size in tests.ROW_SIZES} == every
 
 
 @pytest.mark.parametrize("m,n,k,tile", [
