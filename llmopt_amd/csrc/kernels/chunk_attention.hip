@@ -10,9 +10,11 @@
 //
 //  * chunk_prefill_kernel: a portion of a prompt.  Waves of 16 query rows of one head each walk its keys,
 //    64 keys a stage through LDS; keys before the portion come from the ring, the others from the
-//    portion's own rows.  Bound by the latency of a stage (products, softmax, products in turn): eight waves a
-//    workgroup and four a SIMD, where a wave of twice the rows left two, took 16 heads of 128 over 3001 rows from
-//    138 us to 119; matrix units are then busy for 30% of the time, and a second stage in LDS gives nothing.  S^T = K Q^T leaves every lane four consecutive keys of one query row, which is
+//    portion's own rows.  Bound by the latency of a stage (products, softmax, products in turn): matrix units are
+//    busy for 29% of the time and vector units for 50%, and a second stage in LDS gives nothing.  16 heads of 128
+//    over 3001 rows take 92 us (138 with four waves of 32 rows): 119 with eight waves of 16 rows a workgroup, four a
+//    SIMD, 112 with tiles dealt as below, 96 with the border mask behind its own branch, 92 with the weights' parts
+//    converted in pairs.  S^T = K Q^T leaves every lane four consecutive keys of one query row, which is
 //    the B operand of O^T += V^T P^T up to a permutation of the contraction index that the V^T operand
 //    follows: probabilities never leave their lane (bf16: as a high and a low part, so that the weights keep
 //    float32 accuracy in the product).  Caps of at most kFixedMaxCap bound the exponent, so
@@ -35,8 +37,6 @@ namespace {
 constexpr int kStageKeys = 64;
 constexpr float kFixedMaxCap = 40.0f;
 
-constexpr int kCompute = 256;  // compute units
-
 // The stage, and where KS == 2 the second half's sums in its place.
 template <typename T, int ND, int NE, int WAVES, int KS>
 constexpr int prefill_lds_bytes() {
@@ -48,7 +48,7 @@ constexpr int prefill_lds_bytes() {
 // Eight waves keep to the registers that let a compute unit hold two workgroups.
 template <typename T, int ND, int NE, int WAVES, int KS, bool FIXED>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 4 : ND * 2 + NE <= 16 || sizeof(T) == 2 ? 2 : 1) void
-chunk_prefill_kernel(ChunkAttentionArgs a) {
+chunk_prefill_kernel(ChunkAttentionArgs a, uint32_t cus) {
   constexpr int DP = ND * 32, EP = NE * 16;
   constexpr int ROW_WAVES = WAVES / KS, ROWS = ROW_WAVES * 16, KEYS = kStageKeys / KS, KT = KEYS / 16;
   constexpr int SK = DP + 16 / (int)sizeof(T), SV = value_stride<T, NE>();
@@ -67,7 +67,7 @@ chunk_prefill_kernel(ChunkAttentionArgs a) {
   // with the longest first, 112 so).
   const uint32_t per = a.heads / a.kv_heads, group = blockIdx.x % a.kv_heads;
   const uint32_t head = group * per + blockIdx.x / a.kv_heads;
-  const uint32_t around = max(kCompute / a.heads, 1u), round = blockIdx.y / around, step = blockIdx.y % around;
+  const uint32_t around = max(cus / a.heads, 1u), round = blockIdx.y / around, step = blockIdx.y % around;
   const uint32_t left = gridDim.y - round * around;  // tiles of this round and later ones
   const uint32_t p0 = a.state[kStatePosition], slot = a.state[kStateSlot];
   uint32_t tile = gridDim.y <= around || (round & 1) ? left - 1 - step : left - min(left, around) + step;
@@ -384,7 +384,7 @@ hipError_t run_prefill_kernel(const ChunkAttentionArgs &a, hipStream_t stream) {
   const auto kernel = chunk_prefill_kernel<T, ND, NE, WAVES, KS, FIXED>;
   if (bytes > 64 * 1024)
     if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
-  kernel<<<dim3(a.heads, (a.m + rows - 1) / rows), WAVES * 64, bytes, stream>>>(a);
+  kernel<<<dim3(a.heads, (a.m + rows - 1) / rows), WAVES * 64, bytes, stream>>>(a, (uint32_t)device_compute_units());
   return hipGetLastError();
 }
 
@@ -405,7 +405,7 @@ hipError_t run_prefill_tile(const ChunkAttentionArgs &a, hipStream_t stream) {
 template <typename T, int ND, int NE>
 hipError_t run_prefill(const ChunkAttentionArgs &a, hipStream_t stream) {
   if constexpr (sizeof(T) == 2 && ND <= 4 && NE <= 8) {
-    const bool many = (uint64_t)a.heads * ((a.m + 127) / 128) > kCompute;
+    const bool many = (uint64_t)a.heads * ((a.m + 127) / 128) > (uint64_t)device_compute_units();
     if ((many && (ND > 2 || NE > 4)) || (a.m + 63) / 64 > 65536) return run_prefill_tile<T, ND, NE, 8, 1>(a, stream);
     return run_prefill_tile<T, ND, NE, 8, 2>(a, stream);
   } else {

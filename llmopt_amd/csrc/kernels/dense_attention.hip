@@ -515,7 +515,7 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
     // The waves' shares of the slab meet in LDS (the stages are read to the end: the loop's last
     // barrier): per wave the row maxima and denominators, and O^T as floats [d][row] - a lane's
     // values of one register are 32 neighbouring rows.  Thread t then folds row t % 32, head_dim
-    // values (t / 32) * D / 8 .. of the four shares and stores them.
+    // values (t / 32) * D / 2 / WAVES .. of the WAVES shares and stores them.
     float *share_out = reinterpret_cast<float *>(stage_lds);                  // [WAVES][D][32]
     float *share_max = share_out + WAVES * D * 32;                            // [WAVES][32]
     float *share_sum = share_max + WAVES * 32;                                // [WAVES][32]

@@ -160,10 +160,10 @@ __device__ __forceinline__ void delta_columns(const DeltaArgs &a, uint32_t head,
   }
 }
 
-template <typename T, int ND, int NE>
-constexpr int attention_lds_bytes() { return decode_lds_floats<T, NE>() * 4 + raw_row_lds_bytes<T, ND, NE>(); }
+template <int ND, int NE>
+constexpr int attention_lds_bytes() { return decode_lds_floats<__bf16, NE>() * 4 + raw_row_lds_bytes<__bf16, ND, NE>(); }
 
-template <typename T, int ND, int NE, int R>
+template <int ND, int NE, int R>
 __global__ __launch_bounds__(kThreads) void mixer_step_kernel(ChunkAttentionArgs a, DeltaArgs d, uint32_t splits, float *squares) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const uint32_t parts = d.vdim / kColumns, delta_blocks = d.heads * parts;
@@ -173,14 +173,13 @@ __global__ __launch_bounds__(kThreads) void mixer_step_kernel(ChunkAttentionArgs
   }
   if (threadIdx.x >= 256) return;  // (barriers count the waves that are still there)
   const uint32_t share = blockIdx.x - delta_blocks;
-  chunk_decode<T, ND, NE, true>(a, splits, share % a.kv_heads, share / a.kv_heads, lds);
+  chunk_decode<__bf16, ND, NE, true>(a, splits, share % a.kv_heads, share / a.kv_heads, lds);
 }
 
-template <typename T>
 __global__ __launch_bounds__(256) void mixer_finish_kernel(ChunkAttentionArgs a, DeltaArgs d, uint32_t splits, const float *squares) {
   extern __shared__ __attribute__((aligned(16))) float shared[];
   if (blockIdx.x >= d.heads) {
-    chunk_merge<T>(a, splits, blockIdx.x - d.heads, shared);
+    chunk_merge<__bf16>(a, splits, blockIdx.x - d.heads, shared);
     return;
   }
   const uint32_t head = blockIdx.x, c = threadIdx.x, parts = d.vdim / kColumns;
@@ -192,21 +191,21 @@ __global__ __launch_bounds__(256) void mixer_finish_kernel(ChunkAttentionArgs a,
   *out = value * (1.0f / sqrtf(total / (float)d.vdim + d.epsilon));
 }
 
-template <typename T, int ND, int NE, int R>
+template <int ND, int NE, int R>
 hipError_t run(const ChunkAttentionArgs &a, const DeltaArgs &d, float *squares, hipStream_t stream) {
-  constexpr int bytes = std::max<int>(attention_lds_bytes<T, ND, NE>(), (int)sizeof(DeltaStepLds));
+  constexpr int bytes = std::max<int>(attention_lds_bytes<ND, NE>(), (int)sizeof(DeltaStepLds));
   static_assert(bytes <= 64 * 1024, "no raised limit");
   const uint32_t splits = decode_splits(a), blocks = d.heads * (d.vdim / kColumns) + a.kv_heads * splits;
-  mixer_step_kernel<T, ND, NE, R><<<blocks, kThreads, bytes, stream>>>(a, d, splits, squares);
+  mixer_step_kernel<ND, NE, R><<<blocks, kThreads, bytes, stream>>>(a, d, splits, squares);
   if (hipError_t status = hipGetLastError()) return status;
-  mixer_finish_kernel<T><<<d.heads + (splits > 1 ? a.heads : 0), 256, splits * 8, stream>>>(a, d, splits, squares);
+  mixer_finish_kernel<<<d.heads + (splits > 1 ? a.heads : 0), 256, splits * 8, stream>>>(a, d, splits, squares);
   return hipGetLastError();
 }
 
 template <int ND, int NE>
 hipError_t pick_rows(const ChunkAttentionArgs &a, const DeltaArgs &d, float *squares, hipStream_t stream) {
-  if (d.dim <= 128) return run<__bf16, ND, NE, 2>(a, d, squares, stream);
-  return run<__bf16, ND, NE, 4>(a, d, squares, stream);
+  if (d.dim <= 128) return run<ND, NE, 2>(a, d, squares, stream);
+  return run<ND, NE, 4>(a, d, squares, stream);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

@@ -1,6 +1,6 @@
 // W4A16 products of a batch's rows (more than the streaming GEMVs take, fewer than a prompt's) and of prompts over small
-// matrices: tiles of 16, 32 or 64 activation rows by 32 or 64 weight columns, so that the launch has about a workgroup
-// per CU where 128 x 128 tiles leave most of them empty or pad most of their rows.
+// matrices: tiles of 32 or 64 activation rows by 32, 64 or 128 weight columns (w4a16_rows_rule.h), so that the launch has
+// about a workgroup per CU where 128 x 128 tiles leave most of them empty or pad most of their rows.
 //
 // What bounds it at many rows of K: the weights from HBM (31 MB at 4096 x 14336: 6.5 us at a copy's rate) and the
 // activation rows, which every workgroup reads again, from L2; at a CU's rate of filling LDS (about 80 bytes a
@@ -85,7 +85,8 @@ __global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
   constexpr bool PACK = std::is_same_v<Params, PackParams>;
   static_assert(!PACK || (!DUAL && CT % 2 == 0), "whole heads in a tile");
   constexpr int WAVES = CT * P, COLUMNS = CT * 32, STEP = P * 64;
-  constexpr int RT = (ROWS + 31) / 32;                      // 32-row blocks of a wave
+  static_assert(ROWS % 32 == 0, "whole blocks of rows");
+  constexpr int RT = ROWS / 32;                             // 32-row blocks of a wave
   constexpr int X_PIECES = STEP / 8, W_PIECES = STEP / 32;  // 16-byte pieces of a row and step
   constexpr int X_BYTES = ROWS * X_PIECES * 16, W_BYTES = COLUMNS * W_PIECES * 16, STAGE_BYTES = X_BYTES + W_BYTES;
   constexpr int X_COPIES = X_BYTES / 1024 / WAVES, COPIES = X_COPIES + 1;  // of a wave and step
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
     for (int i = 0; i < 16; ++i) acc[r][i] = 0.0f;
 
   const int column = ct * 32 + (lane & 31), half = lane >> 5;
-  const uint32_t x_read_row = ROWS < 32 ? (lane & (ROWS - 1)) : (lane & 31);
+  const uint32_t x_read_row = lane & 31;
   const uint32_t w_read = X_BYTES + (column * W_PIECES + ((part * 2 + half) ^ w_twist(column))) * 16;
   uint32_t x_read[4];
 #pragma unroll
@@ -211,7 +212,7 @@ __global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int row = r * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-      if (ROWS >= 32 || row < ROWS) sums[(part * ROWS + row) * COLUMNS + column] = acc[r][i];
+      sums[(part * ROWS + row) * COLUMNS + column] = acc[r][i];
     }
   __syncthreads();
   constexpr int OUT = DUAL ? COLUMNS / 2 : COLUMNS, QUADS = ROWS * OUT / 4;

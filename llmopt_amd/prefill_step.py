@@ -119,7 +119,9 @@ class PrefillStep:
                 out.append(("llmopt_cache_pack_attention_q8_simd", [w["v"], self.slots, self.pool],
                             pack(value_offset, 1, kvd), (t * kvd // 64 * 32, 1, 1), group))
             elif self.packed_projection:
-                # projection, rotation and every token's Q8 slot as one entry: the same bytes out, three entries fewer a layer
+                # projection, rotation and every token's Q8 slot as one entry: the same arithmetic, and the
+                # same bytes where the joined launch takes the tile that the projection alone takes (a tile of whole heads
+                # in the place of a narrower one sums K's parts in another order)
                 out.append(("llmopt_rms_w4a16_qkv_rotary_pack_prompt_q8_f16_g64",
                             [*qkv_inputs, self.cos, self.sin, w["q_rot"], w["k_rot"], w["v"], self.slots, self.pool],
                             qkv_params + pack_params, rows_grid(qd + 2 * kvd), group))
