@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from tests import test_gpu_dense_tiles, test_gpu_w4a16_rows
+from tests import test_gpu_delta_chunks, test_gpu_dense_tiles, test_gpu_w4a16_rows
 
 CUS = 256
 KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "kernels")
@@ -111,6 +111,12 @@ def test_eight_waves_a_slab(rules, causal, rows, keys, past, heads, eight):
 def test_three_workgroups_of_the_delta_rule(rules, tokens, heads, three):
     """Where they save a round, and only there."""
     assert rules.three_workgroups(tokens, heads, CUS) == three
+
+
+def test_gpu_tests_reach_three_workgroups(rules):
+    names = "m,heads,kv_heads,dim,vdim"
+    for m, heads, _, dim, _ in sizes(test_gpu_delta_chunks.test_three_workgroups_against_float64, names):
+        assert 64 < dim <= 128 and rules.three_workgroups(m, heads, CUS) == 1
 
 
 def test_gpu_tests_reach_every_product_tile(rules):
