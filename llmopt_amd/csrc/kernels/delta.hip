@@ -810,7 +810,7 @@ __global__ __launch_bounds__(512) void delta_state_kernel(DeltaArgs a, DeltaWork
 // The parallel part: a workgroup per chunk and head, 16 tokens a wave, all value columns, so that a head's norm
 // stays in the wave.  The workgroups behind the chunks' ones: the step's last inputs into the convolution's ring.
 // Bound by the latency of its operands (the chunk's state, U and queries: 130 KB a workgroup): 3001 tokens of 16 heads
-// of 128 x 128 take 32 us with three workgroups a compute unit, 58 with one.
+// of 128 x 128 take 32 us with three workgroups a compute unit, 58 with one (38 and 63 inside a prompt).
 template <typename T, int STEPS, int NE>
 __global__ __launch_bounds__(256, STEPS <= 4 && NE <= 8 ? 3 : 1) void delta_output_kernel(DeltaArgs a, DeltaWorkspace w) {
   constexpr uint32_t np = STEPS * 32;

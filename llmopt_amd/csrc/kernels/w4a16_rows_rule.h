@@ -64,6 +64,10 @@ inline bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k, bool few) {
 // 3072 (264) 53.2 / 45.5, 384 x 4096 x 6144 (288) 53.4 / 45.2; a long K that the large tiles split over workgroups while
 // half the CUs have none of them, 300 x 3072 x 4096 22.3 / 21.4, 300 x 4096 x 4096 28.8 / 28.0, 200 x 6144 x 6144 42.1 /
 // 38.7, 600 x 6144 x 2048 42.5 / 32.6.
+// Beyond K = 6144 the tiles of 64 rows fit LDS up to 8192 and would win where they are one round and the large tiles pad their
+// rows, not where those fill: large tiles / 64-row tiles 48 x 7168 x 14336 44.0 / 28.3, 48 x 8192 x 14336 49.4 / 32.4, 128 x
+// 7168 x 8192 31.8 / 29.0, 512 x 7168 x 2048 30.4 / 28.4, 256 x 8192 x 4096 32.2 / 32.4, 200 x 7168 x 6144 43.9 / 47.9, 200 x
+// 8192 x 6144 47.9 / 52.9.  They have not been taken there.
 // With few steps (K < 1536) three workgroups of the shallow 32 x 64 ring share a CU: two rounds of it are still fast.
 inline RowsTile rows_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint32_t k, uint32_t cus) {
   auto rounds = [&](uint32_t rows, uint32_t columns) {
