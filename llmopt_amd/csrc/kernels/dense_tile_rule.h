@@ -8,48 +8,55 @@ namespace llmopt {
 
 enum class DenseTile { k256x256, k128x128, k192x128, k128x192, k192x128Eight, k128x128Eight, k64x128Eight, k64x64, k32x64, k64x128 };
 
-// Tiles in that order, and what a round of them takes on 256 CUs at K = 2048 (us, weights from HBM; a round's time goes with
-// K): with one workgroup on a CU, and with two where the tile's ring leaves room for them.  The eight-wave tiles keep two
+// Tiles in that order, and an estimate of a launch on 256 CUs (us, K in 1024, weights from HBM).  `start` comes once, and a
+// round of workgroups takes a constant, its start and its outputs, and a part that goes with K: with one workgroup on a CU,
+// and with two where the tile's ring leaves room for them (`two_k` == 0: it takes the CU).  A last round on few CUs takes the
+// share `few` of a whole one, which grows evenly to the whole.  The step from one workgroup on a CU to two comes to the share
+// `pair` with the first CU that has two and is whole once the share `span` of the CUs have.  The eight-wave tiles keep two
 // stages of copies under way instead of one, which covers the trip to HBM when a CU has no second workgroup to fill the wait.
-struct TileRound {
+struct TileTime {
   uint32_t rows, columns;
-  float one, two;  // two == 0: the ring takes the CU
+  float start, one, one_k, few, two, two_k, pair, span;
 };
-constexpr TileRound kTileRounds[] = {
-    {256, 256, 53.0f, 0.0f},  // 8 waves, 2 stages
-    {128, 128, 31.0f, 38.0f}, // 4 waves, 2 stages
-    {192, 128, 34.0f, 52.0f}, // 4 waves, 2 stages
-    {128, 192, 35.0f, 55.0f}, // 4 waves, 2 stages
-    {192, 128, 29.0f, 0.0f},  // 8 waves, 3 stages
-    {128, 128, 23.0f, 0.0f},  // 8 waves, 3 stages
-    {64, 128, 15.3f, 0.0f},   // 8 waves, 4 stages
-    {64, 64, 11.2f, 17.0f},   // 4 waves, 4 stages
-    {32, 64, 8.5f, 13.7f},    // 4 waves, 6 stages
+constexpr TileTime kTileTimes[] = {
+    {256, 256, 0.01f, 14.10f, 24.56f, 1.00f, 0.00f, 0.00f, 0.00f, 0.00f},     // 8 waves, 2 stages
+    {128, 128, 0.00f, 7.54f, 20.73f, 0.47f, 8.85f, 15.57f, 0.02f, 0.65f},     // 4 waves, 2 stages
+    {192, 128, 0.00f, 7.79f, 14.79f, 1.00f, 11.91f, 19.36f, 1.00f, 0.06f},    // 4 waves, 2 stages
+    {128, 192, 5.82f, 1.85f, 15.16f, 1.00f, 7.30f, 21.46f, 0.99f, 0.17f},     // 4 waves, 2 stages
+    {192, 128, 0.00f, 6.73f, 12.92f, 0.99f, 0.00f, 0.00f, 0.00f, 0.00f},      // 8 waves, 3 stages
+    {128, 128, 0.01f, 5.78f, 9.27f, 0.92f, 0.00f, 0.00f, 0.00f, 0.00f},       // 8 waves, 3 stages
+    {64, 128, 1.22f, 2.87f, 6.83f, 0.91f, 0.00f, 0.00f, 0.00f, 0.00f},        // 8 waves, 4 stages
+    {64, 64, 0.98f, 2.42f, 4.09f, 1.00f, 2.29f, 9.08f, 0.00f, 0.22f},         // 4 waves, 4 stages
+    {32, 64, 1.84f, 1.05f, 3.37f, 0.97f, 1.18f, 7.21f, 0.96f, 0.38f},         // 4 waves, 6 stages
+    {64, 128, 0.07f, 4.40f, 8.62f, 0.78f, 4.57f, 12.70f, 0.81f, 0.13f},       // 4 waves, 3 stages
 };
 
-// The tile with the least time by these (columns: a gated pair's both matrices).  Measured, us (m x n x k), before (the
-// largest tile that gives every CU work) and now: 2048 x 2048 x 4096 58 / 47, 2048 x 2048 x 8192 97 / 86, 2048 x 8576 x 2048
-// 94 / 80, 2048 x 6144 x 2048 69 / 56, 3001 x 2048 x 4096 67 / 63, 1024 x 2048 x 4096 34 / 31, 512 x 6144 x 2048 28 / 23;
-// 3001 x 9504 x 2048 118, 512 x 2048 x 4096 22, 64 x 4384 x 1024 7.0 as before.  Over 720 sizes (K 64 to 8192, 512 to 16384
-// columns, 2 to 3001 rows) it is 4% faster than that rule on average and 1% off the best tile.  It is furthest off with a few
-// tiles of 64 x 64 more than CUs, which it counts as two on every CU: 700 x 1500 x 8192 51 for 42, 1500 x 1024 x 4096 29
-// for 27 (1024 x 1500 x 4096 is the other way round, 29 for 33).
-// With a short K the start and the end of a workgroup decide, not its steps: where the estimate takes 128 x 128 tiles of eight
-// waves, twice as many of 64 x 128 and four waves, several on a CU, are over sooner (700 x 4096 x 128 7.6 / 7.0, 1500 x 2048 x
-// 128 7.25 / 7.0, 3001 x 1024 x 256 8.45 / 8.1, 700 x 4096 x 256 8.6 / 7.95; at K = 64 the same either way, at 512 11.2 / 12.2).
+// The tile with the least time by these (columns: a gated pair's both matrices).  The constants are a fit to all ten tiles at
+// 1900 sizes (8 to 3001 rows, 64 to 16384 columns, K 64 to 8192; 600 MB of weights in turn, so that none is in a cache), weighed
+// by what a wrong choice costs: the choice is 0.5% off the best tile on average, and 7% faster than the largest tile that gives
+// every CU work, which is more than 3% ahead at 29 of them.  An estimate of rounds that go with K alone was 0.8% off, and
+// behind that tile by more than 3% at 72 (us, that tile / such an estimate: 384 x 2816 x 8192 41.0 / 52.0, 700 x 1500 x 8192 41.5
+// / 50.4, 300 x 12288 x 512 12.4 / 13.4: these are back; 384 x 3072 x 8192, with 288 tiles of 64 x 64, 43.6 / 52.5 is not).
 inline DenseTile dense_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus) {
   int best = 0;
   float least = 3.4e38f;
-  for (int i = 0; i < (int)(sizeof(kTileRounds) / sizeof(kTileRounds[0])); ++i) {
-    const TileRound &t = kTileRounds[i];
+  for (int i = 0; i < (int)(sizeof(kTileTimes) / sizeof(kTileTimes[0])); ++i) {
+    const TileTime &t = kTileTimes[i];
+    const bool pairs = t.two_k > 0.0f;
     const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns);
-    const uint64_t slots = t.two > 0.0f ? 2ull * cus : cus, rest = tiles % slots;
-    const float full = t.two > 0.0f ? t.two : t.one;
-    const float time = (float)(tiles / slots) * full + (rest == 0 ? 0.0f : rest <= cus ? t.one : t.two);
+    const uint64_t slots = pairs ? 2ull * cus : cus, rest = tiles % slots;
+    const float one = t.one + t.one_k * (float)k / 1024.0f, two = pairs ? t.two + t.two_k * (float)k / 1024.0f : one;
+    const float share = (float)rest / (float)cus;  // of the CUs, in the last round
+    float time = t.start + (float)(tiles / slots) * two;
+    if (share > 1.0f) {
+      const float more = share - 1.0f < t.span ? (share - 1.0f) / t.span : 1.0f;
+      time += one + (two - one) * (t.pair + (1.0f - t.pair) * more);
+    } else if (rest > 0) {
+      time += one * (t.few + (1.0f - t.few) * share);
+    }
     if (time < least) least = time, best = i;
   }
-  const DenseTile tile = (DenseTile)best;
-  return tile == DenseTile::k128x128Eight && k > 64 && k <= 256 ? DenseTile::k64x128 : tile;
+  return (DenseTile)best;
 }
 
 }  // namespace llmopt

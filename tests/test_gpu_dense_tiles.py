@@ -29,7 +29,8 @@ def values(rng, *shape, gain=1.0):
 @pytest.mark.parametrize("m,n,k", [(2, 5, 64), (33, 700, 192), (500, 2000, 64), (700, 1023, 128), (1023, 2047, 64),
                                    (2047, 2045, 192), (1500, 6001, 64), (2999, 2046, 128), (2047, 8570, 64),
                                    (2046, 6200, 128), (3000, 9503, 64), (1000, 5551, 64), (1000, 6357, 64), (2047, 2045, 64),
-                                   (1499, 2047, 256)])
+                                   (1499, 2047, 256), (1345, 8857, 256), (1413, 8123, 256), (195, 8311, 2560),
+                                   (203, 8125, 2304)])
 def test_tiles(runtime, m, n, k):
     rng = np.random.default_rng(m + n + k)
     (x, fx), (w, fw) = values(rng, m, k), values(rng, n, k)
@@ -43,7 +44,8 @@ def test_tiles(runtime, m, n, k):
 
 @pytest.mark.parametrize("m,width,ff", [(40, 128, 300), (500, 128, 1000), (700, 64, 3000), (1023, 128, 1500),
                                         (2047, 64, 4285), (3000, 64, 3999), (500, 64, 1210), (1000, 64, 2827),
-                                        (1000, 64, 3230), (2047, 64, 3129), (1023, 64, 1500)])
+                                        (1000, 64, 3230), (2047, 64, 3129), (1023, 64, 1500), (1345, 256, 4429),
+                                        (1413, 256, 4061), (195, 2560, 4155), (203, 2304, 4062)])
 def test_gated_tiles(runtime, m, width, ff):
     """Norm, gated pair and down projection: what is rounded to bfloat16 between them (the normed rows and the products,
     half a unit, 2^-9, each) shows in the output at that size."""
@@ -64,7 +66,8 @@ def test_gated_tiles(runtime, m, width, ff):
 
 
 ROW_SIZES = [(33, 701, 64), (500, 2000, 64), (1023, 2047, 64), (2047, 2045, 64), (1000, 5551, 64), (1000, 6357, 64),
-             (1500, 6001, 64), (2999, 2046, 64), (3000, 9503, 64), (1499, 2047, 256)]
+             (1500, 6001, 64), (2999, 2046, 64), (3000, 9503, 64), (1499, 2047, 256), (1345, 8857, 256), (1413, 8123, 256),
+             (195, 8311, 2560), (203, 8125, 2304)]
 
 
 def normed(rng, m, k):

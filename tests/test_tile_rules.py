@@ -127,8 +127,13 @@ def test_gpu_tests_reach_every_product_tile(rules):
 
 
 @pytest.mark.parametrize("m,n,k,tile", [
-    (700, 4096, 128, "64x128"), (1500, 2048, 128, "64x128"), (3001, 1024, 256, "64x128"), (700, 4096, 512, "128x128 eight waves"),
-    (1500, 2048, 64, "128x128 eight waves"), (2048, 2048, 4096, "128x128 eight waves"), (64, 4096, 128, "32x64"),
-    (3001, 2048, 128, "192x128 eight waves"), (2048, 6144, 2048, "256x256"), (512, 6144, 2048, "128x128 eight waves")])
+    (1500, 2048, 128, "64x128"), (3001, 1024, 256, "64x128"), (700, 4096, 128, "64x128"), (64, 4096, 128, "32x64"),
+    (700, 4096, 512, "128x128 eight waves"), (2048, 2048, 4096, "128x128 eight waves"), (512, 6144, 2048, "128x128 eight waves"),
+    (3001, 2048, 128, "192x128 eight waves"), (3001, 2048, 4096, "192x128 eight waves"), (2048, 6144, 2048, "128x192"),
+    (300, 12288, 512, "64x128"), (384, 2816, 8192, "64x64"), (700, 5632, 2048, "64x128"), (900, 8192, 1024, "128x128"),
+    (2048, 9504, 1024, "192x128"), (2048, 12288, 512, "128x192"), (700, 1500, 8192, "64x64"), (3001, 9504, 2048, "256x256"),
+    (512, 2048, 4096, "64x64"), (64, 4384, 1024, "32x64"), (3001, 8192, 2048, "192x128"), (2048, 4224, 2048, "192x128"),
+    (1024, 2048, 4096, "64x128 eight waves")])
 def test_product_tiles(rules, m, n, k, tile):
+    """The fastest of the ten."""
     assert DENSE[rules.product_tile(m, n, k, CUS)] == tile
