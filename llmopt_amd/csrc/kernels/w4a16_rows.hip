@@ -1,5 +1,5 @@
 // W4A16 products of a batch's rows (more than the streaming GEMVs take, fewer than a prompt's) and of prompts over small
-// matrices: tiles of 32 or 64 activation rows by 32, 64 or 128 weight columns (w4a16_rows_rule.h), so that the launch has
+// matrices: tiles of 32 to 96 activation rows by 32, 64 or 128 weight columns (w4a16_rows_rule.h), so that the launch has
 // about a workgroup per CU where 128 x 128 tiles leave most of them empty or pad most of their rows.
 //
 // What bounds it at many rows of K: the weights from HBM (31 MB at 4096 x 14336: 6.5 us at a copy's rate) and the
@@ -348,6 +348,7 @@ hipError_t launch_tile(RowsTile tile, Params &p, hipStream_t stream) {
     case RowsTile::k32x64Long: return run_rows<32, 2, 4, 4, DUAL>(p, stream);
     case RowsTile::k64x64: return run_rows<64, 2, 4, 3, DUAL>(p, stream);
     case RowsTile::k64x128: return run_rows<64, 4, 2, 2, DUAL>(p, stream);
+    case RowsTile::k96x128: return run_rows<96, 4, 2, 2, DUAL>(p, stream);
     case RowsTile::kNone: break;
   }
   return hipErrorInvalidValue;

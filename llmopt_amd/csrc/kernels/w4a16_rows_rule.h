@@ -8,7 +8,7 @@ namespace llmopt {
 
 // Rows by columns of a workgroup's tile; kNone: another kernel (the matrix-core GEMV's row groups, or the 128 x 128 and
 // larger tiles of w4a16_gemm.hip).
-enum class RowsTile { kNone, k32x32, k32x64, k32x64Deep, k32x64Long, k64x64, k64x128 };
+enum class RowsTile { kNone, k32x32, k32x64, k32x64Deep, k32x64Long, k64x64, k64x128, k96x128 };
 
 // The matrix-core GEMV: rows of one group, and the longest K that one workgroup covers.
 constexpr uint32_t kRowGroup = 8, kRowGroupK = 4096;
@@ -53,15 +53,16 @@ inline bool rows_wanted(uint32_t m, uint64_t columns, uint32_t k, bool few) {
 
 // A launch takes as long as one workgroup while each CU has at most one of them, and a workgroup the longer the larger
 // its tile and K are (us, K = 576 / 2048 / 4096 / 8192, one round): 32 x 32 4.1 / 6.1 / 8.8 / 13.7, 32 x 64 4.6 / 7.8 /
-// 11.3 / 21, 64 x 64 5.9 / 10.3 / 16.4 / 29, 64 x 128 7.1 / 14.9 / 25.7 / 47.  So: the smallest tile that needs one round,
-// and the large tiles once even 64 x 128 would need more than an eighth of a second one.  Measured against those, us (m, K,
+// 11.3 / 21, 64 x 64 5.9 / 10.3 / 16.4 / 29, 64 x 128 7.1 / 14.9 / 25.7 / 47, 96 x 128 9.5 / 18.6 / 32.4.  So: the smallest
+// tile that needs one round, and the large tiles once even 96 x 128 would need a second one.  Measured against those, us (m, K,
 // n):
 // 24 x 4096 x 14336 13.3 / 30.8; 24 x 4096 x 4096 8.7 / 16.7; 64 x 14336 x 4096 23.5 / 38.5; 128 x 4096 x 4096 11.8 / 17.4;
 // 200 x 4096 x 4096 16.9 / 21.4; 512 x 4096 x 4096 28 / 33; 1024 x 2048 x 2048 16.5 / 28.3; 700 x 576 x 576 5.3 / 9.5;
 // 700 x 1536 x 576 7.0 / 13.7; 700 x 576 x 1536 7.4 / 9.5; beyond: 200 x 4096 x 14336 53.6 / 43.5, 700 x 8192 x 2048 47 / 42.
 // At the line the small tiles are not the faster ones, but the more exact ones: the large tiles round q * s to half, 2.8e-4
-// off float64 for 2.1e-4.  The first tiles of a second round, 700 x 1472 x 3000 (264 of 64 x 128) 19.2 / 17.0, 700 x 4096 x
-// 3072 (264) 53.2 / 45.5, 384 x 4096 x 6144 (288) 53.4 / 45.2; a long K that the large tiles split over workgroups while
+// off float64 for 2.1e-4.  Where 64 x 128 would begin a second round and 96 x 128 is one, us 64 x 128 / 96 x 128 / large: 700 x
+// 576 x 3072 11.3 / 9.5 / 10.3, 900 x 1024 x 3072 14.4 / 12.0 / 12.1, 288 x 2048 x 7680 22.2 / 19.0 / 20.0, 700 x 4096 x 3072
+// 49.4 / 32.3 / 33.9, 540 x 4096 x 4096 49.1 / 32.6 / 34.0.  A long K that the large tiles split over workgroups while
 // half the CUs have none of them, 300 x 3072 x 4096 22.3 / 21.4, 300 x 4096 x 4096 28.8 / 28.0, 200 x 6144 x 6144 42.1 /
 // 38.7, 600 x 6144 x 2048 42.5 / 32.6.
 // Beyond K = 6144 the tiles of 64 rows fit LDS up to 8192 and would win where they are one round and the large tiles pad their
@@ -83,7 +84,9 @@ inline RowsTile rows_tile(uint32_t m, const uint32_t *n, uint32_t matrices, uint
     if (rows_lds_bytes<32, 2, 4, 4>(k) <= kRowsLdsBytes) return RowsTile::k32x64Long;
   }
   if (k >= 1536 && k <= 6144 && rounds(64, 64) <= 1) return RowsTile::k64x64;
-  if (k <= 6144 && rounds(64, 128) <= 1.125) return RowsTile::k64x128;
+  if (k <= 6144 && rounds(64, 128) <= 1) return RowsTile::k64x128;
+  if (k <= 6144 && rounds(96, 128) <= 1) return RowsTile::k96x128;
+  if (k <= 6144 && rounds(64, 128) <= 1.125) return RowsTile::k64x128;  // (rows that 96 divides no better than 64)
   return RowsTile::kNone;
 }
 
@@ -108,7 +111,9 @@ inline RowsTile pack_rows_tile(uint32_t m, const uint32_t *n, uint32_t k, uint32
 // A gated pair, by output columns (half of a tile's).  The large tiles take two accumulator sets, so the
 // small ones win for longer: us (m, K, n) 24 x 4096 x 14336 20.4 / 61.7, 64 x 4096 x 4096 12.6 / 58, 64 x 8192 x 2048
 // 26 / 108, 128 x 4096 x 14336 55 / 64 (two rounds), 512 x 2048 x 2048 15.9 / 31.8, 1024 x 2048 x 2048 26.3 / 34.4,
-// 700 x 576 x 1536 10.9 / 16.0; beyond: 200 x 4096 x 14336 105 / 78, 2048 x 2048 x 2048 49 / 46.
+// 700 x 576 x 1536 10.9 / 16.0; beyond: 200 x 4096 x 14336 105 / 78, 2048 x 2048 x 2048 49 / 46.  Where 96 x 128 is one round and
+// 64 x 128 is not, us 64 x 128 / 96 x 128: 700 x 576 x 1536 10.6 / 9.0, 900 x 1024 x 1536 13.6 / 11.4, 540 x 2048 x 2048 21.7 /
+// 18.0, 700 x 4096 x 1536 50.6 / 31.4.
 inline RowsTile gated_rows_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
   if (!rows_wanted(m, 2ull * n, k, row_groups_few(m, n, k, cus))) return RowsTile::kNone;
   auto rounds = [&](uint32_t rows, uint32_t columns) {
@@ -121,6 +126,7 @@ inline RowsTile gated_rows_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus
   }
   if (rounds(64, 32) <= 1 && rows_lds_bytes<64, 2, 4, 3>(k) <= kRowsLdsBytes) return RowsTile::k64x64;
   if (rounds(32, 32) <= 2 && k <= 8192) return RowsTile::k32x64;
+  if (rounds(64, 64) > 1 && rounds(96, 64) <= 1 && rows_lds_bytes<96, 4, 2, 2>(k) <= kRowsLdsBytes) return RowsTile::k96x128;
   if (rounds(64, 64) <= 2 && rows_lds_bytes<64, 4, 2, 2>(k) <= kRowsLdsBytes) return RowsTile::k64x128;
   return RowsTile::kNone;
 }

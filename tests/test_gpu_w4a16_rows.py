@@ -97,6 +97,26 @@ def test_small_tiles_over_three_matrices(runtime, m, k, sizes):
         assert_close_to_oracle(out.numpy(np.float16, (m, n)), product(x, packed, scale), f"three matrices {m}x{n}x{k}")
 
 
+# 96 x 128: rows and columns that end inside a tile, a last step of one group (K = 576) and of two, the longest K
+TALL = [(700, 3072, 576), (575, 5201, 64), (300, 8100, 1600), (481, 4099, 4160), (289, 7900, 6144)]
+TALL_PAIRS = [(700, 1536, 576), (575, 2561, 64), (300, 4033, 1600), (481, 2050, 4096)]
+
+
+@pytest.mark.parametrize("m,n,k", TALL)
+def test_tiles_of_96_rows(runtime, m, n, k):
+    test_small_tiles(runtime, m, n, k, "residual")
+
+
+@pytest.mark.parametrize("m,n,k", TALL_PAIRS)
+def test_pair_tiles_of_96_rows(runtime, m, n, k):
+    test_small_pair_tiles(runtime, m, n, k)
+
+
+@pytest.mark.parametrize("k,heads,kv_heads,tokens", [(576, 32, 8, 700), (64, 30, 10, 705)])
+def test_projection_with_rotation_and_pack_on_96_rows(runtime, k, heads, kv_heads, tokens):
+    test_projection_with_rotation_and_pack(runtime, k, heads, kv_heads, 64, tokens)
+
+
 # float32 logits from pairs of rows: one round of small tiles, 32 x 64 with short and with long K, 64 x 128, and the
 # matrix-core GEMV on the other side of the rule (few rows, long K)
 @pytest.mark.parametrize("m,n,k", [

@@ -63,6 +63,17 @@ def test_gpu_tests_reach_every_tile(rules):
     assert heads >= {NONE, K32X32, K32X64, K64X128}
 
 
+def test_96_rows_where_they_are_one_round_and_64_are_not(rules):
+    tests, tall = test_gpu_w4a16_rows, K64X128 + 1
+    assert {rules.linear_tile(m, n, k, CUS) for m, n, k in tests.TALL} == {tall}
+    assert {rules.gated_tile(m, n, k, CUS) for m, n, k in tests.TALL_PAIRS} == {tall}
+    assert rules.qkv_tile(700, 2048, 512, 576, CUS) == rules.qkv_tile(705, 1920, 640, 64, CUS) == tall
+    # one round of 64 rows; more than one of 96; as many tiles of either
+    assert rules.linear_tile(640, 3200, 576, CUS) == rules.gated_tile(640, 1536, 576, CUS) == K64X128
+    assert rules.linear_tile(1000, 3072, 576, CUS) == NONE and rules.gated_tile(1000, 1536, 576, CUS) == K64X128
+    assert rules.linear_tile(128, 17000, 1600, CUS) == K64X128
+
+
 @pytest.mark.parametrize("m,k,n", [(64, 1024, 1024), (32, 2048, 2048), (64, 4096, 1024), (16, 2048, 4096), (80, 3072, 768),
                                    (40, 1536, 1536), (128, 4096, 512), (40, 1280, 1280)])
 def test_few_row_groups(rules, m, k, n):
