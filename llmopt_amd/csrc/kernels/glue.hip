@@ -84,7 +84,9 @@ __global__ __launch_bounds__(kRowWaves * 64) void rms_norm_split_kernel(const In
 // loop above walks the row one 2-byte load latency at a time, twice).
 constexpr int kRmsVectors = 4;
 
-template <bool WEIGHT_FIRST>
+// SPLIT: the two rows of rms_norm_split_kernel.  (The head of one token, K = 2048: 5 us less than by its loops, a load latency
+// for every 64 values, twice.)
+template <bool WEIGHT_FIRST, bool SPLIT = false>
 __global__ __launch_bounds__(kRowWaves * 64) void rms_norm_f16_rows_kernel(const uint16_t *input,
                                                                            const uint16_t *weight,
                                                                            uint16_t *output, uint32_t rows,
@@ -111,20 +113,23 @@ __global__ __launch_bounds__(kRowWaves * 64) void rms_norm_f16_rows_kernel(const
   }
   square_sum = wave_sum(square_sum);
   const float inverse = rsqrtf(square_sum / (float)width + epsilon);
-  uint4 *out = reinterpret_cast<uint4 *>(output + (size_t)row * width);
+  uint4 *out = reinterpret_cast<uint4 *>(output + (size_t)row * width * (SPLIT ? 2 : 1));
 #pragma unroll
   for (int v = 0; v < kRmsVectors; ++v) {
     const uint32_t index = lane + 64 * v;
     if (index >= vectors) continue;
     const h8_t x = __builtin_bit_cast(h8_t, x_raw[v]);
     const h8_t g = __builtin_bit_cast(h8_t, w_raw[v]);
-    h8_t y;
+    h8_t y, low;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float value = (float)x[e], gain = (float)g[e];
-      y[e] = (_Float16)(WEIGHT_FIRST ? value * gain * inverse : value * inverse * gain);
+      const float result = WEIGHT_FIRST ? value * gain * inverse : value * inverse * gain;
+      y[e] = (_Float16)result;
+      if (SPLIT) low[e] = (_Float16)(result - (float)y[e]);
     }
     out[index] = __builtin_bit_cast(uint4, y);
+    if (SPLIT) out[vectors + index] = __builtin_bit_cast(uint4, low);
   }
 }
 
@@ -233,107 +238,135 @@ __device__ __forceinline__ bool better(float value, uint32_t index, float best_v
 // hands to its reduce kernel (lib/metal_w4a16_source.ml:1256-1283; there one
 // candidate per threadgroup of columns, here candidate t is the best of columns
 // t, t + 256, ... - the reduce step only needs every column covered once and
-// ties resolved to the lowest index).  Four slices of 256 threads scan a quarter
+// ties resolved to the lowest index).  Four slices of threads scan a quarter
 // of those columns each with several independent loads in flight, then meet in
 // LDS: a single thread per candidate would walk its 192 columns of a 49152-wide
 // vocabulary one load latency at a time.
 constexpr int kArgmaxSlices = 4;
-constexpr int kArgmaxUnroll = 4;
+constexpr int kArgmaxUnroll = 16;
 
-// `pairs`: logits holds two rows per output row (the products with the hi and
-// the lo half of the activation, see rms_norm_split_kernel) whose sum is the
-// logit; `half_logits`, when not null, receives half(logit) [rows, n].
-__global__ __launch_bounds__(256 * kArgmaxSlices) void argmax_candidates_kernel(const float *logits,
-                                                                                Candidate *candidates,
-                                                                                uint32_t n, bool pairs,
-                                                                                uint16_t *half_logits) {
-  __shared__ float slice_values[kArgmaxSlices][256];
-  __shared__ uint32_t slice_indices[kArgmaxSlices][256];
-  const uint32_t row = blockIdx.x;
-  const uint32_t t = threadIdx.x & 255;
-  const uint32_t slice = threadIdx.x >> 8;
-  const float *row_logits = logits + (size_t)row * n * (pairs ? 2 : 1);
-  const float *row_low = row_logits + n;  // read only with `pairs`
-  uint16_t *row_half = half_logits != nullptr ? half_logits + (size_t)row * n : nullptr;
+// Logits of a row: `low`, when not null, is the row of the products with the lo half of the activation (see
+// rms_norm_split_kernel), whose sum with the hi half's is the logit; `half`, when not null, receives half(logit).
+struct ArgmaxRow {
+  const float *logits, *low;
+  uint16_t *half;
+  uint32_t n;
+};
+
+__device__ __forceinline__ ArgmaxRow argmax_row(const float *logits, uint32_t n, bool pairs, uint16_t *half_logits, uint32_t row) {
+  const float *of_row = logits + (size_t)row * n * (pairs ? 2 : 1);
+  return {of_row, pairs ? of_row + n : nullptr, half_logits != nullptr ? half_logits + (size_t)row * n : nullptr, n};
+}
+
+// Columns t + 256 slice, then every 1024th; index 0xffffffff: there are none.
+__device__ __forceinline__ Candidate argmax_scan(const ArgmaxRow &row, uint32_t t, uint32_t slice) {
   float best_value = -3.402823466e+38f;
   uint32_t best_index = 0;
   bool found = false;
-  const uint32_t step = 256 * kArgmaxSlices;
-  uint32_t col = t + 256 * slice;
   // columns are visited in increasing order, so `>` alone keeps the lowest index among equals
-  for (; col + (kArgmaxUnroll - 1) * step < n; col += kArgmaxUnroll * step) {
+  auto take = [&](uint32_t col, float value) __attribute__((always_inline)) {
+    if (found && !(value > best_value)) return;
+    best_value = value;
+    best_index = col;
+    found = true;
+  };
+  constexpr uint32_t step = 256 * kArgmaxSlices;
+  uint32_t col = t + 256 * slice;
+  for (; col < row.n && row.n - col > (kArgmaxUnroll - 1) * step; col += kArgmaxUnroll * step) {
     float value[kArgmaxUnroll], low[kArgmaxUnroll];
 #pragma unroll
     for (int u = 0; u < kArgmaxUnroll; ++u) {
-      value[u] = row_logits[col + u * step];
-      low[u] = pairs ? row_low[col + u * step] : 0.0f;
+      value[u] = row.logits[col + u * step];
+      low[u] = row.low != nullptr ? row.low[col + u * step] : 0.0f;
     }
 #pragma unroll
     for (int u = 0; u < kArgmaxUnroll; ++u) {
       value[u] += low[u];
-      if (row_half != nullptr) row_half[col + u * step] = float_to_half_bits(value[u]);
+      if (row.half != nullptr) row.half[col + u * step] = float_to_half_bits(value[u]);
     }
 #pragma unroll
-    for (int u = 0; u < kArgmaxUnroll; ++u)
-      if (!found || value[u] > best_value) {
-        best_value = value[u];
-        best_index = col + u * step;
-        found = true;
-      }
+    for (int u = 0; u < kArgmaxUnroll; ++u) take(col + u * step, value[u]);
   }
-  for (; col < n; col += step) {
-    const float value = row_logits[col] + (pairs ? row_low[col] : 0.0f);
-    if (row_half != nullptr) row_half[col] = float_to_half_bits(value);
-    if (!found || value > best_value) {
-      best_value = value;
-      best_index = col;
-      found = true;
-    }
+  for (; col < row.n; col += step) {
+    const float value = row.logits[col] + (row.low != nullptr ? row.low[col] : 0.0f);
+    if (row.half != nullptr) row.half[col] = float_to_half_bits(value);
+    take(col, value);
   }
-  // a slice that saw no column keeps (lowest float, index 0), which never beats a real column
-  // except against equal values at a higher index - impossible for index 0
-  slice_values[slice][t] = found ? best_value : -3.402823466e+38f;
-  slice_indices[slice][t] = found ? best_index : 0xffffffffu;
+  return {best_value, found ? best_index : 0xffffffffu};
+}
+
+// Candidate t from its slices (`stride` apart).
+__device__ __forceinline__ Candidate argmax_join(const Candidate *slices, uint32_t stride) {
+  Candidate best = slices[0];
+#pragma unroll
+  for (int other = 1; other < kArgmaxSlices; ++other) {
+    const Candidate c = slices[other * stride];
+    if (c.index != 0xffffffffu && (best.index == 0xffffffffu || better(c.value, c.index, best.value, best.index))) best = c;
+  }
+  // a candidate with no column at all (n <= t): the reference's initial (lowest float, 0)
+  if (best.index == 0xffffffffu) best = {-3.402823466e+38f, 0};
+  return best;
+}
+
+// The best of 256 candidates by one wave, in the order of the reference's tree (lib/metal_w4a16_source.ml:1287-1315): lane l
+// holds candidates l, l + 64, l + 128 and l + 192.  Lane 0 ends with it.
+__device__ __forceinline__ Candidate argmax_tree(Candidate (&c)[4]) {
+  auto keep = [](Candidate &mine, const Candidate &other) __attribute__((always_inline)) {
+    if (better(other.value, other.index, mine.value, mine.index)) mine = other;
+  };
+  keep(c[0], c[2]);
+  keep(c[1], c[3]);
+  keep(c[0], c[1]);
+#pragma unroll
+  for (int width = 32; width > 0; width >>= 1) {
+    const Candidate other = {__shfl_down(c[0].value, width, 64), (uint32_t)__shfl_down((int)c[0].index, width, 64)};
+    keep(c[0], other);
+  }
+  return c[0];
+}
+
+// A workgroup owns kArgmaxGroup candidates of a row: a row of 49152 pairs is 393 KB, which one CU takes 5 us to read.
+constexpr uint32_t kArgmaxGroup = 16;
+
+__global__ __launch_bounds__(kArgmaxGroup * kArgmaxSlices) void argmax_candidates_kernel(const float *logits, Candidate *candidates,
+                                                                                        uint32_t n, bool pairs, uint16_t *half_logits) {
+  __shared__ Candidate slices[kArgmaxGroup * kArgmaxSlices];
+  const uint32_t row = blockIdx.x, within = threadIdx.x % kArgmaxGroup, t = blockIdx.y * kArgmaxGroup + within;
+  slices[threadIdx.x] = argmax_scan(argmax_row(logits, n, pairs, half_logits, row), t, threadIdx.x / kArgmaxGroup);
   __syncthreads();
-  if (slice == 0) {
-    float value = slice_values[0][t];
-    uint32_t index = slice_indices[0][t];
-#pragma unroll
-    for (int other = 1; other < kArgmaxSlices; ++other)
-      if (slice_indices[other][t] != 0xffffffffu &&
-          (index == 0xffffffffu || better(slice_values[other][t], slice_indices[other][t], value, index))) {
-        value = slice_values[other][t];
-        index = slice_indices[other][t];
-      }
-    // a candidate with no column at all (n <= t): the reference's initial (lowest float, 0)
-    if (index == 0xffffffffu) {
-      value = -3.402823466e+38f;
-      index = 0;
-    }
-    candidates[row * 256 + t] = {value, index};
-  }
+  if (threadIdx.x < kArgmaxGroup) candidates[(size_t)row * 256 + t] = argmax_join(slices + within, kArgmaxGroup);
 }
 
 // lib/metal_w4a16_source.ml:1287-1315
-__global__ __launch_bounds__(256) void argmax_reduce_kernel(const Candidate *candidates, uint32_t *token_ids) {
-  __shared__ float best_values[256];
-  __shared__ uint32_t best_indices[256];
-  const uint32_t row = blockIdx.x, tid = threadIdx.x;
-  best_values[tid] = candidates[row * 256 + tid].value;
-  best_indices[tid] = candidates[row * 256 + tid].index;
+__global__ __launch_bounds__(64) void argmax_reduce_kernel(const Candidate *candidates, uint32_t *token_ids) {
+  Candidate c[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) c[j] = candidates[(size_t)blockIdx.x * 256 + threadIdx.x + 64 * j];
+  const Candidate best = argmax_tree(c);
+  if (threadIdx.x == 0) token_ids[blockIdx.x] = best.index;
+}
+
+// Both steps of a row by one workgroup.
+__global__ __launch_bounds__(256 * kArgmaxSlices) void argmax_rows_kernel(const float *logits, uint32_t *token_ids, uint32_t n,
+                                                                         bool pairs, uint16_t *half_logits) {
+  __shared__ Candidate slices[kArgmaxSlices * 256];
+  slices[threadIdx.x] = argmax_scan(argmax_row(logits, n, pairs, half_logits, blockIdx.x), threadIdx.x & 255, threadIdx.x >> 8);
   __syncthreads();
-  for (uint32_t width = 128; width > 0; width >>= 1) {
-    if (tid < width && better(best_values[tid + width], best_indices[tid + width], best_values[tid],
-                              best_indices[tid])) {
-      best_values[tid] = best_values[tid + width];
-      best_indices[tid] = best_indices[tid + width];
-    }
-    __syncthreads();
-  }
-  if (tid == 0) token_ids[row] = best_indices[0];
+  if (threadIdx.x >= 64) return;
+  Candidate c[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) c[j] = argmax_join(slices + threadIdx.x + 64 * j, 256);
+  const Candidate best = argmax_tree(c);
+  if (threadIdx.x == 0) token_ids[blockIdx.x] = best.index;
 }
 
 }  // namespace
+
+// 16-byte requests of whole rows that fit a wave's registers.
+static bool vector_rows(const RmsNormArgs &a) {
+  return !a.input_f32 && a.width % 8 == 0 && a.width <= 64 * 8 * kRmsVectors &&
+         ((reinterpret_cast<uintptr_t>(a.input) | reinterpret_cast<uintptr_t>(a.weight) | reinterpret_cast<uintptr_t>(a.output)) & 15) == 0;
+}
 
 hipError_t launch_rms_norm(const RmsNormArgs &a, hipStream_t stream) {
   const dim3 grid((a.rows + kRowWaves - 1) / kRowWaves), block(kRowWaves * 64);
@@ -347,11 +380,7 @@ hipError_t launch_rms_norm(const RmsNormArgs &a, hipStream_t stream) {
                          a.rows, a.width, a.epsilon);
   } else {
     const uint16_t *in = static_cast<const uint16_t *>(a.input);
-    const bool vector_rows = a.width % 8 == 0 && a.width <= 64 * 8 * kRmsVectors &&
-                             reinterpret_cast<uintptr_t>(in) % 16 == 0 &&
-                             reinterpret_cast<uintptr_t>(a.weight) % 16 == 0 &&
-                             reinterpret_cast<uintptr_t>(a.output) % 16 == 0;
-    if (vector_rows) {
+    if (vector_rows(a)) {
       if (a.weight_first)
         hipLaunchKernelGGL((rms_norm_f16_rows_kernel<true>), grid, block, 0, stream, in, a.weight, a.output, a.rows,
                            a.width, a.epsilon);
@@ -466,14 +495,33 @@ hipError_t launch_copy_bytes(void *destination, const void *source, size_t bytes
 
 hipError_t launch_argmax_candidates(const float *logits, void *candidates, uint32_t rows, uint32_t n, bool pairs,
                                     uint16_t *half_logits, hipStream_t stream) {
-  hipLaunchKernelGGL(argmax_candidates_kernel, dim3(rows), dim3(256 * kArgmaxSlices), 0, stream, logits,
-                     static_cast<Candidate *>(candidates), n, pairs, half_logits);
+  hipLaunchKernelGGL(argmax_candidates_kernel, dim3(rows, 256 / kArgmaxGroup), dim3(kArgmaxGroup * kArgmaxSlices), 0, stream,
+                     logits, static_cast<Candidate *>(candidates), n, pairs, half_logits);
   return hipGetLastError();
+}
+
+// One workgroup a row up to 144 KB of logits, us one launch / two: 8192 3.6 / 4.2, 32768 5.1 / 5.4, 49152 6.2 / 6.2, 65536 7.2 /
+// 7.0, 49152 pairs with their halves stored (behind the head's product) 21.7 / 19.7.  (A thread for every candidate and slice in
+// one workgroup, then a launch that joined them over eight barriers: 5.9 at 32768, 26.8 with the head.)
+constexpr uint64_t kArgmaxOneLaunchBytes = 144 << 10;
+
+hipError_t launch_argmax(const float *logits, void *candidates, uint32_t *token_ids, uint32_t rows, uint32_t n, bool pairs,
+                         uint16_t *half_logits, hipStream_t stream) {
+  if ((uint64_t)n * (pairs ? 8 : 4) <= kArgmaxOneLaunchBytes) {
+    hipLaunchKernelGGL(argmax_rows_kernel, dim3(rows), dim3(256 * kArgmaxSlices), 0, stream, logits, token_ids, n, pairs,
+                       half_logits);
+    return hipGetLastError();
+  }
+  if (hipError_t status = launch_argmax_candidates(logits, candidates, rows, n, pairs, half_logits, stream)) return status;
+  return launch_argmax_reduce(candidates, token_ids, rows, stream);
 }
 
 hipError_t launch_rms_norm_split(const RmsNormArgs &a, hipStream_t stream) {
   const dim3 grid((a.rows + kRowWaves - 1) / kRowWaves), block(kRowWaves * 64);
-  if (a.input_f32)
+  if (vector_rows(a))
+    hipLaunchKernelGGL((rms_norm_f16_rows_kernel<true, true>), grid, block, 0, stream, static_cast<const uint16_t *>(a.input),
+                       a.weight, a.output, a.rows, a.width, a.epsilon);
+  else if (a.input_f32)
     hipLaunchKernelGGL(rms_norm_split_kernel<float>, grid, block, 0, stream, static_cast<const float *>(a.input),
                        a.weight, a.output, a.rows, a.width, a.epsilon);
   else
@@ -483,7 +531,7 @@ hipError_t launch_rms_norm_split(const RmsNormArgs &a, hipStream_t stream) {
 }
 
 hipError_t launch_argmax_reduce(const void *candidates, uint32_t *token_ids, uint32_t rows, hipStream_t stream) {
-  hipLaunchKernelGGL(argmax_reduce_kernel, dim3(rows), dim3(256), 0, stream,
+  hipLaunchKernelGGL(argmax_reduce_kernel, dim3(rows), dim3(64), 0, stream,
                      static_cast<const Candidate *>(candidates), token_ids);
   return hipGetLastError();
 }

@@ -362,6 +362,9 @@ hipError_t launch_nan_scan(const void *data, size_t bytes, bool f32, uint32_t *f
 // half_logits, when not null, receives half(logit) [rows, n].
 hipError_t launch_argmax_candidates(const float *logits, void *candidates, uint32_t rows, uint32_t n, bool pairs,
                                     uint16_t *half_logits, hipStream_t stream);
+// Both: `candidates` is scratch.
+hipError_t launch_argmax(const float *logits, void *candidates, uint32_t *token_ids, uint32_t rows, uint32_t n, bool pairs,
+                         uint16_t *half_logits, hipStream_t stream);
 hipError_t launch_argmax_reduce(const void *candidates, uint32_t *token_ids, uint32_t rows,
                                 hipStream_t stream);
 

@@ -120,12 +120,8 @@ int argmax_f32(llmopt_hip_context *context, const DispatchRecord &record) {
   Scratch scratch;
   const size_t candidates = scratch.want((size_t)rows * 256 * 8);
   if (!scratch.get(context)) return LLMOPT_ERR_FAILURE;
-  if (int status = launched(launch_argmax_candidates(as_f32(record.buffers[0]), scratch.at<void>(candidates), rows, n,
-                                                     false, nullptr, context->stream),
-                            record.name.c_str()))
-    return status;
-  return launched(launch_argmax_reduce(scratch.at<void>(candidates),
-                                       reinterpret_cast<uint32_t *>(record.buffers[1].device), rows, context->stream),
+  return launched(launch_argmax(as_f32(record.buffers[0]), scratch.at<void>(candidates),
+                                reinterpret_cast<uint32_t *>(record.buffers[1].device), rows, n, false, nullptr, context->stream),
                   record.name.c_str());
 }
 

@@ -277,12 +277,10 @@ int lm_head(llmopt_hip_context *context, const DispatchRecord &record, LmHeadVar
       return status;
   }
   uint16_t *half_logits = variant.extra ? as_f16_out(record.buffers[5]) : nullptr;
-  if (int status = launched(launch_argmax_candidates(logits, candidates, m, n, !tiles, half_logits, context->stream),
-                            name))
-    return status;
-  if (variant.stage1) return LLMOPT_OK;
-  return launched(launch_argmax_reduce(candidates, reinterpret_cast<uint32_t *>(record.buffers[4].device), m,
-                                       context->stream),
+  if (variant.stage1)
+    return launched(launch_argmax_candidates(logits, candidates, m, n, !tiles, half_logits, context->stream), name);
+  return launched(launch_argmax(logits, candidates, reinterpret_cast<uint32_t *>(record.buffers[4].device), m, n, !tiles,
+                                half_logits, context->stream),
                   name);
 }
 

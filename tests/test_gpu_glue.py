@@ -437,3 +437,65 @@ def test_swiglu_ffn_three_stage_chain(runtime):
     prod = oracle.silu_mul(gate, up).astype(np.float16)
     expected = oracle.add(oracle.w4a16_linear(prod, down_w, down_s, None), residual.astype(np.float32))
     assert_close_to_oracle(out.numpy(np.float16, (m, k)), expected, "swiglu ffn chain")
+
+
+def argmax_candidate_tree(row):
+    """Slices of every 1024th column, the first one kept until a larger one comes; four slices a candidate; a tree of 256."""
+    better = lambda a, b: a[0] > b[0] or (a[0] == b[0] and a[1] < b[1])
+    best = []
+    for t in range(256):
+        mine = None
+        for slice_ in range(4):
+            columns = range(t + 256 * slice_, len(row), 1024)
+            if not columns:
+                continue
+            found = (row[columns[0]], columns[0])
+            for col in columns[1:]:
+                if row[col] > found[0]:
+                    found = (row[col], col)
+            if mine is None or better(found, mine):
+                mine = found
+        best.append(mine or (np.float32(-3.402823466e+38), 0))
+    for width in (128, 64, 32, 16, 8, 4, 2, 1):
+        best[:width] = [best[i + width] if better(best[i + width], best[i]) else best[i] for i in range(width)]
+    return best[0][1]
+
+
+# one launch and two, ends inside and between the blocks of sixteen columns of a thread
+@pytest.mark.parametrize("rows,n", [(1, 1), (3, 255), (2, 1025), (5, 16384), (1, 16385), (2, 32768), (2, 36864), (3, 36865), (9, 49153),
+                                    (1, 70001)])
+def test_argmax_of_rows(runtime, rows, n):
+    rng = np.random.default_rng(n)
+    logits = rng.integers(-40, 40, (rows, n)).astype(np.float32)  # ties
+    kinds = [logits, np.full((rows, n), -np.inf, dtype=np.float32), np.where(rng.random((rows, n)) < 0.5, np.inf, logits).astype(np.float32)]
+    for values in kinds:
+        out = runtime.create_buffer(rows * 4)
+        runtime.dispatch("llmopt_argmax_f32", [runtime.buffer_of_bytes(values), out], u32s(rows, n), (256, 1, 1), (256, 1, 1))
+        np.testing.assert_array_equal(out.numpy(np.uint32), values.argmax(axis=1))
+
+
+@pytest.mark.parametrize("n", [300, 2500, 36864, 36865])
+def test_argmax_passes_nan_as_a_scan_does(runtime, n):
+    rng = np.random.default_rng(n)
+    values = rng.standard_normal((3, n)).astype(np.float32)
+    values[0, rng.integers(0, n, 40)] = np.nan
+    values[1, :200] = np.nan
+    values[2] = np.nan
+    out = runtime.create_buffer(3 * 4)
+    runtime.dispatch("llmopt_argmax_f32", [runtime.buffer_of_bytes(values), out], u32s(3, n), (256, 1, 1), (256, 1, 1))
+    np.testing.assert_array_equal(out.numpy(np.uint32), [argmax_candidate_tree(row) for row in values])
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 64, 64), (5, 100, 2048), (2, 100, 2112), (1, 300, 576)])
+def test_head_rows_in_registers_and_in_a_loop(runtime, m, n, k):
+    """Rows of up to 2048 values stay in registers, also where the input is not 16-byte aligned they do not."""
+    test_lm_head_argmax(runtime, m, n, k, np.float16, True, False)
+    rng = np.random.default_rng(k)
+    x, packed, scale, _ = w4_case(rng, m, n, k)
+    norm_weight = rng.uniform(0.5, 1.5, k).astype(np.float16)
+    b = runtime.buffer_of_bytes
+    held = b(np.concatenate([np.zeros(1, dtype=np.float16), x.reshape(-1)]))
+    ids, logits = runtime.create_buffer(m * 4), runtime.create_buffer(m * n * 2)
+    runtime.dispatch("llmopt_w4a16_lm_head_argmax_extra_f16", [held.view(2, m * k * 2), b(norm_weight), b(packed), b(scale), ids, logits],
+                     u32s(m, n, k) + struct.pack("<f", 1e-5), (256, 1, 1), (256, 1, 1))
+    assert_close_to_oracle(logits.numpy(np.float16, (m, n)), lm_head_oracle(x, norm_weight, packed, scale, 1e-5), "unaligned rows")
