@@ -282,7 +282,8 @@ hipError_t launch_route_combine(const RouteCombineArgs &args, hipStream_t stream
 // One token: every workgroup selects the experts from the logits itself.
 struct MoeGemvArgs {
   bool f32;
-  const float *logits;  // f32 [experts (+ 1: the shared expert's gate)]
+  const uint16_t *router;  // bf16 [experts (+ 1), width]: the up launch makes the logits; null: they are made
+  float *logits;           // f32 [experts (+ 1: the shared expert's gate)]
   uint32_t experts, top, width, ff, shared_ff;
   const float *x;                 // f32 [width]
   const uint16_t *norm_weight;
@@ -294,6 +295,8 @@ struct MoeGemvArgs {
   float *stream;                  // f32 [width]
   uint32_t activation;
 };
+// The up launch can, and had better, multiply the router itself.
+bool moe_gemv_routes(const MoeGemvArgs &args);
 hipError_t launch_moe_gemv_up(const MoeGemvArgs &args, hipStream_t stream);
 hipError_t launch_moe_gemv_down(const MoeGemvArgs &args, hipStream_t stream);
 

@@ -432,15 +432,18 @@ __device__ __forceinline__ void select_experts(const float *logits, uint32_t exp
 }
 
 // blockIdx.y: choice 0 .. top - 1, or `top`: the shared expert.  A wave owns kUpOutputs hidden values.
-constexpr int kUpOutputs = 4, kUpSteps = 2;
+// ROUTER: every workgroup of a choice multiplies the staged row into the router itself, kRouterRows rows a wave, in the
+// order of the product kernel above (the same bits), and the first one stores the logits for the down launch.
+constexpr int kUpOutputs = 4, kUpSteps = 2, kRouterRows = 5;
 
-template <bool VEC, Staging STAGING>
+template <bool VEC, Staging STAGING, bool ROUTER>
 __global__ __launch_bounds__(256) void moe_gemv_up_kernel(MoeGemvArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   __shared__ float scratch[kWaves];
   const uint32_t plane = ((a.width + 7) >> 3) << 2;
   float *xs = lds, *z = lds + 2 * plane, *weights = z + a.experts;
   uint32_t *ids = reinterpret_cast<uint32_t *>(weights + a.top);
+  float *routed = reinterpret_cast<float *>(ids + a.top);  // ROUTER: the logits
   const bool shared = blockIdx.y == a.top;
   const uint32_t n_total = shared ? a.shared_ff : a.ff;
   if (blockIdx.x * kWaves * kUpOutputs >= n_total) return;
@@ -453,11 +456,10 @@ __global__ __launch_bounds__(256) void moe_gemv_up_kernel(MoeGemvArgs a) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint32_t first = (blockIdx.x * kWaves + wave) * kUpOutputs;
   RowStream<2 * kUpOutputs, VEC, kUpSteps> stream;
-  // the choice is made, and its weights are requested, while the activation is on its way to LDS
-  stage_activation<float, STAGING>(in, xs, plane, scratch, [&] {
+  auto request_expert = [&](const float *logits) __attribute__((always_inline)) {
     uint32_t expert = 0;
     if (!shared) {
-      select_experts<256>(a.logits, a.experts, a.top, z, ids, weights);
+      select_experts<256>(logits, a.experts, a.top, z, ids, weights);
       expert = ids[blockIdx.y];
     }
     const uint16_t *gate = shared ? a.shared_gate : a.gate + (size_t)expert * a.ff * a.width;
@@ -467,7 +469,26 @@ __global__ __launch_bounds__(256) void moe_gemv_up_kernel(MoeGemvArgs a) {
       stream.rows[r] =
           reinterpret_cast<const __bf16 *>((r & 1) ? up : gate) + (size_t)min(first + r / 2, n_total - 1) * a.width;
     stream.request(a.width, lane);
-  });
+  };
+  if (ROUTER && !shared) {
+    const uint32_t columns = a.experts + (a.shared_ff != 0 ? 1 : 0);
+    RowStream<kRouterRows, VEC> router;
+    const uint32_t row = wave * kRouterRows;
+#pragma unroll
+    for (int r = 0; r < kRouterRows; ++r)
+      router.rows[r] = reinterpret_cast<const __bf16 *>(a.router) + (size_t)min(row + r, columns - 1) * a.width;
+    stage_activation<float, STAGING>(in, xs, plane, scratch, [&] { router.request(a.width, lane); });
+    router.run(xs, plane, a.width, lane);
+#pragma unroll
+    for (int r = 0; r < kRouterRows; ++r)
+      if (lane == r && row + r < columns) routed[row + r] = router.sums[r];
+    __syncthreads();
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < columns) a.logits[threadIdx.x] = routed[threadIdx.x];
+    request_expert(routed);
+  } else {
+    // the choice is made, and its weights are requested, while the activation is on its way to LDS
+    stage_activation<float, STAGING>(in, xs, plane, scratch, [&] { request_expert(a.logits); });
+  }
   if (first >= n_total) return;
   stream.run(xs, plane, a.width, lane);
   float g = 0.0f, u = 0.0f;
@@ -548,15 +569,24 @@ hipError_t launch_dense_gemv(const DenseGemvArgs &a, hipStream_t stream) {
   return a.f32 ? pick_gemv<float>(a, stream) : pick_gemv<__bf16>(a, stream);
 }
 
+// Up to as many rows as the four waves take at once: another pass costs what the router's own launch does.  The whole
+// feed-forward, us with the router inside / apart (width, experts, chosen, shared): 1024, 8, 2 + shared 12.2 / 14.3; 1024, 16, 4 +
+// shared 14.6 / 16.7; 2048, 16, 4 + shared 24.0 / 25.7; 4096, 16, 2 27.1 / 28.9; beyond: 1024, 32, 4 + shared 17.0 / 17.6; 2048,
+// 32, 4 + shared 25.0 / 24.7; 1024, 64, 6 + shared 24.3 / 22.3; 2048, 128, 8 40.7 / 29.9.
+bool moe_gemv_routes(const MoeGemvArgs &a) {
+  return a.width % 8 == 0 && a.width <= 4096 && a.experts + (a.shared_ff != 0 ? 1 : 0) <= kWaves * kRouterRows;
+}
+
 hipError_t launch_moe_gemv_up(const MoeGemvArgs &a, hipStream_t stream) {
-  const uint32_t bytes = ((a.width + 7) / 8) * 32 + (a.experts + 2 * a.top) * 4;
+  const uint32_t bytes = ((a.width + 7) / 8) * 32 + (a.experts + 2 * a.top + (a.router ? a.experts + 1 : 0)) * 4;
   if (bytes > 60 * 1024) return hipErrorInvalidValue;
   const uint32_t widest = std::max(a.ff, a.shared_ff);
   const dim3 grid((widest + kUpOutputs * kWaves - 1) / (kUpOutputs * kWaves), a.top + (a.shared_ff ? 1 : 0));
   const bool small = a.width % 4 == 0 && a.width <= 4096;
-  if (a.width % 8 != 0) moe_gemv_up_kernel<false, Staging::kNormed><<<grid, 256, bytes, stream>>>(a);
-  else if (small) moe_gemv_up_kernel<true, Staging::kNormedShort><<<grid, 256, bytes, stream>>>(a);
-  else moe_gemv_up_kernel<true, Staging::kNormed><<<grid, 256, bytes, stream>>>(a);
+  if (a.width % 8 != 0) moe_gemv_up_kernel<false, Staging::kNormed, false><<<grid, 256, bytes, stream>>>(a);
+  else if (small && a.router) moe_gemv_up_kernel<true, Staging::kNormedShort, true><<<grid, 256, bytes, stream>>>(a);
+  else if (small) moe_gemv_up_kernel<true, Staging::kNormedShort, false><<<grid, 256, bytes, stream>>>(a);
+  else moe_gemv_up_kernel<true, Staging::kNormed, false><<<grid, 256, bytes, stream>>>(a);
   return hipGetLastError();
 }
 

@@ -548,7 +548,6 @@ int rms_routed_ffn_add(llmopt_hip_context *context, const DispatchRecord &record
     route.epilogue = GemvEpilogue::kStoreF32;
     route.out_f32 = scratch.at<float>(logits);
     if (!dense_gemv_ok(route)) return fail(LLMOPT_ERR_INVALID, "%s takes rows of at most 36864 values", name);
-    if (int status = launched(launch_dense_gemv(route, context->stream), name)) return status;
     MoeGemvArgs a = {};
     a.f32 = F32;
     a.logits = scratch.at<float>(logits);
@@ -569,6 +568,11 @@ int rms_routed_ffn_add(llmopt_hip_context *context, const DispatchRecord &record
     a.hidden = scratch.at<float>(hidden);
     a.stream = stream;
     a.activation = activation;
+    if (moe_gemv_routes(a)) {
+      a.router = router;
+    } else if (int status = launched(launch_dense_gemv(route, context->stream), name)) {
+      return status;
+    }
     if (int status = launched(launch_moe_gemv_up(a, context->stream), name)) return status;
     return launched(launch_moe_gemv_down(a, context->stream), name);
   }

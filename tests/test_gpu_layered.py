@@ -393,3 +393,36 @@ def test_sizes_of_a_real_layer(runtime, dtype):
     for index in range(2):
         assert_close(got[index], streams[index], dtype, index)
     assert_close(logits, expected[[0, 1, 255, 256, 329]], dtype)
+
+
+# the router inside the launch of the experts (up to twenty rows with the shared expert's gate, whole pieces, up to 4096
+# values) and in a launch of its own
+@pytest.mark.parametrize("width,experts,top,ff,shared", [
+    (8, 3, 2, 16, 0), (1024, 19, 4, 40, 24), (1024, 20, 4, 40, 0), (2056, 5, 1, 33, 50), (4096, 2, 2, 64, 0),
+    (1024, 20, 4, 40, 24), (1024, 21, 4, 40, 0), (4104, 4, 2, 24, 0), (1028, 4, 2, 24, 8)])
+def test_experts_of_one_token_and_their_router(runtime, width, experts, top, ff, shared):
+    """Float32 sums of up to 4104 products: 1e-5 covers sqrt(K) 2^-24 of each of three products in a row several times."""
+    import struct
+    from llmopt_amd.safetensors_file import from_bfloat16, to_bfloat16
+    rng = np.random.default_rng(width + experts)
+    put = runtime.buffer_of_bytes
+    shapes = [(width,), (experts + (shared > 0), width), (experts, ff, width), (experts, ff, width), (experts, width, ff),
+              (max(shared, 1), width), (max(shared, 1), width), (width, max(shared, 1))]
+    patterns = [to_bfloat16((rng.standard_normal(s) * (1.0 if len(s) == 1 else s[-1] ** -0.5)).astype(np.float32)) for s in shapes]
+    norm, router, gate, up, down, s_gate, s_up, s_down = (from_bfloat16(p).reshape(s).astype(np.float64)
+                                                         for p, s in zip(patterns, shapes))
+    x = rng.standard_normal(width).astype(np.float32)
+    h = x / np.sqrt(np.mean(x.astype(np.float64) ** 2) + 1e-6) * norm
+    logits = router @ h
+    chosen = np.argsort(-logits[:experts], kind="stable")[:top]
+    weights = np.exp(logits[chosen] - logits[chosen[0]])
+    silu = lambda z: z / (1.0 + np.exp(-z))
+    add = sum(w * (down[e] @ (silu(gate[e] @ h) * (up[e] @ h))) for w, e in zip(weights / weights.sum(), chosen))
+    if shared:
+        add = add + s_down @ (silu(s_gate @ h) * (s_up @ h)) / (1.0 + np.exp(-logits[experts]))
+    for _ in range(2):  # (a second time on the same scratch)
+        stream = put(x)
+        runtime.dispatch("llmopt_rms_routed_ffn_add_bf16", [stream] + [put(p) for p in patterns],
+                         struct.pack("<6IfI", 1, width, experts, top, ff, shared, 1e-6, 0), (1, 1, 1), (256, 1, 1))
+        got = stream.numpy(np.float32).astype(np.float64) - x
+        assert np.linalg.norm(got - add) <= 1e-5 * np.linalg.norm(add) + 2.0 ** -24 * np.linalg.norm(x)
