@@ -58,6 +58,17 @@ __device__ __forceinline__ void store4(T *out, f32x4 v, uint32_t count, bool vec
 __device__ __forceinline__ void mix_values(const DenseLinearArgs &a, uint32_t r, uint32_t c, f32x4 &v) {
   if (a.mix.mode == 0 || c + 3 < a.split) return;
   const uint32_t n_v = a.n - a.split;
+  if (c >= a.split && c + 4 <= a.n && ((n_v | (c - a.split)) & 3) == 0 && (reinterpret_cast<uintptr_t>(a.mix.v_first) & 15) == 0) {
+    f32x4 *first = reinterpret_cast<f32x4 *>(a.mix.v_first + (size_t)r * n_v + (c - a.split));
+    if (a.mix.mode == 1) {
+      *first = v;
+    } else {
+      const f32x4 other = *first;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (1.0f - a.mix.lambda) * v[i] + a.mix.lambda * other[i];
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     if (c + i < a.n && c + i >= a.split) {
@@ -468,6 +479,334 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParam
                            stage_rows + wave * 16 * (NT * 16 + 8));
 }
 
+// A barrier that nothing moves across.
+__device__ __forceinline__ void meet() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("" ::: "memory");
+}
+template <int COUNT>
+__device__ __forceinline__ void copies_landed() {  // all but the last COUNT
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(COUNT) : "memory");
+}
+__device__ __forceinline__ void lds_read() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// The same product for large launches: 256 x 256 tiles of eight waves, two on a SIMD, of which one reads operands and
+// requests copies while the other one multiplies.  With all waves in step (dense_gemm_direct_kernel) the matrix cores had
+// work half of the time: LDS reads are a fifth of it, and what a copy's trip to memory takes hardly counts (activations that
+// were all in L2 gave 5%).
+//
+//  * A wave's 128 x 64 outputs are four quadrants of 64 x 32, a phase each: operands into registers, a barrier, sixteen
+//    products, a barrier.  Waves 4 .. 7 are a barrier behind, so that their products fall into the others' reads.
+//  * A stage of 64 K values is four halves of 16 KB (rows 0, rows 1, columns 0, columns 1), which are read in a phase each:
+//    columns 0 of the next stage in the last phase, so that no phase reads more than eight operands.  The two phases behind
+//    that (the second group is one barrier behind, and its reads have returned when its products start), the half's place is
+//    requested again for two stages later: five halves are under way, waited for by count.
+//  * The order of a sum's products is that of dense_gemm_direct_kernel: results are the same.
+// us, 256 x 256 tiles of that kernel / these: 2048 x (2 x 8192) x 2048 gated 127 / 106, 3001 x (2 x 8192) x 2048 196 / 157,
+// 4096 x 4096 x 8192 207 / 179 (1.53 PFLOP/s), 8192 x 8192 x 4096 416 / 367.
+template <int GATED>
+__global__ __launch_bounds__(512) void dense_gemm_phased_kernel(GemmParams p) {
+  constexpr int BM = 256, BN = 256, COLUMNS = GATED ? BN / 2 : BN, HALF = 16384, STAGE = 4 * HALF;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const DenseLinearArgs &a = p.a;
+  TilePlace place;
+  if (!place_tile<BM, COLUMNS, false>(p, place)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+
+  // Rows of half h: h * 64 .. + 63 of each 128; columns: h * 32 .. + 31 of each 64 (a wave's own lie together).
+  enum { kRows0, kRows1, kColumns0, kColumns1 };
+  const __bf16 *source[4][2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int row = (c * 8 + wave) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t at = (row >> 6) * 128 + h * 64 + (row & 63);
+      source[h][c] = static_cast<const __bf16 *>(a.x) + (size_t)(place.m_first + min(at, place.m_rows - 1)) * a.ldx + piece * 8;
+      const int w_row = (row >> 5) * 64 + h * 32 + (row & 31);
+      const uint16_t *matrix = a.w;
+      uint32_t col = place.n_first + w_row;
+      if (GATED) {
+        if ((w_row >> 4) & 1) matrix = a.w_up;
+        col = place.n_first + (w_row >> 5) * 16 + (w_row & 15);
+      }
+      col = min(col, a.n - 1);
+      source[2 + h][c] = reinterpret_cast<const __bf16 *>(matrix) + (size_t)col * a.k + piece * 8;
+    }
+  }
+  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)lds;
+  auto request = [&](int half, int step) __attribute__((always_inline)) {
+    const uint32_t slot = lds_base + (step & 1) * STAGE + half * HALF;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) copy_to_lds(source[half][c] + step * kStageK, slot + (c * 8 + wave) * 1024);
+  };
+  f32x4 acc[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int steps = (int)(a.k / kStageK);
+  const int fr = lane & 15, quad = lane >> 4, twist = (fr >> 1) & 7;
+  const int at0 = (quad ^ twist) * 16, at1 = ((4 + quad) ^ twist) * 16;
+  const int read_a = (wm * 64 + fr) * 128, read_b = (wn * 32 + fr) * 128 + 2 * HALF;
+  bf16x8 fa[4][2], fb0[2][2][2], fb1[2][2];
+  auto read_rows = [&](int half, int step) __attribute__((always_inline)) {
+    const char *base = lds + (step & 1) * STAGE + half * HALF + read_a;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      fa[i][0] = *reinterpret_cast<const bf16x8 *>(base + i * 2048 + at0);
+      fa[i][1] = *reinterpret_cast<const bf16x8 *>(base + i * 2048 + at1);
+    }
+  };
+  auto read_columns = [&](bf16x8 (&fb)[2][2], int half, int step) __attribute__((always_inline)) {
+    const char *base = lds + (step & 1) * STAGE + half * HALF + read_b;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      fb[j][0] = *reinterpret_cast<const bf16x8 *>(base + j * 2048 + at0);
+      fb[j][1] = *reinterpret_cast<const bf16x8 *>(base + j * 2048 + at1);
+    }
+  };
+  auto multiply = [&](const bf16x8 (&fb)[2][2], int i0, int j0) __attribute__((always_inline)) {
+    lds_read();
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i0 * 4 + i][j0 * 2 + j] = mma(fb[j][kk], fa[i][kk], acc[i0 * 4 + i][j0 * 2 + j]);
+    __builtin_amdgcn_s_setprio(0);
+  };
+  request(kColumns0, 0), request(kRows0, 0), request(kColumns1, 0), request(kRows1, 0);
+  if (steps > 1) {
+    request(kColumns0, 1), request(kRows0, 1), request(kColumns1, 1);
+    copies_landed<10>();
+  } else {
+    copies_landed<4>();
+  }
+  meet();
+  read_columns(fb0[0], 0, 0);
+  lds_read();
+  meet();
+  if (wm == 1) meet();
+  auto step = [&](int t, const bf16x8 (&now)[2][2], bf16x8 (&next)[2][2]) __attribute__((always_inline)) {
+    const bool more = t + 1 < steps, more2 = t + 2 < steps;
+    read_rows(0, t);
+    if (more) {
+      request(kRows1, t + 1);
+      copies_landed<10>();
+    } else {
+      copies_landed<2>();
+    }
+    meet();
+    multiply(now, 0, 0);
+    meet();
+    read_columns(fb1, 1, t);
+    if (more2) {
+      request(kColumns0, t + 2);
+      copies_landed<10>();
+    } else if (more) {
+      copies_landed<8>();
+    } else {
+      copies_landed<0>();
+    }
+    meet();
+    multiply(fb1, 0, 1);
+    meet();
+    read_rows(1, t);
+    if (more2) {
+      request(kRows0, t + 2);
+      copies_landed<10>();
+    } else {
+      copies_landed<6>();
+    }
+    meet();
+    multiply(fb1, 1, 1);
+    meet();
+    if (more) read_columns(next, 0, t + 1);
+    if (more2) {
+      request(kColumns1, t + 2);
+      copies_landed<10>();
+    } else {
+      copies_landed<4>();
+    }
+    meet();
+    multiply(now, 1, 0);
+    meet();
+  };
+  int t = 0;
+  for (; t + 1 < steps; t += 2) {
+    step(t, fb0[0], fb0[1]);
+    step(t + 1, fb0[1], fb0[0]);
+  }
+  if (t < steps) step(t, fb0[0], fb0[1]);
+  if (wm == 0) meet();
+  if (a.epilogue == DenseEpilogue::kAdd || a.epilogue == DenseEpilogue::kStoreF32) {
+    emit_tile<__bf16, 8, 4, GATED>(a, acc, place.m_first, place.m_rows, place.n_first, wm * 128, wn * 64, lane);
+    return;
+  }
+  __syncthreads();
+  emit_rows<8, 4, GATED>(a, acc, place.m_first, place.m_rows, place.n_first, wm * 128, wn * 64, lane,
+                         reinterpret_cast<__bf16 *>(lds) + wave * 16 * (4 * 16 + 8));
+}
+
+// The same product for launches of about a round of middle tiles: two groups of four waves (2 x 2, a wave on every SIMD) take
+// the stages of 64 K values in turn, each for the whole tile; while one multiplies, the other one reads its operands, and
+// their sums meet in LDS at the end.  A wave's tile is twice as large as with eight waves on a stage, so that the operands
+// of a product come to two thirds of the LDS reads, and a stage is two barriers for a group whose products last between them.
+// A stage's place is free behind the barrier that ends its reads and is requested in the next turn, by the other group:
+// an odd STAGES requests a group's own stages, an even one the other group's.
+// us, eight waves in step / in turns: 128 x 128 tiles 2048 x 2048 x 4096 41 / 33, x 8192 83 / 60 (1.15 PFLOP/s); 192 x 128
+// 3001 x 2048 x 4096 54 / 44, x 8192 103 / 80 (1.26 PFLOP/s).
+template <int BM, int BN, int STAGES, int GATED, bool ROUTED>
+__global__ __launch_bounds__(512) void dense_gemm_turns_kernel(GemmParams p) {
+  constexpr int COLUMNS = GATED ? BN / 2 : BN, MT = BM / 32, NT = BN / 32, ROWS = BM + BN;
+  constexpr int COPIES = ROWS / 32;  // 8-row copies of a wave and step
+  constexpr int BEHIND = STAGES % 2 ? (STAGES - 3) / 2 * COPIES : COPIES;  // copies that may be under way when the next step has landed
+  static_assert(MT % 2 == 0 && (!GATED || NT % 2 == 0) && ROWS % 32 == 0 && STAGES >= 3, "tile");
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const DenseLinearArgs &a = p.a;
+  TilePlace place;
+  if (!place_tile<BM, COLUMNS, ROUTED>(p, place)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wave >> 2, own = wave & 3, wm = own >> 1, wn = own & 1;
+
+  const __bf16 *source[COPIES];
+#pragma unroll
+  for (int i = 0; i < COPIES; ++i) {
+    const int row = (i * 4 + own) * 8 + (lane >> 3);
+    const int piece = (lane & 7) ^ ((row >> 1) & 7);
+    if (row < BM) {
+      uint32_t r = place.m_first + min((uint32_t)row, place.m_rows - 1);
+      if (ROUTED && a.row_source) r = a.row_source[r];
+      source[i] = static_cast<const __bf16 *>(a.x) + (size_t)r * a.ldx + piece * 8;
+    } else {
+      const int w_row = row - BM;
+      const uint16_t *matrix = a.w;
+      uint32_t c = place.n_first + w_row;
+      if (GATED) {
+        if ((w_row >> 4) & 1) matrix = a.w_up;
+        c = place.n_first + (w_row >> 5) * 16 + (w_row & 15);
+      }
+      c = min(c, a.n - 1);
+      source[i] = reinterpret_cast<const __bf16 *>(matrix) + ((size_t)place.expert * a.n + c) * a.k + piece * 8;
+    }
+  }
+  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)lds;
+  auto request = [&](int step) __attribute__((always_inline)) {
+    const uint32_t slot = lds_base + (step % STAGES) * ROWS * 128;
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) copy_to_lds(source[i] + step * kStageK, slot + (i * 4 + own) * 1024);
+  };
+  f32x4 acc[2][MT / 2][NT];  // of the upper and the lower half of the wave's rows
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i / (MT / 2)][i % (MT / 2)][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int steps = (int)(a.k / kStageK);
+  const int fr = lane & 15, quad = lane >> 4, twist = (fr >> 1) & 7;
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < steps && ((s - (STAGES - 1)) & 1) == group) request(s);
+  if (steps >= STAGES - 1) copies_landed<BEHIND>();
+  else copies_landed<0>();
+  meet();
+  if (group == 1) meet();
+  for (int s = group; s < steps; s += 2) {
+    const char *rows = lds + (s % STAGES) * ROWS * 128;
+    const char *la = rows + (wm * (BM / 2) + fr) * 128, *lw = rows + (BM + wn * (BN / 2) + fr) * 128;
+    bf16x8 fa[MT][2], fw[NT][2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int at = ((kk * 4 + quad) ^ twist) * 16;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) fw[j][kk] = *reinterpret_cast<const bf16x8 *>(lw + j * 2048 + at);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) fa[i][kk] = *reinterpret_cast<const bf16x8 *>(la + i * 2048 + at);
+    }
+    const bool more = s + STAGES - 1 < steps;
+    if (more) request(s + STAGES - 1);
+    if (STAGES % 2 == 0) {
+      if (more) copies_landed<BEHIND>();
+      else copies_landed<0>();
+    }
+    lds_read();  // read: the slot is free behind the barrier
+    meet();
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          f32x4 &sum = acc[i / (MT / 2)][i % (MT / 2)][j];
+          sum = mma(fw[j][kk], fa[i][kk], sum);
+        }
+    __builtin_amdgcn_s_setprio(0);
+    if (STAGES % 2 == 1) {
+      if (more) copies_landed<BEHIND>();
+      else copies_landed<0>();
+    }
+    meet();
+  }
+  if ((steps & 1) == group) meet();
+  // The groups' sums meet: each finishes half of the rows.
+  if (group == 1) {
+#pragma unroll
+    for (int i = 0; i < MT / 2; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const f32x4 v = acc[0][i][j];
+        acc[0][i][j] = acc[1][i][j];
+        acc[1][i][j] = v;
+      }
+  }
+  constexpr int PART = MT / 2 * NT * 1024;
+  char *mine = lds + wave * PART + lane * 16, *other = lds + (wave ^ 4) * PART + lane * 16;
+#pragma unroll
+  for (int i = 0; i < MT / 2; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4 *>(mine + (i * NT + j) * 1024) = acc[1][i][j];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < MT / 2; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(other + (i * NT + j) * 1024);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[0][i][j][e] += v[e];
+    }
+  const int row_offset = wm * (BM / 2) + group * (BM / 4);
+  if (a.epilogue == DenseEpilogue::kAdd || a.epilogue == DenseEpilogue::kStoreF32) {
+    emit_tile<__bf16, MT / 2, NT, GATED>(a, acc[0], place.m_first, place.m_rows, place.n_first, row_offset, wn * (BN / 2), lane);
+    return;
+  }
+  __syncthreads();  // the sums are read
+  emit_rows<MT / 2, NT, GATED>(a, acc[0], place.m_first, place.m_rows, place.n_first, row_offset, wn * (BN / 2), lane,
+                               reinterpret_cast<__bf16 *>(lds) + wave * 16 * (NT * 16 + 8));
+}
+template <int BM, int BN, int STAGES, int GATED, bool ROUTED>
+hipError_t run_turns(const DenseLinearArgs &a, hipStream_t stream) {
+  constexpr int bytes = STAGES * (BM + BN) * 128;
+  static bool allowed[kMaxDevices] = {};
+  const auto kernel = dense_gemm_turns_kernel<BM, BN, STAGES, GATED, ROUTED>;
+  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
+  dim3 grid;
+  const GemmParams p = gemm_params<BM, GATED ? BN / 2 : BN, ROUTED>(a, &grid);
+  kernel<<<grid, 512, bytes, stream>>>(p);
+  return hipGetLastError();
+}
+
 template <int BM, int BN, int WM, int WAVES, int STAGES, int GATED, bool ROUTED>
 hipError_t run_direct(const DenseLinearArgs &a, hipStream_t stream) {
   constexpr int bytes = STAGES * (BM + BN) * 128;
@@ -481,6 +820,18 @@ hipError_t run_direct(const DenseLinearArgs &a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <int GATED>
+hipError_t run_phased(const DenseLinearArgs &a, hipStream_t stream) {
+  constexpr int bytes = 2 * 4 * 16384;
+  static bool allowed[kMaxDevices] = {};
+  const auto kernel = dense_gemm_phased_kernel<GATED>;
+  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
+  dim3 grid;
+  const GemmParams p = gemm_params<256, GATED ? 128 : 256, false>(a, &grid);
+  kernel<<<grid, 512, bytes, stream>>>(p);
+  return hipGetLastError();
+}
+
 // Rows whose length is no multiple of the stage, and float32 rows: through registers.
 template <typename T, int BM, int GATED, bool ROUTED>
 hipError_t run_registers(const DenseLinearArgs &a, hipStream_t stream) {
@@ -491,7 +842,7 @@ hipError_t run_registers(const DenseLinearArgs &a, hipStream_t stream) {
 template <int GATED>
 hipError_t pick_routed(const DenseLinearArgs &a, hipStream_t stream) {
   const bool direct = !a.f32 && a.k % kStageK == 0 && a.ldx % 8 == 0;
-  if (a.tile == 128) return direct ? run_direct<128, 128, 2, 4, 2, GATED, true>(a, stream) : hipErrorInvalidValue;
+  if (a.tile == 128) return direct ? run_turns<128, 128, 5, GATED, true>(a, stream) : hipErrorInvalidValue;
   if (direct) return run_direct<64, 128, 2, 4, 3, GATED, true>(a, stream);
   return a.f32 ? run_registers<float, 64, GATED, true>(a, stream) : run_registers<__bf16, 64, GATED, true>(a, stream);
 }
@@ -500,8 +851,8 @@ template <int GATED>
 hipError_t pick_gemm(const DenseLinearArgs &a, hipStream_t stream) {
   if (a.f32) return run_registers<float, 32, GATED, false>(a, stream);
   if (a.k % kStageK != 0 || a.ldx % 8 != 0) return run_registers<__bf16, 32, GATED, false>(a, stream);
-  switch (dense_tile(a.m, (uint64_t)a.n * (GATED ? 2 : 1), a.k, (uint32_t)device_compute_units())) {
-    case DenseTile::k256x256: return run_direct<256, 256, 2, 8, 2, GATED, false>(a, stream);
+  switch (dense_product_tile(a.m, (uint64_t)a.n * (GATED ? 2 : 1), a.k, (uint32_t)device_compute_units())) {
+    case DenseTile::k256x256: return run_phased<GATED>(a, stream);
     case DenseTile::k128x128: return run_direct<128, 128, 2, 4, 2, GATED, false>(a, stream);
     case DenseTile::k192x128: return run_direct<192, 128, 2, 4, 2, GATED, false>(a, stream);
     case DenseTile::k128x192: return run_direct<128, 192, 2, 4, 2, GATED, false>(a, stream);
@@ -511,6 +862,11 @@ hipError_t pick_gemm(const DenseLinearArgs &a, hipStream_t stream) {
     case DenseTile::k64x64: return run_direct<64, 64, 2, 4, 4, GATED, false>(a, stream);
     case DenseTile::k32x64: return run_direct<32, 64, 2, 4, 6, GATED, false>(a, stream);
     case DenseTile::k64x128: return run_direct<64, 128, 2, 4, 3, GATED, false>(a, stream);
+    case DenseTile::kTurns192x128: return run_turns<192, 128, 3, GATED, false>(a, stream);
+    case DenseTile::kTurns128x128: return run_turns<128, 128, 5, GATED, false>(a, stream);
+    case DenseTile::kTurns128x192: return run_turns<128, 192, 3, GATED, false>(a, stream);
+    case DenseTile::kTurns256x128: return run_turns<256, 128, 3, GATED, false>(a, stream);
+    case DenseTile::kTurns128x64: return run_turns<128, 64, 5, GATED, false>(a, stream);
   }
   return hipErrorInvalidValue;
 }

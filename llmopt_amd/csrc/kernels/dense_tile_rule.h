@@ -6,9 +6,13 @@
 
 namespace llmopt {
 
-enum class DenseTile { k256x256, k128x128, k192x128, k128x192, k192x128Eight, k128x128Eight, k64x128Eight, k64x64, k32x64, k64x128 };
+// (the turns: two groups of four waves that take stages in turn)
+enum class DenseTile {
+  k256x256, k128x128, k192x128, k128x192, k192x128Eight, k128x128Eight, k64x128Eight, k64x64, k32x64, k64x128,
+  kTurns192x128, kTurns128x128, kTurns128x192, kTurns256x128, kTurns128x64
+};
 
-// Tiles in that order, and an estimate of a launch on 256 CUs (us, K in 1024, weights from HBM).  `start` comes once, and a
+// The first ten in that order, and an estimate of a launch on 256 CUs (us, K in 1024, weights from HBM).  `start` comes once, and a
 // round of workgroups takes a constant, its start and its outputs, and a part that goes with K: with one workgroup on a CU,
 // and with two where the tile's ring leaves room for them (`two_k` == 0: it takes the CU).  A last round on few CUs takes the
 // share `few` of a whole one, which grows evenly to the whole.  The step from one workgroup on a CU to two comes to the share
@@ -19,7 +23,7 @@ struct TileTime {
   float start, one, one_k, few, two, two_k, pair, span;
 };
 constexpr TileTime kTileTimes[] = {
-    {256, 256, 0.01f, 14.10f, 24.56f, 1.00f, 0.00f, 0.00f, 0.00f, 0.00f},     // 8 waves, 2 stages
+    {256, 256, 0.01f, 14.10f, 24.56f, 1.00f, 0.00f, 0.00f, 0.00f, 0.00f},     // 8 waves, 2 stages, all in step
     {128, 128, 0.00f, 7.54f, 20.73f, 0.47f, 8.85f, 15.57f, 0.02f, 0.65f},     // 4 waves, 2 stages
     {192, 128, 0.00f, 7.79f, 14.79f, 1.00f, 11.91f, 19.36f, 1.00f, 0.06f},    // 4 waves, 2 stages
     {128, 192, 5.82f, 1.85f, 15.16f, 1.00f, 7.30f, 21.46f, 0.99f, 0.17f},     // 4 waves, 2 stages
@@ -37,7 +41,7 @@ constexpr TileTime kTileTimes[] = {
 // every CU work, which is more than 3% ahead at 29 of them.  An estimate of rounds that go with K alone was 0.8% off, and
 // behind that tile by more than 3% at 72 (us, that tile / such an estimate: 384 x 2816 x 8192 41.0 / 52.0, 700 x 1500 x 8192 41.5
 // / 50.4, 300 x 12288 x 512 12.4 / 13.4: these are back; 384 x 3072 x 8192, with 288 tiles of 64 x 64, 43.6 / 52.5 is not).
-inline DenseTile dense_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus) {
+inline DenseTile dense_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus, float *estimate = nullptr) {
   int best = 0;
   float least = 3.4e38f;
   for (int i = 0; i < (int)(sizeof(kTileTimes) / sizeof(kTileTimes[0])); ++i) {
@@ -56,7 +60,44 @@ inline DenseTile dense_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t c
     }
     if (time < least) least = time, best = i;
   }
+  if (estimate != nullptr) *estimate = least;
   return (DenseTile)best;
+}
+
+// The same estimate for the tiles whose waves multiply and read at different times, one workgroup on a CU: a fit at 1700 sizes
+// (8 to 3001 rows, 64 to 16384 columns, K 64 to 8192, 640 MB of weights in turn).
+struct StaggeredTime {
+  DenseTile tile;
+  uint32_t rows, columns;
+  float start, one, one_k, few;
+};
+constexpr StaggeredTime kStaggeredTimes[] = {
+    {DenseTile::k256x256, 256, 256, 2.83f, 7.36f, 20.88f, 0.66f},      // 8 waves, 2 stages
+    {DenseTile::kTurns192x128, 192, 128, 2.04f, 5.54f, 10.32f, 0.73f}, // 2 x 4 waves, 3 stages
+    {DenseTile::kTurns128x128, 128, 128, 1.75f, 4.03f, 7.81f, 0.78f},  // 2 x 4 waves, 5 stages
+    {DenseTile::kTurns128x192, 128, 192, 3.31f, 4.26f, 10.58f, 0.72f}, // 2 x 4 waves, 3 stages
+    {DenseTile::kTurns256x128, 256, 128, 1.98f, 7.19f, 11.84f, 0.69f}, // 2 x 4 waves, 3 stages
+    {DenseTile::kTurns128x64, 128, 64, 1.88f, 2.42f, 5.50f, 0.76f},    // 2 x 4 waves, 5 stages
+};
+
+// The tile a product runs on: one of the ten, or from K = 1024 on (below, what the meeting of two groups' sums costs is not
+// made up for) one of these where its estimate is 7% less.  The two estimates are fits to launches of their own, and 7% keeps
+// the cases that lose by that few: of the 649 sizes beyond 12 us the choice is 4.6% faster than the ten on average and more
+// than 3% slower at 17 (us, ten / this: 2048 x 2048 x 8192 74 / 63, 3001 x 2048 x 8192 100 / 83, 2048 x 6144 x 2048
+// 50.7 / 46.8, 700 x 2048 x 2048 15.6 / 14.0; the other way 994 x 2816 x 1152 14.0 / 15.1, 1008 x 1088 x 4288 25.9 / 27.8).
+inline DenseTile dense_product_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus) {
+  float least = 0.0f;
+  DenseTile best = dense_tile(m, columns, k, cus, &least);
+  if (k < 1024) return best;
+  least *= 0.93f;
+  for (const StaggeredTime &t : kStaggeredTimes) {
+    const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns), rest = tiles % cus;
+    const float one = t.one + t.one_k * (float)k / 1024.0f;
+    float time = t.start + (float)(tiles / cus) * one;
+    if (rest > 0) time += one * (t.few + (1.0f - t.few) * (float)rest / (float)cus);
+    if (time < least) least = time, best = t.tile;
+  }
+  return best;
 }
 
 }  // namespace llmopt

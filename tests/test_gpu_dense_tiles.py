@@ -124,3 +124,58 @@ def test_rows_split_in_two(runtime, m, n, k):
                      u32s(m, k, heads, vdim, 1, states, 4, 1) + struct.pack("<f", 1e-6), *GRID)
     assert_rows(from_bfloat16(out.numpy(np.uint16)).reshape(m, columns).astype(np.float64), h, fweight[:columns])
     assert_rows(steps.numpy(np.float32, (m, heads)).astype(np.float64), h, fweight[columns:])
+
+
+# Tiles whose waves multiply and read at different times: 256 x 256, in turns 192 x 128, 128 x 128, 128 x 192, 256 x 128 and
+# 128 x 64, each with remainders, an even and an odd number of stages (test_tile_rules.py checks which sizes take which)
+STAGGERED = [(1345, 6001, 1024), (3000, 3001, 1088), (3000, 1500, 1024), (1345, 3001, 1088), (1345, 1500, 1024),
+             (200, 9503, 1088), (500, 9503, 1152), (500, 9503, 1088), (1345, 5001, 1024), (1345, 5001, 1088),
+             (257, 4095, 1024), (200, 5001, 1088)]
+
+
+@pytest.mark.parametrize("m,n,k", STAGGERED)
+def test_staggered_tiles(runtime, m, n, k):
+    test_tiles(runtime, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", STAGGERED)
+def test_staggered_tiles_of_rows(runtime, m, n, k):
+    test_rows_with_mixed_values(runtime, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", STAGGERED)
+def test_staggered_tiles_of_pairs(runtime, m, n, k):
+    test_gated_tiles(runtime, m, k, n // 2)
+
+
+# tiles of 128 rows of an expert: 1 to 5 stages and 16, experts with a remainder
+@pytest.mark.parametrize("m,width,ff", [(200, 64, 128), (400, 128, 64), (333, 192, 320), (250, 256, 192), (1024, 1024, 320)])
+def test_routed_tiles(runtime, m, width, ff):
+    rng = np.random.default_rng(m + ff)
+    experts, top = 5, 2
+    stream = rng.standard_normal((m, width)).astype(np.float32)
+    norm, fnorm = values(rng, width)
+    router, frouter = values(rng, experts, width, gain=width ** -0.5)
+    (gate, fgate), (up, fup) = (values(rng, experts, ff, width, gain=width ** -0.5) for _ in range(2))
+    down, fdown = values(rng, experts, width, ff, gain=ff ** -0.5)
+    put = runtime.buffer_of_bytes
+    out, none = put(stream), put(np.zeros(width, dtype=np.uint16))
+    runtime.dispatch("llmopt_rms_routed_ffn_add_bf16", [out] + [put(a) for a in (norm, router, gate, up, down)] + [none] * 3,
+                     u32s(m, width, experts, top, ff, 0) + struct.pack("<f", 1e-6) + u32s(0), *GRID)
+    x = stream.astype(np.float64)
+    h = x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-6) * fnorm
+    scores = h @ frouter.T
+    order = np.sort(scores, axis=1)
+    clear = order[:, -top] - order[:, -top - 1] > 0.1  # (a close call may go the other way with rounded rows)
+    chosen = np.argsort(-scores, axis=1)[:, :top]
+    weights = np.exp(np.take_along_axis(scores, chosen, 1))
+    weights /= weights.sum(axis=1, keepdims=True)
+    expected = np.zeros_like(x)
+    for e in range(experts):
+        g = h @ fgate[e].T
+        y = (g / (1.0 + np.exp(-g)) * (h @ fup[e].T)) @ fdown[e].T
+        expected += np.where(chosen == e, weights, 0.0).sum(axis=1, keepdims=True) * y
+    error = (out.numpy(np.float32, (m, width)) - x - expected)[clear]
+    # normed rows, products and an expert's outputs are rounded to bfloat16 (half a unit, 2^-9, each), and the weights of the
+    # experts follow from scores of rounded rows
+    assert clear.sum() > m // 2 and np.sqrt(np.mean(error ** 2)) <= 6 * 2.0 ** -9 * np.sqrt(np.mean(expected[clear] ** 2))
