@@ -29,6 +29,11 @@ constexpr int kStageK = 64;
 struct GemmParams {
   DenseLinearArgs a;
   uint32_t tiles_m, tiles_n, total, per_xcd;
+  uint32_t first_column;  // of the launch; its tiles end with a.n or with the columns of another launch
+};
+
+struct Columns {
+  uint32_t first, end;
 };
 
 template <typename T>
@@ -146,7 +151,7 @@ __device__ __forceinline__ bool place_tile(const GemmParams &p, TilePlace &t) {
   const uint32_t rows_here = min(8u, p.tiles_m - group * 8);
   t.m_first = (group * 8 + within % rows_here) * BM;
   t.m_rows = min((uint32_t)BM, a.m - t.m_first);
-  t.n_first = within / rows_here * COLUMNS;
+  t.n_first = p.first_column + within / rows_here * COLUMNS;
   return true;
 }
 
@@ -293,10 +298,11 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_kernel(GemmParams p) {
 }
 
 template <int BM, int COLUMNS, bool ROUTED>
-GemmParams gemm_params(const DenseLinearArgs &a, dim3 *grid) {
+GemmParams gemm_params(const DenseLinearArgs &a, dim3 *grid, Columns c) {
   GemmParams p = {};
   p.a = a;
-  p.tiles_n = (a.n + COLUMNS - 1) / COLUMNS;
+  p.first_column = c.first;
+  p.tiles_n = (c.end - c.first + COLUMNS - 1) / COLUMNS;
   if (ROUTED) {
     *grid = dim3(p.tiles_n, a.tiles);
   } else {
@@ -317,7 +323,7 @@ hipError_t run_gemm(const DenseLinearArgs &a, hipStream_t stream) {
             reinterpret_cast<const void *>(dense_gemm_kernel<T, BM, BN, WM, GATED, ROUTED, VEC, WAVES>), bytes, allowed))
       return status;
   dim3 grid;
-  const GemmParams p = gemm_params<BM, GATED ? BN / 2 : BN, ROUTED>(a, &grid);
+  const GemmParams p = gemm_params<BM, GATED ? BN / 2 : BN, ROUTED>(a, &grid, {0, a.n});
   dense_gemm_kernel<T, BM, BN, WM, GATED, ROUTED, VEC, WAVES><<<grid, WAVES * 64, bytes, stream>>>(p);
   return hipGetLastError();
 }
@@ -796,38 +802,38 @@ __global__ __launch_bounds__(512) void dense_gemm_turns_kernel(GemmParams p) {
                                reinterpret_cast<__bf16 *>(lds) + wave * 16 * (NT * 16 + 8));
 }
 template <int BM, int BN, int STAGES, int GATED, bool ROUTED>
-hipError_t run_turns(const DenseLinearArgs &a, hipStream_t stream) {
+hipError_t run_turns(const DenseLinearArgs &a, Columns c, hipStream_t stream) {
   constexpr int bytes = STAGES * (BM + BN) * 128;
   static bool allowed[kMaxDevices] = {};
   const auto kernel = dense_gemm_turns_kernel<BM, BN, STAGES, GATED, ROUTED>;
   if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
   dim3 grid;
-  const GemmParams p = gemm_params<BM, GATED ? BN / 2 : BN, ROUTED>(a, &grid);
+  const GemmParams p = gemm_params<BM, GATED ? BN / 2 : BN, ROUTED>(a, &grid, c);
   kernel<<<grid, 512, bytes, stream>>>(p);
   return hipGetLastError();
 }
 
 template <int BM, int BN, int WM, int WAVES, int STAGES, int GATED, bool ROUTED>
-hipError_t run_direct(const DenseLinearArgs &a, hipStream_t stream) {
+hipError_t run_direct(const DenseLinearArgs &a, Columns c, hipStream_t stream) {
   constexpr int bytes = STAGES * (BM + BN) * 128;
   static bool allowed[kMaxDevices] = {};
   const auto kernel = dense_gemm_direct_kernel<BM, BN, WM, WAVES, STAGES, GATED, ROUTED>;
   if (bytes > 64 * 1024)
     if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
   dim3 grid;
-  const GemmParams p = gemm_params<BM, GATED ? BN / 2 : BN, ROUTED>(a, &grid);
+  const GemmParams p = gemm_params<BM, GATED ? BN / 2 : BN, ROUTED>(a, &grid, c);
   kernel<<<grid, WAVES * 64, bytes, stream>>>(p);
   return hipGetLastError();
 }
 
 template <int GATED>
-hipError_t run_phased(const DenseLinearArgs &a, hipStream_t stream) {
+hipError_t run_phased(const DenseLinearArgs &a, Columns c, hipStream_t stream) {
   constexpr int bytes = 2 * 4 * 16384;
   static bool allowed[kMaxDevices] = {};
   const auto kernel = dense_gemm_phased_kernel<GATED>;
   if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
   dim3 grid;
-  const GemmParams p = gemm_params<256, GATED ? 128 : 256, false>(a, &grid);
+  const GemmParams p = gemm_params<256, GATED ? 128 : 256, false>(a, &grid, c);
   kernel<<<grid, 512, bytes, stream>>>(p);
   return hipGetLastError();
 }
@@ -842,33 +848,44 @@ hipError_t run_registers(const DenseLinearArgs &a, hipStream_t stream) {
 template <int GATED>
 hipError_t pick_routed(const DenseLinearArgs &a, hipStream_t stream) {
   const bool direct = !a.f32 && a.k % kStageK == 0 && a.ldx % 8 == 0;
-  if (a.tile == 128) return direct ? run_turns<128, 128, 5, GATED, true>(a, stream) : hipErrorInvalidValue;
-  if (direct) return run_direct<64, 128, 2, 4, 3, GATED, true>(a, stream);
+  if (a.tile == 128) return direct ? run_turns<128, 128, 5, GATED, true>(a, {0, a.n}, stream) : hipErrorInvalidValue;
+  if (direct) return run_direct<64, 128, 2, 4, 3, GATED, true>(a, {0, a.n}, stream);
   return a.f32 ? run_registers<float, 64, GATED, true>(a, stream) : run_registers<__bf16, 64, GATED, true>(a, stream);
+}
+
+template <int GATED>
+hipError_t run_tile(DenseTile tile, const DenseLinearArgs &a, Columns c, hipStream_t stream) {
+  switch (tile) {
+    case DenseTile::k256x256: return run_phased<GATED>(a, c, stream);
+    case DenseTile::k128x128: return run_direct<128, 128, 2, 4, 2, GATED, false>(a, c, stream);
+    case DenseTile::k192x128: return run_direct<192, 128, 2, 4, 2, GATED, false>(a, c, stream);
+    case DenseTile::k128x192: return run_direct<128, 192, 2, 4, 2, GATED, false>(a, c, stream);
+    case DenseTile::k192x128Eight: return run_direct<192, 128, 2, 8, 3, GATED, false>(a, c, stream);
+    case DenseTile::k128x128Eight: return run_direct<128, 128, 4, 8, 3, GATED, false>(a, c, stream);
+    case DenseTile::k64x128Eight: return run_direct<64, 128, 2, 8, 4, GATED, false>(a, c, stream);
+    case DenseTile::k64x64: return run_direct<64, 64, 2, 4, 4, GATED, false>(a, c, stream);
+    case DenseTile::k32x64: return run_direct<32, 64, 2, 4, 6, GATED, false>(a, c, stream);
+    case DenseTile::k64x128: return run_direct<64, 128, 2, 4, 3, GATED, false>(a, c, stream);
+    case DenseTile::kTurns192x128: return run_turns<192, 128, 3, GATED, false>(a, c, stream);
+    case DenseTile::kTurns128x128: return run_turns<128, 128, 5, GATED, false>(a, c, stream);
+    case DenseTile::kTurns128x192: return run_turns<128, 192, 3, GATED, false>(a, c, stream);
+    case DenseTile::kTurns256x128: return run_turns<256, 128, 3, GATED, false>(a, c, stream);
+    case DenseTile::kTurns128x64: return run_turns<128, 64, 5, GATED, false>(a, c, stream);
+  }
+  return hipErrorInvalidValue;
 }
 
 template <int GATED>
 hipError_t pick_gemm(const DenseLinearArgs &a, hipStream_t stream) {
   if (a.f32) return run_registers<float, 32, GATED, false>(a, stream);
   if (a.k % kStageK != 0 || a.ldx % 8 != 0) return run_registers<__bf16, 32, GATED, false>(a, stream);
-  switch (dense_product_tile(a.m, (uint64_t)a.n * (GATED ? 2 : 1), a.k, (uint32_t)device_compute_units())) {
-    case DenseTile::k256x256: return run_phased<GATED>(a, stream);
-    case DenseTile::k128x128: return run_direct<128, 128, 2, 4, 2, GATED, false>(a, stream);
-    case DenseTile::k192x128: return run_direct<192, 128, 2, 4, 2, GATED, false>(a, stream);
-    case DenseTile::k128x192: return run_direct<128, 192, 2, 4, 2, GATED, false>(a, stream);
-    case DenseTile::k192x128Eight: return run_direct<192, 128, 2, 8, 3, GATED, false>(a, stream);
-    case DenseTile::k128x128Eight: return run_direct<128, 128, 4, 8, 3, GATED, false>(a, stream);
-    case DenseTile::k64x128Eight: return run_direct<64, 128, 2, 8, 4, GATED, false>(a, stream);
-    case DenseTile::k64x64: return run_direct<64, 64, 2, 4, 4, GATED, false>(a, stream);
-    case DenseTile::k32x64: return run_direct<32, 64, 2, 4, 6, GATED, false>(a, stream);
-    case DenseTile::k64x128: return run_direct<64, 128, 2, 4, 3, GATED, false>(a, stream);
-    case DenseTile::kTurns192x128: return run_turns<192, 128, 3, GATED, false>(a, stream);
-    case DenseTile::kTurns128x128: return run_turns<128, 128, 5, GATED, false>(a, stream);
-    case DenseTile::kTurns128x192: return run_turns<128, 192, 3, GATED, false>(a, stream);
-    case DenseTile::kTurns256x128: return run_turns<256, 128, 3, GATED, false>(a, stream);
-    case DenseTile::kTurns128x64: return run_turns<128, 64, 5, GATED, false>(a, stream);
-  }
-  return hipErrorInvalidValue;
+  constexpr uint32_t MATRICES = GATED ? 2 : 1;
+  const uint32_t cus = (uint32_t)device_compute_units();
+  const DenseSplit split = dense_column_split(a.m, (uint64_t)a.n * MATRICES, a.k, cus);
+  const uint32_t first = (uint32_t)(split.columns / MATRICES);
+  if (first > 0)
+    if (hipError_t status = run_tile<GATED>(split.tile, a, {0, first}, stream)) return status;
+  return run_tile<GATED>(dense_product_tile(a.m, (uint64_t)(a.n - first) * MATRICES, a.k, cus), a, {first, a.n}, stream);
 }
 
 // ---- row-wise kernels ------------------------------------------------------------------------------

@@ -80,24 +80,60 @@ constexpr StaggeredTime kStaggeredTimes[] = {
     {DenseTile::kTurns128x64, 128, 64, 1.88f, 2.42f, 5.50f, 0.76f},    // 2 x 4 waves, 5 stages
 };
 
-// The tile a product runs on: one of the ten, or from K = 1024 on (below, what the meeting of two groups' sums costs is not
-// made up for) one of these where its estimate is 7% less.  The two estimates are fits to launches of their own, and 7% keeps
-// the cases that lose by that few: of the 649 sizes beyond 12 us the choice is 4.6% faster than the ten on average and more
-// than 3% slower at 17 (us, ten / this: 2048 x 2048 x 8192 74 / 63, 3001 x 2048 x 8192 100 / 83, 2048 x 6144 x 2048
-// 50.7 / 46.8, 700 x 2048 x 2048 15.6 / 14.0; the other way 994 x 2816 x 1152 14.0 / 15.1, 1008 x 1088 x 4288 25.9 / 27.8).
-inline DenseTile dense_product_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus) {
+inline float staggered_time(const StaggeredTime &t, uint64_t tiles, uint32_t k, uint32_t cus) {
+  const uint64_t rest = tiles % cus;
+  const float one = t.one + t.one_k * (float)k / 1024.0f;
+  return t.start + (float)(tiles / cus) * one + (rest > 0 ? one * (t.few + (1.0f - t.few) * (float)rest / (float)cus) : 0.0f);
+}
+
+// The tile a product runs on: one of the ten, or from K = 1024 on, in turns from 1280 (below, what the meeting of two groups'
+// sums costs is not made up for: 128 x 128 tiles 0.99 of the ten's time on average, up to 1.16), one of these where its
+// estimate is 7% less.  The two estimates are fits to launches of their own, and 7% keeps the cases that lose by that few: of
+// 649 sizes beyond 12 us the choice is 4.6% faster than the ten on average and more than 3% slower at 12 (us, ten / this:
+// 2048 x 2048 x 8192 74 / 63, 3001 x 2048 x 8192 100 / 83, 2048 x 6144 x 2048 50.7 / 46.8, 700 x 2048 x 2048 15.6 / 14.0; the
+// other way 2048 x 2048 x 2048 21.9 / 23.0, 1008 x 1088 x 4288 25.9 / 27.8).
+inline DenseTile dense_product_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus, float *estimate = nullptr) {
   float least = 0.0f;
   DenseTile best = dense_tile(m, columns, k, cus, &least);
-  if (k < 1024) return best;
-  least *= 0.93f;
-  for (const StaggeredTime &t : kStaggeredTimes) {
-    const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns), rest = tiles % cus;
-    const float one = t.one + t.one_k * (float)k / 1024.0f;
-    float time = t.start + (float)(tiles / cus) * one;
-    if (rest > 0) time += one * (t.few + (1.0f - t.few) * (float)rest / (float)cus);
-    if (time < least) least = time, best = t.tile;
+  if (k >= 1024) {
+    least *= 0.93f;
+    for (const StaggeredTime &t : kStaggeredTimes) {
+      if (k < 1280 && t.tile != DenseTile::k256x256) continue;
+      const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns);
+      const float time = staggered_time(t, tiles, k, cus);
+      if (time < least) least = time, best = t.tile;
+    }
   }
+  if (estimate != nullptr) *estimate = least;
   return best;
+}
+
+// A product in two launches: the first `columns` on whole rounds of a large tile, the rest on the tile that suits it (0: one
+// launch).  A round of the 256 CUs that is a tenth filled costs most of a whole one, and smaller tiles for all of the columns
+// are the slower ones.  Taken where the two estimates together are 5% less; us, one launch / two: 2048 x 8512 x 2048 94.9 /
+// 76.3, 3001 x 7312 x 2048 102.9 / 91.3, 2701 x 12096 x 3520 232 / 194, 1451 x 13760 x 3776 157 / 138, 0.99 to 1.01 of one at
+// four of sixteen sizes drawn and less at the others.
+struct DenseSplit {
+  DenseTile tile;
+  uint64_t columns;
+};
+inline DenseSplit dense_column_split(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus) {
+  DenseSplit split = {DenseTile::k256x256, 0};
+  if (k < 1024) return split;
+  float least = 0.0f;
+  dense_product_tile(m, columns, k, cus, &least);
+  least *= 0.95f;
+  for (const StaggeredTime &t : kStaggeredTimes) {
+    if (k < 1280 && t.tile != DenseTile::k256x256) continue;
+    const uint64_t tiles_m = (m + t.rows - 1) / t.rows, tiles = tiles_m * ((columns + t.columns - 1) / t.columns);
+    const uint64_t whole = tiles / cus * cus / tiles_m;  // tile columns of whole rounds
+    if (whole == 0 || tiles % cus == 0 || whole * t.columns >= columns) continue;
+    float rest = 0.0f;
+    dense_product_tile(m, columns - whole * t.columns, k, cus, &rest);
+    const float time = staggered_time(t, whole * tiles_m, k, cus) + rest;
+    if (time < least) least = time, split = {t.tile, whole * t.columns};
+  }
+  return split;
 }
 
 }  // namespace llmopt

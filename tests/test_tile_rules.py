@@ -28,6 +28,7 @@ int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
 }
 int product_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_tile(m, n, k, cus); }
 int staggered_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_product_tile(m, n, k, cus); }
+int split_columns(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_column_split(m, n, k, cus).columns; }
 int qkv_tile(uint32_t m, uint32_t q, uint32_t kv, uint32_t k, uint32_t cus) {
   const uint32_t n[3] = {q, kv, kv};
   return (int)qkv_rows_tile(m, n, k, cus);
@@ -155,9 +156,16 @@ def test_gpu_tests_reach_every_staggered_tile(rules):
     every = {DENSE.index("256x256")} | set(range(len(DENSE), len(DENSE) + 5))
     assert {rules.staggered_tile(*size, CUS) for size in test_gpu_dense_tiles.STAGGERED} == every
     assert {rules.staggered_tile(m, n // 2 * 2, k, CUS) for m, n, k in test_gpu_dense_tiles.STAGGERED} == every
+    assert all(0 < rules.split_columns(m, n // 2 * 2, k, CUS) < n for m, n, k in test_gpu_dense_tiles.SPLIT)
 
 
 @pytest.mark.parametrize("m,n,k", [(2048, 2048, 1000), (64, 4096, 1024), (3001, 2048, 128), (2048, 2048, 512), (330, 700, 2048)])
 def test_products_that_stay_in_step(rules, m, n, k):
     """A short K, and launches that no staggered tile fills."""
     assert rules.staggered_tile(m, n, k, CUS) == rules.product_tile(m, n, k, CUS)
+
+
+@pytest.mark.parametrize("m,n,k,first", [(2048, 8512, 2048, 8192), (3001, 7312, 2048, 5376), (2048, 9504, 2048, 8192),
+                                         (2048, 16384, 2048, 0), (3001, 16384, 2048, 0), (2048, 2048, 8192, 0), (2048, 8512, 960, 0)])
+def test_columns_in_two_launches(rules, m, n, k, first):
+    assert rules.split_columns(m, n, k, CUS) == first
