@@ -60,6 +60,9 @@ hipError_t launch_w4a16_rows_qkv(const W4QkvArgs &args, hipStream_t stream);
 bool w4a16_rows_pack_ok(const W4QkvArgs &args, const RotaryPackArgs &rotary);
 hipError_t launch_w4a16_rows_qkv_pack(const W4QkvArgs &args, const RotaryPackArgs &rotary, hipStream_t stream);
 hipError_t launch_w4a16_rows_dual_swiglu(const W4DualSwigluArgs &args, hipStream_t stream);
+// True when these launches can normalise the rows of x themselves (args.norm is then `norm` for them).
+bool w4a16_rows_norm_ok(const W4QkvArgs &args, const W4Norm &norm, const RotaryPackArgs &rotary);
+bool w4a16_rows_norm_ok(const W4DualSwigluArgs &args, const W4Norm &norm);
 // y [rows / 2, n]: the float32 sums of the products of rows 2r and 2r + 1 (see launch_rms_norm_split).
 bool w4a16_rows_pairs_ok(const uint16_t *x, const W4Matrix &w, uint32_t rows, uint32_t n, uint32_t k);
 hipError_t launch_w4a16_rows_pairs(const uint16_t *x, const W4Matrix &w, float *y, uint32_t rows, uint32_t n, uint32_t k,

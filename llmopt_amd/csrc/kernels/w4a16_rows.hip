@@ -80,133 +80,21 @@ __device__ __forceinline__ h8_t w4_exact_natural(uint32_t word) {
   return __builtin_bit_cast(h8_t, packed);
 }
 
-template <int ROWS, int CT, int P, int STAGES, bool DUAL, class Params>
-__global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
+// What a workgroup's lanes need of their place in the launch.
+struct TileLane {
+  uint32_t segment, n, m0, n0;  // the matrix, its columns, the tile's first row and column
+  int part, column, half;       // of the wave's K groups; of the tile; which half of a block's rows
+};
+
+// The end of a tile: the waves' sums meet in LDS, [part][row][column], added in the order of the parts, and go out.
+template <int ROWS, int CT, int P, bool DUAL, class Params>
+__device__ __forceinline__ void finish_rows(const Params &p, const f16x_t (&acc)[ROWS / 32], const TileLane &at_tile, float *sums) {
   constexpr bool PACK = std::is_same_v<Params, PackParams>;
-  static_assert(!PACK || (!DUAL && CT % 2 == 0), "whole heads in a tile");
-  constexpr int WAVES = CT * P, COLUMNS = CT * 32, STEP = P * 64;
-  static_assert(ROWS % 32 == 0, "whole blocks of rows");
-  constexpr int RT = ROWS / 32;                             // 32-row blocks of a wave
-  constexpr int X_PIECES = STEP / 8, W_PIECES = STEP / 32;  // 16-byte pieces of a row and step
-  constexpr int X_BYTES = ROWS * X_PIECES * 16, W_BYTES = COLUMNS * W_PIECES * 16, STAGE_BYTES = X_BYTES + W_BYTES;
-  constexpr int X_COPIES = X_BYTES / 1024 / WAVES, COPIES = X_COPIES + 1;  // of a wave and step
-  static_assert(X_BYTES == X_COPIES * WAVES * 1024 && W_BYTES == WAVES * 1024, "a step divides over the waves");
-  static_assert(!DUAL || CT % 2 == 0, "gate and up columns of an output lie in one tile");
-  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ct = wave / P, part = wave % P;
-  const uint32_t groups = p.k / 64, steps = (groups + P - 1) / P;
-
-  uint32_t segment = 0, tile = blockIdx.x;
-  if (!DUAL)
-    while (segment + 1 < p.segments && tile >= p.tiles[segment]) tile -= p.tiles[segment++];
-  const uint32_t n = p.n[segment], m0 = blockIdx.y * ROWS;
-  const uint32_t n0 = tile * (DUAL ? COLUMNS / 2 : COLUMNS);
-  // Of a tile column: its row in the matrix, from the tile's first one (columns past n are never stored).  The 32-column
-  // blocks of a pair's tile alternate between gate and up.
-  auto weight_row = [&](uint32_t column) __attribute__((always_inline)) {
-    return min(DUAL ? (column >> 6) * 32 + (column & 31) : column, n - 1 - n0);
-  };
-  auto matrix_of = [&](uint32_t column) __attribute__((always_inline)) { return DUAL ? (column >> 5) & 1 : segment; };
-
-  const uint32_t scale_bytes = scale_lds_bytes(COLUMNS, groups);
-  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)rows_lds;
-  const uint32_t ring = lds_base + scale_bytes;
-  const uint32_t group_blocks = (groups + 7) / 8;
-  for (uint32_t block = wave; block < COLUMNS / 8 * group_blocks; block += WAVES) {
-    const uint32_t column = block / group_blocks * 8;
-    const uint16_t *scales = p.s[matrix_of(column)] + (size_t)n0 * groups;
-    const uint32_t row = weight_row(column + (lane & 7)), group = min(block % group_blocks * 8 + (lane >> 3), groups - 1);
-    copy2_to_lds(scales, (row * groups + group) * 2, lds_base + block * 256);
-  }
-
-  // Copies of a step: lane l fills consecutive 16-byte places; the piece it fetches is the one that the swizzle puts there.
-  const uint8_t *x_base = reinterpret_cast<const uint8_t *>(p.x + (size_t)m0 * p.k);
-  uint32_t x_row[X_COPIES], x_at[X_COPIES];  // bytes
-#pragma unroll
-  for (int c = 0; c < X_COPIES; ++c) {
-    const uint32_t place = (wave * X_COPIES + c) * 64 + lane, row = place / X_PIECES;
-    x_row[c] = min(row, p.m - 1 - m0) * p.k * 2;
-    x_at[c] = (place % X_PIECES ^ (row & 15)) * 16;
-  }
-  auto w_twist = [](uint32_t row) __attribute__((always_inline)) {
-    return W_PIECES >= 16 ? row & 15 : W_PIECES == 8 ? (row >> 1) & 7 : (row >> 2) & 3;
-  };
-  const uint32_t w_place = wave * 64 + lane, w_column = w_place / W_PIECES;
-  const uint8_t *w_base = p.w[matrix_of(wave * 64 / W_PIECES)] + (size_t)n0 * (p.k / 2);
-  const uint32_t w_row = weight_row(w_column) * (p.k / 2), w_at = (w_place % W_PIECES ^ w_twist(w_column)) * 16;
-  auto request = [&](uint32_t step) __attribute__((always_inline)) {
-    const uint32_t stage = ring + step % STAGES * STAGE_BYTES, k0 = step * STEP;
-    const uint8_t *x = x_base + (size_t)k0 * 2, *w = w_base + k0 / 2;
-    if (k0 + STEP <= p.k) {
-      copy16_to_lds(w, w_row + w_at, stage + X_BYTES + wave * 1024);
-#pragma unroll
-      for (int c = 0; c < X_COPIES; ++c) copy16_to_lds(x, x_row[c] + x_at[c], stage + (wave * X_COPIES + c) * 1024);
-    } else {  // the end of the rows: their last pieces again, which nothing multiplies
-      copy16_to_lds(w, w_row + min(w_at, (p.k - k0) / 2 - 16), stage + X_BYTES + wave * 1024);
-#pragma unroll
-      for (int c = 0; c < X_COPIES; ++c)
-        copy16_to_lds(x, x_row[c] + min(x_at[c], (p.k - k0) * 2 - 16), stage + (wave * X_COPIES + c) * 1024);
-    }
-  };
-
-  f16x_t acc[RT];
-#pragma unroll
-  for (int r = 0; r < RT; ++r)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[r][i] = 0.0f;
-
-  const int column = ct * 32 + (lane & 31), half = lane >> 5;
-  const uint32_t x_read_row = lane & 31;
-  const uint32_t w_read = X_BYTES + (column * W_PIECES + ((part * 2 + half) ^ w_twist(column))) * 16;
-  uint32_t x_read[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) x_read[j] = (x_read_row * X_PIECES + ((part * 8 + half * 4 + j) ^ (x_read_row & 15))) * 16;
-  const uint32_t *scale_read = reinterpret_cast<const uint32_t *>(rows_lds) + (column >> 3) * group_blocks * 64 + (column & 7);
-#pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
-    if (s < (int)steps) request(s);
-  for (uint32_t s = 0; s < steps; ++s) {
-    // this step has landed once only the copies of the STAGES - 2 steps behind it are under way
-    if (s + STAGES - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"((STAGES - 2) * COPIES) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (s + STAGES - 1 < steps) request(s + STAGES - 1);  // into the place of the step before, which every wave has read
-    const uint32_t group = s * P + part;
-    if (group >= groups) continue;  // (the same for the whole wave, and its last step)
-    const unsigned char *stage = rows_lds + scale_bytes + s % STAGES * STAGE_BYTES;
-    const u32x4_t packed = *reinterpret_cast<const u32x4_t *>(stage + w_read);
-    h8_t x[RT][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < RT; ++r)
-        x[r][j] = *reinterpret_cast<const h8_t *>(stage + x_read[j] + r * 32 * X_PIECES * 16);
-    const float scale = half_bits_to_float((uint16_t)scale_read[(group >> 3) * 64 + (group & 7) * 8]);
-    f16x_t sum[RT];
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sum[r][i] = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const h8_t w = w4_exact_natural(packed[j]);
-#pragma unroll
-      for (int r = 0; r < RT; ++r) sum[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[r][j], w, sum[r], 0, 0, 0);
-    }
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[r][i] = fmaf(scale, sum[r][i], acc[r][i]);
-  }
-
-  // The waves' sums meet in LDS: [part][row][column], added in the order of the parts.
+  constexpr int WAVES = CT * P, COLUMNS = CT * 32, RT = ROWS / 32;
+  const int tid = threadIdx.x, part = at_tile.part, column = at_tile.column, half = at_tile.half;
+  const uint32_t segment = at_tile.segment, n = at_tile.n, m0 = at_tile.m0, n0 = at_tile.n0;
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __syncthreads();
-  float *sums = reinterpret_cast<float *>(rows_lds + scale_bytes);
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -323,6 +211,298 @@ __global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
   }
 }
 
+
+template <int ROWS, int CT, int P, int STAGES, bool DUAL, class Params>
+__global__ __launch_bounds__(CT *P * 64) void w4a16_rows_kernel(Params p) {
+  constexpr bool PACK = std::is_same_v<Params, PackParams>;
+  static_assert(!PACK || (!DUAL && CT % 2 == 0), "whole heads in a tile");
+  constexpr int WAVES = CT * P, COLUMNS = CT * 32, STEP = P * 64;
+  static_assert(ROWS % 32 == 0, "whole blocks of rows");
+  constexpr int RT = ROWS / 32;                             // 32-row blocks of a wave
+  constexpr int X_PIECES = STEP / 8, W_PIECES = STEP / 32;  // 16-byte pieces of a row and step
+  constexpr int X_BYTES = ROWS * X_PIECES * 16, W_BYTES = COLUMNS * W_PIECES * 16, STAGE_BYTES = X_BYTES + W_BYTES;
+  constexpr int X_COPIES = X_BYTES / 1024 / WAVES, COPIES = X_COPIES + 1;  // of a wave and step
+  static_assert(X_BYTES == X_COPIES * WAVES * 1024 && W_BYTES == WAVES * 1024, "a step divides over the waves");
+  static_assert(!DUAL || CT % 2 == 0, "gate and up columns of an output lie in one tile");
+  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ct = wave / P, part = wave % P;
+  const uint32_t groups = p.k / 64, steps = (groups + P - 1) / P;
+
+  uint32_t segment = 0, tile = blockIdx.x;
+  if (!DUAL)
+    while (segment + 1 < p.segments && tile >= p.tiles[segment]) tile -= p.tiles[segment++];
+  const uint32_t n = p.n[segment], m0 = blockIdx.y * ROWS;
+  const uint32_t n0 = tile * (DUAL ? COLUMNS / 2 : COLUMNS);
+  // Of a tile column: its row in the matrix, from the tile's first one (columns past n are never stored).  The 32-column
+  // blocks of a pair's tile alternate between gate and up.
+  auto weight_row = [&](uint32_t column) __attribute__((always_inline)) {
+    return min(DUAL ? (column >> 6) * 32 + (column & 31) : column, n - 1 - n0);
+  };
+  auto matrix_of = [&](uint32_t column) __attribute__((always_inline)) { return DUAL ? (column >> 5) & 1 : segment; };
+
+  const uint32_t scale_bytes = scale_lds_bytes(COLUMNS, groups);
+  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)rows_lds;
+  const uint32_t ring = lds_base + scale_bytes;
+  const uint32_t group_blocks = (groups + 7) / 8;
+  for (uint32_t block = wave; block < COLUMNS / 8 * group_blocks; block += WAVES) {
+    const uint32_t column = block / group_blocks * 8;
+    const uint16_t *scales = p.s[matrix_of(column)] + (size_t)n0 * groups;
+    const uint32_t row = weight_row(column + (lane & 7)), group = min(block % group_blocks * 8 + (lane >> 3), groups - 1);
+    copy2_to_lds(scales, (row * groups + group) * 2, lds_base + block * 256);
+  }
+
+  // Copies of a step: lane l fills consecutive 16-byte places; the piece it fetches is the one that the swizzle puts there.
+  const uint8_t *x_base = reinterpret_cast<const uint8_t *>(p.x + (size_t)m0 * p.k);
+  uint32_t x_row[X_COPIES], x_at[X_COPIES];  // bytes
+#pragma unroll
+  for (int c = 0; c < X_COPIES; ++c) {
+    const uint32_t place = (wave * X_COPIES + c) * 64 + lane, row = place / X_PIECES;
+    x_row[c] = min(row, p.m - 1 - m0) * p.k * 2;
+    x_at[c] = (place % X_PIECES ^ (row & 15)) * 16;
+  }
+  auto w_twist = [](uint32_t row) __attribute__((always_inline)) {
+    return W_PIECES >= 16 ? row & 15 : W_PIECES == 8 ? (row >> 1) & 7 : (row >> 2) & 3;
+  };
+  const uint32_t w_place = wave * 64 + lane, w_column = w_place / W_PIECES;
+  const uint8_t *w_base = p.w[matrix_of(wave * 64 / W_PIECES)] + (size_t)n0 * (p.k / 2);
+  const uint32_t w_row = weight_row(w_column) * (p.k / 2), w_at = (w_place % W_PIECES ^ w_twist(w_column)) * 16;
+  auto request = [&](uint32_t step) __attribute__((always_inline)) {
+    const uint32_t stage = ring + step % STAGES * STAGE_BYTES, k0 = step * STEP;
+    const uint8_t *x = x_base + (size_t)k0 * 2, *w = w_base + k0 / 2;
+    if (k0 + STEP <= p.k) {
+      copy16_to_lds(w, w_row + w_at, stage + X_BYTES + wave * 1024);
+#pragma unroll
+      for (int c = 0; c < X_COPIES; ++c) copy16_to_lds(x, x_row[c] + x_at[c], stage + (wave * X_COPIES + c) * 1024);
+    } else {  // the end of the rows: their last pieces again, which nothing multiplies
+      copy16_to_lds(w, w_row + min(w_at, (p.k - k0) / 2 - 16), stage + X_BYTES + wave * 1024);
+#pragma unroll
+      for (int c = 0; c < X_COPIES; ++c)
+        copy16_to_lds(x, x_row[c] + min(x_at[c], (p.k - k0) * 2 - 16), stage + (wave * X_COPIES + c) * 1024);
+    }
+  };
+
+  f16x_t acc[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[r][i] = 0.0f;
+
+  const int column = ct * 32 + (lane & 31), half = lane >> 5;
+  const uint32_t x_read_row = lane & 31;
+  const uint32_t w_read = X_BYTES + (column * W_PIECES + ((part * 2 + half) ^ w_twist(column))) * 16;
+  uint32_t x_read[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x_read[j] = (x_read_row * X_PIECES + ((part * 8 + half * 4 + j) ^ (x_read_row & 15))) * 16;
+  const uint32_t *scale_read = reinterpret_cast<const uint32_t *>(rows_lds) + (column >> 3) * group_blocks * 64 + (column & 7);
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < (int)steps) request(s);
+  for (uint32_t s = 0; s < steps; ++s) {
+    // this step has landed once only the copies of the STAGES - 2 steps behind it are under way
+    if (s + STAGES - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"((STAGES - 2) * COPIES) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (s + STAGES - 1 < steps) request(s + STAGES - 1);  // into the place of the step before, which every wave has read
+    const uint32_t group = s * P + part;
+    if (group >= groups) continue;  // (the same for the whole wave, and its last step)
+    const unsigned char *stage = rows_lds + scale_bytes + s % STAGES * STAGE_BYTES;
+    const u32x4_t packed = *reinterpret_cast<const u32x4_t *>(stage + w_read);
+    h8_t x[RT][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+        x[r][j] = *reinterpret_cast<const h8_t *>(stage + x_read[j] + r * 32 * X_PIECES * 16);
+    const float scale = half_bits_to_float((uint16_t)scale_read[(group >> 3) * 64 + (group & 7) * 8]);
+    f16x_t sum[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum[r][i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const h8_t w = w4_exact_natural(packed[j]);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) sum[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[r][j], w, sum[r], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[r][i] = fmaf(scale, sum[r][i], acc[r][i]);
+  }
+
+  finish_rows<ROWS, CT, P, DUAL>(p, acc, {segment, n, m0, n0, part, column, half}, reinterpret_cast<float *>(rows_lds + scale_bytes));
+}
+
+// The value of another lane of the same sixteen.
+template <int CONTROL>
+__device__ __forceinline__ float lane_of(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CONTROL, 0xf, 0xf, true));
+}
+
+// half(x * gain * inverse) (FIRST) or half(x * inverse * gain) of two values, every product rounded to float32 and the last one
+// then to half.  Halves are read where they lie: without their conversions it is 3.5 instructions a value for 5.5.  (A zero may
+// lose its sign, which no sum shows.)
+template <bool FIRST>
+__device__ __forceinline__ uint32_t normed_pair(uint32_t x, uint32_t gain, float inverse) {
+  float low, high;
+  if (FIRST) {
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,1,0]" : "=v"(low) : "v"(x), "v"(gain));
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(high) : "v"(x), "v"(gain));
+    asm("v_mul_f32 %0, %1, %2" : "=v"(low) : "v"(low), "v"(inverse));  // (a product that the compiler sees it rounds to half at once)
+    asm("v_mul_f32 %0, %1, %2" : "=v"(high) : "v"(high), "v"(inverse));
+  } else {
+    float turned[2];
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(turned[0]) : "v"(x), "v"(inverse));
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(turned[1]) : "v"(x), "v"(inverse));
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(low) : "v"(turned[0]), "v"(gain));
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(high) : "v"(turned[1]), "v"(gain));
+  }
+  return (uint32_t)float_to_half_bits(low) | (uint32_t)float_to_half_bits(high) << 16;
+}
+
+// The same tiles over rows that the kernel normalises itself, for a K whose rows and weights fit LDS as a whole: everything is
+// requested at once, waves normalise the rows where they lie, eight lanes a row, and the products follow without a barrier
+// between them.  The launch of the norm ahead, 3.4 us of starting and a trip to memory and back, and its boundary go.  With 32
+// rows of 576 values that is the better one (QKV with rotation and pack, 700 rows: 8.0 + 3.4 us and the boundary / 11.2; prompts of
+// 64 to 900 tokens of a 30-layer transformer 1.5 to 3.5% less), with 96 rows the copies that no product covers cost as much
+// (a pair of 700 x 576 x 1536: 10.8 + 3.4 / 15.6).
+//
+//  * Rows lie as blocks of eight rows by one scale group, 1 KB that a copy fills from whole lines, pieces XOR-ed by half the row;
+//    weights as blocks of sixteen columns by two groups, pieces XOR-ed by a quarter of the column.  Operand reads of sixteen
+//    lanes touch every bank once.
+//  * The arithmetic is that of rms_norm_f16_rows_kernel and w4a16_rows_kernel in their order: the same values.
+template <int ROWS, int CT, int P, bool DUAL, class Params>
+__global__ __launch_bounds__(CT *P * 64) void w4a16_normed_rows_kernel(Params p, W4Norm norm) {
+  static_assert(!std::is_same_v<Params, PackParams> || (!DUAL && CT % 2 == 0), "whole heads in a tile");
+  static_assert(ROWS % 32 == 0 && (!DUAL || CT % 2 == 0), "whole blocks; gate and up columns of an output in one tile");
+  constexpr int WAVES = CT * P, COLUMNS = CT * 32, RT = ROWS / 32;
+  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ct = wave / P, part = wave % P;
+  const uint32_t groups = p.k / 64, pairs = (groups + 1) / 2;
+
+  uint32_t segment = 0, tile = blockIdx.x;
+  if (!DUAL)
+    while (segment + 1 < p.segments && tile >= p.tiles[segment]) tile -= p.tiles[segment++];
+  const uint32_t n = p.n[segment], m0 = blockIdx.y * ROWS, n0 = tile * (DUAL ? COLUMNS / 2 : COLUMNS);
+  auto weight_row = [&](uint32_t column) __attribute__((always_inline)) {
+    return min(DUAL ? (column >> 6) * 32 + (column & 31) : column, n - 1 - n0);
+  };
+  auto matrix_of = [&](uint32_t column) __attribute__((always_inline)) { return DUAL ? (column >> 5) & 1 : segment; };
+
+  const uint32_t scale_bytes = scale_lds_bytes(COLUMNS, groups), x_bytes = ROWS * groups * 128;
+  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)rows_lds;
+  // rows: lane l fetches the piece that the swizzle puts at place l % 8 of row l / 8
+  for (uint32_t copy = wave; copy < ROWS / 8 * groups; copy += WAVES) {
+    const uint32_t block = copy % (ROWS / 8), group = copy / (ROWS / 8), row = block * 8 + (lane >> 3);
+    const uint16_t *x = p.x + (size_t)m0 * p.k + group * 64;
+    copy16_to_lds(x, min(row, p.m - 1 - m0) * p.k * 2 + (((lane & 7) ^ ((row >> 1) & 7)) * 16),
+                  lds_base + scale_bytes + (block * groups + group) * 1024);
+  }
+  // weights: a block's columns lie in one matrix; the second half of the last pair of an odd K is the first one again
+  for (uint32_t copy = wave; copy < COLUMNS / 16 * pairs; copy += WAVES) {
+    const uint32_t block = copy % (COLUMNS / 16), pair = copy / (COLUMNS / 16), first = block * 16, column = first + (lane >> 2);
+    const uint8_t *w = p.w[matrix_of(first)] + (size_t)n0 * (p.k / 2);
+    const uint32_t piece = (lane & 3) ^ ((column >> 2) & 3), group = min(pair * 2 + piece / 2, groups - 1);
+    copy16_to_lds(w, weight_row(column) * (p.k / 2) + group * 32 + piece % 2 * 16, lds_base + scale_bytes + x_bytes + (block * pairs + pair) * 1024);
+  }
+  const uint32_t group_blocks = (groups + 7) / 8;
+  for (uint32_t copy = wave; copy < COLUMNS / 8 * group_blocks; copy += WAVES) {
+    const uint32_t block = copy % (COLUMNS / 8), eight = copy / (COLUMNS / 8), column = block * 8;
+    const uint16_t *scales = p.s[matrix_of(column)] + (size_t)n0 * groups;
+    const uint32_t row = weight_row(column + (lane & 7)), group = min(eight * 8 + (lane >> 3), groups - 1);
+    copy2_to_lds(scales, (row * groups + group) * 2, lds_base + (block * group_blocks + eight) * 256);
+  }
+  const uint32_t gain_offset = x_bytes + COLUMNS / 16 * pairs * 1024;
+  for (uint32_t block = wave; block * 8 < groups; block += WAVES)
+    copy16_to_lds(norm.weight, min(block * 64 + lane, groups * 8 - 1) * 16, lds_base + scale_bytes + gain_offset + block * 1024);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  unsigned char *rows = rows_lds + scale_bytes;
+  for (uint32_t block = wave; block < ROWS / 8; block += WAVES) {
+    const uint32_t row = block * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+    unsigned char *place = rows + block * groups * 1024 + lane * 16;
+    const unsigned char *gains = rows + gain_offset + piece * 16;
+    u32x4_t x[kNormedGroups];
+#pragma unroll
+    for (uint32_t group = 0; group < kNormedGroups; ++group)
+      x[group] = group < groups ? *reinterpret_cast<const u32x4_t *>(place + group * 1024) : u32x4_t{0, 0, 0, 0};
+    // in the order of rms_norm_f16_rows_kernel, whose lane l has pieces l, l + 64, ..: here the lane's pieces of groups b, b + 8
+    float eight[8];
+#pragma unroll
+    for (uint32_t b = 0; b < 8; ++b) {
+      float sum = 0.0f;
+#pragma unroll
+      for (uint32_t group = b; group < kNormedGroups; group += 8)
+        if (group < groups) {
+          const h8_t v = __builtin_bit_cast(h8_t, x[group]);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) sum += (float)v[e] * (float)v[e];
+        }
+      sum += lane_of<0xb1>(sum);   // neighbours
+      sum += lane_of<0x4e>(sum);   // pairs
+      sum += lane_of<0x141>(sum);  // halves of eight lanes
+      eight[b] = sum;
+    }
+    const float square_sum = ((eight[0] + eight[1]) + (eight[2] + eight[3])) + ((eight[4] + eight[5]) + (eight[6] + eight[7]));
+    const float inverse = rsqrtf(square_sum / (float)p.k + norm.epsilon);
+#pragma unroll
+    for (uint32_t group = 0; group < kNormedGroups; ++group)
+      if (group < groups) {
+        const u32x4_t g = *reinterpret_cast<const u32x4_t *>(gains + group * 128);
+        u32x4_t y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = normed_pair<DUAL>(x[group][e], g[e], inverse);
+        *reinterpret_cast<u32x4_t *>(place + group * 1024) = y;
+      }
+  }
+  __syncthreads();
+
+  f16x_t acc[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[r][i] = 0.0f;
+  const int column = ct * 32 + (lane & 31), half = lane >> 5;
+  const uint32_t row = lane & 31, row_twist = (row >> 1) & 7, column_twist = (column >> 2) & 3;
+  const unsigned char *x_own = rows + (row >> 3) * groups * 1024 + (row & 7) * 128;
+  const unsigned char *w_own = rows + x_bytes + (column >> 4) * pairs * 1024 + (column & 15) * 64;
+  const uint32_t *scale_own = reinterpret_cast<const uint32_t *>(rows_lds) + (column >> 3) * group_blocks * 64 + (column & 7);
+  for (uint32_t group = part; group < groups; group += P) {
+    const u32x4_t packed = *reinterpret_cast<const u32x4_t *>(w_own + (group >> 1) * 1024 + (((group & 1) * 2 + half) ^ column_twist) * 16);
+    h8_t x[RT][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+        x[r][j] = *reinterpret_cast<const h8_t *>(x_own + (r * 4 * groups + group) * 1024 + ((half * 4 + j) ^ row_twist) * 16);
+    const float scale = half_bits_to_float((uint16_t)scale_own[(group >> 3) * 64 + (group & 7) * 8]);
+    f16x_t sum[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum[r][i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const h8_t w = w4_exact_natural(packed[j]);
+#pragma unroll
+      for (int r = 0; r < RT; ++r) sum[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[r][j], w, sum[r], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[r][i] = fmaf(scale, sum[r][i], acc[r][i]);
+  }
+  finish_rows<ROWS, CT, P, DUAL>(p, acc, {segment, n, m0, n0, part, column, half}, reinterpret_cast<float *>(rows));
+}
+
 template <int ROWS, int CT, int P, int STAGES, bool DUAL, class Params>
 hipError_t run_rows(Params &p, hipStream_t stream) {
   const auto kernel = w4a16_rows_kernel<ROWS, CT, P, STAGES, DUAL, Params>;
@@ -352,6 +532,20 @@ hipError_t launch_tile(RowsTile tile, Params &p, hipStream_t stream) {
     case RowsTile::kNone: break;
   }
   return hipErrorInvalidValue;
+}
+
+template <int ROWS, int CT, int P, bool DUAL, class Params>
+hipError_t run_normed_rows(Params &p, const W4Norm &norm, hipStream_t stream) {
+  const auto kernel = w4a16_normed_rows_kernel<ROWS, CT, P, DUAL, Params>;
+  const uint32_t bytes = normed_rows_lds_bytes<ROWS, CT, P>(p.k);
+  if (bytes > kRowsLdsBytes) return hipErrorInvalidValue;
+  static bool allowed[kMaxDevices] = {};
+  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), kRowsLdsBytes, allowed)) return status;
+  constexpr uint32_t columns = DUAL ? CT * 16 : CT * 32;
+  uint32_t tiles = 0;
+  for (uint32_t i = 0; i < p.segments; ++i) tiles += p.tiles[i] = (p.n[i] + columns - 1) / columns;
+  kernel<<<dim3(tiles, (p.m + ROWS - 1) / ROWS), CT * P * 64, bytes, stream>>>(p, norm);
+  return hipGetLastError();
 }
 
 static_assert(kRowGroup == kGemvMaxRows);
@@ -447,7 +641,19 @@ hipError_t launch_w4a16_rows_qkv_pack(const W4QkvArgs &a, const RotaryPackArgs &
   p.token_stride = r.pack.token_stride;
   p.token_elements = r.pack.token_elements;
   for (int i = 0; i < 2; ++i) p.segment_offset[i] = r.pack.segment_offset[i];
-  return launch_tile<false>(pack_rows_tile(a.m, a.n, a.k, cus()), p, stream);
+  const RowsTile tile = pack_rows_tile(a.m, a.n, a.k, cus());
+  return a.norm.weight != nullptr ? run_normed_rows<32, 2, 4, false>(p, a.norm, stream) : launch_tile<false>(tile, p, stream);
+}
+
+bool w4a16_rows_norm_ok(const W4QkvArgs &a, const W4Norm &norm, const RotaryPackArgs &r) {
+  return pieces_aligned(a.x, norm.weight) && norm.weight_first == 0 && w4a16_rows_pack_ok(a, r) &&
+         normed_rows(pack_rows_tile(a.m, a.n, a.k, cus()), a.m, a.n, 3, a.k, cus());
+}
+
+bool w4a16_rows_norm_ok(const W4DualSwigluArgs &a, const W4Norm &norm) {
+  const uint32_t columns = 2 * a.n;
+  return pieces_aligned(a.x, norm.weight) && norm.weight_first != 0 && w4a16_rows_ok(a) && a.n <= 0x7fffffffu &&
+         normed_rows(gated_rows_tile(a.m, a.n, a.k, cus()), a.m, &columns, 1, a.k, cus());
 }
 
 bool w4a16_rows_ok(const W4DualSwigluArgs &a) {
@@ -467,7 +673,8 @@ hipError_t launch_w4a16_rows_dual_swiglu(const W4DualSwigluArgs &a, hipStream_t 
   p.y[0] = a.product;
   p.n[0] = a.n;
   p.segments = 1;
-  return launch_tile<true>(gated_rows_tile(a.m, a.n, a.k, cus()), p, stream);
+  const RowsTile tile = gated_rows_tile(a.m, a.n, a.k, cus());
+  return a.norm.weight != nullptr ? run_normed_rows<32, 2, 4, true>(p, a.norm, stream) : launch_tile<true>(tile, p, stream);
 }
 
 }  // namespace llmopt

@@ -28,6 +28,15 @@ constexpr uint32_t rows_lds_bytes(uint32_t k) {
   return scale_lds_bytes(CT * 32, k / 64) + (ring > sums ? ring : sums);
 }
 
+// Rows, weights and norm weights of a whole K (w4a16_normed_rows_kernel), whose lanes hold a piece of every group.
+constexpr uint32_t kNormedGroups = 12;
+template <int ROWS, int CT, int P>
+constexpr uint32_t normed_rows_lds_bytes(uint32_t k) {
+  const uint32_t groups = k / 64, sums = P * ROWS * CT * 32 * 4;
+  const uint32_t whole = ROWS * groups * 128 + CT * 32 * ((groups + 1) / 2) * 64 + (groups + 7) / 8 * 1024;
+  return scale_lds_bytes(CT * 32, groups) + (whole > sums ? whole : sums);
+}
+
 // The matrix-core GEMV's row groups are the better ones while they are few: up to two workgroups a CU, counted as eight
 // rows by sixteen columns, of which a gated pair has both matrices in one.  The tiles' shortest launch is longer than
 // theirs, more so with a long K; a third workgroup on a CU adds a whole round to them.  Each call behind the launch that
@@ -149,6 +158,14 @@ inline RowsTile logits_rows_tile(uint32_t rows, uint32_t n, uint32_t k, uint32_t
   if (rows > 32 && rows <= 65536 * 64 && rows_lds_bytes<64, 4, 2, 2>(k) <= kRowsLdsBytes) return RowsTile::k64x128;
   if (rows <= 65536 * 32 && rows_lds_bytes<32, 2, 4, 2>(k) <= kRowsLdsBytes) return RowsTile::k32x64;
   return RowsTile::kNone;
+}
+
+// Whether a tile normalises its rows itself: tiles of 32 rows and a K that fits LDS as a whole, in one round of workgroups.
+inline bool normed_rows(RowsTile tile, uint32_t m, const uint32_t *n, uint32_t matrices, uint32_t k, uint32_t cus) {
+  if (tile != RowsTile::k32x64 || k > kNormedGroups * 64) return false;
+  uint64_t tiles = 0;
+  for (uint32_t i = 0; i < matrices; ++i) tiles += ((uint64_t)n[i] + 63) / 64;
+  return tiles * ((m + 31) / 32) <= (uint64_t)cus * (kRowsLdsBytes / normed_rows_lds_bytes<32, 2, 4>(k));
 }
 
 }  // namespace llmopt

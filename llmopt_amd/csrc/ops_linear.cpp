@@ -83,13 +83,14 @@ int w4a16_linear(llmopt_hip_context *context, const DispatchRecord &record) {
 
 // The activation of a normalising entry: either the kernel normalises (*norm is set and *x stays
 // the raw input) or the rows are normalised into the context's scratch here (*x moves there).
+// in_tiles: the small tiles' launch can take the raw input.
 int normalise_input(llmopt_hip_context *context, const DispatchRecord &record, const W4Norm &wanted, uint32_t m,
-                    uint32_t k, uint64_t columns, const uint16_t **x, W4Norm *norm) {
+                    uint32_t k, uint64_t columns, const uint16_t **x, W4Norm *norm, bool in_tiles = false) {
   if (!std::isfinite(wanted.epsilon) || wanted.epsilon <= 0.0f)
     return fail(LLMOPT_ERR_INVALID, "%s requires a positive finite epsilon", record.name.c_str());
   if (int status = require_buffer_size(record.buffers[1], (uint64_t)k * 2, "norm weight")) return status;
   const bool aligned = ((reinterpret_cast<uintptr_t>(*x) | reinterpret_cast<uintptr_t>(wanted.weight)) & 15) == 0;
-  if (aligned && w4a16_norm_in_kernel(m, columns, k)) {
+  if (in_tiles || (aligned && w4a16_norm_in_kernel(m, columns, k))) {
     *norm = wanted;
     return LLMOPT_OK;
   }
@@ -195,10 +196,10 @@ int rms_w4a16_qkv_rotary_pack_prompt(llmopt_hip_context *context, const Dispatch
   args.y[2] = reinterpret_cast<uint16_t *>(record.buffers[12].device);
   args.x = as_f16(record.buffers[0]);
   const W4Norm norm = {as_f16(record.buffers[1]), param_f32(record, 20), 0};
-  if (int status = normalise_input(context, record, norm, args.m, args.k, (uint64_t)args.n[0] + 2 * (uint64_t)args.n[1], &args.x,
-                                   &args.norm))
-    return status;
-  if (w4a16_rows_pack_ok(args, pack)) return launched(launch_w4a16_rows_qkv_pack(args, pack, context->stream), name);
+  const uint64_t columns = (uint64_t)args.n[0] + 2 * (uint64_t)args.n[1];
+  const bool in_tiles = !w4a16_norm_in_kernel(args.m, columns, args.k) && w4a16_rows_norm_ok(args, norm, pack);
+  if (int status = normalise_input(context, record, norm, args.m, args.k, columns, &args.x, &args.norm, in_tiles)) return status;
+  if (in_tiles || w4a16_rows_pack_ok(args, pack)) return launched(launch_w4a16_rows_qkv_pack(args, pack, context->stream), name);
   if (int status = launched(launch_w4a16_qkv(args, context->stream), name)) return status;
   return launched(launch_rotary_qk_pack(pack, context->stream), name);
 }
@@ -226,7 +227,9 @@ int dual_swiglu(llmopt_hip_context *context, const DispatchRecord &record, bool 
   args.k = k;
   if (normalised) {
     const W4Norm norm = {as_f16(record.buffers[1]), param_f32(record, 12), 1};  // llmopt_w4a16_swiglu_rms_f16_g64's order
-    if (int status = normalise_input(context, record, norm, m, k, 2ull * n, &args.x, &args.norm)) return status;
+    const bool in_tiles = !w4a16_norm_in_kernel(m, 2ull * n, k) && w4a16_rows_norm_ok(args, norm);
+    if (int status = normalise_input(context, record, norm, m, k, 2ull * n, &args.x, &args.norm, in_tiles)) return status;
+    if (in_tiles) return launched(launch_w4a16_rows_dual_swiglu(args, context->stream), record.name.c_str());
   }
   return launched(launch_w4a16_dual_swiglu(args, context->stream), record.name.c_str());
 }

@@ -214,3 +214,27 @@ def test_logits_of_more_rows_than_a_grid_of_tiles_has():
     chosen = expected.gather(1, ids.long()[:, None])[:, 0]
     assert (chosen >= expected.max(1).values - 2 * sums.max(1).values).all()
     runtime.close()
+
+
+# One launch that normalises its rows: one to twelve scale groups, an odd and an even number of them, remainders of rows and
+# columns, a row of zeros and one of the largest values
+NORMED_PAIRS = [(300, 200, 64), (130, 1500, 192), (300, 401, 448), (100, 1537, 576), (129, 1000, 640), (140, 801, 768)]
+
+
+@pytest.mark.parametrize("m,n,k", NORMED_PAIRS)
+def test_pairs_of_rows_that_are_normalised_in_the_tile(runtime, m, n, k):
+    """Bit for bit what the norm and the pair leave as launches of their own."""
+    rng = np.random.default_rng(m + n + k)
+    x, gate, gate_scale, _ = w4_case(rng, m, n, k)
+    _, up, up_scale, _ = w4_case(rng, 1, n, k)
+    x[m // 2], x[m - 1] = 0, 65504
+    norm = rng.uniform(0.5, 1.5, k).astype(np.float16)
+    put = runtime.buffer_of_bytes
+    params, weights = u32s(m, n, k) + struct.pack("<f", 1e-5), [put(a) for a in (gate, gate_scale, up, up_scale)]
+    normed, (one, two) = put(np.zeros((m, k), dtype=np.float16)), (put(np.full((m, n), np.nan, dtype=np.float16)) for _ in range(2))
+    runtime.dispatch("llmopt_w4a16_swiglu_rms_f16_g64", [put(x), put(norm), normed], params, (m, 1, 1), (256, 1, 1))
+    grid = (linear_grid(((m + 3) // 4) * n), 1, 1)
+    runtime.dispatch("llmopt_w4a16_dual_swiglu_f16_g64_m4", [normed, *weights, two], params, grid, (256, 1, 1))
+    runtime.dispatch("llmopt_rms_w4a16_dual_swiglu_f16_g64", [put(x), put(norm), *weights, one], params, grid, (256, 1, 1))
+    np.testing.assert_array_equal(one.numpy(np.uint16), two.numpy(np.uint16))
+    assert np.isfinite(one.numpy(np.float16)).all()

@@ -29,6 +29,14 @@ int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
 int product_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_tile(m, n, k, cus); }
 int staggered_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_product_tile(m, n, k, cus); }
 int split_columns(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_column_split(m, n, k, cus).columns; }
+int normed_pair(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
+  const uint32_t columns = 2 * n;
+  return normed_rows(gated_rows_tile(m, n, k, cus), m, &columns, 1, k, cus);
+}
+int normed_qkv(uint32_t m, uint32_t q, uint32_t kv, uint32_t k, uint32_t cus) {
+  const uint32_t n[3] = {q, kv, kv};
+  return normed_rows(pack_rows_tile(m, n, k, cus), m, n, 3, k, cus);
+}
 int qkv_tile(uint32_t m, uint32_t q, uint32_t kv, uint32_t k, uint32_t cus) {
   const uint32_t n[3] = {q, kv, kv};
   return (int)qkv_rows_tile(m, n, k, cus);
@@ -169,3 +177,12 @@ def test_products_that_stay_in_step(rules, m, n, k):
                                          (2048, 16384, 2048, 0), (3001, 16384, 2048, 0), (2048, 2048, 8192, 0), (2048, 8512, 960, 0)])
 def test_columns_in_two_launches(rules, m, n, k, first):
     assert rules.split_columns(m, n, k, CUS) == first
+
+
+def test_rows_normalised_in_the_tile(rules):
+    """Tiles of 32 rows in one round, and a whole K in LDS."""
+    assert all(rules.normed_pair(m, n, k, CUS) for m, n, k in test_gpu_w4a16_rows.NORMED_PAIRS)
+    assert rules.normed_qkv(700, 576, 192, 576, CUS) and rules.normed_qkv(90, 576, 192, 576, CUS)
+    assert not rules.normed_pair(700, 1536, 576, CUS)       # 96 rows
+    assert not rules.normed_pair(100, 1000, 832, CUS)       # thirteen groups
+    assert not rules.normed_qkv(1300, 576, 192, 576, CUS)   # a second round
