@@ -119,6 +119,7 @@ struct DenseGemvArgs {
   // input: norm_weight == null: activation-type row, or f32 (x_is_f32); else the f32 row normalised on the way in
   const void *x;
   bool x_is_f32;
+  const uint32_t *row_index;  // null, or with a norm: which row of x (and of a pending output) it is
   const uint16_t *norm_weight;
   uint32_t norm_groups;
   float epsilon;

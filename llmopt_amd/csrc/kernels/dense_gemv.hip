@@ -24,12 +24,17 @@ __device__ __forceinline__ uint32_t staged_index(uint32_t k, uint32_t plane) {
   return ((k >> 2) & 1) * plane + ((k >> 3) << 2) + (k & 3);
 }
 
+// Where the launch's row begins (another trip to memory only where its number is not known ahead).
+__device__ __forceinline__ size_t first_value(const DenseGemvArgs &a) {
+  return a.row_index ? (size_t)*a.row_index * a.k : 0;
+}
+
 // A row of at most PIECES * 1024 values through registers: one trip to memory.
 template <int PIECES, typename Ahead>
 __device__ __forceinline__ void stage_normed_row(const DenseGemvArgs &a, float *xs, uint32_t plane, float *scratch,
                                                  Ahead ahead) {
   const uint32_t k = a.k;
-  const float *x = static_cast<const float *>(a.x);
+  const float *x = static_cast<const float *>(a.x) + first_value(a);
   const __bf16 *weight = reinterpret_cast<const __bf16 *>(a.norm_weight);
   f32x4 v[PIECES];
   bf16x4 w[PIECES];
@@ -68,7 +73,8 @@ template <int PIECES, typename Ahead>
 __device__ __forceinline__ void stage_pending_row(const DenseGemvArgs &a, float *xs, uint32_t plane, float *scratch,
                                                   Ahead ahead) {
   const uint32_t k = a.k;
-  const float *x = static_cast<const float *>(a.x);
+  const size_t first = first_value(a);
+  const float *x = static_cast<const float *>(a.x) + first, *pending = a.pending + first;
   const __bf16 *add = reinterpret_cast<const __bf16 *>(a.pending_weight);
   const __bf16 *weight = reinterpret_cast<const __bf16 *>(a.norm_weight);
   f32x4 v[PIECES], y[PIECES];
@@ -81,7 +87,7 @@ __device__ __forceinline__ void stage_pending_row(const DenseGemvArgs &a, float 
     w[q] = bf16x4{0, 0, 0, 0};
     if (i < k) {
       v[q] = *reinterpret_cast<const f32x4 *>(x + i);
-      y[q] = *reinterpret_cast<const f32x4 *>(a.pending + i);
+      y[q] = *reinterpret_cast<const f32x4 *>(pending + i);
       w[q] = *reinterpret_cast<const bf16x4 *>(add + i);
     }
   }
@@ -125,14 +131,15 @@ __device__ __forceinline__ void stage_pending_row(const DenseGemvArgs &a, float 
 // The same for any length, through the staged row.
 __device__ __forceinline__ void stage_pending_any(const DenseGemvArgs &a, float *xs, uint32_t plane, float *scratch) {
   const uint32_t k = a.k;
-  const float *x = static_cast<const float *>(a.x);
+  const size_t first = first_value(a);
+  const float *x = static_cast<const float *>(a.x) + first, *pending = a.pending + first;
   float sum = 0.0f;
-  for (uint32_t i = threadIdx.x; i < k; i += kWaves * 64) sum += a.pending[i] * a.pending[i];
+  for (uint32_t i = threadIdx.x; i < k; i += kWaves * 64) sum += pending[i] * pending[i];
   const float factor = a.pending_scale / sqrtf(block_sum<kWaves>(sum, scratch) / (float)k + a.epsilon);
   sum = 0.0f;
   for (uint32_t i = threadIdx.x; i < k; i += kWaves * 64) {
     const float w = a.norm_offset + (float)reinterpret_cast<const __bf16 *>(a.pending_weight)[i];
-    const float v = fmaf(a.pending[i] * factor, w, x[i]);
+    const float v = fmaf(pending[i] * factor, w, x[i]);
     if (blockIdx.x == 0 && a.stream_out) a.stream_out[i] = v;
     sum += v * v;
     xs[staged_index(i, plane)] = v;
@@ -213,7 +220,7 @@ __device__ __forceinline__ void stage_activation(const DenseGemvArgs &a, float *
   if (a.norm_groups == 1 && (k & 3) == 0 && k <= 8 * 4 * kWaves * 64)
     return stage_normed_row<8>(a, xs, plane, scratch, ahead);
   ahead();
-  const float *x = static_cast<const float *>(a.x);
+  const float *x = static_cast<const float *>(a.x) + first_value(a);
   const __bf16 *weight = reinterpret_cast<const __bf16 *>(a.norm_weight);
   const uint32_t part = k / a.norm_groups;
   for (uint32_t g = 0; g < a.norm_groups; ++g) {

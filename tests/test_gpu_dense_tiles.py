@@ -185,3 +185,31 @@ def test_routed_tiles(runtime, m, width, ff):
 
 def test_split_columns_of_steps(runtime):
     test_rows_split_in_two(runtime, *SPLIT[0])
+
+
+# The logits of one row among several: short rows, more than 4096 values, no whole pieces of four or eight
+@pytest.mark.parametrize("m,width,vocabulary,row", [(5, 64, 100, 3), (2, 2048, 1001, 0), (700, 1000, 333, 699), (3, 4104, 50, 1),
+                                                    (4, 1001, 77, 2)])
+@pytest.mark.parametrize("pending", [False, True])
+def test_logits_of_one_row(runtime, m, width, vocabulary, row, pending):
+    """Float32 sums of `width` products: 2^-24 of a sum of magnitudes each, a few units for the norms and the cap."""
+    rng = np.random.default_rng(m + width)
+    x, y = (rng.standard_normal((m, width)).astype(np.float32) for _ in range(2))
+    (add, fadd), (norm, fnorm), (head, fhead) = values(rng, width), values(rng, width), values(rng, vocabulary, width, gain=width ** -0.5)
+    put, rms = runtime.buffer_of_bytes, lambda v: v / np.sqrt(np.mean(v * v) + 1e-6)
+    out, index = put(np.full(vocabulary, np.nan, dtype=np.float32)), put(np.array([row], dtype=np.uint32))
+    stream = x[row].astype(np.float64)
+    if pending:
+        stream = stream + 0.5 * rms(y[row].astype(np.float64)) * (1.0 + fadd)
+        normed = rms(stream) * (1.0 + fnorm)
+        runtime.dispatch("llmopt_pending_logits_bf16", [put(x), put(y), put(add), put(x), index, put(norm), put(head), out],
+                         u32s(1, width, vocabulary, m, 1) + struct.pack("<4f", 1e-6, 1.0, 0.5, 30.0), *GRID)
+    else:
+        normed = rms(stream) * fnorm
+        runtime.dispatch("llmopt_rms_logits_bf16", [put(x), index, put(norm), put(head), out],
+                         u32s(1, width, vocabulary) + struct.pack("<fI", 1e-6, m), *GRID)
+    expected = fhead @ normed
+    bound = (width + 16) * 2.0 ** -24 * (np.abs(fhead) @ np.abs(normed))
+    if pending:
+        expected, bound = 30.0 * np.tanh(expected / 30.0), bound + 16 * 2.0 ** -24 * 30.0
+    assert np.all(np.abs(out.numpy(np.float32) - expected) <= bound)
