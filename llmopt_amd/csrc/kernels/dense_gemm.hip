@@ -20,6 +20,7 @@
 #include "dense_common.h"
 #include "dense_tile_rule.h"
 #include "kernels_internal.h"
+#include "staggered.h"
 
 namespace llmopt {
 namespace {
@@ -484,20 +485,6 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParam
   emit_rows<MT, NT, GATED>(a, acc, place.m_first, place.m_rows, place.n_first, wm * (BM / WM), wn * (BN / WN), lane,
                            stage_rows + wave * 16 * (NT * 16 + 8));
 }
-
-// A barrier that nothing moves across.
-__device__ __forceinline__ void meet() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("" ::: "memory");
-}
-template <int COUNT>
-__device__ __forceinline__ void copies_landed() {  // all but the last COUNT
-  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(COUNT) : "memory");
-}
-__device__ __forceinline__ void lds_read() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // The same product for large launches: 256 x 256 tiles of eight waves, two on a SIMD, of which one reads operands and
 // requests copies while the other one multiplies.  With all waves in step (dense_gemm_direct_kernel) the matrix cores had

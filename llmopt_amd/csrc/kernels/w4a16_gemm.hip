@@ -22,6 +22,7 @@
 
 #include "kernels.h"
 #include "kernels_internal.h"
+#include "staggered.h"
 #include "w4_common.h"
 
 namespace llmopt {
@@ -476,6 +477,231 @@ hipError_t launch_tile(GemmParams &p, hipStream_t stream, uint32_t splits = 1) {
   return hipGetLastError();
 }
 
+// Large launches: 256 x 256 tiles in four phases a K step, half of the waves a barrier behind, as dense_gemm_phased_kernel
+// (dense_gemm.hip): a wave's 128 x 64 outputs are four quadrants of 64 x 32, whose operands it reads while the other wave of
+// its SIMD multiplies.  The activations are the B operand, so that a lane ends with four columns of a row.
+//
+//  * The weights of step t + 1 are decoded (w4_scaled_natural: q * s in half) and written to their stage between the reads of
+//    the first three phases of step t, where the second group's writes are there before the first group reads them.
+//  * A wave's requests of a step are rows 1 of the next step (two copies, phase 0), rows 0 of the one behind it (two, phase 2)
+//    and the thread's weights and scale three steps ahead (two loads, phase 3): whatever is waited for, six younger ones may
+//    be under way.  Requests past the end fetch the last step again, which nothing reads.
+// us, the same tiles with all waves in step / these: 2048 x 4096 x 14336 240 / 214.
+__global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
+  constexpr int HALF = 16384, STAGE = 4 * HALF;  // halves of a stage: rows 0, rows 1, columns 0, columns 1
+  extern __shared__ __attribute__((aligned(16))) unsigned char gemm_lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const uint32_t total = p.tiles_m * p.tiles_n;
+  uint32_t logical = blockIdx.x;
+  if (total % 8 == 0) logical = (blockIdx.x % 8) * (total / 8) + blockIdx.x / 8;
+  const uint32_t m0 = logical % p.tiles_m * 256, n0 = logical / p.tiles_m * 256;
+  const uint32_t K = p.k;
+  const int steps = (int)(K / BK);
+
+  // rows of half h: h * 64 .. + 63 of each 128; columns: h * 32 .. + 31 of each 64 (a wave's own lie together)
+  const uint8_t *x_base = reinterpret_cast<const uint8_t *>(p.x + (size_t)m0 * K);
+  uint32_t x_at[2][2];  // bytes from the tile's first row
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const uint32_t row = (c * 8 + wave) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) x_at[h][c] = (min((row >> 6) * 128 + h * 64 + (row & 63), p.m - 1 - m0) * K + piece * 8) * 2;
+  }
+  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)gemm_lds;
+  auto request = [&](int half, int step) __attribute__((always_inline)) {
+    const uint32_t slot = lds_base + (step & 1) * STAGE + half * HALF;
+    const uint8_t *x = x_base + (size_t)min(step, steps - 1) * (BK * 2);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                   :
+                   : "v"(x_at[half][c]), "s"(x), "s"(slot + (c * 8 + wave) * 1024)
+                   : "memory");
+  };
+  // A thread's weights of a step: half of a column's 64.  (As in w4a16_gemm_kernel, nothing may copy a set between its
+  // request and its wait.)
+  struct Fetched {
+    u32x4_t w;
+    uint32_t s;  // fp16 bits in the low half
+  };
+  Fetched fetched[2];
+  const uint32_t column = tid >> 1, part = tid & 1;
+  const uint32_t w_col = min(column, p.n - 1 - n0);
+  const uint8_t *w_base = p.w[0] + (size_t)n0 * (K / 2), *s_base = reinterpret_cast<const uint8_t *>(p.s[0] + (size_t)n0 * (K / 64));
+  const uint32_t w_at = w_col * (K / 2) + part * 16, s_at = w_col * (K / 64) * 2;
+  auto fetch = [&](Fetched &f, int step) __attribute__((always_inline)) {
+    const uint32_t at = (uint32_t)min(step, steps - 1);
+    asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(f.w) : "v"(w_at), "s"(w_base + (size_t)at * 32) : "memory");
+    asm volatile("global_load_ushort %0, %1, %2" : "=&v"(f.s) : "v"(s_at), "s"(s_base + (size_t)at * 2) : "memory");
+  };
+  auto fetched_but = [&](Fetched &f, auto younger) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(f.w), "+v"(f.s) : "n"(decltype(younger)::value) : "memory");
+  };
+  const uint32_t w_row = (column >> 6) * 32 + (column & 31), w_twist = (w_row >> 1) & 7;
+  unsigned char *w_place = gemm_lds + (2 + ((column >> 5) & 1)) * HALF + w_row * 128;
+  auto decode = [&](const Fetched &f, int step, int item) __attribute__((always_inline)) {
+    const uint4 halves = w4_scaled_natural(f.w[item], __builtin_bit_cast(_Float16, (uint16_t)f.s));
+    *reinterpret_cast<uint4 *>(w_place + (step & 1) * STAGE + ((part * 4 + item) ^ w_twist) * 16) = halves;
+  };
+
+  f4_t acc[8][4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  const int fr = lane & 15, quad = lane >> 4, twist = (fr >> 1) & 7;
+  const int at0 = (quad ^ twist) * 16, at1 = ((4 + quad) ^ twist) * 16;
+  const int read_x = (wm * 64 + fr) * 128, read_w = (wn * 32 + fr) * 128 + 2 * HALF;
+  h8_t fx[4][2], fw[2][2][2];
+  auto read_rows = [&](int half, int step) __attribute__((always_inline)) {
+    const unsigned char *base = gemm_lds + (step & 1) * STAGE + half * HALF + read_x;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      fx[i][0] = *reinterpret_cast<const h8_t *>(base + i * 2048 + at0);
+      fx[i][1] = *reinterpret_cast<const h8_t *>(base + i * 2048 + at1);
+    }
+  };
+  auto read_columns = [&](int half, int step) __attribute__((always_inline)) {
+    const unsigned char *base = gemm_lds + (step & 1) * STAGE + half * HALF + read_w;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      fw[half][j][0] = *reinterpret_cast<const h8_t *>(base + j * 2048 + at0);
+      fw[half][j][1] = *reinterpret_cast<const h8_t *>(base + j * 2048 + at1);
+    }
+  };
+  auto multiply = [&](int i0, int j0) __attribute__((always_inline)) {
+    lds_read();  // (and what this wave wrote is there)
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i0 * 4 + i][j0 * 2 + j] =
+              __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[j0][j][kk], fx[i][kk], acc[i0 * 4 + i][j0 * 2 + j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  fetch(fetched[0], 0);
+  request(0, 0);
+  fetch(fetched[1], 1);
+  fetched_but(fetched[0], std::integral_constant<int, 4>{});
+#pragma unroll
+  for (int item = 0; item < 4; ++item) decode(fetched[0], 0, item);
+  request(1, 0);
+  request(0, 1);
+  fetch(fetched[0], 2);
+  copies_landed<8>();  // rows 0 of step 0
+  lds_read();
+  meet();
+  if (wm == 1) meet();
+  auto step = [&](int t, Fetched &next) __attribute__((always_inline)) {  // next: the weights of step t + 1
+    fetched_but(next, std::integral_constant<int, 6>{});
+    read_columns(0, t);
+    read_rows(0, t);
+    decode(next, t + 1, 0);
+    decode(next, t + 1, 1);
+    request(1, t + 1);
+    meet();
+    multiply(0, 0);
+    meet();
+    read_columns(1, t);
+    decode(next, t + 1, 2);
+    copies_landed<6>();  // rows 1 of this step
+    meet();
+    multiply(0, 1);
+    meet();
+    read_rows(1, t);
+    decode(next, t + 1, 3);
+    request(0, t + 2);
+    meet();
+    multiply(1, 1);
+    meet();
+    copies_landed<6>();  // rows 0 of the next step
+    fetch(next, t + 3);
+    meet();
+    multiply(1, 0);
+    meet();
+  };
+  int t = 0;
+  for (; t + 1 < steps; t += 2) {
+    step(t, fetched[1]);
+    step(t + 1, fetched[0]);
+  }
+  if (t < steps) step(t, fetched[1]);
+  fetched_but(fetched[0], std::integral_constant<int, 0>{});  // the surplus requests still target live registers
+  fetched_but(fetched[1], std::integral_constant<int, 0>{});
+  if (wm == 0) meet();
+  __syncthreads();  // the stages' LDS is free
+
+  // sixteen rows at a time through the wave's own LDS rows, so that a store covers whole lines
+  constexpr int WIDTH = 64, STRIDE = WIDTH + 8, PIECES = WIDTH / 8;
+  uint16_t *rows = reinterpret_cast<uint16_t *>(gemm_lds) + wave * 16 * STRIDE;
+  const uint32_t c_first = n0 + wn * WIDTH;
+  const bool whole_addend = (p.addend_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(p.addend) & 7) == 0;
+  const bool whole = (p.n & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t row = min(m0 + wm * 128 + i * 16 + fr, p.m - 1);
+    ushort4 addend[4] = {};
+    if (p.has_addend) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t c = c_first + j * 16 + quad * 4;
+        const uint16_t *from = p.addend + (size_t)row * p.addend_stride;
+        if (whole_addend && c + 4 <= p.n) addend[j] = *reinterpret_cast<const ushort4 *>(from + c);
+        else addend[j] = ushort4{from[min(c, p.n - 1)], from[min(c + 1, p.n - 1)], from[min(c + 2, p.n - 1)], from[min(c + 3, p.n - 1)]};
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < WIDTH / 16; ++j) {
+      f4_t v = acc[i][j];
+      if (p.has_addend) {
+        v[0] += half_bits_to_float(addend[j].x);
+        v[1] += half_bits_to_float(addend[j].y);
+        v[2] += half_bits_to_float(addend[j].z);
+        v[3] += half_bits_to_float(addend[j].w);
+      }
+      *reinterpret_cast<ushort4 *>(rows + fr * STRIDE + j * 16 + quad * 4) =
+          ushort4{float_to_half_bits(v[0]), float_to_half_bits(v[1]), float_to_half_bits(v[2]), float_to_half_bits(v[3])};
+    }
+    lds_read();
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < 16 * PIECES / 64; ++q) {
+      const int index = q * 64 + lane, r = index / PIECES, piece = index % PIECES;
+      const uint32_t at = m0 + wm * 128 + i * 16 + r, c = c_first + piece * 8;
+      if (at >= p.m || c >= p.n) continue;
+      const uint16_t *from = rows + r * STRIDE + piece * 8;
+      uint16_t *to = p.y + (size_t)at * p.n + c;
+      if (whole) {
+        *reinterpret_cast<uint4 *>(to) = *reinterpret_cast<const uint4 *>(from);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (c + e < p.n) to[e] = from[e];
+      }
+    }
+    lds_read();
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+hipError_t launch_phased(GemmParams &p, hipStream_t stream) {
+  constexpr int bytes = 2 * 4 * 16384;
+  static bool configured[kMaxDevices] = {};
+  const auto kernel = w4a16_gemm_phased_kernel;
+  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, configured)) return status;
+  p.tiles_m = (p.m + 255) / 256;
+  p.tiles_n = (p.n + 255) / 256;
+  kernel<<<p.tiles_m * p.tiles_n, kThreads, bytes, stream>>>(p);
+  return hipGetLastError();
+}
+
 // K ranges per tile when 128 x 128 tiles leave at least half the CUs without one (1: no split):
 // as many as fill the device, each a whole number of four-step loop passes.
 uint32_t gemm_k_splits(uint32_t m, uint32_t n, uint32_t k) {
@@ -498,15 +724,16 @@ hipError_t launch_gemm(GemmParams &p, hipStream_t stream) {
     if (small_pair <= (uint64_t)cus) return launch_tile<1, 2, true, 4>(p, stream);
     return launch_tile<2, 2, true>(p, stream);
   }
-  // 256 x 256 when that still gives every CU a tile, otherwise 256 x 128 / 128 x 256 / 128 x 128
-  const uint64_t big = (uint64_t)((p.m + 255) / 256) * ((p.n + 255) / 256);
-  if (big >= (uint64_t)cus) return launch_tile<2, 4, false>(p, stream);
-  // Half that size, tall (256 x 128) or wide (128 x 256), whichever pads less; the tall one when
+  // Tall (256 x 128) or wide (128 x 256) tiles, whichever pads less; the tall one when
   // they tie (its waves read 16 operand vectors from LDS per 16 MFMAs, the wide one's 20: 76.5
   // against 80 us at 512 x 14336, 81.7 against 86.3 at 2048 x 4096).  Also when a few CUs stay
   // without a tile: 224 such tiles beat 448 of 128 x 128, two on most CUs.
   const uint64_t tall = (uint64_t)((p.m + 255) / 256) * ((p.n + 127) / 128);
   const uint64_t wide = (uint64_t)((p.m + 127) / 128) * ((p.n + 255) / 256);
+  // 256 x 256 once even the better of those would begin a second round (offsets from a tile's first row are 32 bits there): us,
+  // 256 x 128 or 128 x 256 / 256 x 256: 2048 x 2048 x 6144 82 / 63, 1024 x 4096 x 14336 154 / 118, 1430 x 576 x 5632 30.5 / 22.9;
+  // where they are one round 1134 x 2112 x 6720 45 / 55, 541 x 576 x 11840 20 / 23.
+  if (std::min(tall, wide) > (uint64_t)cus && p.k <= (1u << 22)) return launch_phased(p, stream);
   if (std::min(tall, wide) * 8 >= (uint64_t)cus * 7)
     return tall <= wide ? launch_tile<2, 2, false>(p, stream) : launch_tile<1, 4, false>(p, stream);
   // 128 x 128 tiles have steps shorter than a trip to memory.  With two stages they fit a CU

@@ -238,3 +238,25 @@ def test_pairs_of_rows_that_are_normalised_in_the_tile(runtime, m, n, k):
     runtime.dispatch("llmopt_rms_w4a16_dual_swiglu_f16_g64", [put(x), put(norm), *weights, one], params, grid, (256, 1, 1))
     np.testing.assert_array_equal(one.numpy(np.uint16), two.numpy(np.uint16))
     assert np.isfinite(one.numpy(np.float16)).all()
+
+
+# 256 x 256 tiles: one to nine K steps, remainders of rows and columns, whole and odd rows of outputs and addends
+@pytest.mark.parametrize("m,n,k,addend", [(4000, 4100, 64, "none"), (4001, 4097, 128, "bias"), (2050, 7301, 192, "residual"),
+                                          (2300, 7304, 256, "residual"), (4096, 4096, 320, "bias"), (2049, 7425, 576, "none"),
+                                          (1290, 5637, 192, "bias")])
+def test_tiles_of_256(runtime, m, n, k, addend):
+    test_small_tiles(runtime, m, n, k, addend)
+
+
+def test_tiles_of_256_keep_infinities_in_their_row(runtime):
+    m, n, k = 4001, 4099, 192
+    rng = np.random.default_rng(1)
+    x, packed, _, _ = w4_case(rng, m, n, k)
+    x = rng.integers(-4, 5, (m, k)).astype(np.float16)
+    scale = np.ones((n, k // 64), dtype=np.float16)
+    expected = product(x, packed, scale)
+    np.testing.assert_array_equal(run_linear(runtime, x, packed, scale), expected.astype(np.float16))
+    x[m - 1, k - 1] = np.inf
+    out = run_linear(runtime, x, packed, scale)
+    assert not np.isfinite(out[m - 1]).any()
+    np.testing.assert_array_equal(out[:m - 1], expected.astype(np.float16)[:m - 1])
