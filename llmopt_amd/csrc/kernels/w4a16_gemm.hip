@@ -487,6 +487,7 @@ hipError_t launch_tile(GemmParams &p, hipStream_t stream, uint32_t splits = 1) {
 //    and the thread's weights and scale three steps ahead (two loads, phase 3): whatever is waited for, six younger ones may
 //    be under way.  Requests past the end fetch the last step again, which nothing reads.
 // us, the same tiles with all waves in step / these: 2048 x 4096 x 14336 240 / 214.
+template <bool DUAL>
 __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
   constexpr int HALF = 16384, STAGE = 4 * HALF;  // halves of a stage: rows 0, rows 1, columns 0, columns 1
   extern __shared__ __attribute__((aligned(16))) unsigned char gemm_lds[];
@@ -496,7 +497,7 @@ __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
   const uint32_t total = p.tiles_m * p.tiles_n;
   uint32_t logical = blockIdx.x;
   if (total % 8 == 0) logical = (blockIdx.x % 8) * (total / 8) + blockIdx.x / 8;
-  const uint32_t m0 = logical % p.tiles_m * 256, n0 = logical / p.tiles_m * 256;
+  const uint32_t m0 = logical % p.tiles_m * 256, n0 = logical / p.tiles_m * (DUAL ? 128 : 256);
   const uint32_t K = p.k;
   const int steps = (int)(K / BK);
 
@@ -527,9 +528,12 @@ __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
     uint32_t s;  // fp16 bits in the low half
   };
   Fetched fetched[2];
-  const uint32_t column = tid >> 1, part = tid & 1;
-  const uint32_t w_col = min(column, p.n - 1 - n0);
-  const uint8_t *w_base = p.w[0] + (size_t)n0 * (K / 2), *s_base = reinterpret_cast<const uint8_t *>(p.s[0] + (size_t)n0 * (K / 64));
+  // (of a pair the columns alternate by sixteen between gate and up: a wave has those of one matrix)
+  const uint32_t matrix = DUAL ? wave & 1 : 0, part = tid & 1;
+  const uint32_t column = DUAL ? (wave >> 1) * 64 + (lane >> 5) * 32 + matrix * 16 + ((lane >> 1) & 15) : tid >> 1;
+  const uint32_t w_col = min(DUAL ? (column >> 5) * 16 + (column & 15) : column, p.n - 1 - n0);
+  const uint8_t *w_base = p.w[matrix] + (size_t)n0 * (K / 2);
+  const uint8_t *s_base = reinterpret_cast<const uint8_t *>(p.s[matrix] + (size_t)n0 * (K / 64));
   const uint32_t w_at = w_col * (K / 2) + part * 16, s_at = w_col * (K / 64) * 2;
   auto fetch = [&](Fetched &f, int step) __attribute__((always_inline)) {
     const uint32_t at = (uint32_t)min(step, steps - 1);
@@ -639,7 +643,7 @@ __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
   __syncthreads();  // the stages' LDS is free
 
   // sixteen rows at a time through the wave's own LDS rows, so that a store covers whole lines
-  constexpr int WIDTH = 64, STRIDE = WIDTH + 8, PIECES = WIDTH / 8;
+  constexpr int WIDTH = DUAL ? 32 : 64, STRIDE = WIDTH + 8, PIECES = WIDTH / 8;
   uint16_t *rows = reinterpret_cast<uint16_t *>(gemm_lds) + wave * 16 * STRIDE;
   const uint32_t c_first = n0 + wn * WIDTH;
   const bool whole_addend = (p.addend_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(p.addend) & 7) == 0;
@@ -648,7 +652,7 @@ __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
   for (int i = 0; i < 8; ++i) {
     const uint32_t row = min(m0 + wm * 128 + i * 16 + fr, p.m - 1);
     ushort4 addend[4] = {};
-    if (p.has_addend) {
+    if (!DUAL && p.has_addend) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const uint32_t c = c_first + j * 16 + quad * 4;
@@ -659,8 +663,17 @@ __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
     }
 #pragma unroll
     for (int j = 0; j < WIDTH / 16; ++j) {
-      f4_t v = acc[i][j];
-      if (p.has_addend) {
+      f4_t v;
+      if constexpr (DUAL) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float gate = acc[i][2 * j][e];
+          v[e] = gate / (1.0f + __expf(-gate)) * acc[i][2 * j + 1][e];
+        }
+      } else {
+        v = acc[i][j];
+      }
+      if (!DUAL && p.has_addend) {
         v[0] += half_bits_to_float(addend[j].x);
         v[1] += half_bits_to_float(addend[j].y);
         v[2] += half_bits_to_float(addend[j].z);
@@ -691,13 +704,14 @@ __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
   }
 }
 
+template <bool DUAL>
 hipError_t launch_phased(GemmParams &p, hipStream_t stream) {
   constexpr int bytes = 2 * 4 * 16384;
   static bool configured[kMaxDevices] = {};
-  const auto kernel = w4a16_gemm_phased_kernel;
+  const auto kernel = w4a16_gemm_phased_kernel<DUAL>;
   if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, configured)) return status;
   p.tiles_m = (p.m + 255) / 256;
-  p.tiles_n = (p.n + 255) / 256;
+  p.tiles_n = DUAL ? (p.n + 127) / 128 : (p.n + 255) / 256;
   kernel<<<p.tiles_m * p.tiles_n, kThreads, bytes, stream>>>(p);
   return hipGetLastError();
 }
@@ -722,6 +736,7 @@ hipError_t launch_gemm(GemmParams &p, hipStream_t stream) {
     // whose nine two-stage steps each wait out a trip to memory)
     const uint64_t small_pair = (uint64_t)((p.m + 127) / 128) * ((p.n + 127) / 128);
     if (small_pair <= (uint64_t)cus) return launch_tile<1, 2, true, 4>(p, stream);
+    if (p.k <= (1u << 22)) return launch_phased<true>(p, stream);
     return launch_tile<2, 2, true>(p, stream);
   }
   // Tall (256 x 128) or wide (128 x 256) tiles, whichever pads less; the tall one when
@@ -733,7 +748,7 @@ hipError_t launch_gemm(GemmParams &p, hipStream_t stream) {
   // 256 x 256 once even the better of those would begin a second round (offsets from a tile's first row are 32 bits there): us,
   // 256 x 128 or 128 x 256 / 256 x 256: 2048 x 2048 x 6144 82 / 63, 1024 x 4096 x 14336 154 / 118, 1430 x 576 x 5632 30.5 / 22.9;
   // where they are one round 1134 x 2112 x 6720 45 / 55, 541 x 576 x 11840 20 / 23.
-  if (std::min(tall, wide) > (uint64_t)cus && p.k <= (1u << 22)) return launch_phased(p, stream);
+  if (std::min(tall, wide) > (uint64_t)cus && p.k <= (1u << 22)) return launch_phased<false>(p, stream);
   if (std::min(tall, wide) * 8 >= (uint64_t)cus * 7)
     return tall <= wide ? launch_tile<2, 2, false>(p, stream) : launch_tile<1, 4, false>(p, stream);
   // 128 x 128 tiles have steps shorter than a trip to memory.  With two stages they fit a CU

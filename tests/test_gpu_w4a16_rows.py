@@ -260,3 +260,8 @@ def test_tiles_of_256_keep_infinities_in_their_row(runtime):
     out = run_linear(runtime, x, packed, scale)
     assert not np.isfinite(out[m - 1]).any()
     np.testing.assert_array_equal(out[:m - 1], expected.astype(np.float16)[:m - 1])
+
+
+@pytest.mark.parametrize("m,n,k", [(4000, 2100, 64), (4001, 2049, 128), (2050, 3701, 192), (2300, 3704, 320), (2049, 3713, 576)])
+def test_pair_tiles_of_256(runtime, m, n, k):
+    test_small_pair_tiles(runtime, m, n, k)
