@@ -150,15 +150,25 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(SsmArgs a, SsmWorkspace w
     float sum[kConvTokens];
 #pragma unroll
     for (int i = 0; i < kConvTokens; ++i) sum[i] = bias;
-    // the input of token t (negative: before the step)
-    auto at = [&](int t) {
-      if (t >= 0) return t < (int)a.m ? to_f32(input[(size_t)t * ld]) : 0.0f;
-      return (int64_t)position + t >= 0 ? ring[(size_t)((position + t) % a.taps) * channels] : 0.0f;
-    };
+    // the input of a token before the step, and of any
+    auto before = [&](int t) { return (int64_t)position + t >= 0 ? ring[(size_t)((position + t) % a.taps) * channels] : 0.0f; };
+    auto at = [&](int t) { return t < 0 ? before(t) : t < (int)a.m ? to_f32(input[(size_t)t * ld]) : 0.0f; };
     if (TAPS > 0) {
-      float window[kConvTokens + TAPS - 1];
+      // All are requested, at tokens of the step, before the first is used: under a test each, one after the other, 2048 tokens
+      // of 4352 channels took 24.4 us for 15.3.
+      constexpr int BEFORE = TAPS > 0 ? TAPS - 1 : 0;
+      static_assert(BEFORE <= kConvTokens, "only the first tokens of a step reach behind it");
+      const int last = (int)a.m - 1;
+      T raw[kConvTokens + BEFORE];
 #pragma unroll
-      for (int i = 0; i < kConvTokens + TAPS - 1; ++i) window[i] = at((int)t0 + i - (TAPS - 1));
+      for (int i = 0; i < kConvTokens + BEFORE; ++i) raw[i] = input[(size_t)(uint32_t)min(max((int)t0 + i - BEFORE, 0), last) * ld];
+      float window[kConvTokens + BEFORE];
+#pragma unroll
+      for (int i = 0; i < kConvTokens + BEFORE; ++i) window[i] = (int)t0 + i - BEFORE <= last ? to_f32(raw[i]) : 0.0f;
+      if (t0 == 0) {
+#pragma unroll
+        for (int i = 0; i < BEFORE; ++i) window[i] = before(i - BEFORE);
+      }
 #pragma unroll
       for (int tap = 0; tap < TAPS; ++tap) {
         const float weight = bf16_at(a.conv, (size_t)channel * TAPS + tap);
@@ -173,7 +183,7 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(SsmArgs a, SsmWorkspace w
       }
     }
 #pragma unroll
-    for (int i = 0; i < kConvTokens; ++i) out[i] = t0 + i < a.m ? (T)silu_f32(sum[i]) : (T)0.0f;
+    for (int i = 0; i < kConvTokens; ++i) out[i] = t0 + i < a.m ? (T)silu_f32<sizeof(T) == 2>(sum[i]) : (T)0.0f;
   } else {
 #pragma unroll
     for (int i = 0; i < kConvTokens; ++i) out[i] = (T)0.0f;
