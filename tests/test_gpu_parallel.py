@@ -409,3 +409,13 @@ def test_entries_refuse_what_does_not_fit(runtime, mixed):
         with pytest.raises(LlmoptError):
             batch.dispatch_all(DispatchList([(name, buffers, grown.tobytes(), grid, group)]))
             batch.commit()
+
+
+# heads of 64, 128 and 256 values in bfloat16: several rows of several vectors a wave, all, some or none of a head turned, a
+# number of vectors and of rows that leaves lanes and waves without one
+@pytest.mark.parametrize("heads,kv_heads,dim,rotated,count", [
+    (4, 2, 64, 64, 75), (6, 2, 64, 32, 41), (3, 1, 64, 48, 3), (4, 1, 128, 128, 30), (3, 3, 128, 16, 77), (1, 1, 256, 256, 22),
+    (2, 1, 256, 224, 18), (5, 1, 128, 0, 21)])
+def test_rotation_of_whole_heads(runtime, heads, kv_heads, dim, rotated, count):
+    side = window(heads=heads, kv_heads=kv_heads, dim=dim, vdim=32, size=40, scale=dim ** -0.5, rotated=rotated or 16)
+    check_streams(runtime, config(parallel(left=side if rotated else {**side, "rot": None}, **only("left"))), "bfloat16", count=count)
