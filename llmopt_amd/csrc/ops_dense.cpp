@@ -88,7 +88,7 @@ int rms_logits(llmopt_hip_context *context, const DispatchRecord &record) {
                                           {3, (uint64_t)vocabulary * width * 2},
                                           {4, (uint64_t)rows * vocabulary * 4}}))
     return status;
-  // (The logits of a prompt's one row as a token's: 32768 x 2048 4.9 + 29 us as the norm and a product of padded tiles / 27.)
+  // (The logits of a prompt's one row as a token's: 32768 x 2048 behind a prompt 4.9 + 29 us as norm and padded tiles / 30.)
   if (rows == 1) {
     DenseGemvArgs a = normed_gemv(F32, as_f32(record.buffers[0]), as_bf16(record.buffers[2]), epsilon,
                                   as_bf16(record.buffers[3]), vocabulary, width);

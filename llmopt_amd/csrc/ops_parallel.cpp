@@ -124,7 +124,7 @@ int pending_logits(llmopt_hip_context *context, const DispatchRecord &record) {
     return status;
   const bool single = m == 1 && rows == 1;
   const uint16_t *head = as_bf16(record.buffers[6]);
-  // (A prompt's one row as a token's: 32768 x 2048 4.8 + 36.7 + 4.2 us as norm, padded tiles and cap / 28.)
+  // (A prompt's one row as a token's: 32768 x 2048 behind a prompt 4.8 + 36.7 + 4.2 us as norm, padded tiles and cap / 38.)
   if (rows == 1) {
     DenseGemvArgs a = row_product(F32, p, head, vocabulary, width);
     a.row_index = single ? nullptr : as_u32(record.buffers[4]);
