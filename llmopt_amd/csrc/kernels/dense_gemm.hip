@@ -835,7 +835,15 @@ hipError_t run_registers(const DenseLinearArgs &a, hipStream_t stream) {
 template <int GATED>
 hipError_t pick_routed(const DenseLinearArgs &a, hipStream_t stream) {
   const bool direct = !a.f32 && a.k % kStageK == 0 && a.ldx % 8 == 0;
-  if (a.tile == 128) return direct ? run_turns<128, 128, 5, GATED, true>(a, {0, a.n}, stream) : hipErrorInvalidValue;
+  if (a.tile == 128) {
+    if (!direct) return hipErrorInvalidValue;
+    // In turns while the launch is one round of workgroups at most; beyond, two workgroups in step on a CU fill each other's waits
+    // and the last round.  Whole feed-forward, us, in step / in turns (tokens, width, expert's width): one round 500 x 1024 x 512
+    // 46.7 / 43.9, 2048 x 512 x 256 41.3 / 39.6; more 3001 x 1024 x 512 100 / 118, 2048 x 1024 x 512 84 / 90.
+    const uint64_t most = (uint64_t)a.tiles * ((a.n + (GATED ? 63 : 127)) / (GATED ? 64 : 128));
+    if (most <= (uint64_t)device_compute_units()) return run_turns<128, 128, 5, GATED, true>(a, {0, a.n}, stream);
+    return run_direct<128, 128, 2, 4, 2, GATED, true>(a, {0, a.n}, stream);
+  }
   if (direct) return run_direct<64, 128, 2, 4, 3, GATED, true>(a, {0, a.n}, stream);
   return a.f32 ? run_registers<float, 64, GATED, true>(a, stream) : run_registers<__bf16, 64, GATED, true>(a, stream);
 }

@@ -150,8 +150,9 @@ def test_staggered_tiles_of_pairs(runtime, m, n, k):
     test_gated_tiles(runtime, m, k, n // 2)
 
 
-# tiles of 128 rows of an expert: 1 to 5 stages and 16, experts with a remainder
-@pytest.mark.parametrize("m,width,ff", [(200, 64, 128), (400, 128, 64), (333, 192, 320), (250, 256, 192), (1024, 1024, 320)])
+# tiles of 128 rows of an expert, in turns and (more than a round of them) in step: 1 to 5 stages and 16, experts with a remainder
+@pytest.mark.parametrize("m,width,ff", [(200, 64, 128), (400, 128, 64), (333, 192, 320), (250, 256, 192), (1024, 1024, 320),
+                                        (1500, 512, 1600), (1024, 2048, 64)])
 def test_routed_tiles(runtime, m, width, ff):
     rng = np.random.default_rng(m + ff)
     experts, top = 5, 2
