@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void ssm_conv_kernel(SsmArgs a, SsmWorkspace w
       }
     }
 #pragma unroll
-    for (int i = 0; i < kConvTokens; ++i) out[i] = t0 + i < a.m ? (T)silu_f32<sizeof(T) == 2>(sum[i]) : (T)0.0f;
+    for (int i = 0; i < kConvTokens; ++i) out[i] = t0 + i < a.m ? (T)silu_f32(sum[i]) : (T)0.0f;
   } else {
 #pragma unroll
     for (int i = 0; i < kConvTokens; ++i) out[i] = (T)0.0f;

@@ -395,6 +395,35 @@ def test_sizes_of_a_real_layer(runtime, dtype):
     assert_close(logits, expected[[0, 1, 255, 256, 329]], dtype)
 
 
+@pytest.mark.parametrize("taps", [4, 3])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_convolution_whose_reciprocal_is_no_normal_number(runtime, dtype, taps):
+    """silu(-88) = -88 / (1 + e^88) = -5.3e-37 in front of a skip gain of 1e36: the quotient is a normal float32, the reciprocal
+    of its denominator is not.  bfloat16 rounds the input, the gain and the output (half a unit, 2^-9, each)."""
+    import struct
+    from llmopt_amd.safetensors_file import from_bfloat16, to_bfloat16
+    m, heads, vdim, state = 20, 2, 8, 16
+    inner = heads * vdim
+    channels = inner + 2 * state
+    bf16 = lambda v: to_bfloat16(np.asarray(v, dtype=np.float32))
+    put = runtime.buffer_of_bytes
+    projected = np.zeros((m, inner + channels), dtype=np.float32)
+    projected[:, inner:2 * inner] = -88.0  # (b and c stay zero: no recurrence)
+    conv = np.zeros((channels, taps), dtype=np.float32)
+    conv[:, -1] = 1.0
+    f32 = dtype == "float32"
+    out = put(np.full((m, inner), np.nan, dtype=np.float32) if f32 else np.full((m, inner), 0x7fc0, dtype=np.uint16))
+    zeros = lambda *shape: np.zeros(shape, dtype=np.float32)
+    runtime.dispatch("llmopt_ssm_mix_f32" if f32 else "llmopt_ssm_mix_bf16",
+                     [put(np.zeros(2, dtype=np.uint32)), put(projected if f32 else bf16(projected)), put(zeros(m, heads)),
+                      put(bf16(conv)), put(bf16(zeros(channels))), put(bf16(zeros(heads))), put(bf16(zeros(heads))),
+                      put(bf16(np.full(heads, 1e36))), put(zeros(taps, channels)), put(zeros(heads, vdim, state)), out],
+                     struct.pack("<7I", m, heads, vdim, 1, state, taps, 1), (1, 1, 1), (256, 1, 1))
+    expected = -88.0 / (1.0 + np.exp(88.0)) * float(from_bfloat16(bf16([1e36]))[0])
+    got = (out.numpy(np.float32, (m, inner)) if f32 else from_bfloat16(out.numpy(np.uint16)).reshape(m, inner)).astype(np.float64)
+    assert np.all(np.abs(got - expected) <= 3 * 2.0 ** -9 * abs(expected))
+
+
 # the router inside the launch of the experts (up to twenty rows with the shared expert's gate, whole pieces, up to 4096
 # values) and in a launch of its own
 @pytest.mark.parametrize("width,experts,top,ff,shared", [
