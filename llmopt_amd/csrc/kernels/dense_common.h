@@ -121,21 +121,12 @@ __device__ __forceinline__ bf16x8 convert_frag<__bf16, bf16x8>(const bf16x8 &fro
   return from;
 }
 
-// QUICK: by the hardware's reciprocal (one unit in the last place), for results that are rounded to bfloat16 next; a division
-// is ten instructions.
-template <bool QUICK = false>
-__device__ __forceinline__ float quotient(float a, float b) {
-  return QUICK ? a * __builtin_amdgcn_rcpf(b) : a / b;
-}
-template <bool QUICK = false>
-__device__ __forceinline__ float sigmoid_f32(float z) { return quotient<QUICK>(1.0f, 1.0f + __expf(-z)); }
-template <bool QUICK = false>
-__device__ __forceinline__ float silu_f32(float z) { return quotient<QUICK>(z, 1.0f + __expf(-z)); }
+__device__ __forceinline__ float sigmoid_f32(float z) { return 1.0f / (1.0f + __expf(-z)); }
+__device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + __expf(-z)); }
 // tanh through one exponential; |error| of a few 2^-24
-template <bool QUICK = false>
 __device__ __forceinline__ float tanh_f32(float z) {
   const float e = __expf(2.0f * fabsf(z));
-  return copysignf(1.0f - quotient<QUICK>(2.0f, e + 1.0f), z);
+  return copysignf(1.0f - 2.0f / (e + 1.0f), z);
 }
 __device__ __forceinline__ float softplus_f32(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 
@@ -148,20 +139,18 @@ __device__ __forceinline__ float softplus_fast_f32(float z) {
 
 // Activation of a gated feed-forward.
 enum GateActivation : uint32_t { kGateSilu = 0, kGateGeluTanh = 1, kGateClamped = 2 };
-template <bool QUICK = false>
 __device__ __forceinline__ float gate_activation(float z, uint32_t kind) {
-  if (kind == kGateGeluTanh) return 0.5f * z * (1.0f + tanh_f32<QUICK>(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-  return silu_f32<QUICK>(z);
+  if (kind == kGateGeluTanh) return 0.5f * z * (1.0f + tanh_f32(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+  return silu_f32(z);
 }
 
 // act(gate) up; clamped: both halves limited, a steeper sigmoid, and one more than the up half.
-template <bool QUICK = false>
 __device__ __forceinline__ float gated_value(float gate, float up, uint32_t kind, float limit) {
   if (kind == kGateClamped) {
     const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
-    return g * sigmoid_f32<QUICK>(1.702f * g) * (u + 1.0f);
+    return g * sigmoid_f32(1.702f * g) * (u + 1.0f);
   }
-  return gate_activation<QUICK>(gate, kind) * up;
+  return gate_activation(gate, kind) * up;
 }
 __device__ __forceinline__ float soft_capped(float z, float cap) { return cap > 0.0f ? cap * tanh_f32(z / cap) : z; }
 

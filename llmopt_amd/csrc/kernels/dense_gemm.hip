@@ -159,10 +159,10 @@ __device__ __forceinline__ bool place_tile(const GemmParams &p, TilePlace &t) {
 // GATED of the kernels: 0 no, 1 an activation of the gate alone, 2 the clamped pair.  (Apart: the epilogue's code is
 // repeated for every value of a tile, and an activation more costs the large tiles a few percent.)
 constexpr int kOneSided = 1, kClampedPair = 2;
-template <int GATED, bool QUICK = false>
+template <int GATED>
 __device__ __forceinline__ float gated(const DenseLinearArgs &a, float gate, float up) {
-  if (GATED == kClampedPair) return gated_value<QUICK>(gate, up, kGateClamped, a.limit);
-  return gate_activation<QUICK>(gate, a.activation) * up;
+  if (GATED == kClampedPair) return gated_value(gate, up, kGateClamped, a.limit);
+  return gate_activation(gate, a.activation) * up;
 }
 
 // A wave's accumulators: MT x NT groups of 16 x 16 from row `row_offset` and tile column `column_offset` on.
@@ -347,7 +347,7 @@ __device__ __forceinline__ void emit_rows(const DenseLinearArgs &a, const f32x4 
       f32x4 v;
       if (GATED) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = gated<GATED, true>(a, acc[i][2 * j][e], acc[i][2 * j + 1][e]);
+        for (int e = 0; e < 4; ++e) v[e] = gated<GATED>(a, acc[i][2 * j][e], acc[i][2 * j + 1][e]);
       } else {
         v = acc[i][j];
         if (a.epilogue == DenseEpilogue::kQkv && r_in_tile < m_rows) mix_values(a, r, c, v);

@@ -65,6 +65,23 @@ def test_gated_tiles(runtime, m, width, ff):
     assert np.sqrt(np.mean(error ** 2)) <= 4 * 2.0 ** -9 * np.sqrt(np.mean(expected ** 2))
 
 
+def test_gate_whose_reciprocal_is_no_normal_number(runtime):
+    """silu(-88) = -88 / (1 + e^88) = -5.3e-37, whose quotient is one and whose reciprocal, 6e-39, is less than the smallest normal
+    float32.  An up half of 1e36 shows it; bfloat16 rounds gate, up, product and row, half a unit (2^-9) each, and e^88 is good to
+    88 log2(e) 2^-24 ln(2) < 2^-17."""
+    m, width = 40, 64
+    column = np.zeros((width, width), dtype=np.float32)
+    column[:, 0] = 1.0
+    put, bf16 = runtime.buffer_of_bytes, lambda v: to_bfloat16(v.astype(np.float32))
+    norm, gate, up, down = bf16(np.ones(width)), bf16(-88.0 * column), bf16(1e36 * column), bf16(np.eye(width))
+    out = put(np.ones((m, width), dtype=np.float32))
+    runtime.dispatch("llmopt_rms_gated_ffn_add_bf16", [out] + [put(a) for a in (norm, gate, up, down)],
+                     u32s(m, width, width) + struct.pack("<f", 1e-9) + u32s(0), *GRID)
+    expected = -88.0 / (1.0 + np.exp(88.0)) * float(from_bfloat16(bf16(np.array([1e36])))[0])
+    got = out.numpy(np.float32, (m, width)).astype(np.float64) - 1.0
+    assert np.all(np.abs(got - expected) <= 4 * 2.0 ** -9 * abs(expected))
+
+
 ROW_SIZES = [(33, 701, 64), (500, 2000, 64), (1023, 2047, 64), (2047, 2045, 64), (1000, 5551, 64), (1000, 6357, 64),
              (1500, 6001, 64), (2999, 2046, 64), (3000, 9503, 64), (1499, 2047, 256), (1345, 8857, 256), (1413, 8123, 256),
              (195, 8311, 2560), (203, 8125, 2304)]
