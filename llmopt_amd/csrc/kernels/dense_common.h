@@ -137,6 +137,10 @@ __device__ __forceinline__ float softplus_fast_f32(float z) {
   return fmaxf(z, 0.0f) + (u == 1.0f ? e : __logf(u) * e * __builtin_amdgcn_rcpf(u - 1.0f));
 }
 
+// A router's logit as the selection takes it: NaN as infinity, whose weight is NaN again.  Comparisons that a NaN fails gave rank
+// 0 to several experts, and the indices of the ranks that none had then, which address the experts' weights, were never written.
+__device__ __forceinline__ float expert_logit(float v) { return v == v ? v : __builtin_inff(); }
+
 // Activation of a gated feed-forward.
 enum GateActivation : uint32_t { kGateSilu = 0, kGateGeluTanh = 1, kGateClamped = 2 };
 __device__ __forceinline__ float gate_activation(float z, uint32_t kind) {

@@ -414,7 +414,7 @@ hipError_t pick_gemv(const DenseGemvArgs &a, hipStream_t stream) {
 template <int THREADS>
 __device__ __forceinline__ void select_experts(const float *logits, uint32_t experts, uint32_t top, float *z,
                                                uint32_t *ids, float *weights) {
-  for (uint32_t e = threadIdx.x; e < experts; e += THREADS) z[e] = logits[e];
+  for (uint32_t e = threadIdx.x; e < experts; e += THREADS) z[e] = expert_logit(logits[e]);
   __syncthreads();
   for (uint32_t e = threadIdx.x; e < experts; e += THREADS) {
     const float mine = z[e];

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256) void route_select_kernel(RoutePlan p) {
   float *z = lds + wave * (p.experts + p.top), *chosen = z + p.experts;
   const bool live = t < p.m;
   if (live)
-    for (uint32_t e = lane; e < p.experts; e += 64) z[e] = p.logits[(size_t)t * p.ld_logits + e];
+    for (uint32_t e = lane; e < p.experts; e += 64) z[e] = expert_logit(p.logits[(size_t)t * p.ld_logits + e]);
   __syncthreads();
   if (live)
     for (uint32_t e = lane; e < p.experts; e += 64) {

@@ -455,3 +455,31 @@ def test_experts_of_one_token_and_their_router(runtime, width, experts, top, ff,
                          struct.pack("<6IfI", 1, width, experts, top, ff, shared, 1e-6, 0), (1, 1, 1), (256, 1, 1))
         got = stream.numpy(np.float32).astype(np.float64) - x
         assert np.linalg.norm(got - add) <= 1e-5 * np.linalg.norm(add) + 2.0 ** -24 * np.linalg.norm(x)
+
+
+@pytest.mark.parametrize("m,width,experts,top,bad", [(1, 64, 3, 2, 0), (1, 1024, 20, 20, 0), (1, 1024, 33, 4, 0), (1, 4104, 4, 3, 0),
+                                                     (5, 64, 3, 2, 4), (300, 64, 5, 3, 7)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_router_logits_that_are_no_numbers(runtime, dtype, m, width, experts, top, bad):
+    """A token whose logits are NaN gets a row of NaN out of experts that exist; the other tokens' rows do not change."""
+    import struct
+    from llmopt_amd.safetensors_file import to_bfloat16
+    rng, ff, put = np.random.default_rng(width + experts), 64, runtime.buffer_of_bytes
+    shapes = [(width,), (experts, width), (experts, ff, width), (experts, ff, width), (experts, width, ff)]
+    weights = [put(to_bfloat16((rng.standard_normal(s) * (1.0 if len(s) == 1 else s[-1] ** -0.5)).astype(np.float32))) for s in shapes]
+    none, name = put(np.zeros(width, dtype=np.uint16)), "llmopt_rms_routed_ffn_add_" + ("f32" if dtype == "float32" else "bf16")
+    x = rng.standard_normal((m, width)).astype(np.float32)
+
+    def run(rows):
+        stream = put(rows)
+        runtime.dispatch(name, [stream] + weights + [none] * 3, struct.pack("<6IfI", m, width, experts, top, ff, 0, 1e-6, 0),
+                         (1, 1, 1), (256, 1, 1))
+        return stream.numpy(np.float32, (m, width))
+
+    good, spoiled = run(x), x.copy()
+    spoiled[bad, 3] = np.nan
+    got = run(spoiled)
+    assert np.isnan(got[bad]).all() and np.isfinite(good).all()
+    others = np.arange(m) != bad
+    # (another row's place in a tile may change, the order of its sums does not)
+    assert np.array_equal(got[others], good[others])
