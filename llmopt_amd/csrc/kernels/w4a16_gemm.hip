@@ -522,7 +522,8 @@ __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
                    : "memory");
   };
   // A thread's weights of a step: half of a column's 64.  (As in w4a16_gemm_kernel, nothing may copy a set between its
-  // request and its wait.)
+  // request and its wait, at the border of the odd tail step's copy of the body least of all: a host test follows every
+  // load through the listing.)
   struct Fetched {
     u32x4_t w;
     uint32_t s;  // fp16 bits in the low half
