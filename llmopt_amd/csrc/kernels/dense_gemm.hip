@@ -503,6 +503,7 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParam
 template <int GATED>
 __global__ __launch_bounds__(512) void dense_gemm_phased_kernel(GemmParams p) {
   constexpr int BM = 256, BN = 256, COLUMNS = GATED ? BN / 2 : BN, HALF = 16384, STAGE = 4 * HALF;
+  static_assert(8 * 16 * (4 * 16 + 8) * 2 <= 2 * STAGE, "the waves' output rows fit");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const DenseLinearArgs &a = p.a;
   TilePlace place;
@@ -655,16 +656,18 @@ __global__ __launch_bounds__(512) void dense_gemm_phased_kernel(GemmParams p) {
 // the stages of 64 K values in turn, each for the whole tile; while one multiplies, the other one reads its operands, and
 // their sums meet in LDS at the end.  A wave's tile is twice as large as with eight waves on a stage, so that the operands
 // of a product come to two thirds of the LDS reads, and a stage is two barriers for a group whose products last between them.
-// A stage's place is free behind the barrier that ends its reads and is requested in the next turn, by the other group:
-// an odd STAGES requests a group's own stages, an even one the other group's.
+// A stage's place is free behind the barrier that ends its reads and is requested in the next turn, by the other group: with an
+// odd number of them for a stage of its own, which it waits for behind its products.
 // us, eight waves in step / in turns: 128 x 128 tiles 2048 x 2048 x 4096 41 / 33, x 8192 83 / 60 (1.15 PFLOP/s); 192 x 128
 // 3001 x 2048 x 4096 54 / 44, x 8192 103 / 80 (1.26 PFLOP/s).
 template <int BM, int BN, int STAGES, int GATED, bool ROUTED>
 __global__ __launch_bounds__(512) void dense_gemm_turns_kernel(GemmParams p) {
   constexpr int COLUMNS = GATED ? BN / 2 : BN, MT = BM / 32, NT = BN / 32, ROWS = BM + BN;
   constexpr int COPIES = ROWS / 32;  // 8-row copies of a wave and step
-  constexpr int BEHIND = STAGES % 2 ? (STAGES - 3) / 2 * COPIES : COPIES;  // copies that may be under way when the next step has landed
-  static_assert(MT % 2 == 0 && (!GATED || NT % 2 == 0) && ROWS % 32 == 0 && STAGES >= 3, "tile");
+  constexpr int BEHIND = (STAGES - 3) / 2 * COPIES;  // copies that may be under way when the next step has landed
+  constexpr int RING = STAGES * ROWS * 128, PART = MT / 2 * NT * 1024;  // bytes: the stages; a wave's half of its sums
+  static_assert(MT % 2 == 0 && (!GATED || NT % 2 == 0) && ROWS % 32 == 0 && STAGES >= 3 && STAGES % 2 == 1, "tile");
+  static_assert(RING <= 160 * 1024 && 8 * PART <= RING && 8 * 16 * (NT * 16 + 8) * 2 <= RING, "the ring, the sums and the output rows fit");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const DenseLinearArgs &a = p.a;
   TilePlace place;
@@ -710,7 +713,7 @@ __global__ __launch_bounds__(512) void dense_gemm_turns_kernel(GemmParams p) {
   const int fr = lane & 15, quad = lane >> 4, twist = (fr >> 1) & 7;
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
-    if (s < steps && ((s - (STAGES - 1)) & 1) == group) request(s);
+    if (s < steps && (s & 1) == group) request(s);
   if (steps >= STAGES - 1) copies_landed<BEHIND>();
   else copies_landed<0>();
   meet();
@@ -729,10 +732,6 @@ __global__ __launch_bounds__(512) void dense_gemm_turns_kernel(GemmParams p) {
     }
     const bool more = s + STAGES - 1 < steps;
     if (more) request(s + STAGES - 1);
-    if (STAGES % 2 == 0) {
-      if (more) copies_landed<BEHIND>();
-      else copies_landed<0>();
-    }
     lds_read();  // read: the slot is free behind the barrier
     meet();
     __builtin_amdgcn_s_setprio(1);
@@ -746,10 +745,8 @@ __global__ __launch_bounds__(512) void dense_gemm_turns_kernel(GemmParams p) {
           sum = mma(fw[j][kk], fa[i][kk], sum);
         }
     __builtin_amdgcn_s_setprio(0);
-    if (STAGES % 2 == 1) {
-      if (more) copies_landed<BEHIND>();
-      else copies_landed<0>();
-    }
+    if (more) copies_landed<BEHIND>();
+    else copies_landed<0>();
     meet();
   }
   if ((steps & 1) == group) meet();
@@ -764,7 +761,6 @@ __global__ __launch_bounds__(512) void dense_gemm_turns_kernel(GemmParams p) {
         acc[1][i][j] = v;
       }
   }
-  constexpr int PART = MT / 2 * NT * 1024;
   char *mine = lds + wave * PART + lane * 16, *other = lds + (wave ^ 4) * PART + lane * 16;
 #pragma unroll
   for (int i = 0; i < MT / 2; ++i)
