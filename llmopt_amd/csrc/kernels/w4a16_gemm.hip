@@ -24,6 +24,7 @@
 #include "kernels_internal.h"
 #include "staggered.h"
 #include "w4_common.h"
+#include "w4a16_gemm_rule.h"
 
 namespace llmopt {
 namespace {
@@ -490,6 +491,7 @@ hipError_t launch_tile(GemmParams &p, hipStream_t stream, uint32_t splits = 1) {
 template <bool DUAL>
 __global__ __launch_bounds__(512) void w4a16_gemm_phased_kernel(GemmParams p) {
   constexpr int HALF = 16384, STAGE = 4 * HALF;  // halves of a stage: rows 0, rows 1, columns 0, columns 1
+  static_assert(8 * 16 * ((DUAL ? 32 : 64) + 8) * 2 <= 2 * STAGE, "the waves' output rows fit");
   extern __shared__ __attribute__((aligned(16))) unsigned char gemm_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -730,40 +732,23 @@ uint32_t gemm_k_splits(uint32_t m, uint32_t n, uint32_t k) {
 
 template <bool DUAL>
 hipError_t launch_gemm(GemmParams &p, hipStream_t stream) {
-  const int cus = device_compute_units();
-  if (DUAL) {
-    // 256 x 128, two accumulator sets; 128 x 128 with four activation stages when even those tiles
-    // leave CUs without one (the decode model's 576 -> 1536 pair at 2048 rows: 96 tiles of 256 x 128,
-    // whose nine two-stage steps each wait out a trip to memory)
-    const uint64_t small_pair = (uint64_t)((p.m + 127) / 128) * ((p.n + 127) / 128);
-    if (small_pair <= (uint64_t)cus) return launch_tile<1, 2, true, 4>(p, stream);
-    if (p.k <= (1u << 22)) return launch_phased<true>(p, stream);
-    return launch_tile<2, 2, true>(p, stream);
+  const uint32_t cus = (uint32_t)device_compute_units();
+  if constexpr (DUAL) {
+    return w4_gemm_pair_tile(p.m, p.n, p.k, cus) == W4GemmTile::k256x256 ? launch_phased<true>(p, stream)
+                                                                         : launch_tile<1, 2, true, 4>(p, stream);
+  } else {
+    const W4GemmTile tile = w4_gemm_tile(p.m, p.n, p.k, cus);
+    if (tile == W4GemmTile::k256x256) return launch_phased<false>(p, stream);
+    if (tile == W4GemmTile::k256x128) return launch_tile<2, 2, false>(p, stream);
+    if (tile == W4GemmTile::k128x256) return launch_tile<1, 4, false>(p, stream);
+    // Fewer tiles than half the CUs: K is split over workgroups as well, so that every CU holds a
+    // tile (128 tiles at 512 x 4096 x 4096 left half the device idle).
+    const uint32_t splits = gemm_k_splits(p.m, p.n, p.k);
+    if (splits > 1 && p.partials != nullptr && p.counters != nullptr)
+      return launch_tile<1, 2, false, 4, true>(p, stream, splits);
+    if (tile == W4GemmTile::k128x128Deep) return launch_tile<1, 2, false, 4>(p, stream);
+    return launch_tile<1, 2, false>(p, stream);
   }
-  // Tall (256 x 128) or wide (128 x 256) tiles, whichever pads less; the tall one when
-  // they tie (its waves read 16 operand vectors from LDS per 16 MFMAs, the wide one's 20: 76.5
-  // against 80 us at 512 x 14336, 81.7 against 86.3 at 2048 x 4096).  Also when a few CUs stay
-  // without a tile: 224 such tiles beat 448 of 128 x 128, two on most CUs.
-  const uint64_t tall = (uint64_t)((p.m + 255) / 256) * ((p.n + 127) / 128);
-  const uint64_t wide = (uint64_t)((p.m + 127) / 128) * ((p.n + 255) / 256);
-  // 256 x 256 once even the better of those would begin a second round (offsets from a tile's first row are 32 bits there): us,
-  // 256 x 128 or 128 x 256 / 256 x 256: 2048 x 2048 x 6144 82 / 63, 1024 x 4096 x 14336 154 / 118, 1430 x 576 x 5632 30.5 / 22.9;
-  // where they are one round 1134 x 2112 x 6720 45 / 55, 541 x 576 x 11840 20 / 23.
-  if (std::min(tall, wide) > (uint64_t)cus && p.k <= (1u << 22)) return launch_phased<false>(p, stream);
-  if (std::min(tall, wide) * 8 >= (uint64_t)cus * 7)
-    return tall <= wide ? launch_tile<2, 2, false>(p, stream) : launch_tile<1, 4, false>(p, stream);
-  // 128 x 128 tiles have steps shorter than a trip to memory.  With two stages they fit a CU
-  // twice, which covers the loads; when there is at most one tile per CU anyway, four
-  // activation stages do (measured 58 -> 49 us at 512 x 4096 x 4096, and nothing for the 128 x 256
-  // tiles, which stay with two).
-  const uint64_t small = (uint64_t)((p.m + 127) / 128) * ((p.n + 127) / 128);
-  // Fewer tiles than half the CUs: K is split over workgroups as well, so that every CU holds a
-  // tile (128 tiles at 512 x 4096 x 4096 left half the device idle).
-  const uint32_t splits = gemm_k_splits(p.m, p.n, p.k);
-  if (splits > 1 && p.partials != nullptr && p.counters != nullptr)
-    return launch_tile<1, 2, false, 4, true>(p, stream, splits);
-  if (small <= (uint64_t)cus) return launch_tile<1, 2, false, 4>(p, stream);
-  return launch_tile<1, 2, false>(p, stream);
 }
 
 }  // namespace

@@ -240,11 +240,16 @@ def test_pairs_of_rows_that_are_normalised_in_the_tile(runtime, m, n, k):
     assert np.isfinite(one.numpy(np.float16)).all()
 
 
-# 256 x 256 tiles: one to nine K steps, remainders of rows and columns, whole and odd rows of outputs and addends
+# 256 x 256 tiles (test_tile_rules.py checks which sizes take them): one to nine K steps, remainders of rows and columns, whole and odd rows of outputs and addends
 @pytest.mark.parametrize("m,n,k,addend", [(4000, 4100, 64, "none"), (4001, 4097, 128, "bias"), (2050, 7301, 192, "residual"),
                                           (2300, 7304, 256, "residual"), (4096, 4096, 320, "bias"), (2049, 7425, 576, "none"),
-                                          (1290, 5637, 192, "bias")])
+                                          (1290, 5889, 192, "bias")])
 def test_tiles_of_256(runtime, m, n, k, addend):
+    test_small_tiles(runtime, m, n, k, addend)
+
+
+@pytest.mark.parametrize("m,n,k,addend", [(1290, 5637, 192, "bias")])
+def test_tiles_of_128_by_256(runtime, m, n, k, addend):
     test_small_tiles(runtime, m, n, k, addend)
 
 

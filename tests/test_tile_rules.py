@@ -14,6 +14,7 @@ SOURCE = """
 #include "delta_rule.h"
 #include "dense_attention_rule.h"
 #include "dense_tile_rule.h"
+#include "w4a16_gemm_rule.h"
 #include "w4a16_rows_rule.h"
 using namespace llmopt;
 extern "C" {
@@ -26,6 +27,8 @@ int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, ui
 int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
   return three_delta_workgroups((tokens + 63) / 64 * heads, cus);
 }
+int large_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)w4_gemm_tile(m, n, k, cus); }
+int large_pair_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)w4_gemm_pair_tile(m, n, k, cus); }
 int product_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_tile(m, n, k, cus); }
 int staggered_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_product_tile(m, n, k, cus); }
 int split_columns(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)dense_column_split(m, n, k, cus).columns; }
@@ -45,6 +48,7 @@ int qkv_tile(uint32_t m, uint32_t q, uint32_t kv, uint32_t k, uint32_t cus) {
 """
 DENSE = ("256x256", "128x128", "192x128", "128x192", "192x128 eight waves", "128x128 eight waves", "64x128 eight waves", "64x64",
          "32x64", "64x128")
+LARGE = ("128x128", "128x128 deep", "256x128", "128x256", "256x256")
 NONE, K32X32, K32X64, K32X64_DEEP, K32X64_LONG, K64X64, K64X128 = range(7)
 
 
@@ -186,3 +190,28 @@ def test_rows_normalised_in_the_tile(rules):
     assert not rules.normed_pair(700, 1536, 576, CUS)       # 96 rows
     assert not rules.normed_pair(100, 1000, 832, CUS)       # thirteen groups
     assert not rules.normed_qkv(1300, 576, 192, 576, CUS)   # a second round
+
+
+def test_gpu_tests_reach_the_256_tiles_of_w4a16(rules):
+    """Products and pairs that the small tiles and the GEMV's row groups leave alone, by more than a round of the middle tiles."""
+    tests = test_gpu_w4a16_rows
+    for m, n, k, _ in sizes(tests.test_tiles_of_256, "m,n,k,addend"):
+        assert rules.linear_tile(m, n, k, CUS) == NONE and LARGE[rules.large_tile(m, n, k, CUS)] == "256x256", (m, n, k)
+    for m, n, k, _ in sizes(tests.test_tiles_of_128_by_256, "m,n,k,addend"):
+        assert rules.linear_tile(m, n, k, CUS) == NONE and LARGE[rules.large_tile(m, n, k, CUS)] == "128x256", (m, n, k)
+    for m, n, k in sizes(tests.test_pair_tiles_of_256, "m,n,k"):
+        assert rules.gated_tile(m, n, k, CUS) == NONE and LARGE[rules.large_pair_tile(m, n, k, CUS)] == "256x256", (m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k,tile", [(2048, 14336, 4096, "256x256"), (2048, 6144, 2048, "256x256"), (1430, 5632, 576, "256x256"),
+                                        (1134, 6720, 2112, "128x256"), (541, 11840, 576, "128x256"), (512, 14336, 4096, "256x128"),
+                                        (2048, 4096, 4096, "256x128"), (512, 4096, 4096, "128x128 deep"),
+                                        (1600, 3000, 576, "128x128"), (2048, 14336, 1 << 23, "256x128")])
+def test_large_w4a16_tiles(rules, m, n, k, tile):
+    assert LARGE[rules.large_tile(m, n, k, CUS)] == tile
+
+
+@pytest.mark.parametrize("m,n,k,tile", [(2048, 1536, 576, "128x128 deep"), (2048, 14336, 4096, "256x256"), (2049, 2048, 576, "256x256"),
+                                        (2048, 2048, 576, "128x128 deep"), (2048, 14336, 1 << 23, "128x128 deep")])
+def test_large_w4a16_pair_tiles(rules, m, n, k, tile):
+    assert LARGE[rules.large_pair_tile(m, n, k, CUS)] == tile
