@@ -91,7 +91,9 @@ inline float staggered_time(const StaggeredTime &t, uint64_t tiles, uint32_t k, 
 // estimate is 7% less.  The two estimates are fits to launches of their own, and 7% keeps the cases that lose by that few: of
 // 649 sizes beyond 12 us the choice is 4.6% faster than the ten on average and more than 3% slower at 12 (us, ten / this:
 // 2048 x 2048 x 8192 74 / 63, 3001 x 2048 x 8192 100 / 83, 2048 x 6144 x 2048 50.7 / 46.8, 700 x 2048 x 2048 15.6 / 14.0; the
-// other way 2048 x 2048 x 2048 21.9 / 23.0, 1008 x 1088 x 4288 25.9 / 27.8).
+// other way 2048 x 2048 x 2048 21.9 / 23.0, 1008 x 1088 x 4288 25.9 / 27.8).  Rows of outputs that are no whole pieces of
+// eight are stored value by value, which takes 256 x 256 tiles 15 us a round more and the others less: without the 6 us of
+// difference 897 x 11657 x 1024 took 44.7 us for 40.5, 1223 x 9265 x 1408 51.7 for 49.1.
 inline DenseTile dense_product_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus, float *estimate = nullptr) {
   float least = 0.0f;
   DenseTile best = dense_tile(m, columns, k, cus, &least);
@@ -100,7 +102,8 @@ inline DenseTile dense_product_tile(uint32_t m, uint64_t columns, uint32_t k, ui
     for (const StaggeredTime &t : kStaggeredTimes) {
       if (k < 1280 && t.tile != DenseTile::k256x256) continue;
       const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns);
-      const float time = staggered_time(t, tiles, k, cus);
+      float time = staggered_time(t, tiles, k, cus);
+      if (t.tile == DenseTile::k256x256 && columns % 8 != 0) time += 6.0f * (float)((tiles + cus - 1) / cus);
       if (time < least) least = time, best = t.tile;
     }
   }

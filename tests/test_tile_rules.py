@@ -183,6 +183,14 @@ def test_columns_in_two_launches(rules, m, n, k, first):
     assert rules.split_columns(m, n, k, CUS) == first
 
 
+@pytest.mark.parametrize("m,n,k", [(897, 11657, 1024), (1223, 9265, 1408), (2535, 3665, 2688), (1412, 6260, 1024)])
+def test_columns_that_are_no_whole_pieces(rules, m, n, k):
+    """256 x 256 tiles store them more slowly than the others do: not these sizes, which whole pieces give to them."""
+    assert DENSE[rules.staggered_tile(m, n // 8 * 8, k, CUS)] == "256x256"
+    assert rules.staggered_tile(m, n, k, CUS) == rules.product_tile(m, n, k, CUS)
+    assert all(DENSE[rules.staggered_tile(*size, CUS)] == "192x128" for size in test_gpu_dense_tiles.ODD)
+
+
 def test_rows_normalised_in_the_tile(rules):
     """Tiles of 32 rows in one round, and a whole K in LDS."""
     assert all(rules.normed_pair(m, n, k, CUS) for m, n, k in test_gpu_w4a16_rows.NORMED_PAIRS)
