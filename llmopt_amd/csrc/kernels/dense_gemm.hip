@@ -872,10 +872,9 @@ hipError_t pick_gemm(const DenseLinearArgs &a, hipStream_t stream) {
   if (a.k % kStageK != 0 || a.ldx % 8 != 0) return run_registers<__bf16, 32, GATED, false>(a, stream);
   constexpr uint32_t MATRICES = GATED ? 2 : 1;
   const uint32_t cus = (uint32_t)device_compute_units();
-  const DenseSplit split = dense_column_split(a.m, (uint64_t)a.n * MATRICES, a.k, cus);
-  const uint32_t first = (uint32_t)(split.columns / MATRICES);
+  const uint32_t first = (uint32_t)(dense_first_columns(a.m, (uint64_t)a.n * MATRICES, a.k, cus) / MATRICES);
   if (first > 0)
-    if (hipError_t status = run_tile<GATED>(split.tile, a, {0, first}, stream)) return status;
+    if (hipError_t status = run_phased<GATED>(a, {0, first}, stream)) return status;
   return run_tile<GATED>(dense_product_tile(a.m, (uint64_t)(a.n - first) * MATRICES, a.k, cus), a, {first, a.n}, stream);
 }
 

@@ -23,7 +23,7 @@ struct TileTime {
   float start, one, one_k, few, two, two_k, pair, span;
 };
 constexpr TileTime kTileTimes[] = {
-    {256, 256, 0.01f, 14.10f, 24.56f, 1.00f, 0.00f, 0.00f, 0.00f, 0.00f},     // 8 waves, 2 stages, all in step
+    {256, 256, 0.01f, 14.10f, 24.56f, 1.00f, 0.00f, 0.00f, 0.00f, 0.00f},     // (see dense_tile)
     {128, 128, 0.00f, 7.54f, 20.73f, 0.47f, 8.85f, 15.57f, 0.02f, 0.65f},     // 4 waves, 2 stages
     {192, 128, 0.00f, 7.79f, 14.79f, 1.00f, 11.91f, 19.36f, 1.00f, 0.06f},    // 4 waves, 2 stages
     {128, 192, 5.82f, 1.85f, 15.16f, 1.00f, 7.30f, 21.46f, 0.99f, 0.17f},     // 4 waves, 2 stages
@@ -41,6 +41,10 @@ constexpr TileTime kTileTimes[] = {
 // every CU work, which is more than 3% ahead at 29 of them.  An estimate of rounds that go with K alone was 0.8% off, and
 // behind that tile by more than 3% at 72 (us, that tile / such an estimate: 384 x 2816 x 8192 41.0 / 52.0, 700 x 1500 x 8192 41.5
 // / 50.4, 300 x 12288 x 512 12.4 / 13.4: these are back; 384 x 3072 x 8192, with 288 tiles of 64 x 64, 43.6 / 52.5 is not).
+// The row of 256 x 256 tiles is that of all their waves in step.  With half of them a barrier behind, as they run now, a launch is
+// 0.82 to 0.97 of it; from K = 1024 on dense_product_tile asks for their own times, below it this row is the line.  Own times on
+// the scale of the others (1.64, 11.58, 21.16, 0.67) chose 0.1% faster tiles on average at 795 sizes and 3 to 10% slower ones at nine
+// (2283 x 4608 x 448 17.9 / 18.7 us, 918 x 11008 x 192 12.3 / 13.4); this row a slower one than the other nine at none.
 inline DenseTile dense_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus, float *estimate = nullptr) {
   int best = 0;
   float least = 3.4e38f;
@@ -72,71 +76,63 @@ struct StaggeredTime {
   float start, one, one_k, few;
 };
 constexpr StaggeredTime kStaggeredTimes[] = {
-    {DenseTile::k256x256, 256, 256, 2.83f, 7.36f, 20.88f, 0.66f},      // 8 waves, 2 stages
+    {DenseTile::k256x256, 256, 256, 2.83f, 7.36f, 20.88f, 0.66f},      // 8 waves, 2 stages, half of them behind
     {DenseTile::kTurns192x128, 192, 128, 2.04f, 5.54f, 10.32f, 0.73f}, // 2 x 4 waves, 3 stages
     {DenseTile::kTurns128x128, 128, 128, 1.75f, 4.03f, 7.81f, 0.78f},  // 2 x 4 waves, 5 stages
     {DenseTile::kTurns128x192, 128, 192, 3.31f, 4.26f, 10.58f, 0.72f}, // 2 x 4 waves, 3 stages
     {DenseTile::kTurns256x128, 256, 128, 1.98f, 7.19f, 11.84f, 0.69f}, // 2 x 4 waves, 3 stages
     {DenseTile::kTurns128x64, 128, 64, 1.88f, 2.42f, 5.50f, 0.76f},    // 2 x 4 waves, 5 stages
 };
+static_assert(kStaggeredTimes[0].tile == DenseTile::k256x256);
 
-inline float staggered_time(const StaggeredTime &t, uint64_t tiles, uint32_t k, uint32_t cus) {
+// `columns` of the whole product.  Rows of outputs that are no whole pieces of eight are stored value by value, which takes 256 x 256
+// tiles 15 us a round more and the others less: without the 6 us of difference 897 x 11657 x 1024 took 44.7 us for 40.5, 1223 x
+// 9265 x 1408 51.7 for 49.1.
+inline float staggered_time(const StaggeredTime &t, uint64_t tiles, uint64_t columns, uint32_t k, uint32_t cus) {
   const uint64_t rest = tiles % cus;
-  const float one = t.one + t.one_k * (float)k / 1024.0f;
-  return t.start + (float)(tiles / cus) * one + (rest > 0 ? one * (t.few + (1.0f - t.few) * (float)rest / (float)cus) : 0.0f);
+  const float one = t.one + t.one_k * (float)k / 1024.0f, odd = t.tile == DenseTile::k256x256 && columns % 8 != 0 ? 6.0f : 0.0f;
+  return t.start + (float)(tiles / cus) * one + (rest > 0 ? one * (t.few + (1.0f - t.few) * (float)rest / (float)cus) : 0.0f) +
+         odd * (float)((tiles + cus - 1) / cus);
 }
 
-// The tile a product runs on: one of the ten, or from K = 1024 on, in turns from 1280 (below, what the meeting of two groups'
-// sums costs is not made up for: 128 x 128 tiles 0.99 of the ten's time on average, up to 1.16), one of these where its
-// estimate is 7% less.  The two estimates are fits to launches of their own, and 7% keeps the cases that lose by that few: of
-// 649 sizes beyond 12 us the choice is 4.6% faster than the ten on average and more than 3% slower at 12 (us, ten / this:
-// 2048 x 2048 x 8192 74 / 63, 3001 x 2048 x 8192 100 / 83, 2048 x 6144 x 2048 50.7 / 46.8, 700 x 2048 x 2048 15.6 / 14.0; the
-// other way 2048 x 2048 x 2048 21.9 / 23.0, 1008 x 1088 x 4288 25.9 / 27.8).  Rows of outputs that are no whole pieces of
-// eight are stored value by value, which takes 256 x 256 tiles 15 us a round more and the others less: without the 6 us of
-// difference 897 x 11657 x 1024 took 44.7 us for 40.5, 1223 x 9265 x 1408 51.7 for 49.1.
+// The ten's estimates are a fit of their own and come out longer than launches behind each other, which the staggered ones' are of:
+// 1.07 times at the median of 470 sizes beyond 25 us, where the two are compared.  This puts them on one scale.
+constexpr float kInStepScale = 0.93f;
+
+// Where the staggered tiles begin: in turns from 1280 (below, what the meeting of two groups' sums costs is not made up for:
+// 128 x 128 tiles 0.99 of the ten's time on average, up to 1.16).
+inline uint32_t staggered_from_k(DenseTile tile) { return tile == DenseTile::k256x256 ? 1024 : 1280; }
+
+// The tile a product runs on: one of the ten, or from K = 1024 on one of the staggered ones where its estimate is less: 0.96 of the
+// ten's time on average from there on (us, ten / this: 2048 x 2048 x 8192 74 / 63, 2048 x 2048 x 2048 23.2 / 21.1, 3001 x 2048 x 8192
+// 100 / 83, 2048 x 6144 x 2048 51.7 / 48.1, 700 x 2048 x 2048 15.6 / 14.0, 1008 x 1088 x 4288 26.2 / 25.0).
 inline DenseTile dense_product_tile(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus, float *estimate = nullptr) {
   float least = 0.0f;
   DenseTile best = dense_tile(m, columns, k, cus, &least);
-  if (k >= 1024) {
-    least *= 0.93f;
-    for (const StaggeredTime &t : kStaggeredTimes) {
-      if (k < 1280 && t.tile != DenseTile::k256x256) continue;
-      const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns);
-      float time = staggered_time(t, tiles, k, cus);
-      if (t.tile == DenseTile::k256x256 && columns % 8 != 0) time += 6.0f * (float)((tiles + cus - 1) / cus);
-      if (time < least) least = time, best = t.tile;
-    }
+  least *= kInStepScale;
+  for (const StaggeredTime &t : kStaggeredTimes) {
+    if (k < staggered_from_k(t.tile)) continue;
+    const uint64_t tiles = ((m + t.rows - 1) / t.rows) * ((columns + t.columns - 1) / t.columns);
+    const float time = staggered_time(t, tiles, columns, k, cus);
+    if (time < least) least = time, best = t.tile;
   }
   if (estimate != nullptr) *estimate = least;
   return best;
 }
 
-// A product in two launches: the first `columns` on whole rounds of a large tile, the rest on the tile that suits it (0: one
+// A product in two launches: the first `columns` on whole rounds of 256 x 256 tiles, the rest on the tile that suits it (0: one
 // launch).  A round of the 256 CUs that is a tenth filled costs most of a whole one, and smaller tiles for all of the columns
-// are the slower ones.  Taken where the two estimates together are 5% less; us, one launch / two: 2048 x 8512 x 2048 94.9 /
-// 76.3, 3001 x 7312 x 2048 102.9 / 91.3, 2701 x 12096 x 3520 232 / 194, 1451 x 13760 x 3776 157 / 138, 0.99 to 1.01 of one at
-// four of sixteen sizes drawn and less at the others.
-struct DenseSplit {
-  DenseTile tile;
-  uint64_t columns;
-};
-inline DenseSplit dense_column_split(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus) {
-  DenseSplit split = {DenseTile::k256x256, 0};
-  if (k < 1024) return split;
-  float least = 0.0f;
-  dense_product_tile(m, columns, k, cus, &least);
-  least *= 0.95f;
-  for (const StaggeredTime &t : kStaggeredTimes) {
-    if (k < 1280 && t.tile != DenseTile::k256x256) continue;
-    const uint64_t tiles_m = (m + t.rows - 1) / t.rows, tiles = tiles_m * ((columns + t.columns - 1) / t.columns);
-    const uint64_t whole = tiles / cus * cus / tiles_m;  // tile columns of whole rounds
-    if (whole == 0 || tiles % cus == 0 || whole * t.columns >= columns) continue;
-    float rest = 0.0f;
-    dense_product_tile(m, columns - whole * t.columns, k, cus, &rest);
-    const float time = staggered_time(t, whole * tiles_m, k, cus) + rest;
-    if (time < least) least = time, split = {t.tile, whole * t.columns};
-  }
-  return split;
+// are the slower ones.  Taken where the two estimates together are 5% less than the one launch's: at 108 sizes drawn, on four
+// GPUs, 0.90 to 0.92 of one launch on average and 1.02 at most (us, one launch / two: 2048 x 8512 x 2048 94.9 / 76.3, 3001 x 7312 x 2048
+// 102.9 / 91.3, 2701 x 12096 x 3520 232 / 194).  Whole rounds of 256 x 128 tiles in turns gain nothing: 0.96 to 1.03 on average at 48.
+inline uint64_t dense_first_columns(uint32_t m, uint64_t columns, uint32_t k, uint32_t cus) {
+  const uint64_t tiles_m = ((uint64_t)m + 255) / 256, tiles_n = (columns + 255) / 256;
+  const uint64_t whole = tiles_m * tiles_n / cus * cus / tiles_m;  // tile columns of whole rounds
+  if (k < staggered_from_k(DenseTile::k256x256) || whole == 0 || tiles_m * tiles_n % cus == 0 || whole * 256 >= columns) return 0;
+  float one = 0.0f, rest = 0.0f;
+  dense_product_tile(m, columns, k, cus, &one);
+  dense_product_tile(m, columns - whole * 256, k, cus, &rest);
+  return staggered_time(kStaggeredTimes[0], whole * tiles_m, columns, k, cus) + rest < 0.95f * one ? whole * 256 : 0;
 }
 
 }  // namespace llmopt
