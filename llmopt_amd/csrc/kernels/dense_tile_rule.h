@@ -99,9 +99,14 @@ inline float staggered_time(const StaggeredTime &t, uint64_t tiles, uint64_t col
 // 1.07 times at the median of 470 sizes beyond 25 us, where the two are compared.  This puts them on one scale.
 constexpr float kInStepScale = 0.93f;
 
-// Where the staggered tiles begin: in turns from 1280 (below, what the meeting of two groups' sums costs is not made up for:
-// 128 x 128 tiles 0.99 of the ten's time on average, up to 1.16).
-inline uint32_t staggered_from_k(DenseTile tile) { return tile == DenseTile::k256x256 ? 1024 : 1280; }
+// Where the staggered tiles begin: in turns from 1280 (below, what the meeting of two groups' sums costs is not made up for: 0.99 of
+// the ten's time on average, up to 1.16), 128 x 128 ones, which have the most sums to a product, from 1792: from 1280 on 0.98 of the
+// eight waves in step, but more than 3% slower at 5 of 18 sizes (us, in step / in turns: 223 x 10624 x 1408 16.8 / 17.5, 751 x 5312 x
+// 1408 17.3 / 18.1; the medians of three GPUs), from 1792 on 0.95 and 2 of 13, beyond 2560 0.93 and none of 16.
+inline uint32_t staggered_from_k(DenseTile tile) {
+  if (tile == DenseTile::k256x256) return 1024;
+  return tile == DenseTile::kTurns128x128 ? 1792 : 1280;
+}
 
 // The tile a product runs on: one of the ten, or from K = 1024 on one of the staggered ones where its estimate is less: 0.96 of the
 // ten's time on average from there on (us, ten / this: 2048 x 2048 x 8192 74 / 63, 2048 x 2048 x 2048 23.2 / 21.1, 3001 x 2048 x 8192

@@ -145,26 +145,28 @@ def test_rows_split_in_two(runtime, m, n, k):
 
 # Tiles whose waves multiply and read at different times: 256 x 256, in turns 192 x 128, 128 x 128, 128 x 192, 256 x 128 and
 # 128 x 64, each with remainders, an even and an odd number of stages (test_tile_rules.py checks which sizes take which)
-STAGGERED = [(1030, 10967, 1024), (1345, 8853, 1088), (3000, 1500, 1280), (1345, 3001, 1344), (1345, 1500, 1280),
-             (200, 9503, 1344), (500, 9503, 1280), (500, 9503, 1344), (1345, 5001, 1280), (1345, 5001, 1344),
+STAGGERED = [(1030, 10967, 1024), (1345, 8853, 1088), (3000, 1500, 1280), (1345, 3001, 1344), (1345, 1500, 1792),
+             (200, 9503, 1856), (500, 9503, 1280), (500, 9503, 1344), (1345, 5001, 1280), (1345, 5001, 1344),
              (257, 4095, 1280), (200, 5001, 1344)]
 # two launches: whole rounds of 256 x 256, then 64 x 64 or smaller ones, and in turns
-SPLIT = [(2047, 8300, 1024), (2047, 9503, 1344)]
+SPLIT = [(2047, 8300, 1024), (2047, 9503, 1344), (2047, 9503, 1792)]
 # columns that are no whole pieces, where whole ones take 256 x 256
 ODD = [(1345, 6001, 1024), (3000, 3001, 1088)]
+# 128 x 128 tiles in step up to K = 1791
+SHORT = [(1345, 1500, 1280), (200, 9503, 1344)]
 
 
-@pytest.mark.parametrize("m,n,k", STAGGERED + SPLIT + ODD)
+@pytest.mark.parametrize("m,n,k", STAGGERED + SPLIT + ODD + SHORT)
 def test_staggered_tiles(runtime, m, n, k):
     test_tiles(runtime, m, n, k)
 
 
-@pytest.mark.parametrize("m,n,k", STAGGERED + SPLIT + ODD)
+@pytest.mark.parametrize("m,n,k", STAGGERED + SPLIT + ODD + SHORT)
 def test_staggered_tiles_of_rows(runtime, m, n, k):
     test_rows_with_mixed_values(runtime, m, n, k)
 
 
-@pytest.mark.parametrize("m,n,k", STAGGERED + SPLIT + ODD)
+@pytest.mark.parametrize("m,n,k", STAGGERED + SPLIT + ODD + SHORT)
 def test_staggered_tiles_of_pairs(runtime, m, n, k):
     test_gated_tiles(runtime, m, k, n // 2)
 

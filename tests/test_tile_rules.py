@@ -197,6 +197,12 @@ def test_products_that_stay_in_step(rules, m, n, k):
     assert rules.staggered_tile(m, n, k, CUS) == rules.product_tile(m, n, k, CUS)
 
 
+@pytest.mark.parametrize("m,n,k", [(223, 10624, 1408), (751, 5312, 1408), (220, 9984, 1600), (213, 14656, 1408), *test_gpu_dense_tiles.SHORT])
+def test_128_rows_and_columns_stay_in_step_below_1792(rules, m, n, k):
+    assert DENSE[rules.staggered_tile(m, n, k, CUS)] == "128x128 eight waves"
+    assert rules.staggered_tile(m, n, 1792, CUS) == len(DENSE) + 1
+
+
 @pytest.mark.parametrize("m,n,k,first", [(2048, 8512, 2048, 8192), (3001, 7312, 2048, 5376), (2048, 9504, 2048, 8192),
                                          (2048, 16384, 2048, 0), (3001, 16384, 2048, 0), (2048, 2048, 8192, 0), (2048, 8512, 960, 0)])
 def test_columns_in_two_launches(rules, m, n, k, first):
