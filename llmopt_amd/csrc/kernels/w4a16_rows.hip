@@ -365,12 +365,12 @@ __device__ __forceinline__ uint32_t normed_pair(uint32_t x, uint32_t gain, float
   return (uint32_t)float_to_half_bits(low) | (uint32_t)float_to_half_bits(high) << 16;
 }
 
-// The same tiles over rows that the kernel normalises itself, for a K whose rows and weights fit LDS as a whole: everything is
-// requested at once, waves normalise the rows where they lie, eight lanes a row, and the products follow without a barrier
-// between them.  The launch of the norm ahead, 3.4 us of starting and a trip to memory and back, and its boundary go.  With 32
-// rows of 576 values that is the better one (QKV with rotation and pack, 700 rows: 8.0 + 3.4 us and the boundary / 11.2; prompts of
-// 64 to 900 tokens of a 30-layer transformer 1.5 to 3.5% less), with 96 rows the copies that no product covers cost as much
-// (a pair of 700 x 576 x 1536: 10.8 + 3.4 / 15.6).
+// The same tiles over rows that the kernel normalises itself, for a short K (kNormedGroups) all of whose rows and weights lie in
+// LDS: everything is requested at once, waves normalise the rows where they lie, eight lanes a row, and the products follow without
+// a barrier between them.  The launch of the norm ahead, 3.4 us of starting and a trip to memory and back, and its boundary go.
+// With 32 rows of 576 values that is the better one (QKV with rotation and pack, 700 rows: 8.0 + 3.4 us and the boundary / 11.2; a
+// pair of 64 x 576 x 1536 10.2 / 8.7 a call; prompts of 64 to 900 tokens of a 30-layer transformer 1.5 to 3.5% less), with 96 rows the
+// copies that no product covers cost as much (a pair of 700 x 576 x 1536: 10.8 + 3.4 / 15.6).
 //
 //  * Rows lie as blocks of eight rows by one scale group, 1 KB that a copy fills from whole lines, pieces XOR-ed by half the row;
 //    weights as blocks of sixteen columns by two groups, pieces XOR-ed by a quarter of the column.  Operand reads of sixteen

@@ -28,7 +28,11 @@ constexpr uint32_t rows_lds_bytes(uint32_t k) {
   return scale_lds_bytes(CT * 32, k / 64) + (ring > sums ? ring : sums);
 }
 
-// Rows, weights and norm weights of a whole K (w4a16_normed_rows_kernel), whose lanes hold a piece of every group.
+// Rows, weights and norm weights of a whole K (w4a16_normed_rows_kernel), whose lanes hold a piece of every group.  Up to twelve groups:
+// LDS has room for 24, but from thirteen on the copies that no product covers take what the norm's launch does.  us a call, norm
+// apart / in the tile: QKV 90 x 576 x (576, 192) 11.4 / 9.6, 700 x 576 13.5 / 12.8, 200 x 768 x (768, 256) 11.5 / 11.1; pairs 64 x 576 x 1536
+// 10.2 / 8.7, 140 x 768 x 801 11.1 / 9.5; beyond: QKV 100 x 1024 x (768, 256) 11.1 / 12.1, 128 x 1024 x (1024, 256) 11.1 / 12.2, pairs 100 x
+// 1024 x 1024 10.6 / 10.9, 128 x 960 x 1024 11.0 / 10.7.
 constexpr uint32_t kNormedGroups = 12;
 template <int ROWS, int CT, int P>
 constexpr uint32_t normed_rows_lds_bytes(uint32_t k) {
@@ -160,7 +164,7 @@ inline RowsTile logits_rows_tile(uint32_t rows, uint32_t n, uint32_t k, uint32_t
   return RowsTile::kNone;
 }
 
-// Whether a tile normalises its rows itself: tiles of 32 rows and a K that fits LDS as a whole, in one round of workgroups.
+// Whether a tile normalises its rows itself: tiles of 32 rows and at most kNormedGroups groups of K, in one round of workgroups.
 inline bool normed_rows(RowsTile tile, uint32_t m, const uint32_t *n, uint32_t matrices, uint32_t k, uint32_t cus) {
   if (tile != RowsTile::k32x64 || k > kNormedGroups * 64) return false;
   uint64_t tiles = 0;
