@@ -667,7 +667,8 @@ __global__ __launch_bounds__(512) void dense_gemm_turns_kernel(GemmParams p) {
   constexpr int BEHIND = (STAGES - 3) / 2 * COPIES;  // copies that may be under way when the next step has landed
   constexpr int RING = STAGES * ROWS * 128, PART = MT / 2 * NT * 1024;  // bytes: the stages; a wave's half of its sums
   static_assert(MT % 2 == 0 && (!GATED || NT % 2 == 0) && ROWS % 32 == 0 && STAGES >= 3 && STAGES % 2 == 1, "tile");
-  static_assert(RING <= 160 * 1024 && 8 * PART <= RING && 8 * 16 * (NT * 16 + 8) * 2 <= RING, "the ring, the sums and the output rows fit");
+  static_assert(RING <= 160 * 1024, "the ring fits a CU");
+  static_assert(8 * PART <= RING && 8 * 16 * (NT * 16 + 8) * 2 <= RING, "the sums and the output rows fit the ring");
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const DenseLinearArgs &a = p.a;
   TilePlace place;
@@ -835,7 +836,8 @@ hipError_t pick_routed(const DenseLinearArgs &a, hipStream_t stream) {
     if (!direct) return hipErrorInvalidValue;
     // In turns while the launch is one round of workgroups at most; beyond, two workgroups in step on a CU fill each other's waits
     // and the last round.  Whole feed-forward, us, in step / in turns (tokens, width, expert's width): one round 500 x 1024 x 512
-    // 46.7 / 43.9, 2048 x 512 x 256 41.3 / 39.6; more 3001 x 1024 x 512 100 / 118, 2048 x 1024 x 512 84 / 90.
+    // 46.7 / 43.9, 2048 x 512 x 256 41.3 / 39.6; more 3001 x 1024 x 512 102 / 118, 2048 x 1024 x 512 85 / 90, 1024 x 2048 x 1024
+    // 119 / 123, 2048 x 2048 x 1024 195 / 197, 3001 x 2048 x 1024 258 / 267; the other way 600 x 2048 x 4096 175 / 164.
     const uint64_t most = (uint64_t)a.tiles * ((a.n + (GATED ? 63 : 127)) / (GATED ? 64 : 128));
     if (most <= (uint64_t)device_compute_units()) return run_turns<128, 128, 5, GATED, true>(a, {0, a.n}, stream);
     return run_direct<128, 128, 2, 4, 2, GATED, true>(a, {0, a.n}, stream);
