@@ -8,12 +8,16 @@
 // kv_head = head / (h / kvh), output head-major [b, h, q, D] or token-major
 // [b, q, h, D]; a row with no allowed key is zero.  Scores and softmax in fp32.
 //
-//  * dense_attention_tile32_kernel<D> (D = 64, 128): 32 x 32 wave tiles on
+//  * dense_attention_turns_kernel<D> (D = 64, 128; no mask, launches that fill the device): 32 x 32 wave tiles, two groups of
+//    waves in turns at the matrix cores and the exponentials (attention_turns.h).
+//  * dense_attention_tile32_kernel<D> (D = 64, 128, 256): 32 x 32 wave tiles on
 //    v_mfma_f32_32x32x16_f16 over K / V stages shared through LDS; described at the kernel.
 //  * dense_attention_rows_kernel: one wave per output row, serial over the keys
 //    (any D up to 512, every option); the direct restatement.
 #include <algorithm>
+#include <cfloat>
 
+#include "attention_turns.h"
 #include "dense_attention_rule.h"
 #include "kernels.h"
 #include "kernels_internal.h"
@@ -714,6 +718,98 @@ __global__ __launch_bounds__(256) void tree_mask_kernel(TreeMaskArgs a) {
   a.mask[index] = allowed ? 1 : 0;
 }
 
+}  // namespace
+
+// ---- two groups of waves in turns: 128 rows of a head without a mask --------------------------
+
+template <>
+struct TurnsOperand<_Float16> {
+  typedef h8_t x8;
+  struct Weights {
+    x8 v;
+    __device__ __forceinline__ void set_pair(int i, float x, float y) { v[i] = (_Float16)x, v[i + 1] = (_Float16)y; }
+  };
+  static __device__ __forceinline__ f32x16 product(x8 a, x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x16 weighted(x8 a, const Weights &w, f32x16 c) { return product(a, w.v, c); }
+};
+
+namespace {
+
+// Bound by the softmax of one wave beside the products of the other: a step of 64 keys is about 1250 cycles of products
+// (1024 of them the matrix core's) beside 1000 of softmax and 200 of copies, where two free waves took 3200 for it; no copies at
+// all would save another tenth, no exponentials 4 %.  32 / 8 heads of 128, causal: 4096 rows 180 -> 155 us (886 TFLOP/s),
+// 2048 59 -> 48, 1500 46 -> 32; 16 / 4: 4096 105 -> 83, 1900 62 -> 35; 16 / 4 of 64, 4096 rows 68 -> 55.
+// Later rows see more keys and come first, a workgroup a CU; heads of one key / value head follow each other kv_heads apart,
+// so that they share an XCD's L2 when kv_heads is a multiple of the eight XCDs.
+template <int D, bool SPLIT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_attention_turns_kernel(DenseAttentionArgs a) {
+  constexpr int JJ = D / 32, WAVES = SPLIT ? 4 : 8;
+  constexpr uint32_t ROWS = turns_rows<SPLIT>();
+  extern __shared__ __attribute__((aligned(16))) unsigned char stage_lds[];
+  const uint32_t lane = threadIdx.x & 63, row_lane = lane & 31, half = lane >> 5;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t slabs = (a.query_length + ROWS - 1) / ROWS, per_slab = a.heads * a.batches;
+  const uint32_t kv_heads = a.kv_heads > 0 ? a.kv_heads : a.heads, per = a.heads / kv_heads;
+  const uint32_t rank = blockIdx.x, within = rank % per_slab, slab = a.causal ? slabs - 1 - rank / per_slab : rank / per_slab;
+  const uint32_t batch = within / a.heads, kv_head = within % a.heads % kv_heads;
+  const uint32_t head = kv_head * per + within % a.heads / kv_heads;
+  const uint32_t L = a.key_length, wave_row = slab * ROWS + wave % WAVES * 32;
+  const uint32_t own = min(wave_row + row_lane, a.query_length - 1);
+
+  h8_t q[D / 16];
+  const uint16_t *q_row = a.query + (((size_t)batch * a.heads + head) * a.query_length + own) * D;
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) q[ks] = *reinterpret_cast<const h8_t *>(q_row + ks * 16 + half * 8);
+  const auto last_of = [&](uint32_t r) {
+    return a.causal ? (uint32_t)min((uint64_t)a.past_length + min(r, a.query_length - 1), (uint64_t)L - 1) : L - 1;
+  };
+  const TurnsBounds bounds = {0, last_of(own), 0, 0, last_of(wave_row), last_of(wave_row + 31)};
+  const uint32_t stages = last_of(slab * ROWS + ROWS - 1) / kTurnsKeys + 1;
+  const uint16_t *keys = a.key + ((size_t)batch * kv_heads + kv_head) * L * D;
+  const uint32_t value_stride = a.token_first_value ? kv_heads * D : D;
+  const uint16_t *values = a.value + (a.token_first_value ? ((size_t)batch * L * kv_heads + kv_head) * D
+                                                          : ((size_t)batch * kv_heads + kv_head) * L * D);
+  const TurnsCopy<D, WAVES, false> k_rows(D * 2);
+  const TurnsCopy<D, WAVES, true> v_rows(value_stride * 2);
+  const auto copy_k = [&](uint32_t key, uint32_t stage) {
+    if (key + kTurnsKeys <= L) k_rows.whole(keys + (size_t)key * D, stage);
+    else k_rows.rows([&](uint32_t r) { return keys + (size_t)min(key + r, L - 1) * D; }, stage);
+  };
+  const auto copy_v = [&](uint32_t key, uint32_t stage) {
+    if (key + kTurnsKeys <= L) v_rows.whole(values + (size_t)key * value_stride, stage);
+    else v_rows.rows([&](uint32_t r) { return values + (size_t)min(key + r, L - 1) * value_stride; }, stage);
+  };
+  float top = -FLT_MAX, total = 0.0f;
+  f32x16 out[JJ];
+#pragma unroll
+  for (int jj = 0; jj < JJ; ++jj)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) out[jj][r] = 0.0f;
+  if (!attention_turns<_Float16, D, SPLIT, TurnsScores::kPlain>(stage_lds, q, bounds, 0, stages, a.scale * 1.4426950408889634f,
+                                                                0.0f, top, total, out, copy_k, copy_v))
+    return;
+  float low, high;
+  both_halves(total, low, high);
+  total = low + high;
+  if (wave_row >= a.query_length) return;
+  const float inverse = total != 0.0f ? 1.0f / total : 0.0f;
+  const size_t first = a.token_first_output ? ((size_t)batch * a.query_length + wave_row) * a.heads + head
+                                            : ((size_t)batch * a.heads + head) * a.query_length + wave_row;
+  constexpr int FROM = SPLIT ? turns_share_bytes<D>() : 0;
+  static_assert(FROM + WAVES * store_rows_bytes<D>() <= turns_lds_bytes<D, SPLIT>(), "the rows fit the stages");
+  store_rows<D>(stage_lds + FROM + wave * store_rows_bytes<D>(), a.output + first * D, (a.token_first_output ? a.heads : 1) * (size_t)(D * 2),
+                a.query_length - wave_row, [&](int jj, int r) {
+                  uint2 packed;
+                  packed.x = (uint32_t)float_to_half_bits(out[jj][r] * inverse) |
+                             ((uint32_t)float_to_half_bits(out[jj][r + 1] * inverse) << 16);
+                  packed.y = (uint32_t)float_to_half_bits(out[jj][r + 2] * inverse) |
+                             ((uint32_t)float_to_half_bits(out[jj][r + 3] * inverse) << 16);
+                  return packed;
+                });
+}
+
 // ---- row-serial kernel (every other configuration) ---------------------------
 
 constexpr int kMaxFragments = 8;  // head_dim <= 512
@@ -796,13 +892,25 @@ hipError_t launch_tile32_instance(uint32_t grid, const DenseAttentionArgs &a, hi
   return hipGetLastError();
 }
 
+template <int D, bool SPLIT>
+hipError_t launch_turns(const DenseAttentionArgs &a, hipStream_t stream) {
+  static bool configured[kMaxDevices] = {};
+  const auto kernel = &dense_attention_turns_kernel<D, SPLIT>;
+  constexpr int bytes = turns_lds_bytes<D, SPLIT>();
+  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, configured)) return status;
+  const uint64_t grid = (uint64_t)((a.query_length + turns_rows<SPLIT>() - 1) / turns_rows<SPLIT>()) * a.heads * a.batches;
+  hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(512), bytes, stream, a);
+  return hipGetLastError();
+}
+
 // mask: 0 none, 1 bytes, 2 halves, 3 bits
 template <int D, int WAVES, int STAGE_KEYS, bool KEYSPLIT, bool PAIR = false>
 hipError_t launch_tile32(int mask, uint32_t grid, const DenseAttentionArgs &a, hipStream_t stream) {
   if (mask == 3) return launch_tile32_instance<D, WAVES, STAGE_KEYS, 3, KEYSPLIT, PAIR>(grid, a, stream);
   if (mask == 2) return launch_tile32_instance<D, WAVES, STAGE_KEYS, 2, KEYSPLIT, PAIR>(grid, a, stream);
   if (mask == 1) return launch_tile32_instance<D, WAVES, STAGE_KEYS, 1, KEYSPLIT, PAIR>(grid, a, stream);
-  return launch_tile32_instance<D, WAVES, STAGE_KEYS, 0, KEYSPLIT, PAIR>(grid, a, stream);
+  if constexpr (PAIR) return hipErrorInvalidValue;  // (without a mask such launches go in turns)
+  else return launch_tile32_instance<D, WAVES, STAGE_KEYS, 0, KEYSPLIT, PAIR>(grid, a, stream);
 }
 
 // Which kernel a launch takes and the slabs and stages it works in.
@@ -903,6 +1011,10 @@ hipError_t launch_dense_attention(const DenseAttentionArgs &a, hipStream_t strea
           mask_kind = 3;
         }
       }
+      const TurnsForm turns = turns_form(a.head_dim, mask != 0, a.query_length, a.key_length, workgroups,
+                                         (uint32_t)device_compute_units());
+      if (turns == TurnsForm::kSplit) return a.head_dim == 64 ? launch_turns<64, true>(a, stream) : launch_turns<128, true>(a, stream);
+      if (turns == TurnsForm::kRows) return a.head_dim == 64 ? launch_turns<64, false>(a, stream) : launch_turns<128, false>(a, stream);
       if (geometry.key_split) {
         const uint32_t grid = (uint32_t)((a.query_length + 31) / 32) * a.heads * a.batches;
         if (eight_wave_slabs(a.head_dim, mask != 0, a.causal != 0, a.query_length, a.key_length, a.past_length, grid,
@@ -917,12 +1029,12 @@ hipError_t launch_dense_attention(const DenseAttentionArgs &a, hipStream_t strea
       // tokens - one tile per barrier, half the sharing.)  Heads of 256: 128 KB of stages, one
       // workgroup per CU with all of its registers.
       if (a.head_dim == 256) return launch_tile32<256, 4, 64, false>(mask_kind, (uint32_t)workgroups, scheduled, stream);
-      // One or two workgroups per CU: two groups of four waves per slab, each with half of the stages (a
+      // One or two workgroups per CU under a mask: two groups of four waves per slab, each with half of the stages (a
       // CU then holds one workgroup at a time, at the same two waves per SIMD): 32 heads x 2048 tokens,
-      // 512 workgroups, 72.9 -> 67.6 us.  The groups meet at every stage's barrier, so two of them get
+      // 512 workgroups, 72.9 -> 67.6 us (without one, before such launches went in turns).  The groups meet at every stage's barrier, so two of them get
       // less out of a CU than two workgroups of four waves that run side by side freely - launches with
       // enough of those keep them.
-      if (workgroups <= 2 * (uint64_t)device_compute_units() && a.key_length >= 256) {
+      if (mask != 0 && workgroups <= 2 * (uint64_t)device_compute_units() && a.key_length >= 256) {
         if (a.head_dim == 64) return launch_tile32<64, 4, 64, false, true>(mask_kind, (uint32_t)workgroups, scheduled, stream);
         return launch_tile32<128, 4, 64, false, true>(mask_kind, (uint32_t)workgroups, scheduled, stream);
       }

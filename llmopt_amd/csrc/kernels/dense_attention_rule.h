@@ -1,5 +1,5 @@
-// Which launch of the key-splitting dense attention takes eight waves a slab: a rule on sizes alone, without HIP, so that a
-// host test can ask it.
+// Which dense attention launches take two groups of waves in turns, and which of the key-splitting ones eight waves a slab:
+// rules on sizes alone, without HIP, so that a host test can ask them.
 #pragma once
 
 #include <stdint.h>
@@ -21,6 +21,26 @@ inline bool eight_wave_slabs(uint32_t head_dim, bool masked, bool causal, uint32
   const uint64_t walk = causal && last < key_length ? last : key_length;
   const uint64_t room = causal && walk > 640 ? (uint64_t)cus * 9 / 8 : cus;
   return head_dim == 64 && !masked && key_length > 512 && walk > 256 && slabs <= room;
+}
+
+enum class TurnsForm { kNone, kSplit, kRows };
+
+// Without a mask, from 256 keys on (below that the groups have a stage or two each); workgroups: of 128 rows.
+// kSplit, 128 rows whose keys the groups share, against the key-splitting slabs of 32 rows: heads of 128 as soon as those are
+// more than a workgroup a CU, their stages' room (us, heads x rows: 32 x 300 10.9 / 14.3, 32 x 700 16.2 / 29.0, 16 x 700 15.8 /
+// 17.7, 16 x 1900 34.5 / 61.5; 16 x 500 14.1 / 12.4, 4 x 1500 25.1 / 24.2), heads of 64, of which a CU takes more, from three
+// quarters of the CUs on (9 x 3000 33.0 / 34.7, 16 x 1900 24.1 / 26.7; 16 x 1500 20.4 / 20.0, 9 x 2048 24.5 / 20.0).
+// kRows, 256 rows and their own group each, half the copies and no sums to hand over, once the longer workgroups still come to
+// more than a round and a half (32 heads of 128: 4096 rows 162 / 167, 3500 126 / 131, 3000 102 / 100, 2048 62 / 48), and
+// only where rows fill them.
+// Many workgroups that each walk a few stages are better off two a CU (64 x 32 heads of 128, 16 rows, 260 keys 72.7 / 66.4;
+// 16 x 32 of 64, 300 of 300 39.2 / 35.5; 8 x 32 of 128, 300 of 300 29.4 / 29.8; 32 x 32, 64 rows, 512 keys 51.5 / 53.6).
+inline TurnsForm turns_form(uint32_t head_dim, bool masked, uint32_t query_length, uint32_t key_length, uint64_t workgroups,
+                            uint32_t cus) {
+  if (masked || (head_dim != 64 && head_dim != 128) || key_length < 256) return TurnsForm::kNone;
+  if (workgroups > 3 * (uint64_t)cus && key_length < 512) return TurnsForm::kNone;
+  if (workgroups > 3 * (uint64_t)cus && query_length >= 1024) return TurnsForm::kRows;
+  return 4 * workgroups > (head_dim == 64 ? 3 : 1) * (uint64_t)cus ? TurnsForm::kSplit : TurnsForm::kNone;
 }
 
 }  // namespace llmopt

@@ -341,6 +341,35 @@ def test_long_walks_of_few_slabs_take_eight_waves(runtime, heads, kv_heads, new,
     check_attention_case(runtime, 64, heads, kv_heads, new, past, mode)
 
 
+@pytest.mark.parametrize("dim,batches,heads,kv_heads,new,past,mode", [
+    (128, 1, 12, 4, 700, 0, "causal"), (128, 2, 33, 11, 33, 223, "none"), (128, 3, 11, 11, 257, 130, "causal"),
+    (128, 1, 80, 10, 1, 255, "none"), (64, 2, 50, 25, 129, 383, "causal"), (64, 1, 40, 8, 640, 1, "none"),
+    (128, 1, 86, 43, 1031, 0, "causal"), (64, 2, 43, 43, 1100, 77, "causal"), (64, 1, 96, 8, 1024, 3, "none"),
+])
+def test_groups_of_waves_in_turns(runtime, dim, batches, heads, kv_heads, new, past, mode):
+    """Launches without a mask that fill the device: 128 rows whose keys two groups of waves share, and 256 rows; partial
+    last stages and slabs, groups and waves without keys, both layouts.  Heads of every batch against the oracle."""
+    rng = np.random.default_rng(dim + heads + new + past)
+    length, scale, causal = past + new, 1.0 / math.sqrt(dim), mode == "causal"
+    query = rng.standard_normal((batches, heads, new, dim)).astype(np.float16)
+    key = (rng.standard_normal((batches, kv_heads, length, dim)) * 2).astype(np.float16)
+    value = rng.standard_normal((batches, kv_heads, length, dim)).astype(np.float16)
+    token_major = new % 2
+    params = attention_params(batches, heads, new, length, dim, 0, 0, causal, scale, kv_heads, token_first_output=token_major,
+                              past_length=past if causal else 0, token_first_value=token_major)
+    value_in = np.ascontiguousarray(value.transpose(0, 2, 1, 3)) if token_major else value
+    got = run(runtime, f"llmopt_attention_f16_simd_h{dim}", query, key, value_in, None, params,
+              (batches, new, heads, dim) if token_major else (batches, heads, new, dim))
+    got = got.transpose(0, 2, 1, 3) if token_major else got
+    allowed = np.arange(length)[None, :] <= past + np.arange(new)[:, None] if causal else np.ones((new, length), dtype=bool)
+    for batch in range(batches):
+        for head in {0, heads // 2, heads - 1}:
+            one = (slice(batch, batch + 1), slice(head, head + 1))
+            kv = (one[0], slice(head // (heads // kv_heads), head // (heads // kv_heads) + 1))
+            want = expected(query[one], key[kv], value[kv], allowed[None, None], scale)
+            assert_close_to_oracle(got[one], want, f"D={dim} {heads}/{kv_heads} {new} after {past}, {mode}, {batch}/{head}")
+
+
 @pytest.mark.parametrize("heads,kv_heads,new,past,mode", [
     (4, 2, 300, 0, "causal"), (2, 1, 45, 211, "causal"), (2, 2, 33, 100, "none"), (3, 1, 130, 70, "bool"),
     (2, 2, 64, 191, "f16"), (8, 4, 16, 0, "causal"),

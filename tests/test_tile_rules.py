@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from tests import test_gpu_delta_chunks, test_gpu_dense_tiles, test_gpu_w4a16_rows
+from tests import test_gpu_delta_chunks, test_gpu_dense_attention, test_gpu_dense_tiles, test_gpu_w4a16_rows
 
 CUS = 256
 KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "kernels")
@@ -23,6 +23,9 @@ int gated_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) { return (int)g
 int logits_tile(uint32_t tokens, uint32_t n, uint32_t k, uint32_t cus) { return (int)logits_rows_tile(2 * tokens, n, k, cus); }
 int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, uint32_t heads, uint32_t cus) {
   return eight_wave_slabs(64, false, causal != 0, rows, keys, past, (rows + 31) / 32 * heads, cus);
+}
+int turns(uint32_t dim, uint32_t masked, uint32_t rows, uint32_t keys, uint32_t heads, uint32_t cus) {
+  return (int)turns_form(dim, masked != 0, rows, keys, (uint64_t)((rows + 127) / 128) * heads, cus);
 }
 int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
   return three_delta_workgroups((tokens + 63) / 64 * heads, cus);
@@ -149,6 +152,22 @@ def test_logits(rules, tokens, k, n, tiles):
     (1, 32, 4096, 0, 9, 0), (1, 64, 2000, 0, 16, 0), (1, 100, 520, 0, 3, 0), (1, 32, 4096, 224, 9, 0), (1, 32, 4096, 225, 9, 1), (1, 400, 4000, 0, 9, 1)])
 def test_eight_waves_a_slab(rules, causal, rows, keys, past, heads, eight):
     assert rules.eight_waves(causal, rows, keys, past, heads, CUS) == eight
+
+
+@pytest.mark.parametrize("dim,masked,rows,keys,heads,form", [
+    (128, 0, 4096, 4096, 32, 2), (128, 0, 3500, 3500, 32, 2), (128, 0, 3000, 3000, 32, 1), (128, 0, 1000, 9000, 128, 1),
+    (128, 0, 300, 300, 32, 1), (128, 0, 700, 700, 16, 1), (128, 0, 500, 500, 16, 0), (128, 0, 255, 255, 64, 0),
+    (128, 0, 255, 256, 64, 1), (64, 0, 1900, 1900, 16, 1), (64, 0, 1500, 1500, 16, 0), (64, 0, 4096, 4096, 32, 2),
+    (256, 0, 4096, 4096, 32, 0), (128, 0, 300, 300, 512, 0), (128, 0, 300, 300, 256, 1), (128, 0, 64, 512, 1024, 1), (128, 1, 4096, 4096, 32, 0)])
+def test_attention_in_turns(rules, dim, masked, rows, keys, heads, form):
+    assert rules.turns(dim, masked, rows, keys, heads, CUS) == form
+
+
+def test_gpu_tests_reach_both_forms_of_turns(rules):
+    names = "dim,batches,heads,kv_heads,new,past,mode"
+    reached = [(dim, rules.turns(dim, 0, new, new + past, heads * batches, CUS))
+               for dim, batches, heads, _, new, past, _ in sizes(test_gpu_dense_attention.test_groups_of_waves_in_turns, names)]
+    assert set(reached) == {(64, 1), (64, 2), (128, 1), (128, 2)}
 
 
 @pytest.mark.parametrize("tokens,heads,three", [(3001, 16, 1), (2115, 16, 1), (4096, 32, 1), (3001, 32, 1), (3001, 8, 0),
