@@ -1,4 +1,5 @@
-// Attention of a prompt's rows by two groups of waves that take turns at the matrix cores (dense_attention.hip).
+// Attention of a prompt's rows by two groups of waves that take turns at the matrix cores (dense_attention.hip,
+// chunk_attention.hip).
 //
 // A workgroup is eight waves, two on each SIMD, over the rows of one head, 32 a wave.  A wave's step is
 //
@@ -35,7 +36,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr uint32_t kTurnsKeys = 64;
 
 // The element's matrix operands, specialised beside each kernel: x8, eight elements; Weights, those of eight keys
-// (set_pair(i, x, y) for an even i); product(a, b, c) and weighted(a, weights, c), 32 x 32 += 32 x 16 times 16 x 32.
+// (set_pair(i, x, y) for an even i); product(a, b, c) and weighted(a, weights, c), kProducts of it, 32 x 32 += 32 x 16 times
+// 16 x 32.
 template <typename E>
 struct TurnsOperand;
 
@@ -74,10 +76,10 @@ struct TurnsCopy {
   // Where a lane reads for each copy of a stage whose rows are one stride behind each other; the instruction's own offset
   // moves both ends, so that all copies share an address and a target.
   uint32_t offset[COUNT], wave;
-  __device__ __forceinline__ explicit TurnsCopy(uint32_t stride_bytes)
+  __device__ __forceinline__ TurnsCopy(uint32_t stride_bytes, uint32_t thread)
       : wave((uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) {
 #pragma unroll
-    for (int c = 0; c < COUNT; ++c) offset[c] = row(threadIdx.x, c) * stride_bytes + piece_bytes(threadIdx.x, c) - c * 1024;
+    for (int c = 0; c < COUNT; ++c) offset[c] = row(thread, c) * stride_bytes + piece_bytes(thread, c) - c * 1024;
   }
   // the stage from `first` on, the same for the whole wave
   __device__ __forceinline__ void whole(const void *first, uint32_t stage) const {
@@ -142,7 +144,6 @@ __device__ __forceinline__ bool attention_turns(unsigned char *lds, const typena
   constexpr int KSTEPS = D / 16, JJ = D / 32, ROW = D * 2, PIECES = D / 8, STAGE = turns_stage_bytes<D>();
   constexpr int kCopies = 2 * TurnsCopy<D, SPLIT ? 4 : 8, false>::COUNT;
   constexpr uint32_t RING = SPLIT ? 2 : 3, EVERY = SPLIT ? 2 : 1;  // stages in LDS; every which stage is this group's
-  constexpr float kSlack = 0.0f;
   const uint32_t lane = threadIdx.x & 63, row_lane = lane & 31, half = lane >> 5;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), group = wave >> 2;
   unsigned char *own = lds + (SPLIT ? group * 4 * STAGE : 0);
@@ -258,7 +259,7 @@ __device__ __forceinline__ bool attention_turns(unsigned char *lds, const typena
         float low, high;
         both_halves(best, low, high);
         best = fmaxf(low, high) * (SCORES == TurnsScores::kPlain ? inner : 1.0f);
-        const bool above = best > top + kSlack;
+        const bool above = best > top;
         if (__builtin_amdgcn_ballot_w64(above) != 0) {
           const float higher = above ? best : top;
           const float alpha = __builtin_amdgcn_exp2f(top - higher);
@@ -288,7 +289,7 @@ __device__ __forceinline__ bool attention_turns(unsigned char *lds, const typena
       if (group == 1) __builtin_amdgcn_s_setprio(1);  // against the older wave's softmax
       scores(step + 1);  // (behind the last step they are of whatever is there, and nothing reads them)
       values(step);
-      // operands come from LDS four products ahead
+      // operands come from LDS four ahead of their products
       constexpr int kProduct = 0x8, kRead = 0x100, kAhead = 4, kScores = 2 * KSTEPS, kValues = 4 * JJ;
       __builtin_amdgcn_sched_group_barrier(kRead, kAhead, 0);
 #pragma unroll
@@ -297,11 +298,16 @@ __device__ __forceinline__ bool attention_turns(unsigned char *lds, const typena
         __builtin_amdgcn_sched_group_barrier(kRead, 1, 0);
       }
 #pragma unroll
-      for (int i = 0; i < kValues; ++i) {
+      for (int i = 0; i < kAhead; ++i) {
         __builtin_amdgcn_sched_group_barrier(kProduct, 1, 0);
         __builtin_amdgcn_sched_group_barrier(kRead, 2, 0);
       }
-      __builtin_amdgcn_sched_group_barrier(kProduct, kAhead, 0);
+#pragma unroll
+      for (int i = 0; i < kValues - kAhead; ++i) {
+        __builtin_amdgcn_sched_group_barrier(kProduct, Operand::kProducts, 0);
+        __builtin_amdgcn_sched_group_barrier(kRead, 2, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(kProduct, kAhead * Operand::kProducts, 0);
       if (group == 1) __builtin_amdgcn_s_setprio(0);
     }
     for (uint32_t step = last; step < steps; ++step) idle(step);

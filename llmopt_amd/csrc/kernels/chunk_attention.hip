@@ -8,7 +8,8 @@
 // Keys and values live in a ring per sequence slot and head: position p in row p % capacity, capacity >=
 // chunk or window, so that a ring of one holds everything later tokens can see.
 //
-//  * chunk_prefill_kernel: a portion of a prompt.  Waves of 16 query rows of one head each walk its keys,
+//  * chunk_turns_kernel: a portion of a prompt in bfloat16 whose rows walk over many keys; described at the kernel.
+//  * chunk_prefill_kernel: any other portion of a prompt.  Waves of 16 query rows of one head each walk its keys,
 //    64 keys a stage through LDS; keys before the portion come from the ring, the others from the
 //    portion's own rows.  Bound by the latency of a stage (products, softmax, products in turn): matrix units are
 //    busy for 29% of the time and vector units for 50%, and a second stage in LDS gives nothing.  16 heads of 128
@@ -25,13 +26,31 @@
 //    key first (in LDS) and leaves key and value in the ring; the own key and value never come from there.
 //  * rotate_heads_kernel: the same norm and rotation for a portion of a prompt, in place.
 #include <algorithm>
+#include <cfloat>
+#include <type_traits>
 
+#include "attention_turns.h"
 #include "chunk_decode.h"
+#include "dense_attention_rule.h"
 #include "dense.h"
 #include "dense_common.h"
 #include "kernels_internal.h"
 
 namespace llmopt {
+
+template <>
+struct TurnsOperand<__bf16> {
+  typedef bf16x8 x8;
+  typedef WideFrag<__bf16> Weights;  // the weights keep float32 accuracy
+  static constexpr int kProducts = 2;
+  static __device__ __forceinline__ f32x16 product(x8 a, x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x16 weighted(x8 a, const Weights &w, f32x16 c) {
+    return product(a, w.lo, product(a, w.hi, c));
+  }
+};
+
 namespace {
 
 constexpr int kStageKeys = 64;
@@ -303,6 +322,88 @@ chunk_prefill_kernel(ChunkAttentionArgs a, uint32_t cus) {
   }
 }
 
+// A long portion of a prompt, bfloat16: 32 rows a wave and two groups of waves in turns (attention_turns.h), the keys of 128 rows
+// shared between them.  Bound by both sides of a turn alike: 48 products of 64 keys, of which the weights' low part is a third,
+// take 2050 cycles beside the other wave's softmax and split (1500 and 250 of copies; under a cap 2650), 1536 by themselves.
+// 16 heads of 128 over 3001 rows with a window of 2048, norm and cache writes included: 96 -> 75 us; 32 heads over 2048 under a
+// cap 90 -> 74.  The weights packed beside the products instead: 77 / 81 for 74 / 76.
+template <int D, TurnsScores SCORES>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_turns_kernel(ChunkAttentionArgs a) {
+  constexpr int JJ = D / 32, WAVES = 4;
+  constexpr uint32_t ROWS = turns_rows<true>();
+  extern __shared__ __attribute__((aligned(16))) unsigned char stage_lds[];
+  const uint32_t lane = threadIdx.x & 63, row_lane = lane & 31, half = lane >> 5;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t slabs = (a.m + ROWS - 1) / ROWS, within = blockIdx.x % a.heads, slab = slabs - 1 - blockIdx.x / a.heads;
+  const uint32_t per = a.heads / a.kv_heads, kv_head = within % a.kv_heads, head = kv_head * per + within / a.kv_heads;
+  const uint32_t p0 = a.state[kStatePosition], slot = a.state[kStateSlot], ld = a.ld, capacity = a.cache.capacity;
+  const uint32_t wave_row = slab * ROWS + wave % WAVES * 32, own = min(wave_row + row_lane, a.m - 1);
+  const __bf16 *qkv = static_cast<const __bf16 *>(a.qkv);
+
+  bf16x8 q[D / 16];
+  const __bf16 *q_row = qkv + (size_t)own * ld + head * D;
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) q[ks] = *reinterpret_cast<const bf16x8 *>(q_row + ks * 16 + half * 8);
+  const uint32_t first_row = p0 + min(wave_row, a.m - 1), last_row = p0 + min(wave_row + 31, a.m - 1);
+  const TurnsBounds bounds = {first_seen(p0 + own, a.cache), p0 + own, first_seen(first_row, a.cache), first_seen(last_row, a.cache),
+                              first_row, last_row};
+  const uint32_t last = p0 + min(slab * ROWS + ROWS, a.m) - 1, begin = first_seen(p0 + slab * ROWS, a.cache);
+
+  const __bf16 *fresh_k = qkv + (a.heads + kv_head) * D, *fresh_v = fresh_k + a.kv_heads * D;
+  const size_t ring = ((size_t)slot * a.kv_heads + kv_head) * capacity * D;
+  const __bf16 *cache_k = static_cast<const __bf16 *>(a.cache.keys) + ring, *cache_v = static_cast<const __bf16 *>(a.cache.values) + ring;
+  const TurnsCopy<D, WAVES, false> k_rows(ld * 2, threadIdx.x);
+  const TurnsCopy<D, WAVES, true> v_rows(ld * 2, threadIdx.x);
+  // a row of a stage that begins before the portion or goes beyond its last row, which is then repeated
+  const auto row_of = [&](const __bf16 *fresh, const __bf16 *cache, uint32_t key, uint32_t r) {
+    const uint32_t j = min(key + r, last);
+    uint32_t at = key % capacity + (j - key);
+    at -= at >= capacity ? capacity : 0;
+    return j < p0 ? cache + (size_t)at * D : fresh + (size_t)(j - p0) * ld;
+  };
+  const auto copy = [&](const auto &rows, const __bf16 *fresh, const __bf16 *cache, uint32_t key, uint32_t stage) {
+    const uint32_t at = key % capacity;
+    if (key >= p0 && key + kTurnsKeys - 1 <= last) {
+      rows.whole(fresh + (size_t)(key - p0) * ld, stage);
+    } else if (key + kTurnsKeys <= p0 && at + kTurnsKeys <= capacity) {
+      uint32_t thread = threadIdx.x;
+      asm volatile("" : "+v"(thread));  // (made anew: these stages are the earlier portions' only)
+      std::decay_t<decltype(rows)>(D * 2, thread).whole(cache + (size_t)at * D, stage);
+    } else {
+      rows.rows([&](uint32_t r) { return row_of(fresh, cache, key, r); }, stage);
+    }
+  };
+  const auto copy_k = [&](uint32_t key, uint32_t stage) { copy(k_rows, fresh_k, cache_k, key, stage); };
+  const auto copy_v = [&](uint32_t key, uint32_t stage) { copy(v_rows, fresh_v, cache_v, key, stage); };
+
+  const bool has_sink = a.sink != nullptr && wave < WAVES;
+  const float sink = has_sink ? (float)reinterpret_cast<const __bf16 *>(a.sink)[head] * kLog2e : -FLT_MAX;
+  const float inner = (SCORES == TurnsScores::kPlain ? a.scale : 2.0f * a.scale / a.softcap) * kLog2e;
+  float top = SCORES == TurnsScores::kFixed ? fmaxf(sink, 0.0f) : sink;
+  float total = has_sink && half == 0 ? exp2_raw(sink - top) : 0.0f;
+  f32x16 out[JJ];
+#pragma unroll
+  for (int jj = 0; jj < JJ; ++jj)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) out[jj][r] = 0.0f;
+  if (!attention_turns<__bf16, D, true, SCORES>(stage_lds, q, bounds, begin, (last - begin) / kTurnsKeys + 1, inner,
+                                                 a.softcap * kLog2e, top, total, out, copy_k, copy_v))
+    return;
+  float low, high;
+  both_halves(total, low, high);
+  const float inverse = a.out_scale / (low + high);
+  if (wave_row >= a.m) return;
+  constexpr int FROM = turns_share_bytes<D>();
+  static_assert(FROM + WAVES * store_rows_bytes<D>() <= turns_lds_bytes<D, true>(), "the rows fit the stages");
+  store_rows<D>(stage_lds + FROM + wave * store_rows_bytes<D>(), static_cast<__bf16 *>(a.out) + (size_t)wave_row * a.ld_out + head * D,
+                (size_t)a.ld_out * 2, a.m - wave_row, [&](int jj, int r) {
+                  bf16x4 packed;
+#pragma unroll
+                  for (int i = 0; i < 4; ++i) packed[i] = (__bf16)(out[jj][r + i] * inverse);
+                  return __builtin_bit_cast(uint2, packed);
+                });
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void chunk_cache_write_kernel(ChunkAttentionArgs a, uint32_t first_row) {
   const uint32_t r = first_row + blockIdx.x;
@@ -452,6 +553,35 @@ hipError_t run_prefill_tile(const ChunkAttentionArgs &a, hipStream_t stream) {
   return run_prefill_kernel<T, ND, NE, WAVES, KS, false>(a, stream);
 }
 
+template <int D, TurnsScores SCORES>
+hipError_t run_turns_kernel(const ChunkAttentionArgs &a, hipStream_t stream) {
+  constexpr int bytes = turns_lds_bytes<D, true>();
+  constexpr uint32_t rows = turns_rows<true>();
+  static bool allowed[kMaxDevices] = {};
+  const auto kernel = chunk_turns_kernel<D, SCORES>;
+  if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
+  kernel<<<a.heads * ((a.m + rows - 1) / rows), 512, bytes, stream>>>(a);
+  return hipGetLastError();
+}
+
+template <int D>
+hipError_t run_turns(const ChunkAttentionArgs &a, hipStream_t stream) {
+  if constexpr (D == 128) {
+    if (a.softcap > 0.0f && a.softcap <= kFixedMaxCap) return run_turns_kernel<D, TurnsScores::kFixed>(a, stream);
+    if (a.softcap > 0.0f) return run_turns_kernel<D, TurnsScores::kCapped>(a, stream);
+  }
+  return run_turns_kernel<D, TurnsScores::kPlain>(a, stream);
+}
+
+// Whole pieces of sixteen bytes, rows that the ring holds a stage of, and maxima taken before the scale.
+bool turns_ok(const ChunkAttentionArgs &a) {
+  const auto aligned = [](const void *p, uint32_t bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; };
+  return !a.f32 && a.dim == a.vdim && chunk_turns(a.dim, a.softcap > 0.0f, a.m, a.cache.span) && a.cache.capacity >= kTurnsKeys &&
+         a.ld % 8 == 0 && a.ld < (1u << 24) && a.ld_out % 4 == 0 && aligned(a.qkv, 16) && aligned(a.cache.keys, 16) &&
+         aligned(a.cache.values, 16) && aligned(a.out, 8) && (a.softcap > 0.0f || (a.scale > 0.0f && a.scale < INFINITY)) &&
+         (uint64_t)a.heads * ((a.m + 127) / 128) <= 0x7fffffffull;
+}
+
 // A wave's registers hold 16 query rows of heads up to 128 twice a SIMD beside a second workgroup (bfloat16); wider
 // heads and float32 leave room for four waves.  Eight waves are 128 rows, or 64 rows of which each half of the waves
 // takes half the keys of a stage: twice the workgroups, half the chain.  That is the better one while 128-row tiles
@@ -473,6 +603,9 @@ hipError_t run_prefill(const ChunkAttentionArgs &a, hipStream_t stream) {
 
 template <typename T, int ND, int NE>
 hipError_t run_attention(const ChunkAttentionArgs &a, hipStream_t stream) {
+  if constexpr (sizeof(T) == 2 && ((ND == 2 && NE == 4) || (ND == 4 && NE == 8))) {
+    if (a.m > 1 && turns_ok(a)) return run_turns<ND * 32>(a, stream);
+  }
   if (a.m > 1) return run_prefill<T, ND, NE>(a, stream);
   return a.row ? run_decode<T, ND, NE, true>(a, stream) : run_decode<T, ND, NE, false>(a, stream);
 }

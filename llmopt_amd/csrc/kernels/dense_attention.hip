@@ -725,6 +725,7 @@ __global__ __launch_bounds__(256) void tree_mask_kernel(TreeMaskArgs a) {
 template <>
 struct TurnsOperand<_Float16> {
   typedef h8_t x8;
+  static constexpr int kProducts = 1;
   struct Weights {
     x8 v;
     __device__ __forceinline__ void set_pair(int i, float x, float y) { v[i] = (_Float16)x, v[i + 1] = (_Float16)y; }
@@ -771,8 +772,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const uint32_t value_stride = a.token_first_value ? kv_heads * D : D;
   const uint16_t *values = a.value + (a.token_first_value ? ((size_t)batch * L * kv_heads + kv_head) * D
                                                           : ((size_t)batch * kv_heads + kv_head) * L * D);
-  const TurnsCopy<D, WAVES, false> k_rows(D * 2);
-  const TurnsCopy<D, WAVES, true> v_rows(value_stride * 2);
+  const TurnsCopy<D, WAVES, false> k_rows(D * 2, threadIdx.x);
+  const TurnsCopy<D, WAVES, true> v_rows(value_stride * 2, threadIdx.x);
   const auto copy_k = [&](uint32_t key, uint32_t stage) {
     if (key + kTurnsKeys <= L) k_rows.whole(keys + (size_t)key * D, stage);
     else k_rows.rows([&](uint32_t r) { return keys + (size_t)min(key + r, L - 1) * D; }, stage);

@@ -43,4 +43,16 @@ inline TurnsForm turns_form(uint32_t head_dim, bool masked, uint32_t query_lengt
   return 4 * workgroups > (head_dim == 64 ? 3 : 1) * (uint64_t)cus ? TurnsForm::kSplit : TurnsForm::kNone;
 }
 
+// The same over a portion of a prompt in bfloat16, 128 rows and their keys shared.  A workgroup starts and ends in some 8 us of
+// which nothing overlaps, so that it pays for long walks; how long is known from the rows and the span alone (earlier portions'
+// keys only make it longer).  us, heads x rows of span, turns / 16-row tiles: heads of 128 16 x 3001 of 2048 75 / 96, 32 x 3001 of
+// 1024 102 / 118, 16 x 700 28 / 31, 16 x 500 25.1 / 25.8, 32 x 1500 of 512 54.5 / 53.9; of 64 16 x 3001 of 2048 51 / 60, 16 x 1500
+// 33 / 37, 16 x 3001 of 1024 46.6 / 45.6.  A cap's two more exponentials a score hide better behind four waves a SIMD: heads of
+// 128 32 x 2048 74 / 90, 32 x 3001 of 1024 70 / 80, 32 x 1000 34 / 34, 32 x 2000 of 512 40 / 35; of 64 16 x 2048 41 / 40.
+inline bool chunk_turns(uint32_t dim, bool capped, uint32_t m, uint32_t span) {
+  const uint32_t walk = span != 0 && span < m ? span : m;
+  if (dim == 128) return walk > (capped ? 1000 : 512);
+  return dim == 64 && !capped && walk > 1024;
+}
+
 }  // namespace llmopt

@@ -89,6 +89,20 @@ def test_tiles(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sli
         assert (error <= 2.0 ** -8 * np.abs(expected) + 2.0 ** -13 * np.abs(values).max()).all(), (head, error.max())
 
 
+@pytest.mark.parametrize("m,heads,kv,dim,vdim,span,softcap,sink,first,sliding", [
+    (513, 4, 2, 128, 128, 4096, 0.0, True, 0, False),         # one key more than eight stages
+    (1100, 4, 1, 128, 128, 1500, 0.0, True, 1437, False),     # a chunk's end in the second tile
+    (640, 2, 2, 128, 128, 700, 0.0, False, 2000, True),       # a window whose ring has turned
+    (1001, 3, 3, 128, 128, 1007, 30.0, True, 940, False),     # bounded scores, stages across the ring's end
+    (1025, 2, 1, 128, 128, 4096, 50.0, True, 63, False),
+    (1061, 4, 2, 64, 64, 1040, 0.0, False, 1000, True),
+    (1030, 6, 2, 64, 64, 2048, 0.0, True, 1, False),
+])
+def test_groups_of_waves_in_turns(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sliding):
+    """Portions whose rows walk over many keys: 128 rows whose stages two groups of waves share."""
+    test_tiles(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sliding)
+
+
 # rows, heads, kv_heads, dim, span, position of the first row: tiles in the order of their keys (several rounds of up to 64
 # tiles, a chunk's end among them: 5, 16 and 64 tiles), more tiles than are ranked, one chunk, one round
 @pytest.mark.parametrize("m,heads,kv,dim,span,first", [

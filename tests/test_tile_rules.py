@@ -6,7 +6,8 @@ import subprocess
 
 import pytest
 
-from tests import test_gpu_delta_chunks, test_gpu_dense_attention, test_gpu_dense_tiles, test_gpu_w4a16_rows
+from tests import (test_gpu_attention_tiles, test_gpu_delta_chunks, test_gpu_dense_attention, test_gpu_dense_tiles,
+                   test_gpu_w4a16_rows)
 
 CUS = 256
 KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "kernels")
@@ -27,6 +28,7 @@ int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, ui
 int turns(uint32_t dim, uint32_t masked, uint32_t rows, uint32_t keys, uint32_t heads, uint32_t cus) {
   return (int)turns_form(dim, masked != 0, rows, keys, (uint64_t)((rows + 127) / 128) * heads, cus);
 }
+int chunked(uint32_t dim, uint32_t capped, uint32_t m, uint32_t span) { return chunk_turns(dim, capped != 0, m, span); }
 int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
   return three_delta_workgroups((tokens + 63) / 64 * heads, cus);
 }
@@ -168,6 +170,20 @@ def test_gpu_tests_reach_both_forms_of_turns(rules):
     reached = [(dim, rules.turns(dim, 0, new, new + past, heads * batches, CUS))
                for dim, batches, heads, _, new, past, _ in sizes(test_gpu_dense_attention.test_groups_of_waves_in_turns, names)]
     assert set(reached) == {(64, 1), (64, 2), (128, 1), (128, 2)}
+
+
+@pytest.mark.parametrize("dim,capped,m,span,turns", [
+    (128, 0, 3001, 2048, 1), (128, 0, 513, 0, 1), (128, 0, 1500, 512, 0), (128, 0, 500, 2048, 0), (128, 1, 2048, 2048, 1),
+    (128, 1, 3001, 1024, 1), (128, 1, 1000, 2048, 0), (128, 1, 2000, 512, 0), (64, 0, 1500, 2048, 1), (64, 0, 3001, 1024, 0),
+    (64, 1, 3001, 2048, 0), (96, 0, 3001, 2048, 0), (256, 0, 3001, 2048, 0)])
+def test_portions_in_turns(rules, dim, capped, m, span, turns):
+    assert rules.chunked(dim, capped, m, span) == turns
+
+
+def test_gpu_tests_of_portions_go_in_turns(rules):
+    for m, _, _, dim, _, span, softcap, *_ in sizes(test_gpu_attention_tiles.test_groups_of_waves_in_turns,
+                                                    "m,heads,kv,dim,vdim,span,softcap,sink,first,sliding"):
+        assert rules.chunked(dim, int(softcap > 0), m, span) == 1
 
 
 @pytest.mark.parametrize("tokens,heads,three", [(3001, 16, 1), (2115, 16, 1), (4096, 32, 1), (3001, 32, 1), (3001, 8, 0),
