@@ -9,6 +9,8 @@ include/llmopt_hip.h.  hipcc cross-compiles without a GPU.
 retained plans, the entry points, the operator mirror, the sampler) traps on undefined behaviour
 and out-of-bounds array indices; the GPU code is the same.  Run the tests against it with
 LLMOPT_HIP_LIBRARY=llmopt_amd/libllmopt_hip_ubsan.so: a trap ends the process with SIGILL.
+
+libllmopt_torch.so, the native side of torch_ops, is built beside it where torch is installed.
 """
 from __future__ import annotations
 
@@ -22,6 +24,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(CSRC, "build")
 LIBRARY = os.path.join(HERE, "libllmopt_hip.so")
+TORCH_SOURCE = os.path.join(CSRC, "torch", "linear_op.cpp")
+TORCH_LIBRARY = os.path.join(HERE, "libllmopt_torch.so")
 UBSAN_BUILD = os.path.join(CSRC, "build", "ubsan")
 UBSAN_LIBRARY = os.path.join(HERE, "libllmopt_hip_ubsan.so")
 # host pass only (each -fsanitize option directly behind -Xarch_host): no runtime library needed
@@ -80,11 +84,34 @@ def _compile(source: str, force: bool, host_ubsan: bool = False) -> str:
     return obj
 
 
+def _build_torch(force: bool) -> None:
+    """The operator's kernel against the installed torch; without one there is no operator either."""
+    try:
+        import torch
+        from torch.utils import cpp_extension
+    except ImportError:
+        return
+    newest = max(os.path.getmtime(p) for p in (TORCH_SOURCE, os.path.abspath(__file__), torch.__file__))
+    if not force and os.path.exists(TORCH_LIBRARY) and os.path.getmtime(TORCH_LIBRARY) >= newest:
+        return
+    libraries = os.path.join(os.path.dirname(torch.__file__), "lib")
+    command = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+               *(f"-isystem{path}" for path in cpp_extension.include_paths() + [os.path.join(cpp_extension.ROCM_HOME, "include")]),
+               TORCH_SOURCE, "-o", TORCH_LIBRARY,
+               f"-L{libraries}", "-lc10", "-lc10_hip", "-ltorch_cpu"]
+    result = subprocess.run(command, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"g++ failed for {TORCH_SOURCE}:\n{result.stderr}")
+
+
 def build(force: bool = False, host_ubsan: bool = False) -> str:
     os.makedirs(UBSAN_BUILD if host_ubsan else BUILD, exist_ok=True)
     library = UBSAN_LIBRARY if host_ubsan else LIBRARY
     with concurrent.futures.ThreadPoolExecutor(max_workers=6) as pool:
+        beside = pool.submit(_build_torch, force)
         objects = list(pool.map(lambda s: _compile(s, force, host_ubsan), sources()))
+        beside.result()
     newest = max(os.path.getmtime(o) for o in objects)
     if force or not os.path.exists(library) or os.path.getmtime(library) < newest:
         command = ["hipcc", "-shared", "-fPIC", "--offload-arch=gfx950", "-fno-gpu-sanitize",

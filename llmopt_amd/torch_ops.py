@@ -6,7 +6,8 @@ in the `llmopt` namespace (python/llmopt_backend/quantization.py:174-185) and
 backs it with its native runtime (native/metal_runtime.cpp:139-147).  This
 module registers the same schema for ROCm tensors: the kernel runs on the
 tensors' own device memory (no copies), is queued on torch's current stream
-and nothing waits for it.
+and nothing waits for it.  Calls with nothing to refuse or lay out anew are native
+code from torch's dispatcher on (csrc/torch/linear_op.cpp); the others come here.
 
     import llmopt_amd.torch_ops            # registers the operator
     y = torch.ops.llmopt.w4a16_linear(x, packed, scale, bias)
@@ -16,18 +17,22 @@ activations and bias, uint8 `[N, K/2]` weights, fp16 `[N, K/64]` scales.
 """
 from __future__ import annotations
 
+import ctypes
+import os
 import struct
 import threading
 from typing import Optional
 
 import torch
 
-from .native import Runtime
+from .native import Runtime, lib
 
 GROUP_SIZE = 64
 _ONE_ROW, _ROWS = b"llmopt_w4a16_linear_f16_g64", b"llmopt_w4a16_linear_f16_g64_m4"
 _PARAMETERS = struct.Struct("<5I").pack  # m, n, k, has_bias, bias_row_stride
+_NATIVE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libllmopt_torch.so")
 _library: Optional[torch.library.Library] = None
+_native: Optional[ctypes.CDLL] = None
 _runtimes: dict[int, Runtime] = {}
 _lock = threading.Lock()
 
@@ -41,6 +46,8 @@ def _runtime(device_index: int) -> Runtime:
         if runtime is None:
             runtime = Runtime(device=device_index)
             _runtimes[device_index] = runtime
+            # further calls on this device that need nothing but the launch no longer come here
+            _native.llmopt_torch_bind(device_index, runtime.library, ctypes.cast(lib().llmopt_hip_launch, ctypes.c_void_p))
         return runtime
 
 
@@ -93,14 +100,21 @@ def _w4a16_linear_meta(input, packed_weight, scale, bias=None):
 
 def register() -> None:
     """Defines `llmopt::w4a16_linear` (once) with a ROCm implementation and a meta kernel."""
-    global _library
+    global _library, _native
     if _library is not None:
         return
+    if not os.path.exists(_NATIVE_PATH):
+        raise ImportError(f"{_NATIVE_PATH} is missing: build it with `python -m llmopt_amd.build`")
     library = torch.library.Library("llmopt", "DEF")
     library.define("w4a16_linear(Tensor input, Tensor packed_weight, Tensor scale, Tensor? bias) -> Tensor")
-    library.impl("w4a16_linear", _w4a16_linear_hip, "CUDA")  # ROCm tensors carry the CUDA dispatch key
+    # what the native kernel of the above leaves to Python
+    library.define("w4a16_linear_general(Tensor input, Tensor packed_weight, Tensor scale, Tensor? bias) -> Tensor")
+    library.impl("w4a16_linear_general", _w4a16_linear_hip, "CUDA")  # ROCm tensors carry the CUDA dispatch key
     library.impl("w4a16_linear", _w4a16_linear_meta, "Meta")
-    _library = library
+    native = ctypes.CDLL(_NATIVE_PATH)  # (its kernel registers itself as it is loaded)
+    native.llmopt_torch_bind.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    native.llmopt_torch_bind.restype = None
+    _library, _native = library, native
 
 
 register()

@@ -121,3 +121,35 @@ def test_a_stream_under_capture_is_refused(op, same):
         torch.cuda.synchronize()
         assert torch.equal(y, x + 1)
         assert_close_to_oracle(op(*tensors).cpu().numpy(), oracle.w4a16_linear(*case[:3], None), "after the capture")
+
+
+@pytest.mark.parametrize("layout", ["plain", "strided input", "strided weights", "offset input", "bias of two dimensions", "vector"])
+def test_native_calls_and_those_left_to_python(op, layout):
+    """Once a device has a runtime, calls that need nothing but the launch never reach Python; the others give the same."""
+    from llmopt_amd.native import LlmoptError
+    rng = np.random.default_rng(11)
+    device = torch.device("cuda:0")
+    case = w4_case(rng, 4, 96, 128, bias=True)
+    x, packed, scale, bias = (torch.from_numpy(a).to(device) for a in case)
+    op(x, packed, scale, bias)
+    if layout == "strided input":
+        x = torch.cat([x, x], dim=1)[:, :128]
+    elif layout == "strided weights":
+        packed, scale = torch.cat([packed, packed], dim=1)[:, :64], scale.t().contiguous().t()
+    elif layout == "offset input":
+        x = torch.cat([x, x])[4:]
+    elif layout == "bias of two dimensions":
+        bias = bias.reshape(2, 48)
+    elif layout == "vector":
+        x = x[0]
+    for _ in range(2):
+        out = op(x, packed, scale, bias)
+        assert out.shape == (*x.shape[:-1], 96) and out.is_contiguous()
+        want = oracle.w4a16_linear(*case)
+        assert_close_to_oracle(out.cpu().numpy().reshape(-1, 96), want[:1] if layout == "vector" else want, layout)
+    with pytest.raises(ValueError, match="features"):
+        op(x[..., :64].contiguous(), packed, scale, bias)
+    with pytest.raises(TypeError, match="bias must be"):
+        op(x, packed, scale, bias.float())
+    with pytest.raises(LlmoptError):
+        op(x.new_zeros((3, 64)), packed.new_zeros((0, 32)), scale.new_zeros((0, 1)), None)
