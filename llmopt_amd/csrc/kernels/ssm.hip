@@ -288,13 +288,22 @@ struct StateOperands {
   float end;
 };
 
+// What `uniform` points at, `bytes` further on in this lane: scalar addresses and one offset.
+template <typename P>
+__device__ __forceinline__ const P *lane_at(const void *uniform, uint32_t bytes) {
+  return reinterpret_cast<const P *>(static_cast<const char *>(uniform) + bytes);
+}
+
 // The serial part: a workgroup owns 16 state rows of one head, its waves the 16-column tiles wave + 4 t
 // (state_size <= 64 NT); the chunks' incoming states go to the workspace.  No exchange between waves.
+// Bound by what a wave issues in turn: a chunk's fourteen requests and 250 vector instructions, most for the high and low parts of
+// the inputs and of the state.  2048 tokens, 64 heads of 64 rows, 128 columns: 36.4 us; with an address of its own per lane and
+// request and an exit behind every chunk, 40.0.  (Without the requests it takes 25.5, without the stores 30.2.)
 template <typename T, int NT>
 __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspace w) {
   const uint32_t head = blockIdx.x, v0 = blockIdx.y * 16, group = head / (a.heads / a.groups);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, column = lane & 15, quad = lane >> 4;
-  const uint32_t n = a.state_size, slot = a.step[kStateSlot];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, column = lane & 15, quad = lane >> 4;
+  const uint32_t n = a.state_size, slot = a.step[kStateSlot], tiles = w.np / 16;
   const bool fresh = a.step[kStatePosition] == 0;
   const size_t ld = (size_t)a.groups * w.np;
   // lane: state row v, columns k .. k + 3 of every tile; rows beyond the head's end repeat its last one
@@ -310,37 +319,42 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
       state[t][r] = !fresh && k < n ? saved[k] : 0.0f;
     }
 
-  auto load = [&](StateOperands<T, NT> &o, uint32_t chunk) {
-    const T *x = static_cast<const T *>(w.xt) + ((size_t)chunk * w.inner + head * a.vdim + v_row) * Q + quad * 8;
-    const float *tail = w.tail + ((size_t)chunk * a.heads + head) * Q + quad * 8;
+  const uint32_t x_at = (v_row * Q + quad * 8) * sizeof(T), b_at = (column * Q + quad * 8) * sizeof(T), tail_at = quad * 32;
+  auto load = [&](StateOperands<T, NT> &o, uint32_t chunk) __attribute__((always_inline)) {
+    const T *x = static_cast<const T *>(w.xt) + ((size_t)chunk * w.inner + head * a.vdim) * Q;
+    const float *tail = w.tail + ((size_t)chunk * a.heads + head) * Q;
     o.end = w.sum[((size_t)chunk * a.heads + head) * 2 * Q + Q - 1];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      o.x[s] = *reinterpret_cast<const Frag<T> *>(x + s * 32);
-      o.tail[s] = *reinterpret_cast<const f32x8 *>(tail + s * 32);
+      o.x[s] = *lane_at<Frag<T>>(x + s * 32, x_at);
+      o.tail[s] = *lane_at<f32x8>(tail + s * 32, tail_at);
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if ((wave + 4 * t) * 16 < (int)w.np)
-          o.b[t][s] = *reinterpret_cast<const Frag<T> *>(
-              static_cast<const T *>(w.bt) +
-              ((size_t)chunk * ld + group * w.np + (wave + 4 * t) * 16 + column) * Q + s * 32 + quad * 8);
+      for (int t = 0; t < NT; ++t)  // (a tile that is not there: the last again)
+        o.b[t][s] = *lane_at<Frag<T>>(static_cast<const T *>(w.bt) +
+                                          ((size_t)chunk * ld + group * w.np + min((uint32_t)wave + 4 * t, tiles - 1) * 16) * Q + s * 32,
+                                      b_at);
     }
   };
-  auto step = [&](const StateOperands<T, NT> &o, uint32_t chunk) {
+  auto step = [&](const StateOperands<T, NT> &o, uint32_t chunk) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const uint32_t k = (wave + 4 * t) * 16;
-      if (k >= w.np) continue;
+      if ((uint32_t)wave + 4 * t >= tiles) continue;
       typedef T x4 __attribute__((ext_vector_type(4)));
-      x4 high, low;
+      const uint32_t at = (wave + 4 * t) / 2 * 512 + (((wave + 4 * t) % 2 * 2 + quad / 2) * 16 + column) * 8 + quad % 2 * 4;
+      x4 high;
+      if constexpr (kStatePlanes<T> == 2) {
+        WideFrag<T> pairs;
+        pairs.set_pair(0, state[t][0], state[t][1]);
+        pairs.set_pair(2, state[t][2], state[t][3]);
+        x4 low;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        high[r] = (T)state[t][r];
-        low[r] = (T)(state[t][r] - (float)high[r]);
+        for (int r = 0; r < 4; ++r) high[r] = pairs.hi[r], low[r] = pairs.lo[r];
+        *reinterpret_cast<x4 *>(state_block<T>(a, w, chunk, head, 1, v0) + at) = low;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) high[r] = state[t][r];
       }
-      const uint32_t at = k / 32 * 512 + ((k / 16 % 2 * 2 + quad / 2) * 16 + column) * 8 + quad % 2 * 4;
       *reinterpret_cast<x4 *>(state_block<T>(a, w, chunk, head, 0, v0) + at) = high;
-      if (kStatePlanes<T> == 2) *reinterpret_cast<x4 *>(state_block<T>(a, w, chunk, head, 1, v0) + at) = low;
     }
     const float carry = __expf(o.end);
 #pragma unroll
@@ -351,26 +365,28 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
     for (int s = 0; s < 2; ++s) {
       WideFrag<T> fx;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) fx.set(e, to_f32(o.x[s][e]) * o.tail[s][e]);
+      for (int e = 0; e < 8; e += 2) fx.set_pair(e, to_f32(o.x[s][e]) * o.tail[s][e], to_f32(o.x[s][e + 1]) * o.tail[s][e + 1]);
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-        if ((wave + 4 * t) * 16 < (int)w.np) state[t] = mma_wide_b(o.b[t][s], fx, state[t]);
+      for (int t = 0; t < NT; ++t) state[t] = mma_wide_b(o.b[t][s], fx, state[t]);
     }
   };
 
-  // operands two chunks ahead
+  // operands two chunks ahead (one exit from the loop: with one behind every step the compiler waits for all requests at its head)
   StateOperands<T, NT> ring[3];
   load(ring[0], 0);
   load(ring[1], min(1u, w.chunks - 1));
-  for (uint32_t chunk = 0; chunk < w.chunks; chunk += 3) {
+  uint32_t chunk = 0;
+  for (; chunk + 3 <= w.chunks; chunk += 3) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      if (chunk + i >= w.chunks) break;
       load(ring[(i + 2) % 3], min(chunk + i + 2, w.chunks - 1));
       __builtin_amdgcn_sched_barrier(0);  // the requests stay ahead of the arithmetic
       step(ring[i], chunk + i);
     }
   }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (chunk + i < w.chunks) step(ring[i], chunk + i);
   if (v < a.vdim)
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -387,7 +403,7 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
 template <typename T, int STEPS>
 __global__ __launch_bounds__(256) void ssm_output_kernel(SsmArgs a, SsmWorkspace w) {
   const uint32_t chunk = blockIdx.x, head = blockIdx.y, group = head / (a.heads / a.groups);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, column = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, column = lane & 15, quad = lane >> 4;
   const size_t ld = (size_t)a.groups * w.np;
   const int token = wave * 16 + column;  // of the lane's output column
   const uint32_t row = chunk * Q + token;
@@ -415,21 +431,34 @@ __global__ __launch_bounds__(256) void ssm_output_kernel(SsmArgs a, SsmWorkspace
     }
   }
   const float scale = __expf(own_high);
+  const uint32_t lane_bytes = lane * 8 * sizeof(T);
+  const T *x_head = static_cast<const T *>(w.xt) + ((size_t)chunk * w.inner + head * a.vdim) * Q;
   for (uint32_t v0 = blockIdx.z * 16; v0 < a.vdim; v0 += gridDim.z * 16) {
-    const uint32_t v_row = min(v0 + column, a.vdim - 1);
+    // A tile's operands are requested together, at scalar addresses: 31.4 us at the sizes above, where each request waited in front
+    // of its product 35.3.  (The next tile's as well: 34.4, fewer waves fit; two workgroups over a head's tiles: 42.3.)
+    Frag<T> state[kStatePlanes<T>][STEPS], x[2];
+#pragma unroll
+    for (int plane = 0; plane < kStatePlanes<T>; ++plane) {
+      const T *from = state_block<T>(a, w, chunk, head, plane, v0);
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s)
+        if (s * 32 < (int)w.np) state[plane][s] = *lane_at<Frag<T>>(from + s * 512, lane_bytes);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+      x[s] = *lane_at<Frag<T>>(x_head + s * 32, (min(v0 + column, a.vdim - 1) * Q + quad * 8) * sizeof(T));
+    __builtin_amdgcn_sched_barrier(0);  // the requests stay ahead of the arithmetic
     f32x4 high = {0.0f, 0.0f, 0.0f, 0.0f}, low = high, within = high;
 #pragma unroll
     for (int s = 0; s < STEPS; ++s)
       if (s * 32 < (int)w.np) {
-        high = mma(reinterpret_cast<const Frag<T> *>(state_block<T>(a, w, chunk, head, 0, v0))[s * 64 + lane], fc[s], high);
-        if (kStatePlanes<T> == 2)
-          low = mma(reinterpret_cast<const Frag<T> *>(state_block<T>(a, w, chunk, head, 1, v0))[s * 64 + lane], fc[s], low);
+        high = mma(state[0][s], fc[s], high);
+        if constexpr (kStatePlanes<T> == 2) low = mma(state[1][s], fc[s], low);
       }
-    const T *x = static_cast<const T *>(w.xt) + ((size_t)chunk * w.inner + head * a.vdim + v_row) * Q + quad * 8;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
       if (s * 32 <= wave * 16 + 15)  // the others come later than all of the wave's tokens
-        within = mma_wide_b(*reinterpret_cast<const Frag<T> *>(x + s * 32), weight[s], within);
+        within = mma_wide_b(x[s], weight[s], within);
     if (row >= a.m) continue;
     T *out = static_cast<T *>(a.y) + (size_t)row * w.inner + head * a.vdim + v0 + quad * 4;
     typedef T x4 __attribute__((ext_vector_type(4)));
