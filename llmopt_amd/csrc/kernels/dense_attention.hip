@@ -122,6 +122,7 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
                 "stage");
   static_assert(!KEYSPLIT || STAGE_KEYS == 32 * WAVES, "a tile of every stage per wave");
   constexpr int ROWS = KEYSPLIT ? 32 : WAVES * 32;  // query rows per workgroup
+  constexpr bool OWN_STAGES = KEYSPLIT && !MASKED;  // (a loop of their own)
   extern __shared__ __attribute__((aligned(16))) unsigned char stage_lds[];  // [group][2 stages][K | V]
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave_of_all = threadIdx.x >> 6;
@@ -151,19 +152,20 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
       taken = start + a.cus_per_xcd + (run - 1 - within);
     rank = taken * 8 + xcd;
   }
-  const uint32_t slab = longest_first ? slabs - 1 - rank / per_slab : rank / per_slab;
-  const uint32_t head = rank % per_slab % a.heads;
-  const uint32_t batch = rank % per_slab / a.heads;
+  const uint32_t in_order = rank / per_slab, in_slab = rank - in_order * per_slab;
+  const uint32_t slab = longest_first ? slabs - 1 - in_order : in_order;
+  const uint32_t batch = a.batches == 1 ? 0 : in_slab / a.heads;
+  const uint32_t head = in_slab - batch * a.heads;
   const uint32_t q0 = KEYSPLIT ? slab * 32 : (slab * WAVES + wave) * 32;
   const bool has_rows = q0 < a.query_length;  // a wave without rows still copies and meets the barriers
   const uint32_t kv_heads = a.kv_heads > 0 ? a.kv_heads : a.heads;
-  const uint32_t kv_head = kv_heads < a.heads ? head / (a.heads / kv_heads) : head;
+  const uint32_t kv_head = kv_heads < a.heads ? head * kv_heads / a.heads : head;  // (the heads divide over them)
   constexpr bool masked = MASKED;
   const uint32_t L = a.key_length;
 
   // B operand of the score MFMAs: Q[row = row_lane][d = ks * 16 + half * 8 ..]; rows past the end repeat the last
   h8_t q_frag[KSTEPS];
-  {
+  if constexpr (!OWN_STAGES) {
     const uint32_t row = min(q0 + row_lane, a.query_length - 1);
     const uint16_t *q_row = a.query + (((size_t)batch * a.heads + head) * a.query_length + row) * D;
 #pragma unroll
@@ -365,7 +367,7 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
   const uint32_t steps = PAIR ? (walk + 1) / 2 : walk;
   auto walk_index = [&](uint32_t step) __attribute__((always_inline)) { return PAIR ? 2 * step + group : step; };
   MaskRaw mask_raw[TILES];
-  if (walk > 0) {
+  if (!OWN_STAGES && walk > 0) {
     if (walk_index(0) < walk) {
       const uint32_t first = stage_at(walk_index(0));
       if constexpr (MASKED) {
@@ -395,12 +397,12 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
   // softmax update and P V product of one tile from its scores; v_tile = its first V row in the stage
   auto tile_update = [&](uint32_t key0, f16x_t score, const unsigned char *v_tile, uint32_t allowed_bits)
                          __attribute__((always_inline)) {
-    // a tile of existing keys, all below the causal limit of the wave's first row, of existing
-    // rows and without a mask needs no per-score test.  Maxima are taken over the scores as the MFMAs left them; the
+    // a tile of existing keys, all below the causal limit of the wave's first row and without a mask
+    // needs no per-score test (rows past the end repeat the last, and nothing stores them).  Maxima are taken over the scores as the MFMAs left them; the
     // scale (positive) goes into the exponent's multiply-add.
     // (with a mask: when it allows all 32 x 32 scores of the tile)
     const bool interior = (!masked || __builtin_amdgcn_ballot_w64(allowed_bits != 0xffffu) == 0) && key0 + 32 <= L &&
-                          q0 + 32 <= a.query_length && (!a.causal || key0 + 31 <= a.past_length + q0);
+                          (!a.causal || key0 + 31 <= a.past_length + q0);
     float tile_max = -INFINITY;
     if (interior) {
 #pragma unroll
@@ -410,7 +412,7 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const uint32_t key = key0 + (r >> 2) * 8 + half * 4 + (r & 3);
-        bool allowed = key < L && row < a.query_length;
+        bool allowed = key < L;
         if (a.causal) allowed = allowed && key <= a.past_length + row;
         if constexpr (masked) allowed = allowed && ((allowed_bits >> r) & 1u) != 0;
         score[r] = allowed ? score[r] : -INFINITY;
@@ -455,9 +457,89 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
       }
   };
 
+  if constexpr (OWN_STAGES) {
+    // A wave copies the 32 keys of a stage that it works on and nobody else's: its tiles need no barrier.  A launch this small is
+    // as long as the trips to memory that wait for each other, so three tiles are asked for at once: two into LDS, where there
+    // is room for two, and the third into registers, which go to the first one's place when it is read.  The query rows come
+    // through LDS as well: loads into registers would be waited for with everything asked for before them.
+    // us, stages shared at a barrier / this: nine heads of 64, 700 rows 10.8 / 8.1 (0.6 of it the copies, 2 the meeting of the
+    // shares and no tests of scores for rows past the end), 16 of 128, 500 rows 12.8 / 9.4, 4 of 64, 4096 rows 31.1 / 25.5.  Without the
+    // copies the first takes 6.3, without the products 5.3.
+    const uint32_t own = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
+    const uint32_t mine = key_end > own * 32 ? (key_end - own * 32 + STAGE_KEYS - 1) / STAGE_KEYS : 0;
+    const uint32_t row_in_copy = lane / PIECES, piece = lane % PIECES;
+    const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) unsigned char *)stage_lds;
+    const auto copy = [](const void *base, uint32_t offset, uint32_t target) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "s"(target) : "memory");
+#endif
+    };
+    // rows of 32 from `first` on, those past the last again: where copy c of them reads (the piece XOR-ed by `times` the row)
+    const auto offset_of = [&](int c, uint32_t stride, uint32_t last, uint32_t times, uint32_t mask) __attribute__((always_inline)) {
+      const uint32_t local = c * KEYS_PER_COPY + row_in_copy;
+      return min(row_in_copy * stride + c * KEYS_PER_COPY * stride, last * stride) + ((piece ^ (times * local & mask)) * 16);
+    };
+    const uint32_t k_stride = ROW_BYTES, v_stride = (uint32_t)value_row_stride * 2;
+    const auto for_tile = [&](uint32_t t, auto &&each_k, auto &&each_v) __attribute__((always_inline)) {
+      const uint32_t first = t * STAGE_KEYS + own * 32, last = min(31u, L - 1 - first);
+      const char *k = reinterpret_cast<const char *>(key_base) + (size_t)first * k_stride;
+      const char *v = reinterpret_cast<const char *>(value_base) + (size_t)first * v_stride;
+#pragma unroll
+      for (int c = 0; c < COPIES; ++c) each_k(c, k, offset_of(c, k_stride, last, 1, PIECES - 1));
+#pragma unroll
+      for (int c = 0; c < COPIES; ++c) each_v(c, v, offset_of(c, v_stride, last, 2, VMASK));
+    };
+    const auto copy_tile = [&](uint32_t t) __attribute__((always_inline)) {
+      const uint32_t k_target = lds_base + (t & 1) * 2 * STAGE_BYTES + own * COPIES * 1024;
+      for_tile(t, [&](int c, const char *k, uint32_t at) __attribute__((always_inline)) { copy(k, at, k_target + c * 1024); },
+               [&](int c, const char *v, uint32_t at) __attribute__((always_inline)) { copy(v, at, k_target + STAGE_BYTES + c * 1024); });
+    };
+    constexpr int Q_COPIES = 32 / KEYS_PER_COPY;
+    unsigned char *q_lds = stage_lds + 4 * STAGE_BYTES;
+#pragma unroll
+    for (int c = 0; c < (Q_COPIES + WAVES - 1) / WAVES; ++c) {
+      const uint32_t at = c * WAVES + own, row = at * KEYS_PER_COPY + row_in_copy;
+      if (at < Q_COPIES)
+        copy(a.query + (((size_t)batch * a.heads + head) * a.query_length + q0) * D,
+             min(row, a.query_length - 1 - q0) * ROW_BYTES + ((piece ^ (row & (PIECES - 1))) * 16),
+             lds_base + 4 * STAGE_BYTES + at * 1024);
+    }
+    if (mine > 0) copy_tile(0);
+    if (mine > 1) copy_tile(1);
+    typedef uint32_t piece_t __attribute__((ext_vector_type(4)));
+    piece_t third_k[COPIES], third_v[COPIES];
+    if (mine > 2)
+      for_tile(2, [&](int c, const char *k, uint32_t at) __attribute__((always_inline)) { third_k[c] = *reinterpret_cast<const piece_t *>(k + at); },
+               [&](int c, const char *v, uint32_t at) __attribute__((always_inline)) { third_v[c] = *reinterpret_cast<const piece_t *>(v + at); });
+    // (what is younger than tile 0 are tile 1's copies and perhaps the loads of tile 2, which are the compiler's to place)
+    if (mine > 1) copies_landed<2 * COPIES>();
+    else copies_landed<0>();
+    meet();  // the query rows
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks)
+      q_frag[ks] = *reinterpret_cast<const h8_t *>(q_lds + row_lane * ROW_BYTES + (((ks * 2 + half) ^ (row_lane & (PIECES - 1))) * 16));
+    for (uint32_t t = 0; t < mine; ++t) {
+      if (t > 0) {
+        if (t + 1 < mine) copies_landed<2 * COPIES>();
+        else copies_landed<0>();
+      }
+      unsigned char *k_tile = stage_lds + (t & 1) * 2 * STAGE_BYTES + own * 32 * ROW_BYTES;
+      tile_update(t * STAGE_KEYS + own * 32, tile_scores(k_tile, own * 32), k_tile + STAGE_BYTES, 0xffffu);
+      lds_read();  // the tile's place is free
+      if (t == 0 && mine > 2) {
+#pragma unroll
+        for (int c = 0; c < COPIES; ++c) {
+          *reinterpret_cast<piece_t *>(k_tile + c * 1024 + lane * 16) = third_k[c];
+          *reinterpret_cast<piece_t *>(k_tile + STAGE_BYTES + c * 1024 + lane * 16) = third_v[c];
+        }
+      }
+      if (t > 0 && t + 2 < mine) copy_tile(t + 2);
+    }
+    __syncthreads();
+  }
   // The tiles of a stage.  Two: both score chains go to the matrix pipe first, so the second runs
   // while the vector unit works on the first tile's softmax.
-  for (uint32_t step = 0; step < steps; ++step) {
+  for (uint32_t step = 0; step < (OWN_STAGES ? 0 : steps); ++step) {
     const uint32_t index = walk_index(step);
     const bool active = index < walk;  // (PAIR: the last step may have an entry for group 0 only)
     const uint32_t stage = active ? stage_at(index) : 0;
@@ -560,8 +642,10 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
       for (int i = 0; i < 4; ++i) {
         float sum = 0.0f;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w)
-          if (weight[w] != 0.0f) sum += weight[w] * share_out[(w * D + d0 + e + i) * 32 + (threadIdx.x & 31)];
+        for (int w = 0; w < WAVES; ++w) {  // (a share that has no weight may be infinite; a branch would wait for each)
+          const float share = share_out[(w * D + d0 + e + i) * 32 + (threadIdx.x & 31)];
+          sum += weight[w] * (weight[w] != 0.0f ? share : 0.0f);
+        }
         value[i] = sum * inverse;
       }
       uint2 packed;
@@ -883,7 +967,8 @@ __global__ __launch_bounds__(256) void dense_attention_rows_kernel(DenseAttentio
 
 template <int D, int WAVES, int STAGE_KEYS, int MASK, bool KEYSPLIT, bool PAIR = false>
 hipError_t launch_tile32_instance(uint32_t grid, const DenseAttentionArgs &a, hipStream_t stream) {
-  constexpr size_t bytes = (PAIR ? 2 : 1) * 2 * 2 * (size_t)STAGE_KEYS * D * 2;  // two stages of K and V per group
+  // two stages of K and V per group (and the query rows of slabs whose waves copy their own keys)
+  constexpr size_t bytes = (PAIR ? 2 : 1) * 2 * 2 * (size_t)STAGE_KEYS * D * 2 + (KEYSPLIT && MASK == 0 ? 32 * D * 2 : 0);
   auto kernel = &dense_attention_tile32_kernel<D, WAVES, STAGE_KEYS, MASK, KEYSPLIT, PAIR>;
   if constexpr (bytes >= 64 * 1024) {
     static bool configured[kMaxDevices] = {};  // the attribute is per device function and device
@@ -938,7 +1023,8 @@ Tile32Geometry tile32_geometry(const DenseAttentionArgs &a) {
   g.workgroups = (uint64_t)((a.query_length + kWavesPerBlock * 32 - 1) / (kWavesPerBlock * 32)) * a.heads * a.batches;
   if (!staged || g.workgroups > 0x7fffffffull) return g;
   g.tiled = true;
-  g.key_split = g.workgroups < (uint64_t)device_compute_units() && a.key_length >= 256 && a.head_dim <= 128;
+  g.key_split = g.workgroups < (uint64_t)device_compute_units() && a.key_length >= 256 && a.head_dim <= 128 &&
+                value_row_halfs < (1u << 25);  // (offsets from a tile's first row in 32 bits)
   if (g.key_split) g.rows_per_slab = 32, g.stage_keys = 128;
   g.slabs = (a.query_length + g.rows_per_slab - 1) / g.rows_per_slab;
   return g;

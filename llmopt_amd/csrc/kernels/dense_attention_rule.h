@@ -8,13 +8,13 @@ namespace llmopt {
 
 // The waves of a workgroup share 32 query rows and a stage of 32 keys each.  One workgroup per CU that walks several stages:
 // eight waves and 256-key stages (128 KB) halve the walk again (us, query rows / keys they see / heads, eight / four waves:
-// 700 / 700 / 9 10.2 / 11.5, 900 / 900 / 9 11.7 / 14.5, 64 / 2000 / 9 15.1 / 17.3, 400 / 4000 / 9 29.8 / 40.5).  Walks of a few
-// stages are as short either way (512 / 512 / 9 8.4 / 8.3, 300 rows that see 300 of 900 keys 10.6 / 10.6; 400 of 4000 11.0 /
-// 11.7) or shorter with four (32 rows that see 32 of 4096 keys 8.7 / 8.0, 100 that see 100 of 520 9.0 / 8.5), and where two
-// workgroups would share a CU that room is worth more (700 / 700 / 32 20.6 / 14.0, 2048 / 2048 / 9 26.7 / 20.0).
+// 700 / 700 / 9 8.3 / 8.5, 900 / 900 / 9 9.6 / 10.4, 64 / 2000 / 9 12.5 / 14.2, 400 / 4000 / 9 19.8 / 24.0).  Walks of a few
+// stages are as short either way (512 / 512 / 9 7.2 / 7.4, 300 rows that see 300 of 900 keys 7.0 / 6.7, 400 of 4000 7.4 / 7.5, 32
+// that see 32 of 4096 6.8 / 6.8), and where two workgroups would share a CU that room is worth more (700 / 700 / 32 16.0 / 12.1,
+// 2048 / 2048 / 9 21.0 / 17.2).
 // A few slabs more than CUs are a second round, which is short under a causal limit once the walk is long (32 slabs of 9 heads
-// over 1000 keys 15.0 / 17.5; 18 of 16 heads over 560 14.2 / 13.5) and as long as the first without one (18 of 16 heads over
-// 560 20.2 / 15.0).  With a mask the map of stages counts in 128 keys.
+// over 1000 keys 9.4 / 10.0; 18 of 16 heads over 560 8.7 / 8.1) and as long as the first without one (18 of 16 heads over
+// 560 12.0 / 9.5).  With a mask the map of stages counts in 128 keys.
 inline bool eight_wave_slabs(uint32_t head_dim, bool masked, bool causal, uint32_t query_length, uint32_t key_length,
                              uint32_t past_length, uint64_t slabs, uint32_t cus) {
   const uint64_t last = (uint64_t)past_length + query_length;  // keys that the last row sees under a causal limit
@@ -26,10 +26,11 @@ inline bool eight_wave_slabs(uint32_t head_dim, bool masked, bool causal, uint32
 enum class TurnsForm { kNone, kSplit, kRows };
 
 // Without a mask, from 256 keys on (below that the groups have a stage or two each); workgroups: of 128 rows.
-// kSplit, 128 rows whose keys the groups share, against the key-splitting slabs of 32 rows: heads of 128 as soon as those are
-// more than a workgroup a CU, their stages' room (us, heads x rows: 32 x 300 10.9 / 14.3, 32 x 700 16.2 / 29.0, 16 x 700 15.8 /
-// 17.7, 16 x 1900 34.5 / 61.5; 16 x 500 14.1 / 12.4, 4 x 1500 25.1 / 24.2), heads of 64, of which a CU takes more, from three
-// quarters of the CUs on (9 x 3000 33.0 / 34.7, 16 x 1900 24.1 / 26.7; 16 x 1500 20.4 / 20.0, 9 x 2048 24.5 / 20.0).
+// kSplit, 128 rows whose keys the groups share, against the key-splitting slabs of 32 rows, of which there is a workgroup a CU at
+// most once there are as many of 128 rows as CUs.  Heads of 128 from half of the CUs on (us, heads x rows: 32 x 700 16.5 / 21.4,
+// 16 x 1200 21.5 / 25.9, 16 x 1900 32 / 47, 8 x 3000 42 / 51; at half of them 32 x 500 13.8 / 14.7, 4 x 4096 54.1 / 53.6, 16 x 900 18.5 /
+// 16.9; 16 x 700 15.5 / 12.3, 32 x 300 10.8 / 9.9), heads of 64, two slabs of which fit a CU, not before (32 x 1000 15.2 / 23.2,
+// 9 x 3600 39 / 73; 32 x 800 12.8 / 12.8, 9 x 3500 37.2 / 35.5, 16 x 1900 23.7 / 21.3, 9 x 2048 24.5 / 16.2).
 // kRows, 256 rows and their own group each, half the copies and no sums to hand over, once the longer workgroups still come to
 // more than a round and a half (32 heads of 128: 4096 rows 162 / 167, 3500 126 / 131, 3000 102 / 100, 2048 62 / 48), and
 // only where rows fill them.
@@ -40,7 +41,7 @@ inline TurnsForm turns_form(uint32_t head_dim, bool masked, uint32_t query_lengt
   if (masked || (head_dim != 64 && head_dim != 128) || key_length < 256) return TurnsForm::kNone;
   if (workgroups > 3 * (uint64_t)cus && key_length < 512) return TurnsForm::kNone;
   if (workgroups > 3 * (uint64_t)cus && query_length >= 1024) return TurnsForm::kRows;
-  return 4 * workgroups > (head_dim == 64 ? 3 : 1) * (uint64_t)cus ? TurnsForm::kSplit : TurnsForm::kNone;
+  return (head_dim == 64 ? workgroups >= cus : 2 * workgroups > cus) ? TurnsForm::kSplit : TurnsForm::kNone;
 }
 
 // The same over a portion of a prompt in bfloat16, 128 rows and their keys shared.  A workgroup starts and ends in some 8 us of

@@ -341,9 +341,20 @@ def test_long_walks_of_few_slabs_take_eight_waves(runtime, heads, kv_heads, new,
     check_attention_case(runtime, 64, heads, kv_heads, new, past, mode)
 
 
+@pytest.mark.parametrize("dim,heads,kv_heads,new,past,mode", [
+    (64, 3, 1, 31, 225, "none"), (64, 3, 1, 32, 225, "causal"), (64, 2, 2, 40, 472, "none"), (64, 2, 1, 31, 482, "none"),
+    (64, 9, 3, 20, 749, "causal"), (64, 9, 3, 64, 1216, "none"), (64, 4, 1, 33, 1760, "causal"), (128, 2, 1, 17, 240, "none"),
+    (128, 2, 1, 33, 351, "none"), (128, 2, 2, 32, 353, "causal"), (128, 3, 1, 5, 508, "none"),
+])
+def test_own_tiles_of_a_slab(runtime, dim, heads, kv_heads, new, past, mode):
+    """A wave's one to six tiles of 32 keys: the third goes through registers, the others straight to LDS; last tiles of one
+    key, a whole tile, and waves that have a tile less."""
+    check_attention_case(runtime, dim, heads, kv_heads, new, past, mode)
+
+
 @pytest.mark.parametrize("dim,batches,heads,kv_heads,new,past,mode", [
-    (128, 1, 12, 4, 700, 0, "causal"), (128, 2, 33, 11, 33, 223, "none"), (128, 3, 11, 11, 257, 130, "causal"),
-    (128, 1, 80, 10, 1, 255, "none"), (64, 2, 50, 25, 129, 383, "causal"), (64, 1, 40, 8, 640, 1, "none"),
+    (128, 1, 24, 8, 700, 0, "causal"), (128, 2, 66, 22, 33, 223, "none"), (128, 3, 15, 15, 257, 130, "causal"),
+    (128, 1, 130, 13, 1, 255, "none"), (64, 2, 64, 32, 129, 383, "causal"), (64, 1, 56, 8, 640, 1, "none"),
     (128, 1, 86, 43, 1031, 0, "causal"), (64, 2, 43, 43, 1100, 77, "causal"), (64, 1, 96, 8, 1024, 3, "none"),
 ])
 def test_groups_of_waves_in_turns(runtime, dim, batches, heads, kv_heads, new, past, mode):

@@ -158,8 +158,8 @@ def test_eight_waves_a_slab(rules, causal, rows, keys, past, heads, eight):
 
 @pytest.mark.parametrize("dim,masked,rows,keys,heads,form", [
     (128, 0, 4096, 4096, 32, 2), (128, 0, 3500, 3500, 32, 2), (128, 0, 3000, 3000, 32, 1), (128, 0, 1000, 9000, 128, 1),
-    (128, 0, 300, 300, 32, 1), (128, 0, 700, 700, 16, 1), (128, 0, 500, 500, 16, 0), (128, 0, 255, 255, 64, 0),
-    (128, 0, 255, 256, 64, 1), (64, 0, 1900, 1900, 16, 1), (64, 0, 1500, 1500, 16, 0), (64, 0, 4096, 4096, 32, 2),
+    (128, 0, 300, 300, 32, 0), (128, 0, 700, 700, 32, 1), (128, 0, 1000, 1000, 16, 0), (128, 0, 1100, 1100, 16, 1),
+    (128, 0, 255, 255, 80, 0), (128, 0, 255, 256, 80, 1), (64, 0, 2040, 2040, 16, 1), (64, 0, 1900, 1900, 16, 0), (64, 0, 4096, 4096, 32, 2),
     (256, 0, 4096, 4096, 32, 0), (128, 0, 300, 300, 512, 0), (128, 0, 300, 300, 256, 1), (128, 0, 64, 512, 1024, 1), (128, 1, 4096, 4096, 32, 0)])
 def test_attention_in_turns(rules, dim, masked, rows, keys, heads, form):
     assert rules.turns(dim, masked, rows, keys, heads, CUS) == form
