@@ -159,7 +159,7 @@ __global__ __launch_bounds__(WAVES * 64 * (PAIR ? 2 : 1))
   const uint32_t q0 = KEYSPLIT ? slab * 32 : (slab * WAVES + wave) * 32;
   const bool has_rows = q0 < a.query_length;  // a wave without rows still copies and meets the barriers
   const uint32_t kv_heads = a.kv_heads > 0 ? a.kv_heads : a.heads;
-  const uint32_t kv_head = kv_heads < a.heads ? head * kv_heads / a.heads : head;  // (the heads divide over them)
+  const uint32_t kv_head = kv_head_of(head, a.heads, kv_heads);
   constexpr bool masked = MASKED;
   const uint32_t L = a.key_length;
 
@@ -908,7 +908,7 @@ __global__ __launch_bounds__(256) void dense_attention_rows_kernel(DenseAttentio
   const uint32_t head = (row_index / a.query_length) % a.heads;
   const uint32_t batch = row_index / (a.query_length * a.heads);
   const uint32_t kv_heads = a.kv_heads > 0 ? a.kv_heads : a.heads;
-  const uint32_t kv_head = kv_heads < a.heads ? head / (a.heads / kv_heads) : head;
+  const uint32_t kv_head = kv_head_of(head, a.heads, kv_heads);
   const uint32_t D = a.head_dim;
   const uint32_t fragments = (D + 63) / 64;
   const bool masked = a.mask != nullptr && a.mask_batches > 0;

@@ -6,6 +6,12 @@
 
 namespace llmopt {
 
+// The key / value head of a query head; the query heads are a multiple of them.  (head * kv_heads / heads is one division fewer
+// and wraps from 2^32 on: 131072 heads over 65536.)
+constexpr uint32_t kv_head_of(uint32_t head, uint32_t heads, uint32_t kv_heads) {
+  return kv_heads < heads ? head / (heads / kv_heads) : head;
+}
+
 // The waves of a workgroup share 32 query rows and a stage of 32 keys each.  One workgroup per CU that walks several stages:
 // eight waves and 256-key stages (128 KB) halve the walk again (us, query rows / keys they see / heads, eight / four waves:
 // 700 / 700 / 9 8.3 / 8.5, 900 / 900 / 9 9.6 / 10.4, 64 / 2000 / 9 12.5 / 14.2, 400 / 4000 / 9 19.8 / 24.0).  Walks of a few

@@ -341,6 +341,19 @@ def test_long_walks_of_few_slabs_take_eight_waves(runtime, heads, kv_heads, new,
     check_attention_case(runtime, 64, heads, kv_heads, new, past, mode)
 
 
+@pytest.mark.parametrize("masked", [False, True])
+def test_more_heads_times_key_heads_than_32_bits(runtime, masked):
+    """131072 heads over 65536, each with its own number in its values: no query, so a row is its head's value."""
+    heads, kv_heads, new, dim = 131072, 65536, 16, 64
+    value = np.zeros((1, kv_heads, new, dim), dtype=np.float16)
+    value[0, :, :, 0] = (np.arange(kv_heads) % 256)[:, None]
+    value[0, :, :, 1] = (np.arange(kv_heads) // 256)[:, None]
+    params = attention_params(1, heads, new, new, dim, int(masked), int(masked), False, 0.125, kv_heads, mask_dtype=int(masked))
+    got = run(runtime, "llmopt_attention_f16_simd_h64", np.zeros((1, heads, new, dim), dtype=np.float16), np.zeros_like(value), value,
+              np.ones((1, 1, new, new), dtype=np.uint8) if masked else None, params, (1, heads, new, dim))
+    assert (got[0, ..., 0] + 256 * got[0, ..., 1].astype(np.float32) == (np.arange(heads) // 2)[:, None]).all()
+
+
 @pytest.mark.parametrize("dim,heads,kv_heads,new,past,mode", [
     (64, 3, 1, 31, 225, "none"), (64, 3, 1, 32, 225, "causal"), (64, 2, 2, 40, 472, "none"), (64, 2, 1, 31, 482, "none"),
     (64, 9, 3, 20, 749, "causal"), (64, 9, 3, 64, 1216, "none"), (64, 4, 1, 33, 1760, "causal"), (128, 2, 1, 17, 240, "none"),

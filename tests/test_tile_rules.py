@@ -28,6 +28,7 @@ int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, ui
 int turns(uint32_t dim, uint32_t masked, uint32_t rows, uint32_t keys, uint32_t heads, uint32_t cus) {
   return (int)turns_form(dim, masked != 0, rows, keys, (uint64_t)((rows + 127) / 128) * heads, cus);
 }
+uint32_t kv_head(uint32_t head, uint32_t heads, uint32_t kv_heads) { return kv_head_of(head, heads, kv_heads); }
 int chunked(uint32_t dim, uint32_t capped, uint32_t m, uint32_t span) { return chunk_turns(dim, capped != 0, m, span); }
 int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
   return three_delta_workgroups((tokens + 63) / 64 * heads, cus);
@@ -154,6 +155,15 @@ def test_logits(rules, tokens, k, n, tiles):
     (1, 32, 4096, 0, 9, 0), (1, 64, 2000, 0, 16, 0), (1, 100, 520, 0, 3, 0), (1, 32, 4096, 224, 9, 0), (1, 32, 4096, 225, 9, 1), (1, 400, 4000, 0, 9, 1)])
 def test_eight_waves_a_slab(rules, causal, rows, keys, past, heads, eight):
     assert rules.eight_waves(causal, rows, keys, past, heads, CUS) == eight
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(9, 3), (32, 32), (7, 1), (131072, 65536), (100000, 50000), (131070, 43690),
+                                            (1 << 31, 1 << 30), (0xfffffffe, 0x7fffffff)])
+def test_key_head_of_a_query_head(rules, heads, kv_heads):
+    """Also where heads times kv_heads is more than 32 bits hold."""
+    rules.kv_head.restype = ctypes.c_uint32
+    for head in {0, 1, heads // kv_heads, heads // 3, heads // 2, heads - 2, heads - 1}:
+        assert rules.kv_head(ctypes.c_uint32(head), ctypes.c_uint32(heads), ctypes.c_uint32(kv_heads)) == head * kv_heads // heads
 
 
 @pytest.mark.parametrize("dim,masked,rows,keys,heads,form", [
