@@ -1005,10 +1005,11 @@ struct Tile32Geometry {
   bool key_split;   // 32-row slabs whose keys are split over the waves, 128-key stages
   uint32_t rows_per_slab, stage_keys, slabs;
   uint64_t workgroups;  // of 128 rows
+  uint64_t value_row_halfs;
 };
 
 Tile32Geometry tile32_geometry(const DenseAttentionArgs &a) {
-  Tile32Geometry g = {false, false, 128, 64, 0, 0};
+  Tile32Geometry g = {false, false, 128, 64, 0, 0, 0};
   const bool aligned = reinterpret_cast<uintptr_t>(a.query) % 16 == 0 && reinterpret_cast<uintptr_t>(a.key) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(a.value) % 8 == 0 && reinterpret_cast<uintptr_t>(a.output) % 8 == 0;
   if (!((a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256) && aligned &&
@@ -1016,15 +1017,14 @@ Tile32Geometry tile32_geometry(const DenseAttentionArgs &a) {
     return g;
   // K and V stages are copied as 16-byte pieces of whole rows (16-byte aligned K and V rows), and the
   // maxima are taken before scaling (a positive, finite scale); anything else takes the row kernel
-  const size_t value_row_halfs = a.token_first_value ? (size_t)(a.kv_heads > 0 ? a.kv_heads : a.heads) * a.head_dim
-                                                     : a.head_dim;
-  const bool staged = reinterpret_cast<uintptr_t>(a.value) % 16 == 0 && value_row_halfs % 8 == 0 &&
+  g.value_row_halfs = a.token_first_value ? (uint64_t)(a.kv_heads > 0 ? a.kv_heads : a.heads) * a.head_dim : a.head_dim;
+  const bool staged = reinterpret_cast<uintptr_t>(a.value) % 16 == 0 && g.value_row_halfs % 8 == 0 &&
                       a.scale > 0.0f && a.scale < INFINITY;
   g.workgroups = (uint64_t)((a.query_length + kWavesPerBlock * 32 - 1) / (kWavesPerBlock * 32)) * a.heads * a.batches;
   if (!staged || g.workgroups > 0x7fffffffull) return g;
   g.tiled = true;
   g.key_split = g.workgroups < (uint64_t)device_compute_units() && a.key_length >= 256 && a.head_dim <= 128 &&
-                value_row_halfs < (1u << 25);  // (offsets from a tile's first row in 32 bits)
+                short_value_rows(g.value_row_halfs);
   if (g.key_split) g.rows_per_slab = 32, g.stage_keys = 128;
   g.slabs = (a.query_length + g.rows_per_slab - 1) / g.rows_per_slab;
   return g;
@@ -1098,7 +1098,7 @@ hipError_t launch_dense_attention(const DenseAttentionArgs &a, hipStream_t strea
           mask_kind = 3;
         }
       }
-      const TurnsForm turns = turns_form(a.head_dim, mask != 0, a.query_length, a.key_length, workgroups,
+      const TurnsForm turns = turns_form(a.head_dim, mask != 0, a.query_length, a.key_length, workgroups, geometry.value_row_halfs,
                                          (uint32_t)device_compute_units());
       if (turns == TurnsForm::kSplit) return a.head_dim == 64 ? launch_turns<64, true>(a, stream) : launch_turns<128, true>(a, stream);
       if (turns == TurnsForm::kRows) return a.head_dim == 64 ? launch_turns<64, false>(a, stream) : launch_turns<128, false>(a, stream);

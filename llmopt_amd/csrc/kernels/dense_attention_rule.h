@@ -29,6 +29,9 @@ inline bool eight_wave_slabs(uint32_t head_dim, bool masked, bool causal, uint32
   return head_dim == 64 && !masked && key_length > 512 && walk > 256 && slabs <= room;
 }
 
+// Forms that keep a value row's place behind its stage's first one in 32 bits, for up to 63 rows of halves.
+constexpr bool short_value_rows(uint64_t value_row_halfs) { return value_row_halfs < (1u << 25); }
+
 enum class TurnsForm { kNone, kSplit, kRows };
 
 // Without a mask, from 256 keys on (below that the groups have a stage or two each); workgroups: of 128 rows.
@@ -43,7 +46,8 @@ enum class TurnsForm { kNone, kSplit, kRows };
 // Many workgroups that each walk a few stages are better off two a CU (64 x 32 heads of 128, 16 rows, 260 keys 72.7 / 66.4;
 // 16 x 32 of 64, 300 of 300 39.2 / 35.5; 8 x 32 of 128, 300 of 300 29.4 / 29.8; 32 x 32, 64 rows, 512 keys 51.5 / 53.6).
 inline TurnsForm turns_form(uint32_t head_dim, bool masked, uint32_t query_length, uint32_t key_length, uint64_t workgroups,
-                            uint32_t cus) {
+                            uint64_t value_row_halfs, uint32_t cus) {
+  if (!short_value_rows(value_row_halfs)) return TurnsForm::kNone;
   if (masked || (head_dim != 64 && head_dim != 128) || key_length < 256) return TurnsForm::kNone;
   if (workgroups > 3 * (uint64_t)cus && key_length < 512) return TurnsForm::kNone;
   if (workgroups > 3 * (uint64_t)cus && query_length >= 1024) return TurnsForm::kRows;

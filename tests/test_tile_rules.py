@@ -26,7 +26,10 @@ int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, ui
   return eight_wave_slabs(64, false, causal != 0, rows, keys, past, (rows + 31) / 32 * heads, cus);
 }
 int turns(uint32_t dim, uint32_t masked, uint32_t rows, uint32_t keys, uint32_t heads, uint32_t cus) {
-  return (int)turns_form(dim, masked != 0, rows, keys, (uint64_t)((rows + 127) / 128) * heads, cus);
+  return (int)turns_form(dim, masked != 0, rows, keys, (uint64_t)((rows + 127) / 128) * heads, dim, cus);
+}
+int turns_of(uint32_t dim, uint32_t rows, uint32_t keys, uint64_t workgroups, uint64_t value_row_halfs, uint32_t cus) {
+  return (int)turns_form(dim, false, rows, keys, workgroups, value_row_halfs, cus);
 }
 uint32_t kv_head(uint32_t head, uint32_t heads, uint32_t kv_heads) { return kv_head_of(head, heads, kv_heads); }
 int chunked(uint32_t dim, uint32_t capped, uint32_t m, uint32_t span) { return chunk_turns(dim, capped != 0, m, span); }
@@ -173,6 +176,35 @@ def test_key_head_of_a_query_head(rules, heads, kv_heads):
     (256, 0, 4096, 4096, 32, 0), (128, 0, 300, 300, 512, 0), (128, 0, 300, 300, 256, 1), (128, 0, 64, 512, 1024, 1), (128, 1, 4096, 4096, 32, 0)])
 def test_attention_in_turns(rules, dim, masked, rows, keys, heads, form):
     assert rules.turns(dim, masked, rows, keys, heads, CUS) == form
+
+
+def turns_offsets(dim, waves, values, stride_bytes):
+    """TurnsCopy::offset (attention_turns.h) of every copy and thread: where it reads behind the stage's first row, less what the
+    instruction's own offset adds."""
+    pieces = dim // 8
+    keys = 64 // pieces
+    count = 64 // keys // waves
+    for c in range(count):
+        for thread in range(64 * waves):
+            row = (thread // 64 % waves * count + c) * keys + thread % 64 // pieces
+            piece = (thread % pieces) ^ ((2 if values else 1) * row & (pieces - 1))
+            yield row * stride_bytes + piece * 16 - c * 1024
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_value_rows_of_turns_in_32_bits(rules, dim):
+    """Token-first values of many key heads: the longest rows that go in turns have all their places in 32 bits; longer ones,
+    from 262144 heads of 128 on, keep the tiles of 64-bit addresses."""
+    form = lambda halfs: rules.turns_of(dim, 128, 512, ctypes.c_uint64(halfs // dim), ctypes.c_uint64(halfs), CUS)
+    longest = (1 << 25) - dim
+    assert form(longest) != 0
+    for waves in (4, 8):
+        for values in (False, True):
+            for stride in (dim, longest):
+                offsets = list(turns_offsets(dim, waves, values, stride * 2))
+                assert min(offsets) >= 0 and max(offsets) < 1 << 32
+    for halfs in (1 << 25, 266306 * 128, 1 << 31, 1 << 33):
+        assert form(halfs) == 0
 
 
 def test_gpu_tests_reach_both_forms_of_turns(rules):
