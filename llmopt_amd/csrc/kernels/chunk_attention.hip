@@ -576,10 +576,10 @@ hipError_t run_turns(const ChunkAttentionArgs &a, hipStream_t stream) {
 // Whole pieces of sixteen bytes, rows that the ring holds a stage of, and maxima taken before the scale.
 bool turns_ok(const ChunkAttentionArgs &a) {
   const auto aligned = [](const void *p, uint32_t bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; };
-  return !a.f32 && a.dim == a.vdim && chunk_turns(a.dim, a.softcap > 0.0f, a.m, a.cache.span) && a.cache.capacity >= kTurnsKeys &&
-         a.ld % 8 == 0 && a.ld < (1u << 24) && a.ld_out % 4 == 0 && aligned(a.qkv, 16) && aligned(a.cache.keys, 16) &&
-         aligned(a.cache.values, 16) && aligned(a.out, 8) && (a.softcap > 0.0f || (a.scale > 0.0f && a.scale < INFINITY)) &&
-         (uint64_t)a.heads * ((a.m + 127) / 128) <= 0x7fffffffull;
+  return !a.f32 && a.dim == a.vdim && chunk_turns(a.dim, a.softcap > 0.0f, a.m, a.cache.span, a.heads) &&
+         a.cache.capacity >= kTurnsKeys && a.ld % 8 == 0 && a.ld < (1u << 24) && a.ld_out % 4 == 0 && aligned(a.qkv, 16) &&
+         aligned(a.cache.keys, 16) && aligned(a.cache.values, 16) && aligned(a.out, 8) &&
+         (a.softcap > 0.0f || (a.scale > 0.0f && a.scale < INFINITY));
 }
 
 // A wave's registers hold 16 query rows of heads up to 128 twice a SIMD beside a second workgroup (bfloat16); wider

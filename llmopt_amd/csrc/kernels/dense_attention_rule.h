@@ -32,6 +32,9 @@ inline bool eight_wave_slabs(uint32_t head_dim, bool masked, bool causal, uint32
 // Forms that keep a value row's place behind its stage's first one in 32 bits, for up to 63 rows of halves.
 constexpr bool short_value_rows(uint64_t value_row_halfs) { return value_row_halfs < (1u << 25); }
 
+// Workgroups of 512 threads in a grid, which has fewer than 2^32 threads.  Workgroups of 256 go on to twice as many.
+constexpr bool turns_grid(uint64_t workgroups) { return workgroups * 512 < (1ull << 32); }
+
 enum class TurnsForm { kNone, kSplit, kRows };
 
 // Without a mask, from 256 keys on (below that the groups have a stage or two each); workgroups: of 128 rows.
@@ -47,7 +50,7 @@ enum class TurnsForm { kNone, kSplit, kRows };
 // 16 x 32 of 64, 300 of 300 39.2 / 35.5; 8 x 32 of 128, 300 of 300 29.4 / 29.8; 32 x 32, 64 rows, 512 keys 51.5 / 53.6).
 inline TurnsForm turns_form(uint32_t head_dim, bool masked, uint32_t query_length, uint32_t key_length, uint64_t workgroups,
                             uint64_t value_row_halfs, uint32_t cus) {
-  if (!short_value_rows(value_row_halfs)) return TurnsForm::kNone;
+  if (!short_value_rows(value_row_halfs) || !turns_grid(workgroups)) return TurnsForm::kNone;
   if (masked || (head_dim != 64 && head_dim != 128) || key_length < 256) return TurnsForm::kNone;
   if (workgroups > 3 * (uint64_t)cus && key_length < 512) return TurnsForm::kNone;
   if (workgroups > 3 * (uint64_t)cus && query_length >= 1024) return TurnsForm::kRows;
@@ -60,7 +63,8 @@ inline TurnsForm turns_form(uint32_t head_dim, bool masked, uint32_t query_lengt
 // 1024 102 / 118, 16 x 700 28 / 31, 16 x 500 25.1 / 25.8, 32 x 1500 of 512 54.5 / 53.9; of 64 16 x 3001 of 2048 51 / 60, 16 x 1500
 // 33 / 37, 16 x 3001 of 1024 46.6 / 45.6.  A cap's two more exponentials a score hide better behind four waves a SIMD: heads of
 // 128 32 x 2048 74 / 90, 32 x 3001 of 1024 70 / 80, 32 x 1000 34 / 34, 32 x 2000 of 512 40 / 35; of 64 16 x 2048 41 / 40.
-inline bool chunk_turns(uint32_t dim, bool capped, uint32_t m, uint32_t span) {
+inline bool chunk_turns(uint32_t dim, bool capped, uint32_t m, uint32_t span, uint32_t heads) {
+  if (!turns_grid((uint64_t)heads * ((m + 127) / 128))) return false;
   const uint32_t walk = span != 0 && span < m ? span : m;
   if (dim == 128) return walk > (capped ? 1000 : 512);
   return dim == 64 && !capped && walk > 1024;

@@ -32,7 +32,9 @@ int turns_of(uint32_t dim, uint32_t rows, uint32_t keys, uint64_t workgroups, ui
   return (int)turns_form(dim, false, rows, keys, workgroups, value_row_halfs, cus);
 }
 uint32_t kv_head(uint32_t head, uint32_t heads, uint32_t kv_heads) { return kv_head_of(head, heads, kv_heads); }
-int chunked(uint32_t dim, uint32_t capped, uint32_t m, uint32_t span) { return chunk_turns(dim, capped != 0, m, span); }
+int chunked(uint32_t dim, uint32_t capped, uint32_t m, uint32_t span, uint32_t heads) {
+  return chunk_turns(dim, capped != 0, m, span, heads);
+}
 int three_workgroups(uint32_t tokens, uint32_t heads, uint32_t cus) {
   return three_delta_workgroups((tokens + 63) / 64 * heads, cus);
 }
@@ -207,6 +209,16 @@ def test_value_rows_of_turns_in_32_bits(rules, dim):
         assert form(halfs) == 0
 
 
+@pytest.mark.parametrize("dim,rows,keys", [(64, 16, 512), (128, 128, 4096), (64, 1024, 1024)])
+def test_turns_keep_to_grids_of_fewer_than_32_bits_of_threads(rules, dim, rows, keys):
+    """2^23 workgroups of 512 threads are more than a launch takes; 256-thread workgroups are not."""
+    form = lambda workgroups: rules.turns_of(dim, rows, keys, ctypes.c_uint64(workgroups), ctypes.c_uint64(dim), CUS)
+    assert form((1 << 23) - 1) != 0
+    assert form(1 << 23) == form((1 << 24) - 1) == form((1 << 31) - 1) == 0
+    assert rules.chunked(dim, 0, 1025, 4096, ((1 << 23) - 1) // 9) == 1
+    assert rules.chunked(dim, 0, 1025, 4096, (1 << 23) // 9 + 1) == 0
+
+
 def test_gpu_tests_reach_both_forms_of_turns(rules):
     names = "dim,batches,heads,kv_heads,new,past,mode"
     reached = [(dim, rules.turns(dim, 0, new, new + past, heads * batches, CUS))
@@ -219,13 +231,13 @@ def test_gpu_tests_reach_both_forms_of_turns(rules):
     (128, 1, 3001, 1024, 1), (128, 1, 1000, 2048, 0), (128, 1, 2000, 512, 0), (64, 0, 1500, 2048, 1), (64, 0, 3001, 1024, 0),
     (64, 1, 3001, 2048, 0), (96, 0, 3001, 2048, 0), (256, 0, 3001, 2048, 0)])
 def test_portions_in_turns(rules, dim, capped, m, span, turns):
-    assert rules.chunked(dim, capped, m, span) == turns
+    assert rules.chunked(dim, capped, m, span, 16) == turns
 
 
 def test_gpu_tests_of_portions_go_in_turns(rules):
-    for m, _, _, dim, _, span, softcap, *_ in sizes(test_gpu_attention_tiles.test_groups_of_waves_in_turns,
+    for m, heads, _, dim, _, span, softcap, *_ in sizes(test_gpu_attention_tiles.test_groups_of_waves_in_turns,
                                                     "m,heads,kv,dim,vdim,span,softcap,sink,first,sliding"):
-        assert rules.chunked(dim, int(softcap > 0), m, span) == 1
+        assert rules.chunked(dim, int(softcap > 0), m, span, heads) == 1
 
 
 @pytest.mark.parametrize("tokens,heads,three", [(3001, 16, 1), (2115, 16, 1), (4096, 32, 1), (3001, 32, 1), (3001, 8, 0),
