@@ -27,13 +27,12 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "dense_attention_rule.h"
 #include "staggered.h"
 
 namespace llmopt {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr uint32_t kTurnsKeys = 64;
 
 // The element's matrix operands, specialised beside each kernel: x8, eight elements; Weights, those of eight keys
 // (set_pair(i, x, y) for an even i); product(a, b, c) and weighted(a, weights, c), kProducts of it, 32 x 32 += 32 x 16 times
@@ -121,9 +120,11 @@ __device__ __forceinline__ void both_halves(float v, float &low, float &high) {
   low = __builtin_bit_cast(float, (uint32_t)swapped[0]), high = __builtin_bit_cast(float, (uint32_t)swapped[1]);
 }
 
-// The keys low .. high of a lane's query row, and of the wave's rows the first and last of both (the same for the wave).
+// The keys low .. high of a lane's query row, of the wave's rows the first and last of both, and whether any of the rows exist (the
+// same for the wave).
 struct TurnsBounds {
   uint32_t low, high, low_first, low_last, high_first, high_last;
+  bool rows;
 };
 
 // How a score s becomes an exponent to base two: s * inner (inner > 0); cap tanh, by inner = 2 scale / softcap * log2 e and
@@ -170,9 +171,8 @@ __device__ __forceinline__ bool attention_turns(unsigned char *lds, const typena
   meet();
   if (group == 1) meet();
 
-  // The wave's rows see the stages of steps first .. last - 1 (possibly none): in the others it only copies and waits.
-  const uint32_t first = bounds.low_first > start ? (bounds.low_first - start + (EVERY - 1) * kTurnsKeys) / (EVERY * kTurnsKeys) : 0;
-  const uint32_t last = bounds.high_last < start ? 0 : min((bounds.high_last - start) / (EVERY * kTurnsKeys) + 1, here);
+  // in the other steps the wave only copies and waits
+  const auto [first, last] = turns_steps(bounds.rows, bounds.low_first, bounds.high_last, start, EVERY, here);
 
   f32x16 score[2];
   typename Operand::Weights weights[4];

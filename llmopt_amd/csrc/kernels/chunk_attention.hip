@@ -346,7 +346,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   for (int ks = 0; ks < D / 16; ++ks) q[ks] = *reinterpret_cast<const bf16x8 *>(q_row + ks * 16 + half * 8);
   const uint32_t first_row = p0 + min(wave_row, a.m - 1), last_row = p0 + min(wave_row + 31, a.m - 1);
   const TurnsBounds bounds = {first_seen(p0 + own, a.cache), p0 + own, first_seen(first_row, a.cache), first_seen(last_row, a.cache),
-                              first_row, last_row};
+                              first_row, last_row, wave_row < a.m};
   const uint32_t last = p0 + min(slab * ROWS + ROWS, a.m) - 1, begin = first_seen(p0 + slab * ROWS, a.cache);
 
   const __bf16 *fresh_k = qkv + (a.heads + kv_head) * D, *fresh_v = fresh_k + a.kv_heads * D;

@@ -850,7 +850,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const auto last_of = [&](uint32_t r) {
     return a.causal ? (uint32_t)min((uint64_t)a.past_length + min(r, a.query_length - 1), (uint64_t)L - 1) : L - 1;
   };
-  const TurnsBounds bounds = {0, last_of(own), 0, 0, last_of(wave_row), last_of(wave_row + 31)};
+  const TurnsBounds bounds = {0, last_of(own), 0, 0, last_of(wave_row), last_of(wave_row + 31), wave_row < a.query_length};
   const uint32_t stages = last_of(slab * ROWS + ROWS - 1) / kTurnsKeys + 1;
   const uint16_t *keys = a.key + ((size_t)batch * kv_heads + kv_head) * L * D;
   const uint32_t value_stride = a.token_first_value ? kv_heads * D : D;

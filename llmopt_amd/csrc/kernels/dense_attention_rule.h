@@ -70,4 +70,19 @@ inline bool chunk_turns(uint32_t dim, bool capped, uint32_t m, uint32_t span, ui
   return dim == 64 && !capped && walk > 1024;
 }
 
+constexpr uint32_t kTurnsKeys = 64;  // of a stage
+
+// The steps first .. last - 1 (none if first >= last) of `here`, one for the 64 keys behind start + step * every * 64, that hold keys
+// which a wave's rows see: its first row from low_first on, its last one up to high_last.  A wave whose rows all lie past the end
+// sees none, it only copies and waits: 700 rows leave half of every head's last and longest slab to such waves.
+struct TurnsSteps {
+  uint32_t first, last;
+};
+constexpr TurnsSteps turns_steps(bool any_rows, uint32_t low_first, uint32_t high_last, uint32_t start, uint32_t every, uint32_t here) {
+  const uint32_t apart = every * kTurnsKeys;
+  const uint32_t first = low_first > start ? (low_first - start + (every - 1) * kTurnsKeys) / apart : 0;
+  const uint32_t end = high_last < start || !any_rows ? 0 : (high_last - start) / apart + 1;
+  return {first, end < here ? end : here};
+}
+
 }  // namespace llmopt

@@ -32,6 +32,10 @@ int turns_of(uint32_t dim, uint32_t rows, uint32_t keys, uint64_t workgroups, ui
   return (int)turns_form(dim, false, rows, keys, workgroups, value_row_halfs, cus);
 }
 uint32_t kv_head(uint32_t head, uint32_t heads, uint32_t kv_heads) { return kv_head_of(head, heads, kv_heads); }
+uint32_t walked(uint32_t any, uint32_t low, uint32_t high, uint32_t start, uint32_t every, uint32_t here) {
+  const TurnsSteps steps = turns_steps(any != 0, low, high, start, every, here);
+  return steps.first < steps.last ? steps.first << 16 | steps.last : 0;
+}
 int chunked(uint32_t dim, uint32_t capped, uint32_t m, uint32_t span, uint32_t heads) {
   return chunk_turns(dim, capped != 0, m, span, heads);
 }
@@ -207,6 +211,18 @@ def test_value_rows_of_turns_in_32_bits(rules, dim):
                 assert min(offsets) >= 0 and max(offsets) < 1 << 32
     for halfs in (1 << 25, 266306 * 128, 1 << 31, 1 << 33):
         assert form(halfs) == 0
+
+
+@pytest.mark.parametrize("every", [1, 2])
+def test_steps_that_a_wave_of_rows_walks(rules, every):
+    """The steps whose 64 keys hold any that the wave's rows see, and none for a wave whose rows lie past the end."""
+    for start in (0, 64, 100, 1437):
+        for here in (0, 1, 2, 9):
+            for low in (0, 1, 63, 64, 100, 127, 128, 129, 164, 1436, 1500, 1501, 1629):
+                for high in (low + 31, low + 100, low + 700):
+                    seen = [s for s in range(here) if start + s * every * 64 <= high and start + s * every * 64 + 63 >= low]
+                    assert rules.walked(1, low, high, start, every, here) == (seen[0] << 16 | seen[-1] + 1 if seen else 0)
+                    assert rules.walked(0, low, high, start, every, here) == 0
 
 
 @pytest.mark.parametrize("dim,rows,keys", [(64, 16, 512), (128, 128, 4096), (64, 1024, 1024)])
