@@ -826,8 +826,7 @@ namespace {
 // (1024 of them the matrix core's) beside 1000 of softmax and 200 of copies, where two free waves took 3200 for it; no copies at
 // all would save another tenth, no exponentials 4 %.  32 / 8 heads of 128, causal: 4096 rows 180 -> 155 us (886 TFLOP/s),
 // 2048 59 -> 48, 1500 46 -> 32; 16 / 4: 4096 105 -> 83, 1900 62 -> 35; 16 / 4 of 64, 4096 rows 68 -> 55.
-// Later rows see more keys and come first, a workgroup a CU; heads of one key / value head follow each other kv_heads apart,
-// so that they share an XCD's L2 when kv_heads is a multiple of the eight XCDs.
+// Later rows see more keys and come first, a workgroup a CU.
 template <int D, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_attention_turns_kernel(DenseAttentionArgs a) {
   constexpr int JJ = D / 32, WAVES = SPLIT ? 4 : 8;
@@ -836,10 +835,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const uint32_t lane = threadIdx.x & 63, row_lane = lane & 31, half = lane >> 5;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t slabs = (a.query_length + ROWS - 1) / ROWS, per_slab = a.heads * a.batches;
-  const uint32_t kv_heads = a.kv_heads > 0 ? a.kv_heads : a.heads, per = a.heads / kv_heads;
+  const uint32_t kv_heads = a.kv_heads > 0 ? a.kv_heads : a.heads;
   const uint32_t rank = blockIdx.x, within = rank % per_slab, slab = a.causal ? slabs - 1 - rank / per_slab : rank / per_slab;
-  const uint32_t batch = within / a.heads, kv_head = within % a.heads % kv_heads;
-  const uint32_t head = kv_head * per + within % a.heads / kv_heads;
+  const uint32_t batch = within / a.heads, head = turns_head(within % a.heads, a.heads, kv_heads);
+  const uint32_t kv_head = head / (a.heads / kv_heads);
   const uint32_t L = a.key_length, wave_row = slab * ROWS + wave % WAVES * 32;
   const uint32_t own = min(wave_row + row_lane, a.query_length - 1);
 

@@ -70,6 +70,14 @@ inline bool chunk_turns(uint32_t dim, bool capped, uint32_t m, uint32_t span, ui
   return dim == 64 && !capped && walk > 1024;
 }
 
+// The head that workgroup `rank` of a slab takes.  Workgroups go to the eight XCDs in turn: the heads of a key head follow each other
+// eight apart, on one XCD's L2 when the key heads come in whole eights, and soon, while its keys are still there.
+constexpr uint32_t turns_head(uint32_t rank, uint32_t heads, uint32_t kv_heads) {
+  const uint32_t per = heads / kv_heads, first = rank / (8 * per) * 8, left = kv_heads - first, width = left < 8 ? left : 8;
+  const uint32_t at = rank - first * per;
+  return (first + at % width) * per + at / width;
+}
+
 constexpr uint32_t kTurnsKeys = 64;  // of a stage
 
 // The steps first .. last - 1 (none if first >= last) of `here`, one for the 64 keys behind start + step * every * 64, that hold keys

@@ -32,6 +32,7 @@ int turns_of(uint32_t dim, uint32_t rows, uint32_t keys, uint64_t workgroups, ui
   return (int)turns_form(dim, false, rows, keys, workgroups, value_row_halfs, cus);
 }
 uint32_t kv_head(uint32_t head, uint32_t heads, uint32_t kv_heads) { return kv_head_of(head, heads, kv_heads); }
+uint32_t head_of(uint32_t rank, uint32_t heads, uint32_t kv_heads) { return turns_head(rank, heads, kv_heads); }
 uint32_t walked(uint32_t any, uint32_t low, uint32_t high, uint32_t start, uint32_t every, uint32_t here) {
   const TurnsSteps steps = turns_steps(any != 0, low, high, start, every, here);
   return steps.first < steps.last ? steps.first << 16 | steps.last : 0;
@@ -211,6 +212,17 @@ def test_value_rows_of_turns_in_32_bits(rules, dim):
                 assert min(offsets) >= 0 and max(offsets) < 1 << 32
     for halfs in (1 << 25, 266306 * 128, 1 << 31, 1 << 33):
         assert form(halfs) == 0
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(32, 8), (16, 4), (9, 3), (7, 7), (130, 13), (60, 20), (3000, 750), (640, 64)])
+def test_order_of_heads_in_turns(rules, heads, kv_heads):
+    """Every head once; those of a key head close together, on one XCD of eight if key heads come in whole eights."""
+    order = [rules.head_of(rank, heads, kv_heads) for rank in range(heads)]
+    assert sorted(order) == list(range(heads))
+    per = heads // kv_heads
+    ranks = [sorted(rank for rank, head in enumerate(order) if head // per == kv) for kv in range(kv_heads)]
+    assert all(r[-1] - r[0] <= 8 * (per - 1) for r in ranks)
+    assert kv_heads % 8 != 0 or all(len({rank % 8 for rank in r}) == 1 for r in ranks)
 
 
 @pytest.mark.parametrize("every", [1, 2])
