@@ -1097,8 +1097,8 @@ hipError_t launch_dense_attention(const DenseAttentionArgs &a, hipStream_t strea
           mask_kind = 3;
         }
       }
-      const TurnsForm turns = turns_form(a.head_dim, mask != 0, a.query_length, a.key_length, workgroups, geometry.value_row_halfs,
-                                         (uint32_t)device_compute_units());
+      const TurnsForm turns = turns_form(a.head_dim, mask != 0, a.causal != 0, a.query_length, a.key_length, a.past_length,
+                                         workgroups, geometry.value_row_halfs, (uint32_t)device_compute_units());
       if (turns == TurnsForm::kSplit) return a.head_dim == 64 ? launch_turns<64, true>(a, stream) : launch_turns<128, true>(a, stream);
       if (turns == TurnsForm::kRows) return a.head_dim == 64 ? launch_turns<64, false>(a, stream) : launch_turns<128, false>(a, stream);
       if (geometry.key_split) {

@@ -46,14 +46,26 @@ enum class TurnsForm { kNone, kSplit, kRows };
 // kRows, 256 rows and their own group each, half the copies and no sums to hand over, once the longer workgroups still come to
 // more than a round and a half (32 heads of 128: 4096 rows 162 / 167, 3500 126 / 131, 3000 102 / 100, 2048 62 / 48), and
 // only where rows fill them.
-// Many workgroups that each walk a few stages are better off two a CU (64 x 32 heads of 128, 16 rows, 260 keys 72.7 / 66.4;
-// 16 x 32 of 64, 300 of 300 39.2 / 35.5; 8 x 32 of 128, 300 of 300 29.4 / 29.8; 32 x 32, 64 rows, 512 keys 51.5 / 53.6).
-inline TurnsForm turns_form(uint32_t head_dim, bool masked, uint32_t query_length, uint32_t key_length, uint64_t workgroups,
-                            uint64_t value_row_halfs, uint32_t cus) {
+// Beyond two workgroups a CU there is more to do than the longest one, and workgroups of four waves that share a CU freely hide
+// their starts and ends behind each other; both groups in turns walk to the end together.  How long a workgroup walks on average
+// decides: on short walks turns lose what they gain on long ones, and heads that share their keys gain most (us, turns / four waves:
+// 16 heads of 128, 30 sequences of 520 tokens 139 / 99, 7 of 668 40.5 / 34.4; 128 rows of 600 keys, 75 x 32 over 8 heads 251 / 183, 44 x
+// 16 heads 69 / 63, 22 x 32 over 8 55 / 58, and of 1000 keys, 75 x 32 over 8 275 / 278; 9 over 3 heads of 64, 20 sequences of 520 tokens
+// 34 / 27, 13 of 668 28.3 / 25.3, 13 of 668 after 332 others 41 / 43.5, 128 rows of 600 keys, 78 sequences, 38.8 / 38).
+// kRows has fewer and longer workgroups (16 heads of 128: 17 sequences of 1030 tokens 150 / 150, 9 of 2048 206 / 230).
+// Up to 32 rows a head leave three of four waves of each group idle, still less than what slabs of 32 rows took whose waves met at
+// every stage (130 over 13 heads of 128, 16 rows: 1000 keys 18.2 / 22, 4000 keys 49.5 / 66.7); their own tiles take 16.5 and 44.4.
+inline TurnsForm turns_form(uint32_t head_dim, bool masked, bool causal, uint32_t query_length, uint32_t key_length,
+                            uint32_t past_length, uint64_t workgroups, uint64_t value_row_halfs, uint32_t cus) {
   if (!short_value_rows(value_row_halfs) || !turns_grid(workgroups)) return TurnsForm::kNone;
   if (masked || (head_dim != 64 && head_dim != 128) || key_length < 256) return TurnsForm::kNone;
-  if (workgroups > 3 * (uint64_t)cus && key_length < 512) return TurnsForm::kNone;
-  if (workgroups > 3 * (uint64_t)cus && query_length >= 1024) return TurnsForm::kRows;
+  const uint64_t seen = (uint64_t)past_length + query_length / 2;  // by a row in the middle
+  const uint64_t walk = causal && seen < key_length ? seen : key_length;
+  if (workgroups > 3 * (uint64_t)cus) {
+    if (query_length >= 1024 && key_length >= 512) return TurnsForm::kRows;
+    return walk >= 900 ? TurnsForm::kSplit : TurnsForm::kNone;
+  }
+  if (workgroups > 2 * (uint64_t)cus) return walk >= (head_dim == 64 ? 500 : 700) ? TurnsForm::kSplit : TurnsForm::kNone;
   return (head_dim == 64 ? workgroups >= cus : 2 * workgroups > cus) ? TurnsForm::kSplit : TurnsForm::kNone;
 }
 
@@ -71,7 +83,8 @@ inline bool chunk_turns(uint32_t dim, bool capped, uint32_t m, uint32_t span, ui
 }
 
 // The head that workgroup `rank` of a slab takes.  Workgroups go to the eight XCDs in turn: the heads of a key head follow each other
-// eight apart, on one XCD's L2 when the key heads come in whole eights, and soon, while its keys are still there.
+// eight apart, on one XCD's L2 when the key heads come in whole eights, and soon, while its keys are still there (3000 heads of 128
+// over 750, 128 rows of 1500 keys: kv_heads apart 533 us, so 416).
 constexpr uint32_t turns_head(uint32_t rank, uint32_t heads, uint32_t kv_heads) {
   const uint32_t per = heads / kv_heads, first = rank / (8 * per) * 8, left = kv_heads - first, width = left < 8 ? left : 8;
   const uint32_t at = rank - first * per;

@@ -25,11 +25,11 @@ int logits_tile(uint32_t tokens, uint32_t n, uint32_t k, uint32_t cus) { return 
 int eight_waves(uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, uint32_t heads, uint32_t cus) {
   return eight_wave_slabs(64, false, causal != 0, rows, keys, past, (rows + 31) / 32 * heads, cus);
 }
-int turns(uint32_t dim, uint32_t masked, uint32_t rows, uint32_t keys, uint32_t heads, uint32_t cus) {
-  return (int)turns_form(dim, masked != 0, rows, keys, (uint64_t)((rows + 127) / 128) * heads, dim, cus);
+int turns(uint32_t dim, uint32_t masked, uint32_t causal, uint32_t rows, uint32_t keys, uint32_t past, uint32_t heads, uint32_t cus) {
+  return (int)turns_form(dim, masked != 0, causal != 0, rows, keys, past, (uint64_t)((rows + 127) / 128) * heads, dim, cus);
 }
 int turns_of(uint32_t dim, uint32_t rows, uint32_t keys, uint64_t workgroups, uint64_t value_row_halfs, uint32_t cus) {
-  return (int)turns_form(dim, false, rows, keys, workgroups, value_row_halfs, cus);
+  return (int)turns_form(dim, false, false, rows, keys, 0, workgroups, value_row_halfs, cus);
 }
 uint32_t kv_head(uint32_t head, uint32_t heads, uint32_t kv_heads) { return kv_head_of(head, heads, kv_heads); }
 uint32_t head_of(uint32_t rank, uint32_t heads, uint32_t kv_heads) { return turns_head(rank, heads, kv_heads); }
@@ -180,9 +180,20 @@ def test_key_head_of_a_query_head(rules, heads, kv_heads):
     (128, 0, 4096, 4096, 32, 2), (128, 0, 3500, 3500, 32, 2), (128, 0, 3000, 3000, 32, 1), (128, 0, 1000, 9000, 128, 1),
     (128, 0, 300, 300, 32, 0), (128, 0, 700, 700, 32, 1), (128, 0, 1000, 1000, 16, 0), (128, 0, 1100, 1100, 16, 1),
     (128, 0, 255, 255, 80, 0), (128, 0, 255, 256, 80, 1), (64, 0, 2040, 2040, 16, 1), (64, 0, 1900, 1900, 16, 0), (64, 0, 4096, 4096, 32, 2),
-    (256, 0, 4096, 4096, 32, 0), (128, 0, 300, 300, 512, 0), (128, 0, 300, 300, 256, 1), (128, 0, 64, 512, 1024, 1), (128, 1, 4096, 4096, 32, 0)])
+    (256, 0, 4096, 4096, 32, 0), (128, 0, 300, 300, 512, 0), (128, 0, 300, 800, 256, 1), (128, 0, 64, 1000, 1024, 1), (128, 1, 4096, 4096, 32, 0)])
 def test_attention_in_turns(rules, dim, masked, rows, keys, heads, form):
-    assert rules.turns(dim, masked, rows, keys, heads, CUS) == form
+    assert rules.turns(dim, masked, 0, rows, keys, 0, heads, CUS) == form
+
+
+@pytest.mark.parametrize("dim,causal,rows,past,heads,form", [
+    (128, 1, 520, 0, 30 * 16, 0), (128, 1, 520, 0, 6 * 16, 1), (128, 1, 700, 0, 20 * 16, 0), (64, 1, 520, 0, 16 * 9, 0), (64, 1, 924, 0, 10 * 9, 0),
+    (64, 1, 300, 0, 52 * 9, 0), (128, 0, 300, 0, 256, 0), (128, 0, 64, 448, 1024, 0), (128, 0, 128, 472, 75 * 32, 0), (128, 0, 128, 872, 75 * 32, 1),
+    (128, 1, 520, 280, 4 * 32, 0), (128, 1, 1000, 300, 3 * 32, 1), (128, 1, 924, 600, 7 * 16, 1), (64, 1, 700, 600, 7 * 16, 1),
+    (128, 1, 1030, 0, 17 * 16, 2), (64, 1, 1100, 0, 24 * 16, 2), (64, 1, 1030, 0, 9 * 9, 1), (128, 1, 1030, 0, 4 * 16, 0),
+    (128, 1, 16, 0xfffffff0, 800, 1)])
+def test_long_walks_of_many_workgroups_go_in_turns(rules, dim, causal, rows, past, heads, form):
+    """More than two workgroups a CU: what a workgroup walks on average decides."""
+    assert rules.turns(dim, 0, causal, rows, min(past + rows, 2000), past if causal else 0, heads, CUS) == form
 
 
 def turns_offsets(dim, waves, values, stride_bytes):
@@ -202,7 +213,7 @@ def turns_offsets(dim, waves, values, stride_bytes):
 def test_value_rows_of_turns_in_32_bits(rules, dim):
     """Token-first values of many key heads: the longest rows that go in turns have all their places in 32 bits; longer ones,
     from 262144 heads of 128 on, keep the tiles of 64-bit addresses."""
-    form = lambda halfs: rules.turns_of(dim, 128, 512, ctypes.c_uint64(halfs // dim), ctypes.c_uint64(halfs), CUS)
+    form = lambda halfs: rules.turns_of(dim, 128, 2000, ctypes.c_uint64(halfs // dim), ctypes.c_uint64(halfs), CUS)
     longest = (1 << 25) - dim
     assert form(longest) != 0
     for waves in (4, 8):
@@ -237,7 +248,7 @@ def test_steps_that_a_wave_of_rows_walks(rules, every):
                     assert rules.walked(0, low, high, start, every, here) == 0
 
 
-@pytest.mark.parametrize("dim,rows,keys", [(64, 16, 512), (128, 128, 4096), (64, 1024, 1024)])
+@pytest.mark.parametrize("dim,rows,keys", [(64, 16, 1500), (128, 128, 4096), (64, 1024, 1024)])
 def test_turns_keep_to_grids_of_fewer_than_32_bits_of_threads(rules, dim, rows, keys):
     """2^23 workgroups of 512 threads are more than a launch takes; 256-thread workgroups are not."""
     form = lambda workgroups: rules.turns_of(dim, rows, keys, ctypes.c_uint64(workgroups), ctypes.c_uint64(dim), CUS)
@@ -249,8 +260,8 @@ def test_turns_keep_to_grids_of_fewer_than_32_bits_of_threads(rules, dim, rows, 
 
 def test_gpu_tests_reach_both_forms_of_turns(rules):
     names = "dim,batches,heads,kv_heads,new,past,mode"
-    reached = [(dim, rules.turns(dim, 0, new, new + past, heads * batches, CUS))
-               for dim, batches, heads, _, new, past, _ in sizes(test_gpu_dense_attention.test_groups_of_waves_in_turns, names)]
+    reached = [(dim, rules.turns(dim, 0, int(mode == "causal"), new, new + past, past, heads * batches, CUS))
+               for dim, batches, heads, _, new, past, mode in sizes(test_gpu_dense_attention.test_groups_of_waves_in_turns, names)]
     assert set(reached) == {(64, 1), (64, 2), (128, 1), (128, 2)}
 
 
