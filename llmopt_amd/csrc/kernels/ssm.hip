@@ -299,20 +299,23 @@ __device__ __forceinline__ const P *lane_at(const void *uniform, uint32_t bytes)
 // Bound by what a wave issues in turn: a chunk's fourteen requests and 250 vector instructions, most for the high and low parts of
 // the inputs and of the state.  2048 tokens, 64 heads of 64 rows, 128 columns: 36.4 us; with an address of its own per lane and
 // request and an exit behind every chunk, 40.0.  (Without the requests it takes 25.5, without the stores 30.2.)
-template <typename T, int NT>
-__global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspace w) {
+// A wave of fewer tiles than NT has a loop for as many: under a test per tile the requests would be waited for one by one, and
+// the last tile's again in place of one that is not there made float32 inputs' the bound (2048 tokens, 8 heads of 32 rows, 16
+// columns 34.8 us for 19.4; 256 columns spilled).
+template <typename T, int TILES>
+__device__ __forceinline__ void ssm_state_walk(const SsmArgs &a, const SsmWorkspace &w, const int wave) {
   const uint32_t head = blockIdx.x, v0 = blockIdx.y * 16, group = head / (a.heads / a.groups);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, column = lane & 15, quad = lane >> 4;
-  const uint32_t n = a.state_size, slot = a.step[kStateSlot], tiles = w.np / 16;
+  const int lane = threadIdx.x & 63, column = lane & 15, quad = lane >> 4;
+  const uint32_t n = a.state_size, slot = a.step[kStateSlot];
   const bool fresh = a.step[kStatePosition] == 0;
   const size_t ld = (size_t)a.groups * w.np;
   // lane: state row v, columns k .. k + 3 of every tile; rows beyond the head's end repeat its last one
   const uint32_t v = v0 + column, v_row = min(v, a.vdim - 1);
   float *saved = a.ssm_state + (((size_t)slot * a.heads + head) * a.vdim + v_row) * n;
 
-  f32x4 state[NT];
+  f32x4 state[TILES];
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+  for (int t = 0; t < TILES; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const uint32_t k = (wave + 4 * t) * 16 + quad * 4 + r;
@@ -320,7 +323,7 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
     }
 
   const uint32_t x_at = (v_row * Q + quad * 8) * sizeof(T), b_at = (column * Q + quad * 8) * sizeof(T), tail_at = quad * 32;
-  auto load = [&](StateOperands<T, NT> &o, uint32_t chunk) __attribute__((always_inline)) {
+  auto load = [&](StateOperands<T, TILES> &o, uint32_t chunk) __attribute__((always_inline)) {
     const T *x = static_cast<const T *>(w.xt) + ((size_t)chunk * w.inner + head * a.vdim) * Q;
     const float *tail = w.tail + ((size_t)chunk * a.heads + head) * Q;
     o.end = w.sum[((size_t)chunk * a.heads + head) * 2 * Q + Q - 1];
@@ -329,16 +332,14 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
       o.x[s] = *lane_at<Frag<T>>(x + s * 32, x_at);
       o.tail[s] = *lane_at<f32x8>(tail + s * 32, tail_at);
 #pragma unroll
-      for (int t = 0; t < NT; ++t)  // (a tile that is not there: the last again)
-        o.b[t][s] = *lane_at<Frag<T>>(static_cast<const T *>(w.bt) +
-                                          ((size_t)chunk * ld + group * w.np + min((uint32_t)wave + 4 * t, tiles - 1) * 16) * Q + s * 32,
-                                      b_at);
+      for (int t = 0; t < TILES; ++t)
+        o.b[t][s] = *lane_at<Frag<T>>(
+            static_cast<const T *>(w.bt) + ((size_t)chunk * ld + group * w.np + ((uint32_t)wave + 4 * t) * 16) * Q + s * 32, b_at);
     }
   };
-  auto step = [&](const StateOperands<T, NT> &o, uint32_t chunk) __attribute__((always_inline)) {
+  auto step = [&](const StateOperands<T, TILES> &o, uint32_t chunk) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if ((uint32_t)wave + 4 * t >= tiles) continue;
+    for (int t = 0; t < TILES; ++t) {
       typedef T x4 __attribute__((ext_vector_type(4)));
       const uint32_t at = (wave + 4 * t) / 2 * 512 + (((wave + 4 * t) % 2 * 2 + quad / 2) * 16 + column) * 8 + quad % 2 * 4;
       x4 high;
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
     }
     const float carry = __expf(o.end);
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < TILES; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) state[t][r] *= carry;
 #pragma unroll
@@ -367,12 +368,12 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
 #pragma unroll
       for (int e = 0; e < 8; e += 2) fx.set_pair(e, to_f32(o.x[s][e]) * o.tail[s][e], to_f32(o.x[s][e + 1]) * o.tail[s][e + 1]);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) state[t] = mma_wide_b(o.b[t][s], fx, state[t]);
+      for (int t = 0; t < TILES; ++t) state[t] = mma_wide_b(o.b[t][s], fx, state[t]);
     }
   };
 
   // operands two chunks ahead (one exit from the loop: with one behind every step the compiler waits for all requests at its head)
-  StateOperands<T, NT> ring[3];
+  StateOperands<T, TILES> ring[3];
   load(ring[0], 0);
   load(ring[1], min(1u, w.chunks - 1));
   uint32_t chunk = 0;
@@ -389,12 +390,23 @@ __global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspa
     if (chunk + i < w.chunks) step(ring[i], chunk + i);
   if (v < a.vdim)
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < TILES; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const uint32_t k = (wave + 4 * t) * 16 + quad * 4 + r;
         if (k < n) saved[k] = state[t][r];
       }
+}
+
+template <typename T, int NT>
+__global__ __launch_bounds__(256, 1) void ssm_state_kernel(SsmArgs a, SsmWorkspace w) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tiles = ((int)w.np / 16 - wave + 3) / 4;  // of this wave (4 NT - 8 < np / 16 <= 4 NT)
+  if (tiles >= NT) ssm_state_walk<T, NT>(a, w, wave);
+  if constexpr (NT > 1)
+    if (tiles == NT - 1) ssm_state_walk<T, NT - 1>(a, w, wave);
+  if constexpr (NT > 2)
+    if (tiles == NT - 2) ssm_state_walk<T, NT - 2>(a, w, wave);
 }
 
 // The parallel part: a workgroup per chunk and head, 16 tokens a wave.  y^T of 16 state rows: the incoming

@@ -40,6 +40,8 @@ MECHANISMS = {
     "mamba2 one group": mamba2(heads=5, vdim=16, state=32, groups=1, norm_groups=1),
     "mamba2 group per head": mamba2(heads=4, vdim=33, state=17, groups=4, norm_groups=2, conv=3),
     "mamba2 state of 128": mamba2(heads=2, vdim=64, state=128, groups=1, norm_groups=4, conv=2),
+    "mamba2 state of 90": mamba2(heads=4, vdim=24, state=90, groups=2, norm_groups=1),  # waves of two tiles of 16 and of one
+    "mamba2 state of 150": mamba2(heads=2, vdim=20, state=150, groups=1, norm_groups=1),  # of three and of two
     "mamba2 state of 200": mamba2(heads=2, vdim=8, state=200, groups=2, norm_groups=1, conv=6),
     "mamba2 one tap": mamba2(conv=1),
 }
