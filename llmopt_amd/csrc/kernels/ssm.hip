@@ -446,31 +446,43 @@ __global__ __launch_bounds__(256) void ssm_output_kernel(SsmArgs a, SsmWorkspace
   const uint32_t lane_bytes = lane * 8 * sizeof(T);
   const T *x_head = static_cast<const T *>(w.xt) + ((size_t)chunk * w.inner + head * a.vdim) * Q;
   for (uint32_t v0 = blockIdx.z * 16; v0 < a.vdim; v0 += gridDim.z * 16) {
-    // A tile's operands are requested together, at scalar addresses: 31.4 us at the sizes above, where each request waited in front
-    // of its product 35.3.  (The next tile's as well: 34.4, fewer waves fit; two workgroups over a head's tiles: 42.3.)
-    Frag<T> state[kStatePlanes<T>][STEPS], x[2];
-#pragma unroll
-    for (int plane = 0; plane < kStatePlanes<T>; ++plane) {
+    // bfloat16: a tile's operands are requested together, at scalar addresses: 31.4 us at the sizes above, where each request waited
+    // in front of its product 35.3.  (The next tile's as well: 34.4, fewer waves fit; two workgroups over a head's tiles: 42.3.)
+    // float32's take twice the registers, and the waves that no longer fit cost more: 2048 tokens, 48 heads of 64 rows, 256 columns
+    // together 74 us, each in front of its product 67; 32 heads of 128 rows, 96 columns 42.1 / 40.4, and 44.2 at scalar addresses.
+    constexpr bool TOGETHER = kStatePlanes<T> == 2;
+    const auto state_at = [&](int plane, int s) {
       const T *from = state_block<T>(a, w, chunk, head, plane, v0);
+      return TOGETHER ? *lane_at<Frag<T>>(from + s * 512, lane_bytes) : reinterpret_cast<const Frag<T> *>(from)[s * 64 + lane];
+    };
+    const auto x_at = [&](int s) {
+      const uint32_t v_row = min(v0 + column, a.vdim - 1);
+      if constexpr (TOGETHER) return *lane_at<Frag<T>>(x_head + s * 32, (v_row * Q + quad * 8) * sizeof(T));
+      const T *x = static_cast<const T *>(w.xt) + ((size_t)chunk * w.inner + head * a.vdim + v_row) * Q + quad * 8;
+      return *reinterpret_cast<const Frag<T> *>(x + s * 32);
+    };
+    [[maybe_unused]] Frag<T> state[kStatePlanes<T>][STEPS], x[2];
+    if constexpr (TOGETHER) {
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s)
-        if (s * 32 < (int)w.np) state[plane][s] = *lane_at<Frag<T>>(from + s * 512, lane_bytes);
+      for (int plane = 0; plane < kStatePlanes<T>; ++plane)
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s)
+          if (s * 32 < (int)w.np) state[plane][s] = state_at(plane, s);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) x[s] = x_at(s);
+      __builtin_amdgcn_sched_barrier(0);  // the requests stay ahead of the arithmetic
     }
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-      x[s] = *lane_at<Frag<T>>(x_head + s * 32, (min(v0 + column, a.vdim - 1) * Q + quad * 8) * sizeof(T));
-    __builtin_amdgcn_sched_barrier(0);  // the requests stay ahead of the arithmetic
     f32x4 high = {0.0f, 0.0f, 0.0f, 0.0f}, low = high, within = high;
 #pragma unroll
     for (int s = 0; s < STEPS; ++s)
       if (s * 32 < (int)w.np) {
-        high = mma(state[0][s], fc[s], high);
+        high = mma(TOGETHER ? state[0][s] : state_at(0, s), fc[s], high);
         if constexpr (kStatePlanes<T> == 2) low = mma(state[1][s], fc[s], low);
       }
 #pragma unroll
     for (int s = 0; s < 2; ++s)
       if (s * 32 <= wave * 16 + 15)  // the others come later than all of the wave's tokens
-        within = mma_wide_b(x[s], weight[s], within);
+        within = mma_wide_b(TOGETHER ? x[s] : x_at(s), weight[s], within);
     if (row >= a.m) continue;
     T *out = static_cast<T *>(a.y) + (size_t)row * w.inner + head * a.vdim + v0 + quad * 4;
     typedef T x4 __attribute__((ext_vector_type(4)));
