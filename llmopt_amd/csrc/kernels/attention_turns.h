@@ -191,12 +191,15 @@ __device__ __forceinline__ bool attention_turns(unsigned char *lds, const typena
   const auto values = [&](uint32_t step) __attribute__((always_inline)) {
     typedef short s4_t __attribute__((ext_vector_type(4)));
     typedef s4_t __attribute__((address_space(3))) * lds_chunk_t;
-    const unsigned char *rows = own + v_place(step);
+    // A weight of zero times an infinite value is NaN: 32 keys that no row of the wave sees take the values of the other 32.
+    const uint32_t key = first_key(step);
+    const unsigned char *stage = own + v_place(step);
+    const unsigned char *rows[2] = {stage + (bounds.low_first > key + 31 ? 32 * ROW : 0), stage + (bounds.high_last < key + 32 ? 0 : 32 * ROW)};
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int jj = 0; jj < JJ; ++jj) {
-        const unsigned char *from = rows + v_lane[jj] + s * 16 * ROW;
+        const unsigned char *from = rows[s / 2] + v_lane[jj] + s % 2 * 16 * ROW;
         const s4_t low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_chunk_t)from);
         const s4_t high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_chunk_t)(from + 8 * ROW));
         const x8 operand = __builtin_bit_cast(x8, __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7));

@@ -103,6 +103,35 @@ def test_groups_of_waves_in_turns(runtime, m, heads, kv, dim, vdim, span, softca
     test_tiles(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sliding)
 
 
+@pytest.mark.parametrize("m,dim,softcap", [(700, 128, 0.0), (1100, 128, 30.0), (1100, 128, 200.0), (1100, 64, 0.0)])
+def test_infinite_values_behind_what_a_row_of_a_portion_sees(runtime, m, dim, softcap):
+    """A weight of zero times an infinite value is NaN: not in rows none of whose 32 see any of its 32 keys."""
+    rng = np.random.default_rng(m)
+    heads, kv, span = 4, 2, 4096
+    rows = to_bfloat16(rng.standard_normal((m, (heads + 2 * kv) * dim), dtype=np.float32))
+    put = runtime.buffer_of_bytes
+    zeros = np.zeros((1, kv, span, dim), dtype=np.uint16)
+
+    def call():
+        out = runtime.create_buffer(m * heads * dim * 2)
+        runtime.dispatch("llmopt_chunk_attention_bf16", [put(rows), put(zeros), put(np.zeros(2, dtype=np.uint32)), put(zeros), put(zeros), out],
+                         u32s(m, heads, kv, dim, dim, span, span, 1, 0) + struct.pack("<ff", dim ** -0.5, softcap), *GRID)
+        return out.numpy(np.uint16).reshape(m, heads, dim)
+
+    last = np.minimum(np.arange(m) // 32 * 32 + 31, m - 1)
+    for bad, what in ((40, np.inf), (m - 70, -np.inf), (m - 1, np.nan)):
+        column = (heads + kv + 1) * dim + 5
+        rows[bad, column] = 0
+        want = call()
+        rows[bad, column] = to_bfloat16(np.array([what], dtype=np.float32))[0]
+        got = call()
+        rows[bad, column] = 0
+        touched = np.zeros(got.shape, dtype=bool)
+        touched[bad // 32 * 32 <= last, 2:, 5] = True
+        assert (got[~touched] == want[~touched]).all(), (bad, what)
+        assert not np.isfinite(from_bfloat16(got[bad:, 2:, 5])).any()
+
+
 # rows, heads, kv_heads, dim, span, position of the first row: tiles in the order of their keys (several rounds of up to 64
 # tiles, a chunk's end among them: 5, 16 and 64 tiles), more tiles than are ranked, one chunk, one round
 @pytest.mark.parametrize("m,heads,kv,dim,span,first", [

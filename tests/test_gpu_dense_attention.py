@@ -394,6 +394,33 @@ def test_groups_of_waves_in_turns(runtime, dim, batches, heads, kv_heads, new, p
             assert_close_to_oracle(got[one], want, f"D={dim} {heads}/{kv_heads} {new} after {past}, {mode}, {batch}/{head}")
 
 
+@pytest.mark.parametrize("dim,heads,kv_heads,new,past", [
+    (128, 24, 8, 700, 0), (128, 66, 22, 97, 170), (64, 64, 32, 500, 13), (128, 86, 43, 1031, 0), (64, 64, 32, 1500, 77), (128, 4, 2, 300, 0)])
+def test_infinite_values_behind_what_a_row_sees(runtime, dim, heads, kv_heads, new, past):
+    """A weight of zero times an infinite value is NaN, and 32 rows share tiles of 32 keys: rows none of whose tiles hold a value
+    that is not finite are what they are without it, and rows that see one are not finite."""
+    rng = np.random.default_rng(dim + new)
+    length = past + new
+    query = rng.standard_normal((1, heads, new, dim)).astype(np.float16)
+    key = rng.standard_normal((1, kv_heads, length, dim)).astype(np.float16)
+    value = rng.standard_normal((1, kv_heads, length, dim)).astype(np.float16)
+    params = attention_params(1, heads, new, length, dim, 0, 0, True, dim ** -0.5, kv_heads, past_length=past)
+    call = lambda v: run(runtime, f"llmopt_attention_f16_simd_h{dim}", query, key, v, None, params, (1, heads, new, dim))[0]
+    last = past + np.minimum(np.arange(new) // 32 * 32 + 31, new - 1)  # what the 32 rows of a row see
+    for bad, what in ((past + 40, np.inf), (past + 97 - 33, -np.inf), (length - 1, np.nan)):
+        value[0, 1, bad, 5] = 0
+        want = call(value)
+        assert np.isfinite(want).all()
+        value[0, 1, bad, 5] = what
+        got = call(value)
+        value[0, 1, bad, 5] = 1
+        per = heads // kv_heads
+        touched = np.zeros(got.shape, dtype=bool)
+        touched[per:2 * per, bad // 32 * 32 <= last, 5] = True
+        assert (got[~touched].view(np.uint16) == want[~touched].view(np.uint16)).all(), (bad, what)
+        assert not np.isfinite(got[per:2 * per, np.arange(new) + past >= bad, 5]).any()
+
+
 @pytest.mark.parametrize("heads,kv_heads,new,past,mode", [
     (4, 2, 300, 0, "causal"), (2, 1, 45, 211, "causal"), (2, 2, 33, 100, "none"), (3, 1, 130, 70, "bool"),
     (2, 2, 64, 191, "f16"), (8, 4, 16, 0, "causal"),
