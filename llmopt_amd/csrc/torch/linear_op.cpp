@@ -14,7 +14,9 @@
 #include <cstddef>
 #include <cstdint>
 #include <limits>
+#include <mutex>
 #include <optional>
+#include <shared_mutex>
 
 namespace {
 
@@ -23,7 +25,8 @@ using Launch = int (*)(void *library, const char *name, void *const *pointers, c
 
 constexpr int64_t kGroup = 64;
 std::atomic<Launch> launch{nullptr};
-std::array<std::atomic<void *>, 64> libraries{};  // by device: a context's library, once there is one
+std::array<std::atomic<void *>, 64> libraries{};  // by device: a context's library, while there is one
+std::shared_mutex in_use;                         // shared: a library is being launched from; alone: one comes or goes
 
 bool plain(const at::Tensor &t, at::ScalarType type, c10::Device device) {
   return t.scalar_type() == type && t.device() == device && t.is_contiguous();
@@ -41,8 +44,9 @@ at::Tensor w4a16_linear(const at::Tensor &input, const at::Tensor &packed, const
                         const std::optional<at::Tensor> &bias) {
   const c10::Device device = input.device();
   const int index = device.index();
-  void *library = index >= 0 && index < (int)libraries.size() ? libraries[index].load(std::memory_order_acquire) : nullptr;
-  if (library == nullptr || input.dim() == 0 || packed.dim() != 2 || scale.dim() != 2 || !plain(input, at::kHalf, device) ||
+  if (index < 0 || index >= (int)libraries.size() || libraries[index].load(std::memory_order_relaxed) == nullptr)
+    return general(input, packed, scale, bias);
+  if (input.dim() == 0 || packed.dim() != 2 || scale.dim() != 2 || !plain(input, at::kHalf, device) ||
       !plain(packed, at::kByte, device) || !plain(scale, at::kHalf, device) || (bias && !plain(*bias, at::kHalf, device)))
     return general(input, packed, scale, bias);
   const int64_t n = packed.size(0), k = packed.size(1) * 2, limit = std::numeric_limits<uint32_t>::max();
@@ -60,9 +64,14 @@ at::Tensor w4a16_linear(const at::Tensor &input, const at::Tensor &packed, const
   const size_t lengths[] = {input.nbytes(), packed.nbytes(), scale.nbytes(), addend.nbytes(), output.nbytes()};
   const uint32_t parameters[] = {(uint32_t)m, (uint32_t)n, (uint32_t)k, bias ? 1u : 0u, 0u};  // rows, columns, k, bias, its stride
   // queued on torch's stream; the tensors outlive the launch call
-  const int status = launch.load(std::memory_order_relaxed)(
-      library, m == 1 ? "llmopt_w4a16_linear_f16_g64" : "llmopt_w4a16_linear_f16_g64_m4", pointers, lengths, 5, parameters,
-      sizeof(parameters), c10::hip::getCurrentHIPStream(index).stream());
+  int status = -1;
+  {
+    std::shared_lock<std::shared_mutex> held(in_use);
+    if (void *library = libraries[index].load(std::memory_order_relaxed))  // (another thread may have closed it meanwhile)
+      status = launch.load(std::memory_order_relaxed)(
+          library, m == 1 ? "llmopt_w4a16_linear_f16_g64" : "llmopt_w4a16_linear_f16_g64_m4", pointers, lengths, 5, parameters,
+          sizeof(parameters), c10::hip::getCurrentHIPStream(index).stream());
+  }
   return status < 0 ? general(input, packed, scale, bias) : output;
 }
 
@@ -70,9 +79,11 @@ TORCH_LIBRARY_IMPL(llmopt, CUDA, m) { m.impl("w4a16_linear", w4a16_linear); }  /
 
 }  // namespace
 
-// From here on calls on `device` go to `library` through `function` (llmopt_hip_launch).
+// From here on calls on `device` go to `library` through `function` (llmopt_hip_launch); without a library they go to Python, and
+// no launch from the former one is under way any more.
 extern "C" __attribute__((visibility("default"))) void llmopt_torch_bind(int device, void *library, void *function) {
   if (device < 0 || device >= (int)libraries.size()) return;
-  launch.store(reinterpret_cast<Launch>(function), std::memory_order_relaxed);
-  libraries[device].store(library, std::memory_order_release);
+  std::unique_lock<std::shared_mutex> alone(in_use);
+  if (library != nullptr) launch.store(reinterpret_cast<Launch>(function), std::memory_order_relaxed);
+  libraries[device].store(library, std::memory_order_relaxed);
 }

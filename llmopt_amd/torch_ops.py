@@ -18,6 +18,7 @@ activations and bias, uint8 `[N, K/2]` weights, fp16 `[N, K/64]` scales.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import struct
 import threading
@@ -37,6 +38,22 @@ _runtimes: dict[int, Runtime] = {}
 _lock = threading.Lock()
 
 
+class _OperatorRuntime(Runtime):
+    """A device's runtime: the native side launches from it until it is closed, and calls behind that say that it is."""
+
+    def __init__(self, device: int):
+        super().__init__(device=device)
+        self._unbind = functools.partial(_native.llmopt_torch_bind, device, None, None)
+        # further calls on this device that need nothing but the launch no longer come here
+        _native.llmopt_torch_bind(device, self.library, ctypes.cast(lib().llmopt_hip_launch, ctypes.c_void_p))
+
+    def close(self) -> None:
+        unbind = self.__dict__.pop("_unbind", None)
+        if unbind is not None:
+            unbind()
+        super().close()
+
+
 def _runtime(device_index: int) -> Runtime:
     runtime = _runtimes.get(device_index)
     if runtime is not None:
@@ -44,10 +61,8 @@ def _runtime(device_index: int) -> Runtime:
     with _lock:
         runtime = _runtimes.get(device_index)
         if runtime is None:
-            runtime = Runtime(device=device_index)
+            runtime = _OperatorRuntime(device_index)
             _runtimes[device_index] = runtime
-            # further calls on this device that need nothing but the launch no longer come here
-            _native.llmopt_torch_bind(device_index, runtime.library, ctypes.cast(lib().llmopt_hip_launch, ctypes.c_void_p))
         return runtime
 
 

@@ -153,3 +153,23 @@ def test_native_calls_and_those_left_to_python(op, layout):
         op(x, packed, scale, bias.float())
     with pytest.raises(LlmoptError):
         op(x.new_zeros((3, 64)), packed.new_zeros((0, 32)), scale.new_zeros((0, 1)), None)
+
+
+def test_a_closed_runtime_is_not_launched_from(op):
+    """After its runtime is closed the operator says so, natively and from Python, and a new one takes the calls again."""
+    from llmopt_amd import torch_ops
+    from llmopt_amd.native import LlmoptError
+    rng = np.random.default_rng(12)
+    device = torch.device("cuda:0")
+    case = w4_case(rng, 2, 64, 128, bias=False)
+    tensors = [torch.from_numpy(a).to(device) for a in case[:3]]
+    index = torch.cuda.current_device()
+    op(*tensors, None)
+    torch.cuda.synchronize()
+    torch_ops._runtimes[index].close()
+    for _ in range(2):
+        with pytest.raises(LlmoptError, match="finalized"):
+            op(*tensors, None)
+    del torch_ops._runtimes[index]
+    for _ in range(2):
+        assert_close_to_oracle(op(*tensors, None).cpu().numpy(), oracle.w4a16_linear(*case[:3], None), "reopened")
