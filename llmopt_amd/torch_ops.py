@@ -7,7 +7,8 @@ backs it with its native runtime (native/metal_runtime.cpp:139-147).  This
 module registers the same schema for ROCm tensors: the kernel runs on the
 tensors' own device memory (no copies), is queued on torch's current stream
 and nothing waits for it.  Calls with nothing to refuse or lay out anew are native
-code from torch's dispatcher on (csrc/torch/linear_op.cpp); the others come here.
+code from torch's dispatcher on (csrc/torch/linear_op.cpp); the others come here, and all of
+them where that code is not built for the installed torch.
 
     import llmopt_amd.torch_ops            # registers the operator
     y = torch.ops.llmopt.w4a16_linear(x, packed, scale, bias)
@@ -19,19 +20,19 @@ from __future__ import annotations
 
 import ctypes
 import functools
-import os
 import struct
 import threading
+import warnings
 from typing import Optional
 
 import torch
 
+from .build import torch_library
 from .native import Runtime, lib
 
 GROUP_SIZE = 64
 _ONE_ROW, _ROWS = b"llmopt_w4a16_linear_f16_g64", b"llmopt_w4a16_linear_f16_g64_m4"
 _PARAMETERS = struct.Struct("<5I").pack  # m, n, k, has_bias, bias_row_stride
-_NATIVE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libllmopt_torch.so")
 _library: Optional[torch.library.Library] = None
 _native: Optional[ctypes.CDLL] = None
 _runtimes: dict[int, Runtime] = {}
@@ -43,6 +44,8 @@ class _OperatorRuntime(Runtime):
 
     def __init__(self, device: int):
         super().__init__(device=device)
+        if _native is None:
+            return
         self._unbind = functools.partial(_native.llmopt_torch_bind, device, None, None)
         # further calls on this device that need nothing but the launch no longer come here
         _native.llmopt_torch_bind(device, self.library, ctypes.cast(lib().llmopt_hip_launch, ctypes.c_void_p))
@@ -118,17 +121,20 @@ def register() -> None:
     global _library, _native
     if _library is not None:
         return
-    if not os.path.exists(_NATIVE_PATH):
-        raise ImportError(f"{_NATIVE_PATH} is missing: build it with `python -m llmopt_amd.build`")
     library = torch.library.Library("llmopt", "DEF")
     library.define("w4a16_linear(Tensor input, Tensor packed_weight, Tensor scale, Tensor? bias) -> Tensor")
     # what the native kernel of the above leaves to Python
     library.define("w4a16_linear_general(Tensor input, Tensor packed_weight, Tensor scale, Tensor? bias) -> Tensor")
     library.impl("w4a16_linear_general", _w4a16_linear_hip, "CUDA")  # ROCm tensors carry the CUDA dispatch key
     library.impl("w4a16_linear", _w4a16_linear_meta, "Meta")
-    native = ctypes.CDLL(_NATIVE_PATH)  # (its kernel registers itself as it is loaded)
-    native.llmopt_torch_bind.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
-    native.llmopt_torch_bind.restype = None
+    try:
+        native = ctypes.CDLL(torch_library(torch.__version__))  # (its kernel registers itself as it is loaded)
+        native.llmopt_torch_bind.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+        native.llmopt_torch_bind.restype = None
+    except OSError as error:
+        warnings.warn(f"llmopt::w4a16_linear takes the longer way through Python ({error}); `python -m llmopt_amd.build` builds the other")
+        native = None
+        library.impl("w4a16_linear", _w4a16_linear_hip, "CUDA")
     _library, _native = library, native
 
 
