@@ -97,6 +97,7 @@ def test_tiles(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sli
     (1025, 2, 1, 128, 128, 4096, 50.0, True, 63, False),
     (1061, 4, 2, 64, 64, 1040, 0.0, False, 1000, True),
     (1030, 6, 2, 64, 64, 2048, 0.0, True, 1, False),
+    (660, 4, 2, 128, 128, 640, 0.0, True, 0, False),          # the last rows behind a chunk's end: one stage, a group without any
 ])
 def test_groups_of_waves_in_turns(runtime, m, heads, kv, dim, vdim, span, softcap, sink, first, sliding):
     """Portions whose rows walk over many keys: 128 rows whose stages two groups of waves share."""

@@ -372,9 +372,19 @@ def test_own_tiles_of_a_slab(runtime, dim, heads, kv_heads, new, past, mode):
 ])
 def test_groups_of_waves_in_turns(runtime, dim, batches, heads, kv_heads, new, past, mode):
     """Launches without a mask that fill the device: 128 rows whose keys two groups of waves share, and 256 rows; partial
-    last stages and slabs, groups and waves without keys, both layouts.  Heads of every batch against the oracle."""
+    last stages and slabs, waves without rows, both layouts.  Heads of every batch against the oracle."""
+    check_turns(runtime, dim, batches, heads, kv_heads, new, past, mode)
+
+
+@pytest.mark.parametrize("dim,heads,kv_heads,new,past", [(128, 132, 66, 33, 0), (128, 140, 20, 60, 2), (64, 256, 64, 20, 44)])
+def test_rows_that_see_one_stage_of_many(runtime, dim, heads, kv_heads, new, past):
+    """Keys behind what any row sees: slabs of one stage, which leave the second group of waves without keys."""
+    check_turns(runtime, dim, 1, heads, kv_heads, new, past, "causal", behind=300)
+
+
+def check_turns(runtime, dim, batches, heads, kv_heads, new, past, mode, behind=0):
     rng = np.random.default_rng(dim + heads + new + past)
-    length, scale, causal = past + new, 1.0 / math.sqrt(dim), mode == "causal"
+    length, scale, causal = past + new + behind, 1.0 / math.sqrt(dim), mode == "causal"
     query = rng.standard_normal((batches, heads, new, dim)).astype(np.float16)
     key = (rng.standard_normal((batches, kv_heads, length, dim)) * 2).astype(np.float16)
     value = rng.standard_normal((batches, kv_heads, length, dim)).astype(np.float16)

@@ -124,14 +124,18 @@ def test_a_stream_under_capture_is_refused(op, same):
 
 
 @pytest.mark.parametrize("layout", ["plain", "strided input", "strided weights", "offset input", "bias of two dimensions", "vector"])
-def test_native_calls_and_those_left_to_python(op, layout):
+def test_native_calls_and_those_left_to_python(op, layout, monkeypatch):
     """Once a device has a runtime, calls that need nothing but the launch never reach Python; the others give the same."""
+    from llmopt_amd import torch_ops
     from llmopt_amd.native import LlmoptError
+    in_python, check = [], torch_ops._check_arguments
+    monkeypatch.setattr(torch_ops, "_check_arguments", lambda *args: in_python.append(args) or check(*args))
     rng = np.random.default_rng(11)
     device = torch.device("cuda:0")
     case = w4_case(rng, 4, 96, 128, bias=True)
     x, packed, scale, bias = (torch.from_numpy(a).to(device) for a in case)
     op(x, packed, scale, bias)
+    in_python.clear()
     if layout == "strided input":
         x = torch.cat([x, x], dim=1)[:, :128]
     elif layout == "strided weights":
@@ -147,12 +151,14 @@ def test_native_calls_and_those_left_to_python(op, layout):
         assert out.shape == (*x.shape[:-1], 96) and out.is_contiguous()
         want = oracle.w4a16_linear(*case)
         assert_close_to_oracle(out.cpu().numpy().reshape(-1, 96), want[:1] if layout == "vector" else want, layout)
+    assert len(in_python) == (2 if layout.startswith("strided") else 0)
     with pytest.raises(ValueError, match="features"):
         op(x[..., :64].contiguous(), packed, scale, bias)
     with pytest.raises(TypeError, match="bias must be"):
         op(x, packed, scale, bias.float())
     with pytest.raises(LlmoptError):
         op(x.new_zeros((3, 64)), packed.new_zeros((0, 32)), scale.new_zeros((0, 1)), None)
+    assert len(in_python) == (5 if layout.startswith("strided") else 3)
 
 
 def test_a_closed_runtime_is_not_launched_from(op):

@@ -263,6 +263,8 @@ def test_gpu_tests_reach_both_forms_of_turns(rules):
     reached = [(dim, rules.turns(dim, 0, int(mode == "causal"), new, new + past, past, heads * batches, CUS))
                for dim, batches, heads, _, new, past, mode in sizes(test_gpu_dense_attention.test_groups_of_waves_in_turns, names)]
     assert set(reached) == {(64, 1), (64, 2), (128, 1), (128, 2)}
+    for dim, heads, _, new, past in sizes(test_gpu_dense_attention.test_rows_that_see_one_stage_of_many, "dim,heads,kv_heads,new,past"):
+        assert rules.turns(dim, 0, 1, new, new + past + 300, past, heads, CUS) == 1
 
 
 @pytest.mark.parametrize("dim,capped,m,span,turns", [
