@@ -9,8 +9,8 @@
 // with a barrier behind each, and group 1 (waves 4 .. 7) is one barrier behind group 0, so that while one wave of a SIMD has
 // the matrix core the other has the vector unit.  Waves that were left to themselves did both one after the other: at 32 x 32
 // tiles of heads of 128 the products, the reads of K and V from LDS and the softmax take about as long as each other, and a step
-// took their sum.  The older wave of a SIMD wins where both want to issue: group 1's products go with a higher priority (1890
-// cycles beside a softmax otherwise, group 0's 1250).
+// took their sum.  The older wave of a SIMD wins where both want to issue: group 1's products go with a higher priority (products of
+// heads of 128 in fp16 take 1535 cycles in both groups then; 1890 in group 1 and 1250 in group 0 without).
 //
 //  * SPLIT: both groups own the same 128 rows and take alternate stages of 64 keys, each through two stages of its own in LDS;
 //    group 0 has both shares in the end.  Else 256 rows, and both groups read the same three stages.

@@ -822,10 +822,12 @@ struct TurnsOperand<_Float16> {
 
 namespace {
 
-// Bound by the softmax of one wave beside the products of the other: a step of 64 keys is about 1250 cycles of products
-// (1024 of them the matrix core's) beside 1000 of softmax and 200 of copies, where two free waves took 3200 for it; no copies at
-// all would save another tenth, no exponentials 4 %.  32 / 8 heads of 128, causal: 4096 rows 180 -> 155 us (886 TFLOP/s),
-// 2048 59 -> 48, 1500 46 -> 32; 16 / 4: 4096 105 -> 83, 1900 62 -> 35; 16 / 4 of 64, 4096 rows 68 -> 55.
+// Bound by both sides of a turn and the barriers behind them: at 4096 rows (256-row workgroups) a step of 64 keys is 3650 cycles,
+// products 1535 (1024 of them the matrix core's) and softmax with the copies' requests 1410, beside those of the other group, and
+// 700 of waits; a workgroup starts and ends in 13 to 22 thousand more.  Over the launch the matrix cores are busy 43 % of the time and
+// LDS 33 %, 11 % in conflicts beside that.  No copies at all would save a tenth, no exponentials 4 %.  us, tiles that are not in turns /
+// these, 32 / 8 heads of 128, causal: 4096 rows 180 / 154 (893 TFLOP/s), 2048 59 / 48, 1500 46 / 32; 16 / 4: 4096 105 / 83, 1900 62 / 35;
+// 16 / 4 of 64, 4096 rows 68 / 55.
 // Later rows see more keys and come first, a workgroup a CU.
 template <int D, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void dense_attention_turns_kernel(DenseAttentionArgs a) {
