@@ -31,7 +31,7 @@ UBSAN_LIBRARY = os.path.join(HERE, "libllmopt_hip_ubsan.so")
 # host pass only (each -fsanitize option directly behind -Xarch_host): no runtime library needed
 HOST_UBSAN = ["-Xarch_host", "-fsanitize=undefined,bounds", "-Xarch_host", "-fsanitize-trap=undefined,bounds"]
 
-# -packed-fp32-ops off: hipcc must not form v_pk_*_f32 on this pool.
+# -packed-fp32-ops off: hipcc must not form v_pk_*_f32, some forms of which have given wrong results now and then.
 COMMON = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-Wall", "-Wno-unused-function", "-fno-gpu-sanitize"]
