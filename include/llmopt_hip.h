@@ -117,6 +117,10 @@ int llmopt_hip_create_buffer(llmopt_hip_context *context, int64_t bytes, llmopt_
 /* caml_llmopt_metal_map_file (:863-943): the whole file becomes one device
  * buffer (tensor payloads keep their 256-byte alignment). */
 int llmopt_hip_map_file(llmopt_hip_context *context, const char *path, llmopt_hip_buffer **out);
+/* Nobody asks for this buffer's contents: what a retained plan writes to it is read by the plan's later
+ * records only, and a plan may hand it on some other way and leave the buffer as it was.  Views made from
+ * it afterwards are scratch too. */
+int llmopt_hip_buffer_set_scratch(llmopt_hip_buffer *buffer);
 /* caml_llmopt_metal_buffer_view (:945-970): shares and retains the parent. */
 int llmopt_hip_buffer_view(llmopt_hip_buffer *parent, int64_t offset, int64_t length,
                            llmopt_hip_buffer **out);
@@ -267,6 +271,9 @@ int llmopt_hip_prebaked_bind_step(llmopt_hip_prebaked *plan, llmopt_hip_buffer *
 /* 1 when execute replays one HIP graph, 0 when it launches record by record
  * (no reference counterpart; for diagnostics and tests). */
 int llmopt_hip_prebaked_is_single_submission(llmopt_hip_prebaked *plan);
+/* The layers of the plan that execute runs as one resident launch, 0 when it launches every record (no
+ * reference counterpart; for diagnostics and tests). */
+int llmopt_hip_prebaked_resident_layers(llmopt_hip_prebaked *plan);
 
 /* ---- ring queue ------------------------------------------------------------ */
 

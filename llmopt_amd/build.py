@@ -46,6 +46,7 @@ PER_FILE = {
     "q8_attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "chunk_attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "delta.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "decode_resident.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "mixer_step.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 

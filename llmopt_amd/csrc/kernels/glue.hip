@@ -434,10 +434,20 @@ namespace {
 // native/ocaml_metal_stubs.m:1570-1577) and the context length every sequence attends to.
 __global__ void plan_state_kernel(int64_t *token, int64_t value, const int32_t *chain_from, uint32_t *past,
                                   uint32_t past_value, uint32_t past_count, uint32_t *checkpoint,
-                                  uint32_t checkpoint_value) {
+                                  uint32_t checkpoint_value, uint32_t *resident, uint32_t resident_tag) {
+  if (threadIdx.x == 0 && resident != nullptr) {
+    resident[0] = resident_tag;
+    resident[1] = 0;
+  }
   if (threadIdx.x == 0 && token != nullptr) *token = chain_from != nullptr ? (int64_t)*chain_from : value;
   if (threadIdx.x == 0 && checkpoint != nullptr) *checkpoint = checkpoint_value;
   for (uint32_t i = threadIdx.x; i < past_count; i += blockDim.x) past[i] = past_value;
+}
+
+__global__ void plan_result_kernel(const int32_t *output, const uint32_t *failed, int32_t *host) {
+  if (threadIdx.x != 0) return;
+  host[0] = output != nullptr ? *output : 0;
+  host[1] = (int32_t)*failed;
 }
 
 // *found = 1 when the range holds a NaN (not an infinity): fp16 words, or float32 words.
@@ -467,9 +477,14 @@ hipError_t launch_nan_scan(const void *data, size_t bytes, bool f32, uint32_t *f
 
 hipError_t launch_plan_state(int64_t *token, int64_t value, const int32_t *chain_from, uint32_t *past,
                              uint32_t past_value, uint32_t past_count, uint32_t *checkpoint, uint32_t checkpoint_value,
-                             hipStream_t stream) {
+                             uint32_t *resident, uint32_t resident_tag, hipStream_t stream) {
   hipLaunchKernelGGL(plan_state_kernel, dim3(1), dim3(256), 0, stream, token, value, chain_from, past, past_value,
-                     past_count, checkpoint, checkpoint_value);
+                     past_count, checkpoint, checkpoint_value, resident, resident_tag);
+  return hipGetLastError();
+}
+
+hipError_t launch_plan_result(const int32_t *output, const uint32_t *failed, int32_t *host, hipStream_t stream) {
+  hipLaunchKernelGGL(plan_result_kernel, dim3(1), dim3(64), 0, stream, output, failed, host);
   return hipGetLastError();
 }
 

@@ -144,6 +144,52 @@ struct FusedFfnArgs {
 bool fused_ffn_ok(uint32_t m, uint32_t n, uint32_t k, bool pending = false, uint32_t slice = 64);
 hipError_t launch_fused_ffn(const FusedFfnArgs &args, hipStream_t stream);
 
+// ---- all layers of a decode step in one resident launch (decode_resident.hip) ---------------------
+struct ResidentLayer {
+  const uint8_t *weight[7];  // q, k, v, o, gate, up, down
+  const uint16_t *scale[7];
+  const uint16_t *attention_norm, *ffn_norm;
+  uint32_t key_offset, value_offset;  // of the layer in a token's slot
+};
+constexpr uint32_t kResidentRows = 48, kResidentLayers = 64;
+// Where the handed-over words of each kind begin, in 64-bit words.
+struct ResidentWords {
+  uint32_t x, mid, qkv, attention, product, parts, total;
+  uint32_t in[4], out[4];  // of the products: QKV, output, gate and up, down
+};
+struct ResidentArgs {
+  const ResidentLayer *layers;  // in device memory
+  uint32_t layer_count;
+  uint32_t m, h, q_heads, kv_heads, per_kv, mlp;  // per_kv = q_heads / kv_heads
+  float attention_epsilon, ffn_epsilon, scale;
+  const uint16_t *x_in;  // f16 [m, h]; may be x_out
+  uint16_t *x_out;
+  const uint16_t *cosine, *sine;  // f16 [m, 64]
+  const uint32_t *new_slots;      // [m]
+  uint8_t *pool;
+  uint32_t token_elements, token_stride;
+  const uint32_t *slots, *past_lengths, *slot_offsets;
+  uint32_t max_past;
+  uint64_t *hand;       // words.total words; zero before the first step
+  ResidentWords words;
+  const uint32_t *tag;  // of the step's first layer: layer_count + 1 apart from step to step, never 0
+  uint32_t *failed;     // set when a wait ran out: what the step left is then not to be used
+  uint64_t wait_ticks;  // of wall_clock64 (10 ns)
+  struct {              // byte offsets in the workgroup's memory, set by resident_lds
+    uint32_t new_rows, new_score, run_out, reduce, scales, gains, squares, patches, slots, layers, merge;
+  } lds;
+  uint32_t unit_rows[4], tiles[4], units[4];  // of the products: sequences and column tiles of a unit, units; set by resident_lds
+};
+bool resident_ok(uint32_t m, uint32_t h, uint32_t q_heads, uint32_t kv_heads, uint32_t mlp, uint32_t layers);
+// At most one a compute unit; at least m, or the launch is refused.
+uint32_t resident_workgroups(uint32_t m, uint32_t h, uint32_t q_heads, uint32_t kv_heads, uint32_t mlp, uint32_t compute_units);
+ResidentWords resident_words(uint32_t m, uint32_t h, uint32_t q_heads, uint32_t kv_heads, uint32_t mlp, uint32_t workgroups);
+// Lays out the workgroup's memory; its bytes.
+uint32_t resident_lds(ResidentArgs &args, uint32_t workgroups);
+// True when the launch's workgroups can all be resident at once and each sequence has one at least.
+bool resident_fits(const ResidentArgs &args, uint32_t workgroups, uint32_t lds);
+hipError_t launch_decode_resident(const ResidentArgs &args, uint32_t workgroups, uint32_t lds, hipStream_t stream);
+
 // The product kernels' own nibble decoders run over a whole matrix, as float32 [n, k]:
 // decoder 0 = w4_decode_pairs and 1 = w4_decode_biased (minus its bias), each times the float32
 // scale, i.e. the exact q * s of python/llmopt_backend/quantization.py:91-121; decoder 2 = the
@@ -345,11 +391,13 @@ struct PointwiseArgs {
 hipError_t launch_add_f16(const PointwiseArgs &args, hipStream_t stream);
 
 hipError_t launch_copy_bytes(void *destination, const void *source, size_t bytes, hipStream_t stream);
-// One small launch that sets a retained plan's per-step state: *token = *chain_from (when not
+// One small launch that sets a retained plan's per-step state: resident (when not null) to {resident_tag, 0}, *token = *chain_from (when not
 // null; int32 widened) or `value` (token may be null), and past[0..past_count) = past_value.
 hipError_t launch_plan_state(int64_t *token, int64_t value, const int32_t *chain_from, uint32_t *past,
                              uint32_t past_value, uint32_t past_count, uint32_t *checkpoint, uint32_t checkpoint_value,
-                             hipStream_t stream);
+                             uint32_t *resident, uint32_t resident_tag, hipStream_t stream);
+// host (pinned memory): the step's output word and whether its resident launch gave up.
+hipError_t launch_plan_result(const int32_t *output, const uint32_t *failed, int32_t *host, hipStream_t stream);
 
 // Sets *found (device memory) to 1 when [data, data + bytes) holds a NaN, read as fp16 words or
 // (f32) as float32 words; leaves it alone otherwise.

@@ -14,6 +14,7 @@
 // per-sequence lengths of the batched extension) are read by the kernels from device memory
 // anyway.
 #include "kernels/kernels.h"
+#include "resident.h"
 #include "runtime.h"
 
 #include <pthread.h>
@@ -27,6 +28,34 @@
 #include <string>
 
 using namespace llmopt;
+
+namespace llmopt {
+
+// The second graph of a plan whose records hold whole layers (find_resident_run): one launch in their place.  The first
+// graph stays for steps that find the device's place for resident launches taken, and for good after a launch of this
+// plan gave up waiting.
+struct ResidentPlan {
+  ResidentRun run;
+  uint32_t workgroups = 0, lds = 0;
+  void *layers = nullptr;       // device
+  uint64_t *hand = nullptr;     // device
+  uint32_t *words = nullptr;    // device: the step's tag, and whether it gave up
+  int32_t *host = nullptr;      // pinned: the output word, and whether the step gave up
+  uint32_t next_tag = 1;
+  bool gave_up = false;
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t executable = nullptr;
+  ~ResidentPlan() {
+    if (executable) (void)hipGraphExecDestroy(executable);
+    if (graph) (void)hipGraphDestroy(graph);
+    if (layers) (void)hipFree(layers);
+    if (hand) (void)hipFree(hand);
+    if (words) (void)hipFree(words);
+    if (host) (void)hipHostFree(host);
+  }
+};
+
+}  // namespace llmopt
 
 struct llmopt_hip_prebaked : llmopt::RefCounted {
   llmopt_hip_library *library = nullptr;
@@ -63,6 +92,7 @@ struct llmopt_hip_prebaked : llmopt::RefCounted {
   hipGraphExec_t executable = nullptr;
   uint64_t workspace_generation = 0;
   uint32_t *debug_flag = nullptr;  // device word of the NaN-check replay
+  std::unique_ptr<ResidentPlan> resident;  // null: every step launches all records
 };
 
 namespace {
@@ -72,19 +102,36 @@ void destroy_graph(llmopt_hip_prebaked *plan) {
   if (plan->graph) (void)hipGraphDestroy(plan->graph);
   plan->executable = nullptr;
   plan->graph = nullptr;
+  if (plan->resident) {
+    if (plan->resident->executable) (void)hipGraphExecDestroy(plan->resident->executable);
+    if (plan->resident->graph) (void)hipGraphDestroy(plan->resident->graph);
+    plan->resident->executable = nullptr;
+    plan->resident->graph = nullptr;
+  }
 }
 
-int launch_records(llmopt_hip_prebaked *plan) {
+int launch_records(llmopt_hip_prebaked *plan, bool resident) {
   llmopt_hip_context *context = plan->library->context;
-  for (const DispatchRecord &record : plan->records)
-    if (int status = launch_record(context, record)) return status;
+  const ResidentPlan *const r = plan->resident.get();
+  for (size_t i = 0; i < plan->records.size(); ++i) {
+    if (resident && i == r->run.first) {
+      LLMOPT_HIP_TRY(launch_decode_resident(r->run.args, r->workgroups, r->lds, context->stream), "HIP resident launch failed");
+      i += r->run.count - 1;
+      continue;
+    }
+    if (int status = launch_record(context, plan->records[i])) return status;
+  }
+  if (resident) {
+    const int32_t *output = plan->output_buffer && plan->output_buffer->length >= 4
+                                ? reinterpret_cast<const int32_t *>(plan->output_buffer->device) : nullptr;
+    LLMOPT_HIP_TRY(launch_plan_result(output, r->words + 1, r->host, context->stream), "HIP could not hand out the step's result");
+  }
   return LLMOPT_OK;
 }
 
-// Captures the records into plan->graph / plan->executable.  Nothing runs on the GPU.
-int capture_plan(llmopt_hip_prebaked *plan) {
+// Captures the records (resident: with the resident launch in the place of its run) into a graph.  Nothing runs on the GPU.
+int capture_records(llmopt_hip_prebaked *plan, bool resident, hipGraph_t *out_graph, hipGraphExec_t *out_executable) {
   llmopt_hip_context *context = plan->library->context;
-  destroy_graph(plan);
   // allocated and cleared outside the capture (kernels that split a tile over workgroups)
   uint32_t counter_count = 0;
   if (context_counters(context, &counter_count) == nullptr) return LLMOPT_ERR_FAILURE;
@@ -95,7 +142,7 @@ int capture_plan(llmopt_hip_prebaked *plan) {
       context->sizing_capture = false;
       return fail(LLMOPT_ERR_FAILURE, "HIP stream capture could not begin");
     }
-    int status = launch_records(plan);
+    int status = launch_records(plan, resident);
     hipGraph_t graph = nullptr;
     const hipError_t ended = hipStreamEndCapture(context->stream, &graph);
     context->sizing_capture = false;
@@ -111,22 +158,78 @@ int capture_plan(llmopt_hip_prebaked *plan) {
       if (context_workspace(context, context->sizing_wanted) == nullptr) return LLMOPT_ERR_FAILURE;
       continue;
     }
-    plan->graph = graph;
-    if (hipGraphInstantiate(&plan->executable, graph, nullptr, nullptr, 0) != hipSuccess) {
-      destroy_graph(plan);
+    *out_graph = graph;
+    if (hipGraphInstantiate(out_executable, graph, nullptr, nullptr, 0) != hipSuccess) {
+      *out_executable = nullptr;
       return fail(LLMOPT_ERR_FAILURE, "HIP graph instantiation failed");
     }
-    plan->workspace_generation = context->workspace_generation;
     return LLMOPT_OK;
   }
   return fail(LLMOPT_ERR_FAILURE, "prebaked HIP plan could not settle its kernel workspace");
+}
+
+int capture_plan(llmopt_hip_prebaked *plan) {
+  destroy_graph(plan);
+  int status = capture_records(plan, false, &plan->graph, &plan->executable);
+  // (the records' own workspace is as large as it gets by now)
+  if (status == LLMOPT_OK && plan->resident)
+    status = capture_records(plan, true, &plan->resident->graph, &plan->resident->executable);
+  if (status != LLMOPT_OK) {
+    destroy_graph(plan);
+    return status;
+  }
+  plan->workspace_generation = plan->library->context->workspace_generation;
+  return LLMOPT_OK;
+}
+
+// Resident launches wait for each other's workgroups only within a launch; two at a time on one device could each hold
+// places that the other needs, so a process has one at a time there.
+std::atomic<bool> resident_busy[64];
+
+// How long a wave of a resident launch waits for a word before it gives up.
+uint64_t resident_wait_ticks() {
+  const char *text = getenv("LLMOPT_RESIDENT_WAIT_US");
+  const long long microseconds = text ? atoll(text) : 500000;
+  return (uint64_t)std::max<long long>(0, microseconds) * 100;  // wall_clock64: 100 MHz
+}
+
+// The resident launch of the plan's records, if they hold one and the device is there for it.  What fails here leaves the
+// plan without.
+void prepare_resident(llmopt_hip_prebaked *plan) {
+  llmopt_hip_context *context = plan->library->context;
+  std::unique_ptr<ResidentPlan> r(new ResidentPlan());
+  if (context->device < 0 || context->device >= 64 || !find_resident_run(plan->records, &r->run)) return;
+  ResidentArgs &a = r->run.args;
+  r->workgroups = resident_workgroups(a.m, a.h, a.q_heads, a.kv_heads, a.mlp, (uint32_t)context->compute_units);
+  a.words = resident_words(a.m, a.h, a.q_heads, a.kv_heads, a.mlp, r->workgroups);
+  a.wait_ticks = resident_wait_ticks();
+  r->lds = resident_lds(a, r->workgroups);
+  if (!resident_fits(a, r->workgroups, r->lds)) return;
+  const size_t layer_bytes = r->run.layers.size() * sizeof(ResidentLayer), hand_bytes = (size_t)a.words.total * 8;
+  bool ok = hipMalloc(&r->layers, layer_bytes) == hipSuccess &&
+            hipMalloc(reinterpret_cast<void **>(&r->hand), hand_bytes) == hipSuccess &&
+            hipMalloc(reinterpret_cast<void **>(&r->words), 8) == hipSuccess &&
+            hipHostMalloc(reinterpret_cast<void **>(&r->host), 8, hipHostMallocDefault) == hipSuccess;
+  if (ok) {
+    a.layers = static_cast<const ResidentLayer *>(r->layers);
+    a.hand = r->hand;
+    a.tag = r->words;
+    a.failed = r->words + 1;
+    ok = hipMemcpy(r->layers, r->run.layers.data(), layer_bytes, hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemset(r->hand, 0, hand_bytes) == hipSuccess && hipMemset(r->words, 0, 8) == hipSuccess && hipDeviceSynchronize() == hipSuccess;
+  }
+  if (!ok) {
+    (void)hipGetLastError();
+    return;
+  }
+  plan->resident = std::move(r);
 }
 
 // Queues one step on the context's stream: state, records, and the copy of the first int32 of
 // the output buffer to `host_token` (pinned memory, or pageable when the caller waits right
 // after).  chain: the input token is the output token the previous step left in the output
 // buffer (the reference's llmopt_chain_token_id launch).
-int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t past_tokens, int32_t *host_token) {
+int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t past_tokens, int32_t *host_token, bool resident = false) {
   const uint32_t checkpoint = plan->checkpoint;
   llmopt_hip_context *context = plan->library->context;
   if (int status = use_device(context)) return status;
@@ -148,11 +251,23 @@ int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t p
     if (plan->executable == nullptr || plan->workspace_generation != context->workspace_generation)
       if (int status = capture_plan(plan)) return status;
     LLMOPT_HIP_TRY(launch_plan_state(token_slot, token, chain_from, plan->past_words(), (uint32_t)past_tokens,
-                                     plan->past_word_count(), plan->checkpoint_word(), checkpoint, context->stream),
+                                     plan->past_word_count(), plan->checkpoint_word(), checkpoint,
+                                     resident ? plan->resident->words : nullptr, resident ? plan->resident->next_tag : 0,
+                                     context->stream),
                    "HIP could not write the decode step's state");
+    if (resident) {
+      ResidentPlan &r = *plan->resident;
+      r.next_tag += r.run.args.layer_count + 1;
+      if (r.next_tag > 0xffffff00u) {  // a word that is not rewritten before the tags come round must not pass for a new one
+        LLMOPT_HIP_TRY(hipMemsetAsync(r.hand, 0, (size_t)r.run.args.words.total * 8, context->stream), "HIP could not clear the handed-over words");
+        r.next_tag = 1;
+      }
+      LLMOPT_HIP_TRY(hipGraphLaunch(r.executable, context->stream), "HIP graph launch failed");
+      return LLMOPT_OK;  // (the result is in r.host)
+    }
     LLMOPT_HIP_TRY(hipGraphLaunch(plan->executable, context->stream), "HIP graph launch failed");
   } else {
-    LLMOPT_HIP_TRY(launch_plan_state(token_slot, token, chain_from, nullptr, 0, 0, nullptr, 0, context->stream),
+    LLMOPT_HIP_TRY(launch_plan_state(token_slot, token, chain_from, nullptr, 0, 0, nullptr, 0, nullptr, 0, context->stream),
                    "HIP could not write the decode token");
     for (size_t i = 0; i < plan->records.size(); ++i) {
       DispatchRecord &record = plan->records[i];
@@ -223,7 +338,7 @@ int debug_step(llmopt_hip_prebaked *plan, int64_t token, int64_t past_tokens, bo
   // frozen records read the context length from the plan's device words, the others from byte 12
   LLMOPT_HIP_TRY(launch_plan_state(token_slot, token, nullptr, plan->single_submission ? plan->past_words() : nullptr,
                                    (uint32_t)past_tokens, plan->single_submission ? plan->past_word_count() : 0,
-                                   plan->single_submission ? plan->checkpoint_word() : nullptr, plan->checkpoint,
+                                   plan->single_submission ? plan->checkpoint_word() : nullptr, plan->checkpoint, nullptr, 0,
                                    context->stream),
                  "HIP could not write the decode step's state");
   hipEvent_t before = nullptr, after = nullptr;
@@ -410,6 +525,11 @@ int llmopt_hip_prebaked_create(llmopt_hip_library *library, const llmopt_hip_dis
           plan->records[i].device_checkpoint = plan->device_checkpoint;
         }
       }
+      try {
+        prepare_resident(plan);
+      } catch (const std::exception &) {
+        plan->resident.reset();
+      }
       status = capture_plan(plan);
     }
   }
@@ -427,6 +547,7 @@ void llmopt_hip_release_prebaked(llmopt_hip_prebaked *plan) {
   (void)hipSetDevice(context->device);
   (void)hipStreamSynchronize(context->stream);
   destroy_graph(plan);
+  plan->resident.reset();
   if (plan->device_past) (void)hipFree(plan->device_past);
   if (plan->debug_flag) (void)hipFree(plan->debug_flag);
   for (DispatchRecord &record : plan->records) drop_record(&record);
@@ -454,6 +575,21 @@ int llmopt_hip_prebaked_execute(llmopt_hip_prebaked *plan, int64_t token, int64_
     if (out_token) *out_token = (int64_t)next_token;
     return LLMOPT_OK;
   }
+  if (plan->resident && !plan->resident->gave_up) {
+    std::atomic<bool> &busy = resident_busy[plan->library->context->device];
+    if (!busy.exchange(true, std::memory_order_acquire)) {
+      int status = enqueue_step(plan, token, false, past_tokens, nullptr, true);
+      if (hipStreamSynchronize(plan->library->context->stream) != hipSuccess && status == LLMOPT_OK)
+        status = fail(LLMOPT_ERR_FAILURE, "Prebaked HIP batch failed");
+      busy.store(false, std::memory_order_release);
+      if (status != LLMOPT_OK) return status;
+      if (plan->resident->host[1] == 0) {
+        if (out_token) *out_token = (int64_t)plan->resident->host[0];
+        return LLMOPT_OK;
+      }
+      plan->resident->gave_up = true;  // the step again, launch by launch: what it wrote so far is written anew
+    }
+  }
   if (int status = enqueue_step(plan, token, false, past_tokens, &next_token)) return status;
   if (hipStreamSynchronize(plan->library->context->stream) != hipSuccess)
     return fail(LLMOPT_ERR_FAILURE, "Prebaked HIP batch failed");
@@ -474,6 +610,11 @@ int llmopt_hip_prebaked_bind_step(llmopt_hip_prebaked *plan, llmopt_hip_buffer *
   plan->past_capacity = (uint32_t)max_past_tokens;
   plan->checkpoint_limit = (uint32_t)slots - 1;
   return LLMOPT_OK;
+}
+
+int llmopt_hip_prebaked_resident_layers(llmopt_hip_prebaked *plan) {
+  if (plan == nullptr) return fail(LLMOPT_ERR_FAILURE, "HIP prebaked plan has been finalized");
+  return plan->resident && !plan->resident->gave_up ? (int)plan->resident->run.args.layer_count : 0;
 }
 
 int llmopt_hip_prebaked_is_single_submission(llmopt_hip_prebaked *plan) {

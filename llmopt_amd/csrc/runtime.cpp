@@ -484,7 +484,14 @@ int llmopt_hip_buffer_view(llmopt_hip_buffer *parent, int64_t offset, int64_t le
   retain(parent);
   view->device = parent->device + offset;
   view->length = (size_t)length;
+  view->scratch = parent->scratch;
   *out = view;
+  return LLMOPT_OK;
+}
+
+int llmopt_hip_buffer_set_scratch(llmopt_hip_buffer *buffer) {
+  if (buffer == nullptr) return fail(LLMOPT_ERR_FAILURE, "HIP buffer has been finalized");
+  buffer->scratch = true;
   return LLMOPT_OK;
 }
 

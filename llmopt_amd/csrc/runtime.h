@@ -70,6 +70,7 @@ struct llmopt_hip_buffer : llmopt::RefCounted {
   uint8_t *device = nullptr;            // address of byte 0 of this buffer
   size_t length = 0;
   bool owns_memory = false;
+  bool scratch = false;  // see llmopt_hip_buffer_set_scratch
 };
 
 struct llmopt_hip_library : llmopt::RefCounted {

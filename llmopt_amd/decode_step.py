@@ -219,10 +219,12 @@ class DecodeStep:
             "layers": [{key: (tuple(b(a) for a in value) if isinstance(value, tuple) else b(value))
                         for key, value in layer.items()} for layer in weights["layers"]],
         }
-        create = runtime.create_buffer
+        # what the launches of a layer hand to each other; the rows that come in and go out are in x[0]
+        # (a runtime that knows no scratch gives ordinary buffers)
+        create = getattr(runtime, "create_scratch", runtime.create_buffer)
         q_bytes, kv_bytes = batch * c.q_heads * c.head_dim * 2, batch * c.kv_heads * c.head_dim * 2
         self.work = {
-            "x": [create(batch * h * 2), create(batch * h * 2)],
+            "x": [runtime.create_buffer(batch * h * 2), create(batch * h * 2)],
             "q": create(q_bytes), "k": create(kv_bytes), "v": create(kv_bytes),
             "q_rot": create(q_bytes), "k_rot": create(kv_bytes),
             "attention": create(q_bytes),

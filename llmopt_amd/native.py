@@ -79,6 +79,7 @@ def lib() -> ctypes.CDLL:
         "llmopt_hip_create_buffer": (ctypes.c_int, [vp, i64, pp]),
         "llmopt_hip_map_file": (ctypes.c_int, [vp, ctypes.c_char_p, pp]),
         "llmopt_hip_buffer_view": (ctypes.c_int, [vp, i64, i64, pp]),
+        "llmopt_hip_buffer_set_scratch": (ctypes.c_int, [vp]),
         "llmopt_hip_buffer_wrap": (ctypes.c_int, [vp, vp, sz, pp]),
         "llmopt_hip_release_buffer": (None, [vp]),
         "llmopt_hip_buffer_contents": (ctypes.c_int, [vp, vp, sz]),
@@ -116,6 +117,7 @@ def lib() -> ctypes.CDLL:
         "llmopt_hip_prebaked_execute": (ctypes.c_int, [vp, i64, i64, i64, ctypes.POINTER(i64)]),
         "llmopt_hip_prebaked_bind_step": (ctypes.c_int, [vp, vp, i64, i64]),
         "llmopt_hip_prebaked_is_single_submission": (ctypes.c_int, [vp]),
+        "llmopt_hip_prebaked_resident_layers": (ctypes.c_int, [vp]),
         "llmopt_hip_ring_create": (ctypes.c_int, [pp]),
         "llmopt_hip_ring_submit": (ctypes.c_int, [vp, i64, i64, i64, i64]),
         "llmopt_hip_ring_wait_completion": (ctypes.c_int, [vp, ctypes.POINTER(i64), ctypes.POINTER(i64),
@@ -142,7 +144,7 @@ EXPORTED_SYMBOLS = (
     "llmopt_hip_load_library", "llmopt_hip_release_library", "llmopt_hip_has_function",
     "llmopt_hip_preload_pipeline", "llmopt_hip_function_count", "llmopt_hip_function_name",
     "llmopt_hip_buffer_of_bytes", "llmopt_hip_create_buffer", "llmopt_hip_map_file",
-    "llmopt_hip_buffer_view", "llmopt_hip_buffer_wrap", "llmopt_hip_release_buffer",
+    "llmopt_hip_buffer_view", "llmopt_hip_buffer_wrap", "llmopt_hip_release_buffer", "llmopt_hip_buffer_set_scratch",
     "llmopt_hip_buffer_contents", "llmopt_hip_buffer_length", "llmopt_hip_buffer_device_pointer",
     "llmopt_hip_buffer_copy", "llmopt_hip_buffer_write", "llmopt_hip_buffer_set_int64",
     "llmopt_hip_buffer_set_u32_array", "llmopt_hip_buffer_argmax_f16", "llmopt_hip_f16_argmax",
@@ -152,7 +154,7 @@ EXPORTED_SYMBOLS = (
     "llmopt_hip_commit_batch", "llmopt_hip_commit_batch_async",
     "llmopt_hip_commit_batch_profiled", "llmopt_hip_commit_batch_profiled_each", "llmopt_hip_abort_batch",
     "llmopt_hip_prebaked_create", "llmopt_hip_release_prebaked", "llmopt_hip_prebaked_execute",
-    "llmopt_hip_prebaked_bind_step", "llmopt_hip_prebaked_is_single_submission",
+    "llmopt_hip_prebaked_bind_step", "llmopt_hip_prebaked_is_single_submission", "llmopt_hip_prebaked_resident_layers",
     "llmopt_hip_ring_create", "llmopt_hip_ring_submit", "llmopt_hip_ring_wait_completion",
     "llmopt_hip_ring_poll_completion", "llmopt_hip_ring_start_worker", "llmopt_hip_ring_start_worker_with",
     "llmopt_hip_ring_destroy",
@@ -350,6 +352,12 @@ class Runtime:
         _check(lib().llmopt_hip_create_buffer(self._context, nbytes, ctypes.byref(out)))
         return Buffer(out.value, self)
 
+    def create_scratch(self, nbytes: int) -> Buffer:
+        """A buffer that the records behind the one that writes it read, and nobody else: a plan may do without it."""
+        buffer = self.create_buffer(nbytes)
+        _check(lib().llmopt_hip_buffer_set_scratch(buffer.handle))
+        return buffer
+
     def map_file(self, path: str) -> Buffer:
         out = ctypes.c_void_p()
         _check(lib().llmopt_hip_map_file(self._context, path.encode(), ctypes.byref(out)))
@@ -482,6 +490,13 @@ class Prebaked:
         """Every execute writes its past_tokens and checkpoint into the two u32 words of `step_words`,
         which the plan's records read as position and state slot."""
         _check(lib().llmopt_hip_prebaked_bind_step(self._handle, step_words.handle, max_past_tokens, slots))
+
+    @property
+    def resident_layers(self) -> int:
+        """Layers that a step runs as one resident launch."""
+        status = lib().llmopt_hip_prebaked_resident_layers(self._handle)
+        _check(status)
+        return status
 
     @property
     def single_submission(self) -> bool:

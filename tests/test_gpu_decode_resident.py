@@ -1,0 +1,165 @@
+"""All layers of a decode step in one resident launch (a retained plan's, kernels/decode_resident.hip): several tokens
+against the oracle chain and against the same records launched one by one."""
+import numpy as np
+import pytest
+
+from oracle.chain import decode_chain
+from tests.test_gpu_prebaked import build_step, make_case
+
+pytestmark = pytest.mark.gpu
+
+# sequences, their contexts, hidden, query and KV heads, mlp, layers
+CASES = [
+    ([2048], 576, 9, 3, 1536, 4),                                # one sequence, many runs
+    ([0], 64, 1, 1, 64, 4),                                      # no context, the smallest sizes
+    ([5, 64, 300], 576, 9, 3, 1536, 5),                          # launches of small batches
+    ([15, 16, 17, 31, 33, 1, 0, 129, 700, 2, 64, 3, 8, 9, 10, 11], 320, 4, 2, 192, 4),  # a whole tile of sequences
+    ([40 * i for i in range(17)], 576, 9, 3, 1536, 4),           # a sequence beyond a tile; five launches a layer
+    ([3000] + [7 * i % 90 for i in range(47)], 256, 16, 4, 2048, 4),  # three tiles, one long context, the most heads
+    ([9000], 64, 1, 1, 64, 4),                                   # more tokens a run than it holds slots of
+    ([100, 90], 1024, 16, 1, 640, 4),                            # the widest rows, all heads on one KV head
+]
+
+
+@pytest.fixture(scope="module")
+def runtime():
+    from llmopt_amd.native import Runtime
+    rt = Runtime()
+    yield rt
+    rt.close()
+
+
+@pytest.mark.parametrize("lengths, hidden, q_heads, kv_heads, mlp, layers", CASES)
+def test_resident_layers(runtime, lengths, hidden, q_heads, kv_heads, mlp, layers):
+    from llmopt_amd.decode_step import DecodeConfig, random_weights
+    from llmopt_amd.native import Prebaked
+    print(f"resident layers m={len(lengths)} hidden={hidden} heads={q_heads}/{kv_heads} mlp={mlp} seed=3", flush=True)
+    rng = np.random.default_rng(3)
+    config = DecodeConfig(hidden=hidden, q_heads=q_heads, kv_heads=kv_heads, head_dim=64, mlp=mlp, layers=layers, vocabulary=500)
+    weights = random_weights(config, rng)
+    room, batch = 66, len(lengths)  # (launches take another form where no context can reach 64 tokens)
+    case = make_case(rng, config, lengths, room)
+    pool_host, slots, offsets, _, capacity, _ = case
+    eager, eager_pool = build_step(runtime, config, weights, case, lengths, room)
+    frozen, frozen_pool = build_step(runtime, config, weights, case, lengths, room)
+    plan = Prebaked(runtime, frozen.dispatches, frozen.tokens, frozen.token_ids)
+    assert plan.resident_layers == layers
+    stride, elements = config.token_stride, config.token_elements
+    tokens = rng.integers(0, config.vocabulary, batch)
+    for index in range(3):
+        past = np.asarray(lengths) + index
+        new_slots = slots[offsets + past]
+        eager.run(tokens)
+        frozen.tokens.write(np.asarray(tokens, dtype=np.int64))
+        before = frozen_pool.numpy(np.uint8).reshape(capacity, stride)
+        first = plan.execute(int(tokens[0]), int(past[0]))
+        got = frozen.work["x"][0].numpy(np.float16, (batch, hidden))
+        assert first == int(frozen.token_ids.numpy(np.uint32)[0])
+        want, _, want_pool = decode_chain(config, weights, before.reshape(-1).copy(), slots, offsets, past, new_slots, past, tokens)
+        # Held to the oracle as the chain's launches are (4e-3), or, where a row's activations amplify every rounding in front of
+        # them, to twice what the launches, rounded at the same places, are off there.
+        other = eager.work["x"][0].numpy(np.float16, (batch, hidden)).astype(np.float64)
+        want, got = np.asarray(want, dtype=np.float64), got.astype(np.float64)
+        norm, rms = np.linalg.norm(want), np.sqrt(np.mean(want ** 2))
+        assert np.isfinite(got).all() and np.linalg.norm(got - want) <= 4e-3 * norm
+        assert np.abs(got - want).max() <= max(2e-2 * rms, 2 * np.abs(other - want).max())
+        after = frozen_pool.numpy(np.uint8).reshape(capacity, stride)
+        untouched = np.ones(capacity, dtype=bool)
+        untouched[new_slots] = False
+        np.testing.assert_array_equal(after[untouched], before[untouched])
+        # The first layer's keys and values come from the same rows: one quantum where a value lies between two.  Behind it a row
+        # may be off by 2e-2 of its RMS, and so its keys and values; a group of 64 has a value of 2 RMS
+        # or more, which its scale makes 127 quanta: 127 * 2e-2 / 2 = 1.3 for the value, as much for the scale, and the one.
+        quanta = lambda rows: rows[new_slots, :elements].view(np.int8).astype(np.int32)
+        off = np.abs(quanta(after) - quanta(want_pool.reshape(capacity, stride)))
+        assert off[:, :2 * kv_heads * 64].max() <= 1 and off.max() <= 3
+        frozen_pool.copy_to(eager_pool)  # one quantum's difference must not grow into another continuation
+        tokens = rng.integers(0, config.vocabulary, batch)
+        eager.advance()
+        frozen.advance()
+    assert plan.resident_layers == layers  # no launch gave up
+
+
+def small_plan(runtime, lengths, layers=5):
+    from llmopt_amd.decode_step import DecodeConfig, random_weights
+    from llmopt_amd.native import Prebaked
+    rng = np.random.default_rng(11)
+    config = DecodeConfig(hidden=192, q_heads=3, kv_heads=1, head_dim=64, mlp=256, layers=layers, vocabulary=300)
+    weights = random_weights(config, rng)
+    case = make_case(rng, config, lengths, 70)
+    eager, eager_pool = build_step(runtime, config, weights, case, lengths, 70)
+    frozen, frozen_pool = build_step(runtime, config, weights, case, lengths, 70)
+    return eager, eager_pool, frozen, frozen_pool, Prebaked(runtime, frozen.dispatches, frozen.tokens, frozen.token_ids)
+
+
+def step_pair(eager, frozen, plan, tokens):
+    want = eager.run(tokens)
+    frozen.tokens.write(np.asarray(tokens, dtype=np.int64))
+    first = plan.execute(int(tokens[0]), int(frozen.host_lengths[0]))
+    got = frozen.token_ids.numpy(np.uint32, (len(tokens),))
+    assert first == int(got[0])
+    eager.advance()
+    frozen.advance()
+    return want, got
+
+
+@pytest.mark.parametrize("lengths", [[70], [70, 65, 3]])
+def test_step_that_gives_up_is_run_by_launches(runtime, lengths, monkeypatch):
+    """No wave waits for anything: the resident launch gives up, the step runs again launch by launch, bit for bit the
+    eager one, and so do all behind it."""
+    monkeypatch.setenv("LLMOPT_RESIDENT_WAIT_US", "0")
+    eager, eager_pool, frozen, frozen_pool, plan = small_plan(runtime, lengths)
+    assert plan.resident_layers == 5
+    for _ in range(3):
+        want, got = step_pair(eager, frozen, plan, [7] * len(lengths))
+        assert plan.resident_layers == 0
+        np.testing.assert_array_equal(got, want)
+        np.testing.assert_array_equal(frozen.work["x"][0].numpy(np.uint16), eager.work["x"][0].numpy(np.uint16))
+        np.testing.assert_array_equal(frozen_pool.numpy(np.uint8), eager_pool.numpy(np.uint8))
+
+
+def test_only_scratch_between_the_records_is_left_out(runtime):
+    """A buffer between the records that somebody may read: the plan launches every record and writes it."""
+    from llmopt_amd.native import Prebaked
+    eager, _, frozen, _, plan = small_plan(runtime, [70])
+    assert plan.resident_layers == 5
+    own = runtime.create_buffer(frozen.work["q_rot"].numpy(np.uint16).nbytes)
+    dispatches = [(name, [own if b is frozen.work["q_rot"] else b for b in buffers], *rest)
+                  for name, buffers, *rest in frozen.dispatches]
+    plan = Prebaked(runtime, dispatches, frozen.tokens, frozen.token_ids)
+    assert plan.resident_layers == 0
+    step_pair(eager, frozen, plan, [7])
+    np.testing.assert_array_equal(own.numpy(np.uint16), eager.work["q_rot"].numpy(np.uint16))
+    # a record behind the layers that reads what one of them leaves
+    x, stream = frozen.work["x"][0], frozen.work["stream"]
+    last = (frozen.dispatches[-1][0], [stream, *frozen.dispatches[-1][1][1:]], *frozen.dispatches[-1][2:])
+    assert Prebaked(runtime, [*frozen.dispatches[:-1], last], frozen.tokens, frozen.token_ids).resident_layers == 0
+
+
+def test_plans_on_two_threads(runtime):
+    """One resident launch at a time on a device: a step that finds the place taken runs by launches."""
+    import threading
+    from llmopt_amd.native import Runtime
+    other = Runtime()
+    try:
+        sets = [small_plan(runtime, [70]), small_plan(other, [90])]
+        failures = []
+
+        def steps(eager, frozen, plan):
+            try:
+                for index in range(40):
+                    want, got = step_pair(eager, frozen, plan, [index % 300])
+                    x, y = (s.work["x"][0].numpy(np.float16).astype(np.float64) for s in (eager, frozen))
+                    assert np.linalg.norm(x - y) <= 2e-2 * np.linalg.norm(x)  # (own caches: a quantum's difference stays in them)
+            except Exception as error:
+                failures.append(error)
+        threads = [threading.Thread(target=steps, args=(s[0], s[2], s[4])) for s in sets]
+        for thread in threads:
+            thread.start()
+        for thread in threads:
+            thread.join()
+        assert not failures, failures
+        assert all(s[4].resident_layers == 5 for s in sets)  # none gave up
+        del sets
+    finally:
+        other.close()
