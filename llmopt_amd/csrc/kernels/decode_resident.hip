@@ -7,20 +7,24 @@
 // stay, and what one hands to the others are words of memory that carry their own tag:
 //
 //   A  norm + QKV + rotation     16 output columns x up to 16 sequences a workgroup
-//   B  attention over the cache  a run of tokens of one sequence, all KV heads; the new token's K and V into its slot
-//   C  merge of the runs         four waves a (sequence, head)
+//   B  attention over the cache  one KV head of a run of a sequence's tokens; the new token's K and V into its slot
+//   C  merge of the runs         one wave or all eight a (sequence, head)
 //   D  output projection + residual, E  norm + gate / up + SwiGLU, F  down projection + residual: as A
 //
 // A handed-over word is 64 bits, two halves or one float32 and the tag of its layer and step, written and read with
 // relaxed device-scope atomics: the reader polls the words that it needs, and a word that carries the tag is there, so a
-// hand-over is one store on its way and one load (1.0 to 1.4 us at 16 to 128 workgroups; a counter that all workgroups
-// add to takes 1.4 at 64 and 4.0 at 256).  No word is written again before all its readers have read it: to write
+// hand-over is one store on its way and one load (alone, 16 to 128 workgroups and 256 to 768 words to each: 1.0 to 1.7 us;
+// a counter that all workgroups add to takes 0.9 at 16, 1.4 at 64, 2.2 at 128 and 4.0 at 256).  No word is written again before all its readers have read it: to write
 // layer l + 1's word a workgroup has seen words that depend, through the phases between, on every reader of layer l's.
 //
-// Eight waves of a workgroup poll and compute, eight fetch: the weights of the workgroup's tiles into LDS as soon as the
-// last layer's have been used, the first cache rows of its run into registers and then LDS.  Loads return in the order of
-// their requests, so a wave that had also fetched would see its polled words only behind its weights (28 us a layer
-// instead of 12).
+// Eight waves of a workgroup poll and multiply, eight walk the cache.  A CU's loads return in the order of their requests:
+// a polled line that takes 320 cycles takes 810 to 870 beside a stream of other loads from the same CU.  So the polling
+// waves request the next use's weights into registers right behind a phase's stores, where they land while the words
+// travel (requested once the rows are staged: 388 us instead of 357 for 30 layers of one sequence); the walking waves
+// request cache tiles a step ahead, registers to LDS, and help stage the rows of several sequences.
+//
+// 30 layers, hidden 576, this launch alone: one sequence behind 512 / 2048 / 8192 tokens 348 / 357 / 399 us, 32 sequences
+// of 1024 to 2048 tokens 746 us.  Whole steps through a plan, launches / resident: 694 / 394 and 1154 / 803 us.
 //
 // Waits are bounded: a wave that has polled for `wait_ticks` gives up, sets *failed and polls no more, as does every wave
 // that sees the word set; all go on to their end with whatever they hold (numbers only: no address depends on them).  The
@@ -991,8 +995,10 @@ bool resident_ok(uint32_t m, uint32_t h, uint32_t q_heads, uint32_t kv_heads, ui
          kv_heads <= 8 && q_heads >= 1 && q_heads <= 16 && q_heads % kv_heads == 0 && mlp % 64 == 0 && mlp >= 64 && mlp <= 2048;
 }
 
-// Workgroups: one a CU at most, so that all are resident together.  One sequence takes as many as its widest phase has tiles (96
-// for 1536 columns of gate and up: 357 us for 30 layers, 64 or 128 workgroups 3 to 10 % more), several take all CUs for the cache.
+// Workgroups: one a CU at most, so that all are resident together.  One sequence takes as many as its widest phase has tiles, the
+// fewest with which no workgroup has two (96 for 1536 columns of gate and up; with 96 / 128 / 192 / 256, 30 layers take 348 / 347 /
+// 348 / 353 us behind 512 tokens, 361 / 355 / 354 / 354 behind 2048, 399 / 406 / 394 / 408 behind 8192: no count is steadily faster,
+// and the rest of the chip stays free).  Several sequences take all CUs for the cache.
 uint32_t resident_workgroups(uint32_t m, uint32_t h, uint32_t q_heads, uint32_t kv_heads, uint32_t mlp, uint32_t compute_units) {
   const uint32_t tiles_m = (m + kTile - 1) / kTile;
   const uint32_t widest = std::max(std::max((q_heads + 2 * kv_heads) * 4, mlp / kTile), h / kTile) * tiles_m;
@@ -1068,8 +1074,8 @@ hipError_t launch_instance(const ResidentArgs &args, uint32_t workgroups, uint32
 hipError_t launch_decode_resident(const ResidentArgs &args, uint32_t workgroups, uint32_t lds, hipStream_t stream) {
   if (!resident_fits(args, workgroups, lds)) return hipErrorInvalidValue;
   if (args.m == 1) return launch_instance<true, true>(args, workgroups, lds, stream);  // (a workgroup a query head and more)
-  // Sixteen runs a sequence and more: four trips of one wave.  us a step, one wave / eight, contexts of 1024 to 2048: 2 sequences
-  // 552 / 477, 4 573 / 525, 8 (ten runs) 518 / 536, 16 599 / 648.
+  // Sixteen runs a sequence and more: four trips of one wave.  us a step, one wave / eight: 2 sequences 442 / 475 behind 512 tokens,
+  // 552 / 481 behind 2048, 641 / 515 behind 8192; 4 sequences 483 / 508, 573 / 527, 618 / 590; 8 (ten runs) 486 / 516, 518 / 536, 706 / 734.
   const bool together = resident_slots(workgroups, args.kv_heads) >= 16 * args.m && args.m * args.q_heads <= workgroups;
   return together ? launch_instance<false, true>(args, workgroups, lds, stream) : launch_instance<false, false>(args, workgroups, lds, stream);
 }
