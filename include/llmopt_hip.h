@@ -133,6 +133,8 @@ void llmopt_hip_release_buffer(llmopt_hip_buffer *buffer);
 /* caml_llmopt_metal_buffer_contents (:750-762): copies the whole buffer out
  * after draining the stream; capacity must be >= the buffer length. */
 int llmopt_hip_buffer_contents(llmopt_hip_buffer *buffer, void *out, size_t capacity);
+/* The buffer's float16 values as float32; count (of floats) must be >= theirs.  No reference counterpart. */
+int llmopt_hip_buffer_contents_widened(llmopt_hip_buffer *buffer, float *out, size_t count);
 /* caml_llmopt_metal_buffer_length (:798-805); negative on error. */
 int64_t llmopt_hip_buffer_length(llmopt_hip_buffer *buffer);
 /* Device address of the first byte (for interop). */

@@ -447,7 +447,7 @@ __global__ void plan_state_kernel(int64_t *token, int64_t value, const int32_t *
 __global__ void plan_result_kernel(const int32_t *output, const uint32_t *failed, int32_t *host) {
   if (threadIdx.x != 0) return;
   host[0] = output != nullptr ? *output : 0;
-  host[1] = (int32_t)*failed;
+  if (failed != nullptr) host[1] = (int32_t)*failed;
 }
 
 // *found = 1 when the range holds a NaN (not an infinity): fp16 words, or float32 words.

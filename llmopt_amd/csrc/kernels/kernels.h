@@ -396,7 +396,7 @@ hipError_t launch_copy_bytes(void *destination, const void *source, size_t bytes
 hipError_t launch_plan_state(int64_t *token, int64_t value, const int32_t *chain_from, uint32_t *past,
                              uint32_t past_value, uint32_t past_count, uint32_t *checkpoint, uint32_t checkpoint_value,
                              uint32_t *resident, uint32_t resident_tag, hipStream_t stream);
-// host (pinned memory): the step's output word and whether its resident launch gave up.
+// host (pinned memory): the step's output word (0: output is null) and, where `failed` is not null, whether its resident launch gave up.
 hipError_t launch_plan_result(const int32_t *output, const uint32_t *failed, int32_t *host, hipStream_t stream);
 
 // Sets *found (device memory) to 1 when [data, data + bytes) holds a NaN, read as fp16 words or

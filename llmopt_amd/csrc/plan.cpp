@@ -92,6 +92,7 @@ struct llmopt_hip_prebaked : llmopt::RefCounted {
   hipGraphExec_t executable = nullptr;
   uint64_t workspace_generation = 0;
   uint32_t *debug_flag = nullptr;  // device word of the NaN-check replay
+  int32_t *host_result = nullptr;  // pinned: the output word of a step that is waited for
   std::unique_ptr<ResidentPlan> resident;  // null: every step launches all records
 };
 
@@ -199,6 +200,7 @@ void prepare_resident(llmopt_hip_prebaked *plan) {
   llmopt_hip_context *context = plan->library->context;
   std::unique_ptr<ResidentPlan> r(new ResidentPlan());
   if (context->device < 0 || context->device >= 64 || !find_resident_run(plan->records, &r->run)) return;
+  if (plan->output_buffer && !plan->output_buffer->of_context()) return;
   ResidentArgs &a = r->run.args;
   r->workgroups = resident_workgroups(a.m, a.h, a.q_heads, a.kv_heads, a.mlp, (uint32_t)context->compute_units);
   a.words = resident_words(a.m, a.h, a.q_heads, a.kv_heads, a.mlp, r->workgroups);
@@ -225,9 +227,8 @@ void prepare_resident(llmopt_hip_prebaked *plan) {
   plan->resident = std::move(r);
 }
 
-// Queues one step on the context's stream: state, records, and the copy of the first int32 of
-// the output buffer to `host_token` (pinned memory, or pageable when the caller waits right
-// after).  chain: the input token is the output token the previous step left in the output
+// Queues one step on the context's stream: state, records, and the first int32 of the output buffer into `host_token`
+// (pinned memory).  chain: the input token is the output token the previous step left in the output
 // buffer (the reference's llmopt_chain_token_id launch).
 int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t past_tokens, int32_t *host_token, bool resident = false) {
   const uint32_t checkpoint = plan->checkpoint;
@@ -284,9 +285,15 @@ int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t p
   }
   if (host_token != nullptr) {
     *host_token = 0;
-    if (plan->output_buffer && plan->output_buffer->length >= 4)
-      LLMOPT_HIP_TRY(hipMemcpyAsync(host_token, plan->output_buffer->device, 4, hipMemcpyDeviceToHost, context->stream),
-                     "HIP could not read the decode output");
+    if (plan->output_buffer && plan->output_buffer->length >= 4) {
+      // by a kernel: a step of 19 records took 168 us with a copy to pageable memory, 159 so
+      if (plan->output_buffer->of_context())
+        LLMOPT_HIP_TRY(launch_plan_result(reinterpret_cast<const int32_t *>(plan->output_buffer->device), nullptr, host_token, context->stream),
+                       "HIP could not read the decode output");
+      else
+        LLMOPT_HIP_TRY(hipMemcpyAsync(host_token, plan->output_buffer->device, 4, hipMemcpyDeviceToHost, context->stream),
+                       "HIP could not read the decode output");
+    }
   }
   return LLMOPT_OK;
 }
@@ -550,6 +557,7 @@ void llmopt_hip_release_prebaked(llmopt_hip_prebaked *plan) {
   plan->resident.reset();
   if (plan->device_past) (void)hipFree(plan->device_past);
   if (plan->debug_flag) (void)hipFree(plan->debug_flag);
+  if (plan->host_result) (void)hipHostFree(plan->host_result);
   for (DispatchRecord &record : plan->records) drop_record(&record);
   if (plan->token_buffer) llmopt_hip_release_buffer(plan->token_buffer);
   if (plan->output_buffer) llmopt_hip_release_buffer(plan->output_buffer);
@@ -590,10 +598,15 @@ int llmopt_hip_prebaked_execute(llmopt_hip_prebaked *plan, int64_t token, int64_
       plan->resident->gave_up = true;  // the step again, launch by launch: what it wrote so far is written anew
     }
   }
-  if (int status = enqueue_step(plan, token, false, past_tokens, &next_token)) return status;
+  if (plan->host_result == nullptr) {
+    if (int status = use_device(plan->library->context)) return status;
+    LLMOPT_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&plan->host_result), 4, hipHostMallocDefault),
+                   "HIP could not allocate pinned memory for the step's result");
+  }
+  if (int status = enqueue_step(plan, token, false, past_tokens, plan->host_result)) return status;
   if (hipStreamSynchronize(plan->library->context->stream) != hipSuccess)
     return fail(LLMOPT_ERR_FAILURE, "Prebaked HIP batch failed");
-  if (out_token) *out_token = (int64_t)next_token;
+  if (out_token) *out_token = (int64_t)*plan->host_result;
   return LLMOPT_OK;
 }
 

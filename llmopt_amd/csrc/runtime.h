@@ -71,6 +71,12 @@ struct llmopt_hip_buffer : llmopt::RefCounted {
   size_t length = 0;
   bool owns_memory = false;
   bool scratch = false;  // see llmopt_hip_buffer_set_scratch
+  // Memory of the context's own, which its kernels can reach.  A wrapped pointer may be one that only copies can.
+  bool of_context() const {
+    const llmopt_hip_buffer *root = this;
+    while (root->parent) root = root->parent;
+    return root->owns_memory;
+  }
 };
 
 struct llmopt_hip_library : llmopt::RefCounted {

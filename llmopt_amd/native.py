@@ -83,6 +83,7 @@ def lib() -> ctypes.CDLL:
         "llmopt_hip_buffer_wrap": (ctypes.c_int, [vp, vp, sz, pp]),
         "llmopt_hip_release_buffer": (None, [vp]),
         "llmopt_hip_buffer_contents": (ctypes.c_int, [vp, vp, sz]),
+        "llmopt_hip_buffer_contents_widened": (ctypes.c_int, [vp, vp, sz]),
         "llmopt_hip_buffer_length": (i64, [vp]),
         "llmopt_hip_buffer_device_pointer": (vp, [vp]),
         "llmopt_hip_buffer_copy": (ctypes.c_int, [vp, vp]),
@@ -145,7 +146,7 @@ EXPORTED_SYMBOLS = (
     "llmopt_hip_preload_pipeline", "llmopt_hip_function_count", "llmopt_hip_function_name",
     "llmopt_hip_buffer_of_bytes", "llmopt_hip_create_buffer", "llmopt_hip_map_file",
     "llmopt_hip_buffer_view", "llmopt_hip_buffer_wrap", "llmopt_hip_release_buffer", "llmopt_hip_buffer_set_scratch",
-    "llmopt_hip_buffer_contents", "llmopt_hip_buffer_length", "llmopt_hip_buffer_device_pointer",
+    "llmopt_hip_buffer_contents", "llmopt_hip_buffer_contents_widened", "llmopt_hip_buffer_length", "llmopt_hip_buffer_device_pointer",
     "llmopt_hip_buffer_copy", "llmopt_hip_buffer_write", "llmopt_hip_buffer_set_int64",
     "llmopt_hip_buffer_set_u32_array", "llmopt_hip_buffer_argmax_f16", "llmopt_hip_f16_argmax",
     "llmopt_hip_sample_f16", "llmopt_hip_f32_argmax", "llmopt_hip_sample_f32", "llmopt_hip_dispatch", "llmopt_hip_launch",
@@ -220,6 +221,15 @@ class Buffer:
         array = np.empty(length // dtype.itemsize, dtype=dtype)
         _check(lib().llmopt_hip_buffer_contents(self.handle, array.ctypes.data, length))
         return array if shape is None else array.reshape(shape)
+
+    def widened(self) -> np.ndarray:
+        """The buffer's float16 values as float32."""
+        length = self.byte_length
+        if length % 2:
+            raise ValueError("buffer size must be a multiple of element size")
+        array = np.empty(length // 2, dtype=np.float32)
+        _check(lib().llmopt_hip_buffer_contents_widened(self.handle, array.ctypes.data, array.size))
+        return array
 
     def write(self, data, offset: int = 0) -> None:
         if isinstance(data, (bytes, bytearray)):

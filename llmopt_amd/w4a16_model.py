@@ -113,7 +113,7 @@ class W4a16Model:
         return self._prompts[slot, tokens]
 
     def logits_row(self) -> np.ndarray:
-        return self._last.numpy(np.float16, (self.vocabulary,)).astype(np.float32)
+        return self._last.widened()
 
     def step(self, sequence: Sequence, tokens: Tokens[int], want: Tokens[int] = ()) -> np.ndarray:
         tokens, want = [int(t) for t in tokens], [int(w) for w in want]
@@ -134,7 +134,7 @@ class W4a16Model:
             batch.commit()
             sequence.position += len(tokens)
             for index, out in enumerate(logits):
-                rows[index] = out.numpy(np.float16, (self.vocabulary,))
+                rows[index] = out.widened()
             return rows
         for place, token in enumerate(tokens):
             self.decode(sequence, token)
