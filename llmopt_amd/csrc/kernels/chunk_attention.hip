@@ -21,8 +21,9 @@
 //    float32 accuracy in the product).  Caps of at most kFixedMaxCap bound the exponent, so
 //    the running maximum (and the rescaling) is dropped for a constant one.
 //  * chunk_decode_kernel: one token.  A workgroup takes kSplitKeys keys of one key / value head for all
-//    query heads on it, which are the operand columns; chunk_merge_kernel joins the splits when the ring is
-//    longer than one.  Over a raw float32 row it norms and rotates the group's queries and the token's own
+//    query heads on it, which are the operand columns; where the ring is longer than one split the last workgroup of a
+//    head joins them, or chunk_merge_kernel (joins_shares:
+//    the line between them).  Over a raw float32 row it norms and rotates the group's queries and the token's own
 //    key first (in LDS) and leaves key and value in the ring; the own key and value never come from there.
 //  * rotate_heads_kernel: the same norm and rotation for a portion of a prompt, in place.
 #include <algorithm>
@@ -510,10 +511,10 @@ __global__ __launch_bounds__(256) void rotate_rows_kernel(ChunkAttentionArgs a) 
   }
 }
 
-template <typename T, int ND, int NE, bool RAW>
-__global__ __launch_bounds__(256) void chunk_decode_kernel(ChunkAttentionArgs a, uint32_t splits) {
+template <typename T, int ND, int NE, bool RAW, bool JOIN>
+__global__ __launch_bounds__(256) void chunk_decode_kernel(ChunkAttentionArgs a, uint32_t splits, uint32_t *counters) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  chunk_decode<T, ND, NE, RAW>(a, splits, blockIdx.x, blockIdx.y, lds);
+  chunk_decode<T, ND, NE, RAW, JOIN>(a, splits, blockIdx.x, blockIdx.y, lds, counters);
 }
 
 template <typename T>
@@ -522,17 +523,17 @@ __global__ __launch_bounds__(256) void chunk_merge_kernel(ChunkAttentionArgs a, 
   chunk_merge<T>(a, splits, blockIdx.x, shared);
 }
 
-template <typename T, int ND, int NE, bool RAW>
+template <typename T, int ND, int NE, bool RAW, bool JOIN>
 hipError_t run_decode(const ChunkAttentionArgs &a, hipStream_t stream) {
   static bool allowed[kMaxDevices] = {};
   constexpr int bytes = decode_lds_floats<T, NE>() * 4 + (RAW ? raw_row_lds_bytes<T, ND, NE>() : 0);
   const uint32_t splits = decode_splits(a);
   if (bytes > 64 * 1024)
-    if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(chunk_decode_kernel<T, ND, NE, RAW>), bytes, allowed))
+    if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(chunk_decode_kernel<T, ND, NE, RAW, JOIN>), bytes, allowed))
       return status;
-  chunk_decode_kernel<T, ND, NE, RAW><<<dim3(a.kv_heads, splits), 256, bytes, stream>>>(a, splits);
+  chunk_decode_kernel<T, ND, NE, RAW, JOIN><<<dim3(a.kv_heads, splits), 256, bytes, stream>>>(a, splits, a.counters);
   if (hipError_t status = hipGetLastError()) return status;
-  if (splits > 1) chunk_merge_kernel<T><<<a.heads, 256, splits * 8, stream>>>(a, splits);
+  if (splits > 1 && !JOIN) chunk_merge_kernel<T><<<a.heads, 256, splits * 8, stream>>>(a, splits);
   return hipGetLastError();
 }
 
@@ -607,7 +608,8 @@ hipError_t run_attention(const ChunkAttentionArgs &a, hipStream_t stream) {
     if (a.m > 1 && turns_ok(a)) return run_turns<ND * 32>(a, stream);
   }
   if (a.m > 1) return run_prefill<T, ND, NE>(a, stream);
-  return a.row ? run_decode<T, ND, NE, true>(a, stream) : run_decode<T, ND, NE, false>(a, stream);
+  if (joins_shares(a)) return a.row ? run_decode<T, ND, NE, true, true>(a, stream) : run_decode<T, ND, NE, false, true>(a, stream);
+  return a.row ? run_decode<T, ND, NE, true, false>(a, stream) : run_decode<T, ND, NE, false, false>(a, stream);
 }
 
 template <typename T, int ND>

@@ -114,15 +114,122 @@ constexpr int raw_row_lds_bytes() {
          ND * 16 * (int)sizeof(Turn);
 }
 
-// The work of one workgroup of 256 threads; lds: decode_lds_floats (and raw_row_lds_bytes behind them).
-template <typename T, int ND, int NE, bool RAW>
+__device__ __forceinline__ void hand_over(float *to, float v) {
+  __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float handed_over(const float *from) {
+  return __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Whether the caller's stores and those of `others` more arrivals are all there.  The caller has waited for its own.
+__device__ __forceinline__ bool last_to_arrive(uint32_t *counter, uint32_t others) {
+  const bool last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == others;
+  if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return last;
+}
+
+template <typename T>
+__device__ __forceinline__ void store_attention(const ChunkAttentionArgs &a, uint32_t head, uint32_t c, float v) {
+  if (a.out_row) a.out_row[head * a.vdim + c] = v * a.out_scale;
+  else static_cast<T *>(a.out)[head * a.vdim + c] = (T)(v * a.out_scale);
+}
+
+// Up to SHARES shares in one trip and without a barrier: every thread forms its head's weights for itself.
+template <typename T, uint32_t SHARES>
+__device__ __forceinline__ void join_in_registers(const ChunkAttentionArgs &a, uint32_t splits, uint32_t group, uint32_t live, const float *partials) {
+  const uint32_t per = a.heads / a.kv_heads, stride = a.vdim + 2;
+  for (uint32_t i = threadIdx.x; i < per * a.vdim; i += 256) {
+    const uint32_t h = i / a.vdim, c = i % a.vdim;
+    const float *shares = partials + (size_t)h * splits * stride;
+    float v[SHARES], best[SHARES], total[SHARES];
+#pragma unroll
+    for (uint32_t s = 0; s < SHARES; ++s) {
+      const float *share = shares + min(s, live - 1) * stride;
+      v[s] = handed_over(share + c);
+      best[s] = handed_over(share + a.vdim);
+      total[s] = handed_over(share + a.vdim + 1);
+    }
+    const float sink = a.sink ? (float)reinterpret_cast<const __bf16 *>(a.sink)[group * per + h] * kLog2e : -INFINITY;
+    float top = sink;
+#pragma unroll
+    for (uint32_t s = 0; s < SHARES; ++s) top = fmaxf(top, best[s]);  // (the last one again behind the last)
+    float denominator = exp2_raw(sink - top), sum = 0.0f;
+#pragma unroll
+    for (uint32_t s = 0; s < SHARES; ++s)
+      if (s < live) {
+        const float weight = exp2_raw(best[s] - top);
+        denominator = fmaf(total[s], weight, denominator);
+        sum = fmaf(v[s], weight, sum);
+      }
+    store_attention<T>(a, group * per + h, c, sum / denominator);
+  }
+}
+
+// The last workgroup of a key / value head to arrive merges the head's shares itself: the sums and their order are
+// chunk_merge's.  lds: two words a share and head, and one a head.
+template <typename T>
+__device__ __forceinline__ void join_shares(const ChunkAttentionArgs &a, uint32_t splits, uint32_t group, uint32_t live, uint32_t *counter,
+                                            char *lds) {
+  const uint32_t per = a.heads / a.kv_heads, stride = a.vdim + 2, tid = threadIdx.x;
+  uint32_t *flag = reinterpret_cast<uint32_t *>(lds);
+  float *denominators = reinterpret_cast<float *>(lds) + 1, *weights = denominators + per, *totals = weights + per * live;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();  // the stores of every wave are there
+  if (tid == 0) *flag = last_to_arrive(counter, live - 1) ? 1u : 0u;
+  __syncthreads();
+  if (*flag == 0) return;
+  const float *partials = static_cast<const float *>(a.workspace) + (size_t)group * per * splits * stride;
+  if (live <= 8) return join_in_registers<T, 8>(a, splits, group, live, partials);
+  if (live <= 16) return join_in_registers<T, 16>(a, splits, group, live, partials);
+  for (uint32_t i = tid; i < per * live; i += 256) {
+    const float *own = partials + ((size_t)(i / live) * splits + i % live) * stride + a.vdim;
+    const float best = handed_over(own), total = handed_over(own + 1);
+    weights[i] = best;
+    totals[i] = total;
+  }
+  __syncthreads();
+  for (uint32_t h = tid; h < per; h += 256) {
+    const float sink = a.sink ? (float)reinterpret_cast<const __bf16 *>(a.sink)[group * per + h] * kLog2e : -INFINITY;
+    float top = sink;
+    for (uint32_t s = 0; s < live; ++s) top = fmaxf(top, weights[h * live + s]);
+    float denominator = exp2_raw(sink - top);
+    for (uint32_t s = 0; s < live; ++s) {
+      const float weight = exp2_raw(weights[h * live + s] - top);
+      weights[h * live + s] = weight;
+      denominator = fmaf(totals[h * live + s], weight, denominator);
+    }
+    denominators[h] = denominator;
+  }
+  __syncthreads();
+  constexpr uint32_t AHEAD = 8;
+  for (uint32_t i = tid; i < per * a.vdim; i += 256) {
+    const uint32_t h = i / a.vdim, c = i % a.vdim;
+    const float *values = partials + (size_t)h * splits * stride + c;
+    float sum = 0.0f;
+    for (uint32_t s0 = 0; s0 < live; s0 += AHEAD) {
+      float v[AHEAD];
+#pragma unroll
+      for (uint32_t s = 0; s < AHEAD; ++s) v[s] = handed_over(values + (size_t)min(s0 + s, live - 1) * stride);
+#pragma unroll
+      for (uint32_t s = 0; s < AHEAD; ++s)
+        if (s0 + s < live) sum = fmaf(v[s], weights[h * live + s0 + s], sum);
+    }
+    store_attention<T>(a, group * per + h, c, sum / denominators[h]);
+  }
+}
+
+// The work of one workgroup of 256 threads; lds: decode_lds_floats (and raw_row_lds_bytes behind them).  JOIN: the last
+// workgroup of a key / value head (counters: one each) joins its shares; else they are a launch of their own.
+template <typename T, int ND, int NE, bool RAW, bool JOIN>
 __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32_t splits, uint32_t group, uint32_t split,
-                                             char *lds) {
+                                             char *lds, uint32_t *counters) {
   constexpr int EP = NE * 16, SV = value_stride<T, NE>(), V_PIECES = EP / 8;
   const uint32_t position = a.state[kStatePosition], slot = a.state[kStateSlot];
   const uint32_t per = a.heads / a.kv_heads;
   const uint32_t begin = first_seen(position, a.cache) + split * kSplitKeys;
   if (begin > position) return;
+  const uint32_t live = min(splits, (position - first_seen(position, a.cache)) / kSplitKeys + 1);
+  const bool alone = splits == 1 || (JOIN && live == 1);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, column = lane & 15, quad = lane >> 4;
   // a wave's own rows: the values [32][SV], then its sums [16][EP] in their place
   constexpr int OWN = 32 * SV * (int)sizeof(T);
@@ -274,26 +381,30 @@ __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32
         top = fmaxf(top, lds_top[w * 16 + h]);
       }
       const uint32_t target = group * per + h0 + h;
-      if (splits == 1) {
+      if (alone) {
         if (a.sink) {
           const float sink = (float)reinterpret_cast<const __bf16 *>(a.sink)[target] * kLog2e, most = fmaxf(top, sink);
           const float mine = exp2_raw(top - most);
           sum *= mine;
-          all = all * mine + exp2_raw(sink - most);
+          all = fmaf(all, mine, exp2_raw(sink - most));
         }
-        if (a.out_row) a.out_row[target * a.vdim + c] = sum / all * a.out_scale;
-        else static_cast<T *>(a.out)[target * a.vdim + c] = (T)(sum / all * a.out_scale);
+        store_attention<T>(a, target, c, sum / all);
       } else {
         float *partial = static_cast<float *>(a.workspace) + ((size_t)target * splits + split) * (a.vdim + 2);
-        partial[c] = sum;
+        const auto leave = [](float *to, float v) {
+          if (JOIN) hand_over(to, v);
+          else *to = v;
+        };
+        leave(partial + c, sum);
         if (c == 0) {
-          partial[a.vdim] = top;
-          partial[a.vdim + 1] = all;
+          leave(partial + a.vdim, top);
+          leave(partial + a.vdim + 1, all);
         }
       }
     }
     __syncthreads();
   }
+  if (JOIN && !alone) join_shares<T>(a, splits, group, live, counters + group, lds);
 }
 
 // 256 threads a head; the splits' weights are formed once, in LDS (two words a split; maxima are exponents of two).
@@ -332,14 +443,27 @@ __device__ __forceinline__ void chunk_merge(const ChunkAttentionArgs &a, uint32_
     if (c < a.vdim) sum = fmaf(partial[s * stride + c], weight, sum);
   }
   if (c >= a.vdim) return;
-  if (a.out_row) a.out_row[head * a.vdim + c] = sum / denominator * a.out_scale;
-  else static_cast<T *>(a.out)[head * a.vdim + c] = (T)(sum / denominator * a.out_scale);
+  store_attention<T>(a, head, c, sum / denominator);
 }
 
 // Most shares of 128 keys that a token can have.
 inline uint32_t decode_splits(const ChunkAttentionArgs &a) {
   const uint32_t span = a.cache.span, capacity = a.cache.capacity, longest = span && span < capacity ? span : capacity;
   return (longest + kSplitKeys - 1) / kSplitKeys;
+}
+
+// Whether the last workgroup of each key / value head joins its shares.  That saves a launch, and with one live share the
+// arrival too, but one workgroup does for all the head's queries what the merge spreads over a workgroup each.  us a call,
+// merge / join, query heads over key heads x width, at the ring's end and (first) with one live share:
+//   16 over 4 x 64 (256 outputs a key head)    6.5 / 4.5;  2 shares 6.6 / 6.2, 16 9.7 / 6.7, 17 10.1 / 8.8, 64 22.8 / 15.2
+//   32 over 8 x 128 (512)                      8.1 / 5.8;  2 shares 8.2 / 8.0, 16 11.2 / 9.7, 17 11.6 / 12.9, 64 27.3 / 25.2
+//   64 over 4 x 64 (1024)                      7.2 / 5.3;  2 shares 7.4 / 8.5, 8 7.5 / 8.6, 16 10.6 / 12.9
+constexpr uint32_t kJoinOutputs = 512, kJoinShares = 16, kJoinOutputsOfMore = 256, kJoinMostShares = 64;
+inline bool joins_shares(const ChunkAttentionArgs &a) {
+  const uint32_t splits = decode_splits(a), per = a.heads / a.kv_heads;
+  return a.counters != nullptr && a.kv_heads <= a.counter_count && splits > 1 && splits <= kJoinMostShares &&
+         (uint64_t)per * a.vdim <= (splits <= kJoinShares ? kJoinOutputs : kJoinOutputsOfMore) &&
+         (uint64_t)per * (2 * splits + 1) + 1 <= (uint64_t)decode_lds_floats<__bf16, 2>();  // (the least a workgroup has)
 }
 
 }  // namespace llmopt

@@ -180,6 +180,8 @@ struct ChunkAttentionArgs {
   float scale, softcap;  // softcap 0: none
   void *workspace;
   size_t workspace_bytes;
+  uint32_t *counters;  // one token: the context's arrival counters, zero between launches; may be null
+  uint32_t counter_count;
 };
 size_t chunk_attention_workspace_bytes(const ChunkAttentionArgs &args);
 bool chunk_attention_ok(const ChunkAttentionArgs &args);

@@ -1,13 +1,16 @@
-// One token through window attention and the gated delta rule side by side: two launches for both mixers.
+// One token through window attention and the gated delta rule side by side: one launch for both mixers, two where the
+// keys' shares are merged apart (joins_shares).
 //
 // Alone, each mixer of a token is a few workgroups that wait for memory (7.2 us attention, 2.2 its merge, 13.8 a workgroup
 // per head of the delta rule, at 16 heads of 64 and 8 of 128 x 128): together they take as long as the longer one.
 //  * mixer_step_kernel: the first workgroups take 32 value columns of a delta-rule head each, the others a share of a
 //    key / value head's keys (chunk_decode.h).  A head's state passes through registers, a row of 32 columns by eight
 //    lanes; every workgroup of a head forms the head's decays and unit vectors for itself.  The output's norm needs all
-//    columns: the workgroups leave their sums of squares.
-//  * mixer_finish_kernel: merges the shares of the keys, and divides every delta-rule head's row by its root mean square.
-// Measured at those sizes, four layers: a prompt of 64 tokens and 24 decoded ones 6226 -> 5080 us (48 us a token, 12 a layer).
+//    columns: the workgroups leave their values and sums of squares, and the last of a head to arrive divides the row by
+//    its root mean square.
+// Measured at those sizes, four layers: a prompt of 64 tokens and 24 decoded ones 6226 us with a launch for every part,
+// 5080 with both mixers in one launch and a finishing one (3.9 us of 34 a layer), 4530 without that and with what is
+// around it as it is now.
 #include <algorithm>
 
 #include "chunk_decode.h"
@@ -34,10 +37,10 @@ __device__ __forceinline__ float bf16_at(const uint16_t *p, size_t i) { return (
 // R: passes of 64 rows over the state (dim <= 64 R).
 template <int R>
 __device__ __forceinline__ void delta_columns(const DeltaArgs &a, uint32_t head, uint32_t part, DeltaStepLds &lds,
-                                              float *squares) {
+                                              float *squares, uint32_t *counter) {
   constexpr int PASSES = 2 * R + 1;  // of 32 rows over those of the low-rank products: dim decays, 32 gates
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const uint32_t group = head / (a.heads / a.kv_heads);
+  const uint32_t group = head / (a.heads / a.kv_heads), parts = a.vdim / kColumns;
   const uint32_t column = part * kColumns + (tid & 7) * 4, first = tid >> 3;
   const bool fresh = a.step[kStatePosition] == 0;
   float *state = a.state + ((size_t)a.step[kStateSlot] * a.heads + head) * a.dim * a.vdim + column;
@@ -146,49 +149,57 @@ __device__ __forceinline__ void delta_columns(const DeltaArgs &a, uint32_t head,
       const float u = beta * (a.row[2 * (size_t)a.kv_heads * a.dim + (size_t)head * a.vdim + c] - read);
       lds.written[lane] = u;
       out = fmaf(lds.product, u, out);
-      a.out_row[(size_t)head * a.vdim + c] = out * bf16_at(a.norm, c) * lds.gate[lane] * a.out_scale;
+      hand_over(a.out_row + (size_t)head * a.vdim + c, out * bf16_at(a.norm, c) * lds.gate[lane] * a.out_scale);
     }
     const float square = wave_sum(out * out);
-    if (lane == 0) squares[head * (a.vdim / kColumns) + part] = square;
+    if (lane == 0) hand_over(squares + head * parts + part, square);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   __syncthreads();
+  // the last part of a head to arrive divides the head's row by its root mean square, all in this wave
+  bool last = false;
+  if (wave == 0) {
+    if (lane == 0) last = last_to_arrive(counter, parts - 1);
+    last = __shfl((int)last, 0, 64) != 0;
+  }
   const f32x4 u = *reinterpret_cast<const f32x4 *>(&lds.written[(tid & 7) * 4]);
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     const uint32_t r = first + kRowsAPass * i;
     if (r < a.dim) *reinterpret_cast<f32x4 *>(state + (size_t)r * a.vdim) = s[i] + lds.key[r] * u;
   }
+  if (last) {
+    float *out = a.out_row + (size_t)head * a.vdim, value[kDeltaMaxWidth / 64], total = 0.0f;
+#pragma unroll
+    for (int i = 0; i < (int)kDeltaMaxWidth / 64; ++i) value[i] = lane + 64 * i < a.vdim ? handed_over(out + lane + 64 * i) : 0.0f;
+    for (uint32_t p = 0; p < parts; ++p) total += handed_over(squares + head * parts + p);
+    const float inverse = 1.0f / sqrtf(total / (float)a.vdim + a.epsilon);
+#pragma unroll
+    for (int i = 0; i < (int)kDeltaMaxWidth / 64; ++i)
+      if (lane + 64 * i < a.vdim) out[lane + 64 * i] = value[i] * inverse;
+  }
 }
 
 template <int ND, int NE>
 constexpr int attention_lds_bytes() { return decode_lds_floats<__bf16, NE>() * 4 + raw_row_lds_bytes<__bf16, ND, NE>(); }
 
-template <int ND, int NE, int R>
-__global__ __launch_bounds__(kThreads) void mixer_step_kernel(ChunkAttentionArgs a, DeltaArgs d, uint32_t splits, float *squares) {
+template <int ND, int NE, int R, bool JOIN>
+__global__ __launch_bounds__(kThreads) void mixer_step_kernel(ChunkAttentionArgs a, DeltaArgs d, uint32_t splits, float *squares, uint32_t *counters) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const uint32_t parts = d.vdim / kColumns, delta_blocks = d.heads * parts;
   if (blockIdx.x < delta_blocks) {
-    delta_columns<R>(d, blockIdx.x / parts, blockIdx.x % parts, *reinterpret_cast<DeltaStepLds *>(lds), squares);
+    delta_columns<R>(d, blockIdx.x / parts, blockIdx.x % parts, *reinterpret_cast<DeltaStepLds *>(lds), squares,
+                     counters + blockIdx.x / parts);
     return;
   }
   if (threadIdx.x >= 256) return;  // (barriers count the waves that are still there)
   const uint32_t share = blockIdx.x - delta_blocks;
-  chunk_decode<__bf16, ND, NE, true>(a, splits, share % a.kv_heads, share / a.kv_heads, lds);
+  chunk_decode<__bf16, ND, NE, true, JOIN>(a, splits, share % a.kv_heads, share / a.kv_heads, lds, counters + d.heads);
 }
 
-__global__ __launch_bounds__(256) void mixer_finish_kernel(ChunkAttentionArgs a, DeltaArgs d, uint32_t splits, const float *squares) {
+__global__ __launch_bounds__(256) void mixer_merge_kernel(ChunkAttentionArgs a, uint32_t splits) {
   extern __shared__ __attribute__((aligned(16))) float shared[];
-  if (blockIdx.x >= d.heads) {
-    chunk_merge<__bf16>(a, splits, blockIdx.x - d.heads, shared);
-    return;
-  }
-  const uint32_t head = blockIdx.x, c = threadIdx.x, parts = d.vdim / kColumns;
-  if (c >= d.vdim) return;
-  float *out = d.out_row + (size_t)head * d.vdim + c;
-  const float value = *out;
-  float total = 0.0f;
-  for (uint32_t p = 0; p < parts; ++p) total += squares[head * parts + p];
-  *out = value * (1.0f / sqrtf(total / (float)d.vdim + d.epsilon));
+  chunk_merge<__bf16>(a, splits, blockIdx.x, shared);
 }
 
 template <int ND, int NE, int R>
@@ -196,9 +207,13 @@ hipError_t run(const ChunkAttentionArgs &a, const DeltaArgs &d, float *squares, 
   constexpr int bytes = std::max<int>(attention_lds_bytes<ND, NE>(), (int)sizeof(DeltaStepLds));
   static_assert(bytes <= 64 * 1024, "no raised limit");
   const uint32_t splits = decode_splits(a), blocks = d.heads * (d.vdim / kColumns) + a.kv_heads * splits;
-  mixer_step_kernel<ND, NE, R><<<blocks, kThreads, bytes, stream>>>(a, d, splits, squares);
+  ChunkAttentionArgs own = a;  // (the attention's counters lie behind the delta rule's)
+  own.counter_count -= d.heads;
+  const bool joins = joins_shares(own);
+  const auto kernel = joins ? mixer_step_kernel<ND, NE, R, true> : mixer_step_kernel<ND, NE, R, false>;
+  kernel<<<blocks, kThreads, bytes, stream>>>(a, d, splits, squares, a.counters);
   if (hipError_t status = hipGetLastError()) return status;
-  mixer_finish_kernel<<<d.heads + (splits > 1 ? a.heads : 0), 256, splits * 8, stream>>>(a, d, splits, squares);
+  if (splits > 1 && !joins) mixer_merge_kernel<<<a.heads, 256, splits * 8, stream>>>(a, splits);
   return hipGetLastError();
 }
 
@@ -215,7 +230,7 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 // The wide loads' conditions: whole sixteen-byte pieces of every low-rank row and of its inputs, whole parts of 32 value
 // columns; heads of attention up to 128 values (wider ones hold too many registers beside the other half).
 bool mixer_step_ok(const ChunkAttentionArgs &a, const DeltaArgs &d) {
-  return !a.f32 && a.m == 1 && d.m == 1 && a.row != nullptr && a.dim <= 128 && a.vdim > 32 && a.vdim <= 128 &&
+  return !a.f32 && a.m == 1 && d.m == 1 && a.row != nullptr && a.counters != nullptr && d.heads <= a.counter_count && a.dim <= 128 && a.vdim > 32 && a.vdim <= 128 &&
          chunk_attention_ok(a) && d.dim <= kDeltaMaxWidth && d.vdim <= kDeltaMaxWidth && d.vdim % kColumns == 0 &&
          d.decay_rank >= 8 && d.gate_rank >= 8 && d.decay_rank <= kMaxRank && d.gate_rank <= kMaxRank &&
          (d.decay_rank | d.gate_rank) % 8 == 0 && aligned16(d.decay_in) && aligned16(d.gate_in) && aligned16(d.w_decay) &&

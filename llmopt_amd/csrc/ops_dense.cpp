@@ -237,6 +237,8 @@ int chunk_attention(llmopt_hip_context *context, const DispatchRecord &record) {
   if (a.workspace_bytes) {
     a.workspace = context_workspace(context, a.workspace_bytes);
     if (a.workspace == nullptr) return LLMOPT_ERR_FAILURE;
+    a.counters = context_counters(context, &a.counter_count);
+    if (a.counters == nullptr) return LLMOPT_ERR_FAILURE;
   }
   if (int status = launched(launch_chunk_attention(a, context->stream), name)) return status;
   return a.m == 1 ? LLMOPT_OK : launched(launch_chunk_cache_write(a, context->stream), name);

@@ -269,6 +269,8 @@ int rotary_attention(llmopt_hip_context *context, const DispatchRecord &record) 
     if (a.workspace_bytes) {
       a.workspace = context_workspace(context, a.workspace_bytes);
       if (a.workspace == nullptr) return LLMOPT_ERR_FAILURE;
+      a.counters = context_counters(context, &a.counter_count);
+      if (a.counters == nullptr) return LLMOPT_ERR_FAILURE;
     }
     return launched(launch_chunk_attention(a, context->stream), name);
   }
@@ -407,6 +409,8 @@ int rotary_attention_gated_delta(llmopt_hip_context *context, const DispatchReco
   DeltaArgs d;
   if (int status = read_rotary_attention<F32>(left, &a)) return status;
   if (int status = read_gated_delta<F32>(right, &d)) return status;
+  a.counters = context_counters(context, &a.counter_count);
+  if (a.counters == nullptr) return LLMOPT_ERR_FAILURE;
   if (!mixer_step_ok(a, d)) {
     if (int status = rotary_attention<F32>(context, left)) return status;
     return gated_delta<F32>(context, right);
