@@ -2,8 +2,8 @@
 //
 //   S_t = exp(-a dt_t) S_(t-1) + dt_t b_t x_t^T,   y_t = S_t^T c_t + d x_t      (per head, S in float32)
 //
-// One token (ssm_step_kernel): a wave per row of the transposed state [vdim][state_size], lanes along the
-// state; the convolution, the softplus and their bookkeeping ran in the projection's epilogue.
+// One token (ssm_step_rows_kernel, other state sizes ssm_step_kernel): half a wave, or a wave, per row of the transposed
+// state [vdim][state_size], lanes along the state; the convolution, the softplus and their bookkeeping ran in the projection's epilogue.
 //
 // Many tokens: chunks of 64.  Within a chunk
 //   y_i = exp(L_i) S c_i + sum_{j <= i} (c_i . b_j) exp(L_i - L_j) dt_j x_j + d x_i
@@ -117,6 +117,48 @@ __global__ __launch_bounds__(256) void ssm_step_kernel(SsmArgs a) {
       const uint32_t row = first + r;
       a.gated[row] = (y[r] + bf16_at(a.d_skip, row / a.vdim) * x[row]) * silu_f32(a.row[row]);
     }
+}
+
+// Rows of whole pieces of four values and at most 128 PIECES: 32 lanes a row, a piece or two a lane, so that one trip brings all
+// a wave needs.  The kernel above, for all other sizes, waits for two or three trips one after the other (scalars, then the state; the skip and the gate
+// behind the sums).  Bound: that trip and the launch.  A token of 32 heads of 64 x 128: 7.9 to 9.3 us -> 3.1 to 3.4.
+template <int PIECES>
+__global__ __launch_bounds__(256) void ssm_step_rows_kernel(SsmArgs a) {
+  const int lane = threadIdx.x & 31;
+  const uint32_t inner = a.heads * a.vdim, n = a.state_size, mine = blockIdx.x * 8 + (threadIdx.x >> 5);
+  const uint32_t row = min(mine, inner - 1), head = row / a.vdim, group = head / (a.heads / a.groups);
+  const float *x = a.row + inner, *b = x + inner, *c = b + a.groups * n, *dt = c + a.groups * n;
+  const float value = x[row], step = dt[head], z = a.row[row], log_rate = bf16_at(a.a_log, head), skip = bf16_at(a.d_skip, head);
+  f32x4 into[PIECES], from[PIECES], s[PIECES];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const uint32_t k = min(p * 128u + lane * 4u, n - 4);
+    into[p] = *reinterpret_cast<const f32x4 *>(b + group * n + k);
+    from[p] = *reinterpret_cast<const f32x4 *>(c + group * n + k);
+  }
+  const bool fresh = a.step[kStatePosition] == 0;
+  float *state = a.ssm_state + ((size_t)a.step[kStateSlot] * inner + row) * n;
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) s[p] = *reinterpret_cast<const f32x4 *>(state + min(p * 128u + lane * 4u, n - 4));
+  const float decay = fresh ? 0.0f : expf(-expf(log_rate) * step), gain = step * value;
+  float y = 0.0f;
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const uint32_t k = p * 128u + lane * 4u;
+    if (k >= n) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[p][e] = fmaf(decay, fresh ? 0.0f : s[p][e], gain * into[p][e]);
+      y = fmaf(s[p][e], from[p][e], y);
+    }
+    if (mine < inner) *reinterpret_cast<f32x4 *>(state + k) = s[p];
+  }
+  y += dpp_f32<0xb1>(y);  // the 32 lanes of the row
+  y += dpp_f32<0x4e>(y);
+  y += dpp_f32<0x141>(y);
+  y += dpp_f32<0x140>(y);
+  y += __shfl_xor(y, 16, 64);
+  if (lane == 0 && mine < inner) a.gated[row] = (y + skip * value) * silu_f32(z);
 }
 
 // ---- many tokens ----------------------------------------------------------------------------------------
@@ -538,6 +580,12 @@ size_t ssm_workspace_bytes(const SsmArgs &a) {
 
 hipError_t launch_ssm_step(const SsmArgs &a, hipStream_t stream) {
   const uint32_t rows = a.heads * a.vdim, per = 4 * kStepRows;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(a.row) | reinterpret_cast<uintptr_t>(a.ssm_state)) & 15) == 0;
+  if (aligned && a.state_size % 4 == 0 && rows % 4 == 0 && a.state_size <= 256) {  // (b and c lie behind two times `rows` values)
+    const auto kernel = a.state_size <= 128 ? ssm_step_rows_kernel<1> : ssm_step_rows_kernel<2>;
+    kernel<<<(rows + 7) / 8, 256, 0, stream>>>(a);
+    return hipGetLastError();
+  }
   ssm_step_kernel<<<(rows + per - 1) / per, 256, 0, stream>>>(a);
   return hipGetLastError();
 }
