@@ -434,14 +434,32 @@ namespace {
 // native/ocaml_metal_stubs.m:1570-1577) and the context length every sequence attends to.
 __global__ void plan_state_kernel(int64_t *token, int64_t value, const int32_t *chain_from, uint32_t *past,
                                   uint32_t past_value, uint32_t past_count, uint32_t *checkpoint,
-                                  uint32_t checkpoint_value, uint32_t *resident, uint32_t resident_tag) {
-  if (threadIdx.x == 0 && resident != nullptr) {
-    resident[0] = resident_tag;
-    resident[1] = 0;
-  }
+                                  uint32_t checkpoint_value) {
   if (threadIdx.x == 0 && token != nullptr) *token = chain_from != nullptr ? (int64_t)*chain_from : value;
   if (threadIdx.x == 0 && checkpoint != nullptr) *checkpoint = checkpoint_value;
   for (uint32_t i = threadIdx.x; i < past_count; i += blockDim.x) past[i] = past_value;
+}
+
+// Loads that pass the caches by (the host writes these words anew for every replay), all in one trip.
+__global__ void plan_begin_kernel(const StepWords *step) {
+  constexpr int WORDS = offsetof(StepWords, result) / 8;
+  static_assert(offsetof(StepWords, result) == 8 * WORDS, "whole words");
+  union {
+    uint64_t words[WORDS];
+    StepWords step;
+  } s;
+#pragma unroll
+  for (int i = 0; i < WORDS; ++i)
+    s.words[i] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(step) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (threadIdx.x == 0) {
+    if (s.step.resident != nullptr) {
+      s.step.resident[0] = s.step.resident_tag;
+      s.step.resident[1] = 0;
+    }
+    if (s.step.token != nullptr) *s.step.token = s.step.value;
+    if (s.step.checkpoint != nullptr) *s.step.checkpoint = s.step.checkpoint_value;
+  }
+  for (uint32_t i = threadIdx.x; i < s.step.past_count; i += blockDim.x) s.step.past[i] = s.step.past_value;
 }
 
 __global__ void plan_result_kernel(const int32_t *output, const uint32_t *failed, int32_t *host) {
@@ -477,9 +495,14 @@ hipError_t launch_nan_scan(const void *data, size_t bytes, bool f32, uint32_t *f
 
 hipError_t launch_plan_state(int64_t *token, int64_t value, const int32_t *chain_from, uint32_t *past,
                              uint32_t past_value, uint32_t past_count, uint32_t *checkpoint, uint32_t checkpoint_value,
-                             uint32_t *resident, uint32_t resident_tag, hipStream_t stream) {
+                             hipStream_t stream) {
   hipLaunchKernelGGL(plan_state_kernel, dim3(1), dim3(256), 0, stream, token, value, chain_from, past, past_value,
-                     past_count, checkpoint, checkpoint_value, resident, resident_tag);
+                     past_count, checkpoint, checkpoint_value);
+  return hipGetLastError();
+}
+
+hipError_t launch_plan_begin(const StepWords *step, hipStream_t stream) {
+  hipLaunchKernelGGL(plan_begin_kernel, dim3(1), dim3(64), 0, stream, step);
   return hipGetLastError();
 }
 

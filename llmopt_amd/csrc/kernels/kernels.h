@@ -391,12 +391,20 @@ struct PointwiseArgs {
 hipError_t launch_add_f16(const PointwiseArgs &args, hipStream_t stream);
 
 hipError_t launch_copy_bytes(void *destination, const void *source, size_t bytes, hipStream_t stream);
-// One small launch that sets a retained plan's per-step state: resident (when not null) to {resident_tag, 0}, *token = *chain_from (when not
-// null; int32 widened) or `value` (token may be null), and past[0..past_count) = past_value.
+// One small launch that sets a retained plan's per-step state: *token = *chain_from (when not null; int32 widened) or `value`
+// (token may be null), and past[0..past_count) = past_value.
 hipError_t launch_plan_state(int64_t *token, int64_t value, const int32_t *chain_from, uint32_t *past,
                              uint32_t past_value, uint32_t past_count, uint32_t *checkpoint, uint32_t checkpoint_value,
-                             uint32_t *resident, uint32_t resident_tag, hipStream_t stream);
-// host (pinned memory): the step's output word (0: output is null) and, where `failed` is not null, whether its resident launch gave up.
+                             hipStream_t stream);
+// The same from pinned memory, at the head of a graph whose every step is waited for: resident (when not null) becomes
+// {resident_tag, 0}.  The step's result comes back behind the values.
+struct StepWords {
+  int64_t *token, value;  // (null: the step has none of these)
+  uint32_t *past, *checkpoint, *resident;
+  uint32_t past_value, past_count, checkpoint_value, resident_tag;
+  int32_t result[2];  // the output word, and whether a resident launch gave up
+};
+hipError_t launch_plan_begin(const StepWords *step, hipStream_t stream);
 hipError_t launch_plan_result(const int32_t *output, const uint32_t *failed, int32_t *host, hipStream_t stream);
 
 // Sets *found (device memory) to 1 when [data, data + bytes) holds a NaN, read as fp16 words or

@@ -7,8 +7,8 @@
 // Here the frozen array becomes ONE HIP graph, instantiated at create: the per-step values live
 // in device memory that the captured kernels read - the token in the caller's token buffer, the
 // context length in a word of the plan that the paged attention launches take instead of
-// parameter byte 12 - and a step is one small state launch, one graph launch and a 4-byte
-// read-back.  The attention launches are sized for the capacity of their slot table, so the same
+// parameter byte 12 - and a step that is waited for is one graph launch: its first kernel takes the
+// step's values from pinned memory, its last one leaves the output word there (StepWords).  The attention launches are sized for the capacity of their slot table, so the same
 // graph serves every step of a sequence.  Buffers the caller updates between steps with
 // llmopt_hip_buffer_write / set_int64 / set_u32_array (rotary rows, the new token's slot, the
 // per-sequence lengths of the batched extension) are read by the kernels from device memory
@@ -40,7 +40,6 @@ struct ResidentPlan {
   void *layers = nullptr;       // device
   uint64_t *hand = nullptr;     // device
   uint32_t *words = nullptr;    // device: the step's tag, and whether it gave up
-  int32_t *host = nullptr;      // pinned: the output word, and whether the step gave up
   uint32_t next_tag = 1;
   bool gave_up = false;
   hipGraph_t graph = nullptr;
@@ -51,7 +50,6 @@ struct ResidentPlan {
     if (layers) (void)hipFree(layers);
     if (hand) (void)hipFree(hand);
     if (words) (void)hipFree(words);
-    if (host) (void)hipHostFree(host);
   }
 };
 
@@ -92,7 +90,10 @@ struct llmopt_hip_prebaked : llmopt::RefCounted {
   hipGraphExec_t executable = nullptr;
   uint64_t workspace_generation = 0;
   uint32_t *debug_flag = nullptr;  // device word of the NaN-check replay
-  int32_t *host_result = nullptr;  // pinned: the output word of a step that is waited for
+  // Whether steps are waited for one by one (execute): their graph begins with the step's values and ends with its result, both in
+  // `step`, pinned.  A queue has steps in flight while it prepares others: there launches around the graph carry them.
+  bool waited = true;
+  StepWords *step = nullptr;
   std::unique_ptr<ResidentPlan> resident;  // null: every step launches all records
 };
 
@@ -111,9 +112,16 @@ void destroy_graph(llmopt_hip_prebaked *plan) {
   }
 }
 
+// The output word, where a kernel can read it.
+const int32_t *output_word(const llmopt_hip_prebaked *plan) {
+  const llmopt_hip_buffer *output = plan->output_buffer;
+  return output && output->of_context() && output->length >= 4 ? reinterpret_cast<const int32_t *>(output->device) : nullptr;
+}
+
 int launch_records(llmopt_hip_prebaked *plan, bool resident) {
   llmopt_hip_context *context = plan->library->context;
   const ResidentPlan *const r = plan->resident.get();
+  if (plan->waited) LLMOPT_HIP_TRY(launch_plan_begin(plan->step, context->stream), "HIP could not write the decode step's state");
   for (size_t i = 0; i < plan->records.size(); ++i) {
     if (resident && i == r->run.first) {
       LLMOPT_HIP_TRY(launch_decode_resident(r->run.args, r->workgroups, r->lds, context->stream), "HIP resident launch failed");
@@ -122,11 +130,9 @@ int launch_records(llmopt_hip_prebaked *plan, bool resident) {
     }
     if (int status = launch_record(context, plan->records[i])) return status;
   }
-  if (resident) {
-    const int32_t *output = plan->output_buffer && plan->output_buffer->length >= 4
-                                ? reinterpret_cast<const int32_t *>(plan->output_buffer->device) : nullptr;
-    LLMOPT_HIP_TRY(launch_plan_result(output, r->words + 1, r->host, context->stream), "HIP could not hand out the step's result");
-  }
+  if (resident || (plan->waited && output_word(plan)))
+    LLMOPT_HIP_TRY(launch_plan_result(output_word(plan), resident ? r->words + 1 : nullptr, plan->step->result, context->stream),
+                   "HIP could not hand out the step's result");
   return LLMOPT_OK;
 }
 
@@ -210,8 +216,7 @@ void prepare_resident(llmopt_hip_prebaked *plan) {
   const size_t layer_bytes = r->run.layers.size() * sizeof(ResidentLayer), hand_bytes = (size_t)a.words.total * 8;
   bool ok = hipMalloc(&r->layers, layer_bytes) == hipSuccess &&
             hipMalloc(reinterpret_cast<void **>(&r->hand), hand_bytes) == hipSuccess &&
-            hipMalloc(reinterpret_cast<void **>(&r->words), 8) == hipSuccess &&
-            hipHostMalloc(reinterpret_cast<void **>(&r->host), 8, hipHostMallocDefault) == hipSuccess;
+            hipMalloc(reinterpret_cast<void **>(&r->words), 8) == hipSuccess;
   if (ok) {
     a.layers = static_cast<const ResidentLayer *>(r->layers);
     a.hand = r->hand;
@@ -227,21 +232,70 @@ void prepare_resident(llmopt_hip_prebaked *plan) {
   plan->resident = std::move(r);
 }
 
-// Queues one step on the context's stream: state, records, and the first int32 of the output buffer into `host_token`
-// (pinned memory).  chain: the input token is the output token the previous step left in the output
-// buffer (the reference's llmopt_chain_token_id launch).
-int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t past_tokens, int32_t *host_token, bool resident = false) {
-  const uint32_t checkpoint = plan->checkpoint;
-  llmopt_hip_context *context = plan->library->context;
-  if (int status = use_device(context)) return status;
+// What a step asks of its plan: room for the context, and where its token goes (null: nowhere).
+int check_step(llmopt_hip_prebaked *plan, int64_t past_tokens, int64_t **token_slot) {
+  if (int status = use_device(plan->library->context)) return status;
   if (past_tokens < 0 || (uint64_t)past_tokens > plan->past_capacity)
     return fail(LLMOPT_ERR_INVALID, "prebaked HIP plan holds %u context tokens, step asks for %lld",
                 plan->past_capacity, (long long)past_tokens);
-  int64_t *token_slot = nullptr;
+  *token_slot = nullptr;
   if (plan->token_buffer) {
     if (plan->token_buffer->length < 8) return fail(LLMOPT_ERR_INVALID, "buffer offset out of bounds");
-    token_slot = reinterpret_cast<int64_t *>(plan->token_buffer->device);
+    *token_slot = reinterpret_cast<int64_t *>(plan->token_buffer->device);
   }
+  return LLMOPT_OK;
+}
+
+// One step of a plan of a single submission, waited for: one graph launch.  Beside a launch each for the step's values and its
+// result, with the host's time for them and the gaps around the graph, a token of the layered decoders took 150 and 160 us, 147 and 157 so.
+int wait_for_step(llmopt_hip_prebaked *plan, int64_t token, int64_t past_tokens, bool resident, int32_t *out) {
+  llmopt_hip_context *context = plan->library->context;
+  int64_t *token_slot = nullptr;
+  if (int status = check_step(plan, past_tokens, &token_slot)) return status;
+  if (plan->executable == nullptr || plan->workspace_generation != context->workspace_generation)
+    if (int status = capture_plan(plan)) return status;
+  StepWords &words = *plan->step;  // (no step of this plan is under way: each is waited for)
+  words = {};
+  words.token = token_slot;
+  words.value = token;
+  words.past = plan->past_words();
+  words.past_value = (uint32_t)past_tokens;
+  words.past_count = plan->past_word_count();
+  words.checkpoint = plan->checkpoint_word();
+  words.checkpoint_value = plan->checkpoint;
+  hipGraphExec_t executable = plan->executable;
+  if (resident) {
+    ResidentPlan &r = *plan->resident;
+    words.resident = r.words;
+    words.resident_tag = r.next_tag;
+    r.next_tag += r.run.args.layer_count + 1;
+    if (r.next_tag > 0xffffff00u) {  // a word that is not rewritten before the tags come round must not pass for a new one
+      LLMOPT_HIP_TRY(hipMemsetAsync(r.hand, 0, (size_t)r.run.args.words.total * 8, context->stream), "HIP could not clear the handed-over words");
+      r.next_tag = 1;
+    }
+    executable = r.executable;
+  }
+  std::atomic_thread_fence(std::memory_order_release);
+  int status = LLMOPT_OK;
+  if (hipGraphLaunch(executable, context->stream) != hipSuccess) status = fail(LLMOPT_ERR_FAILURE, "HIP graph launch failed");
+  const bool copies = plan->output_buffer && plan->output_buffer->length >= 4 && output_word(plan) == nullptr;
+  if (status == LLMOPT_OK && copies &&
+      hipMemcpyAsync(plan->step->result, plan->output_buffer->device, 4, hipMemcpyDeviceToHost, context->stream) != hipSuccess)
+    status = fail(LLMOPT_ERR_FAILURE, "HIP could not read the decode output");
+  if (hipStreamSynchronize(context->stream) != hipSuccess && status == LLMOPT_OK)
+    status = fail(LLMOPT_ERR_FAILURE, "Prebaked HIP batch failed");
+  if (status == LLMOPT_OK) memcpy(out, words.result, sizeof words.result);
+  return status;
+}
+
+// Queues one step on the context's stream: state, records, and the first int32 of the output buffer into `host_token`
+// (pinned memory).  chain: the input token is the output token the previous step left in the output
+// buffer (the reference's llmopt_chain_token_id launch).
+int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t past_tokens, int32_t *host_token) {
+  const uint32_t checkpoint = plan->checkpoint;
+  llmopt_hip_context *context = plan->library->context;
+  int64_t *token_slot = nullptr;
+  if (int status = check_step(plan, past_tokens, &token_slot)) return status;
   const int32_t *chain_from = nullptr;
   if (chain) {
     if (plan->output_buffer == nullptr || plan->output_buffer->length < 4 || token_slot == nullptr)
@@ -252,23 +306,11 @@ int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t p
     if (plan->executable == nullptr || plan->workspace_generation != context->workspace_generation)
       if (int status = capture_plan(plan)) return status;
     LLMOPT_HIP_TRY(launch_plan_state(token_slot, token, chain_from, plan->past_words(), (uint32_t)past_tokens,
-                                     plan->past_word_count(), plan->checkpoint_word(), checkpoint,
-                                     resident ? plan->resident->words : nullptr, resident ? plan->resident->next_tag : 0,
-                                     context->stream),
+                                     plan->past_word_count(), plan->checkpoint_word(), checkpoint, context->stream),
                    "HIP could not write the decode step's state");
-    if (resident) {
-      ResidentPlan &r = *plan->resident;
-      r.next_tag += r.run.args.layer_count + 1;
-      if (r.next_tag > 0xffffff00u) {  // a word that is not rewritten before the tags come round must not pass for a new one
-        LLMOPT_HIP_TRY(hipMemsetAsync(r.hand, 0, (size_t)r.run.args.words.total * 8, context->stream), "HIP could not clear the handed-over words");
-        r.next_tag = 1;
-      }
-      LLMOPT_HIP_TRY(hipGraphLaunch(r.executable, context->stream), "HIP graph launch failed");
-      return LLMOPT_OK;  // (the result is in r.host)
-    }
     LLMOPT_HIP_TRY(hipGraphLaunch(plan->executable, context->stream), "HIP graph launch failed");
   } else {
-    LLMOPT_HIP_TRY(launch_plan_state(token_slot, token, chain_from, nullptr, 0, 0, nullptr, 0, nullptr, 0, context->stream),
+    LLMOPT_HIP_TRY(launch_plan_state(token_slot, token, chain_from, nullptr, 0, 0, nullptr, 0, context->stream),
                    "HIP could not write the decode token");
     for (size_t i = 0; i < plan->records.size(); ++i) {
       DispatchRecord &record = plan->records[i];
@@ -287,9 +329,8 @@ int enqueue_step(llmopt_hip_prebaked *plan, int64_t token, bool chain, int64_t p
     *host_token = 0;
     if (plan->output_buffer && plan->output_buffer->length >= 4) {
       // by a kernel: a step of 19 records took 168 us with a copy to pageable memory, 159 so
-      if (plan->output_buffer->of_context())
-        LLMOPT_HIP_TRY(launch_plan_result(reinterpret_cast<const int32_t *>(plan->output_buffer->device), nullptr, host_token, context->stream),
-                       "HIP could not read the decode output");
+      if (output_word(plan))
+        LLMOPT_HIP_TRY(launch_plan_result(output_word(plan), nullptr, host_token, context->stream), "HIP could not read the decode output");
       else
         LLMOPT_HIP_TRY(hipMemcpyAsync(host_token, plan->output_buffer->device, 4, hipMemcpyDeviceToHost, context->stream),
                        "HIP could not read the decode output");
@@ -345,7 +386,7 @@ int debug_step(llmopt_hip_prebaked *plan, int64_t token, int64_t past_tokens, bo
   // frozen records read the context length from the plan's device words, the others from byte 12
   LLMOPT_HIP_TRY(launch_plan_state(token_slot, token, nullptr, plan->single_submission ? plan->past_words() : nullptr,
                                    (uint32_t)past_tokens, plan->single_submission ? plan->past_word_count() : 0,
-                                   plan->single_submission ? plan->checkpoint_word() : nullptr, plan->checkpoint, nullptr, 0,
+                                   plan->single_submission ? plan->checkpoint_word() : nullptr, plan->checkpoint,
                                    context->stream),
                  "HIP could not write the decode step's state");
   hipEvent_t before = nullptr, after = nullptr;
@@ -459,13 +500,8 @@ bool is_reference_paged_attention(const char *name) {
   return strncmp(name, prefix, sizeof prefix - 1) == 0 && strcmp(name, "llmopt_attention_q8_paged_batched") != 0;
 }
 
-}  // namespace
-
-extern "C" {
-
-int llmopt_hip_prebaked_create(llmopt_hip_library *library, const llmopt_hip_dispatch_item *items, size_t count,
-                               llmopt_hip_buffer *token_buffer, llmopt_hip_buffer *output_buffer,
-                               llmopt_hip_prebaked **out) {
+int create_plan(llmopt_hip_library *library, const llmopt_hip_dispatch_item *items, size_t count, llmopt_hip_buffer *token_buffer,
+                llmopt_hip_buffer *output_buffer, bool waited, llmopt_hip_prebaked **out) {
   if (out == nullptr) return fail(LLMOPT_ERR_INVALID, "plan output pointer is null");
   *out = nullptr;
   if (library == nullptr) return fail(LLMOPT_ERR_FAILURE, "HIP library has been finalized");
@@ -480,6 +516,7 @@ int llmopt_hip_prebaked_create(llmopt_hip_library *library, const llmopt_hip_dis
   if (int status = use_device(context)) return status;
   llmopt_hip_prebaked *plan = new llmopt_hip_prebaked();
   plan->library = library;
+  plan->waited = waited;
   retain(library);
   if (token_buffer) {
     plan->token_buffer = token_buffer;
@@ -491,6 +528,8 @@ int llmopt_hip_prebaked_create(llmopt_hip_library *library, const llmopt_hip_dis
   }
   plan->records.resize(count);
   int status = LLMOPT_OK;
+  if (waited && hipHostMalloc(reinterpret_cast<void **>(&plan->step), sizeof(StepWords), hipHostMallocDefault) != hipSuccess)
+    status = fail(LLMOPT_ERR_FAILURE, "HIP could not allocate pinned memory for the plan's steps");
   for (size_t i = 0; i < count && status == LLMOPT_OK; ++i) {
     status = build_record(library, &items[i], &plan->records[i]);
     if (status != LLMOPT_OK) break;
@@ -533,7 +572,7 @@ int llmopt_hip_prebaked_create(llmopt_hip_library *library, const llmopt_hip_dis
         }
       }
       try {
-        prepare_resident(plan);
+        if (waited) prepare_resident(plan);
       } catch (const std::exception &) {
         plan->resident.reset();
       }
@@ -548,6 +587,16 @@ int llmopt_hip_prebaked_create(llmopt_hip_library *library, const llmopt_hip_dis
   return LLMOPT_OK;
 }
 
+}  // namespace
+
+extern "C" {
+
+int llmopt_hip_prebaked_create(llmopt_hip_library *library, const llmopt_hip_dispatch_item *items, size_t count,
+                               llmopt_hip_buffer *token_buffer, llmopt_hip_buffer *output_buffer,
+                               llmopt_hip_prebaked **out) {
+  return create_plan(library, items, count, token_buffer, output_buffer, true, out);
+}
+
 void llmopt_hip_release_prebaked(llmopt_hip_prebaked *plan) {
   if (!release(plan)) return;
   llmopt_hip_context *context = plan->library->context;
@@ -557,7 +606,7 @@ void llmopt_hip_release_prebaked(llmopt_hip_prebaked *plan) {
   plan->resident.reset();
   if (plan->device_past) (void)hipFree(plan->device_past);
   if (plan->debug_flag) (void)hipFree(plan->debug_flag);
-  if (plan->host_result) (void)hipHostFree(plan->host_result);
+  if (plan->step) (void)hipHostFree(plan->step);
   for (DispatchRecord &record : plan->records) drop_record(&record);
   if (plan->token_buffer) llmopt_hip_release_buffer(plan->token_buffer);
   if (plan->output_buffer) llmopt_hip_release_buffer(plan->output_buffer);
@@ -586,27 +635,27 @@ int llmopt_hip_prebaked_execute(llmopt_hip_prebaked *plan, int64_t token, int64_
   if (plan->resident && !plan->resident->gave_up) {
     std::atomic<bool> &busy = resident_busy[plan->library->context->device];
     if (!busy.exchange(true, std::memory_order_acquire)) {
-      int status = enqueue_step(plan, token, false, past_tokens, nullptr, true);
-      if (hipStreamSynchronize(plan->library->context->stream) != hipSuccess && status == LLMOPT_OK)
-        status = fail(LLMOPT_ERR_FAILURE, "Prebaked HIP batch failed");
+      int32_t result[2] = {0, 0};
+      const int status = wait_for_step(plan, token, past_tokens, true, result);
       busy.store(false, std::memory_order_release);
       if (status != LLMOPT_OK) return status;
-      if (plan->resident->host[1] == 0) {
-        if (out_token) *out_token = (int64_t)plan->resident->host[0];
+      if (result[1] == 0) {
+        if (out_token) *out_token = (int64_t)result[0];
         return LLMOPT_OK;
       }
       plan->resident->gave_up = true;  // the step again, launch by launch: what it wrote so far is written anew
     }
   }
-  if (plan->host_result == nullptr) {
-    if (int status = use_device(plan->library->context)) return status;
-    LLMOPT_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&plan->host_result), 4, hipHostMallocDefault),
-                   "HIP could not allocate pinned memory for the step's result");
+  int32_t result[2] = {0, 0};
+  if (plan->single_submission) {
+    if (int status = wait_for_step(plan, token, past_tokens, false, result)) return status;
+  } else {
+    if (int status = enqueue_step(plan, token, false, past_tokens, plan->step->result)) return status;
+    if (hipStreamSynchronize(plan->library->context->stream) != hipSuccess)
+      return fail(LLMOPT_ERR_FAILURE, "Prebaked HIP batch failed");
+    result[0] = plan->step->result[0];
   }
-  if (int status = enqueue_step(plan, token, false, past_tokens, plan->host_result)) return status;
-  if (hipStreamSynchronize(plan->library->context->stream) != hipSuccess)
-    return fail(LLMOPT_ERR_FAILURE, "Prebaked HIP batch failed");
-  if (out_token) *out_token = (int64_t)*plan->host_result;
+  if (out_token) *out_token = (int64_t)result[0];
   return LLMOPT_OK;
 }
 
@@ -852,7 +901,7 @@ int llmopt_hip_ring_start_worker(llmopt_hip_ring *ring, llmopt_hip_library *libr
                                  llmopt_hip_buffer *output_buffer) {
   if (ring == nullptr) return fail(LLMOPT_ERR_FAILURE, "ring queue has been finalized");
   if (ring->worker_started) return fail(LLMOPT_ERR_INVALID, "ring queue worker is already running");
-  if (int status = llmopt_hip_prebaked_create(library, items, count, token_buffer, output_buffer, &ring->plan))
+  if (int status = create_plan(library, items, count, token_buffer, output_buffer, false, &ring->plan))
     return status;
   void *pinned = nullptr;
   if (hipHostMalloc(&pinned, 2 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess ||

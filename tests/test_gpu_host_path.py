@@ -42,3 +42,19 @@ def test_plan_hands_out_its_word(runtime, wrapped):
         logits[best] = 1
         rows.write(logits)
         assert plan.execute(5, 0) == best
+
+
+# each replay takes its own values, with and without a word to hand out, and beside steps of a second plan
+@pytest.mark.parametrize("output", ["own", "wrapped", "short"])
+def test_plan_takes_each_steps_token(runtime, output):
+    from llmopt_amd.native import Prebaked
+    from tests.gpu_util import u32s
+    rows, best = runtime.buffer_of_bytes(np.arange(300, dtype=np.float32)), runtime.create_buffer(4)
+    word = {"own": best, "wrapped": runtime.wrap(best.device_pointer, 4), "short": runtime.create_buffer(2)}[output]
+    tokens = [runtime.create_buffer(8) for _ in range(2)]
+    plans = [Prebaked(runtime, [("llmopt_argmax_f32", [rows, best], u32s(1, 300), (256, 1, 1), (256, 1, 1))], token, word)
+             for token in tokens]
+    for step in range(6):
+        for number, plan in enumerate(plans):
+            assert plan.execute(100 * number + step, 0) == (0 if output == "short" else 299)
+            assert tokens[number].numpy(np.int64)[0] == 100 * number + step
