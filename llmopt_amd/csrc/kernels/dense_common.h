@@ -170,16 +170,24 @@ template <int CONTROL>
 __device__ __forceinline__ float dpp_f32(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CONTROL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float wave_sum(float v) {
-  // within rows of sixteen lanes: neighbours, pairs, halves, the row
+// Over rows of sixteen lanes: neighbours, pairs, halves, the row.
+__device__ __forceinline__ float row_sum(float v) {
   v += dpp_f32<0xb1>(v);   // quad_perm [1, 0, 3, 2]
   v += dpp_f32<0x4e>(v);   // quad_perm [2, 3, 0, 1]
   v += dpp_f32<0x141>(v);  // row_half_mirror
   v += dpp_f32<0x140>(v);  // row_mirror
-  v += __shfl_xor(v, 16, 64);
-  v += __shfl_xor(v, 32, 64);
   return v;
 }
+// v and that of the lane 16 or 32 away: a swap of registers, where a shuffle goes through LDS.
+__device__ __forceinline__ float add_16_away(float v) {
+  const auto two = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  return __builtin_bit_cast(float, (uint32_t)two[0]) + __builtin_bit_cast(float, (uint32_t)two[1]);
+}
+__device__ __forceinline__ float add_32_away(float v) {
+  const auto two = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, v), __builtin_bit_cast(uint32_t, v), false, false);
+  return __builtin_bit_cast(float, (uint32_t)two[0]) + __builtin_bit_cast(float, (uint32_t)two[1]);
+}
+__device__ __forceinline__ float wave_sum(float v) { return add_32_away(add_16_away(row_sum(v))); }
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int mask = 32; mask >= 1; mask >>= 1) v = fmaxf(v, __shfl_xor(v, mask, 64));

@@ -34,51 +34,56 @@ struct DeltaStepLds {
 
 __device__ __forceinline__ float bf16_at(const uint16_t *p, size_t i) { return (float)reinterpret_cast<const __bf16 *>(p)[i]; }
 
-// R: passes of 64 rows over the state (dim <= 64 R).
+// R: passes of 64 rows over the state (dim <= 64 R).  A wave issues an instruction every four or five cycles and these waves have
+// nothing else to do: what counts is how many there are and how many trips lie behind one another.  With the decays' exponentials one
+// thread a row (five rows one after the other in one lane of sixteen), sums between lanes without LDS and the parts' squares asked
+// for together: 9.1 to 9.8 us -> 7.8 to 8.4 the launch, a token of four layers 161.6 -> 153.6.
 template <int R>
 __device__ __forceinline__ void delta_columns(const DeltaArgs &a, uint32_t head, uint32_t part, DeltaStepLds &lds,
                                               float *squares, uint32_t *counter) {
-  constexpr int PASSES = 2 * R + 1;  // of 32 rows over those of the low-rank products: dim decays, 32 gates
+  constexpr int PASSES = 2 * R;  // of 32 rows over those of the decays' low-rank product; the gate's are kColumns rows, one pass
+  static_assert(kThreads / 16 == kColumns, "a pass takes the rows of the gate");
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const uint32_t group = head / (a.heads / a.kv_heads), parts = a.vdim / kColumns;
   const uint32_t column = part * kColumns + (tid & 7) * 4, first = tid >> 3;
   const bool fresh = a.step[kStatePosition] == 0;
   float *state = a.state + ((size_t)a.step[kStateSlot] * a.heads + head) * a.dim * a.vdim + column;
 
+  // Asked for in the order in which it is needed, all before the first use.
+  const float *queries = a.row + (size_t)group * a.dim, *keys = queries + (size_t)a.kv_heads * a.dim;
+  float q[R], k[R];  // 64 components each: wave 0 takes the query's length, wave 1 the key's, wave 2 their product
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const uint32_t c = lane + 64 * i;
+    q[i] = wave < 3 && wave != 1 && c < a.dim ? queries[c] : 0.0f;
+    k[i] = wave < 3 && wave != 0 && c < a.dim ? keys[c] : 0.0f;
+  }
+  // sixteen lanes a row of the low-rank products, eight values each
+  const uint32_t piece = (tid & 15) * 8, row = tid >> 4;
+  const uint32_t decay_piece = min(piece, a.decay_rank - 8), gate_piece = min(piece, a.gate_rank - 8);
+  bf16x8 weights[PASSES + 1];
+#pragma unroll
+  for (int i = 0; i < PASSES; ++i)
+    weights[i] = *reinterpret_cast<const bf16x8 *>(a.w_decay + ((size_t)head * a.dim + min(row + 32 * i, a.dim - 1)) * a.decay_rank + decay_piece);
+  weights[PASSES] = *reinterpret_cast<const bf16x8 *>(a.w_gate + ((size_t)head * a.vdim + part * kColumns + row) * a.gate_rank + gate_piece);
+  f32x4 inputs[2][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    inputs[0][h] = *reinterpret_cast<const f32x4 *>(a.decay_in + decay_piece + 4 * h);
+    inputs[1][h] = *reinterpret_cast<const f32x4 *>(a.gate_in + gate_piece + 4 * h);
+  }
+  const float dt_bias = bf16_at(a.dt_bias, (size_t)head * a.dim + min((uint32_t)tid, a.dim - 1));
+  const float log_rate = bf16_at(a.a_log, head), raw_beta = a.row_beta[head];
+  const uint32_t own = part * kColumns + (lane & (kColumns - 1));  // the column of wave 0's lane
+  const float own_norm = bf16_at(a.norm, own), own_value = a.row[2 * (size_t)a.kv_heads * a.dim + (size_t)head * a.vdim + own];
   f32x4 s[R];
 #pragma unroll
   for (int i = 0; i < R; ++i) s[i] = *reinterpret_cast<const f32x4 *>(state + (size_t)min(first + kRowsAPass * i, a.dim - 1) * a.vdim);
 
-  // sixteen lanes a row of the low-rank products, eight values each
-  const uint32_t piece = (tid & 15) * 8, row = tid >> 4;
-  bf16x8 weights[PASSES];
-#pragma unroll
-  for (int i = 0; i < PASSES; ++i) {
-    const uint32_t r = min(row + 32 * i, a.dim + kColumns - 1);
-    const bool decays = r < a.dim;
-    const uint32_t rank = decays ? a.decay_rank : a.gate_rank;
-    const uint16_t *w = decays ? a.w_decay + ((size_t)head * a.dim + r) * rank
-                               : a.w_gate + ((size_t)head * a.vdim + part * kColumns + (r - a.dim)) * rank;
-    weights[i] = *reinterpret_cast<const bf16x8 *>(w + min(piece, rank - 8));
-  }
-  f32x4 inputs[2][2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    inputs[0][h] = *reinterpret_cast<const f32x4 *>(a.decay_in + min(piece, a.decay_rank - 8) + 4 * h);
-    inputs[1][h] = *reinterpret_cast<const f32x4 *>(a.gate_in + min(piece, a.gate_rank - 8) + 4 * h);
-  }
-  const float rate = expf(bf16_at(a.a_log, head)), beta = sigmoid_f32(a.row_beta[head]);
-
-  // unit lengths: wave 0 the query, wave 1 the key, wave 2 their product
   if (wave < 3) {
-    constexpr int PARTS = R;  // 64 components each
-    const float *queries = a.row + (size_t)group * a.dim, *keys = queries + (size_t)a.kv_heads * a.dim;
-    float q[PARTS], k[PARTS], qq = 0.0f, kk = 0.0f, qk = 0.0f;
+    float qq = 0.0f, kk = 0.0f, qk = 0.0f;
 #pragma unroll
-    for (int i = 0; i < PARTS; ++i) {
-      const uint32_t c = lane + 64 * i;
-      q[i] = wave != 1 && c < a.dim ? queries[c] : 0.0f;
-      k[i] = wave != 0 && c < a.dim ? keys[c] : 0.0f;
+    for (int i = 0; i < R; ++i) {
       qq += q[i] * q[i];
       kk += k[i] * k[i];
       qk += q[i] * k[i];
@@ -90,27 +95,25 @@ __device__ __forceinline__ void delta_columns(const DeltaArgs &a, uint32_t head,
       if (lane == 0) lds.product = qk * q_scale * k_scale;
     } else {
 #pragma unroll
-      for (int i = 0; i < PARTS; ++i) {
+      for (int i = 0; i < R; ++i) {
         const uint32_t c = lane + 64 * i;
         if (c < a.dim) (wave == 0 ? lds.query : lds.key)[c] = wave == 0 ? q[i] * q_scale : k[i] * k_scale;
       }
     }
   }
+  // the low-rank sums, then one thread a row for what becomes of them
 #pragma unroll
-  for (int i = 0; i < PASSES; ++i) {
-    const uint32_t r = row + 32 * i;
-    const bool decays = r < a.dim;
-    const bool live = piece < (decays ? a.decay_rank : a.gate_rank);
+  for (int i = 0; i < PASSES + 1; ++i) {
+    const bool gates = i == PASSES;
     float sum = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) sum = fmaf((float)weights[i][e], decays ? inputs[0][e / 4][e % 4] : inputs[1][e / 4][e % 4], sum);
-    sum = live ? sum : 0.0f;
-#pragma unroll
-    for (int mask = 8; mask >= 1; mask >>= 1) sum += __shfl_xor(sum, mask, 64);
-    if ((tid & 15) != 0 || r >= a.dim + kColumns) continue;
-    if (decays) lds.decay[r] = expf(-rate * softplus_f32(sum + bf16_at(a.dt_bias, (size_t)head * a.dim + r)));
-    else lds.gate[r - a.dim] = sigmoid_f32(sum);
+    for (int e = 0; e < 8; ++e) sum = fmaf((float)weights[i][e], inputs[gates][e / 4][e % 4], sum);
+    sum = row_sum(piece < (gates ? a.gate_rank : a.decay_rank) ? sum : 0.0f);
+    const uint32_t r = row + 32 * i;
+    if ((tid & 15) == 0 && (gates || r < a.dim)) (gates ? lds.gate[row] : lds.decay[r]) = sum;
   }
+  __syncthreads();
+  if ((uint32_t)tid < a.dim) lds.decay[tid] = expf(-expf(log_rate) * softplus_f32(lds.decay[tid] + dt_bias));
   __syncthreads();
 
   f32x4 from_key = 0.0f, from_query = 0.0f;
@@ -125,12 +128,12 @@ __device__ __forceinline__ void delta_columns(const DeltaArgs &a, uint32_t head,
   }
   // the eight rows of a wave, then the waves
 #pragma unroll
-  for (int mask = 8; mask <= 32; mask <<= 1)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      from_key[e] += __shfl_xor(from_key[e], mask, 64);
-      from_query[e] += __shfl_xor(from_query[e], mask, 64);
-    }
+  for (int e = 0; e < 4; ++e) {
+    from_key[e] += dpp_f32<0x128>(from_key[e]);  // row_ror 8
+    from_query[e] += dpp_f32<0x128>(from_query[e]);
+    from_key[e] = add_32_away(add_16_away(from_key[e]));
+    from_query[e] = add_32_away(add_16_away(from_query[e]));
+  }
   if (lane < 8) {
     *reinterpret_cast<f32x4 *>(&lds.read[wave][lane * 4]) = from_key;
     *reinterpret_cast<f32x4 *>(&lds.out[wave][lane * 4]) = from_query;
@@ -145,39 +148,44 @@ __device__ __forceinline__ void delta_columns(const DeltaArgs &a, uint32_t head,
         read += lds.read[w][lane];
         out += lds.out[w][lane];
       }
-      const uint32_t c = part * kColumns + lane;
-      const float u = beta * (a.row[2 * (size_t)a.kv_heads * a.dim + (size_t)head * a.vdim + c] - read);
+      const float u = sigmoid_f32(raw_beta) * (own_value - read);
       lds.written[lane] = u;
       out = fmaf(lds.product, u, out);
-      hand_over(a.out_row + (size_t)head * a.vdim + c, out * bf16_at(a.norm, c) * lds.gate[lane] * a.out_scale);
+      hand_over(a.out_row + (size_t)head * a.vdim + own, out * own_norm * sigmoid_f32(lds.gate[lane]) * a.out_scale);
     }
     const float square = wave_sum(out * out);
     if (lane == 0) hand_over(squares + head * parts + part, square);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   __syncthreads();
-  // the last part of a head to arrive divides the head's row by its root mean square, all in this wave
-  bool last = false;
-  if (wave == 0) {
-    if (lane == 0) last = last_to_arrive(counter, parts - 1);
-    last = __shfl((int)last, 0, 64) != 0;
-  }
   const f32x4 u = *reinterpret_cast<const f32x4 *>(&lds.written[(tid & 7) * 4]);
+  auto store_state = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const uint32_t r = first + kRowsAPass * i;
-    if (r < a.dim) *reinterpret_cast<f32x4 *>(state + (size_t)r * a.vdim) = s[i] + lds.key[r] * u;
-  }
-  if (last) {
-    float *out = a.out_row + (size_t)head * a.vdim, value[kDeltaMaxWidth / 64], total = 0.0f;
+    for (int i = 0; i < R; ++i) {
+      const uint32_t r = first + kRowsAPass * i;
+      if (r < a.dim) *reinterpret_cast<f32x4 *>(state + (size_t)r * a.vdim) = s[i] + lds.key[r] * u;
+    }
+  };
+  if (wave != 0) return store_state();
+  // the last part of a head to arrive divides the head's row by its root mean square, all in this wave (which stores its share of
+  // the state behind that: loads behind stores wait for them)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  bool last = false;
+  if (lane == 0) last = last_to_arrive(counter, parts - 1);
+  if (__shfl((int)last, 0, 64) != 0) {
+    constexpr int MOST = kDeltaMaxWidth / kColumns;
+    float *out = a.out_row + (size_t)head * a.vdim, value[kDeltaMaxWidth / 64], square[MOST], total = 0.0f;
 #pragma unroll
     for (int i = 0; i < (int)kDeltaMaxWidth / 64; ++i) value[i] = lane + 64 * i < a.vdim ? handed_over(out + lane + 64 * i) : 0.0f;
-    for (uint32_t p = 0; p < parts; ++p) total += handed_over(squares + head * parts + p);
+#pragma unroll
+    for (int p = 0; p < MOST; ++p) square[p] = handed_over(squares + head * parts + min((uint32_t)p, parts - 1));
+#pragma unroll
+    for (int p = 0; p < MOST; ++p) total += p < parts ? square[p] : 0.0f;
     const float inverse = 1.0f / sqrtf(total / (float)a.vdim + a.epsilon);
 #pragma unroll
     for (int i = 0; i < (int)kDeltaMaxWidth / 64; ++i)
       if (lane + 64 * i < a.vdim) out[lane + 64 * i] = value[i] * inverse;
   }
+  store_state();
 }
 
 template <int ND, int NE>
