@@ -326,6 +326,49 @@ __device__ __forceinline__ void ssm_in_store(const DenseGemvArgs &a, uint32_t n,
   a.out_f32[n] = v;
 }
 
+// What the epilogues of the convolution read, requested beside the weights: behind the product it is two trips, the state words'
+// and one for every tap of the ring.  (The same of the sum's epilogue gave nothing.)  One token's projections of 1024 values: into the
+// recurrence, 4384 columns, 5.9 to 6.8 us -> 5.0 to 5.3, into mixers side by side, 4872 columns, 5.8 to 6.2 -> 4.3 to 5.5; a
+// token of two layers of the first and two of attention and experts 146.3 -> 143.3, of four of the second 153.6 -> 150.0.
+enum class Ahead { kNothing, kConv };
+constexpr uint32_t kAheadTaps = 4;
+
+template <Ahead AHEAD>
+struct EpilogueAhead {
+  float bias, taps[kAheadTaps], ring[kAheadTaps];
+  uint32_t position, slot;
+  __device__ __forceinline__ void request(const DenseGemvArgs &a, uint32_t n) {
+    if (AHEAD != Ahead::kConv) return;
+    const uint32_t behind = a.inner + a.channels, c = n < a.inner ? 0 : min(n - a.inner, a.channels - 1);  // (any channel will do for others)
+    position = a.state[kStatePosition], slot = a.state[kStateSlot];
+    const uint16_t *extra = a.epilogue == GemvEpilogue::kSsmIn && n >= behind ? a.dt_bias + (n - behind) : a.conv_bias ? a.conv_bias + c : a.conv;
+    bias = bf16_at(extra, 0);
+    const float *own = a.conv_state + (size_t)slot * a.taps * a.channels + c;
+#pragma unroll
+    for (uint32_t back = 0; back < kAheadTaps; ++back) {
+      const uint32_t tap = min(back, a.taps - 1);
+      taps[back] = bf16_at(a.conv, (size_t)c * a.taps + a.taps - 1 - tap);
+      if (back > 0) ring[back] = own[(size_t)((position - min(tap, position)) % a.taps) * a.channels];
+    }
+  }
+  // conv_step, softplus or nothing, by the row's place (kSsmIn, kConvIn).
+  __device__ __forceinline__ float finish(const DenseGemvArgs &a, uint32_t n, float v) const {
+    if (n < a.inner) return v;
+    if (n >= a.inner + a.channels) return a.epilogue == GemvEpilogue::kSsmIn ? softplus_f32(v + bias) : v;
+    float sum = (a.conv_bias ? bias : 0.0f) + taps[0] * v;
+#pragma unroll
+    for (uint32_t back = 1; back < kAheadTaps; ++back)
+      if (back < a.taps && back <= position) sum = fmaf(taps[back], ring[back], sum);
+    a.conv_state[((size_t)slot * a.taps + position % a.taps) * a.channels + (n - a.inner)] = v;
+    return silu_f32(sum);
+  }
+};
+
+inline Ahead ahead_of(const DenseGemvArgs &a) {
+  const bool conv = a.epilogue == GemvEpilogue::kSsmIn || a.epilogue == GemvEpilogue::kConvIn;
+  return conv && a.channels > 0 && a.taps >= 1 && a.taps <= kAheadTaps ? Ahead::kConv : Ahead::kNothing;
+}
+
 template <typename T>
 __device__ __forceinline__ void gemv_epilogue(const DenseGemvArgs &a, uint32_t n, float v, float up) {
   switch (a.epilogue) {
@@ -344,7 +387,7 @@ __device__ __forceinline__ void gemv_epilogue(const DenseGemvArgs &a, uint32_t n
   }
 }
 
-template <typename T, int ROWS, bool GATED, bool VEC, Staging STAGING>
+template <typename T, int ROWS, bool GATED, bool VEC, Staging STAGING, Ahead AHEAD>
 __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseGemvArgs a) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ float scratch[kWaves];
@@ -359,7 +402,12 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseGemvArgs a) {
     const uint32_t n = min(first + (GATED ? r / 2 : r), a.n - 1);
     stream.rows[r] = reinterpret_cast<const __bf16 *>(matrix) + (size_t)n * a.k;
   }
-  stage_activation<T, STAGING>(a, xs, plane, scratch, [&] { stream.request(a.k, lane); });
+  const uint32_t own = first + lane;
+  EpilogueAhead<AHEAD> ahead;
+  stage_activation<T, STAGING>(a, xs, plane, scratch, [&] {
+    stream.request(a.k, lane);
+    ahead.request(a, min(first + min(lane, OUTPUTS - 1), a.n - 1));
+  });
   if (first >= a.n) return;
   stream.run(xs, plane, a.k, lane);
   const float(&sums)[ROWS] = stream.sums;
@@ -370,19 +418,32 @@ __global__ __launch_bounds__(256) void dense_gemv_kernel(DenseGemvArgs a) {
       mine = sums[GATED ? 2 * o : o];
       if (GATED) up = sums[2 * o + 1];
     }
-  if (lane < OUTPUTS && first + lane < a.n) gemv_epilogue<T>(a, first + lane, mine, up);
+  if (lane >= OUTPUTS || own >= a.n) return;
+  if (AHEAD == Ahead::kConv) a.out_f32[own] = ahead.finish(a, own, mine);
+  else gemv_epilogue<T>(a, own, mine, up);
 }
 
-template <typename T, int ROWS, bool GATED, bool VEC, Staging STAGING>
-hipError_t run_staged(const DenseGemvArgs &a, hipStream_t stream) {
+template <typename T, int ROWS, bool GATED, bool VEC, Staging STAGING, Ahead AHEAD>
+hipError_t run_ahead(const DenseGemvArgs &a, hipStream_t stream) {
   static bool allowed[kMaxDevices] = {};
-  const auto kernel = dense_gemv_kernel<T, ROWS, GATED, VEC, STAGING>;
+  const auto kernel = dense_gemv_kernel<T, ROWS, GATED, VEC, STAGING, AHEAD>;
   const uint32_t bytes = ((a.k + 7) / 8) * 32;
   if (bytes > 48 * 1024)
     if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), kGemvMaxK * 4, allowed)) return status;
   const uint32_t per = kWaves * (GATED ? ROWS / 2 : ROWS);
   kernel<<<(a.n + per - 1) / per, 256, bytes, stream>>>(a);
   return hipGetLastError();
+}
+
+// Kernels that request ahead only for rows of whole pieces that pass through registers (the others have loops before their sums).
+template <typename T, int ROWS, bool GATED, bool VEC, Staging STAGING>
+hipError_t run_staged(const DenseGemvArgs &a, hipStream_t stream) {
+  constexpr bool SHORT = STAGING == Staging::kPlainShort || STAGING == Staging::kNormedShort || STAGING == Staging::kPendingShort ||
+                         STAGING == Staging::kPendingPiece;
+  if constexpr (VEC && !GATED && SHORT) {
+    if (ahead_of(a) == Ahead::kConv) return run_ahead<T, ROWS, GATED, VEC, STAGING, Ahead::kConv>(a, stream);
+  }
+  return run_ahead<T, ROWS, GATED, VEC, STAGING, Ahead::kNothing>(a, stream);
 }
 
 template <typename T, int ROWS, bool GATED, bool VEC>

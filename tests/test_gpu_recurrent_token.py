@@ -63,3 +63,50 @@ def test_state_and_output(runtime, state_size, heads, vdim, groups, position):
     # a sum of state_size products and one, and the gate's quotient and exponential
     bound = (state_size + 32) * ULP * ((size * np.abs(c[group])).sum(-1) + np.abs(skip[head] * x)) * np.abs(gate) * (1.0 + np.abs(z))
     assert (np.abs(out.numpy(np.float32) - y) <= bound + 1e-30).all()
+
+
+# taps whose inputs are asked for beside the weights (up to four) or not; rows that pass through registers (whole pieces of eight, up
+# to 4096) or not; one and two rows a wave
+@pytest.mark.parametrize("taps", [1, 2, 4, 5])
+@pytest.mark.parametrize("position", [0, 1, 2, 11])
+@pytest.mark.parametrize("width,heads,vdim", [(8, 3, 5), (1024, 2, 8), (4096, 3, 5), (4104, 3, 5), (62, 3, 5), (16, 8, 128)])
+def test_projection_and_convolution(runtime, taps, position, width, heads, vdim):
+    rng = np.random.default_rng(width * 8 + taps)
+    groups, state_size, slots, slot, epsilon = 1, 6, 2, 1, np.float32(1e-5)
+    inner = heads * vdim
+    channels = inner + 2 * groups * state_size
+    n = inner + channels + heads
+    stream = rng.standard_normal(width).astype(np.float32)
+    (norm_bits, norm), (weight_bits, weights) = bf16(rng, width), bf16(rng, n, width)
+    (conv_bits, conv), (bias_bits, bias), (dt_bits, dt_bias) = bf16(rng, channels, taps), bf16(rng, channels), bf16(rng, heads)
+    ring = rng.standard_normal((slots, taps, channels)).astype(np.float32)
+    put = runtime.buffer_of_bytes
+    held, out, unused = put(ring), runtime.create_buffer(n * 4), runtime.create_buffer(heads * 4)
+    batch = runtime.begin_batch()
+    batch.dispatch("llmopt_rms_ssm_input_bf16",
+                   [put(stream), put(norm_bits), put(weight_bits), put(np.array([position, slot] + [0] * 6, np.uint32)), put(conv_bits),
+                    put(bias_bits), put(dt_bits), held, out, unused],
+                   u32s(1, width, heads, vdim, groups, state_size, taps, slots) + epsilon.tobytes(), *GRID)
+    batch.commit()
+    x = stream.astype(np.float64)
+    normed = x / np.sqrt(np.mean(x * x) + float(epsilon)) * norm
+    projected = weights @ normed
+    # the product's sum of `width` terms, and a few roundings of each term
+    error = (width + 16) * ULP * (np.abs(weights) @ np.abs(normed))
+    v, dv = projected[inner:inner + channels], error[inner:inner + channels]
+    total, size, dtotal = bias + conv[:, -1] * v, np.abs(bias) + np.abs(conv[:, -1] * v), np.abs(conv[:, -1]) * dv
+    for back in range(1, min(taps - 1, position) + 1):
+        past = conv[:, taps - 1 - back] * ring[slot, (position - back) % taps]
+        total, size = total + past, size + np.abs(past)
+    dtotal = dtotal + (taps + 2) * ULP * size
+    expected, bound = projected.copy(), error.copy()
+    expected[inner:inner + channels] = total / (1.0 + np.exp(-total))
+    bound[inner:inner + channels] = 1.1 * dtotal + 8 * ULP * np.abs(total) * (1.0 + np.abs(total))  # (silu's slope is at most 1.1)
+    z = projected[inner + channels:] + dt_bias
+    expected[inner + channels:] = np.log1p(np.exp(-np.abs(z))) + np.maximum(z, 0.0)
+    bound[inner + channels:] += 8 * ULP * (1.0 + np.abs(z))
+    assert (np.abs(out.numpy(np.float32) - expected) <= bound).all()
+    kept = held.numpy(np.float32, ring.shape)
+    assert (np.abs(kept[slot, position % taps] - v) <= dv).all()
+    ring[slot, position % taps] = kept[slot, position % taps]
+    assert (kept == ring).all()
