@@ -511,10 +511,10 @@ __global__ __launch_bounds__(256) void rotate_rows_kernel(ChunkAttentionArgs a) 
   }
 }
 
-template <typename T, int ND, int NE, bool RAW, bool JOIN>
+template <typename T, int ND, int NE, bool RAW, bool JOIN, bool FULL>
 __global__ __launch_bounds__(256) void chunk_decode_kernel(ChunkAttentionArgs a, uint32_t splits, uint32_t *counters) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  chunk_decode<T, ND, NE, RAW, JOIN>(a, splits, blockIdx.x, blockIdx.y, lds, counters);
+  chunk_decode<T, ND, NE, RAW, JOIN, FULL>(a, splits, blockIdx.x, blockIdx.y, lds, counters);
 }
 
 template <typename T>
@@ -523,15 +523,17 @@ __global__ __launch_bounds__(256) void chunk_merge_kernel(ChunkAttentionArgs a, 
   chunk_merge<T>(a, splits, blockIdx.x, shared);
 }
 
-template <typename T, int ND, int NE, bool RAW, bool JOIN>
+template <typename T, int ND, int NE, bool RAW, bool JOIN, bool FULL = false>
 hipError_t run_decode(const ChunkAttentionArgs &a, hipStream_t stream) {
+  if constexpr (sizeof(T) == 2 && !FULL)
+    if (full_heads<T, ND, NE>(a)) return run_decode<T, ND, NE, RAW, JOIN, true>(a, stream);
   static bool allowed[kMaxDevices] = {};
   constexpr int bytes = decode_lds_floats<T, NE>() * 4 + (RAW ? raw_row_lds_bytes<T, ND, NE>() : 0);
   const uint32_t splits = decode_splits(a);
   if (bytes > 64 * 1024)
-    if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(chunk_decode_kernel<T, ND, NE, RAW, JOIN>), bytes, allowed))
+    if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(chunk_decode_kernel<T, ND, NE, RAW, JOIN, FULL>), bytes, allowed))
       return status;
-  chunk_decode_kernel<T, ND, NE, RAW, JOIN><<<dim3(a.kv_heads, splits), 256, bytes, stream>>>(a, splits, a.counters);
+  chunk_decode_kernel<T, ND, NE, RAW, JOIN, FULL><<<dim3(a.kv_heads, splits), 256, bytes, stream>>>(a, splits, a.counters);
   if (hipError_t status = hipGetLastError()) return status;
   if (splits > 1 && !JOIN) chunk_merge_kernel<T><<<a.heads, 256, splits * 8, stream>>>(a, splits);
   return hipGetLastError();

@@ -63,17 +63,30 @@ struct HeadVector {
   template <typename Exchange>
   __device__ __forceinline__ void norm_and_rotate(const HeadRotation &r, const uint16_t *norm, uint32_t dim,
                                                   const Turn *turns, int lane, Exchange exchange) {
+    float weight[PARTS];
+    norm_weights(norm, dim, lane, weight);
+    normalise(r, weight, dim);
+    rotate(r, turns, lane, exchange);
+  }
+  static __device__ __forceinline__ void norm_weights(const uint16_t *norm, uint32_t dim, int lane, float (&weight)[PARTS]) {
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) {
+      const uint32_t c = lane + 64 * i;
+      weight[i] = c < dim ? (float)reinterpret_cast<const __bf16 *>(norm)[c] : 0.0f;
+    }
+  }
+  __device__ __forceinline__ void normalise(const HeadRotation &r, const float (&weight)[PARTS], uint32_t dim) {
     float sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < PARTS; ++i) sum += v[i] * v[i];
     const float inverse = 1.0f / sqrtf(wave_sum(sum) / (float)dim + r.epsilon);
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) v[i] *= inverse * weight[i];
+  }
+  template <typename Exchange>
+  __device__ __forceinline__ void rotate(const HeadRotation &r, const Turn *turns, int lane, Exchange exchange) {
     float partner[PARTS];
     const uint32_t half = r.dims / 2;
-#pragma unroll
-    for (int i = 0; i < PARTS; ++i) {
-      const uint32_t c = lane + 64 * i;
-      v[i] *= inverse * (c < dim ? (float)reinterpret_cast<const __bf16 *>(norm)[c] : 0.0f);
-    }
     exchange(v, partner, half);
 #pragma unroll
     for (int i = 0; i < PARTS; ++i) {
@@ -220,12 +233,16 @@ __device__ __forceinline__ void join_shares(const ChunkAttentionArgs &a, uint32_
 
 // The work of one workgroup of 256 threads; lds: decode_lds_floats (and raw_row_lds_bytes behind them).  JOIN: the last
 // workgroup of a key / value head (counters: one each) joins its shares; else they are a launch of their own.
-template <typename T, int ND, int NE, bool RAW, bool JOIN>
+// FULL: heads of just ND * 32 and NE * 16 bf16 values.  The code for partial pieces stands behind every load, and is fetched from
+// memory to be jumped over: without it, and with a raw row's vectors asked for ahead of the keys, a token of four layers of
+// 16 heads over 4 of 64 beside the delta rule takes 145.5 us instead of 150.8, of two attention layers among four 140 instead of 143.
+template <typename T, int ND, int NE, bool RAW, bool JOIN, bool FULL>
 __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32_t splits, uint32_t group, uint32_t split,
                                              char *lds, uint32_t *counters) {
   constexpr int EP = NE * 16, SV = value_stride<T, NE>(), V_PIECES = EP / 8;
   const uint32_t position = a.state[kStatePosition], slot = a.state[kStateSlot];
-  const uint32_t per = a.heads / a.kv_heads;
+  const uint32_t per = a.heads / a.kv_heads, dim = FULL ? ND * 32 : a.dim, vdim = FULL ? NE * 16 : a.vdim;
+  const bool vec = FULL || (dim % 8 == 0 && vdim % 8 == 0);
   const uint32_t begin = first_seen(position, a.cache) + split * kSplitKeys;
   if (begin > position) return;
   const uint32_t live = min(splits, (position - first_seen(position, a.cache)) / kSplitKeys + 1);
@@ -236,60 +253,92 @@ __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32
   static_assert(16 * EP * 4 <= OWN, "the sums fit the values' place");
   T *lds_v = reinterpret_cast<T *>(lds + wave * OWN);
   float *lds_top = reinterpret_cast<float *>(lds + 4 * OWN), *lds_total = lds_top + 4 * 16;  // [4][16] each
-  const bool vec = a.dim % 8 == 0 && a.vdim % 8 == 0;
   const size_t ring = ((size_t)slot * a.kv_heads + group) * a.cache.capacity;
-  const T *cache_k = static_cast<const T *>(a.cache.keys) + ring * a.dim;
-  const T *cache_v = static_cast<const T *>(a.cache.values) + ring * a.vdim;
+  const T *cache_k = static_cast<const T *>(a.cache.keys) + ring * dim;
+  const T *cache_v = static_cast<const T *>(a.cache.values) + ring * vdim;
   const uint32_t wave_begin = begin + wave * 32;
 
+  // A raw row's first vectors of each wave, their norms and the own value are asked for ahead of the keys: behind the keys and the
+  // position's turns they were two trips of their own.
+  constexpr int PARTS = ND <= 2 ? 1 : ND / 2, FIRST = 2;
+  HeadVector<PARTS> first[FIRST];
+  float first_weight[FIRST][PARTS], first_value[(EP + 255) / 256];
+  const uint32_t first_queries = min(16u, per);
+  if (RAW) {
+#pragma unroll
+    for (int j = 0; j < FIRST; ++j) {
+      const uint32_t n = min((uint32_t)wave + 4 * j, first_queries);  // (the last one is the key)
+      const bool query = n < first_queries;
+      const float *source = a.row + (query ? (size_t)(group * per + n) * dim : (size_t)(a.heads + group) * dim);
+#pragma unroll
+      for (int i = 0; i < PARTS; ++i) first[j].v[i] = lane + 64 * i < dim ? source[lane + 64 * i] : 0.0f;
+      HeadVector<PARTS>::norm_weights(query ? a.rotation.q_norm : a.rotation.k_norm, dim, lane, first_weight[j]);
+    }
+    const float *value = a.row + (size_t)(a.heads + a.kv_heads) * dim + (size_t)group * vdim;
+#pragma unroll
+    for (int i = 0; i < (EP + 255) / 256; ++i) first_value[i] = tid + 256 * i < vdim ? value[tid + 256 * i] : 0.0f;
+  }
   Frag<T> fk[2][ND], reg_v[NE];
 #pragma unroll
   for (int kt = 0; kt < 2; ++kt) {
-    const T *row = cache_k + (size_t)(min(wave_begin + kt * 16 + column, position) % a.cache.capacity) * a.dim;
+    const T *row = cache_k + (size_t)(min(wave_begin + kt * 16 + column, position) % a.cache.capacity) * dim;
 #pragma unroll
-    for (int d = 0; d < ND; ++d) fk[kt][d] = load_piece(row + d * 32 + quad * 8, (int)a.dim - (d * 32 + quad * 8), vec);
+    for (int d = 0; d < ND; ++d) fk[kt][d] = load_piece(row + d * 32 + quad * 8, FULL ? 8 : (int)dim - (d * 32 + quad * 8), vec);
   }
 #pragma unroll
   for (int i = 0; i < NE; ++i) {
     const int index = i * 64 + lane, row = index / V_PIECES, piece = (index % V_PIECES) * 8;
     const uint32_t j = min(wave_begin + row, position) % a.cache.capacity;
-    reg_v[i] = load_piece(cache_v + (size_t)j * a.vdim + piece, (int)a.vdim - piece, vec);
+    reg_v[i] = load_piece(cache_v + (size_t)j * vdim + piece, FULL ? 8 : (int)vdim - piece, vec);
   }
   const bool capped = a.softcap > 0.0f;
   const float cap = a.softcap * kLog2e;
   const float inner = capped ? 2.0f * a.scale / a.softcap * kLog2e : a.scale * kLog2e;
 
   // a raw row: the first sixteen queries and the own key and value
-  constexpr int SQ = ND * 32 + 16 / (int)sizeof(T), PARTS = ND <= 2 ? 1 : ND / 2;
+  constexpr int SQ = ND * 32 + 16 / (int)sizeof(T);
   T *lds_q = reinterpret_cast<T *>(lds + decode_lds_floats<T, NE>() * 4), *own_k = lds_q + 16 * SQ, *own_v = own_k + SQ;
   float *exchange = reinterpret_cast<float *>(own_v + EP) + wave * PARTS * 64;
   Turn *turns = reinterpret_cast<Turn *>(reinterpret_cast<float *>(own_v + EP) + 4 * PARTS * 64);
-  auto stage_vectors = [&](uint32_t h0, uint32_t count, bool key) {
-    for (uint32_t n = wave; n < count + (key ? 1 : 0); n += 4) {
+  const ThroughLds<PARTS> partners{exchange, a.rotation.dims, lane};
+  auto stage_vector = [&](const HeadVector<PARTS> &h, T *target) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i)
+      if (lane + 64 * i < ND * 32) target[lane + 64 * i] = (T)h.v[i];  // (zeros behind the head's end)
+  };
+  // the vectors from `from` on of the queries h0 .. and the key behind them
+  auto stage_vectors = [&](uint32_t from, uint32_t h0, uint32_t count, bool key) {
+    for (uint32_t n = from + wave; n < count + (key ? 1 : 0); n += 4) {
       const bool query = n < count;
-      const float *source = a.row + (query ? (size_t)(group * per + h0 + n) * a.dim : (size_t)(a.heads + group) * a.dim);
+      const float *source = a.row + (query ? (size_t)(group * per + h0 + n) * dim : (size_t)(a.heads + group) * dim);
       HeadVector<PARTS> h;
 #pragma unroll
-      for (int i = 0; i < PARTS; ++i) h.v[i] = lane + 64 * i < a.dim ? source[lane + 64 * i] : 0.0f;
-      h.norm_and_rotate(a.rotation, query ? a.rotation.q_norm : a.rotation.k_norm, a.dim, turns, lane,
-                        ThroughLds<PARTS>{exchange, a.rotation.dims, lane});
-      T *target = query ? lds_q + n * SQ : own_k;
-#pragma unroll
-      for (int i = 0; i < PARTS; ++i)
-        if (lane + 64 * i < ND * 32) target[lane + 64 * i] = (T)h.v[i];  // (zeros behind the head's end)
+      for (int i = 0; i < PARTS; ++i) h.v[i] = lane + 64 * i < dim ? source[lane + 64 * i] : 0.0f;
+      h.norm_and_rotate(a.rotation, query ? a.rotation.q_norm : a.rotation.k_norm, dim, turns, lane, partners);
+      stage_vector(h, query ? lds_q + n * SQ : own_k);
     }
   };
   if (RAW) {
     fill_turns(a.rotation, position, turns);
+#pragma unroll
+    for (int j = 0; j < FIRST; ++j) first[j].normalise(a.rotation, first_weight[j], dim);
     __syncthreads();
-    stage_vectors(0, min(16u, per), true);
-    const float *value = a.row + (size_t)(a.heads + a.kv_heads) * a.dim + (size_t)group * a.vdim;
-    for (uint32_t c = tid; c < EP; c += 256) own_v[c] = (T)(c < a.vdim ? value[c] : 0.0f);
+#pragma unroll
+    for (int j = 0; j < FIRST; ++j) {
+      const uint32_t n = wave + 4 * j;
+      if (n > first_queries) break;
+      first[j].rotate(a.rotation, turns, lane, partners);
+      stage_vector(first[j], n < first_queries ? lds_q + n * SQ : own_k);
+    }
+    stage_vectors(4 * FIRST, 0, first_queries, true);
+#pragma unroll
+    for (int i = 0; i < (EP + 255) / 256; ++i)
+      if (tid + 256 * i < EP) own_v[tid + 256 * i] = (T)first_value[i];  // (zeros behind the value's end)
     __syncthreads();
     if (begin + kSplitKeys > position) {  // this workgroup's keys end with the own one
       const size_t at = ring + position % a.cache.capacity;
-      for (uint32_t c = tid; c < a.dim; c += 256) static_cast<T *>(a.cache.keys)[at * a.dim + c] = own_k[c];
-      for (uint32_t c = tid; c < a.vdim; c += 256) static_cast<T *>(a.cache.values)[at * a.vdim + c] = own_v[c];
+      for (uint32_t c = tid; c < dim; c += 256) static_cast<T *>(a.cache.keys)[at * dim + c] = own_k[c];
+      for (uint32_t c = tid; c < vdim; c += 256) static_cast<T *>(a.cache.values)[at * vdim + c] = own_v[c];
     }
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
@@ -308,14 +357,14 @@ __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32
     const uint32_t head = group * per + min(h0 + column, per - 1);
     Frag<T> fq[ND];
     if (RAW && h0 > 0) {
-      stage_vectors(h0, min(16u, per - h0), false);
+      stage_vectors(0, h0, min(16u, per - h0), false);
       __syncthreads();
     }
 #pragma unroll
     for (int d = 0; d < ND; ++d)
       fq[d] = RAW ? *reinterpret_cast<const Frag<T> *>(lds_q + min((uint32_t)column, per - 1 - h0) * SQ + d * 32 + quad * 8)
-                  : load_piece(static_cast<const T *>(a.qkv) + (size_t)head * a.dim + d * 32 + quad * 8,
-                               (int)a.dim - (d * 32 + quad * 8), vec);
+                  : load_piece(static_cast<const T *>(a.qkv) + (size_t)head * dim + d * 32 + quad * 8,
+                               FULL ? 8 : (int)dim - (d * 32 + quad * 8), vec);
     f32x4 score[2];
     float best = -1e30f;
 #pragma unroll
@@ -372,7 +421,7 @@ __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32
     const uint32_t live = min(16u, per - h0);
     for (uint32_t i = tid; i < live * EP; i += 256) {
       const uint32_t h = i / EP, c = i % EP;
-      if (c >= a.vdim) continue;
+      if (c >= vdim) continue;
       float sum = 0.0f, all = 0.0f, top = -1e30f;
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
@@ -390,15 +439,15 @@ __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32
         }
         store_attention<T>(a, target, c, sum / all);
       } else {
-        float *partial = static_cast<float *>(a.workspace) + ((size_t)target * splits + split) * (a.vdim + 2);
+        float *partial = static_cast<float *>(a.workspace) + ((size_t)target * splits + split) * (vdim + 2);
         const auto leave = [](float *to, float v) {
           if (JOIN) hand_over(to, v);
           else *to = v;
         };
         leave(partial + c, sum);
         if (c == 0) {
-          leave(partial + a.vdim, top);
-          leave(partial + a.vdim + 1, all);
+          leave(partial + vdim, top);
+          leave(partial + vdim + 1, all);
         }
       }
     }
@@ -444,6 +493,11 @@ __device__ __forceinline__ void chunk_merge(const ChunkAttentionArgs &a, uint32_
   }
   if (c >= a.vdim) return;
   store_attention<T>(a, head, c, sum / denominator);
+}
+
+template <typename T, int ND, int NE>
+bool full_heads(const ChunkAttentionArgs &a) {
+  return sizeof(T) == 2 && a.dim == ND * 32 && a.vdim == NE * 16;
 }
 
 // Most shares of 128 keys that a token can have.

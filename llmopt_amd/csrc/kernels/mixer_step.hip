@@ -191,7 +191,7 @@ __device__ __forceinline__ void delta_columns(const DeltaArgs &a, uint32_t head,
 template <int ND, int NE>
 constexpr int attention_lds_bytes() { return decode_lds_floats<__bf16, NE>() * 4 + raw_row_lds_bytes<__bf16, ND, NE>(); }
 
-template <int ND, int NE, int R, bool JOIN>
+template <int ND, int NE, int R, bool JOIN, bool FULL>
 __global__ __launch_bounds__(kThreads) void mixer_step_kernel(ChunkAttentionArgs a, DeltaArgs d, uint32_t splits, float *squares, uint32_t *counters) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const uint32_t parts = d.vdim / kColumns, delta_blocks = d.heads * parts;
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kThreads) void mixer_step_kernel(ChunkAttentionArgs
   }
   if (threadIdx.x >= 256) return;  // (barriers count the waves that are still there)
   const uint32_t share = blockIdx.x - delta_blocks;
-  chunk_decode<__bf16, ND, NE, true, JOIN>(a, splits, share % a.kv_heads, share / a.kv_heads, lds, counters + d.heads);
+  chunk_decode<__bf16, ND, NE, true, JOIN, FULL>(a, splits, share % a.kv_heads, share / a.kv_heads, lds, counters + d.heads);
 }
 
 __global__ __launch_bounds__(256) void mixer_merge_kernel(ChunkAttentionArgs a, uint32_t splits) {
@@ -218,7 +218,9 @@ hipError_t run(const ChunkAttentionArgs &a, const DeltaArgs &d, float *squares, 
   ChunkAttentionArgs own = a;  // (the attention's counters lie behind the delta rule's)
   own.counter_count -= d.heads;
   const bool joins = joins_shares(own);
-  const auto kernel = joins ? mixer_step_kernel<ND, NE, R, true> : mixer_step_kernel<ND, NE, R, false>;
+  const auto kernel = full_heads<__bf16, ND, NE>(a)
+                          ? (joins ? mixer_step_kernel<ND, NE, R, true, true> : mixer_step_kernel<ND, NE, R, false, true>)
+                          : (joins ? mixer_step_kernel<ND, NE, R, true, false> : mixer_step_kernel<ND, NE, R, false, false>);
   kernel<<<blocks, kThreads, bytes, stream>>>(a, d, splits, squares, a.counters);
   if (hipError_t status = hipGetLastError()) return status;
   if (splits > 1 && !joins) mixer_merge_kernel<<<a.heads, 256, splits * 8, stream>>>(a, splits);
