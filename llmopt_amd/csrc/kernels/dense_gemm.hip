@@ -393,8 +393,11 @@ __device__ __forceinline__ void copy_to_lds(const __bf16 *source, uint32_t lds_a
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(source), "s"(lds_address) : "memory");
 }
 
-template <int BM, int BN, int WM, int WAVES, int STAGES, int GATED, bool ROUTED>
-__global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParams p) {
+//
+// PARTS: as many groups of waves, each with a ring of its own, take the stages in turn, and their sums meet in LDS: for launches
+// of few tiles, where a stage takes what its barrier and its trip take (dense_parts).
+template <int BM, int BN, int WM, int WAVES, int STAGES, int GATED, bool ROUTED, int PARTS = 1>
+__global__ __launch_bounds__(WAVES * PARTS * 64) void dense_gemm_direct_kernel(GemmParams p) {
   constexpr int WN = WAVES / WM;
   constexpr int MT = BM / WM / 16, NT = BN / WN / 16;
   constexpr int ROWS = BM + BN;              // LDS rows of a stage: activations, then weights
@@ -408,7 +411,8 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParam
   if (!place_tile<BM, COLUMNS, ROUTED>(p, place)) return;
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int part = PARTS > 1 ? __builtin_amdgcn_readfirstlane((tid >> 6) / WAVES) : 0;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) - part * WAVES;
   const int wm = wave / WN, wn = wave % WN;
 
   const __bf16 *source[COPIES];
@@ -432,11 +436,11 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParam
       source[i] = reinterpret_cast<const __bf16 *>(matrix) + ((size_t)place.expert * a.n + c) * a.k + piece * 8;
     }
   }
-  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)lds;
+  const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)lds + part * STAGES * ROWS * 128;
   auto request = [&](int stage) {
     const uint32_t slot = lds_base + (stage % STAGES) * ROWS * 128;
 #pragma unroll
-    for (int i = 0; i < COPIES; ++i) copy_to_lds(source[i] + stage * kStageK, slot + (i * WAVES + wave) * 1024);
+    for (int i = 0; i < COPIES; ++i) copy_to_lds(source[i] + (stage * PARTS + part) * kStageK, slot + (i * WAVES + wave) * 1024);
   };
 
   f32x4 acc[MT][NT];
@@ -445,12 +449,13 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParam
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  const int stages = (int)(a.k / kStageK);
+  // of this group, and steps of the workgroup (a group may have none in the last one)
+  const int all = (int)(a.k / kStageK), stages = (all - part + PARTS - 1) / PARTS, steps = (all + PARTS - 1) / PARTS;
   const int fr = lane & 15, quad = lane >> 4, twist = (fr >> 1) & 7;
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < stages) request(s);
-  for (int s = 0; s < stages; ++s) {
+  for (int s = 0; s < steps; ++s) {
     // this stage has landed once at most the copies of the STAGES - 2 later ones are under way (and this wave
     // has all it read of the stage before)
     if (s + STAGES - 2 < stages) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"((STAGES - 2) * COPIES) : "memory");
@@ -459,7 +464,8 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParam
     asm volatile("" ::: "memory");
     // every wave is done with the stage before: its slot is free
     if (s + STAGES - 1 < stages) request(s + STAGES - 1);
-    const __bf16 *rows = stage_rows + (s % STAGES) * ROWS * 64;
+    if (PARTS > 1 && s >= stages) break;  // (the last step)
+    const __bf16 *rows = stage_rows + (part * STAGES + s % STAGES) * ROWS * 64;
     const __bf16 *la = rows + (wm * (BM / WM) + fr) * 64, *lw = rows + (BM + wn * (BN / WN) + fr) * 64;
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -474,6 +480,27 @@ __global__ __launch_bounds__(WAVES * 64) void dense_gemm_direct_kernel(GemmParam
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = mma(fw[j], fa[i], acc[i][j]);
     }
+  }
+  if constexpr (PARTS > 1) {
+    constexpr int BYTES = MT * NT * 1024;  // of a wave's sums
+    static_assert((PARTS - 1) * WAVES * BYTES <= PARTS * STAGES * ROWS * 128, "the sums fit the rings' place");
+    __syncthreads();  // the rings are free
+    if (part > 0) {
+      char *mine = lds + ((part - 1) * WAVES + wave) * BYTES + lane * 16;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4 *>(mine + (i * NT + j) * 1024) = acc[i][j];
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int other = 0; other < PARTS - 1; ++other)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] += *reinterpret_cast<const f32x4 *>(lds + (other * WAVES + wave) * BYTES + lane * 16 + (i * NT + j) * 1024);
   }
   if (a.epilogue == DenseEpilogue::kAdd || a.epilogue == DenseEpilogue::kStoreF32) {
     emit_tile<__bf16, MT, NT, GATED>(a, acc, place.m_first, place.m_rows, place.n_first, wm * (BM / WM),
@@ -797,16 +824,16 @@ hipError_t run_turns(const DenseLinearArgs &a, Columns c, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WAVES, int STAGES, int GATED, bool ROUTED>
+template <int BM, int BN, int WM, int WAVES, int STAGES, int GATED, bool ROUTED, int PARTS = 1>
 hipError_t run_direct(const DenseLinearArgs &a, Columns c, hipStream_t stream) {
-  constexpr int bytes = STAGES * (BM + BN) * 128;
+  constexpr int bytes = PARTS * STAGES * (BM + BN) * 128;
   static bool allowed[kMaxDevices] = {};
-  const auto kernel = dense_gemm_direct_kernel<BM, BN, WM, WAVES, STAGES, GATED, ROUTED>;
+  const auto kernel = dense_gemm_direct_kernel<BM, BN, WM, WAVES, STAGES, GATED, ROUTED, PARTS>;
   if (bytes > 64 * 1024)
     if (hipError_t status = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes, allowed)) return status;
   dim3 grid;
   const GemmParams p = gemm_params<BM, GATED ? BN / 2 : BN, ROUTED>(a, &grid, c);
-  kernel<<<grid, WAVES * 64, bytes, stream>>>(p);
+  kernel<<<grid, WAVES * PARTS * 64, bytes, stream>>>(p);
   return hipGetLastError();
 }
 
@@ -877,7 +904,18 @@ hipError_t pick_gemm(const DenseLinearArgs &a, hipStream_t stream) {
   const uint32_t first = (uint32_t)(dense_first_columns(a.m, (uint64_t)a.n * MATRICES, a.k, cus) / MATRICES);
   if (first > 0)
     if (hipError_t status = run_phased<GATED>(a, {0, first}, stream)) return status;
-  return run_tile<GATED>(dense_product_tile(a.m, (uint64_t)(a.n - first) * MATRICES, a.k, cus), a, {first, a.n}, stream);
+  const DenseTile tile = dense_product_tile(a.m, (uint64_t)(a.n - first) * MATRICES, a.k, cus);
+  switch (first == 0 ? dense_parts(tile, a.m, (uint64_t)a.n * MATRICES, a.k, GATED != 0, cus) : DenseParts::kNone) {
+    case DenseParts::k16x32:
+      if constexpr (!GATED) return run_direct<16, 32, 1, 2, 3, GATED, false, 8>(a, {0, a.n}, stream);
+      break;
+    case DenseParts::k32x32:
+      if constexpr (!GATED) return run_direct<32, 32, 2, 4, 4, GATED, false, 4>(a, {0, a.n}, stream);
+      break;
+    case DenseParts::k32x64: return run_direct<32, 64, 2, 4, 3, GATED, false, 4>(a, {0, a.n}, stream);
+    case DenseParts::kNone: break;
+  }
+  return run_tile<GATED>(tile, a, {first, a.n}, stream);
 }
 
 // ---- row-wise kernels ------------------------------------------------------------------------------

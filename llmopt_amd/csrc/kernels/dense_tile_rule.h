@@ -125,6 +125,23 @@ inline DenseTile dense_product_tile(uint32_t m, uint64_t columns, uint32_t k, ui
   return best;
 }
 
+// Products that 32 x 64 tiles suit best leave CUs without a tile, and each stage of a tile takes what its trip and its barrier
+// take, 0.28 us a stage of 64 values whatever the rest.  They run on the smallest of these whose tiles come to one a CU at most,
+// with groups of waves that take the stages in turn (eight groups of two waves, four of four).  us, one group on 32 x 64 tiles /
+// 32 x 32 / 16 x 32, weights from HBM: 64 x 1024 x 4096 17.9 / 12.1 / 9.9, x 2048 10.1 / 6.3 / 5.3, x 1024 6.5 / 4.7 / 4.2, x 512
+// 4.8 / 4.1 / 3.8, x 256 4.1 / 3.8 / 3.6, x 128 3.0 / 3.2 / 3.2: from K = 256.  Where 32 x 32 tiles are more than the CUs, 32 x 64 ones
+// in four groups: 500 x 1024 x 4096 18.4 / 15.6, x 1024 6.8 / 5.9, x 512 5.0 / 5.0, 64 x 8192 x 1024 7.95 / 7.98: from K = 1024.
+// A pair needs both matrices in a wave, which the smaller ones do not hold: 32 x 64 as well, beyond a quarter of the CUs from K = 2048
+// (of single matrices 16 x 4096 x 1024 7.12 / 7.13, 16 x 8192 x 1024 7.39 / 7.56, x 2048 11.7 / 11.6).
+enum class DenseParts { kNone, k16x32, k32x32, k32x64 };
+inline DenseParts dense_parts(DenseTile tile, uint32_t m, uint64_t columns, uint32_t k, bool pair, uint32_t cus) {
+  const auto tiles = [&](uint32_t rows, uint32_t wide) { return (uint64_t)((m + rows - 1) / rows) * ((columns + wide - 1) / wide); };
+  if (tile != DenseTile::k32x64 || k < 256) return DenseParts::kNone;
+  if (!pair && tiles(16, 32) <= cus) return DenseParts::k16x32;
+  if (!pair && tiles(32, 32) <= cus) return DenseParts::k32x32;
+  return k >= (pair && tiles(32, 64) > cus / 4 ? 2048 : 1024) && tiles(32, 64) <= cus ? DenseParts::k32x64 : DenseParts::kNone;
+}
+
 // A product in two launches: the first `columns` on whole rounds of 256 x 256 tiles, the rest on the tile that suits it (0: one
 // launch).  A round of the 256 CUs that is a tenth filled costs most of a whole one, and smaller tiles for all of the columns
 // are the slower ones.  Taken where the two estimates together are 5% less than the one launch's: at 108 sizes drawn, on four
