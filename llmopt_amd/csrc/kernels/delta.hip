@@ -656,18 +656,42 @@ __global__ __launch_bounds__(256, WAVES) void delta_chunk_kernel(DeltaArgs a, De
                         j + 1 <= token ? lds_t[token * kSliceStride + j + 1] * lds_beta[j + 1] : 0.0f);
     }
   const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (uint32_t tile = 0; tile < w.ep; tile += 16) {
-    const T *v = values + tile * Q + lane * 8;
-    f32x4 x = mma_wide(solve[0], *reinterpret_cast<const Frag<T> *>(v), zero);
-    if (wave >= 2) x = mma_wide(solve[1], *reinterpret_cast<const Frag<T> *>(v + 512), x);
-    *reinterpret_cast<f32x4 *>(w.solved + (each * w.ep + tile) * Q + wave * 256 + lane * 4) = x;
+  // Tiles in groups whose operands are asked for together (those behind the last one again): one by one each is a trip to memory,
+  // which nothing covers in a launch of few workgroups: one chunk of 8 heads 37.5 us -> 33.1, 47 of 16 heads the same.
+  constexpr uint32_t GROUP = 4;
+  for (uint32_t first = 0; first < w.ep; first += 16 * GROUP) {
+    Frag<T> v[GROUP][2];
+#pragma unroll
+    for (uint32_t g = 0; g < GROUP; ++g) {
+      const T *at = values + min(first + 16 * g, w.ep - 16) * Q + lane * 8;
+      v[g][0] = *reinterpret_cast<const Frag<T> *>(at);
+      v[g][1] = *reinterpret_cast<const Frag<T> *>(at + 512);
+    }
+#pragma unroll
+    for (uint32_t g = 0; g < GROUP; ++g) {
+      const uint32_t tile = first + 16 * g;
+      if (tile >= w.ep) break;
+      f32x4 x = mma_wide(solve[0], v[g][0], zero);
+      if (wave >= 2) x = mma_wide(solve[1], v[g][1], x);
+      *reinterpret_cast<f32x4 *>(w.solved + (each * w.ep + tile) * Q + wave * 256 + lane * 4) = x;
+    }
   }
-  for (uint32_t tile = 0; tile < np; tile += 16) {
-    const T *keys = kd + tile * Q + lane * 8;
-    f32x4 x = mma_wide_both(load_wide<T>(keys, plane), solve[0], zero);
-    if (wave >= 2) x = mma_wide_both(load_wide<T>(keys + 512, plane), solve[1], x);
-    const float four[4] = {x[0], x[1], x[2], x[3]};
-    store_wide<T>(w_out + operand_at(token, tile + quad * 4, np), plane, four);
+  static_assert(np % (16 * GROUP) == 0, "whole groups");
+  for (uint32_t first = 0; first < np; first += 16 * GROUP) {
+    WideFrag<T> keys[GROUP][2];
+#pragma unroll
+    for (uint32_t g = 0; g < GROUP; ++g) {
+      const T *at = kd + (first + 16 * g) * Q + lane * 8;
+      keys[g][0] = load_wide<T>(at, plane);
+      keys[g][1] = load_wide<T>(at + 512, plane);
+    }
+#pragma unroll
+    for (uint32_t g = 0; g < GROUP; ++g) {
+      f32x4 x = mma_wide_both(keys[g][0], solve[0], zero);
+      if (wave >= 2) x = mma_wide_both(keys[g][1], solve[1], x);
+      const float four[4] = {x[0], x[1], x[2], x[3]};
+      store_wide<T>(w_out + operand_at(token, first + 16 * g + quad * 4, np), plane, four);
+    }
   }
 }
 
