@@ -643,7 +643,7 @@ int llmopt_hip_prebaked_execute(llmopt_hip_prebaked *plan, int64_t token, int64_
         if (out_token) *out_token = (int64_t)result[0];
         return LLMOPT_OK;
       }
-      plan->resident->gave_up = true;  // the step again, launch by launch: what it wrote so far is written anew
+      plan->resident->gave_up = true;  // the step again, launch by launch (find_resident_run: it reads nothing that it wrote so far)
     }
   }
   int32_t result[2] = {0, 0};

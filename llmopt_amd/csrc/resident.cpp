@@ -23,6 +23,36 @@ const uint16_t *halves(const DispatchRecord &record, size_t index) {
   return reinterpret_cast<const uint16_t *>(record.buffers[index].device);
 }
 
+// The records that may stand beside a run: they read the buffers in front of `outputs` and write the others, the first `bytes`
+// of each.
+struct Beside {
+  const char *name;
+  size_t buffers, parameter_bytes, outputs;
+  size_t (*bytes)(const DispatchRecord &record, size_t index);
+};
+size_t whole(const DispatchRecord &record, size_t index) { return record.buffers[index].length; }
+size_t product(const DispatchRecord &record, size_t first, size_t second, size_t bytes) {
+  return (size_t)param_u32(record, first) * param_u32(record, second) * bytes;
+}
+size_t head_bytes(const DispatchRecord &record, size_t index) {
+  return index == 0 ? product(record, 0, 8, 2) : index == 4 ? (size_t)param_u32(record, 0) * 4 : index == 5 ? product(record, 0, 4, 2) : whole(record, index);
+}
+size_t first_stage_bytes(const DispatchRecord &record, size_t index) {
+  return index == 4 ? (size_t)param_u32(record, 0) * 256 * 8 : head_bytes(record, index);
+}
+const Beside kBeside[] = {
+    {"llmopt_embedding_f16", 3, 12, 2,
+     [](const DispatchRecord &r, size_t i) { return i == 0 ? (size_t)param_u32(r, 0) * 8 : i == 1 ? whole(r, i) : product(r, 0, 8, 2); }},
+    {"llmopt_rms_norm_f16_simd", 3, 12, 2, [](const DispatchRecord &r, size_t i) { return i == 1 ? whole(r, i) : product(r, 0, 4, 2); }},
+    {"llmopt_add_f16", 3, 136, 2, [](const DispatchRecord &r, size_t i) { return i == 2 ? (size_t)param_u32(r, 0) * 2 : whole(r, i); }},
+    {"llmopt_w4a16_lm_head_argmax_f16", 5, 16, 4, head_bytes},
+    {"llmopt_w4a16_lm_head_argmax_extra_f16", 6, 16, 4, head_bytes},
+    {"llmopt_w4a16_lm_head_argmax_stage1_f16", 5, 16, 4, first_stage_bytes},
+    {"llmopt_w4a16_lm_head_argmax_stage1_extra_f16", 6, 16, 4, first_stage_bytes},
+    {"llmopt_w4a16_lm_head_reduce", 2, 4, 1,
+     [](const DispatchRecord &r, size_t i) { return (size_t)param_u32(r, 0) * (i == 0 ? 256 * 8 : 4); }},
+};
+
 struct Stream {  // rows as the next layer takes them
   const uint8_t *rows = nullptr, *partials = nullptr;
   uint32_t partial_count = 0;
@@ -54,7 +84,7 @@ class Finder {
     scratch_.resize(kept_scratch);
     run_.count = kept_records;
     run_.args.layer_count = (uint32_t)kept_layers;
-    return kept_layers >= kLeastLayers && fits() ? kept_records : 0;
+    return kept_layers >= kLeastLayers && fits() && may_run_again() ? kept_records : 0;
   }
   const ResidentRun &run() const { return run_; }
 
@@ -65,6 +95,8 @@ class Finder {
     const uint8_t *device;
     size_t length;
     bool marked;
+    bool overlaps(const Range &other) const { return device < other.device + other.length && other.device < device + length; }
+    bool holds(const Range &other) const { return device <= other.device && other.device + other.length <= device + length; }
   };
   std::vector<Range> scratch_;  // what the launches of the run write and the resident launch does not
   const uint8_t *out_ = nullptr;
@@ -222,18 +254,61 @@ class Finder {
     for (const ResidentLayer &layer : run_.layers)
       for (const uint8_t *weight : layer.weight)
         if ((bits(weight) & 7) != 0) return false;
-    const size_t out_bytes = (size_t)a.m * a.h * 2;
-    const auto overlap = [](const uint8_t *x, size_t nx, const uint8_t *y, size_t ny) { return x < y + ny && y < x + nx; };
-    const uint8_t *const result = reinterpret_cast<const uint8_t *>(a.x_out);
+    const Range result = result_rows();
     for (const Range &range : scratch_) {
-      if (range.device == out_ && range.length >= out_bytes) continue;  // the run's result, which the resident launch writes too
-      if (!range.marked || overlap(range.device, range.length, result, out_bytes)) return false;
+      if (range.device == out_ && range.length >= result.length) continue;  // the run's result, which the resident launch writes too
+      if (!range.marked || range.overlaps(result)) return false;
       for (size_t i = 0; i < records_.size(); ++i) {
         if (i >= run_.first && i < run_.first + run_.count) continue;
         for (const BoundBuffer &buffer : records_[i].buffers)
-          if (overlap(buffer.device, buffer.length, range.device, range.length)) return false;
+          if (range.overlaps({buffer.device, buffer.length, false})) return false;
       }
     }
+    return true;
+  }
+
+  Range result_rows() const { return {out_, (size_t)run_.args.m * run_.args.h * 2, false}; }
+
+  // A step whose resident launch gave up runs again from its first record, and the launch has left numbers where its result
+  // belongs.  That comes to the same as a first run where no record writes what the step finds there and reads: the rows that
+  // come in may be the result's only where a record in front writes all of them anew, and what is known of the records beside the
+  // run must be enough to tell.  (The layers' own cache rows: each writes its new token's before it reads the sequence's.)
+  bool may_run_again() const {
+    std::vector<Range> read, written;  // (read: what the step finds there)
+    const Range rows_in = {reinterpret_cast<const uint8_t *>(run_.args.x_in), result_rows().length, false};
+    const Range pool = {run_.args.pool, records_[run_.first].buffers[15].length, false};
+    const auto reads = [&](const Range &range) {
+      for (const Range &earlier : written)
+        if (earlier.holds(range)) return;
+      read.push_back(range);
+    };
+    for (size_t i = 0; i < records_.size(); ++i) {
+      const DispatchRecord &record = records_[i];
+      if (i >= run_.first && i < run_.first + run_.count) {
+        if (i == run_.first) reads(rows_in);
+        for (const BoundBuffer &buffer : record.buffers) {
+          const Range range = {buffer.device, buffer.length, false};
+          const bool between = std::any_of(scratch_.begin(), scratch_.end(),
+                                           [&](const Range &scratch) { return scratch.device != out_ && scratch.overlaps(range); });
+          if (!between && buffer.device != rows_in.device && buffer.device != out_) reads(range);
+        }
+        if (i + 1 == run_.first + run_.count) written.push_back(result_rows());
+        continue;
+      }
+      const auto known = std::find_if(std::begin(kBeside), std::end(kBeside), [&](const Beside &beside) {
+        return is(record, beside.name, beside.buffers, beside.parameter_bytes);
+      });
+      if (known == std::end(kBeside)) return false;
+      for (size_t b = 0; b < record.buffers.size(); ++b) {
+        const Range range = {record.buffers[b].device, std::min(known->bytes(record, b), record.buffers[b].length), false};
+        if (range.overlaps(pool)) return false;
+        if (b < known->outputs) reads(range);
+        else written.push_back(range);
+      }
+    }
+    for (const Range &range : read)
+      for (const Range &other : written)
+        if (range.overlaps(other)) return false;
     return true;
   }
 };

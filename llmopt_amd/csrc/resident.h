@@ -15,7 +15,8 @@ struct ResidentRun {
 
 // The run of a list of records, if it has one: layers in the forms that a decode step is made of (the three launches of
 // small batches, the five of larger ones), one behind the other on one stream of rows, of sizes that the kernel takes, whose
-// buffers between the records are scratch (llmopt_hip_buffer_set_scratch) and not read outside the run.
+// buffers between the records are scratch (llmopt_hip_buffer_set_scratch) and not read outside the run, in a step that may run
+// again from its first record after the resident launch gave up: no record writes what the step finds there and reads.
 bool find_resident_run(const std::vector<DispatchRecord> &records, ResidentRun *out);
 
 }  // namespace llmopt

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from oracle.chain import decode_chain
+from tests.test_gpu_glue import pointwise_params
 from tests.test_gpu_prebaked import build_step, make_case
 
 pytestmark = pytest.mark.gpu
@@ -163,3 +164,87 @@ def test_plans_on_two_threads(runtime):
         del sets
     finally:
         other.close()
+
+
+def run_list(runtime, dispatches):
+    batch = runtime.begin_batch()
+    for name, buffers, parameters, grid, group in dispatches:
+        batch.dispatch(name, buffers, parameters, grid=grid, group=group)
+    batch.commit()
+
+
+@pytest.mark.parametrize("lengths", [[70], [70, 65, 3]])
+def test_layers_alone_that_give_up(runtime, lengths, monkeypatch):
+    """Layers over rows that the host wrote, which are also the rows that come out: nothing in the plan writes them anew, so they
+    must still be there for the launches."""
+    from llmopt_amd.native import Prebaked
+    monkeypatch.setenv("LLMOPT_RESIDENT_WAIT_US", "0")
+    eager, eager_pool, frozen, frozen_pool, _ = small_plan(runtime, lengths)
+    layers = frozen.dispatches[1:]
+    plan = Prebaked(runtime, layers, frozen.tokens, frozen.token_ids)
+    rows = np.random.default_rng(5).standard_normal((len(lengths), 192)).astype(np.float16)
+    for _ in range(2):
+        for step in (eager, frozen):
+            step.work["x"][0].write(rows)
+        run_list(runtime, eager.dispatches[1:])
+        plan.execute(0, int(frozen.host_lengths[0]))
+        np.testing.assert_array_equal(frozen.work["x"][0].numpy(np.uint16), eager.work["x"][0].numpy(np.uint16))
+        np.testing.assert_array_equal(frozen.token_ids.numpy(np.uint32), eager.token_ids.numpy(np.uint32))
+        np.testing.assert_array_equal(frozen_pool.numpy(np.uint8), eager_pool.numpy(np.uint8))
+
+
+@pytest.mark.parametrize("place", ["in front", "behind", "both"])
+def test_records_beside_the_layers_run_once(runtime, place, monkeypatch):
+    """A record that reads what the step changes (an in-place add; a row that a later record replaces) must not run twice when the
+    layers give up."""
+    from llmopt_amd.native import Prebaked
+    monkeypatch.setenv("LLMOPT_RESIDENT_WAIT_US", "0")
+    eager, _, frozen, _, _ = small_plan(runtime, [70])
+    h = eager.config.hidden
+    params = pointwise_params((h,), (h,), (h,))
+    one = np.full(h, 1.0, dtype=np.float16)
+
+    def around(step):
+        one_row, sum_row, other = (runtime.buffer_of_bytes(v) for v in (one, one * 2, one * 4))
+        add = lambda left, right, out: ("llmopt_add_f16", [left, right, out], params, (h, 1, 1), (256, 1, 1))
+        if place == "in front":
+            return sum_row, [add(sum_row, one_row, sum_row), *step.dispatches]
+        if place == "behind":
+            return sum_row, [*step.dispatches, add(sum_row, one_row, sum_row)]
+        # in front: other = sum + 1; behind: sum = other + 1
+        return sum_row, [add(sum_row, one_row, other), *step.dispatches, add(other, one_row, sum_row)]
+
+    want, eager_list = around(eager)
+    got, frozen_list = around(frozen)
+    plan = Prebaked(runtime, frozen_list, frozen.tokens, frozen.token_ids)
+    eager.tokens.write(np.asarray([7], dtype=np.int64))
+    for _ in range(2):
+        run_list(runtime, eager_list)
+        plan.execute(7, int(frozen.host_lengths[0]))
+        np.testing.assert_array_equal(got.numpy(np.float16), want.numpy(np.float16))
+        np.testing.assert_array_equal(frozen.work["x"][0].numpy(np.uint16), eager.work["x"][0].numpy(np.uint16))
+
+
+def test_which_records_beside_the_layers_may_run_again(runtime):
+    """The layers stay resident beside records that find what they read as it was (an add into the stream in front of the layers,
+    behind the embedding that writes it anew), and not beside others."""
+    from llmopt_amd.native import Prebaked
+    _, _, frozen, _, _ = small_plan(runtime, [70])
+    h, x = frozen.config.hidden, frozen.work["x"][0]
+    params = pointwise_params((h,), (h,), (h,))
+    row, out = (runtime.buffer_of_bytes(np.ones(h, dtype=np.float16)) for _ in range(2))
+    add = lambda left, right, to: ("llmopt_add_f16", [left, right, to], params, (h, 1, 1), (256, 1, 1))
+    resident = lambda records: Prebaked(runtime, records, frozen.tokens, frozen.token_ids).resident_layers
+    embedding, *rest = frozen.dispatches
+    assert resident([embedding, add(x, row, x), *rest]) == 5
+    assert resident([embedding, *rest, add(row, row, out)]) == 5
+    assert resident([embedding, *rest, add(row, row, row)]) == 0
+    assert resident(rest) == 0                               # rows from outside, which the result replaces
+    assert resident([embedding, *rest, add(row, row, x)]) == 5
+    half = x.view(0, h)                                      # half of the rows written anew
+    assert resident([("llmopt_add_f16", [row, row, half], pointwise_params((h // 2,), (h // 2,), (h // 2,)),
+                      (h, 1, 1), (256, 1, 1)), *rest]) == 0
+    # rows written into a buffer of their own: the result replaces nothing that is read
+    own = runtime.create_buffer(h * 2)
+    first = (rest[0][0], [own, *rest[0][1][1:]], *rest[0][2:])
+    assert resident([first, *rest[1:]]) == 5
