@@ -254,6 +254,13 @@ void llmopt_hip_release_prebaked(llmopt_hip_prebaked *plan);
  * :2186-2188), replays all records in order, waits, and returns the first
  * int32 of the output buffer in *out_token.
  * past_tokens beyond the slot tables' capacity is LLMOPT_ERR_INVALID.
+ * Whole layers of the batched decode entries may run as one resident launch
+ * (llmopt_hip_prebaked_resident_layers): the records' arithmetic and rounding
+ * points with sums in another order, so close to, and not bit for bit, what
+ * the records leave one by one.  When that launch gives up waiting (another
+ * process, or long work of another stream, holds the device), or a sequence's
+ * cached slots include one that the step itself writes, the step runs again
+ * by launches, as do all later ones of the plan.
  * Debug replays of the reference, switched on by the same environment
  * variables (:2203-2347): LLMOPT_PROFILE_BREAKDOWN runs the records one at a
  * time and prints GPU time by kernel name to stderr; LLMOPT_DEBUG_NAN_CHECK
@@ -273,8 +280,8 @@ int llmopt_hip_prebaked_bind_step(llmopt_hip_prebaked *plan, llmopt_hip_buffer *
 /* 1 when execute replays one HIP graph, 0 when it launches record by record
  * (no reference counterpart; for diagnostics and tests). */
 int llmopt_hip_prebaked_is_single_submission(llmopt_hip_prebaked *plan);
-/* The layers of the plan that execute runs as one resident launch, 0 when it launches every record (no
- * reference counterpart; for diagnostics and tests). */
+/* The layers of the plan that execute runs as one resident launch, 0 when it launches every record, as it does
+ * after such a launch gave up (no reference counterpart; for diagnostics and tests). */
 int llmopt_hip_prebaked_resident_layers(llmopt_hip_prebaked *plan);
 
 /* ---- ring queue ------------------------------------------------------------ */

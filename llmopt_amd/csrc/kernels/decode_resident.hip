@@ -28,7 +28,7 @@
 //
 // Waits are bounded: a wave that has polled for `wait_ticks` gives up, sets *failed and polls no more, as does every wave
 // that sees the word set; all go on to their end with whatever they hold (numbers only: no address depends on them).  The
-// host then runs the step by launches.
+// host then runs the step by launches, as it does where a sequence reads a slot that the step itself writes.
 #include <algorithm>
 #include <type_traits>
 
@@ -969,7 +969,17 @@ __global__ __launch_bounds__(kThreads) void decode_resident_kernel(ResidentArgs 
   uint32_t *slot_cache = reinterpret_cast<uint32_t *>(resident_lds + a.lds.slots);
   const Run run = {(uint32_t)owner, has_run ? min(tokens, past - begin) : 0,
                    global<uint32_t>(a.slots + (uint32_t)__builtin_amdgcn_readlane((int)runs.offset, owner) + begin), (Local<uint32_t>)slot_cache};
-  for (uint32_t i = threadIdx.x; i < min(run.length, kSlotCache); i += kThreads) slot_cache[i] = run.slots[i];
+  // Launches pack the new tokens of all sequences before any of them reads the cache; here the cache is read layers ahead.  So a
+  // step in which a sequence reads a slot that the step itself writes (consecutive tokens of one sequence as rows of a batch) is left
+  // to them.
+  const uint32_t t64 = threadIdx.x & 63, new_slot = t64 < a.m ? a.new_slots[t64] : 0;
+  bool written_now = false;
+  for (uint32_t i = threadIdx.x; i < run.length; i += kThreads) {
+    const uint32_t slot = run.slots[i];
+    if (i < kSlotCache) slot_cache[i] = slot;
+    for (uint32_t s = 0; s < a.m; ++s) written_now |= slot == (uint32_t)__builtin_amdgcn_readlane((int)new_slot, (int)s);
+  }
+  if (written_now) __hip_atomic_store(a.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (threadIdx.x < a.h) {
     uint16_t *const gains = reinterpret_cast<uint16_t *>(resident_lds + a.lds.gains);
     gains[threadIdx.x] = a.layers[0].attention_norm[threadIdx.x];

@@ -173,7 +173,7 @@ struct ResidentArgs {
   uint64_t *hand;       // words.total words; zero before the first step
   ResidentWords words;
   const uint32_t *tag;  // of the step's first layer: layer_count + 1 apart from step to step, never 0
-  uint32_t *failed;     // set when a wait ran out: what the step left is then not to be used
+  uint32_t *failed;     // set when a wait ran out or a sequence's slots hold one of new_slots: what the step left is then not to be used
   uint64_t wait_ticks;  // of wall_clock64 (10 ns)
   struct {              // byte offsets in the workgroup's memory, set by resident_lds
     uint32_t new_rows, new_score, run_out, reduce, scales, gains, squares, patches, slots, layers, merge;

@@ -248,3 +248,34 @@ def test_which_records_beside_the_layers_may_run_again(runtime):
     own = runtime.create_buffer(h * 2)
     first = (rest[0][0], [own, *rest[0][1][1:]], *rest[0][2:])
     assert resident([first, *rest[1:]]) == 5
+
+
+# slot table offsets, contexts, and the slot table's entry that the new token takes; the sizes of the layers
+@pytest.mark.parametrize("offsets, lengths, new, shape", [
+    ([0, 0, 0], [70, 71, 72], [70, 71, 72], (192, 3, 1, 256)),   # consecutive tokens of one sequence
+    ([0, 100], [70, 90], [70, 5], (192, 3, 1, 256)),             # one sequence's new token in another's context
+    ([0], [70], [69], (192, 3, 1, 256)),                         # in its own, the last token
+    ([0], [9000], [1200], (64, 1, 1, 64)),                       # behind those slots of a run that the launch keeps at hand
+])
+def test_slots_that_the_step_itself_writes(runtime, offsets, lengths, new, shape):
+    """The new tokens are in the cache before any sequence reads it: such a step runs by launches."""
+    from llmopt_amd.decode_step import DecodeConfig, random_weights
+    from llmopt_amd.native import Prebaked
+    rng = np.random.default_rng(23)
+    hidden, q_heads, kv_heads, mlp = shape
+    config = DecodeConfig(hidden=hidden, q_heads=q_heads, kv_heads=kv_heads, head_dim=64, mlp=mlp, layers=4, vocabulary=300)
+    weights = random_weights(config, rng)
+    pool, slots, *_, capacity, _ = make_case(rng, config, [offsets[-1] + lengths[-1]], 70)
+    case = pool, slots, np.asarray(offsets, np.uint32), slots[np.asarray(new)], capacity, len(lengths)
+    eager, eager_pool = build_step(runtime, config, weights, case, lengths, 70)
+    frozen, frozen_pool = build_step(runtime, config, weights, case, lengths, 70)
+    plan = Prebaked(runtime, frozen.dispatches, frozen.tokens, frozen.token_ids)
+    assert plan.resident_layers == 4
+    tokens = rng.integers(0, config.vocabulary, len(lengths))
+    for _ in range(2):
+        want = eager.run(tokens)
+        frozen.tokens.write(np.asarray(tokens, dtype=np.int64))
+        assert plan.execute(int(tokens[0]), lengths[0]) == int(want[0])
+        assert plan.resident_layers == 0
+        np.testing.assert_array_equal(frozen.work["x"][0].numpy(np.uint16), eager.work["x"][0].numpy(np.uint16))
+        np.testing.assert_array_equal(frozen_pool.numpy(np.uint8), eager_pool.numpy(np.uint8))
