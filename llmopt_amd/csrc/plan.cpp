@@ -177,13 +177,14 @@ int capture_records(llmopt_hip_prebaked *plan, bool resident, hipGraph_t *out_gr
 
 int capture_plan(llmopt_hip_prebaked *plan) {
   destroy_graph(plan);
-  int status = capture_records(plan, false, &plan->graph, &plan->executable);
-  // (the records' own workspace is as large as it gets by now)
-  if (status == LLMOPT_OK && plan->resident)
-    status = capture_records(plan, true, &plan->resident->graph, &plan->resident->executable);
-  if (status != LLMOPT_OK) {
+  if (int status = capture_records(plan, false, &plan->graph, &plan->executable)) {
     destroy_graph(plan);
     return status;
+  }
+  // (the records' own workspace is as large as it gets by now; a second graph that fails leaves the plan with its first)
+  if (plan->resident && capture_records(plan, true, &plan->resident->graph, &plan->resident->executable) != LLMOPT_OK) {
+    (void)hipGetLastError();
+    plan->resident.reset();
   }
   plan->workspace_generation = plan->library->context->workspace_generation;
   return LLMOPT_OK;
@@ -254,6 +255,7 @@ int wait_for_step(llmopt_hip_prebaked *plan, int64_t token, int64_t past_tokens,
   if (int status = check_step(plan, past_tokens, &token_slot)) return status;
   if (plan->executable == nullptr || plan->workspace_generation != context->workspace_generation)
     if (int status = capture_plan(plan)) return status;
+  resident = resident && plan->resident;  // (the capture may have left the plan without)
   StepWords &words = *plan->step;  // (no step of this plan is under way: each is waited for)
   words = {};
   words.token = token_slot;
