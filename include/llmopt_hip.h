@@ -260,7 +260,8 @@ void llmopt_hip_release_prebaked(llmopt_hip_prebaked *plan);
  * the records leave one by one.  When that launch gives up waiting (another
  * process, or long work of another stream, holds the device), or a sequence's
  * cached slots include one that the step itself writes, the step runs again
- * by launches, as do all later ones of the plan.
+ * by launches, as do all later ones of the plan.  Steps of other threads do
+ * not change what a plan leaves: such launches wait for room on the device.
  * Debug replays of the reference, switched on by the same environment
  * variables (:2203-2347): LLMOPT_PROFILE_BREAKDOWN runs the records one at a
  * time and prints GPU time by kernel name to stderr; LLMOPT_DEBUG_NAN_CHECK

@@ -2,12 +2,12 @@
 // them.  A record named "layers" is a resident run; its parameters are the workgroups and the layers.
 #include "plan.cpp"
 
-#include <mutex>
-#include <set>
+#include <unistd.h>
 
 namespace {
 struct Graph {
   bool resident = false;
+  uint32_t workgroups = 0;
   const StepWords *step = nullptr;
 };
 struct Launch {
@@ -20,6 +20,7 @@ Graph *capturing = nullptr;  // (plans are made one by one)
 uint32_t layer_workgroups = 0, resident_layers = 4;
 bool refuse_resident_graph = false, gives_up = false;
 int cleared = 0, live_graphs = 0;
+uint32_t under_way = 0, most_under_way = 0;  // workgroups of resident launches
 }  // namespace
 
 extern "C" {
@@ -54,10 +55,16 @@ hipError_t hipGraphInstantiate(hipGraphExec_t *out, hipGraph_t graph, hipGraphNo
 hipError_t hipGraphLaunch(hipGraphExec_t executable, hipStream_t) {
   const Graph &of = *reinterpret_cast<Graph *>(executable);
   StepWords *step = const_cast<StepWords *>(of.step);
-  std::lock_guard<std::mutex> hold(lock);
-  launches.push_back({of.resident, step->resident_tag});
+  {
+    std::lock_guard<std::mutex> hold(lock);
+    launches.push_back({of.resident, step->resident_tag});
+    most_under_way = std::max(most_under_way, under_way += of.workgroups);
+  }
+  if (of.resident) usleep(500);
   step->result[0] = (int32_t)step->value + 1;
   step->result[1] = of.resident && gives_up;
+  std::lock_guard<std::mutex> hold(lock);
+  under_way -= of.workgroups;
   return hipSuccess;
 }
 }  // extern "C"
@@ -95,7 +102,10 @@ ResidentWords resident_words(uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, u
 }
 uint32_t resident_lds(ResidentArgs &, uint32_t) { return 0; }
 bool resident_fits(const ResidentArgs &, uint32_t, uint32_t) { return true; }
-hipError_t launch_decode_resident(const ResidentArgs &, uint32_t, uint32_t, hipStream_t) { return capturing->resident = true, hipSuccess; }
+hipError_t launch_decode_resident(const ResidentArgs &, uint32_t workgroups, uint32_t, hipStream_t) {
+  capturing->resident = true;
+  return capturing->workgroups = workgroups, hipSuccess;
+}
 }  // namespace llmopt
 
 extern "C" {
@@ -106,6 +116,7 @@ void stub_set(uint32_t workgroups, uint32_t layers, int refuse, int give_up) {
   layer_workgroups = workgroups, resident_layers = layers, refuse_resident_graph = refuse != 0, gives_up = give_up != 0;
   launches.clear();
   cleared = 0;
+  most_under_way = 0;
 }
 void *stub_plan(const char *name) {
   llmopt_hip_library *library = new llmopt_hip_library;
@@ -126,5 +137,6 @@ long stub_launches(uint32_t *tags, long most) {  // of each launch the step's ta
   return (long)launches.size();
 }
 int stub_cleared() { return cleared; }
+uint32_t stub_most_under_way() { return most_under_way; }
 int stub_live_graphs() { return live_graphs; }
 }

@@ -2,6 +2,7 @@
 import ctypes
 import os
 import subprocess
+import threading
 
 import pytest
 
@@ -28,8 +29,8 @@ def stub(tmp_path_factory):
 
 
 def tags(stub):
-    out = (ctypes.c_uint32 * 64)()
-    return list(out[:stub.stub_launches(out, 64)])
+    out = (ctypes.c_uint32 * 4096)()
+    return list(out[:stub.stub_launches(out, 4096)])
 
 
 def test_plans_and_their_graphs(stub):
@@ -80,3 +81,31 @@ def test_tags_come_round_over_cleared_words(stub):
     assert tags(stub) == [near - 65, near, near + 65, 1, 66] and near + 65 + 64 < 2 ** 32
     assert cleared == [0, 0, 1, 1, 1]
     stub.llmopt_hip_release_prebaked(plan)
+
+
+@pytest.mark.parametrize("workgroups, most", [([96, 96], 192), ([96] * 5, 192), ([129, 128], 129), ([121, 128], 249), ([256] * 3, 256),
+                                              ([96, 256, 24, 40, 96], 256)])
+def test_resident_launches_of_several_threads(stub, workgroups, most):
+    """Every step of every plan is resident, whatever other threads do; launches share the device as long as all their workgroups,
+    in whole sets of eight, find room."""
+    plans = []
+    for count in workgroups:
+        stub.stub_set(count, 4, 0, 0)
+        plans.append(stub.stub_plan(b"layers"))
+    stub.stub_set(0, 4, 0, 0)
+
+    def steps(plan):
+        for token in range(30):
+            assert stub.stub_step(plan, token) == token + 1
+
+    threads = [threading.Thread(target=steps, args=(plan,)) for plan in plans]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert sorted(tags(stub)) == sorted(1 + 5 * step for step in range(30) for _ in plans)
+    assert max(workgroups) <= stub.stub_most_under_way() <= 256
+    if len(set(workgroups)) <= 2:
+        assert stub.stub_most_under_way() == most
+    for plan in plans:
+        stub.llmopt_hip_release_prebaked(plan)
