@@ -306,7 +306,8 @@ __device__ __forceinline__ void walk_tiles(Attended &state, const uint8_t *patch
 
 // ---- the product phases ---------------------------------------------------------------------------------------
 enum Product { kQkv = 0, kOut = 1, kGateUp = 2, kDown = 3 };
-constexpr int groups_most(int product) { return product == kDown ? 4 : 2; }  // scale groups of a wave: every eighth of the row's
+constexpr uint32_t kMostWidth = 1024, kMostMlp = 2048;  // of rows and of heads together; of the SwiGLU
+constexpr int groups_most(int product) { return (product == kDown ? kMostMlp : kMostWidth) / 64 / kWaves; }  // of a wave: every eighth of the row's
 
 // A wave's scale groups wave, wave + 8, ... of 16 weight rows, as a lane of the matrix instruction holds them (row lane % 16,
 // K values [16 (lane / 16), + 16) of a group), and one of the tile's scales: of row t % 16 and group t / 16.
@@ -389,8 +390,8 @@ struct Resident {
   const uint32_t run_slot, kv_of_run;  // the run's place among all, and the KV head of it that the workgroup takes
   const uint32_t first_tag;  // of the first layer
   Patience patience;
-  TileWeights<2> w_qkv, w_out, w_gate, w_up;
-  TileWeights<4> w_down;
+  TileWeights<groups_most(kQkv)> w_qkv, w_out, w_gate, w_up;
+  TileWeights<groups_most(kDown)> w_down;
 
   __device__ __forceinline__ const ResidentLayer &layer(uint32_t index) const {
     return reinterpret_cast<const ResidentLayer *>(lds + a.lds.layers)[index];
@@ -595,15 +596,15 @@ struct Resident {
       const uint16_t *const x = act + (ONE ? 0 : min(lane & 15, rows - 1) * stride) + quad * 16 + wave * 64;
       f4_t sum[P == kGateUp ? 2 : 1];
       if constexpr (P == kGateUp) {
-        const TileWeights<2> *const both[2] = {&w_gate, &w_up};
-        tile_share<2, 2>(sum, both, scales, x, groups, wave, quad);
+        const TileWeights<groups_most(P)> *const both[2] = {&w_gate, &w_up};
+        tile_share<2, groups_most(P)>(sum, both, scales, x, groups, wave, quad);
         leave(reduce + kReduceWords, sum[1]);
       } else if constexpr (P == kDown) {
-        const TileWeights<4> *const one[1] = {&w_down};
-        tile_share<1, 4>(sum, one, scales, x, groups, wave, quad);
+        const TileWeights<groups_most(P)> *const one[1] = {&w_down};
+        tile_share<1, groups_most(P)>(sum, one, scales, x, groups, wave, quad);
       } else {
-        const TileWeights<2> *const one[1] = {P == kQkv ? &w_qkv : &w_out};
-        tile_share<1, 2>(sum, one, scales, x, groups, wave, quad);
+        const TileWeights<groups_most(P)> *const one[1] = {P == kQkv ? &w_qkv : &w_out};
+        tile_share<1, groups_most(P)>(sum, one, scales, x, groups, wave, quad);
       }
       leave(reduce, sum[0]);
       __syncthreads();
@@ -1001,8 +1002,8 @@ uint32_t padded(uint32_t bytes) { return (bytes + 15) & ~15u; }
 }  // namespace
 
 bool resident_ok(uint32_t m, uint32_t h, uint32_t q_heads, uint32_t kv_heads, uint32_t mlp, uint32_t layers) {
-  return m >= 1 && m <= kResidentRows && layers >= 1 && layers <= kResidentLayers && h % 64 == 0 && h >= 64 && h <= 1024 && kv_heads >= 1 &&
-         kv_heads <= 8 && q_heads >= 1 && q_heads <= 16 && q_heads % kv_heads == 0 && mlp % 64 == 0 && mlp >= 64 && mlp <= 2048;
+  return m >= 1 && m <= kResidentRows && layers >= 1 && layers <= kResidentLayers && h % 64 == 0 && h >= 64 && h <= kMostWidth && kv_heads >= 1 &&
+         kv_heads <= 8 && q_heads >= 1 && q_heads * 64 <= kMostWidth && q_heads % kv_heads == 0 && mlp % 64 == 0 && mlp >= 64 && mlp <= kMostMlp;
 }
 
 // Workgroups: one a CU at most, so that all are resident together.  One sequence takes as many as its widest phase has tiles, the
@@ -1035,8 +1036,8 @@ ResidentWords resident_words(uint32_t m, uint32_t h, uint32_t q_heads, uint32_t 
   return words;
 }
 
-// Lays out a workgroup's memory and deals the products to the workgroups: units of as few sequences as still leave each
-// workgroup at most one (fewer words for each to poll), sixteen at most.
+// Lays out a workgroup's memory and deals the products to the workgroups: units of as few sequences (four, eight or
+// sixteen) as still leave each workgroup at most one: fewer words for each to poll.
 uint32_t resident_lds(ResidentArgs &a, uint32_t workgroups) {
   const uint32_t qd = a.q_heads * 64, kvd = a.kv_heads * 64;
   const uint32_t k[4] = {a.h, qd, a.h, a.mlp}, tiles[4] = {(qd + 2 * kvd) / kTile, a.h / kTile, a.mlp / kTile, a.h / kTile};
