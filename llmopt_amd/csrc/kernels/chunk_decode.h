@@ -2,6 +2,7 @@
 // keys, the merge of the shares, and the norm and rotation of heads.
 #pragma once
 
+#include "chunk_join_rule.h"
 #include "dense.h"
 #include "dense_common.h"
 
@@ -506,18 +507,8 @@ inline uint32_t decode_splits(const ChunkAttentionArgs &a) {
   return (longest + kSplitKeys - 1) / kSplitKeys;
 }
 
-// Whether the last workgroup of each key / value head joins its shares.  That saves a launch, and with one live share the
-// arrival too, but one workgroup does for all the head's queries what the merge spreads over a workgroup each.  us a call,
-// merge / join, query heads over key heads x width, at the ring's end and (first) with one live share:
-//   16 over 4 x 64 (256 outputs a key head)    6.5 / 4.5;  2 shares 6.6 / 6.2, 16 9.7 / 6.7, 17 10.1 / 8.8, 64 22.8 / 15.2
-//   32 over 8 x 128 (512)                      8.1 / 5.8;  2 shares 8.2 / 8.0, 16 11.2 / 9.7, 17 11.6 / 12.9, 64 27.3 / 25.2
-//   64 over 4 x 64 (1024)                      7.2 / 5.3;  2 shares 7.4 / 8.5, 8 7.5 / 8.6, 16 10.6 / 12.9
-constexpr uint32_t kJoinOutputs = 512, kJoinShares = 16, kJoinOutputsOfMore = 256, kJoinMostShares = 64;
 inline bool joins_shares(const ChunkAttentionArgs &a) {
-  const uint32_t splits = decode_splits(a), per = a.heads / a.kv_heads;
-  return a.counters != nullptr && a.kv_heads <= a.counter_count && splits > 1 && splits <= kJoinMostShares &&
-         (uint64_t)per * a.vdim <= (splits <= kJoinShares ? kJoinOutputs : kJoinOutputsOfMore) &&
-         (uint64_t)per * (2 * splits + 1) + 1 <= (uint64_t)decode_lds_floats<__bf16, 2>();  // (the least a workgroup has)
+  return a.counters != nullptr && joins(decode_splits(a), a.heads, a.kv_heads, a.vdim, a.counter_count, decode_lds_floats<__bf16, 2>());
 }
 
 }  // namespace llmopt

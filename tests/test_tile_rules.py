@@ -7,11 +7,12 @@ import subprocess
 import pytest
 
 from tests import (test_gpu_attention_tiles, test_gpu_delta_chunks, test_gpu_dense_attention, test_gpu_dense_tiles,
-                   test_gpu_w4a16_rows)
+                   test_gpu_joined_shares, test_gpu_product_parts, test_gpu_w4a16_rows)
 
 CUS = 256
 KERNELS = os.path.join(os.path.dirname(__file__), "..", "llmopt_amd", "csrc", "kernels")
 SOURCE = """
+#include "chunk_join_rule.h"
 #include "delta_rule.h"
 #include "dense_attention_rule.h"
 #include "dense_tile_rule.h"
@@ -64,6 +65,14 @@ float product_estimate(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
   float time = 0.0f;
   dense_product_tile(m, n, k, cus, &time);
   return time;
+}
+int product_parts(uint32_t m, uint32_t n, uint32_t k, uint32_t pair, uint32_t cus) {
+  const uint64_t columns = (uint64_t)n * (pair ? 2 : 1);
+  if (dense_first_columns(m, columns, k, cus) != 0) return 0;
+  return (int)dense_parts(dense_product_tile(m, columns, k, cus), m, columns, k, pair != 0, cus);
+}
+int joined(uint32_t capacity, uint32_t heads, uint32_t kv_heads, uint32_t vdim, uint32_t counters) {
+  return joins((capacity + 127) / 128, heads, kv_heads, vdim, counters, 3200);
 }
 int normed_pair(uint32_t m, uint32_t n, uint32_t k, uint32_t cus) {
   const uint32_t columns = 2 * n;
@@ -395,3 +404,43 @@ def test_large_w4a16_tiles(rules, m, n, k, tile):
                                         (2048, 2048, 576, "128x128 deep"), (2048, 14336, 1 << 23, "128x128 deep")])
 def test_large_w4a16_pair_tiles(rules, m, n, k, tile):
     assert LARGE[rules.large_pair_tile(m, n, k, CUS)] == tile
+
+
+PARTS = ("none", "16x32", "32x32", "32x64")
+
+
+def test_gpu_tests_reach_every_product_in_parts(rules):
+    tests = test_gpu_product_parts.SIZES
+    assert {PARTS[rules.product_parts(m, n, k, 0, CUS)] for m, n, k in tests} == set(PARTS)
+    assert {PARTS[rules.product_parts(m, n + 40, k, 0, CUS)] for m, n, k in tests} == set(PARTS)
+    assert {PARTS[rules.product_parts(m, max(16, n // 2), k, 1, CUS)] for m, n, k in tests} == {"none", "32x64"}
+
+
+@pytest.mark.parametrize("m,n,k,pair,form", [
+    (64, 1024, 4096, 0, "16x32"), (64, 1024, 256, 0, "16x32"), (64, 1024, 192, 0, "none"),    # a tile a CU, K = 256
+    (64, 2048, 256, 0, "16x32"), (64, 2049, 256, 0, "32x32"), (64, 4096, 512, 0, "32x32"),    # 256 tiles of 16 x 32, of 32 x 32
+    (64, 4097, 1024, 0, "32x64"), (64, 4097, 960, 0, "none"), (64, 8192, 1024, 0, "32x64"),   # of 32 x 64, K = 1024
+    (64, 8193, 1024, 0, "none"), (500, 1024, 1024, 0, "32x64"),
+    (64, 512, 1024, 1, "32x64"), (64, 512, 960, 1, "none"),                                   # a pair: a quarter of the CUs
+    (16, 4096, 1024, 1, "none"), (16, 4096, 2048, 1, "32x64"),
+])
+def test_products_in_parts(rules, m, n, k, pair, form):
+    assert PARTS[rules.product_parts(m, n, k, pair, CUS)] == form
+
+
+def test_gpu_tests_reach_both_ends_of_the_join(rules):
+    tests = test_gpu_joined_shares.test_shares_of_a_token
+    shapes, rings = sizes(tests, "heads,kv_heads,dim,vdim"), sizes(tests, "capacity")
+    for per_ring in ([rules.joined(ring, heads, kv, vdim, 1024) for ring in rings] for heads, kv, _, vdim in shapes):
+        assert not per_ring[0] and not per_ring[-1]  # one share, more than 64
+    assert len({tuple(rules.joined(ring, heads, kv, vdim, 1024) for ring in rings) for heads, kv, _, vdim in shapes}) >= 3
+
+
+@pytest.mark.parametrize("heads,kv_heads,vdim,capacity,join", [
+    (16, 4, 64, 256, 1), (16, 4, 64, 8192, 1), (16, 4, 64, 8193, 0), (16, 4, 64, 128, 0),     # 256 outputs: up to 64 shares
+    (32, 8, 128, 2048, 1), (32, 8, 128, 2049, 0), (64, 4, 64, 256, 0),                        # 512: up to 16; 1024: never
+    (96, 1, 5, 2048, 1), (97, 1, 5, 2048, 0),                                                 # what a workgroup's memory holds
+])
+def test_joined_shares(rules, heads, kv_heads, vdim, capacity, join):
+    assert rules.joined(capacity, heads, kv_heads, vdim, kv_heads) == join
+    assert rules.joined(capacity, heads, kv_heads, vdim, kv_heads - 1) == 0  # too few counters
