@@ -81,6 +81,70 @@ def test_resident_layers(runtime, lengths, hidden, q_heads, kv_heads, mlp, layer
     assert plan.resident_layers == layers  # no launch gave up
 
 
+@pytest.mark.parametrize("lengths", [[300], [20 * i for i in range(11)]])
+def test_thirty_layers(runtime, lengths):
+    """The depth of a real model, held to the oracle as the chain's launches are."""
+    from llmopt_amd.decode_step import DecodeConfig, random_weights
+    from llmopt_amd.native import Prebaked
+    rng = np.random.default_rng(8)
+    config = DecodeConfig(hidden=256, q_heads=4, kv_heads=2, mlp=512, layers=30, vocabulary=500)
+    weights = random_weights(config, rng)
+    case = make_case(rng, config, lengths, 66)
+    pool_host, slots, offsets, new_slots, capacity, batch = case
+    eager, _ = build_step(runtime, config, weights, case, lengths, 66)
+    frozen, frozen_pool = build_step(runtime, config, weights, case, lengths, 66)
+    plan = Prebaked(runtime, frozen.dispatches, frozen.tokens, frozen.token_ids)
+    assert plan.resident_layers == 30
+    tokens = rng.integers(0, config.vocabulary, batch)
+    eager.run(tokens)
+    frozen.tokens.write(np.asarray(tokens, dtype=np.int64))
+    plan.execute(int(tokens[0]), lengths[0])
+    want, logits, _ = decode_chain(config, weights, pool_host.copy(), slots, offsets, lengths, new_slots, lengths, tokens)
+    want = np.asarray(want, dtype=np.float64)
+    got, launched = (step.work["x"][0].numpy(np.float16, want.shape).astype(np.float64) for step in (frozen, eager))
+    off, launched_off = (np.linalg.norm(rows - want) / np.linalg.norm(want) for rows in (got, launched))
+    print(f"30 layers: {off:.2e} off the oracle, the launches {launched_off:.2e}", flush=True)
+    assert off <= 4e-3
+    top, rms = frozen.token_ids.numpy(np.uint32, (batch,)), np.sqrt(np.mean(logits.astype(np.float64) ** 2))
+    assert (logits[np.arange(batch), top] >= logits.max(axis=1) - 2e-2 * rms).all()
+    after = frozen_pool.numpy(np.uint8).reshape(capacity, -1)
+    untouched = np.setdiff1d(np.arange(capacity), new_slots)
+    np.testing.assert_array_equal(after[untouched], pool_host.reshape(capacity, -1)[untouched])
+    assert plan.resident_layers == 30
+
+
+# what a workgroup's memory holds: 48 sequences of the widest rows, the most layers, and heads whose runs just fit beside them
+@pytest.mark.parametrize("kv_heads, layers, resident", [(4, 64, 64), (2, 64, 0), (4, 65, 0)])
+def test_most_memory(runtime, kv_heads, layers, resident):
+    from llmopt_amd.decode_step import DecodeConfig, random_weights
+    from llmopt_amd.native import Prebaked
+    rng = np.random.default_rng(9)
+    one = DecodeConfig(hidden=1024, q_heads=16, kv_heads=kv_heads, mlp=2048, layers=1, vocabulary=64)
+    config = DecodeConfig(hidden=1024, q_heads=16, kv_heads=kv_heads, mlp=2048, layers=layers, vocabulary=64)
+    weights = random_weights(one, rng)
+    lengths = [3 * i for i in range(48)]
+    case = make_case(rng, config, lengths, 66)
+    first, _ = build_step(runtime, one, weights, case, lengths, 66)
+    device = {**first.device, "layers": first.device["layers"] * layers}  # (one layer's weights for all)
+    frozen, frozen_pool = build_step(runtime, config, {}, case, lengths, 66, device_weights=device)
+    plan = Prebaked(runtime, frozen.dispatches, frozen.tokens, frozen.token_ids)
+    assert plan.resident_layers == resident
+    if resident == 0:
+        return
+    eager, eager_pool = build_step(runtime, config, {}, case, lengths, 66, device_weights=device)
+    tokens = rng.integers(0, config.vocabulary, 48)
+    eager.run(tokens)
+    frozen.tokens.write(np.asarray(tokens, dtype=np.int64))
+    plan.execute(int(tokens[0]), lengths[0])
+    got, want = (step.work["x"][0].numpy(np.float16, (48, 1024)).astype(np.float64) for step in (frozen, eager))
+    # two chains that round at the same places, each within the chain's tolerance
+    assert np.isfinite(want).all() and np.linalg.norm(got - want) <= 8e-3 * np.linalg.norm(want)
+    stride = config.token_stride
+    untouched = np.setdiff1d(np.arange(case[4]), case[3])
+    np.testing.assert_array_equal(frozen_pool.numpy(np.uint8).reshape(-1, stride)[untouched], case[0].reshape(-1, stride)[untouched])
+    assert plan.resident_layers == 64
+
+
 def small_plan(runtime, lengths, layers=5):
     from llmopt_amd.decode_step import DecodeConfig, random_weights
     from llmopt_amd.native import Prebaked
