@@ -235,8 +235,8 @@ __device__ __forceinline__ void join_shares(const ChunkAttentionArgs &a, uint32_
 // The work of one workgroup of 256 threads; lds: decode_lds_floats (and raw_row_lds_bytes behind them).  JOIN: the last
 // workgroup of a key / value head (counters: one each) joins its shares; else they are a launch of their own.
 // FULL: heads of just ND * 32 and NE * 16 bf16 values.  The code for partial pieces stands behind every load, and is fetched from
-// memory to be jumped over: without it, and with a raw row's vectors asked for ahead of the keys, a token of four layers of
-// 16 heads over 4 of 64 beside the delta rule takes 145.5 us instead of 150.8, of two attention layers among four 140 instead of 143.
+// memory to be jumped over.  A token of four layers of 16 heads over 4 of 64 beside the delta rule: 146.9 us, with a raw row's vectors
+// asked for ahead of the keys 145.2, without that code too 142.9; of two attention layers among four 144.9, 144.2, 142.5.
 template <typename T, int ND, int NE, bool RAW, bool JOIN, bool FULL>
 __device__ __forceinline__ void chunk_decode(const ChunkAttentionArgs &a, uint32_t splits, uint32_t group, uint32_t split,
                                              char *lds, uint32_t *counters) {
